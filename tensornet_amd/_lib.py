@@ -166,6 +166,19 @@ def load():
     return lib
 
 
+def load_bind():
+    """The native module that marshals the operators' tensors (csrc/bind.cc); raises if it is not built."""
+    load()
+    try:
+        from . import _bind
+    except ImportError as e:
+        raise RuntimeError(
+            "tensornet_amd: the operator binding _bind.so is missing or does not load -- build it with "
+            "`python -m tensornet_amd.build`: %s" % e
+        )
+    return _bind
+
+
 def check(rc):
     if rc != TN_OK:
         raise TensorNetError(rc, load().tn_last_error().decode("utf-8", "replace"))

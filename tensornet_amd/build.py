@@ -1,4 +1,5 @@
-"""Builds the HIP library (libtensornet_amd.so) in-tree with hipcc for gfx950.
+"""Builds the HIP library (libtensornet_amd.so) in-tree with hipcc for gfx950, and the Python
+binding of its operators (_bind.so).
 
     python -m tensornet_amd.build
 
@@ -31,6 +32,9 @@ FLAGS = [
 ]
 
 
+BIND_SRC = os.path.join(CSRC, "bind.cc")
+BIND = os.path.join(HERE, "_bind.so")
+
 HOST_TEST_SRC = os.path.join(ROOT, "tests", "cpp", "host_mirror_test.cc")
 HOST_TEST_BIN = os.path.join(ROOT, "tests", "cpp", "host_mirror_test")
 
@@ -43,6 +47,26 @@ def build(verbose=True):
         print(" ".join(cmd), flush=True)
     subprocess.check_call(cmd)
     return LIB
+
+
+def build_bind(verbose=True):
+    """Builds the Python binding of the operators (host code over torch's C++ headers, linked to the library)."""
+    import sysconfig
+
+    import torch
+    from torch.utils.cpp_extension import include_paths, library_paths
+
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1",
+           "-DUSE_ROCM=1", "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch._C._GLIBCXX_USE_CXX11_ABI,
+           "-I", os.path.join(ROOT, "include"), "-I", os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "include"),
+           "-I", sysconfig.get_paths()["include"]]
+    cmd += [a for p in include_paths() for a in ("-isystem", p)]
+    cmd += [BIND_SRC, "-o", BIND, "-L", HERE, "-ltensornet_amd", "-Wl,-rpath,$ORIGIN"]
+    cmd += [a for p in library_paths() for a in ("-L", p)] + ["-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip"]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    subprocess.check_call(cmd)
+    return BIND
 
 
 def build_host_test(verbose=True):
@@ -58,5 +82,6 @@ def build_host_test(verbose=True):
 
 if __name__ == "__main__":
     build()
+    build_bind()
     build_host_test()
     sys.exit(0)

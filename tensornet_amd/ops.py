@@ -3,7 +3,8 @@
 wrappers tensornet/core/gen_sparse_table_ops.py / gen_dense_table_ops.py) with
 the same names and argument order, taking torch tensors that live on the GPU.
 Tensors are only used as device memory: every call goes through the C ABI with
-raw device pointers and the current HIP stream.
+raw device pointers and the current HIP stream.  The operators that run in every
+step are marshalled by a native module (csrc/bind.cc), the others through ctypes.
 
 A "resource" (tf.Variable handle in the reference) is here the variable's
 torch tensor itself, updated in place.
@@ -13,6 +14,8 @@ import ctypes as C
 import torch
 
 from . import _lib
+
+_bind = _lib.load_bind()
 
 
 def _stream():
@@ -35,86 +38,21 @@ class BoundSparseTablePull:
     stream current at that moment).  Calling it returns the N mapped-id tensors."""
 
     def __init__(self, resources, values, table_handle):
-        n = len(values)
-        if len(resources) != n:
-            raise ValueError("SparseTable pull num_inputs: %d not equal: %d" % (len(resources) + n, n * 2))
-        if n == 0:
-            raise ValueError("SparseTable pull needs at least one slot")
-        dim = None
-        for i in range(n):
-            _require(resources[i], torch.float32, "resources[%d]" % i)
-            _require(values[i], torch.int64, "values[%d]" % i)
-            if resources[i].dim() != 2:
-                raise ValueError(
-                    "sparse pull variable must Matrix(sign_id_cnt, dim), saw: %s" % (tuple(resources[i].shape),)
-                )
-            if values[i].dim() != 1:
-                raise ValueError("values[%d] must have rank 1" % i)
-            if dim is None:
-                dim = resources[i].shape[1]
-            elif dim != resources[i].shape[1]:
-                raise _lib.TensorNetError(3, "all variables of one pull must have the same dim")
-        lens = [v.numel() for v in values]
-        # one allocation for all mapped ids, handed out as per-slot views
-        flat = torch.empty(sum(lens), dtype=torch.int64, device=values[0].device)
-        self.mapped = list(flat.split(lens)) if sum(lens) > 0 else [torch.empty_like(v) for v in values]
-        self._keep = (list(resources), list(values), flat)
-        self._fn = _lib.load().tn_sparse_table_pull_op
-        self._args = (
-            table_handle,
-            n,
-            _lib.ptr_array([v.data_ptr() for v in values]),
-            _lib.i64_array(lens),
-            _lib.ptr_array([r.data_ptr() for r in resources]),
-            _lib.i64_array([r.shape[0] for r in resources]),
-            int(dim),
-            _lib.ptr_array([m.data_ptr() for m in self.mapped]),
-        )
+        self._call = _bind.bind_pull(resources, values, table_handle)
+        self.mapped = self._call.outputs
 
     def __call__(self):
-        _lib.check(self._fn(*self._args, _stream()))
-        return self.mapped
+        return self._call()
 
 
 class BoundSparseTablePush:
     """SparseTablePush bound to fixed tensors (see BoundSparseTablePull)."""
 
     def __init__(self, values, grads, feature_labels, table_handle):
-        n = len(values)
-        if len(grads) != n or len(feature_labels) != n:
-            raise ValueError(
-                "SparseTable push num_inputs: %d not equal: %d" % (n + len(grads) + len(feature_labels), n * 3)
-            )
-        if n == 0:
-            raise ValueError("SparseTable push needs at least one slot")
-        dim = None
-        for i in range(n):
-            _require(values[i], torch.int64, "values[%d]" % i)
-            _require(grads[i], torch.float32, "grads[%d]" % i)
-            _require(feature_labels[i], torch.int64, "feature_labels[%d]" % i)
-            if grads[i].dim() != 2:
-                raise ValueError("sparse push grad must Matrix(sign_id_cnt, dim), saw: %s" % (tuple(grads[i].shape),))
-            if feature_labels[i].numel() != values[i].numel():
-                raise ValueError("feature_labels[%d] must have one label per lookup" % i)
-            if dim is None:
-                dim = grads[i].shape[1]
-            elif dim != grads[i].shape[1]:
-                raise _lib.TensorNetError(3, "all gradients of one push must have the same dim")
-        self._keep = (list(values), list(grads), list(feature_labels))
-        self._fn = _lib.load().tn_sparse_table_push_op
-        self._args = (
-            table_handle,
-            n,
-            _lib.ptr_array([v.data_ptr() for v in values]),
-            _lib.i64_array([v.numel() for v in values]),
-            _lib.ptr_array([g.data_ptr() for g in grads]),
-            _lib.i64_array([g.shape[0] for g in grads]),
-            int(dim),
-            _lib.ptr_array([l.data_ptr() for l in feature_labels]),
-        )
+        self._call = _bind.bind_push(values, grads, feature_labels, table_handle)
 
     def __call__(self):
-        _lib.check(self._fn(*self._args, _stream()))
+        self._call()
 
 
 def sparse_table_pull(resources, values, table_handle):
@@ -122,14 +60,14 @@ def sparse_table_pull(resources, values, table_handle):
     place: row j <- embedding of the j-th distinct sign of the slot);
     values: N int64 rank-1 tensors of signs.  Returns N int64 tensors of mapped
     ids (same shapes as values)."""
-    return BoundSparseTablePull(resources, values, table_handle)()
+    return _bind.sparse_table_pull(resources, values, table_handle)
 
 
 def sparse_table_push(values, grads, feature_labels, table_handle):
     """SparseTablePush.  grads[i] is [U_i, dim] with row j the gradient of the
     j-th distinct sign of values[i]; feature_labels[i] has one int64 label per
     lookup.  Returns nothing (the update is enqueued on the current stream)."""
-    BoundSparseTablePush(values, grads, feature_labels, table_handle)()
+    _bind.sparse_table_push(values, grads, feature_labels, table_handle)
 
 
 COMBINERS = {"sum": 0, "mean": 1, "sqrtn": 2}
@@ -148,7 +86,7 @@ def embedding_lookup_sparse(resources, mapped_values, example_ids, batch_size, t
     the rows resources[s][mapped_values[s][i]] of the lookups i of example b.
     example_ids[s][i] is the example of lookup i (SparseTensor.indices[:, 0]).
     Returns N float32 tensors [batch_size, dim]."""
-    return BoundEmbeddingLookupSparse(resources, mapped_values, example_ids, batch_size, table_handle, combiner)()
+    return _bind.embedding_lookup_sparse(resources, mapped_values, example_ids, batch_size, table_handle, _combiner(combiner))
 
 
 class BoundEmbeddingLookupSparse:
@@ -156,37 +94,11 @@ class BoundEmbeddingLookupSparse:
     bound pull, the example ids, and outputs allocated once.  Calling it returns the N [batch_size, dim] tensors."""
 
     def __init__(self, resources, mapped_values, example_ids, batch_size, table_handle, combiner="mean"):
-        n = len(mapped_values)
-        if len(resources) != n or len(example_ids) != n or n == 0:
-            raise ValueError("embedding_lookup_sparse needs one variable, id tensor and example-id tensor per slot")
-        for i in range(n):
-            _require(resources[i], torch.float32, "resources[%d]" % i)
-            _require(mapped_values[i], torch.int64, "mapped_values[%d]" % i)
-            _require(example_ids[i], torch.int64, "example_ids[%d]" % i)
-            if example_ids[i].numel() != mapped_values[i].numel():
-                raise ValueError("example_ids[%d] must have one entry per lookup" % i)
-        dim = resources[0].shape[1]
-        flat = torch.empty((n, batch_size, dim), dtype=torch.float32, device=resources[0].device)
-        self.out = list(flat.unbind(0))
-        self._keep = (list(resources), list(mapped_values), list(example_ids), flat)
-        self._fn = _lib.load().tn_sparse_table_combine_op
-        self._args = (
-            table_handle,
-            n,
-            _lib.ptr_array([v.data_ptr() for v in mapped_values]),
-            _lib.i64_array([v.numel() for v in mapped_values]),
-            _lib.ptr_array([e.data_ptr() for e in example_ids]),
-            _lib.ptr_array([r.data_ptr() for r in resources]),
-            _lib.i64_array([r.shape[0] for r in resources]),
-            int(dim),
-            int(batch_size),
-            _combiner(combiner),
-            _lib.ptr_array([o.data_ptr() for o in self.out]),
-        )
+        self._call = _bind.bind_combine(resources, mapped_values, example_ids, batch_size, table_handle, _combiner(combiner))
+        self.out = self._call.outputs
 
     def __call__(self):
-        _lib.check(self._fn(*self._args, _stream()))
-        return self.out
+        return self._call()
 
 
 class BoundSparseTablePushPooled:
@@ -197,39 +109,15 @@ class BoundSparseTablePushPooled:
     BoundSparseTablePush."""
 
     def __init__(self, values, example_ids, pooled_grads, feature_labels, table_handle, combiner="mean"):
-        n = len(values)
-        if len(example_ids) != n or len(pooled_grads) != n or len(feature_labels) != n or n == 0:
-            raise ValueError("SparseTable push (pooled) needs values, example ids, gradients and labels per slot")
-        for i in range(n):
-            _require(values[i], torch.int64, "values[%d]" % i)
-            _require(example_ids[i], torch.int64, "example_ids[%d]" % i)
-            _require(pooled_grads[i], torch.float32, "pooled_grads[%d]" % i)
-            _require(feature_labels[i], torch.int64, "feature_labels[%d]" % i)
-            if pooled_grads[i].dim() != 2 or pooled_grads[i].shape != pooled_grads[0].shape:
-                raise ValueError("pooled_grads must all be Matrix(batch_size, dim)")
-            if example_ids[i].numel() != values[i].numel() or feature_labels[i].numel() != values[i].numel():
-                raise ValueError("example_ids / feature_labels of slot %d must have one entry per lookup" % i)
-        self._keep = (list(values), list(example_ids), list(pooled_grads), list(feature_labels))
-        self._fn = _lib.load().tn_sparse_table_push_pooled_op
-        self._args = (
-            table_handle,
-            n,
-            _lib.ptr_array([v.data_ptr() for v in values]),
-            _lib.i64_array([v.numel() for v in values]),
-            _lib.ptr_array([e.data_ptr() for e in example_ids]),
-            _lib.ptr_array([g.data_ptr() for g in pooled_grads]),
-            int(pooled_grads[0].shape[0]),
-            int(pooled_grads[0].shape[1]),
-            _combiner(combiner),
-            _lib.ptr_array([l.data_ptr() for l in feature_labels]),
-        )
+        self._call = _bind.bind_push_pooled(values, example_ids, pooled_grads, feature_labels, table_handle,
+                                            _combiner(combiner))
 
     def __call__(self):
-        _lib.check(self._fn(*self._args, _stream()))
+        self._call()
 
 
 def sparse_table_push_pooled(values, example_ids, pooled_grads, feature_labels, table_handle, combiner="mean"):
-    BoundSparseTablePushPooled(values, example_ids, pooled_grads, feature_labels, table_handle, combiner)()
+    _bind.sparse_table_push_pooled(values, example_ids, pooled_grads, feature_labels, table_handle, _combiner(combiner))
 
 
 def sparse_table_sync(table_handle):
@@ -260,47 +148,19 @@ def dense_table_init(vars, table_handle):
 def dense_table_push_pull(vars, grads, learning_rate, table_handle):
     """DenseTablePushPull: optimizer step with the concatenated gradients, new
     weights written back into the variables (in place)."""
-    if len(vars) != len(grads):
-        raise ValueError("DenseTable pushpull num_inputs: %d not equal: %d" % (len(vars) + len(grads) + 1, 2 * len(vars) + 1))
-    for i, (v, g) in enumerate(zip(vars, grads)):
-        _require(v, torch.float32, "vars[%d]" % i)
-        _require(g, torch.float32, "grads[%d]" % i)
-        if v.numel() != g.numel():
-            raise ValueError(
-                "DenseTable var tensor length: %d not equal grad tensor length: %d" % (v.numel(), g.numel())
-            )
-    rc = _lib.load().tn_dense_table_push_pull(
-        table_handle,
-        len(vars),
-        _lib.ptr_array([v.data_ptr() for v in vars]),
-        _lib.ptr_array([g.data_ptr() for g in grads]),
-        _lib.i64_array([g.numel() for g in grads]),
-        float(learning_rate),
-        _stream(),
-    )
-    _lib.check(rc)
+    _bind.dense_table_push_pull(vars, grads, learning_rate, table_handle)
 
 
 # ------------------------------------------------------------ table level
 def table_pull(table_handle, signs, dim):
     """SparseTable::Pull: signs int64/uint64-as-int64 [n] -> float32 [n, dim]."""
-    _require(signs, torch.int64, "signs")
-    out = torch.empty((signs.numel(), dim), dtype=torch.float32, device=signs.device)
-    rc = _lib.load().tn_sparse_table_pull(table_handle, signs.data_ptr(), signs.numel(), dim, out.data_ptr(), _stream())
-    _lib.check(rc)
-    return out
+    return _bind.table_pull(table_handle, signs, dim)
 
 
 def table_push(table_handle, sign_infos, grads):
     """SparseTable::Push: sign_infos is an int64 tensor [n, 2] holding the 16-byte
     records (sign, batch_show | batch_click << 32); grads float32 [n, dim]."""
-    _require(sign_infos, torch.int64, "sign_infos")
-    _require(grads, torch.float32, "grads")
-    n = grads.shape[0]
-    rc = _lib.load().tn_sparse_table_push(
-        table_handle, sign_infos.data_ptr(), grads.data_ptr(), n, grads.shape[1], _stream()
-    )
-    _lib.check(rc)
+    _bind.table_push(table_handle, sign_infos, grads)
 
 
 def make_sign_infos(signs, shows, clicks):
