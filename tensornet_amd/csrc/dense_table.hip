@@ -5,7 +5,7 @@
 //
 // The update is a pure stream: per parameter it reads g,w,m,v and writes
 // w,m,v (28 bytes) plus the 4-byte copy of w into the caller's variable, so it
-// is bound by HBM bandwidth.  One thread handles one float4 of each array.
+// is bound by HBM bandwidth.  One thread handles four elements of each array.
 // The reference's 8 blocks all step together on a single worker, so their
 // beta powers are identical and one pair is kept on the host.
 //
@@ -67,84 +67,89 @@ __device__ __forceinline__ void adagrad_elem(float g, float& w, float& d2, float
     w -= a.lr * m / (sqrtf(g2) / sqrtf(d2) + a.eps);
 }
 
-// n4 float4 groups starting at the (16-byte aligned) pointers.
-__global__ __launch_bounds__(256) void k_dense_adam_v4(const float4* __restrict__ g, float4* __restrict__ w,
-                                                       float4* __restrict__ m, float4* __restrict__ v,
-                                                       float4* __restrict__ out, int64_t n4, AdamArgs a) {
-    // every element is read once and written once per step: the accesses are marked non-temporal
-    // so that the stream does not displace the caches' contents
-    int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n4; i += stride) {
-        float4 gg = stream_load(&g[i]);
-        float4 ww = stream_load(&w[i]), mm = stream_load(&m[i]), vv = stream_load(&v[i]);
-        adam_elem(gg.x, ww.x, mm.x, vv.x, a);
-        adam_elem(gg.y, ww.y, mm.y, vv.y, a);
-        adam_elem(gg.z, ww.z, mm.z, vv.z, a);
-        adam_elem(gg.w, ww.w, mm.w, vv.w, a);
-        stream_store(&w[i], ww);
-        stream_store(&m[i], mm);
-        stream_store(&v[i], vv);
-        if (out) stream_store(&out[i], ww);
+// A float4 at any element of an array: the offset of a variable in the table is whatever the variables before it
+// leave (a bias of odd length, a shard's boundary), and gfx950 reads and writes 16 bytes at any 4-byte boundary.
+// Every element is read once and written once per step: the accesses are non-temporal, so that the stream does not
+// displace the caches' contents.
+typedef float any_float4 __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ float4 load4(const float* p) {
+    const any_float4 v = __builtin_nontemporal_load(reinterpret_cast<const any_float4*>(p));
+    return make_float4(v.x, v.y, v.z, v.w);
+}
+__device__ __forceinline__ void store4(float* p, float4 v) {
+    any_float4 n;
+    n.x = v.x, n.y = v.y, n.z = v.z, n.w = v.w;
+    __builtin_nontemporal_store(n, reinterpret_cast<any_float4*>(p));
+}
+
+// The variables of one launch: a step updates all of a network's variables at once.  One launch per variable, as
+// before, kept the host busy for 3 us each (8 variables of 0.75 M parameters in all: 33 us for a step whose
+// traffic takes 4 us), and a variable off a 16-byte boundary went element by element.
+constexpr int SEGMENTS = 64;          // variables per launch: what the lanes of a wavefront look through in one go
+constexpr int SEGMENT_BLOCK = 1024;   // elements of a variable per workgroup, four to a thread
+struct Segments {
+    uint32_t first_block[SEGMENTS];   // workgroups of the variables before this one (unused ones: 0xFFFFFFFF)
+    uint32_t off[SEGMENTS], len[SEGMENTS];  // the variable's range in the table's arrays (a table has less than 2^31 elements)
+    const float* g[SEGMENTS];
+    float* out[SEGMENTS];             // nullptr: no write-back
+};
+
+struct DenseArrays {
+    float *w, *s0, *s1, *s2;
+};
+
+// Adam (s0 = m, s1 = v) and AdaGrad (s0 = d2sum, s1 = g2sum, s2 = m).
+template <int KIND, typename Args>
+__device__ __forceinline__ void dense_step(const DenseArrays& t, const Segments& seg, const Args& a) {
+    // which variable this workgroup belongs to: the last one that starts at or before it
+    const int k = __popcll(__ballot(seg.first_block[threadIdx.x & 63] <= blockIdx.x)) - 1;
+    const uint32_t at = (blockIdx.x - seg.first_block[k]) * SEGMENT_BLOCK + threadIdx.x * 4;
+    const uint32_t len = seg.len[k];
+    if (at >= len) return;
+    const uint32_t i = seg.off[k] + at;
+    const float* g = seg.g[k] + at;
+    float* out = seg.out[k] ? seg.out[k] + at : nullptr;
+    auto elem = [&](float gv, float& w, float& x, float& y, float& z) {
+        if constexpr (KIND == OPT_ADAM)
+            adam_elem(gv, w, x, y, a);
+        else
+            adagrad_elem(gv, w, x, y, z, a);
+    };
+    if (at + 4 <= len) {
+        const float4 gg = load4(g);
+        float4 ww = load4(t.w + i), xx = load4(t.s0 + i), yy = load4(t.s1 + i), zz = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (KIND == OPT_ADAGRAD) zz = load4(t.s2 + i);
+        elem(gg.x, ww.x, xx.x, yy.x, zz.x);
+        elem(gg.y, ww.y, xx.y, yy.y, zz.y);
+        elem(gg.z, ww.z, xx.z, yy.z, zz.z);
+        elem(gg.w, ww.w, xx.w, yy.w, zz.w);
+        store4(t.w + i, ww);
+        store4(t.s0 + i, xx);
+        store4(t.s1 + i, yy);
+        if (KIND == OPT_ADAGRAD) store4(t.s2 + i, zz);
+        if (out) store4(out, ww);
+    } else {
+        for (uint32_t j = 0; at + j < len; j++) {
+            float z = KIND == OPT_ADAGRAD ? t.s2[i + j] : 0.f;
+            elem(g[j], t.w[i + j], t.s0[i + j], t.s1[i + j], z);
+            if (KIND == OPT_ADAGRAD) t.s2[i + j] = z;
+            if (out) out[j] = t.w[i + j];
+        }
     }
 }
 
-__global__ __launch_bounds__(256) void k_dense_adam_s(const float* __restrict__ g, float* __restrict__ w,
-                                                      float* __restrict__ m, float* __restrict__ v,
-                                                      float* __restrict__ out, int64_t n, AdamArgs a) {
-    int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
-        float ww = w[i], mm = m[i], vv = v[i];
-        adam_elem(g[i], ww, mm, vv, a);
-        w[i] = ww;
-        m[i] = mm;
-        v[i] = vv;
-        if (out) out[i] = ww;
-    }
+// Bound by HBM: 32 / 40 bytes per parameter.
+__global__ __launch_bounds__(256) void k_dense_adam_v4(DenseArrays t, Segments seg, AdamArgs a) {
+    dense_step<OPT_ADAM>(t, seg, a);
 }
-
-// The same for AdaGrad (ada_grad_kernel.cc:25-48): five arrays in, four (five with the variable) out.
-__global__ __launch_bounds__(256) void k_dense_adagrad_v4(const float4* __restrict__ g, float4* __restrict__ w,
-                                                          float4* __restrict__ d2, float4* __restrict__ g2,
-                                                          float4* __restrict__ m, float4* __restrict__ out, int64_t n4,
-                                                          AdaGradArgs a) {
-    int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n4; i += stride) {
-        float4 gg = stream_load(&g[i]);
-        float4 ww = stream_load(&w[i]), dd = stream_load(&d2[i]), ss = stream_load(&g2[i]), mm = stream_load(&m[i]);
-        adagrad_elem(gg.x, ww.x, dd.x, ss.x, mm.x, a);
-        adagrad_elem(gg.y, ww.y, dd.y, ss.y, mm.y, a);
-        adagrad_elem(gg.z, ww.z, dd.z, ss.z, mm.z, a);
-        adagrad_elem(gg.w, ww.w, dd.w, ss.w, mm.w, a);
-        stream_store(&w[i], ww);
-        stream_store(&d2[i], dd);
-        stream_store(&g2[i], ss);
-        stream_store(&m[i], mm);
-        if (out) stream_store(&out[i], ww);
-    }
-}
-
-__global__ __launch_bounds__(256) void k_dense_adagrad_s(const float* __restrict__ g, float* __restrict__ w,
-                                                         float* __restrict__ d2, float* __restrict__ g2,
-                                                         float* __restrict__ m, float* __restrict__ out, int64_t n,
-                                                         AdaGradArgs a) {
-    int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
-        float ww = w[i], dd = d2[i], gg2 = g2[i], mm = m[i];
-        adagrad_elem(g[i], ww, dd, gg2, mm, a);
-        w[i] = ww;
-        d2[i] = dd;
-        g2[i] = gg2;
-        m[i] = mm;
-        if (out) out[i] = ww;
-    }
+__global__ __launch_bounds__(256) void k_dense_adagrad_v4(DenseArrays t, Segments seg, AdaGradArgs a) {
+    dense_step<OPT_ADAGRAD>(t, seg, a);
 }
 
 __global__ __launch_bounds__(256) void k_fill_f32(float* p, int64_t n, float val) {
     int64_t stride = (int64_t)gridDim.x * blockDim.x;
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) p[i] = val;
 }
-
-bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 }  // namespace
 
@@ -336,41 +341,35 @@ int tn_dense_table_push_pull(uint32_t handle, int N, float* const* vars, const f
         ga.eps = o.epsilon;
     }
     int64_t var_off = 0;
+    Segments seg;
+    int k = 0;
+    uint32_t blocks = 0;
+    auto launch = [&] {
+        if (k == 0) return;
+        for (int j = k; j < SEGMENTS; j++) seg.first_block[j] = 0xFFFFFFFFu;
+        const DenseArrays arrays{t->w, t->s0, t->s1, t->s2};
+        if (o.kind == OPT_ADAM)
+            TN_LAUNCH(k_dense_adam_v4, dim3(blocks), dim3(256), st, arrays, seg, aa);
+        else
+            TN_LAUNCH(k_dense_adagrad_v4, dim3(blocks), dim3(256), st, arrays, seg, ga);
+        k = 0;
+        blocks = 0;
+    };
     for (int i = 0; i < N; i++) {
         // the part of variable i inside this shard's range
         const int64_t lo = std::max(var_off, t->begin), hi = std::min(var_off + lens[i], t->end);
         const int64_t skip = lo - var_off;
         var_off += lens[i];
         if (lo >= hi) continue;
-        const int64_t n = hi - lo, off = lo - t->begin;
-        float* out = (vars && vars[i]) ? vars[i] + skip : nullptr;
-        const float* g = grads[i] + skip;
-        if (o.kind == OPT_ADAM) {
-            bool vec = (off % 4 == 0) && aligned16(g) && (!out || aligned16(out));
-            int64_t n4 = vec ? n / 4 : 0;
-            if (n4 > 0) {
-                int blocks = launch_grid(n4, 256, 1 << 20);
-                TN_LAUNCH(k_dense_adam_v4, dim3(blocks), dim3(256), st, (const float4*)g, (float4*)(t->w + off), (float4*)(t->s0 + off), (float4*)(t->s1 + off), (float4*)out, n4, aa);
-            }
-            int64_t done = n4 * 4;
-            if (done < n) {
-                int blocks = launch_grid(n - done, 256, 1 << 20);
-                TN_LAUNCH(k_dense_adam_s, dim3(blocks), dim3(256), st, g + done, t->w + off + done, t->s0 + off + done, t->s1 + off + done, out ? out + done : nullptr, n - done, aa);
-            }
-        } else {
-            bool vec = (off % 4 == 0) && aligned16(g) && (!out || aligned16(out));
-            int64_t n4 = vec ? n / 4 : 0;
-            if (n4 > 0) {
-                int blocks = launch_grid(n4, 256, 1 << 20);
-                TN_LAUNCH(k_dense_adagrad_v4, dim3(blocks), dim3(256), st, (const float4*)g, (float4*)(t->w + off), (float4*)(t->s0 + off), (float4*)(t->s1 + off), (float4*)(t->s2 + off), (float4*)out, n4, ga);
-            }
-            int64_t done = n4 * 4;
-            if (done < n) {
-                int blocks = launch_grid(n - done, 256, 1 << 20);
-                TN_LAUNCH(k_dense_adagrad_s, dim3(blocks), dim3(256), st, g + done, t->w + off + done, t->s0 + off + done, t->s1 + off + done, t->s2 + off + done, out ? out + done : nullptr, n - done, ga);
-            }
-        }
+        seg.first_block[k] = blocks;
+        seg.off[k] = (uint32_t)(lo - t->begin);
+        seg.len[k] = (uint32_t)(hi - lo);
+        seg.g[k] = grads[i] + skip;
+        seg.out[k] = (vars && vars[i]) ? vars[i] + skip : nullptr;
+        blocks += (seg.len[k] + SEGMENT_BLOCK - 1) / SEGMENT_BLOCK;
+        if (++k == SEGMENTS) launch();
     }
+    launch();
     TN_HIP(hipGetLastError());
     return TN_OK;
 }
