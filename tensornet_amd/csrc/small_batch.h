@@ -498,7 +498,7 @@ inline size_t small_apply_big_lds(int D) { return 4 * small_apply_wave_lds(D); }
 // Nothing is reported to the host but that this kernel runs, which tells it that the comparison of the signs,
 // launched before, is complete: on the plan of the last pull every sign has its row, and the host has compared
 // the slots' distinct counts with the rows of the gradient matrices itself.
-template <int KIND, int LPG>
+template <int KIND, int LPG, bool ANY>
 __global__ __launch_bounds__(256) void k_small_apply(Store s, OptDev o, PushSrc src, int N, DevStatus* status,
                                                      const uint32_t* __restrict__ grp_row,
                                                      const uint32_t* __restrict__ grp_off,
@@ -546,7 +546,7 @@ __global__ __launch_bounds__(256) void k_small_apply(Store s, OptDev o, PushSrc 
         if (row > s.cap) continue;  // NO_ROW, or no row number at all: never address the table with it
         const uint32_t k = grp_cnt[g];
         if (is_big(k, big_k)) continue;
-        apply_group_vec<KIND, LPG, 4>(s, o, src, status, row, k, list + grp_off[g], nullptr, sub, lane0, c1, c2);
+        apply_group_vec<KIND, LPG, ANY, 4>(s, o, src, status, row, k, list + grp_off[g], nullptr, sub, lane0, c1, c2);
     }
 }
 

@@ -1452,10 +1452,52 @@ __device__ __forceinline__ void ftrl_elem(const OptDev& o, float g, float& w, fl
     }
 }
 
+// The update kernels' view of a row: lane `sub` of the LPG lanes that share it owns elements [4 sub, 4 sub + 4).  With
+// ANY the row has any length up to 4 LPG and stands at any 4-byte boundary -- rows of 1, 6 or 10 elements, gradients
+// of rows with the two cvm columns (10 floats apart for 8 elements): a lane whose part is whole moves it with one
+// unaligned 16-byte access, which gfx950 takes, the last one element by element, lanes beyond the row hold zeros
+// (which change neither a sum of squares nor anything that is stored).  One thread per sign, as such rows had before,
+// cost 78 us for 282 k lookups of 8 + 2 elements (k_apply_scalar); this way it is 28 (k_apply_single 10, k_apply_vec 18).
+typedef float any_float4 __attribute__((ext_vector_type(4), aligned(4)));
+template <bool ANY>
+__device__ __forceinline__ float4 row_part(const float* p, int sub, int D) {
+    if (!ANY) return reinterpret_cast<const float4*>(p)[sub];
+    const int left = D - 4 * sub;
+    p += 4 * sub;
+    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (left >= 4) {
+        const any_float4 q = *reinterpret_cast<const any_float4*>(p);
+        v = make_float4(q.x, q.y, q.z, q.w);
+    } else if (left > 0) {
+        v.x = p[0];
+        if (left > 1) v.y = p[1];
+        if (left > 2) v.z = p[2];
+    }
+    return v;
+}
+template <bool ANY>
+__device__ __forceinline__ void put_row_part(float* p, int sub, int D, float4 v) {
+    if (!ANY) {
+        reinterpret_cast<float4*>(p)[sub] = v;
+        return;
+    }
+    const int left = D - 4 * sub;
+    p += 4 * sub;
+    if (left >= 4) {
+        any_float4 q;
+        q.x = v.x, q.y = v.y, q.z = v.z, q.w = v.w;
+        *reinterpret_cast<any_float4*>(p) = q;
+    } else if (left > 0) {
+        p[0] = v.x;
+        if (left > 1) p[1] = v.y;
+        if (left > 2) p[2] = v.z;
+    }
+}
+
 // Most signs occur in one slot only: one record, no ordering problem, no
 // loop.  LPG lanes update the row of one such sign; its member entry sits at
 // the place of its group number.
-template <int KIND, int LPG>
+template <int KIND, int LPG, bool ANY>
 __global__ __launch_bounds__(256) void k_apply_single(Store s, OptDev o, PushSrc src, DevStatus* status,
                                                       const uint32_t* __restrict__ grp_row,
                                                       const Member* __restrict__ list) {
@@ -1478,8 +1520,8 @@ __global__ __launch_bounds__(256) void k_apply_single(Store s, OptDev o, PushSrc
         }
         float* wp = s.w + (uint64_t)row * s.wstride;
         float* sp = s.st + (uint64_t)row * s.sstride;
-        const float4 gr = reinterpret_cast<const float4*>(gp)[sub];
-        float4 w = reinterpret_cast<float4*>(wp)[sub];
+        const float4 gr = row_part<ANY>(gp, sub, D);
+        float4 w = row_part<ANY>(wp, sub, D);
         if (KIND == OPT_ADAGRAD) {
             const float4 h = *reinterpret_cast<const float4*>(sp);
             const float p0 = gr.x * gr.x, p1 = gr.y * gr.y, p2 = gr.z * gr.z, p3 = gr.w * gr.w;
@@ -1498,7 +1540,7 @@ __global__ __launch_bounds__(256) void k_apply_single(Store s, OptDev o, PushSrc
             w.y -= o.lr * gr.y / den;
             w.z -= o.lr * gr.z / den;
             w.w -= o.lr * gr.w / den;
-            reinterpret_cast<float4*>(wp)[sub] = w;
+            put_row_part<ANY>(wp, sub, D, w);
             if (sub == 0) {
                 const float show = h.y + (float)bshow, click = h.z + (float)bclick;
                 *reinterpret_cast<float4*>(sp) = make_float4(g2sum, show, click, 0.f);  // no_show_days = 0
@@ -1508,8 +1550,8 @@ __global__ __launch_bounds__(256) void k_apply_single(Store s, OptDev o, PushSrc
                 }
             }
         } else {
-            float4 a = reinterpret_cast<float4*>(sp)[sub];
-            float4 b = reinterpret_cast<float4*>(sp + D)[sub];
+            float4 a = row_part<ANY>(sp, sub, D);
+            float4 b = row_part<ANY>(sp + D, sub, D);
             if (KIND == OPT_ADAM) {
                 adam_elem(o, c1, c2, gr.x, w.x, a.x, b.x);
                 adam_elem(o, c1, c2, gr.y, w.y, a.y, b.y);
@@ -1521,9 +1563,9 @@ __global__ __launch_bounds__(256) void k_apply_single(Store s, OptDev o, PushSrc
                 ftrl_elem(o, gr.z, w.z, a.z, b.z);
                 ftrl_elem(o, gr.w, w.w, a.w, b.w);
             }
-            reinterpret_cast<float4*>(wp)[sub] = w;
-            reinterpret_cast<float4*>(sp)[sub] = a;
-            reinterpret_cast<float4*>(sp + D)[sub] = b;
+            put_row_part<ANY>(wp, sub, D, w);
+            put_row_part<ANY>(sp, sub, D, a);
+            put_row_part<ANY>(sp + D, sub, D, b);
             if (sub == 0) sp[2 * D + 1] = __int_as_float(__float_as_int(sp[2 * D + 1]) + bshow);
         }
     }
@@ -1539,14 +1581,14 @@ __global__ __launch_bounds__(256) void k_apply_single(Store s, OptDev o, PushSrc
 // of the next AHEAD and the member entries of the AHEAD after those in flight meanwhile: a chain of k records
 // costs k / AHEAD round trips instead of 2 k, which is what a small batch, whose kernels are as long as their
 // longest chain, is after.
-template <int KIND, int LPG, int AHEAD = 1>
+template <int KIND, int LPG, bool ANY, int AHEAD = 1>
 __device__ __forceinline__ void apply_group_vec(const Store& s, const OptDev& o, const PushSrc& src, DevStatus* status,
                                                 uint32_t row, uint32_t k, const Member* mem, const float* const* ga,
                                                 int sub, int lane0, float c1, float c2) {
     const int D = s.D;
     float* wp = s.w + (uint64_t)row * s.wstride;
     float* sp = s.st + (uint64_t)row * s.sstride;
-    float4 w = reinterpret_cast<float4*>(wp)[sub];
+    float4 w = row_part<ANY>(wp, sub, D);
     float4 a, b;          // Adam m,v / Ftrl z,n
     float g2sum = 0.f, show = 0.f, click = 0.f;
     int delta_show = 0;
@@ -1556,8 +1598,8 @@ __device__ __forceinline__ void apply_group_vec(const Store& s, const OptDev& o,
         show = h.y;
         click = h.z;
     } else {
-        a = reinterpret_cast<float4*>(sp)[sub];
-        b = reinterpret_cast<float4*>(sp + D)[sub];
+        a = row_part<ANY>(sp, sub, D);
+        b = row_part<ANY>(sp + D, sub, D);
         delta_show = __float_as_int(sp[2 * D + 1]);
     }
     bool any = false;
@@ -1606,14 +1648,14 @@ __device__ __forceinline__ void apply_group_vec(const Store& s, const OptDev& o,
         int nshow = 0, nclick = 0;
         bool nok = record_at(src, mem, ga, 0, gp, nshow, nclick);
         float4 gnext = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (nok) gnext = reinterpret_cast<const float4*>(gp)[sub];
+        if (nok) gnext = row_part<ANY>(gp, sub, D);
         for (uint32_t j = 0; j < k; j++) {
             const float4 gr = gnext;
             const int bshow = nshow, bclick = nclick;
             const bool ok = nok;
             if (j + 1 < k) {
                 nok = record_at(src, mem, ga, j + 1, gp, nshow, nclick);
-                if (nok) gnext = reinterpret_cast<const float4*>(gp)[sub];
+                if (nok) gnext = row_part<ANY>(gp, sub, D);
             }
             if (!ok) {
                 no_gradient();
@@ -1644,7 +1686,7 @@ __device__ __forceinline__ void apply_group_vec(const Store& s, const OptDev& o,
                 } else {
                     ok[q] = src_record(src, m[q], gp, sh[q], ck[q]) && first + q < k;
                 }
-                g[q] = reinterpret_cast<const float4*>(ok[q] ? gp : wp)[sub];
+                g[q] = row_part<ANY>(ok[q] ? gp : wp, sub, D);
             }
         };
 #pragma unroll
@@ -1742,7 +1784,7 @@ __device__ __forceinline__ void apply_group_vec(const Store& s, const OptDev& o,
         }
     }
     if (!any) return;
-    reinterpret_cast<float4*>(wp)[sub] = w;
+    put_row_part<ANY>(wp, sub, D, w);
     if (KIND == OPT_ADAGRAD) {
         if (sub == 0) {
             *reinterpret_cast<float4*>(sp) = make_float4(g2sum, show, click, 0.f);  // no_show_days = 0
@@ -1752,13 +1794,13 @@ __device__ __forceinline__ void apply_group_vec(const Store& s, const OptDev& o,
             }
         }
     } else {
-        reinterpret_cast<float4*>(sp)[sub] = a;
-        reinterpret_cast<float4*>(sp + D)[sub] = b;
+        put_row_part<ANY>(sp, sub, D, a);
+        put_row_part<ANY>(sp + D, sub, D, b);
         if (sub == 0) sp[2 * D + 1] = __int_as_float(delta_show);
     }
 }
 
-template <int KIND, int LPG>
+template <int KIND, int LPG, bool ANY>
 __global__ __launch_bounds__(256) void k_apply_vec(Store s, OptDev o, PushSrc src, DevStatus* status,
                                                    const uint32_t* __restrict__ grp_row,
                                                    const uint32_t* __restrict__ grp_off,
@@ -1778,8 +1820,8 @@ __global__ __launch_bounds__(256) void k_apply_vec(Store s, OptDev o, PushSrc sr
         if (row > s.cap) continue;  // NO_ROW (unknown sign: flagged by the probe), or no row number at all
         const uint32_t k = grp_cnt[g];
         if (is_big(k, big_k)) continue;
-        apply_group_vec<KIND, LPG>(s, o, src, status, row, k, list + grp_off[g],
-                                                 gaddr ? gaddr + grp_off[g] : nullptr, sub, lane0, c1, c2);
+        apply_group_vec<KIND, LPG, ANY>(s, o, src, status, row, k, list + grp_off[g],
+                                        gaddr ? gaddr + grp_off[g] : nullptr, sub, lane0, c1, c2);
     }
 }
 
@@ -2178,7 +2220,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6, 8))) void
 }
 
 
-// Any dim / alignment: one thread per distinct sign, scalar loops.
+// Rows beyond what a wavefront half holds (more than 128 elements): one thread per distinct sign, scalar loops.
 template <int KIND>
 __global__ __launch_bounds__(256) void k_apply_scalar(Store s, OptDev o, PushSrc src, DevStatus* status,
                                                       const uint32_t* __restrict__ grp_row,

@@ -908,6 +908,20 @@ int launch_build_plan(SparseTable* t, const Plan& p, const Scratch& w, int N, ui
     return TN_OK;
 }
 
+// How the update kernels share a row out: `lanes` lanes, four elements each (0: the row is too long for that).
+// any: the rows do not fill the lanes, or stand at other than 16-byte boundaries (row_part<true>).
+struct RowShare {
+    int lanes;
+    bool any;
+};
+RowShare row_share(const Store& s, bool aligned) {
+    RowShare r{1, !aligned || s.D % 4 != 0};
+    while (4 * r.lanes < s.D) r.lanes *= 2;
+    if (4 * r.lanes != s.D) r.any = true;
+    if (r.lanes > 32) r.lanes = 0;
+    return r;
+}
+
 // The three kernels touch disjoint rows.  k_apply_single saturates the memory system (it runs
 // at the device's rate for random row updates); k_apply_big and k_apply_vec are bound by
 // dependent chains and instruction issue, so they run one after the other beside it.  The pair is
@@ -918,13 +932,13 @@ int launch_build_plan(SparseTable* t, const Plan& p, const Scratch& w, int N, ui
 // detach: none of them on the caller's stream, which does not wait for them either -- k_apply_single on the
 // auxiliary stream; the caller of this function records their end (see SparseTable::upd_ev).
 template <int KIND>
-int launch_apply_kind(SparseTable* t, int lpg, const Store& s, const OptDev& o, const PushSrc& src, DevStatus* ds,
+int launch_apply_kind(SparseTable* t, RowShare share, const Store& s, const OptDev& o, const PushSrc& src, DevStatus* ds,
                       const Plan& p, int64_t n_upper, hipStream_t st, bool addr_ready, uint32_t big_k, bool detach,
                       bool big_desc) {
     const uint32_t ids_cap = (uint32_t)n_upper;
     const bool with_big = big_k != 0xFFFFFFFFu;
     const float* const* gaddr = (with_big && !src.infos && !src.flat) ? p.gaddr : nullptr;
-    detach = detach && !t->one_stream && lpg != 0;
+    detach = detach && !t->one_stream && share.lanes != 0;
     t->detached_now = detach;
     const bool forked = (with_big || detach) && !t->one_stream;
     // op-level gradients: their addresses for the records of the groups with several records, once, in a
@@ -956,15 +970,22 @@ int launch_apply_kind(SparseTable* t, int lpg, const Store& s, const OptDev& o, 
                           p.big_list, p.grp_row, p.grp_off, p.grp_cnt, p.list, gfloats, gaddr);
 #undef TN_LAUNCH_BIG_ADAGRAD
     }
-#define TN_LAUNCH_VEC(LPG)                                                                                        \
+#define TN_LAUNCH_VEC_ANY(LPG, ANY)                                                                                \
     do {                                                                                                          \
-        TN_LAUNCH((k_apply_single<KIND, LPG>), dim3(launch_grid(n_upper * LPG, 256, GRID_CAP * 4)), dim3(256),    \
+        TN_LAUNCH((k_apply_single<KIND, LPG, ANY>), dim3(launch_grid(n_upper * LPG, 256, GRID_CAP * 4)), dim3(256), \
                   detach ? t->aux : (forked ? t->side : st), s, o, src, ds, p.grp_row, p.list);                   \
-        TN_LAUNCH((k_apply_vec<KIND, LPG>), dim3(launch_grid(n_upper * LPG / 2, 256, GRID_CAP * 4)), dim3(256),    \
+        TN_LAUNCH((k_apply_vec<KIND, LPG, ANY>), dim3(launch_grid(n_upper * LPG / 2, 256, GRID_CAP * 4)), dim3(256), \
                   detach ? t->side : st, s, o, src, ds, p.grp_row, p.grp_off, p.grp_cnt, p.list, big_k, ids_cap,  \
                   gaddr);                                                                                         \
     } while (0)
-    switch (lpg) {
+#define TN_LAUNCH_VEC(LPG)                        \
+    do {                                          \
+        if (share.any)                            \
+            TN_LAUNCH_VEC_ANY(LPG, true);         \
+        else                                      \
+            TN_LAUNCH_VEC_ANY(LPG, false);        \
+    } while (0)
+    switch (share.lanes) {
         case 1: TN_LAUNCH_VEC(1); break;
         case 2: TN_LAUNCH_VEC(2); break;
         case 4: TN_LAUNCH_VEC(4); break;
@@ -976,18 +997,12 @@ int launch_apply_kind(SparseTable* t, int lpg, const Store& s, const OptDev& o, 
                       p.grp_row, p.grp_off, p.grp_cnt, p.list, big_k, ids_cap);
     }
 #undef TN_LAUNCH_VEC
+#undef TN_LAUNCH_VEC_ANY
     if (forked && !detach) {
         TN_HIP(hipEventRecord(t->join_ev, t->side));
         TN_HIP(hipStreamWaitEvent(st, t->join_ev, 0));
     }
     return TN_OK;
-}
-
-// Lanes that share a row in the update kernels (a float4 each), 0 if the rows cannot be handled that way.
-int lanes_per_group(const Store& s, bool vec_ok) {
-    if (!vec_ok || s.D % 4 != 0) return 0;
-    const int q = s.D / 4;
-    return (q >= 1 && q <= 32 && (q & (q - 1)) == 0) ? q : 0;
 }
 
 // Applies the grouped records; n_upper bounds the number of records.
@@ -998,12 +1013,12 @@ int launch_apply(SparseTable* t, const Plan& p, const PushSrc& src, DevStatus* d
                  hipStream_t st, bool addr_ready = false, uint32_t big_k = 0, bool detach = false, bool big_desc = false) {
     const Store& s = t->store;
     const OptDev o = make_optdev(t);
-    const int lpg = lanes_per_group(s, vec_ok);
+    const RowShare share = row_share(s, vec_ok);
     if (big_k == 0) big_k = big_threshold(s);
     switch (o.kind) {
-        case OPT_ADAGRAD: return launch_apply_kind<OPT_ADAGRAD>(t, lpg, s, o, src, ds, p, n_upper, st, addr_ready, big_k, detach, big_desc);
-        case OPT_ADAM: return launch_apply_kind<OPT_ADAM>(t, lpg, s, o, src, ds, p, n_upper, st, addr_ready, big_k, detach, big_desc);
-        default: return launch_apply_kind<OPT_FTRL>(t, lpg, s, o, src, ds, p, n_upper, st, addr_ready, big_k, detach, big_desc);
+        case OPT_ADAGRAD: return launch_apply_kind<OPT_ADAGRAD>(t, share, s, o, src, ds, p, n_upper, st, addr_ready, big_k, detach, big_desc);
+        case OPT_ADAM: return launch_apply_kind<OPT_ADAM>(t, share, s, o, src, ds, p, n_upper, st, addr_ready, big_k, detach, big_desc);
+        default: return launch_apply_kind<OPT_FTRL>(t, share, s, o, src, ds, p, n_upper, st, addr_ready, big_k, detach, big_desc);
     }
 }
 
@@ -1012,7 +1027,7 @@ int launch_apply(SparseTable* t, const Plan& p, const PushSrc& src, DevStatus* d
 // after this one, k_apply_big made 4096 x 26 slots, Adam, 0.080 ms per pull + push; beside it on the table's side
 // stream 0.113 ms: the events that fork and join the streams cost more than the overlap wins).
 template <int KIND>
-int launch_small_apply_kind(SparseTable* t, int lpg, int N, const OptDev& o, const PushSrc& src, DevStatus* ds,
+int launch_small_apply_kind(SparseTable* t, RowShare share, int N, const OptDev& o, const PushSrc& src, DevStatus* ds,
                             const Plan& p, int64_t n_upper, hipStream_t st, uint32_t* host_seq, uint32_t seq) {
     const Store& s = t->store;
     const uint32_t big_k = t->plan_big_k;
@@ -1020,15 +1035,22 @@ int launch_small_apply_kind(SparseTable* t, int lpg, int N, const OptDev& o, con
     // (a wavefront per sign with big_k records or more, four to a workgroup, 512 workgroups at most)
     const int big_blocks = with_big ? launch_grid((n_upper / big_k + 1 + 3) / 4, 1, 512) : 0;
     const size_t lds = with_big ? small_apply_big_lds(s.D) : 0;
-#define TN_LAUNCH_SMALL(LPG)                                                                                          \
+#define TN_LAUNCH_SMALL_ANY(LPG, ANY)                                                                                 \
     do {                                                                                                              \
         const int group_blocks = launch_grid(n_upper * LPG, 256, GRID_CAP * 4);                                       \
-        TN_LAUNCH_LDS((k_small_apply<KIND, LPG>), dim3(group_blocks + big_blocks), dim3(256), lds, st, s, o, src, N, ds, \
-                      p.grp_row, p.grp_off, p.grp_cnt, p.list, big_k, (uint32_t)n_upper, host_seq, seq,              \
+        TN_LAUNCH_LDS((k_small_apply<KIND, LPG, ANY>), dim3(group_blocks + big_blocks), dim3(256), lds, st, s, o, src, N, \
+                      ds, p.grp_row, p.grp_off, p.grp_cnt, p.list, big_k, (uint32_t)n_upper, host_seq, seq,           \
                       (uint32_t)big_blocks, p.big_list, big_gbuf_floats(s.D), (uint32_t)small_apply_wave_lds(s.D),    \
-                      (uint32_t)align_up(big_lds_bytes(s.D), 8));                                                    \
+                      (uint32_t)align_up(big_lds_bytes(s.D), 8));                                                     \
     } while (0)
-    switch (lpg) {
+#define TN_LAUNCH_SMALL(LPG)                  \
+    do {                                      \
+        if (share.any)                        \
+            TN_LAUNCH_SMALL_ANY(LPG, true);   \
+        else                                  \
+            TN_LAUNCH_SMALL_ANY(LPG, false);  \
+    } while (0)
+    switch (share.lanes) {
         case 1: TN_LAUNCH_SMALL(1); break;
         case 2: TN_LAUNCH_SMALL(2); break;
         case 4: TN_LAUNCH_SMALL(4); break;
@@ -1037,16 +1059,17 @@ int launch_small_apply_kind(SparseTable* t, int lpg, int N, const OptDev& o, con
         default: TN_LAUNCH_SMALL(32); break;
     }
 #undef TN_LAUNCH_SMALL
+#undef TN_LAUNCH_SMALL_ANY
     return TN_OK;
 }
 
-int launch_small_apply(SparseTable* t, int lpg, int N, const PushSrc& src, DevStatus* ds, const Plan& p, int64_t n_upper,
+int launch_small_apply(SparseTable* t, RowShare share, int N, const PushSrc& src, DevStatus* ds, const Plan& p, int64_t n_upper,
                        hipStream_t st, uint32_t* host_seq, uint32_t seq) {
     const OptDev o = make_optdev(t);
     switch (o.kind) {
-        case OPT_ADAGRAD: return launch_small_apply_kind<OPT_ADAGRAD>(t, lpg, N, o, src, ds, p, n_upper, st, host_seq, seq);
-        case OPT_ADAM: return launch_small_apply_kind<OPT_ADAM>(t, lpg, N, o, src, ds, p, n_upper, st, host_seq, seq);
-        default: return launch_small_apply_kind<OPT_FTRL>(t, lpg, N, o, src, ds, p, n_upper, st, host_seq, seq);
+        case OPT_ADAGRAD: return launch_small_apply_kind<OPT_ADAGRAD>(t, share, N, o, src, ds, p, n_upper, st, host_seq, seq);
+        case OPT_ADAM: return launch_small_apply_kind<OPT_ADAM>(t, share, N, o, src, ds, p, n_upper, st, host_seq, seq);
+        default: return launch_small_apply_kind<OPT_FTRL>(t, share, N, o, src, ds, p, n_upper, st, host_seq, seq);
     }
 }
 
@@ -2068,8 +2091,8 @@ int push_op_impl(uint32_t table_handle, int N, const int64_t* const* values, con
         src.flat = flat;
         return TN_OK;
     };
-    const int small_lpg = lanes_per_group(t->store, vec && t->store.wstride % 4 == 0);
-    if (reuse && t->plan_small && t->small_path && !pooled && small_lpg != 0 && N <= SMALL_SLOTS) {
+    const RowShare small_share = row_share(t->store, vec && t->store.wstride % 4 == 0);
+    if (reuse && t->plan_small && t->small_path && !pooled && small_share.lanes != 0 && N <= SMALL_SLOTS) {
         // A small batch on the plan of its small pull: slot descriptors, comparison of the signs and click sums by
         // one launch, the updates by one or two more (small_batch.h).  The call's status block is the plan's:
         // nothing of the next call runs beside this one.  The device has nothing to report: every sign of the plan
@@ -2104,7 +2127,7 @@ int push_op_impl(uint32_t table_handle, int N, const int64_t* const* values, con
         // whatever rewrites the plan's)
         PushSrc small_src = op_source(p, grad_dim, true);
         small_src.ubase = p.ubase;
-        TN_TRY(launch_small_apply(t, small_lpg, N, small_src, ds, p, (int64_t)L, st, t->hseq + 1, seq_v));
+        TN_TRY(launch_small_apply(t, small_share, N, small_src, ds, p, (int64_t)L, st, t->hseq + 1, seq_v));
         // what a call on another stream has to wait for: the updates are still running when this call returns
         TN_HIP(hipEventRecord(t->tail_ev, st));
         t->tail_recorded = true;
