@@ -892,22 +892,39 @@ __global__ __launch_bounds__(256) void k_init_new_recs(Store s, OptDev o, uint64
 // (rrow, from k_probe_recs)}; the groups get the rows too.  A group with big_k records or more is listed in
 // big_list and, with {row, first member, records, group}, in big_desc.
 //
-// SLOT_RANKS: a record carries its rank in its slot instead of the position of its first occurrence
-// (the pull of a small batch); its distinct index is the slot's base plus that rank.
-template <bool SLOT_RANKS>
-__global__ __launch_bounds__(EMIT_THREADS) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_group_emit(uint32_t nb2, const uint32_t* __restrict__ cursor2,
-                                                    const GroupRec* __restrict__ recs, const uint2* __restrict__ aux,
-                                                    const uint4* __restrict__ bbase,
-                                                    const uint4* __restrict__ bcounts,
-                                                    const uint8_t* __restrict__ flag8,
-                                                    const uint32_t* __restrict__ wordpre, uint32_t ids_cap,
-                                                    uint32_t big_k, uint64_t* __restrict__ grp_sign,
-                                                    uint32_t* __restrict__ grp_off, uint32_t* __restrict__ grp_cnt,
-                                                    uint32_t* __restrict__ big_list, uint4* __restrict__ big_desc,
-                                                    Member* __restrict__ list, uint2* __restrict__ where_u,
-                                                    const uint32_t* __restrict__ rrow,
-                                                    uint32_t* __restrict__ grp_row, DevStatus* status,
-                                                    const uint32_t* __restrict__ ubase, uint32_t n_slots) {
+template <bool SMALL>
+struct EmitArgs;  // (the small batches' grouping has the same place in a pull and works on what their first pass leaves: small_batch.h)
+template <>
+struct EmitArgs<false> {
+    static constexpr int THREADS = EMIT_THREADS;
+    uint32_t nb2;
+    const uint32_t* cursor2;
+    const GroupRec* recs;
+    const uint2* aux;
+    const uint4* bbase;
+    const uint4* bcounts;
+    const uint8_t* flag8;
+    const uint32_t* wordpre;
+    uint32_t ids_cap, big_k;
+    uint64_t* grp_sign;
+    uint32_t *grp_off, *grp_cnt, *big_list;
+    uint4* big_desc;
+    Member* list;
+    uint2* where_u;
+    const uint32_t* rrow;
+    uint32_t* grp_row;
+    DevStatus* status;
+};
+__device__ __forceinline__ void emit_buckets(uint32_t nb2, const uint32_t* __restrict__ cursor2,
+                                             const GroupRec* __restrict__ recs, const uint2* __restrict__ aux,
+                                             const uint4* __restrict__ bbase, const uint4* __restrict__ bcounts,
+                                             const uint8_t* __restrict__ flag8, const uint32_t* __restrict__ wordpre,
+                                             uint32_t ids_cap, uint32_t big_k, uint64_t* __restrict__ grp_sign,
+                                             uint32_t* __restrict__ grp_off, uint32_t* __restrict__ grp_cnt,
+                                             uint32_t* __restrict__ big_list, uint4* __restrict__ big_desc,
+                                             Member* __restrict__ list, uint2* __restrict__ where_u,
+                                             const uint32_t* __restrict__ rrow, uint32_t* __restrict__ grp_row,
+                                             DevStatus* status) {
     // [0, n1): the groups of one record (group = member); from n1 on: in s_mem the members of the other groups,
     // last group first, in s_sign / s_row those groups themselves, whose offsets and sizes have arrays of their
     // own (such a group has two records at least, so there are n / 2 of them at most).  A member entry is packed
@@ -918,9 +935,6 @@ __global__ __launch_bounds__(EMIT_THREADS) __attribute__((amdgpu_waves_per_eu(8,
     __shared__ uint32_t s_off[GRP_CAP / 2];
     __shared__ uint16_t s_cnt[GRP_CAP / 2];  // at most GRP_SLOTS records per group
     __shared__ uint4 s_part[EMIT_THREADS / 64];
-    __shared__ uint32_t s_ub[SLOT_RANKS ? GRP_SLOTS + 1 : 1];  // the slots' bases (a small batch: one round trip less per record)
-    if (SLOT_RANKS)
-        for (uint32_t i = threadIdx.x; i <= n_slots && i <= (uint32_t)GRP_SLOTS; i += EMIT_THREADS) s_ub[i] = ubase[i];
     for (uint32_t c = blockIdx.x; c < nb2; c += gridDim.x) {
         const uint32_t n = min(cursor2[c], (uint32_t)GRP_CAP);
         const size_t first = (size_t)c * GRP_CAP;
@@ -931,8 +945,7 @@ __global__ __launch_bounds__(EMIT_THREADS) __attribute__((amdgpu_waves_per_eu(8,
 #pragma unroll
         for (int j = 0; j < EMIT_RECS; j++) {
             const uint32_t i = j * EMIT_THREADS + threadIdx.x;
-            // (a small batch reads the bucket's whole room, wanted or not: the loads do not wait for its count then)
-            if (SLOT_RANKS || i < n) {
+            if (i < n) {
                 rs[j] = recs[first + i];
                 as[j] = aux[first + i];
                 rows[j] = rrow[first + i];
@@ -976,7 +989,7 @@ __global__ __launch_bounds__(EMIT_THREADS) __attribute__((amdgpu_waves_per_eu(8,
 #pragma unroll
         for (int j = 0; j < EMIT_RECS; j++)
             if (j * EMIT_THREADS + threadIdx.x < n)
-                us[j] = SLOT_RANKS ? s_ub[(rs[j].cnt >> 24) & (GRP_SLOTS - 1)] + rs[j].gi : rank_of(flag8, wordpre, rs[j].gi);
+                us[j] = rank_of(flag8, wordpre, rs[j].gi);
 #pragma unroll
         for (int j = 0; j < EMIT_RECS; j++) {
             if (j * EMIT_THREADS + threadIdx.x >= n) continue;
@@ -1039,6 +1052,18 @@ __global__ __launch_bounds__(EMIT_THREADS) __attribute__((amdgpu_waves_per_eu(8,
             grp_row[g] = s_row[n1 + i];
         }
         __syncthreads();
+    }
+}
+
+template <bool SMALL>
+__global__ __launch_bounds__(EmitArgs<SMALL>::THREADS) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_group_emit(
+    EmitArgs<SMALL> a) {
+    if constexpr (SMALL) {
+        extern __shared__ uint32_t emit_lds[];
+        small_emit_bucket(a, emit_lds);
+    } else {
+        emit_buckets(a.nb2, a.cursor2, a.recs, a.aux, a.bbase, a.bcounts, a.flag8, a.wordpre, a.ids_cap, a.big_k, a.grp_sign,
+                     a.grp_off, a.grp_cnt, a.big_list, a.big_desc, a.list, a.where_u, a.rrow, a.grp_row, a.status);
     }
 }
 

@@ -1,22 +1,20 @@
-// Pull and push of a small batch (every slot fits one workgroup's LDS table): the same plan as the
-// path through two levels of buckets leaves, from far fewer launches.  A batch of a few thousand
-// lookups spends its time in the dependent launches of that path (about 3 us each, whatever the
-// kernel does), not in its kernels, so here
+// Pull and push of a small batch (slots of a few thousand lookups at most) in few launches.  A batch of a few
+// thousand lookups spends its time in dependent launches (2 to 3 us each, whatever the kernel does) and in the round
+// trips inside them, so here
 //
-//   pull  k_small_slots          one workgroup per slot: per-slot first-occurrence remap in LDS
-//                                (sparse_table_ops.cc:115-137), lookup-or-insert of every distinct sign
-//                                (sparse_table.cc:52-66), its record handed to its second-level bucket
-//         k_small_group_finish   the first pass of the grouping (what k_group_count does) beside: the slots'
-//                                counts added up, the call's status published to the host (which returns as
-//                                soon as it sees it), rows into the variables (sparse_table_ops.cc:244-265),
-//                                distinct indices made global
-//         k_group_emit<true>     the groups of equal signs over all slots, as ever
-//   push  k_small_verify         slot descriptors in, comparison with the plan's signs, click sums
-//         k_small_apply          every group by one launch (tells the host that the comparison is complete); with
-//                                more than 12 slots the signs with 5 records or more by wavefronts of their own in it
+//   pull  k_small_slots          per slot and share of its signs: first occurrences in LDS (sparse_table_ops.cc:115-137),
+//                                lookup-or-insert of every distinct sign (sparse_table.cc:52-66), its record filed by
+//                                bucket; every workgroup reports to the host, which returns when it has them all
+//         k_small_group_finish   ranks of the first occurrences -> mapped ids, rows into the variables
+//                                (sparse_table_ops.cc:244-265)
+//         k_group_emit<true>     per bucket: the groups of equal signs over all slots, their records in slot order
+//   push  k_small_verify         comparison with the plan's signs, click sums
+//         k_small_pool           (pooled gradients) the gradient of every distinct sign from those of its examples
+//         k_small_apply          per bucket: every sign's records in order (tells the host that the comparison is complete)
 //
-// Workgroups of one launch never wait for each other, and none needs another's results: what needs them runs
-// in the next launch.
+// Workgroups of one launch never wait for each other, and none needs another's results: what needs them runs in the
+// next launch.  The host waits for the first launch of a pull and the first of a push only; the launches behind those
+// run while it prepares the next call.
 #ifndef TN_SMALL_BATCH_H_
 #define TN_SMALL_BATCH_H_
 
@@ -24,460 +22,465 @@
 
 namespace tn {
 
-constexpr int SMALL_THREADS = 1024;
-constexpr int SMALL_ITEMS = 4;                               // lookups per thread of k_small_slots
-constexpr int SMALL_SLOT_MAX = SMALL_THREADS * SMALL_ITEMS;  // lookups of a slot at most
-constexpr int SMALL_SLOTS = GRP_SLOTS;                       // slots at most (the grouping's slot masks)
-constexpr int SMALL_NB2_MAX = 512;                           // second-level buckets at most
-constexpr int SMALL_PARTS_MAX = 8;                           // workgroups of k_small_slots per slot at most
-constexpr int SMALL_SLOT_WORKGROUPS = 256;                   // ... and for all slots together
-constexpr int SMALL_TILE = 1024;                             // lookups per workgroup of k_small_verify
+constexpr int SMALL_SLOT_MAX = 4096;         // lookups of a slot at most
+constexpr int SMALL_SLOT_BITS = 13;          // a position in a slot, its rank, its occurrences fit in 13, 13 and 14 bits
+constexpr int SMALL_SLOTS = 512;             // slots at most
+constexpr int SMALL_PARTS_MAX = 16;          // workgroups of k_small_slots per slot at most
+constexpr int SMALL_SEGMENTS = 256;          // ... and for all slots together where a slot has more than one
+constexpr int SMALL_WORKGROUPS = SMALL_SLOTS > SMALL_SEGMENTS ? SMALL_SLOTS : SMALL_SEGMENTS;  // of k_small_slots at most
+constexpr int SMALL_PART_LOOKUPS = 128;      // lookups of a slot per workgroup aimed at
+constexpr int SMALL_BUCKET_RECORDS = 64;     // records per bucket aimed at (if every lookup were distinct)
+constexpr int SMALL_BUCKETS_MAX = 2048;
+constexpr int SMALL_THREADS = 512;           // k_small_slots, k_small_group_finish
+constexpr int SMALL_ITEMS = SMALL_SLOT_MAX / SMALL_THREADS;
+constexpr int SMALL_WORDS = SMALL_SLOT_MAX / 64;  // 64-lookup words of a slot
+constexpr int SMALL_NEW = 512;               // rows a workgroup of k_small_slots lists to fill them with all its threads
+constexpr int EMIT_SMALL_THREADS = 256;
+constexpr int SMALL_TILE = 1024;             // lookups per workgroup of k_small_verify
+static_assert(SMALL_SLOT_MAX < (1 << SMALL_SLOT_BITS), "positions fit");
 
-// What a workgroup of k_small_slots leaves for the launch after it: the slot's distinct signs (the same in
-// every workgroup of the slot), the rows it inserted and the error flags it raised.
-struct SlotOut {
-    uint32_t n_unique, n_new, err, pad;
+// How a small batch is laid out: worked out by the pull, kept with its plan.
+struct SmallShape {
+    int N;
+    uint32_t L, max_len;
+    uint32_t parts;    // workgroups of k_small_slots per slot, each with a share of the signs (by hash range)
+    uint32_t nbp;      // buckets per part: parts * nbp buckets in all, a bucket's signs all lie in one part
+    uint32_t words;    // 64-lookup words of the longest slot
+    uint32_t cap;      // room of a bucket, in records
+    __host__ __device__ uint32_t buckets() const { return parts * nbp; }
 };
 
-// Persistent device state of the small path (zero when allocated).  A call uses one of the two sets of
-// bucket cursors and clears the other for the call after it.
-struct SmallState {
-    uint32_t cursor2[2][SMALL_NB2_MAX];
-    SlotOut slot_out[SMALL_SLOT_WORKGROUPS];  // one per workgroup of k_small_slots
+// The plan of a small batch.  Lookups are numbered through the slots (gi); a distinct sign of a slot is known by its
+// first lookup.
+struct SmallPlan {
+    SlotDesc* descs;       // the slots' tensors (pull)
+    SlotDesc* push_descs;  // ... (push)
+    uint64_t* vals_copy;   // sign of every lookup
+    uint16_t* first_of;    // position in its slot of the first lookup with the same sign
+    uint32_t* row_at;      // first lookups: table row of the sign
+    uint16_t* rank_at;     // first lookups: rank among the slot's first lookups
+    int32_t* click_at;     // first lookups: sum of the labels (a push adds them, the updates take them back to zero)
+    uint64_t* bits;        // [slot][part][words]: first lookups found by the part's workgroup
+    uint2* recs;           // records {row, position | occurrences << 13} of slot s, part p from parts * lbase(s) + p * len(s) on, by bucket
+    uint16_t* boff;        // [slot][part][nbp + 1]: where the buckets start in them
+    uint4* head;           // per bucket {signs with one record, with a few, with many, records of the latter two}
+    uint2* group;          // per bucket, `cap` each: {row, first record | records << 16}; those with many records from the end on
+    uint4* member;         // per bucket, `cap` each: records {gi, rank | slot << 16, occurrences, 0}, those of a sign in slot order
+    uint32_t* bad;         // != 0: a bucket did not fit, a push has to analyse the batch itself
 };
-
-// Bytes of dynamic LDS of k_small_slots for a table of `entries` entries and nb2 second-level buckets.
-inline size_t small_slots_lds(uint32_t entries, uint32_t nb2) {
-    return ((size_t)entries + 1) * 16 + (size_t)nb2 * sizeof(uint32_t);
-}
 
 __device__ __forceinline__ void host_store(uint32_t* p, uint32_t v) {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-// First launch of a small pull (see the head of the file).  host_descs: the slot descriptors in the host's pinned
-// staging buffer; descs, lbase: where they go in device memory, for the launches after this one.  entries: the
-// size of the workgroup's LDS table, a power of two and at least twice the longest slot.  prow[first lookup of
-// the slot + r]: table row of the slot's distinct sign of rank r.  cursor2 / recs / rrow: the second-level
-// buckets, as k_lds_dedup<true> and k_probe_recs fill them, but a record carries its rank in its slot (gi).
-__global__ __launch_bounds__(SMALL_THREADS) void k_small_slots(
-    const SlotDesc* host_descs, SlotDesc* descs, uint32_t* lbase, int N, uint32_t L, uint32_t entries,
-    Store s, OptDev o, uint64_t seed, uint64_t* __restrict__ vals_copy, uint32_t* __restrict__ u_of_gi,
-    uint32_t* __restrict__ prow, uint32_t nb2, uint32_t* cursor2, uint32_t* cursor2_next, GroupRec* __restrict__ recs,
-    uint32_t* __restrict__ rrow, SmallState* state, uint32_t parts) {
+// What a workgroup of k_small_slots tells the host, in one word: its distinct signs, the rows it inserted, whether the
+// table is full, and the number of the call, which says that the word is this call's.
+constexpr int SMALL_REPORT_BITS = 14;
+__host__ __device__ inline uint64_t small_report(uint32_t n_first, uint32_t n_new, bool full, uint32_t seq) {
+    return (uint64_t)n_first | ((uint64_t)n_new << SMALL_REPORT_BITS) | ((uint64_t)(full ? 1 : 0) << (2 * SMALL_REPORT_BITS)) |
+           ((uint64_t)seq << 32);
+}
+
+// Entries of the LDS table of k_small_slots: room for a slot of distinct signs that all fall into one part, and two
+// per lookup expected.
+inline uint32_t small_entries(uint32_t max_len, uint32_t parts) {
+    const uint32_t expected = 2 * ((max_len + parts - 1) / parts) + 64;
+    return expected > max_len + 64 ? expected : max_len + 64;
+}
+inline size_t small_slots_lds(uint32_t entries, uint32_t max_len, uint32_t nbp) {
+    // keys and words (entry `entries`: the sign EMPTY_KEY), bucket counters, list of the entries in use
+    return ((size_t)entries + 1) * 12 + (size_t)(nbp + 1) * 4 + align_up((size_t)max_len * 2, 8);
+}
+
+// First launch of a small pull: `parts` workgroups per slot.  Each of them reads all signs of the slot and keeps those
+// of its hash range: the shares of a slot need nothing of each other (workgroups that each worked out the whole slot
+// and then took a share of the probes repeated the slot's remap up to eight times).  What bounds it is a chain of
+// round trips -- descriptor, signs, probe, second probe -- and a CU's rate of random 64-byte reads (0.2 per ns), hence
+// many workgroups with about a hundred signs each.
+__global__ __launch_bounds__(SMALL_THREADS) void k_small_slots(SmallShape b, SmallPlan p, const SlotDesc* host_descs,
+                                                               uint32_t entries, Store s, OptDev o, uint64_t seed,
+                                                               DevStatus* status, uint64_t* host_words, uint32_t seq) {
     extern __shared__ unsigned long long smem64[];
-    unsigned long long* keys = smem64;  // entry `entries`: the sign EMPTY_KEY itself
-    uint32_t* minpos = reinterpret_cast<uint32_t*>(keys + entries + 1);
-    uint32_t* cnts = minpos + entries + 1;
-    uint32_t* hist2 = cnts + entries + 1;
+    unsigned long long* keys = smem64;
+    uint32_t* word = reinterpret_cast<uint32_t*>(keys + entries + 1);  // bits 16-31 smallest position, 0-15 occurrences
+    uint32_t* hist = word + entries + 1;                              // [nbp + 1]
+    uint16_t* used = reinterpret_cast<uint16_t*>(hist + b.nbp + 1);   // [max_len]: the entries in use
     __shared__ SlotDesc sd;
+    __shared__ unsigned long long bits[SMALL_WORDS];
     __shared__ uint32_t wsum[SMALL_THREADS / 64];
-    __shared__ uint32_t sh_new, sh_err;
-    // `parts` workgroups per slot: each of them works out the whole remap of the slot (in LDS, the same in all),
-    // then takes every parts-th distinct sign through the table and every parts-th wavefront's lookups to the
-    // outputs.  A CU sustains about 0.2 random 64-byte reads per nanosecond: the 2600 probes of a slot of 4096
-    // lookups keep one CU busy for 13 us (measured with the device's clock around the kernel's phases), while
-    // most of the device has nothing to do.
-    const int sl = blockIdx.x / parts;
-    const uint32_t part = blockIdx.x % parts;
+    __shared__ uint32_t sh_first, sh_new, sh_full;
+    __shared__ uint32_t new_row[SMALL_NEW];
+    __shared__ uint16_t new_ent[SMALL_NEW];
+    const int sl = blockIdx.x / b.parts;
+    const uint32_t part = blockIdx.x % b.parts;
     const uint32_t tid = threadIdx.x;
-    // the slot's descriptor comes straight out of the host's staging buffer (one round trip over the bus,
-    // in flight while the tables are cleared)
-    if (tid < sizeof(SlotDesc) / 4)
-        reinterpret_cast<uint32_t*>(&sd)[tid] = reinterpret_cast<const uint32_t*>(host_descs + sl)[tid];
+    // the slot's descriptor comes straight out of the host's staging buffer (one round trip over the bus, in flight
+    // while the tables are cleared)
+    uint32_t dword = 0;
+    if (tid < sizeof(SlotDesc) / 4) dword = reinterpret_cast<const uint32_t*>(host_descs + sl)[tid];
     for (uint32_t i = tid; i <= entries; i += SMALL_THREADS) {
         keys[i] = EMPTY_KEY;
-        minpos[i] = 0xFFFFFFFFu;
-        cnts[i] = 0;
+        word[i] = 0xFFFF0000u;
     }
-    for (uint32_t i = tid; i < nb2; i += SMALL_THREADS) hist2[i] = 0;
-    if (blockIdx.x == 0)
-        for (uint32_t i = tid; i < (uint32_t)SMALL_NB2_MAX; i += SMALL_THREADS) cursor2_next[i] = 0;
-    if (tid == 0) {
-        sh_new = 0;
-        sh_err = 0;
+    for (uint32_t i = tid; i <= b.nbp; i += SMALL_THREADS) hist[i] = 0;
+    for (uint32_t i = tid; i < SMALL_WORDS; i += SMALL_THREADS) bits[i] = 0;
+    if (tid == 0) sh_first = sh_new = sh_full = 0;
+    if (blockIdx.x == 0) {
+        if (tid < sizeof(DevStatus) / 4) reinterpret_cast<uint32_t*>(status)[tid] = 0;
+        if (tid == 0) *p.bad = 0;
+    }
+    if (tid < sizeof(SlotDesc) / 4) {
+        reinterpret_cast<uint32_t*>(&sd)[tid] = dword;
+        if (part == 0) reinterpret_cast<uint32_t*>(p.descs + sl)[tid] = dword;  // for the launches after this one
     }
     __syncthreads();
-    const SlotDesc d = sd;
-    if (tid == 0 && part == 0) {
-        descs[sl] = d;
-        lbase[sl] = d.lbase;
-        if (sl == N - 1) lbase[N] = L;
-    }
-    const uint32_t n = d.len;
-    // a thread's lookups are consecutive: the ranks of its first occurrences are, too
+    const int64_t* values = sd.values;
+    const uint32_t len = sd.len, lbase = sd.lbase;
     uint64_t sg[SMALL_ITEMS];
-    uint32_t h[SMALL_ITEMS];
-    const uint32_t p0 = tid * SMALL_ITEMS;
-#pragma unroll
-    for (int j = 0; j < SMALL_ITEMS; j++) sg[j] = p0 + j < n ? (uint64_t)d.values[p0 + j] : 0;
-    const int lane = (int)(tid & 63);
 #pragma unroll
     for (int j = 0; j < SMALL_ITEMS; j++) {
-        h[j] = entries;
-        const bool valid = p0 + j < n;
-        const uint64_t sign = sg[j];
-        // A frequent sign fills whole wavefronts: the lanes that hold the same sign as the first valid lane let
-        // that lane (the lowest position among them) enter it with their number, instead of queueing up on
-        // one LDS address, and take its entry from it.
-        const unsigned long long vmask = __ballot(valid);
-        if (vmask == 0) continue;
-        const int leader = __ffsll((long long)vmask) - 1;
-        const uint64_t lead_sign = ((uint64_t)(uint32_t)__shfl((int)(sign >> 32), leader) << 32) |
-                                   (uint32_t)__shfl((int)(uint32_t)sign, leader);
-        const bool same = valid && sign == lead_sign;
-        const unsigned long long smask = __ballot(same);
-        const bool pooled = __popcll(smask) >= 8;
-        const bool follower = pooled && same && lane != leader;
-        if (valid && !follower) {
-            if (sign != EMPTY_KEY) {
-                uint32_t e = (uint32_t)(mix64(sign) >> 7) & (entries - 1);
-                for (;;) {  // entries >= 2 n: a free entry exists
-                    unsigned long long old = keys[e];
-                    if (old == EMPTY_KEY) old = atomicCAS(&keys[e], (unsigned long long)EMPTY_KEY, sign);
-                    if (old == EMPTY_KEY || old == sign) break;
-                    e = (e + 1) & (entries - 1);
-                }
-                h[j] = e;
+        const uint32_t pos = j * SMALL_THREADS + tid;
+        sg[j] = pos < len ? (uint64_t)values[pos] : 0;
+    }
+    // the lookups of my share: entry of the sign, smallest position
+    uint32_t ent[SMALL_ITEMS];
+#pragma unroll
+    for (int j = 0; j < SMALL_ITEMS; j++) {
+        const uint32_t pos = j * SMALL_THREADS + tid;
+        ent[j] = 0xFFFFFFFFu;
+        if (pos >= len) continue;
+        if (part == 0) p.vals_copy[lbase + pos] = sg[j];
+        const uint64_t h = mix64(sg[j]);
+        if (scale32((uint32_t)(h >> 32), b.parts) != part) continue;
+        uint32_t e = entries;
+        if (sg[j] != EMPTY_KEY) {
+            e = scale32((uint32_t)h, entries);
+            for (;;) {  // more entries than lookups: a free one exists
+                unsigned long long old = keys[e];
+                if (old == EMPTY_KEY) old = atomicCAS(&keys[e], (unsigned long long)EMPTY_KEY, sg[j]);
+                if (old == EMPTY_KEY || old == sg[j]) break;
+                e = e + 1 == entries ? 0 : e + 1;
             }
-            atomicMin(&minpos[h[j]], p0 + j);
-            atomicAdd(&cnts[h[j]], pooled && lane == leader ? (uint32_t)__popcll(smask) : 1u);
         }
-        const uint32_t lead_h = (uint32_t)__shfl((int)h[j], leader);
-        if (follower) h[j] = lead_h;
+        atomicMin(&word[e], pos << 16);
+        ent[j] = e;
     }
     __syncthreads();
-    uint32_t firsts = 0;
 #pragma unroll
-    for (int j = 0; j < SMALL_ITEMS; j++)
-        if (p0 + j < n && minpos[h[j]] == p0 + j) firsts |= 1u << j;
-    uint32_t total = 0;
-    uint32_t rank0 = block_excl_scan<uint32_t, SMALL_THREADS / 64>(__popc(firsts), wsum, &total);  // (barriers inside)
-    // the entry of a distinct sign now takes its rank in place of the position (every thread has read the positions)
-    uint32_t mine = 0;  // the distinct signs this workgroup takes through the table
-    {
-        uint32_t r = rank0;
-#pragma unroll
-        for (int j = 0; j < SMALL_ITEMS; j++)
-            if (firsts & (1u << j)) {
-                if (r % parts == part) mine |= 1u << j;
-                minpos[h[j]] = r++;
-            }
+    for (int j = 0; j < SMALL_ITEMS; j++) {
+        if (ent[j] == 0xFFFFFFFFu) continue;
+        const uint32_t pos = j * SMALL_THREADS + tid;
+        const uint32_t f = atomicAdd(&word[ent[j]], 1u) >> 16;
+        p.first_of[lbase + pos] = (uint16_t)f;
+        if (f == pos) {
+            atomicOr(&bits[pos >> 6], 1ull << (pos & 63));
+            used[atomicAdd(&sh_first, 1u)] = (uint16_t)ent[j];
+        }
     }
     __syncthreads();
-    // lookup-or-insert of the distinct signs (optimizer_kernel.h:299-308; the probe sequence of probe_slot).  A
-    // thread's signs go through their sequences side by side: the key groups of all of them are read in one round
-    // trip, the compare-and-swaps of those that found a free slot go out together, and so on round by round --
-    // one after the other, a wavefront would spend a round trip on every sign that needs a second group or
-    // claims a slot, in every one of its four places.  A row this workgroup inserts is listed in LDS (the key
-    // table is dead) and filled further down by all threads: one lane of a wavefront drawing the normal deviates
-    // of a row would hold up the other sixty-three.  The rows are read by the next launch only: another slot's
-    // workgroup may be filling the row of a sign that this one finds claimed.
-    unsigned long long* new_sign = keys;                                   // [n] at most
-    uint32_t* new_row = reinterpret_cast<uint32_t*>(keys + n);            // (the table has 2 n + 1 entries or more)
-    uint32_t rows[SMALL_ITEMS], place[SMALL_ITEMS];
-    uint32_t err = 0, fresh = 0;
-    {
-        uint64_t at[SMALL_ITEMS];
-        uint32_t live = 0;
+    // A thread per distinct sign (a slot that is all one part's may have more of them than the workgroup has threads):
+    // lookup-or-insert in the table (optimizer_kernel.h:299-308), place in its bucket.  The rows it inserts are listed
+    // and filled by all threads: one lane of a wavefront drawing the normal deviates of a row would hold up the others.
+    const uint32_t n_first = sh_first;
+    uint32_t row[SMALL_ITEMS], place[SMALL_ITEMS], bk[SMALL_ITEMS];
 #pragma unroll
-        for (int j = 0; j < SMALL_ITEMS; j++) {
-            rows[j] = NO_ROW;
-            at[j] = 0;
-            if (!(mine & (1u << j))) continue;
-            if (sg[j] == EMPTY_KEY) {
-                bool is_new = false;
-                rows[j] = probe_slot<true>(s, sg[j], is_new);
-                if (is_new) fresh |= 1u << j;
-            } else {
-                at[j] = home_group(sg[j], s.cap);
-                live |= 1u << j;
-            }
-        }
-        const uint64_t groups = s.cap / PROBE_WIDTH;
-        for (uint64_t round = 0; live != 0 && round < 2 * groups + 64; round++) {
-            ulonglong2 q[SMALL_ITEMS][4];
-#pragma unroll
-            for (int j = 0; j < SMALL_ITEMS; j++) {
-                if (!(live & (1u << j))) continue;
-                const ulonglong2* g = reinterpret_cast<const ulonglong2*>(s.keys + at[j]);
-                q[j][0] = g[0], q[j][1] = g[1], q[j][2] = g[2], q[j][3] = g[3];
-            }
-            uint32_t claim = 0, where[SMALL_ITEMS];
-#pragma unroll
-            for (int j = 0; j < SMALL_ITEMS; j++) {
-                where[j] = PROBE_WIDTH;
-                if (!(live & (1u << j))) continue;
-                const uint64_t k[PROBE_WIDTH] = {q[j][0].x, q[j][0].y, q[j][1].x, q[j][1].y,
-                                                 q[j][2].x, q[j][2].y, q[j][3].x, q[j][3].y};
-                bool free_slot = false;
-#pragma unroll
-                for (int e = PROBE_WIDTH - 1; e >= 0; e--)  // the first slot of the group that holds the sign or is free
-                    if (k[e] == sg[j] || k[e] == EMPTY_KEY) {
-                        where[j] = (uint32_t)e;
-                        free_slot = k[e] == EMPTY_KEY;
-                    }
-                if (where[j] == PROBE_WIDTH) {
-                    at[j] = at[j] + PROBE_WIDTH >= s.cap ? 0 : at[j] + PROBE_WIDTH;  // on to the next group
-                } else if (free_slot) {
-                    claim |= 1u << j;
-                } else {
-                    rows[j] = (uint32_t)(at[j] + where[j]);
-                    live &= ~(1u << j);
-                }
-            }
-            uint64_t old[SMALL_ITEMS];
-#pragma unroll
-            for (int j = 0; j < SMALL_ITEMS; j++)
-                if (claim & (1u << j)) old[j] = atomicCAS(ull(&s.keys[at[j] + where[j]]), EMPTY_KEY, sg[j]);
-#pragma unroll
-            for (int j = 0; j < SMALL_ITEMS; j++) {
-                if (!(claim & (1u << j))) continue;
-                if (old[j] == EMPTY_KEY || old[j] == sg[j]) {
-                    rows[j] = (uint32_t)(at[j] + where[j]);
-                    if (old[j] == EMPTY_KEY) fresh |= 1u << j;
-                    live &= ~(1u << j);
-                }  // else another sign took the slot: the group is read again
-            }
-        }
-        uint32_t r = rank0;
-#pragma unroll
-        for (int j = 0; j < SMALL_ITEMS; j++) {
-            if (!(firsts & (1u << j))) continue;
-            if (!(mine & (1u << j))) {
-                r++;
-                continue;
-            }
-            if (rows[j] == NO_ROW) {
-                err |= DEV_ERR_TABLE_FULL;
-            } else if (fresh & (1u << j)) {
+    for (int r = 0; r < SMALL_ITEMS; r++) {
+        const uint32_t i = r * SMALL_THREADS + tid;
+        row[r] = NO_ROW;
+        place[r] = bk[r] = 0;
+        if (i < n_first) {
+            const uint32_t e = used[i];
+            const uint64_t sign = (uint64_t)keys[e];
+            bool is_new = false;
+            row[r] = probe_slot<true>(s, sign, is_new);
+            if (is_new) {
                 const uint32_t k = atomicAdd(&sh_new, 1u);
-                new_sign[k] = sg[j];
-                new_row[k] = rows[j];
+                if (k < (uint32_t)SMALL_NEW) {
+                    new_row[k] = row[r];
+                    new_ent[k] = (uint16_t)e;
+                } else {
+                    init_row(s, o, seed, sign, row[r]);
+                }
             }
-            prow[d.lbase + r] = rows[j];
-            place[j] = atomicAdd(&hist2[group_bucket(sg[j], nb2)], 1u);
-            r++;
+            if (row[r] == NO_ROW) sh_full = 1;
+            bk[r] = scale32((uint32_t)(mix64(sign) >> 32), b.buckets()) - part * b.nbp;
+            place[r] = atomicAdd(&hist[bk[r]], 1u);
         }
     }
     __syncthreads();
-    for (uint32_t b = tid; b < nb2; b += SMALL_THREADS) {
-        const uint32_t c = hist2[b];
-        hist2[b] = c ? atomicAdd(&cursor2[b], c) : 0u;  // this slot's slice of the bucket
+    if (tid == 0) {
+        __hip_atomic_store(reinterpret_cast<unsigned long long*>(host_words + blockIdx.x),
+                           (unsigned long long)small_report(n_first, sh_new, sh_full != 0, seq), __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_SYSTEM);
+        if (sh_new) atomicAdd(s.count, (unsigned long long)sh_new);
     }
-    {
-        // the new rows (row initialiser of init_row): a thread per pair of elements
-        const uint32_t pairs = (uint32_t)(s.D + 1) / 2;
-        const uint32_t work = sh_new * pairs;
+    // where the buckets start among the part's records
+    uint32_t at = 0;
+    for (uint32_t i0 = 0; i0 < b.nbp; i0 += SMALL_THREADS) {
+        const uint32_t c = i0 + tid < b.nbp ? hist[i0 + tid] : 0u;
+        uint32_t total;
+        const uint32_t x = at + block_excl_scan<uint32_t, SMALL_THREADS / 64>(c, wsum, &total);
+        if (i0 + tid < b.nbp) {
+            hist[i0 + tid] = x;
+            p.boff[(size_t)blockIdx.x * (b.nbp + 1) + i0 + tid] = (uint16_t)x;
+        }
+        at += total;
+    }
+    if (tid == 0) p.boff[(size_t)blockIdx.x * (b.nbp + 1) + b.nbp] = (uint16_t)at;
+    __syncthreads();
+    const uint32_t rbase = b.parts * lbase + part * len;
+#pragma unroll
+    for (int r = 0; r < SMALL_ITEMS; r++) {
+        const uint32_t i = r * SMALL_THREADS + tid;
+        if (i < n_first) {
+            const uint32_t w = word[used[i]], pos = w >> 16, cnt = w & 0xFFFFu;
+            // batch_show = occurrences (sparse_table_ops.cc:290-293)
+            p.recs[rbase + hist[bk[r]] + place[r]] = make_uint2(row[r], pos | (cnt << SMALL_SLOT_BITS));
+            p.row_at[lbase + pos] = row[r];
+            p.click_at[lbase + pos] = 0;
+        }
+    }
+    for (uint32_t i = tid; i < b.words; i += SMALL_THREADS) p.bits[(size_t)blockIdx.x * b.words + i] = bits[i];
+    if (sh_new) {
+        const uint32_t pairs = (uint32_t)(s.D + 1) / 2, work = min(sh_new, (uint32_t)SMALL_NEW) * pairs;
         const float stddev = (float)(1.0 / sqrt((double)s.D));
-        for (uint32_t t = tid; t < work; t += SMALL_THREADS) {
-            const uint32_t k = t / pairs;
-            init_row_pair(s, o, seed, (uint64_t)new_sign[k], new_row[k], t - k * pairs, stddev);
+        for (uint32_t q = tid; q < work; q += SMALL_THREADS) {
+            const uint32_t k = q / pairs;
+            init_row_pair(s, o, seed, (uint64_t)keys[new_ent[k]], new_row[k], q - k * pairs, stddev);
         }
-    }
-    __syncthreads();
-    {
-        uint32_t r = rank0;
-#pragma unroll
-        for (int j = 0; j < SMALL_ITEMS; j++) {
-            if (!(firsts & (1u << j))) continue;
-            if (!(mine & (1u << j))) {
-                r++;
-                continue;
-            }
-            const uint32_t b = group_bucket(sg[j], nb2);
-            const uint32_t at = hist2[b] + place[j];
-            if (at < (uint32_t)GRP_CAP) {
-                GroupRec rec;
-                rec.sign = sg[j];
-                rec.gi = r;  // the record's rank in its slot (k_group_emit<true> adds the slot's base)
-                rec.cnt = cnts[h[j]] | ((uint32_t)sl << 24);  // batch_show = occurrences (sparse_table_ops.cc:290-293)
-                recs[(size_t)b * GRP_CAP + at] = rec;
-                rrow[(size_t)b * GRP_CAP + at] = rows[j];
-            } else {
-                err |= DEV_ERR_REMAP_OVERFLOW;  // the host repeats the call with more buckets
-            }
-            r++;
-        }
-    }
-    if (err) atomicOr(&sh_err, err);
-    __syncthreads();
-    // the lookups' outputs last: nothing in this kernel waits for these stores
-#pragma unroll
-    for (int j = 0; j < SMALL_ITEMS; j++) {
-        if (p0 + j >= n || (tid >> 6) % parts != part) continue;
-        const uint32_t r = minpos[h[j]];
-        d.mapped[p0 + j] = (int64_t)r;
-        vals_copy[d.lbase + p0 + j] = sg[j];
-        u_of_gi[d.lbase + p0 + j] = r | ((firsts & (1u << j)) ? FIRST_BIT : 0u);  // relative to the slot until the next launch
-    }
-    if (tid == 0) {  // for the next launch, which adds up the slots' counts and publishes the call's status
-        SlotOut out;
-        out.n_unique = total;
-        out.n_new = sh_new;
-        out.err = sh_err;
-        out.pad = 0;
-        state->slot_out[blockIdx.x] = out;
     }
 }
 
-// Second launch of a small pull, two kinds of workgroups.  The first nb2 group the second-level buckets
-// (group_count_bucket: what k_group_count does).  The others finish what the slots' workgroups began:
-// vars[slot][rank, :] = table row of the slot's distinct sign of that rank (PopulatePulledVariable_,
-// sparse_table_ops.cc:244-265), and the distinct indices of the lookups made global (rank in the slot + base
-// of the slot; the ranks of a slot occupy the first positions of its window of lookup positions).  Each of them
-// adds up the slots' counts itself; the first also leaves the bases and the call's status in device memory and
-// publishes them to the host, which returns from the call when it sees them.
+// Second launch of a small pull: mapped ids (rank of the sign's first lookup) and, for the first lookups, the table row
+// into the variable.  A workgroup takes a run of positions of one slot, a thread per position and part of a row.
 template <int VEC>
-__global__ __launch_bounds__(GRP_THREADS) void k_small_group_finish(
-    uint32_t nb2, const uint32_t* __restrict__ cursor2, const GroupRec* __restrict__ recs, uint32_t big_k,
-    uint2* __restrict__ aux, uint4* __restrict__ bcounts, Store s, const SlotDesc* __restrict__ descs,
-    const uint32_t* __restrict__ lbase, uint32_t* ubase, int N, uint32_t L, const uint32_t* __restrict__ prow,
-    uint32_t* __restrict__ u_of_gi, const SmallState* __restrict__ state, uint32_t parts, DevStatus* status,
-    uint32_t* host_dst, uint32_t* host_seq, uint32_t seq) {
-    __shared__ GroupCountLds lds;
-    if (blockIdx.x < nb2) {
-        group_count_bucket(blockIdx.x, lds, cursor2, recs, big_k, aux, bcounts);
+__global__ __launch_bounds__(SMALL_THREADS) void k_small_group_finish(SmallShape b, SmallPlan p,
+                                                                      uint32_t chunks, Store s) {
+    __shared__ unsigned long long bits[SMALL_WORDS];
+    __shared__ uint32_t before[SMALL_WORDS];
+    const int sl = blockIdx.x / chunks;
+    const uint32_t C = (uint32_t)(s.wdim / VEC), per = SMALL_THREADS / C;  // positions per workgroup
+    const uint32_t p0 = (blockIdx.x % chunks) * per;
+    const SlotDesc d = p.descs[sl];
+    if (p0 >= d.len) return;
+    const uint32_t tid = threadIdx.x;
+    const uint32_t pos = p0 + tid / C, c = tid % C;
+    const bool active = tid < per * C && pos < d.len;
+    const uint32_t gi = d.lbase + pos;
+    const uint32_t f = active ? p.first_of[gi] : 0u;
+    const uint32_t row = active ? p.row_at[gi] : NO_ROW;  // (of a first lookup only)
+    const bool first = active && f == pos;
+    if (tid < SMALL_WORDS) {
+        uint64_t v = 0;
+        if (tid < b.words) {
+            const uint64_t* w = p.bits + (size_t)sl * b.parts * b.words + tid;
+            for (uint32_t q = 0; q < b.parts; q++) v |= w[(size_t)q * b.words];
+        }
+        bits[tid] = v;
+        const uint32_t n = (uint32_t)__popcll(v);
+        uint32_t inc = n;
+        for (int x = 1; x < 64; x <<= 1) {
+            const uint32_t y = __shfl_up(inc, x);
+            if ((int)tid >= x) inc += y;
+        }
+        before[tid] = inc - n;
+    }
+    static_assert(SMALL_WORDS == 64, "one wavefront scans the words");
+    const bool copy = first && row <= s.cap;  // NO_ROW (table full): never address the table with it
+    float4 v4 = make_float4(0.f, 0.f, 0.f, 0.f);
+    float v1 = 0.f;
+    if (copy) {
+        if (VEC == 4)
+            v4 = *reinterpret_cast<const float4*>(s.w + (uint64_t)row * s.wstride + c * 4);
+        else
+            v1 = s.w[(uint64_t)row * s.wstride + c];
+    }
+    __syncthreads();
+    if (!active) return;
+    const uint32_t rank = before[f >> 6] + (uint32_t)__popcll(bits[f >> 6] & ((1ull << (f & 63)) - 1ull));
+    if (c == 0) {
+        d.mapped[pos] = (int64_t)rank;
+        if (first) p.rank_at[gi] = (uint16_t)rank;
+    }
+    if (!copy || (int64_t)rank >= d.rows) return;  // (the host reports a variable that is too small)
+    if (VEC == 4)
+        *reinterpret_cast<float4*>(d.var + (uint64_t)rank * s.wdim + c * 4) = v4;
+    else
+        d.var[(uint64_t)rank * s.wdim + c] = v1;
+}
+
+// Third launch of a small pull, a workgroup per bucket: its records, slot after slot, grouped by row in LDS.
+template <>
+struct EmitArgs<true> {
+    static constexpr int THREADS = EMIT_SMALL_THREADS;
+    SmallShape b;
+    SmallPlan p;
+    uint32_t table;  // entries of the LDS hash table of rows at most: a power of two, 5/4 of the room of a bucket
+    uint32_t big_k;
+};
+inline uint32_t small_emit_table(uint32_t cap) {
+    uint32_t n = 64;
+    while (n < cap + cap / 4) n *= 2;
+    return n;
+}
+inline size_t small_emit_lds(int N, uint32_t cap, uint32_t table) {
+    // per slot: records before it, where its records are, its first lookup; table: row, records / number;
+    // per record: row, gi, rank | slot, occurrences | entry, arrival, list
+    return align_up((size_t)(N + 1) * 4 + (size_t)N * 8 + (size_t)table * 12 + (size_t)cap * 22, 8);
+}
+
+__device__ __forceinline__ void small_emit_bucket(const EmitArgs<true>& a, uint32_t* lds) {
+    const SmallShape& b = a.b;
+    const SmallPlan& p = a.p;
+    const uint32_t N = (uint32_t)b.N;
+    uint32_t* spre = lds;                    // [N + 1]
+    uint32_t* sstart = spre + N + 1;         // [N]
+    uint32_t* slb = sstart + N;              // [N]
+    uint32_t* trow = slb + N;                // [table]
+    uint32_t* tcnt = trow + a.table;         // [table]
+    uint32_t* tinfo = tcnt + a.table;        // [table]: number of the group | first record << 16 (several records)
+    uint32_t* rrow = tinfo + a.table;        // [cap]
+    uint32_t* rgi = rrow + b.cap;            // [cap]
+    uint32_t* rrs = rgi + b.cap;             // [cap]
+    uint32_t* rce = rrs + b.cap;             // [cap]: occurrences (14 bits) | entry << 14
+    uint32_t* rarr = rce + b.cap;            // [cap]
+    uint16_t* list = reinterpret_cast<uint16_t*>(rarr + b.cap);  // [cap]
+    __shared__ uint32_t wsum[EMIT_SMALL_THREADS / 64];
+    __shared__ uint32_t n1, nm, nbig, nmem;
+    const uint32_t tid = threadIdx.x, c = blockIdx.x, part = c / b.nbp, cl = c % b.nbp;
+    if (tid == 0) n1 = nm = nbig = nmem = 0;
+    uint32_t m = 0;
+    for (uint32_t s0 = 0; s0 < N; s0 += EMIT_SMALL_THREADS) {
+        const uint32_t sl = s0 + tid;
+        uint32_t cnt = 0;
+        if (sl < N) {
+            const uint32_t len = p.descs[sl].len, lbase = p.descs[sl].lbase;
+            const uint16_t* off = p.boff + (size_t)(sl * b.parts + part) * (b.nbp + 1) + cl;
+            const uint32_t lo = off[0];
+            cnt = off[1] - lo;
+            sstart[sl] = b.parts * lbase + part * len + lo;
+            slb[sl] = lbase;
+        }
+        uint32_t total;
+        const uint32_t x = m + block_excl_scan<uint32_t, EMIT_SMALL_THREADS / 64>(cnt, wsum, &total);
+        if (sl < N) spre[sl] = x;
+        m += total;
+    }
+    if (tid == 0) spre[N] = m;
+    if (m > b.cap) {  // more records of few signs than a bucket has room for: a push analyses the batch itself
+        if (tid == 0) {
+            *p.bad = 1;
+            p.head[c] = make_uint4(0, 0, 0, 0);
+        }
         return;
     }
-    // (the grouping's LDS is free here)
-    uint32_t* lb = reinterpret_cast<uint32_t*>(lds.mlo);  // lb[N + 1]
-    uint32_t* ub = reinterpret_cast<uint32_t*>(lds.mhi);  // ub[N + 1]
-    uint32_t* wsum = reinterpret_cast<uint32_t*>(lds.sh);
-    uint32_t* misc = reinterpret_cast<uint32_t*>(lds.rech);  // [0] new rows, [1] error flags, [2] distinct signs
-    SlotDesc* sd = reinterpret_cast<SlotDesc*>(lds.keys);  // the slots' descriptors (N <= SMALL_SLOTS: 8 KB of the 16)
-    const uint32_t tid = threadIdx.x;
-    const bool publisher = blockIdx.x == nb2;
-    static_assert(SMALL_SLOT_WORKGROUPS <= GRP_THREADS && SMALL_SLOTS <= SMALL_SLOT_WORKGROUPS, "a thread per workgroup of k_small_slots");
-    // what this thread moves: one 16-byte (or 4-byte) part of the row of one lookup position.  Its row number and
-    // the descriptors are read at once, beside the slots' counts: one round trip instead of three in a row.
-    const uint32_t chunks = (uint32_t)(s.wdim / VEC);
-    const uint64_t t = (uint64_t)(blockIdx.x - nb2) * GRP_THREADS + tid;
-    const bool in_range = t < (uint64_t)L * chunks;
-    const uint32_t gi = in_range ? (uint32_t)(t / chunks) : 0u;
-    const uint32_t c = (uint32_t)(t - (uint64_t)gi * chunks);
-    const uint32_t row = in_range ? prow[gi] : NO_ROW;
-    for (uint32_t i = tid; i < (uint32_t)N * (uint32_t)(sizeof(SlotDesc) / 4); i += GRP_THREADS)
-        reinterpret_cast<uint32_t*>(sd)[i] = reinterpret_cast<const uint32_t*>(descs)[i];
-    uint32_t mine = 0, nn = 0, ee = 0;
-    if (tid < (uint32_t)N * parts) {  // (every workgroup of a slot leaves the slot's count, and its own share of the rest)
-        const SlotOut so = state->slot_out[tid];
-        nn = so.n_new;
-        ee = so.err;
-    }
-    if (tid < (uint32_t)N) mine = state->slot_out[tid * parts].n_unique;
-    for (uint32_t i = tid; i <= (uint32_t)N; i += GRP_THREADS) lb[i] = lbase[i];
-    if (tid < 2) misc[tid] = 0;
-    const uint32_t base = block_excl_scan<uint32_t, GRP_THREADS / 64>(mine, wsum, &misc[2]);  // (barriers inside)
-    if (tid < (uint32_t)N) ub[tid] = base;
-    if (publisher) {
-        if (nn) atomicAdd(&misc[0], nn);
-        if (ee) atomicOr(&misc[1], ee);
+    uint32_t table = 64;  // of the records there are
+    while (table < m + m / 4) table *= 2;
+    for (uint32_t i = tid; i < table; i += EMIT_SMALL_THREADS) {
+        trow[i] = NO_ROW;
+        tcnt[i] = 0;
     }
     __syncthreads();
-    const uint32_t U = misc[2];
-    if (tid == 0) ub[N] = U;
-    if (publisher && tid < 64) {  // one wavefront: device copies, then the host's, then the word the host polls
-        const uint32_t sw = sizeof(DevStatus) / 4;
-        for (uint32_t i = tid; i <= (uint32_t)N; i += 64) {
-            const uint32_t v = i < (uint32_t)N ? ub[i] : U;
-            ubase[i] = v;
-            host_store(host_dst + sw + i, v);
+    for (uint32_t i = tid; i < m; i += EMIT_SMALL_THREADS) {
+        const uint32_t sl = (uint32_t)find_slot(spre, (int)N, i);
+        const uint2 r = p.recs[sstart[sl] + i - spre[sl]];
+        const uint32_t gi = slb[sl] + (r.y & ((1u << SMALL_SLOT_BITS) - 1u));
+        const uint32_t rank = p.rank_at[gi];
+        uint32_t e = 0;
+        if (r.x != NO_ROW) {  // (a sign the table had no room for: nothing to update)
+            e = (r.x * 2654435761u >> 12) & (table - 1);
+            for (;;) {  // more entries than records
+                uint32_t old = trow[e];
+                if (old == NO_ROW) old = atomicCAS(&trow[e], NO_ROW, r.x);
+                if (old == NO_ROW || old == r.x) break;
+                e = (e + 1) & (table - 1);
+            }
+            rarr[i] = atomicAdd(&tcnt[e], 1u);
         }
-        if (tid == 0) {
-            DevStatus st{};
-            st.err = misc[1];
-            st.n_unique = U;
-            st.n_new = misc[0];
-            st.gcap = U + U / 2 < 16 ? 16 : U + U / 2;
-            *status = st;
-            *s.count += misc[0];
-            const uint32_t* sp = reinterpret_cast<const uint32_t*>(&st);
-            for (uint32_t i = 0; i < sw; i++) host_store(host_dst + i, sp[i]);
-        }
-        __threadfence_system();
-        if (tid == 0) host_store(host_seq, seq);
+        rrow[i] = r.x;
+        rgi[i] = gi;
+        rrs[i] = rank | (sl << 16);
+        rce[i] = (r.y >> SMALL_SLOT_BITS) | (e << 14);
     }
     __syncthreads();
-    // (one thread per position and part of the row: few rows per thread would leave the rows' round trips in a queue)
-    if (!in_range) return;
-    const int sl = find_slot(lb, N, gi);
-    if (c == 0) u_of_gi[gi] += ub[sl];
-    const uint32_t r = gi - lb[sl];
-    if (r >= ub[sl + 1] - ub[sl]) return;  // beyond the slot's distinct signs
-    const SlotDesc& d = sd[sl];
-    if ((int64_t)r >= d.rows) return;      // the host reports the variable as too small
-    if (row > s.cap) return;  // NO_ROW (table full): never address the table with it
-    if (VEC == 4) {
-        const float4 v = *reinterpret_cast<const float4*>(s.w + (uint64_t)row * s.wstride + c * 4);
-        *reinterpret_cast<float4*>(d.var + (uint64_t)r * s.wdim + c * 4) = v;
-    } else {
-        d.var[(uint64_t)r * s.wdim + c] = s.w[(uint64_t)row * s.wstride + c];
+    const size_t first = (size_t)c * b.cap;
+    // signs with one record: numbered and written at once; with several: a number and a stretch of the records for each
+    for (uint32_t i = tid; i < m; i += EMIT_SMALL_THREADS) {
+        if (rrow[i] == NO_ROW) continue;
+        const uint32_t e = rce[i] >> 14, k = tcnt[e];
+        if (k == 1) {
+            const uint32_t g = atomicAdd(&n1, 1u);
+            p.group[first + g] = make_uint2(rrow[i], g | (1u << 16));
+            p.member[first + g] = make_uint4(rgi[i], rrs[i], rce[i] & 0x3FFFu, 0u);
+        } else if (rarr[i] == 0) {
+            tinfo[e] = atomicAdd(is_big(k, a.big_k) ? &nbig : &nm, 1u) | (atomicAdd(&nmem, k) << 16);
+        }
     }
+    __syncthreads();
+    for (uint32_t i = tid; i < m; i += EMIT_SMALL_THREADS) {
+        if (rrow[i] == NO_ROW) continue;
+        const uint32_t e = rce[i] >> 14, k = tcnt[e];
+        if (k > 1) list[(tinfo[e] >> 16) + rarr[i]] = (uint16_t)i;
+    }
+    __syncthreads();
+    for (uint32_t i = tid; i < m; i += EMIT_SMALL_THREADS) {
+        if (rrow[i] == NO_ROW) continue;
+        const uint32_t e = rce[i] >> 14, k = tcnt[e];
+        if (k == 1) continue;
+        const uint32_t at = tinfo[e] >> 16;
+        uint32_t place = 0;  // records of the sign in earlier slots
+        for (uint32_t j = 0; j < k; j++) place += list[at + j] < i ? 1u : 0u;
+        p.member[first + n1 + at + place] = make_uint4(rgi[i], rrs[i], rce[i] & 0x3FFFu, 0u);
+        if (rarr[i] == 0) {
+            const uint32_t g = tinfo[e] & 0xFFFFu;
+            p.group[first + (is_big(k, a.big_k) ? b.cap - 1 - g : n1 + g)] = make_uint2(rrow[i], (n1 + at) | (k << 16));
+        }
+    }
+    if (tid == 0) p.head[c] = make_uint4(n1, nm, nbig, nmem);
 }
 
-// First launch of a small push on the last pull's plan: the slot descriptors come in from the host's staging
-// buffer (a workgroup reads those of its tile's slots into LDS, the first also copies all of them to device
-// memory for the update kernels), the signs are compared with the plan's copy, and with CLICKS the non-zero labels are added to
-// the click sums of the member lists (sparse_table_ops.cc:283-296; a few thousand lookups do not queue up on
-// any entry).  A mismatch also goes to the host (pinned memory); that the comparison is complete, the kernel
-// launched next tells it.
+// First launch of a small push on the last pull's plan: the signs are compared with the plan's copy, and with CLICKS the
+// non-zero labels are added to the click sums (sparse_table_ops.cc:283-296; a few thousand lookups do not queue up on
+// any entry).  A mismatch also goes to the host (pinned memory); that the comparison is complete, the last launch tells it.
 template <bool CLICKS>
-__global__ __launch_bounds__(256) void k_small_verify(const SlotDesc* host_descs, SlotDesc* push_descs,
-                                                      const uint32_t* __restrict__ lbase, int N, uint32_t L,
-                                                      const uint64_t* __restrict__ vals_copy, DevStatus* status,
-                                                      const uint32_t* __restrict__ u_of_gi,
-                                                      const uint2* __restrict__ where_u, Member* list,
-                                                      uint32_t* host_mismatch) {
-    extern __shared__ uint32_t lb[];      // lb[N + 1]
-    __shared__ SlotDesc sd[SMALL_SLOTS];  // the descriptors of the slots the tile touches: sd[0] is slot s0's
-    for (int i = threadIdx.x; i <= N; i += 256) lb[i] = lbase[i];
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        status->err = 0;  // what the pull reported is on the host; the update kernels start from a clean slate
-        status->abort = 0;
-    }
-    __syncthreads();
-    constexpr uint32_t DW = sizeof(SlotDesc) / 4;
-    const int s0 = find_slot(lb, N, blockIdx.x * SMALL_TILE);
-    const int s1 = find_slot(lb, N, min(L, (blockIdx.x + 1) * (uint32_t)SMALL_TILE) - 1);
-    {
-        const uint32_t* src = reinterpret_cast<const uint32_t*>(host_descs + s0);
-        const uint32_t words = (uint32_t)(s1 - s0 + 1) * DW;
-        for (uint32_t i = threadIdx.x; i < words; i += 256) reinterpret_cast<uint32_t*>(sd)[i] = src[i];
-    }
-    if (blockIdx.x == 0) {  // all of them into device memory, for the update kernels
-        const uint32_t words = (uint32_t)N * DW;
-        for (uint32_t i = threadIdx.x; i < words; i += 256)
-            reinterpret_cast<uint32_t*>(push_descs)[i] = reinterpret_cast<const uint32_t*>(host_descs)[i];
-    }
-    __syncthreads();
-    const uint32_t g0 = blockIdx.x * SMALL_TILE;
-    const uint32_t g1 = min(L, g0 + (uint32_t)SMALL_TILE);
-    bool bad = false;
+__global__ __launch_bounds__(256) void k_small_verify(SmallShape b, SmallPlan p, const SlotDesc* host_descs, uint32_t chunks,
+                                                      DevStatus* status, uint32_t* host_mismatch) {
+    __shared__ SlotDesc sd;
+    const int sl = blockIdx.x / chunks;
+    const uint32_t p0 = (blockIdx.x % chunks) * SMALL_TILE;
+    // what the pull left of these positions is on its way while the descriptor comes in from the host's staging buffer
+    const uint32_t lbase = p.descs[sl].lbase, len = p.descs[sl].len;  // (the shape is the pull's)
     constexpr int PER = SMALL_TILE / 256;
     uint64_t now[PER], then[PER];
     int label[PER];
-    uint32_t u[PER];
+    uint32_t f[PER];
 #pragma unroll
     for (int j = 0; j < PER; j++) {
-        const uint32_t gi = g0 + j * 256 + threadIdx.x;
-        now[j] = then[j] = 0;
-        label[j] = 0;
-        u[j] = 0;
-        if (gi < g1) {
-            const int sl = find_slot(lb, N, gi);
-            now[j] = (uint64_t)sd[sl - s0].values[gi - lb[sl]];
-            then[j] = vals_copy[gi];
-            if (CLICKS) {
-                label[j] = (int)sd[sl - s0].labels[gi - lb[sl]];
-                u[j] = u_of_gi[gi] & ~FIRST_BIT;
-            }
-        }
+        const uint32_t pos = p0 + j * 256 + threadIdx.x;
+        then[j] = pos < len ? p.vals_copy[lbase + pos] : 0;
+        f[j] = CLICKS && pos < len ? p.first_of[lbase + pos] : 0u;
+    }
+    if (threadIdx.x < sizeof(SlotDesc) / 4) {
+        const uint32_t w = reinterpret_cast<const uint32_t*>(host_descs + sl)[threadIdx.x];
+        reinterpret_cast<uint32_t*>(&sd)[threadIdx.x] = w;
+        if (p0 == 0) reinterpret_cast<uint32_t*>(p.push_descs + sl)[threadIdx.x] = w;  // for the launches after this one
+    }
+    bool bad = false;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        bad = *p.bad != 0;
+        status->abort = 0;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < PER; j++) {
+        const uint32_t pos = p0 + j * 256 + threadIdx.x;
+        now[j] = pos < len ? (uint64_t)sd.values[pos] : 0;
+        label[j] = CLICKS && pos < len ? (int)sd.labels[pos] : 0;
     }
 #pragma unroll
     for (int j = 0; j < PER; j++) {
         bad |= now[j] != then[j];
-        if (CLICKS && label[j] != 0) atomicAdd(&list[where_u[u[j]].x & WHERE_PLACE].click, label[j]);
+        if (CLICKS && label[j] != 0) atomicAdd(&p.click_at[lbase + f[j]], label[j]);
     }
     if (bad) {
         atomicOr(&status->mismatch, 1u);
@@ -485,68 +488,478 @@ __global__ __launch_bounds__(256) void k_small_verify(const SlotDesc* host_descs
     }
 }
 
+// Pooled gradients: the gradient of every distinct sign of a slot is the sum over its lookups, in order, of their
+// examples' rows times 1 / d(lookups of the example); a workgroup per slot.  The lookups are ordered by their sign's
+// first position with a stable radix sort in LDS (two passes of 7 bits, a wavefront's lanes told apart by ballots) and
+// every stretch of POOL_PIECE lookups of one sign is summed by a group of lanes; the sums of a sign with several
+// stretches are added in order.  The order of all additions is fixed.  flat[gi of the sign's first lookup, :] = sum, over
+// the D elements the updates read (rows of `dim`: with the cvm columns).
+constexpr int POOL_THREADS = 1024;
+constexpr int POOL_ITEMS = SMALL_SLOT_MAX / POOL_THREADS;
+constexpr int POOL_WAVES = POOL_THREADS / 64;
+constexpr int POOL_RUN = SMALL_SLOT_MAX / POOL_WAVES;  // consecutive lookups a wavefront sorts
+constexpr uint32_t POOL_PIECE = 32;
+constexpr int POOL_DIGIT = 7;
+enum { POOL_SUM = 0, POOL_MEAN = 1, POOL_SQRTN = 2 };  // (the combiners of the C ABI)
+static_assert(2 * POOL_DIGIT >= SMALL_SLOT_BITS && POOL_RUN == 64 * POOL_ITEMS, "two passes sort a slot");
+
+// Last set bit at or below i, first one above it (or `none`), in a bitmap in LDS.
+__device__ __forceinline__ uint32_t bit_at_or_below(const unsigned long long* bm, uint32_t i) {
+    uint32_t w = i >> 6;
+    unsigned long long v = bm[w] & (~0ull >> (63 - (i & 63)));
+    while (v == 0) v = bm[--w];  // (bit 0 is set)
+    return w * 64 + 63 - (uint32_t)__clzll((long long)v);
+}
+__device__ __forceinline__ uint32_t bit_above(const unsigned long long* bm, uint32_t i, uint32_t words, uint32_t none) {
+    uint32_t w = i >> 6;
+    unsigned long long v = (i & 63) == 63 ? 0ull : bm[w] & (~0ull << ((i & 63) + 1));
+    while (v == 0) {
+        if (++w >= words) return none;
+        v = bm[w];
+    }
+    return w * 64 + (uint32_t)__ffsll((long long)v) - 1;
+}
+
+template <int LPG, bool ANY>
+__global__ __launch_bounds__(POOL_THREADS) void k_small_pool(SmallShape b, SmallPlan p, const SlotDesc* __restrict__ descs,
+                                                             int64_t batch, int dim, int D, int combiner,
+                                                             float* __restrict__ flat, float* __restrict__ partial,
+                                                             DevStatus* status,
+                                                             uint32_t* host_err) {
+    __shared__ uint16_t fo[SMALL_SLOT_MAX];             // first position of the lookup's sign
+    __shared__ uint32_t xb[SMALL_SLOT_MAX];             // example of the lookup
+    __shared__ uint16_t ord[SMALL_SLOT_MAX];            // the lookups in the order of their signs
+    __shared__ uint16_t piece[SMALL_SLOT_MAX + 1];      // where the pieces start in it
+    __shared__ uint32_t work[SMALL_SLOT_MAX];           // while sorting: the order after the first pass, counters; then the scales
+    __shared__ unsigned long long heads[SMALL_WORDS];   // starts: of the examples by position, then of the signs in the order
+    __shared__ uint32_t wsum[POOL_WAVES];
+    __shared__ uint32_t bad;
+    uint16_t* const half = reinterpret_cast<uint16_t*>(work);                          // [SMALL_SLOT_MAX]
+    uint32_t* const digit = work + SMALL_SLOT_MAX / 2;                                 // [1 << POOL_DIGIT][POOL_WAVES]
+    float* const scale = reinterpret_cast<float*>(work);                               // [SMALL_SLOT_MAX], by position
+    static_assert((POOL_WAVES << POOL_DIGIT) <= SMALL_SLOT_MAX / 2, "the counters fit");
+    const SlotDesc d = descs[blockIdx.x];
+    const uint32_t n = d.len, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    if (n == 0 || status->mismatch) return;
+    const int64_t* ex = d.mapped;
+    if (tid == 0) bad = 0;
+    for (uint32_t i = tid; i < SMALL_WORDS; i += POOL_THREADS) heads[i] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < POOL_ITEMS; j++) {
+        const uint32_t i = wave * POOL_RUN + j * 64 + lane;
+        bool head = false;
+        if (i < n) {
+            const int64_t x = ex[i], prev = i > 0 ? ex[i - 1] : -1;
+            if (x < 0 || x >= batch || prev > x) bad = 1;
+            fo[i] = p.first_of[d.lbase + i];
+            xb[i] = (uint32_t)x;
+            head = x != prev;
+        }
+        const unsigned long long m = __ballot(head);
+        if (lane == 0) heads[i >> 6] = m;
+    }
+    __syncthreads();
+    if (bad) {  // unsorted or out-of-range example ids: nothing of this push is applied
+        if (tid == 0) {
+            status->abort = 1;
+            host_store(host_err, 1u);
+        }
+        return;
+    }
+    const uint32_t words = (n + 63) / 64;
+    float mine[POOL_ITEMS];  // 1 / d(lookups of the example) of my lookups
+#pragma unroll
+    for (int j = 0; j < POOL_ITEMS; j++) {
+        const uint32_t i = wave * POOL_RUN + j * 64 + lane;
+        mine[j] = 1.f;
+        if (i < n && combiner != POOL_SUM) {
+            const float cnt = (float)(bit_above(heads, i, words, n) - bit_at_or_below(heads, i));
+            mine[j] = 1.f / (combiner == POOL_MEAN ? cnt : sqrtf(cnt));
+        }
+    }
+    // stable sort by fo: pass 0 takes the lookups in order, pass 1 the order of pass 0
+    for (int pass = 0; pass < 2; pass++) {
+        for (uint32_t i = tid; i < POOL_WAVES << POOL_DIGIT; i += POOL_THREADS) digit[i] = 0;
+        __syncthreads();
+        uint32_t item[POOL_ITEMS], dg[POOL_ITEMS], at[POOL_ITEMS];
+#pragma unroll
+        for (int j = 0; j < POOL_ITEMS; j++) {
+            const uint32_t i = wave * POOL_RUN + j * 64 + lane;
+            const bool valid = i < n;
+            item[j] = valid ? (pass == 0 ? i : (uint32_t)half[i]) : 0u;
+            dg[j] = valid ? ((uint32_t)fo[item[j]] >> (pass * POOL_DIGIT)) & ((1u << POOL_DIGIT) - 1u) : 0u;
+            unsigned long long same = __ballot(valid);
+#pragma unroll
+            for (int q = 0; q < POOL_DIGIT; q++) {
+                const unsigned long long m = __ballot((dg[j] >> q) & 1u);
+                same &= ((dg[j] >> q) & 1u) ? m : ~m;
+            }
+            at[j] = 0;
+            const uint32_t k = dg[j] * POOL_WAVES + wave;
+            if (valid) at[j] = digit[k] + (uint32_t)__popcll(same & ((1ull << lane) - 1ull));  // (before this round)
+            wave_sync();
+            if (valid && (uint32_t)__ffsll((long long)same) - 1 == lane) digit[k] += (uint32_t)__popcll(same);
+            wave_sync();
+        }
+        __syncthreads();
+        {  // digit by digit and wavefront by wavefront: where they go
+            constexpr uint32_t EACH = (POOL_WAVES << POOL_DIGIT) / POOL_THREADS;
+            uint32_t c[EACH], sum = 0;
+#pragma unroll
+            for (uint32_t q = 0; q < EACH; q++) {
+                c[q] = digit[tid * EACH + q];
+                sum += c[q];
+            }
+            uint32_t x = block_excl_scan<uint32_t, POOL_WAVES>(sum, wsum, nullptr);
+#pragma unroll
+            for (uint32_t q = 0; q < EACH; q++) {
+                digit[tid * EACH + q] = x;
+                x += c[q];
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < POOL_ITEMS; j++)
+            if (wave * POOL_RUN + j * 64 + lane < n)
+                (pass == 0 ? half : ord)[digit[dg[j] * POOL_WAVES + wave] + at[j]] = (uint16_t)item[j];
+        __syncthreads();
+    }
+    // starts of the signs in the order; the scales in the counters' place
+#pragma unroll
+    for (int j = 0; j < POOL_ITEMS; j++) {
+        const uint32_t i = wave * POOL_RUN + j * 64 + lane;
+        const bool head = i < n && (i == 0 || fo[ord[i]] != fo[ord[i - 1]]);
+        const unsigned long long m = __ballot(head);
+        if (lane == 0) heads[i >> 6] = m;
+        if (i < n) scale[i] = mine[j];
+    }
+    __syncthreads();
+    // pieces: every POOL_PIECE lookups of a sign
+    uint32_t starts = 0;
+#pragma unroll
+    for (int j = 0; j < POOL_ITEMS; j++) {
+        const uint32_t i = tid * POOL_ITEMS + j;
+        if (i < n && ((i - bit_at_or_below(heads, i)) % POOL_PIECE) == 0) starts |= 1u << j;
+    }
+    uint32_t pieces;
+    uint32_t k = block_excl_scan<uint32_t, POOL_WAVES>(__popc(starts), wsum, &pieces);
+#pragma unroll
+    for (int j = 0; j < POOL_ITEMS; j++)
+        if (starts & (1u << j)) piece[k++] = (uint16_t)(tid * POOL_ITEMS + j);
+    if (tid == 0) piece[pieces] = (uint16_t)n;
+    __syncthreads();
+    const float* pooled = d.grads;
+    const int sub = tid % LPG;
+    for (uint32_t q = tid / LPG; q < pieces; q += POOL_THREADS / LPG) {
+        const uint32_t lo = piece[q], hi = piece[q + 1];
+        float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+        for (uint32_t j0 = lo; j0 < hi; j0 += 8) {  // eight rows in flight
+            float4 g[8];
+            float sc[8];
+#pragma unroll
+            for (uint32_t w = 0; w < 8; w++) {
+                const uint32_t i = ord[min(j0 + w, hi - 1)];
+                sc[w] = scale[i];
+                g[w] = row_part<ANY>(pooled + (uint64_t)xb[i] * dim, sub, D);
+            }
+#pragma unroll
+            for (uint32_t w = 0; w < 8; w++) {
+                if (j0 + w >= hi) break;
+                acc.x += g[w].x * sc[w];
+                acc.y += g[w].y * sc[w];
+                acc.z += g[w].z * sc[w];
+                acc.w += g[w].w * sc[w];
+            }
+        }
+        const uint32_t head = bit_at_or_below(heads, lo);
+        const bool whole = head == lo && (hi == n || ((heads[hi >> 6] >> (hi & 63)) & 1ull));
+        float* out = whole ? flat + (uint64_t)(d.lbase + fo[ord[lo]]) * dim : partial + (uint64_t)(d.lbase + q) * dim;
+        put_row_part<ANY>(out, sub, D, acc);
+    }
+    __syncthreads();
+    for (uint32_t q = tid / LPG; q < pieces; q += POOL_THREADS / LPG) {
+        const uint32_t lo = piece[q], hi = piece[q + 1];
+        if (bit_at_or_below(heads, lo) != lo || hi == n || ((heads[hi >> 6] >> (hi & 63)) & 1ull)) continue;
+        float4 acc = row_part<ANY>(partial + (uint64_t)(d.lbase + q) * dim, sub, D);
+        for (uint32_t r = q + 1; r < pieces; r++) {
+            const uint32_t at = piece[r];
+            if ((heads[at >> 6] >> (at & 63)) & 1ull) break;  // the next sign
+            const float4 g = row_part<ANY>(partial + (uint64_t)(d.lbase + r) * dim, sub, D);
+            acc.x += g.x;
+            acc.y += g.y;
+            acc.z += g.z;
+            acc.w += g.w;
+        }
+        put_row_part<ANY>(flat + (uint64_t)(d.lbase + fo[ord[lo]]) * dim, sub, D, acc);
+    }
+}
+
+// Where the update kernels find the gradient of a record: the slots' matrices (in LDS), or the reduced rows of a push
+// of pooled gradients, one per first lookup.
+struct SmallSrc {
+    const float* const* grads;
+    const uint32_t* rows;
+    const float* flat;
+    int32_t* click_at;
+    int dim;
+    __device__ __forceinline__ const float* gradient(uint4 m) const {
+        if (flat) return flat + (uint64_t)m.x * dim;
+        const uint32_t sl = m.y >> 16, rank = m.y & 0xFFFFu;
+        return rank < rows[sl] ? grads[sl] + (uint64_t)rank * dim : nullptr;  // (the host reports a matrix with too few rows)
+    }
+    // the record's click sum; zero again for a further push on the plan
+    __device__ __forceinline__ int click(uint4 m) const { return click_at[m.x]; }
+};
+
+// One sign with a few records by a group of LPG lanes, AHEAD records at a time: the gradients of the next AHEAD and the
+// member entries of the AHEAD after those are in flight meanwhile, so that a chain of k records costs k / AHEAD round
+// trips instead of 2 k (a small batch's kernels are as long as their longest chain).  Every load is issued whether its
+// record exists or not (past the end: the group's last member again, the row in place of a gradient): a load under a
+// condition makes the compiler wait for all loads where the branches join.
+template <int KIND, int LPG, bool ANY, int AHEAD>
+__device__ __forceinline__ void small_apply_group(const Store& s, const OptDev& o, const SmallSrc& src, uint32_t row,
+                                                  uint32_t k, const uint4* mem, int sub, int lane0, float c1, float c2) {
+    const int D = s.D;
+    float* wp = s.w + (uint64_t)row * s.wstride;
+    float* sp = s.st + (uint64_t)row * s.sstride;
+    float4 w = row_part<ANY>(wp, sub, D);
+    float4 a, b;  // Adam m, v / Ftrl z, n
+    float g2sum = 0.f, show = 0.f, click = 0.f;
+    int delta_show = 0;
+    if (KIND == OPT_ADAGRAD) {
+        const float4 h = *reinterpret_cast<const float4*>(sp);
+        g2sum = h.x;
+        show = h.y;
+        click = h.z;
+    } else {
+        a = row_part<ANY>(sp, sub, D);
+        b = row_part<ANY>(sp + D, sub, D);
+        delta_show = __float_as_int(sp[2 * D + 1]);
+    }
+    bool any = false;
+    uint4 m1[AHEAD], m2[AHEAD];
+    float4 g0[AHEAD], g1[AHEAD];
+    int sh0[AHEAD], ck0[AHEAD], sh1[AHEAD], ck1[AHEAD];
+    bool ok0[AHEAD], ok1[AHEAD];
+    auto fetch = [&](const uint4 (&m)[AHEAD], uint32_t first, float4 (&g)[AHEAD], int (&sh)[AHEAD], int (&ck)[AHEAD],
+                     bool (&ok)[AHEAD]) {
+#pragma unroll
+        for (int q = 0; q < AHEAD; q++) {
+            const float* gp = src.gradient(m[q]);
+            ok[q] = gp != nullptr && first + q < k;
+            sh[q] = (int)m[q].z;
+            ck[q] = KIND == OPT_ADAGRAD ? src.click(m[q]) : 0;
+            g[q] = row_part<ANY>(ok[q] ? gp : wp, sub, D);
+        }
+    };
+#pragma unroll
+    for (int q = 0; q < AHEAD; q++) {
+        m1[q] = mem[min((uint32_t)q, k - 1)];
+        m2[q] = mem[min((uint32_t)(AHEAD + q), k - 1)];
+    }
+    fetch(m1, 0, g0, sh0, ck0, ok0);
+#pragma unroll
+    for (int q = 0; q < AHEAD; q++) m1[q] = m2[q];
+    for (uint32_t c0 = 0; c0 < k; c0 += AHEAD) {
+#pragma unroll
+        for (int q = 0; q < AHEAD; q++) m2[q] = mem[min(c0 + 2 * AHEAD + q, k - 1)];
+        fetch(m1, c0 + AHEAD, g1, sh1, ck1, ok1);
+        if constexpr (KIND == OPT_ADAGRAD) {
+            // The records of the window depend on each other through g2sum (one rounded addition per record) and
+            // through the row (one subtraction per element and record) only.  Everything else -- the sums of squares
+            // with their hand-over from lane to lane, the square roots, the divisions -- is worked out for all records of
+            // the window side by side; the two chains then run over the results, in record order.  The same operations
+            // on the same operands as record after record.
+            double mq[AHEAD];
+#pragma unroll
+            for (int q = 0; q < AHEAD; q++) mq[q] = 0.0;
+            for (int l = 0; l < LPG; l++) {
+#pragma unroll
+                for (int q = 0; q < AHEAD; q++) {
+                    double cand = mq[q];  // add_g2sum: double accumulator over the float products, element order 0..D-1
+                    cand += (double)(g0[q].x * g0[q].x);
+                    cand += (double)(g0[q].y * g0[q].y);
+                    cand += (double)(g0[q].z * g0[q].z);
+                    cand += (double)(g0[q].w * g0[q].w);
+                    mq[q] = __shfl(cand, lane0 + l);
+                }
+            }
+#pragma unroll
+            for (int q = 0; q < AHEAD; q++) mq[q] = mq[q] / (double)D;
+            float g2[AHEAD];
+#pragma unroll
+            for (int q = 0; q < AHEAD; q++) {
+                if (ok0[q]) {
+                    any = true;
+                    show += (float)sh0[q];
+                    click += (float)ck0[q];
+                    g2sum = (float)((double)g2sum + mq[q]);
+                }
+                g2[q] = g2sum;
+            }
+            float4 st4[AHEAD];
+#pragma unroll
+            for (int q = 0; q < AHEAD; q++) {
+                const float den = o.eps + sqrtf(g2[q]);
+                st4[q] = make_float4(o.lr * g0[q].x / den, o.lr * g0[q].y / den, o.lr * g0[q].z / den, o.lr * g0[q].w / den);
+            }
+#pragma unroll
+            for (int q = 0; q < AHEAD; q++) {
+                if (!ok0[q]) continue;
+                w.x -= st4[q].x;
+                w.y -= st4[q].y;
+                w.z -= st4[q].z;
+                w.w -= st4[q].w;
+            }
+        } else {
+#pragma unroll
+            for (int q = 0; q < AHEAD; q++) {
+                if (!ok0[q]) continue;
+                any = true;
+                delta_show += sh0[q];
+                if (KIND == OPT_ADAM) {
+                    adam_elem(o, c1, c2, g0[q].x, w.x, a.x, b.x);
+                    adam_elem(o, c1, c2, g0[q].y, w.y, a.y, b.y);
+                    adam_elem(o, c1, c2, g0[q].z, w.z, a.z, b.z);
+                    adam_elem(o, c1, c2, g0[q].w, w.w, a.w, b.w);
+                } else {
+                    ftrl_elem(o, g0[q].x, w.x, a.x, b.x);
+                    ftrl_elem(o, g0[q].y, w.y, a.y, b.y);
+                    ftrl_elem(o, g0[q].z, w.z, a.z, b.z);
+                    ftrl_elem(o, g0[q].w, w.w, a.w, b.w);
+                }
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < AHEAD; q++) {
+            g0[q] = g1[q];
+            sh0[q] = sh1[q];
+            ck0[q] = ck1[q];
+            ok0[q] = ok1[q];
+            m1[q] = m2[q];
+        }
+    }
+    if (KIND == OPT_ADAGRAD)
+        for (uint32_t j = sub; j < k; j += LPG) src.click_at[mem[j].x] = 0;
+    if (!any) return;
+    put_row_part<ANY>(wp, sub, D, w);
+    if (KIND == OPT_ADAGRAD) {
+        if (sub == 0) {
+            *reinterpret_cast<float4*>(sp) = make_float4(g2sum, show, click, 0.f);  // no_show_days = 0
+            if (o.use_cvm) {
+                wp[D] = show;
+                wp[D + 1] = logf(click + 1) - logf(show + 1);
+            }
+        }
+    } else {
+        put_row_part<ANY>(sp, sub, D, a);
+        put_row_part<ANY>(sp + D, sub, D, b);
+        if (sub == 0) sp[2 * D + 1] = __int_as_float(delta_show);
+    }
+}
+
 // Bytes of dynamic LDS of k_small_apply when its launch includes the workgroups for the signs with many records:
 // per wavefront the staging and the row of apply_big_groups, then its pointer, count, flag and divisor arrays.
 inline size_t small_apply_wave_lds(int D) { return align_up(big_lds_bytes(D), 8) + BIG_CHUNK * (8 + 4 + 4 + 4); }
-inline size_t small_apply_big_lds(int D) { return 4 * small_apply_wave_lds(D); }
 
-// The updates of a small push by one launch.  The first big_blocks workgroups (if the plan lists signs with many
-// records; they start first, their chains are the longest): each of their wavefronts takes such signs the way
-// k_apply_big does -- as a launch of its own that kernel costs a small batch as much again as this one.  The
-// workgroups after those: every group with fewer than big_k records, one record or several, by the lane groups
-// of k_apply_vec, the records of a sign four at a time.
-// Nothing is reported to the host but that this kernel runs, which tells it that the comparison of the signs,
-// launched before, is complete: on the plan of the last pull every sign has its row, and the host has compared
+__host__ __device__ inline size_t small_apply_slots_lds(int N) { return ((size_t)N * 12 + 7) / 8 * 8; }
+
+// The updates of a small push by one launch, `roles` workgroups per bucket: the signs with one record; with a few, by
+// lane groups, several records at a time; with many (four slots' worth and more), by a wavefront each the way
+// k_apply_big does.  Nothing is reported to the host but that this kernel runs, which tells it that the comparison of
+// the signs, launched before, is complete: on the plan of the last pull every sign has its row, and the host has compared
 // the slots' distinct counts with the rows of the gradient matrices itself.
 template <int KIND, int LPG, bool ANY>
-__global__ __launch_bounds__(256) void k_small_apply(Store s, OptDev o, PushSrc src, int N, DevStatus* status,
-                                                     const uint32_t* __restrict__ grp_row,
-                                                     const uint32_t* __restrict__ grp_off,
-                                                     const uint32_t* __restrict__ grp_cnt,
-                                                     const Member* __restrict__ list, uint32_t big_k,
-                                                     uint32_t ids_cap, uint32_t* host_seq, uint32_t seq,
-                                                     uint32_t big_blocks, const uint32_t* __restrict__ big_list,
-                                                     int gbuf_floats, uint32_t wave_lds, uint32_t wave_arrays) {
-    extern __shared__ unsigned long long big_lds[];  // (only the first big_blocks workgroups use it)
+__global__ __launch_bounds__(256) void k_small_apply(SmallShape b, SmallPlan p, const float* flat, Store s,
+                                                     OptDev o, const DevStatus* __restrict__ status, uint32_t* host_seq,
+                                                     uint32_t seq, int dim, int gbuf_floats, uint32_t wave_lds,
+                                                     uint32_t wave_arrays) {
+    extern __shared__ unsigned long long apply_lds[];  // the slots' gradient matrices and their rows; then the wavefronts' staging
     if (blockIdx.x == 0 && threadIdx.x == 0) host_store(host_seq, seq);
-    // the slots' gradient matrices and bases from LDS: one round trip less in every record's chain of loads
-    __shared__ SlotDesc sd[SMALL_SLOTS];
-    __shared__ uint32_t ub[SMALL_SLOTS + 1];
-    const uint32_t words = (uint32_t)N * (uint32_t)(sizeof(SlotDesc) / 4);
-    for (uint32_t i = threadIdx.x; i < words; i += 256)
-        reinterpret_cast<uint32_t*>(sd)[i] = reinterpret_cast<const uint32_t*>(src.descs)[i];
-    for (uint32_t i = threadIdx.x; i <= (uint32_t)N; i += 256) ub[i] = src.ubase[i];
-    // a plan that turned out not to be this batch's: nothing to do (the host analyses the batch itself)
+    const uint32_t nb = b.buckets();
+    // (the workgroups whose chains are the longest first)
+    const uint32_t c = blockIdx.x % nb, role = gridDim.x / nb - 1 - blockIdx.x / nb;
+    const int sub = threadIdx.x % LPG;
+    const uint32_t g0 = threadIdx.x / LPG;
+    const size_t first = (size_t)c * b.cap;
+    // the first sign and record of a group of lanes before the bucket's counts are known: one round trip less
+    const uint4 head = p.head[c];
+    uint2 gr = make_uint2(NO_ROW, 0);
+    uint4 mem = make_uint4(0, 0, 0, 0);
+    if (role == 0) {
+        gr = p.group[first + min(g0, b.cap - 1)];
+        mem = p.member[first + min(g0, b.cap - 1)];
+    }
     const uint32_t stop = status->mismatch | status->abort;
-    const uint32_t n_single = status->n_single, n_multi = status->n_multi;
-    __syncthreads();
+    const float** grads = reinterpret_cast<const float**>(apply_lds);
+    uint32_t* rows = reinterpret_cast<uint32_t*>(grads + (flat ? 0 : b.N));
+    if (!flat) {
+        for (uint32_t i = threadIdx.x; i < (uint32_t)b.N; i += 256) {
+            grads[i] = p.push_descs[i].grads;
+            rows[i] = (uint32_t)min(p.push_descs[i].rows, (int64_t)SMALL_SLOT_MAX + 1);
+        }
+        __syncthreads();
+    }
+    // a plan that turned out not to be this batch's: nothing to do (the host analyses the batch itself)
     if (stop) return;
-    src.descs = sd;
-    src.ubase = ub;
-    if (blockIdx.x < big_blocks) {
+    SmallSrc src;
+    src.grads = grads;
+    src.rows = rows;
+    src.flat = flat;
+    src.click_at = p.click_at;
+    src.dim = dim;
+    const int lane0 = (int)__lane_id() - sub;
+    const float c1 = 1 - o.beta1, c2 = 1 - o.beta2;
+    if (role == 2) {
         const int wave = (int)(threadIdx.x >> 6), lane = (int)(threadIdx.x & 63);
-        char* base = reinterpret_cast<char*>(big_lds) + (size_t)wave * wave_lds;  // (wave_arrays: where the arrays start in it)
+        char* base = reinterpret_cast<char*>(apply_lds) + small_apply_slots_lds(flat ? 0 : b.N) + (size_t)wave * wave_lds;
         float* gbuf = reinterpret_cast<float*>(base);
         const float** gptr = reinterpret_cast<const float**>(base + wave_arrays);
         int* gshow = reinterpret_cast<int*>(gptr + BIG_CHUNK);
         int* gok = gshow + BIG_CHUNK;
         float* den = reinterpret_cast<float*>(gok + BIG_CHUNK);
-        apply_big_groups<KIND>(s, o, src, status, big_list, grp_row, grp_off, grp_cnt, list, gbuf_floats, nullptr, gbuf,
-                               gptr, gshow, gok, den, lane, blockIdx.x * 4 + (uint32_t)wave, big_blocks * 4,
-                               [] { wave_sync(); });
+        apply_big_groups<KIND>(
+            s, o, gbuf_floats, gbuf, gptr, gshow, gok, den, lane, (uint32_t)wave, 4u, head.z,
+            [&](uint32_t bi, uint32_t& row, uint32_t& off, uint32_t& k) {
+                const uint2 g = p.group[first + b.cap - 1 - bi];
+                row = g.x;
+                off = g.y & 0xFFFFu;
+                k = g.y >> 16;
+            },
+            [&](uint32_t at, const float*& gp, int& sh, int& ck) {
+                const uint4 m = p.member[first + at];
+                gp = src.gradient(m);
+                sh = (int)m.z;
+                if (KIND == OPT_ADAGRAD) {
+                    ck = src.click(m);
+                    src.click_at[m.x] = 0;
+                }
+                return gp != nullptr;
+            },
+            [] {}, [] { wave_sync(); });
         return;
     }
-    const int sub = threadIdx.x % LPG;
-    const int lane0 = (int)__lane_id() - sub;
-    const uint32_t gstride = (gridDim.x - big_blocks) * (blockDim.x / LPG);
-    const float c1 = 1 - o.beta1, c2 = 1 - o.beta2;
-    for (uint32_t t = (blockIdx.x - big_blocks) * (blockDim.x / LPG) + threadIdx.x / LPG; t < n_single + n_multi; t += gstride) {
-        const uint32_t g = group_id(t, n_single, n_multi, ids_cap);
-        const uint32_t row = grp_row[g];
-        if (row > s.cap) continue;  // NO_ROW, or no row number at all: never address the table with it
-        const uint32_t k = grp_cnt[g];
-        if (is_big(k, big_k)) continue;
-        apply_group_vec<KIND, LPG, ANY, 4>(s, o, src, status, row, k, list + grp_off[g], nullptr, sub, lane0, c1, c2);
+    if (role == 1) {
+        for (uint32_t g = g0; g < head.y; g += 256 / LPG) {
+            const uint2 d = p.group[first + head.x + g];
+            if (d.x > s.cap) continue;  // no row number at all: never address the table with it
+            small_apply_group<KIND, LPG, ANY, 4>(s, o, src, d.x, d.y >> 16, p.member + first + (d.y & 0xFFFFu), sub, lane0, c1, c2);
+        }
+        return;
+    }
+    for (uint32_t g = g0; g < head.x; g += 256 / LPG) {
+        if (g != g0) {
+            gr = p.group[first + g];
+            mem = p.member[first + g];
+        }
+        if (gr.x > s.cap) continue;
+        const float* gp = src.gradient(mem);
+        if (!gp) continue;
+        int ck = 0;
+        if (KIND == OPT_ADAGRAD) ck = src.click(mem);
+        apply_one_record<KIND, LPG, ANY>(s, o, gr.x, gp, (int)mem.z, ck, sub, lane0, c1, c2);
+        if (KIND == OPT_ADAGRAD && sub == 0) src.click_at[mem.x] = 0;
     }
 }
 

@@ -1494,6 +1494,63 @@ __device__ __forceinline__ void put_row_part(float* p, int sub, int D, float4 v)
     }
 }
 
+// One record applied to its sign's row by LPG lanes: gradient, row and state once.
+template <int KIND, int LPG, bool ANY>
+__device__ __forceinline__ void apply_one_record(const Store& s, const OptDev& o, uint32_t row, const float* gp, int bshow,
+                                                 int bclick, int sub, int lane0, float c1, float c2) {
+    const int D = s.D;
+    float* wp = s.w + (uint64_t)row * s.wstride;
+    float* sp = s.st + (uint64_t)row * s.sstride;
+    const float4 gr = row_part<ANY>(gp, sub, D);
+    float4 w = row_part<ANY>(wp, sub, D);
+    if (KIND == OPT_ADAGRAD) {
+        const float4 h = *reinterpret_cast<const float4*>(sp);
+        const float p0 = gr.x * gr.x, p1 = gr.y * gr.y, p2 = gr.z * gr.z, p3 = gr.w * gr.w;
+        double tot = 0.0;  // add_g2sum: double accumulator over the float products, element order 0..D-1
+        for (int l = 0; l < LPG; l++) {
+            double cand = tot;
+            cand += (double)p0;
+            cand += (double)p1;
+            cand += (double)p2;
+            cand += (double)p3;
+            tot = __shfl(cand, lane0 + l);
+        }
+        const float g2sum = (float)((double)h.x + tot / (double)D);
+        const float den = o.eps + sqrtf(g2sum);
+        w.x -= o.lr * gr.x / den;
+        w.y -= o.lr * gr.y / den;
+        w.z -= o.lr * gr.z / den;
+        w.w -= o.lr * gr.w / den;
+        put_row_part<ANY>(wp, sub, D, w);
+        if (sub == 0) {
+            const float show = h.y + (float)bshow, click = h.z + (float)bclick;
+            *reinterpret_cast<float4*>(sp) = make_float4(g2sum, show, click, 0.f);  // no_show_days = 0
+            if (o.use_cvm) {
+                wp[D] = show;
+                wp[D + 1] = logf(click + 1) - logf(show + 1);
+            }
+        }
+    } else {
+        float4 a = row_part<ANY>(sp, sub, D);
+        float4 b = row_part<ANY>(sp + D, sub, D);
+        if (KIND == OPT_ADAM) {
+            adam_elem(o, c1, c2, gr.x, w.x, a.x, b.x);
+            adam_elem(o, c1, c2, gr.y, w.y, a.y, b.y);
+            adam_elem(o, c1, c2, gr.z, w.z, a.z, b.z);
+            adam_elem(o, c1, c2, gr.w, w.w, a.w, b.w);
+        } else {
+            ftrl_elem(o, gr.x, w.x, a.x, b.x);
+            ftrl_elem(o, gr.y, w.y, a.y, b.y);
+            ftrl_elem(o, gr.z, w.z, a.z, b.z);
+            ftrl_elem(o, gr.w, w.w, a.w, b.w);
+        }
+        put_row_part<ANY>(wp, sub, D, w);
+        put_row_part<ANY>(sp, sub, D, a);
+        put_row_part<ANY>(sp + D, sub, D, b);
+        if (sub == 0) sp[2 * D + 1] = __int_as_float(__float_as_int(sp[2 * D + 1]) + bshow);
+    }
+}
+
 // Most signs occur in one slot only: one record, no ordering problem, no
 // loop.  LPG lanes update the row of one such sign; its member entry sits at
 // the place of its group number.
@@ -1504,7 +1561,6 @@ __global__ __launch_bounds__(256) void k_apply_single(Store s, OptDev o, PushSrc
     // a push launched on a plan that turned out not to be its batch's (the host redoes it), or whose inputs are unusable
     if (status->mismatch | status->abort) return;
     const uint32_t n_single = status->n_single;
-    const int D = s.D;
     const int sub = threadIdx.x % LPG;
     const int lane0 = (int)__lane_id() - sub;
     const uint32_t gstride = gridDim.x * (blockDim.x / LPG);
@@ -1518,56 +1574,7 @@ __global__ __launch_bounds__(256) void k_apply_single(Store s, OptDev o, PushSrc
             if (sub == 0) atomicOr(&status->err, DEV_ERR_GRAD_ROWS);
             continue;
         }
-        float* wp = s.w + (uint64_t)row * s.wstride;
-        float* sp = s.st + (uint64_t)row * s.sstride;
-        const float4 gr = row_part<ANY>(gp, sub, D);
-        float4 w = row_part<ANY>(wp, sub, D);
-        if (KIND == OPT_ADAGRAD) {
-            const float4 h = *reinterpret_cast<const float4*>(sp);
-            const float p0 = gr.x * gr.x, p1 = gr.y * gr.y, p2 = gr.z * gr.z, p3 = gr.w * gr.w;
-            double tot = 0.0;  // add_g2sum: double accumulator over the float products, element order 0..D-1
-            for (int l = 0; l < LPG; l++) {
-                double cand = tot;
-                cand += (double)p0;
-                cand += (double)p1;
-                cand += (double)p2;
-                cand += (double)p3;
-                tot = __shfl(cand, lane0 + l);
-            }
-            const float g2sum = (float)((double)h.x + tot / (double)D);
-            const float den = o.eps + sqrtf(g2sum);
-            w.x -= o.lr * gr.x / den;
-            w.y -= o.lr * gr.y / den;
-            w.z -= o.lr * gr.z / den;
-            w.w -= o.lr * gr.w / den;
-            put_row_part<ANY>(wp, sub, D, w);
-            if (sub == 0) {
-                const float show = h.y + (float)bshow, click = h.z + (float)bclick;
-                *reinterpret_cast<float4*>(sp) = make_float4(g2sum, show, click, 0.f);  // no_show_days = 0
-                if (o.use_cvm) {
-                    wp[D] = show;
-                    wp[D + 1] = logf(click + 1) - logf(show + 1);
-                }
-            }
-        } else {
-            float4 a = row_part<ANY>(sp, sub, D);
-            float4 b = row_part<ANY>(sp + D, sub, D);
-            if (KIND == OPT_ADAM) {
-                adam_elem(o, c1, c2, gr.x, w.x, a.x, b.x);
-                adam_elem(o, c1, c2, gr.y, w.y, a.y, b.y);
-                adam_elem(o, c1, c2, gr.z, w.z, a.z, b.z);
-                adam_elem(o, c1, c2, gr.w, w.w, a.w, b.w);
-            } else {
-                ftrl_elem(o, gr.x, w.x, a.x, b.x);
-                ftrl_elem(o, gr.y, w.y, a.y, b.y);
-                ftrl_elem(o, gr.z, w.z, a.z, b.z);
-                ftrl_elem(o, gr.w, w.w, a.w, b.w);
-            }
-            put_row_part<ANY>(wp, sub, D, w);
-            put_row_part<ANY>(sp, sub, D, a);
-            put_row_part<ANY>(sp + D, sub, D, b);
-            if (sub == 0) sp[2 * D + 1] = __int_as_float(__float_as_int(sp[2 * D + 1]) + bshow);
-        }
+        apply_one_record<KIND, LPG, ANY>(s, o, row, gp, bshow, bclick, sub, lane0, c1, c2);
     }
 }
 
@@ -1576,12 +1583,7 @@ __global__ __launch_bounds__(256) void k_apply_single(Store s, OptDev o, PushSrc
 // is sorted) and stores the row once.  Each lane holds one float4 of every
 // per-element array; the next record's gradient is fetched while the current
 // one is applied.  Groups with big_k records or more are left to k_apply_big.
-// AHEAD = 1: the next record's gradient is fetched while the current one is applied (what keeps the most
-// wavefronts on a CU: the kernels of a large batch).  AHEAD > 1: records are taken AHEAD at a time, the gradients
-// of the next AHEAD and the member entries of the AHEAD after those in flight meanwhile: a chain of k records
-// costs k / AHEAD round trips instead of 2 k, which is what a small batch, whose kernels are as long as their
-// longest chain, is after.
-template <int KIND, int LPG, bool ANY, int AHEAD = 1>
+template <int KIND, int LPG, bool ANY>
 __device__ __forceinline__ void apply_group_vec(const Store& s, const OptDev& o, const PushSrc& src, DevStatus* status,
                                                 uint32_t row, uint32_t k, const Member* mem, const float* const* ga,
                                                 int sub, int lane0, float c1, float c2) {
@@ -1643,145 +1645,24 @@ __device__ __forceinline__ void apply_group_vec(const Store& s, const OptDev& o,
     auto no_gradient = [&]() {
         if (sub == 0) atomicOr(&status->err, DEV_ERR_GRAD_ROWS);
     };
-    if (AHEAD == 1) {
-        const float* gp;
-        int nshow = 0, nclick = 0;
-        bool nok = record_at(src, mem, ga, 0, gp, nshow, nclick);
-        float4 gnext = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (nok) gnext = row_part<ANY>(gp, sub, D);
-        for (uint32_t j = 0; j < k; j++) {
-            const float4 gr = gnext;
-            const int bshow = nshow, bclick = nclick;
-            const bool ok = nok;
-            if (j + 1 < k) {
-                nok = record_at(src, mem, ga, j + 1, gp, nshow, nclick);
-                if (nok) gnext = row_part<ANY>(gp, sub, D);
-            }
-            if (!ok) {
-                no_gradient();
-                continue;
-            }
-            step(gr, bshow, bclick);
+    const float* gp;
+    int nshow = 0, nclick = 0;
+    bool nok = record_at(src, mem, ga, 0, gp, nshow, nclick);
+    float4 gnext = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (nok) gnext = row_part<ANY>(gp, sub, D);
+    for (uint32_t j = 0; j < k; j++) {
+        const float4 gr = gnext;
+        const int bshow = nshow, bclick = nclick;
+        const bool ok = nok;
+        if (j + 1 < k) {
+            nok = record_at(src, mem, ga, j + 1, gp, nshow, nclick);
+            if (nok) gnext = row_part<ANY>(gp, sub, D);
         }
-    } else {
-        // chunk c: applied; chunk c + 1: gradients in flight; chunk c + 2: member entries in flight.  Every load is
-        // issued whether its record exists or not (past the end: the group's last member again, the row in place of
-        // a gradient): a load under a condition makes the compiler wait for all loads where the branches join.
-        Member m1[AHEAD], m2[AHEAD];
-        const float* a1[AHEAD];  // with ga: the records' gradient addresses, worked out beforehand
-        const float* a2[AHEAD];
-        float4 g0[AHEAD], g1[AHEAD];
-        int sh0[AHEAD], ck0[AHEAD], sh1[AHEAD], ck1[AHEAD];
-        bool ok0[AHEAD], ok1[AHEAD];
-        auto fetch = [&](const Member (&m)[AHEAD], const float* const (&a)[AHEAD], uint32_t first, float4 (&g)[AHEAD],
-                         int (&sh)[AHEAD], int (&ck)[AHEAD], bool (&ok)[AHEAD]) {
-#pragma unroll
-            for (int q = 0; q < AHEAD; q++) {
-                const float* gp = nullptr;
-                if (ga) {
-                    gp = a[q];
-                    sh[q] = m[q].show;
-                    ck[q] = m[q].click;
-                    ok[q] = gp != nullptr && first + q < k;
-                } else {
-                    ok[q] = src_record(src, m[q], gp, sh[q], ck[q]) && first + q < k;
-                }
-                g[q] = row_part<ANY>(ok[q] ? gp : wp, sub, D);
-            }
-        };
-#pragma unroll
-        for (int q = 0; q < AHEAD; q++) {
-            m1[q] = mem[min((uint32_t)q, k - 1)];
-            m2[q] = mem[min((uint32_t)(AHEAD + q), k - 1)];
-            a1[q] = ga ? ga[min((uint32_t)q, k - 1)] : nullptr;
-            a2[q] = ga ? ga[min((uint32_t)(AHEAD + q), k - 1)] : nullptr;
+        if (!ok) {
+            no_gradient();
+            continue;
         }
-        fetch(m1, a1, 0, g0, sh0, ck0, ok0);
-#pragma unroll
-        for (int q = 0; q < AHEAD; q++) {
-            m1[q] = m2[q];
-            a1[q] = a2[q];
-        }
-        for (uint32_t c0 = 0; c0 < k; c0 += AHEAD) {
-#pragma unroll
-            for (int q = 0; q < AHEAD; q++) {
-                m2[q] = mem[min(c0 + 2 * AHEAD + q, k - 1)];
-                a2[q] = ga ? ga[min(c0 + 2 * AHEAD + q, k - 1)] : nullptr;
-            }
-            fetch(m1, a1, c0 + AHEAD, g1, sh1, ck1, ok1);
-            if constexpr (KIND == OPT_ADAGRAD) {
-                // The records of the window depend on each other through g2sum (one rounded addition per record)
-                // and through the row (one subtraction per element and record) only.  Everything else -- the sums of
-                // squares with their hand-over from lane to lane, the square roots, the divisions -- is worked
-                // out for all records of the window side by side; the two chains then run over the results, in
-                // record order.  The same operations on the same operands as record after record.
-                double mq[AHEAD];
-#pragma unroll
-                for (int q = 0; q < AHEAD; q++) mq[q] = 0.0;
-                for (int l = 0; l < LPG; l++) {
-#pragma unroll
-                    for (int q = 0; q < AHEAD; q++) {
-                        double cand = mq[q];  // add_g2sum: double accumulator over the float products, element order 0..D-1
-                        cand += (double)(g0[q].x * g0[q].x);
-                        cand += (double)(g0[q].y * g0[q].y);
-                        cand += (double)(g0[q].z * g0[q].z);
-                        cand += (double)(g0[q].w * g0[q].w);
-                        mq[q] = __shfl(cand, lane0 + l);
-                    }
-                }
-#pragma unroll
-                for (int q = 0; q < AHEAD; q++) mq[q] = mq[q] / (double)D;
-                float g2[AHEAD];
-                bool missing = false;
-#pragma unroll
-                for (int q = 0; q < AHEAD; q++) {
-                    if (ok0[q]) {
-                        any = true;
-                        show += (float)sh0[q];
-                        click += (float)ck0[q];
-                        g2sum = (float)((double)g2sum + mq[q]);
-                    } else if (c0 + q < k) {
-                        missing = true;
-                    }
-                    g2[q] = g2sum;
-                }
-                float4 st4[AHEAD];
-#pragma unroll
-                for (int q = 0; q < AHEAD; q++) {
-                    const float den = o.eps + sqrtf(g2[q]);
-                    st4[q] = make_float4(o.lr * g0[q].x / den, o.lr * g0[q].y / den, o.lr * g0[q].z / den,
-                                         o.lr * g0[q].w / den);
-                }
-#pragma unroll
-                for (int q = 0; q < AHEAD; q++) {
-                    if (!ok0[q]) continue;
-                    w.x -= st4[q].x;
-                    w.y -= st4[q].y;
-                    w.z -= st4[q].z;
-                    w.w -= st4[q].w;
-                }
-                if (missing) no_gradient();
-            } else {
-#pragma unroll
-                for (int q = 0; q < AHEAD; q++) {
-                    if (c0 + q >= k) break;
-                    if (!ok0[q]) {
-                        no_gradient();
-                        continue;
-                    }
-                    step(g0[q], sh0[q], ck0[q]);
-                }
-            }
-#pragma unroll
-            for (int q = 0; q < AHEAD; q++) {
-                g0[q] = g1[q];
-                sh0[q] = sh1[q];
-                ck0[q] = ck1[q];
-                ok0[q] = ok1[q];
-                m1[q] = m2[q];
-                a1[q] = a2[q];
-            }
-        }
+        step(gr, bshow, bclick);
     }
     if (!any) return;
     put_row_part<ANY>(wp, sub, D, w);
@@ -1855,28 +1736,22 @@ inline size_t big_lds_bytes(int D) { return (size_t)(big_gbuf_floats(D) + 3 * D)
 // then the records are applied strictly in order -- for AdaGrad the g2sum
 // chain by one lane, the square roots by one lane per record, the element
 // updates by one lane per element.
-// The groups big_list[first], big_list[first + stride], ... by the wavefront that calls it (lane = the thread's
-// lane).  gbuf: gbuf_floats floats of staging followed by the row (rw[D], ra[D], rb[D]); gptr, gshow, gok,
-// den: BIG_CHUNK entries each, all in LDS and the wavefront's own.  sync(): makes what the lanes wrote to that
-// LDS visible to each other (a workgroup of one wavefront: __syncthreads; a wavefront among others: wave_sync).
-template <int KIND, typename Sync>
-__device__ __forceinline__ void apply_big_groups(const Store& s, const OptDev& o, const PushSrc& src, DevStatus* status,
-                                                 const uint32_t* __restrict__ big_list,
-                                                 const uint32_t* __restrict__ grp_row,
-                                                 const uint32_t* __restrict__ grp_off,
-                                                 const uint32_t* __restrict__ grp_cnt,
-                                                 const Member* __restrict__ list, int gbuf_floats,
-                                                 const float* const* __restrict__ gaddr, float* gbuf, const float** gptr,
-                                                 int* gshow, int* gok, float* den, int lane, uint32_t first,
-                                                 uint32_t stride, Sync sync) {
+// The groups first, first + stride, ... below n_big by the wavefront that calls it (lane = the thread's lane).  gbuf:
+// gbuf_floats floats of staging followed by the row (rw[D], ra[D], rb[D]); gptr, gshow, gok, den: BIG_CHUNK entries
+// each, all in LDS and the wavefront's own.  group(bi, row, off, k): the bi-th group's row, first member and records;
+// record(at, gp, show, click): gradient row and counts of member `at`, false if it has no gradient; missing(): a
+// record without one was met; sync(): makes what the lanes wrote to that LDS visible to each other (a workgroup of
+// one wavefront: __syncthreads; a wavefront among others: wave_sync).
+template <int KIND, typename Group, typename Record, typename Missing, typename Sync>
+__device__ __forceinline__ void apply_big_groups(const Store& s, const OptDev& o, int gbuf_floats, float* gbuf,
+                                                 const float** gptr, int* gshow, int* gok, float* den, int lane,
+                                                 uint32_t first, uint32_t stride, uint32_t n_big, Group group, Record record,
+                                                 Missing missing, Sync sync) {
     const int D = s.D;
     float* rw = gbuf + gbuf_floats;
     float* ra = rw + D;
     float* rb = ra + D;
     const int Dp = D + 1;  // padded staging row: lanes walking down a column hit different banks
-    // a push launched on a plan that turned out not to be its batch's (the host redoes it), or whose inputs are unusable
-    if (status->mismatch | status->abort) return;
-    const uint32_t n_big = status->n_big;
     const int per_chunk = (gbuf_floats / Dp) < BIG_CHUNK ? (gbuf_floats / Dp) : BIG_CHUNK;
     const float c1 = 1 - o.beta1, c2 = 1 - o.beta2;
     const bool pow2 = (D & (D - 1)) == 0;
@@ -1885,11 +1760,9 @@ __device__ __forceinline__ void apply_big_groups(const Store& s, const OptDev& o
     const bool tiled = D <= 64 && 64 % D == 0;
     const int li = tiled ? lane % D : 0, lm = tiled ? lane / D : 0, mstep = tiled ? 64 / D : 1;
     for (uint32_t bi = first; bi < n_big; bi += stride) {
-        const uint32_t g = big_list[bi];
-        const uint32_t row = grp_row[g];
+        uint32_t row, off, k;
+        group(bi, row, off, k);
         if (row > s.cap) continue;  // NO_ROW, or no row number at all: never address the table with it
-        const uint32_t k = grp_cnt[g];
-        const uint32_t off = grp_off[g];
         float* wp = s.w + (uint64_t)row * s.wstride;
         float* sp = s.st + (uint64_t)row * s.sstride;
         for (int i = lane; i < D; i += 64) {
@@ -1918,7 +1791,7 @@ __device__ __forceinline__ void apply_big_groups(const Store& s, const OptDev& o
             int sh = 0, ck = 0;
             if (lane < cn) {
                 const float* gp = nullptr;
-                ok = record_at(src, list + off + c0, gaddr ? gaddr + off + c0 : nullptr, lane, gp, sh, ck);
+                ok = record(off + c0 + (uint32_t)lane, gp, sh, ck);
                 gptr[lane] = gp;
                 gshow[lane] = sh;
                 gok[lane] = ok ? 1 : 0;
@@ -2023,7 +1896,7 @@ __device__ __forceinline__ void apply_big_groups(const Store& s, const OptDev& o
             }
             const unsigned long long chunk_mask = cn == 64 ? ~0ull : (1ull << cn) - 1ull;
             if (okmask) any = true;
-            if (lane == 0 && okmask != chunk_mask) atomicOr(&status->err, DEV_ERR_GRAD_ROWS);
+            if (lane == 0 && okmask != chunk_mask) missing();
             sync();
         }
         if (any) {
@@ -2072,8 +1945,18 @@ __global__ __launch_bounds__(64) void k_apply_big(Store s, OptDev o, PushSrc src
     __shared__ const float* gptr[BIG_CHUNK];
     __shared__ int gshow[BIG_CHUNK], gok[BIG_CHUNK];
     __shared__ float den[BIG_CHUNK];
-    apply_big_groups<KIND>(s, o, src, status, big_list, grp_row, grp_off, grp_cnt, list, gbuf_floats, gaddr, gbuf, gptr,
-                           gshow, gok, den, (int)threadIdx.x, blockIdx.x, gridDim.x, [] { __syncthreads(); });
+    // a push launched on a plan that turned out not to be its batch's (the host redoes it), or whose inputs are unusable
+    if (status->mismatch | status->abort) return;
+    apply_big_groups<KIND>(
+        s, o, gbuf_floats, gbuf, gptr, gshow, gok, den, (int)threadIdx.x, blockIdx.x, gridDim.x, status->n_big,
+        [&](uint32_t bi, uint32_t& row, uint32_t& off, uint32_t& k) {
+            const uint32_t g = big_list[bi];
+            row = grp_row[g];
+            off = grp_off[g];
+            k = grp_cnt[g];
+        },
+        [&](uint32_t at, const float*& gp, int& sh, int& ck) { return record_at(src, list, gaddr, at, gp, sh, ck); },
+        [&] { atomicOr(&status->err, DEV_ERR_GRAD_ROWS); }, [] { __syncthreads(); });
 }
 
 // k_apply_big for AdaGrad rows of D elements, D a power of two from 4 to 64, on a plan whose big_desc lists

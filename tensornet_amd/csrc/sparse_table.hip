@@ -38,16 +38,16 @@ constexpr int GRID_CAP = 256 * 8;                       // 256 CUs x 8 workgroup
 constexpr int TILE_GRID = 256 * 3;                      // workgroups of k_tile_dedup: what the chip holds of it at once
 constexpr size_t LDS_MIN_LOOKUPS = 1024;  // from here on the remap through LDS wins: it also takes fewer launches (cfg1, 8 k lookups: 0.154 -> 0.136 ms)
 
-// Up to this many lookups a batch whose slots each fit one workgroup (SMALL_SLOT_MAX lookups, SMALL_SLOTS slots)
-// takes the path of few launches (small_batch.h).
-constexpr size_t SMALL_MAX_LOOKUPS = 1u << 18;
+// Up to this many lookups a batch whose slots are all short (SMALL_SLOT_MAX lookups, SMALL_SLOTS slots) takes the path
+// of few launches (small_batch.h).
+constexpr size_t SMALL_MAX_LOOKUPS = 1u << 20;
 
 // A small batch of at most this many slots leaves every sign to the lane groups of k_small_apply.  With more slots a
-// sign with SMALL_BIG_GROUP records or more is taken by a wavefront of its own (the first workgroups of the same
-// launch): a small batch's kernels are as long as their longest chain, and the records of a sign applied one after
-// the other by a lane group (four elements per lane) take four times as long as by a wavefront with a lane per
-// element (measured, 4096 x 26 slots, Adam: the updates take 0.040 ms with every sign left to the lane groups,
-// 0.020 ms with the threshold at 5; 1024 x 8 slots: no difference between 4 and 12 slots here).
+// sign with SMALL_BIG_GROUP records or more is taken by a wavefront of its own: a small batch's kernels are as long as
+// their longest chain, and the records of a sign applied one after the other by a lane group (four elements per lane)
+// take four times as long as by a wavefront with a lane per element (measured, 4096 x 26 slots, Adam: the updates take
+// 0.040 ms with every sign left to the lane groups, 0.020 ms with the threshold at 5; 1024 x 8 slots: no difference
+// between 4 and 12 slots here).
 constexpr int SMALL_NO_BIG_SLOTS = 12;
 constexpr uint32_t SMALL_BIG_GROUP = 5;
 constexpr uint32_t BIG_GROUP_DEFAULT = 16;
@@ -93,15 +93,15 @@ struct SparseTable {
     DevBuf comb_buf;                // slot descriptors of a combine op
     DevBuf pooled_ws;               // scratch of a push of pooled gradients (ordered lookups, reduced rows)
     size_t place_lds = 0, huge_lds = 0;  // dynamic LDS of k_place_lookups / k_order_huge on this device (0: not asked yet)
-    // The path of few launches for small batches: its device state, the words in pinned memory its kernels
-    // report through ([0] a pull's status is on the host, [1] a push's signs are compared) with the numbers the
-    // host expects there next, the dynamic LDS k_small_slots may have.
-    SmallState* small_state = nullptr;
+    // The path of few launches for small batches: the words in pinned memory its kernels report through (hwords: one
+    // per workgroup of a pull's first launch; hseq [0] a large pull's status is on the host, [1] a push's signs are
+    // compared) with the numbers the host expects there next, the dynamic LDS its kernels may have.
+    uint64_t* hwords = nullptr;
     uint32_t* hseq = nullptr;
     uint32_t seq_pull = 0, seq_verify = 0;
     std::vector<int64_t> plan_counts;  // distinct signs per slot of the small pull that left the plan
-    uint32_t small_calls = 0;  // (its parity: which set of bucket cursors the next small pull uses)
-    size_t small_lds = 0;
+    SmallShape small_shape{};          // how that pull laid its batch out
+    size_t small_lds = 0, small_emit_lds = 0;
     bool plan_small = false;   // the plan was left by a small pull: a push may take the small path, too
     bool plan_prints = false;  // the plan holds fingerprints of the batch's signs, not a copy of them
     bool exact_verify = false; // pulls that leave fingerprints keep a copy of the signs as well, pushes compare that
@@ -286,8 +286,8 @@ int ensure_side_buffers(SparseTable* t) {
     TN_HIP(hipHostMalloc((void**)&t->hcount, 64, hipHostMallocDefault));
     TN_HIP(hipHostMalloc((void**)&t->hseq, 64, hipHostMallocDefault));
     std::memset(t->hseq, 0, 64);
-    TN_HIP(hipMalloc((void**)&t->small_state, sizeof(SmallState)));
-    TN_HIP(hipMemset(t->small_state, 0, sizeof(SmallState)));
+    TN_HIP(hipHostMalloc((void**)&t->hwords, SMALL_WORKGROUPS * sizeof(uint64_t), hipHostMallocDefault));
+    std::memset(t->hwords, 0, SMALL_WORKGROUPS * sizeof(uint64_t));
     t->hstage_bytes = (size_t)MAX_SLOTS * sizeof(SlotDesc) + (MAX_SLOTS + 1) * sizeof(uint32_t);
     TN_HIP(hipHostMalloc((void**)&t->hstage, t->hstage_bytes, hipHostMallocDefault));
     TN_HIP(hipEventCreateWithFlags(&t->stage_ev, hipEventDisableTiming));
@@ -375,6 +375,18 @@ void latch(SparseTable* t, int code, const std::string& msg) {
     }
 }
 
+// CHECK_LT(signs.size(), max_var_count), sparse_table_ops.cc:136
+void latch_var_capacity(SparseTable* t, int slot, int64_t rows) {
+    latch(t, TN_ERR_VAR_CAPACITY,
+          "sparse pull: slot " + std::to_string(slot) + " has " + std::to_string(t->last_counts[slot]) +
+              " distinct signs, its variable only " + std::to_string(rows) + " rows");
+}
+
+// The share of distinct records among a pull's lookups: rises at once, falls within about ten pulls.
+void note_distinct_share(SparseTable* t, double now) {
+    t->distinct_est = std::min(1.0, std::max(now, 0.75 * t->distinct_est + 0.25 * now));
+}
+
 // Examines the status blocks of finished calls (the stream must have been synchronised).
 void harvest(SparseTable* t) {
     // a pending push is older than a pending pull (a push collects everything before it starts)
@@ -403,9 +415,8 @@ void harvest(SparseTable* t) {
         t->booked = 0;
         t->last_counts.assign(N, 0);
         for (int s = 0; s < N; s++) t->last_counts[s] = (int64_t)h.ubase[s + 1] - (int64_t)h.ubase[s];
-        if (t->pull_lookups > 0) {  // rises at once, falls within about ten pulls
-            const double now = (double)h.ubase[N] / (double)t->pull_lookups;
-            t->distinct_est = std::min(1.0, std::max(now, 0.75 * t->distinct_est + 0.25 * now));
+        if (t->pull_lookups > 0) {
+            note_distinct_share(t, (double)h.ubase[N] / (double)t->pull_lookups);
             if (h.st.tile_share_q16 != 0) {  // (a pull through LDS with a slot of more than one bucket)
                 const double share = (double)h.st.tile_share_q16 / 65536.0;
                 t->tile_est = std::min(1.0, std::max(share, 0.75 * t->tile_est + 0.25 * share));
@@ -413,10 +424,7 @@ void harvest(SparseTable* t) {
         }
         latch(t, dev_err_code(h.st.err), std::string("sparse pull: ") + dev_err_text(h.st.err));
         for (int s = 0; s < N && s < (int)t->pending_rows.size(); s++)
-            if (t->last_counts[s] >= t->pending_rows[s])  // CHECK_LT(signs.size(), max_var_count)
-                latch(t, TN_ERR_VAR_CAPACITY,
-                      "sparse pull: slot " + std::to_string(s) + " has " + std::to_string(t->last_counts[s]) +
-                          " distinct signs, its variable only " + std::to_string(t->pending_rows[s]) + " rows");
+            if (t->last_counts[s] >= t->pending_rows[s]) latch_var_capacity(t, s, t->pending_rows[s]);
     }
 }
 
@@ -579,7 +587,7 @@ void carve_groups(Carver& c, Plan& p, size_t n) {
     p.grp_cnt = c.take<uint32_t>(n);
     p.list = c.take<Member>(n);
     p.where_u = c.take<uint2>(n);
-    p.big_cap = (uint32_t)(n / std::min<uint32_t>(BIG_GROUP, SMALL_BIG_GROUP) + 64);  // (the lowest threshold a plan may use)
+    p.big_cap = (uint32_t)(n / BIG_GROUP + 64);
     p.big_list = c.take<uint32_t>(p.big_cap);
     p.big_desc = c.take<uint4>(p.big_cap);
     p.gaddr = c.take<const float*>(n);
@@ -889,10 +897,28 @@ int launch_build_plan(SparseTable* t, const Plan& p, const Scratch& w, int N, ui
             TN_HIP(hipStreamWaitEvent(st, t->join_ev, 0));
             TN_HIP(hipStreamWaitEvent(st, t->join2_ev, 0));
         }
-        TN_LAUNCH((k_group_emit<false>), dim3(bblocks), dim3(EMIT_THREADS), st, w.nb2, w.cursor2, w.recs, w.aux,
-                  own_offsets ? nullptr : w.bbase, w.bcounts, w.flag8, w.wordpre, L, big_threshold(s),
-                  p.grp_sign, p.grp_off, p.grp_cnt, p.big_list, p.big_desc, p.list, p.where_u, w.rrow, p.grp_row, ds,
-                  (const uint32_t*)nullptr, 0u);
+        EmitArgs<false> ea;
+        ea.nb2 = w.nb2;
+        ea.cursor2 = w.cursor2;
+        ea.recs = w.recs;
+        ea.aux = w.aux;
+        ea.bbase = own_offsets ? nullptr : w.bbase;
+        ea.bcounts = w.bcounts;
+        ea.flag8 = w.flag8;
+        ea.wordpre = w.wordpre;
+        ea.ids_cap = L;
+        ea.big_k = big_threshold(s);
+        ea.grp_sign = p.grp_sign;
+        ea.grp_off = p.grp_off;
+        ea.grp_cnt = p.grp_cnt;
+        ea.big_list = p.big_list;
+        ea.big_desc = p.big_desc;
+        ea.list = p.list;
+        ea.where_u = p.where_u;
+        ea.rrow = w.rrow;
+        ea.grp_row = p.grp_row;
+        ea.status = ds;
+        TN_LAUNCH((k_group_emit<false>), dim3(bblocks), dim3(EMIT_THREADS), st, ea);
         t->plan_big_desc = true;
         return TN_OK;  // the rows were found beside the grouping
     } else if (N <= MASK_SLOTS)
@@ -1022,27 +1048,21 @@ int launch_apply(SparseTable* t, const Plan& p, const PushSrc& src, DevStatus* d
     }
 }
 
-// The updates of a small push, one launch: the lane groups' workgroups for every group below the plan's threshold
-// and, if the plan lists signs with many records, workgroups whose wavefronts take those (as a kernel of its own
-// after this one, k_apply_big made 4096 x 26 slots, Adam, 0.080 ms per pull + push; beside it on the table's side
-// stream 0.113 ms: the events that fork and join the streams cost more than the overlap wins).
+// The updates of a small push, one launch (k_small_apply), with the workgroups for the signs with many records if the
+// plan lists such.  flat: the reduced rows of pooled gradients, else nullptr.
 template <int KIND>
-int launch_small_apply_kind(SparseTable* t, RowShare share, int N, const OptDev& o, const PushSrc& src, DevStatus* ds,
-                            const Plan& p, int64_t n_upper, hipStream_t st, uint32_t* host_seq, uint32_t seq) {
+int launch_small_apply_kind(SparseTable* t, RowShare share, const OptDev& o, const SmallPlan& p, const float* flat, int dim,
+                            hipStream_t st, uint32_t* host_seq, uint32_t seq) {
     const Store& s = t->store;
-    const uint32_t big_k = t->plan_big_k;
-    const bool with_big = big_k != 0xFFFFFFFFu && (uint32_t)N >= big_k;
-    // (a wavefront per sign with big_k records or more, four to a workgroup, 512 workgroups at most)
-    const int big_blocks = with_big ? launch_grid((n_upper / big_k + 1 + 3) / 4, 1, 512) : 0;
-    const size_t lds = with_big ? small_apply_big_lds(s.D) : 0;
-#define TN_LAUNCH_SMALL_ANY(LPG, ANY)                                                                                 \
-    do {                                                                                                              \
-        const int group_blocks = launch_grid(n_upper * LPG, 256, GRID_CAP * 4);                                       \
-        TN_LAUNCH_LDS((k_small_apply<KIND, LPG, ANY>), dim3(group_blocks + big_blocks), dim3(256), lds, st, s, o, src, N, \
-                      ds, p.grp_row, p.grp_off, p.grp_cnt, p.list, big_k, (uint32_t)n_upper, host_seq, seq,           \
-                      (uint32_t)big_blocks, p.big_list, big_gbuf_floats(s.D), (uint32_t)small_apply_wave_lds(s.D),    \
-                      (uint32_t)align_up(big_lds_bytes(s.D), 8));                                                     \
-    } while (0)
+    const SmallShape& b = t->small_shape;
+    const bool with_big = t->plan_big_k != 0xFFFFFFFFu && (uint32_t)b.N >= t->plan_big_k;
+    const int roles = with_big ? 3 : b.N > 1 ? 2 : 1;
+    const size_t wave_lds = small_apply_wave_lds(s.D);
+    const size_t lds = small_apply_slots_lds(flat ? 0 : b.N) + (with_big ? 4 * wave_lds : 0);
+#define TN_LAUNCH_SMALL_ANY(LPG, ANY)                                                                                  \
+    TN_LAUNCH_LDS((k_small_apply<KIND, LPG, ANY>), dim3(b.buckets() * roles), dim3(256), lds, st, b, p, flat, s, o,    \
+                  (const DevStatus*)t->dplan, host_seq, seq, dim, big_gbuf_floats(s.D), (uint32_t)wave_lds,            \
+                  (uint32_t)align_up(big_lds_bytes(s.D), 8))
 #define TN_LAUNCH_SMALL(LPG)                  \
     do {                                      \
         if (share.any)                        \
@@ -1063,14 +1083,42 @@ int launch_small_apply_kind(SparseTable* t, RowShare share, int N, const OptDev&
     return TN_OK;
 }
 
-int launch_small_apply(SparseTable* t, RowShare share, int N, const PushSrc& src, DevStatus* ds, const Plan& p, int64_t n_upper,
-                       hipStream_t st, uint32_t* host_seq, uint32_t seq) {
+int launch_small_apply(SparseTable* t, RowShare share, const SmallPlan& p, const float* flat, int dim, hipStream_t st,
+                       uint32_t* host_seq, uint32_t seq) {
     const OptDev o = make_optdev(t);
     switch (o.kind) {
-        case OPT_ADAGRAD: return launch_small_apply_kind<OPT_ADAGRAD>(t, share, N, o, src, ds, p, n_upper, st, host_seq, seq);
-        case OPT_ADAM: return launch_small_apply_kind<OPT_ADAM>(t, share, N, o, src, ds, p, n_upper, st, host_seq, seq);
-        default: return launch_small_apply_kind<OPT_FTRL>(t, share, N, o, src, ds, p, n_upper, st, host_seq, seq);
+        case OPT_ADAGRAD: return launch_small_apply_kind<OPT_ADAGRAD>(t, share, o, p, flat, dim, st, host_seq, seq);
+        case OPT_ADAM: return launch_small_apply_kind<OPT_ADAM>(t, share, o, p, flat, dim, st, host_seq, seq);
+        default: return launch_small_apply_kind<OPT_FTRL>(t, share, o, p, flat, dim, st, host_seq, seq);
     }
+}
+
+// The gradients of a small push's distinct signs from pooled ones (k_small_pool).
+int launch_small_pool(SparseTable* t, RowShare share, const SmallPlan& p, int64_t batch, int dim, int combiner, float* flat,
+                      float* partial, hipStream_t st, uint32_t* host_err) {
+    static_assert((int)POOL_SUM == (int)COMBINE_SUM && (int)POOL_MEAN == (int)COMBINE_MEAN && (int)POOL_SQRTN == (int)COMBINE_SQRTN, "");
+    const SmallShape& b = t->small_shape;
+#define TN_LAUNCH_POOL_ANY(LPG, ANY)                                                                                 \
+    TN_LAUNCH((k_small_pool<LPG, ANY>), dim3(b.N), dim3(POOL_THREADS), st, b, p, p.push_descs, batch, dim, t->store.D, \
+              combiner, flat, partial, t->dplan, host_err)
+#define TN_LAUNCH_POOL(LPG)                  \
+    do {                                     \
+        if (share.any)                       \
+            TN_LAUNCH_POOL_ANY(LPG, true);   \
+        else                                 \
+            TN_LAUNCH_POOL_ANY(LPG, false);  \
+    } while (0)
+    switch (share.lanes) {
+        case 1: TN_LAUNCH_POOL(1); break;
+        case 2: TN_LAUNCH_POOL(2); break;
+        case 4: TN_LAUNCH_POOL(4); break;
+        case 8: TN_LAUNCH_POOL(8); break;
+        case 16: TN_LAUNCH_POOL(16); break;
+        default: TN_LAUNCH_POOL(32); break;
+    }
+#undef TN_LAUNCH_POOL
+#undef TN_LAUNCH_POOL_ANY
+    return TN_OK;
 }
 
 // Bytes of dynamic LDS a workgroup of `kernel` may have on this device (128 KB at most), after telling the
@@ -1091,23 +1139,54 @@ size_t big_lds_bytes_for(const void* kernel, size_t cap = 128 * 1024) {
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
-// Entries of the LDS table of k_small_slots for slots of at most max_len lookups (load <= 0.5).
-uint32_t small_entries(size_t max_len) {
-    uint32_t e = 64;
-    while ((size_t)e < 2 * max_len) e *= 2;
-    return e;
+size_t carve_small(char* base, SmallPlan& p, const SmallShape& b) {
+    Carver c{base};
+    const size_t L = b.L, segments = (size_t)b.N * b.parts;
+    p.descs = c.take<SlotDesc>(b.N);
+    p.push_descs = c.take<SlotDesc>(b.N);
+    p.vals_copy = c.take<uint64_t>(L);
+    p.first_of = c.take<uint16_t>(L);
+    p.row_at = c.take<uint32_t>(L);
+    p.rank_at = c.take<uint16_t>(L);
+    p.click_at = c.take<int32_t>(L);
+    p.bits = c.take<uint64_t>(segments * b.words);
+    p.recs = c.take<uint2>(L * b.parts);
+    p.boff = c.take<uint16_t>(segments * (b.nbp + 1));
+    p.head = c.take<uint4>(b.buckets());
+    p.group = c.take<uint2>((size_t)b.buckets() * b.cap);
+    p.member = c.take<uint4>((size_t)b.buckets() * b.cap);
+    p.bad = c.take<uint32_t>(1);
+    return align_up(c.off, 256);
 }
 
-// Does the batch qualify for the path of few launches?  (nb2: its second-level buckets.)
-bool small_batch_fits(SparseTable* t, int N, const int64_t* lens, size_t L, uint32_t nb2) {
-    if (!t->small_path || t->async_pull || N > SMALL_SLOTS || L == 0 || L > SMALL_MAX_LOOKUPS || nb2 > (uint32_t)SMALL_NB2_MAX) return false;
-    size_t max_len = 0;
-    for (int s = 0; s < N; s++) max_len = std::max<size_t>(max_len, (size_t)lens[s]);
-    if (max_len > (size_t)SMALL_SLOT_MAX) return false;
-    if (!t->small_lds)
-        t->small_lds = big_lds_bytes_for(reinterpret_cast<const void*>(k_small_slots),
-                                         small_slots_lds(small_entries(SMALL_SLOT_MAX), SMALL_NB2_MAX));
-    return small_slots_lds(small_entries(max_len), nb2) <= t->small_lds;
+// Does the batch qualify for the path of few launches, and how is it laid out on it?
+bool small_batch_shape(SparseTable* t, int N, const int64_t* lens, SmallShape& b) {
+    if (!t->small_path || t->async_pull || N <= 0 || N > SMALL_SLOTS || t->dim > 128) return false;
+    size_t L = 0, max_len = 0;
+    for (int s = 0; s < N; s++) {
+        if (lens[s] < 0 || lens[s] > SMALL_SLOT_MAX) return false;
+        L += (size_t)lens[s];
+        max_len = std::max<size_t>(max_len, (size_t)lens[s]);
+    }
+    if (L == 0 || L > SMALL_MAX_LOOKUPS) return false;
+    b.N = N;
+    b.L = (uint32_t)L;
+    b.max_len = (uint32_t)max_len;
+    b.words = (uint32_t)((max_len + 63) / 64);
+    b.parts = (uint32_t)std::min<size_t>(SMALL_PARTS_MAX, (max_len + SMALL_PART_LOOKUPS - 1) / SMALL_PART_LOOKUPS);
+    while (b.parts > 1 && (size_t)N * b.parts > (size_t)SMALL_SEGMENTS) b.parts--;
+    // (every bucket's workgroup looks at all slots: fewer buckets where there are many)
+    const size_t want = std::min<size_t>({(L + SMALL_BUCKET_RECORDS - 1) / SMALL_BUCKET_RECORDS, (size_t)SMALL_BUCKETS_MAX,
+                                          std::max<size_t>(64, (size_t)(1 << 18) / N)});
+    b.nbp = (uint32_t)std::max<size_t>(1, (want + b.parts - 1) / b.parts);
+    // room for twice the records expected of a batch of distinct signs and for four signs that are in every slot
+    b.cap = (uint32_t)align_up(2 * (L / b.buckets()) + 64 + 4 * (size_t)N, 64);
+    if (!t->small_lds) {
+        t->small_lds = big_lds_bytes_for(reinterpret_cast<const void*>(k_small_slots), 144 * 1024);
+        t->small_emit_lds = big_lds_bytes_for(reinterpret_cast<const void*>(k_group_emit<true>), 144 * 1024);
+    }
+    return small_slots_lds(small_entries(b.max_len, b.parts), b.max_len, b.nbp) <= t->small_lds &&
+           small_emit_lds(N, b.cap, small_emit_table(b.cap)) <= t->small_emit_lds;
 }
 
 // Waits for a kernel of the small path to report through pinned memory: *flag == want.  The word is polled for a
@@ -1130,6 +1209,178 @@ int wait_reported(const uint32_t* flag, uint32_t want, hipStream_t st, const cha
     TN_HIP(hipStreamSynchronize(st));
     if (*f != want) return fail(TN_ERR_HIP, std::string(what) + ": the device did not report");
     std::atomic_thread_fence(std::memory_order_acquire);
+    return TN_OK;
+}
+
+// The same for the words of a small pull's first launch: hwords[0 .. n) all carry `seq`.
+int wait_words(const uint64_t* words, uint32_t n, uint32_t seq, hipStream_t st, const char* what) {
+    const volatile uint64_t* w = words;
+    const auto t0 = std::chrono::steady_clock::now();
+    uint32_t i = 0;
+    for (uint32_t spins = 0;; spins++) {
+        while (i < n && (uint32_t)(w[i] >> 32) == seq) i++;
+        if (i == n) return TN_OK;
+        __builtin_ia32_pause();
+        if ((spins & 255u) == 255u && std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(2)) break;
+    }
+    TN_HIP(hipStreamSynchronize(st));
+    while (i < n && (uint32_t)(w[i] >> 32) == seq) i++;
+    return i == n ? TN_OK : fail(TN_ERR_HIP, std::string(what) + ": the device did not report");
+}
+
+// SparseTablePull of a small batch laid out as `b` (the caller has validated the call and made room in the table).
+int small_pull(SparseTable* t, const SmallShape& b, const int64_t* const* values, const int64_t* lens, float* const* vars,
+               const int64_t* var_rows, int wdim, int64_t* const* mapped, hipStream_t st) {
+    const Store& s = t->store;
+    TN_TRY(order_after_updates(t, st));
+    SmallPlan p{};
+    const size_t bytes = carve_small(nullptr, p, b);
+    // (a plan buffer that has to grow is freed first: not under detached updates that still read it)
+    if (t->upd_pending && bytes > t->plan_buf.bytes) TN_HIP(hipEventSynchronize(t->upd_ev));
+    TN_TRY(t->plan_buf.ensure(bytes));
+    carve_small((char*)t->plan_buf.p, p, b);
+    t->plan_valid = false;
+    if (t->stage_pending) {
+        TN_HIP(hipEventSynchronize(t->stage_ev));
+        t->stage_pending = false;
+    }
+    SlotDesc* descs = reinterpret_cast<SlotDesc*>(t->hstage);
+    bool vec = wdim % 4 == 0 && s.wstride % 4 == 0;
+    uint32_t at = 0;
+    for (int i = 0; i < b.N; i++) {
+        SlotDesc d{};
+        d.values = values[i];
+        d.mapped = mapped[i];
+        d.var = vars[i];
+        d.rows = var_rows[i];
+        d.len = (uint32_t)lens[i];
+        d.lbase = at;
+        descs[i] = d;
+        at += d.len;
+        vec = vec && aligned16(vars[i]);
+    }
+    const uint32_t seq = ++t->seq_pull, workgroups = (uint32_t)b.N * b.parts, entries = small_entries(b.max_len, b.parts);
+    TN_LAUNCH_LDS(k_small_slots, dim3(workgroups), dim3(SMALL_THREADS), small_slots_lds(entries, b.max_len, b.nbp), st, b, p,
+                  (const SlotDesc*)descs, entries, s, make_optdev(t), t->seed, t->dplan, t->hwords, seq);
+    const uint32_t per = SMALL_THREADS / (uint32_t)(vec ? wdim / 4 : wdim), chunks = (b.max_len + per - 1) / per;
+    if (vec)
+        TN_LAUNCH((k_small_group_finish<4>), dim3((uint32_t)b.N * chunks), dim3(SMALL_THREADS), st, b, p, chunks, s);
+    else
+        TN_LAUNCH((k_small_group_finish<1>), dim3((uint32_t)b.N * chunks), dim3(SMALL_THREADS), st, b, p, chunks, s);
+    EmitArgs<true> ea;
+    ea.b = b;
+    ea.p = p;
+    ea.table = small_emit_table(b.cap);
+    ea.big_k = t->plan_big_k = b.N <= SMALL_NO_BIG_SLOTS ? 0xFFFFFFFFu : SMALL_BIG_GROUP;
+    TN_LAUNCH_LDS((k_group_emit<true>), dim3(b.buckets()), dim3(EMIT_SMALL_THREADS), small_emit_lds(b.N, b.cap, ea.table), st, ea);
+    TN_HIP(hipGetLastError());
+    // the call returns when the first launch has reported: what follows is complete in stream order
+    TN_HIP(hipEventRecord(t->tail_ev, st));
+    t->tail_recorded = true;
+    t->small_shape = b;
+    t->plan_valid = true;
+    t->plan_small = true;
+    t->plan_clicks_dirty = false;
+    t->plan_has_show = true;
+    t->plan_prints = false;
+    t->plan_exact = false;
+    t->plan_big_desc = false;
+    t->plan_N = b.N;
+    t->plan_lens.assign(lens, lens + b.N);
+    t->plan_epoch = t->epoch;
+    TN_TRY(wait_words(t->hwords, workgroups, seq, st, "SparseTablePull"));
+    harvest(t);  // (a push before this call)
+    uint64_t n_new = 0, n_distinct = 0;
+    bool full = false;
+    constexpr uint64_t MASK = (1u << SMALL_REPORT_BITS) - 1u;
+    t->last_counts.assign(b.N, 0);
+    for (uint32_t i = 0; i < workgroups; i++) {
+        const uint64_t w = t->hwords[i];
+        t->last_counts[i / b.parts] += (int64_t)(w & MASK);
+        n_new += (w >> SMALL_REPORT_BITS) & MASK;
+        full |= ((w >> (2 * SMALL_REPORT_BITS)) & 1u) != 0;
+    }
+    // the call booked room for every sign it could have inserted; keep what it did insert
+    t->count_upper -= t->booked - n_new;
+    t->booked = 0;
+    if (full) latch(t, TN_ERR_TABLE_FULL, std::string("sparse pull: ") + dev_err_text(DEV_ERR_TABLE_FULL));
+    for (int i = 0; i < b.N; i++) {
+        n_distinct += (uint64_t)t->last_counts[i];
+        if (t->last_counts[i] >= var_rows[i]) latch_var_capacity(t, i, var_rows[i]);
+    }
+    note_distinct_share(t, (double)n_distinct / (double)b.L);
+    t->plan_counts = t->last_counts;
+    return take_latched(t);
+}
+
+// A push on the plan of a small pull (same shape, same table).  *other_batch: its signs turned out to be others.
+int small_push(SparseTable* t, const int64_t* const* values, const float* const* grads, const int64_t* grad_rows, int dim,
+               const int64_t* const* labels, const int64_t* const* example_ids, int64_t batch, int combiner, bool vec,
+               hipStream_t st, bool* other_batch) {
+    const SmallShape& b = t->small_shape;
+    const bool pooled = example_ids != nullptr, clicks = t->opt->kind == OPT_ADAGRAD;  // (the only optimizer that reads batch_click)
+    SmallPlan p{};
+    carve_small((char*)t->plan_buf.p, p, b);
+    float *flat = nullptr, *partial = nullptr;
+    if (pooled) {
+        TN_TRY(t->pooled_ws.ensure(2 * align_up((size_t)b.L * dim * sizeof(float), 256)));
+        Carver c{(char*)t->pooled_ws.p};
+        flat = c.take<float>((size_t)b.L * dim);
+        partial = c.take<float>((size_t)b.L * dim);
+    }
+    if (t->stage_pending) {
+        TN_HIP(hipEventSynchronize(t->stage_ev));
+        t->stage_pending = false;
+    }
+    SlotDesc* descs = reinterpret_cast<SlotDesc*>(t->hstage);
+    uint32_t at = 0;
+    for (int i = 0; i < b.N; i++) {
+        SlotDesc d{};
+        d.values = values[i];
+        d.labels = labels[i];
+        d.grads = grads[i];
+        d.rows = pooled ? batch : grad_rows[i];
+        if (pooled) d.mapped = const_cast<int64_t*>(example_ids[i]);
+        d.len = (uint32_t)t->plan_lens[i];
+        d.lbase = at;
+        descs[i] = d;
+        at += d.len;
+    }
+    t->hpush->st.mismatch = 0;
+    t->hpush->st.abort = 0;
+    const uint32_t seq = ++t->seq_verify, chunks = (b.max_len + SMALL_TILE - 1) / SMALL_TILE;
+    if (clicks)
+        TN_LAUNCH((k_small_verify<true>), dim3((uint32_t)b.N * chunks), dim3(256), st, b, p, (const SlotDesc*)descs, chunks,
+                  t->dplan, &t->hpush->st.mismatch);
+    else
+        TN_LAUNCH((k_small_verify<false>), dim3((uint32_t)b.N * chunks), dim3(256), st, b, p, (const SlotDesc*)descs, chunks,
+                  t->dplan, &t->hpush->st.mismatch);
+    const bool rows16 = dim % 4 == 0 && t->store.wstride % 4 == 0;
+    if (pooled)
+        TN_TRY(launch_small_pool(t, row_share(t->store, vec && rows16), p, batch, dim, combiner, flat, partial, st,
+                                 &t->hpush->st.abort));
+    TN_TRY(launch_small_apply(t, row_share(t->store, (pooled || vec) && rows16), p, flat, dim, st, t->hseq + 1, seq));
+    // what a call on another stream has to wait for: the updates are still running when this call returns
+    TN_HIP(hipEventRecord(t->tail_ev, st));
+    t->tail_recorded = true;
+    TN_HIP(hipGetLastError());
+    // the outcome of the comparison: the updates are queued behind it and do nothing on a mismatch
+    TN_TRY(wait_reported(t->hseq + 1, seq, st, "SparseTablePush"));
+    *other_batch = t->hpush->st.mismatch != 0;
+    if (*other_batch) return TN_OK;
+    t->last_counts = t->plan_counts;
+    if (pooled) {
+        if (t->hpush->st.abort) {  // reported by the next call that waits, like the other errors of a push's device work
+            t->plan_valid = false;  // (its click sums have been added and not taken up)
+            latch(t, TN_ERR_INVALID_ARGUMENT, std::string("sparse push: ") + dev_err_text(DEV_ERR_GRAD_ROWS));
+        }
+        return TN_OK;
+    }
+    // (the records without a gradient row were left out by the update kernel, as on the other paths)
+    for (int i = 0; i < b.N; i++)
+        if (grad_rows[i] < t->plan_counts[i])
+            return fail(TN_ERR_INVALID_ARGUMENT, std::string("sparse push: ") + dev_err_text(DEV_ERR_GRAD_ROWS) + " (slot " +
+                                                     std::to_string(i) + ")");
     return TN_OK;
 }
 
@@ -1698,7 +1949,15 @@ int tn_sparse_table_pull_op(uint32_t table_handle, int N, const int64_t* const* 
     // The remap through LDS needs the call's status on the host to fall back if a
     // bucket overflowed, so it is only used when the pull waits for its stream anyway.
     bool use_lds = !t->async_pull;
-    bool small_allowed = true;
+    SmallShape shape{};
+    if (values && value_lens && small_batch_shape(t, N, value_lens, shape)) {
+        for (int s = 0; s < N; s++)
+            if (var_rows[s] < 0 || !vars[s] || (value_lens[s] > 0 && (!values[s] || !mapped_values[s])))
+                return fail(TN_ERR_INVALID_ARGUMENT, "SparseTablePull: bad tensors of slot " + std::to_string(s));
+        t->one_stream = true;
+        TN_TRY(ensure_room(t, (uint64_t)shape.L, st));
+        return small_pull(t, shape, values, value_lens, vars, var_rows, wdim, mapped_values, st);
+    }
     for (int attempt = 0; attempt < 3; attempt++) {
         const double est_used = std::min(t->distinct_est, t->tile_est);  // what this attempt's buckets are sized from
         std::vector<SlotDesc> descs;
@@ -1723,20 +1982,16 @@ int tn_sparse_table_pull_op(uint32_t table_handle, int N, const int64_t* const* 
         }
         t->one_stream = L < ONE_STREAM_LOOKUPS;
         TN_TRY(ensure_room(t, (uint64_t)L, st));
-        // a batch whose slots each fit one workgroup takes the path of few launches (small_batch.h)
-        const bool small = small_allowed && small_batch_fits(t, N, value_lens, L, second_level_buckets(L, t->distinct_est));
-        const bool lds_scratch = use_lds || small;
-        if (small) dt_entries = 1;  // no first-level buckets
         Plan p{};
         Scratch w{};
-        const bool exact = t->exact_verify && use_lds && !small;
+        const bool exact = t->exact_verify && use_lds;
         // (a plan buffer that has to grow is freed first: not under detached updates that still read it)
         if (t->upd_pending && carve_plan(nullptr, p, N, L, exact) > t->plan_buf.bytes)
             TN_HIP(hipEventSynchronize(t->upd_ev));
         TN_TRY(t->plan_buf.ensure(carve_plan(nullptr, p, N, L, exact)));
         carve_plan((char*)t->plan_buf.p, p, N, L, exact);
-        TN_TRY(t->ws.ensure(carve_scratch(nullptr, w, L, dt_entries, lds_scratch, t->distinct_est, N)));
-        carve_scratch((char*)t->ws.p, w, L, dt_entries, lds_scratch, t->distinct_est, N);
+        TN_TRY(t->ws.ensure(carve_scratch(nullptr, w, L, dt_entries, use_lds, t->distinct_est, N)));
+        carve_scratch((char*)t->ws.p, w, L, dt_entries, use_lds, t->distinct_est, N);
         w.span_cap = span_cap;
         t->plan_valid = false;
         // Detached updates of the push before read its plan in this same buffer.  A batch of the same slot count
@@ -1749,82 +2004,6 @@ int tn_sparse_table_pull_op(uint32_t table_handle, int N, const int64_t* const* 
                                (size_t)((const char*)p.grp_sign - (const char*)t->plan_buf.p) >
                                    t->upd_groups_off + t->upd_slack))
             TN_TRY(order_after_updates(t, st));
-        if (small) {
-            TN_TRY(order_after_updates(t, st));
-            if (t->stage_pending) {
-                TN_HIP(hipEventSynchronize(t->stage_ev));
-                t->stage_pending = false;
-            }
-            std::memcpy(t->hstage, descs.data(), descs.size() * sizeof(SlotDesc));
-            size_t max_len = 0;
-            for (int s = 0; s < N; s++) max_len = std::max<size_t>(max_len, (size_t)value_lens[s]);
-            const uint32_t entries = small_entries(max_len);
-            const uint32_t set = t->small_calls++ & 1u;
-            uint32_t* cur = t->small_state->cursor2[set];
-            uint32_t* next = t->small_state->cursor2[set ^ 1u];
-            const uint32_t seq = ++t->seq_pull;
-            const Store& s = t->store;
-            DevStatus* ds = t->dplan;
-            uint32_t* prow = w.first_of;  // row of the slot's distinct sign of rank r at [first lookup of the slot + r]
-            // workgroups per slot: about five hundred lookups' worth of table probes each, within the device's CUs
-            uint32_t parts = (uint32_t)std::max<size_t>(1, std::min<size_t>(SMALL_PARTS_MAX, (max_len + 511) / 512));
-            while (parts > 1 && (size_t)N * parts > (size_t)SMALL_SLOT_WORKGROUPS) parts--;
-            TN_LAUNCH_LDS(k_small_slots, dim3(N * parts), dim3(SMALL_THREADS), small_slots_lds(entries, w.nb2), st,
-                          reinterpret_cast<const SlotDesc*>(t->hstage), p.descs, p.lbase, N, (uint32_t)L, entries, s,
-                          make_optdev(t), t->seed, p.vals_copy, p.u_of_gi, prow, w.nb2, cur, next, w.recs, w.rrow,
-                          t->small_state, parts);
-            const uint32_t big_k = N <= SMALL_NO_BIG_SLOTS || big_threshold(s) == 0xFFFFFFFFu ? 0xFFFFFFFFu : SMALL_BIG_GROUP;
-            t->plan_big_k = big_k;
-            t->plan_big_desc = false;  // (the small push's update kernel goes through big_list)
-            // the grouping's first pass (one workgroup per second-level bucket) and, beside it, a thread per
-            // (lookup position, part of a row) for the variables
-            const int finish_blocks = (int)(((uint64_t)L * (uint64_t)(vec ? wdim / 4 : wdim) + GRP_THREADS - 1) / GRP_THREADS);
-            if (vec)
-                TN_LAUNCH((k_small_group_finish<4>), dim3(w.nb2 + finish_blocks), dim3(GRP_THREADS), st, w.nb2, cur, w.recs,
-                          big_k, w.aux, w.bcounts, s, p.descs, p.lbase, p.ubase, N, (uint32_t)L, prow, p.u_of_gi,
-                          t->small_state, parts, ds, reinterpret_cast<uint32_t*>(t->hpull), t->hseq + 0, seq);
-            else
-                TN_LAUNCH((k_small_group_finish<1>), dim3(w.nb2 + finish_blocks), dim3(GRP_THREADS), st, w.nb2, cur, w.recs,
-                          big_k, w.aux, w.bcounts, s, p.descs, p.lbase, p.ubase, N, (uint32_t)L, prow, p.u_of_gi,
-                          t->small_state, parts, ds, reinterpret_cast<uint32_t*>(t->hpull), t->hseq + 0, seq);
-            TN_LAUNCH((k_group_emit<true>), dim3(w.nb2), dim3(EMIT_THREADS), st, w.nb2, cur, w.recs, w.aux,
-                      (const uint4*)nullptr, w.bcounts, (const uint8_t*)nullptr, (const uint32_t*)nullptr, (uint32_t)L,
-                      big_k, p.grp_sign, p.grp_off, p.grp_cnt, p.big_list, p.big_desc, p.list, p.where_u, w.rrow,
-                      p.grp_row, ds, p.ubase, (uint32_t)N);
-            TN_HIP(hipGetLastError());
-            // the call returns when the second launch has reported: what follows is complete in stream order
-            TN_HIP(hipEventRecord(t->tail_ev, st));
-            t->tail_recorded = true;
-            t->pull_pending = true;
-            t->pull_slots = N;
-            t->pull_lookups = (uint64_t)L;
-            t->pending_rows.assign(var_rows, var_rows + N);
-            t->plan_valid = true;
-            t->plan_small = true;
-            t->plan_clicks_dirty = false;
-            t->plan_has_show = true;
-            t->plan_prints = false;
-            t->plan_exact = false;
-            t->plan_N = N;
-            t->plan_lens.assign(value_lens, value_lens + N);
-            t->plan_epoch = t->epoch;
-            TN_TRY(wait_reported(t->hseq + 0, seq, st, "SparseTablePull"));
-            if (t->hpull->st.err & DEV_ERR_REMAP_OVERFLOW) {
-                // a second-level bucket overflowed (more distinct records than the recent pulls had): once more
-                // with buckets for a batch of distinct signs only, then on the other paths
-                t->hpull->st.err &= ~DEV_ERR_REMAP_OVERFLOW;
-                harvest(t);
-                if (est_used >= 1.0) small_allowed = false;
-                t->distinct_est = 1.0;
-                t->tile_est = 1.0;
-                t->latched = TN_OK;
-                t->latched_msg.clear();
-                continue;
-            }
-            harvest(t);
-            t->plan_counts = t->last_counts;
-            return take_latched(t);
-        }
         t->plan_small = false;
         t->plan_big_k = big_threshold(t->store);
         t->plan_big_desc = false;
@@ -2091,58 +2270,11 @@ int push_op_impl(uint32_t table_handle, int N, const int64_t* const* values, con
         src.flat = flat;
         return TN_OK;
     };
-    const RowShare small_share = row_share(t->store, vec && t->store.wstride % 4 == 0);
-    if (reuse && t->plan_small && t->small_path && !pooled && small_share.lanes != 0 && N <= SMALL_SLOTS) {
-        // A small batch on the plan of its small pull: slot descriptors, comparison of the signs and click sums by
-        // one launch, the updates by one or two more (small_batch.h).  The call's status block is the plan's:
-        // nothing of the next call runs beside this one.  The device has nothing to report: every sign of the plan
-        // has its row, and whether a gradient matrix has a row for every distinct sign of its slot is known here.
-        carve_plan((char*)t->plan_buf.p, p, N, L);
-        pd = p.push_descs;
-        ds = t->dplan;
-        if (t->stage_pending) {
-            TN_HIP(hipEventSynchronize(t->stage_ev));
-            t->stage_pending = false;
-        }
-        std::memcpy(t->hstage, descs.data(), descs.size() * sizeof(SlotDesc));
-        t->hpush->st.mismatch = 0;
-        const bool clicks = with_click;  // (a small pull's plan has the show counts)
-        if (clicks) {
-            if (t->plan_clicks_dirty)
-                TN_LAUNCH(k_reset_counts, dim3(lblocks), dim3(256), st, p.list, ds, (uint32_t)L, 1);
-            t->plan_clicks_dirty = true;
-        }
-        const uint32_t seq_v = ++t->seq_verify;
-        const int tiles = (int)((L + SMALL_TILE - 1) / SMALL_TILE);
-        const size_t vlds = ((size_t)N + 1) * sizeof(uint32_t);
-        if (clicks)
-            TN_LAUNCH_LDS((k_small_verify<true>), dim3(tiles), dim3(256), vlds, st,
-                          reinterpret_cast<const SlotDesc*>(t->hstage), p.push_descs, p.lbase, N, (uint32_t)L, p.vals_copy,
-                          ds, p.u_of_gi, p.where_u, p.list, &t->hpush->st.mismatch);
-        else
-            TN_LAUNCH_LDS((k_small_verify<false>), dim3(tiles), dim3(256), vlds, st,
-                          reinterpret_cast<const SlotDesc*>(t->hstage), p.push_descs, p.lbase, N, (uint32_t)L, p.vals_copy,
-                          ds, p.u_of_gi, p.where_u, p.list, &t->hpush->st.mismatch);
-        // (the small path stages no copy of the slots' bases: its kernels all run on the caller's stream, ahead of
-        // whatever rewrites the plan's)
-        PushSrc small_src = op_source(p, grad_dim, true);
-        small_src.ubase = p.ubase;
-        TN_TRY(launch_small_apply(t, small_share, N, small_src, ds, p, (int64_t)L, st, t->hseq + 1, seq_v));
-        // what a call on another stream has to wait for: the updates are still running when this call returns
-        TN_HIP(hipEventRecord(t->tail_ev, st));
-        t->tail_recorded = true;
-        TN_HIP(hipGetLastError());
-        // the outcome of the comparison: the updates are queued behind it and do nothing on a mismatch
-        TN_TRY(wait_reported(t->hseq + 1, seq_v, st, "SparseTablePush"));
-        if (t->hpush->st.mismatch == 0) {
-            t->last_counts = t->plan_counts;
-            // (the records without a gradient row were left out by the update kernel, as on the other paths)
-            for (int s = 0; s < N; s++)
-                if (grad_rows[s] < t->plan_counts[s])
-                    return fail(TN_ERR_INVALID_ARGUMENT, std::string("sparse push: ") + dev_err_text(DEV_ERR_GRAD_ROWS) +
-                                                             " (slot " + std::to_string(s) + ")");
-            return TN_OK;
-        }
+    if (reuse && t->plan_small) {
+        bool other_batch = false;
+        TN_TRY(small_push(t, values, grads, grad_rows, grad_dim, feature_labels, example_ids, batch, combiner, vec, st,
+                          &other_batch));
+        if (!other_batch) return TN_OK;
         reuse = false;  // another batch than the last pull's: analysed below
     } else if (reuse) {
         carve_plan((char*)t->plan_buf.p, p, N, L, t->plan_exact);
