@@ -32,96 +32,110 @@ __device__ __forceinline__ float combine_divisor(uint32_t n, int combiner) {
     return combiner == COMBINE_MEAN ? (float)n : sqrtf((float)n);
 }
 
-// Forward, step 1: where the lookups of every example start (rowptr[s * (batch + 1) + b], with
-// rowptr[.. + batch] = lookups of the slot), from the sorted example ids; also checks them.
-__global__ __launch_bounds__(256) void k_example_rowptr(const SlotDesc* __restrict__ descs,
-                                                        const uint32_t* __restrict__ lbase, int N, uint32_t L,
-                                                        int64_t batch, uint32_t* __restrict__ rowptr,
-                                                        DevStatus* status) {
-    __shared__ uint32_t lb[MAX_SLOTS + 1];
-    load_lbase(lb, lbase, N);
-    const uint32_t stride = gridDim.x * blockDim.x;
-    for (uint32_t gi = blockIdx.x * blockDim.x + threadIdx.x; gi < L; gi += stride) {
-        const int sl = find_slot(lb, N, gi);
-        const SlotDesc& d = descs[sl];
-        const int64_t* ex = example_of(d);
-        const uint32_t i = gi - lb[sl];
-        const int64_t b = ex[i];
-        const int64_t prev = i > 0 ? ex[i - 1] : -1;
-        if (b < 0 || b >= batch || prev > b) {
-            atomicOr(&status->err, DEV_ERR_GRAD_ROWS);
-            continue;
-        }
-        uint32_t* rp = rowptr + (size_t)sl * (batch + 1);
-        for (int64_t r = prev + 1; r <= b; r++) rp[r] = i;  // example b starts here; the ones skipped are empty
-        if (i == d.len - 1)
-            for (int64_t r = b + 1; r <= batch; r++) rp[r] = d.len;
+// How many of the sorted ids ex[0 .. n) lie below `x`, by a workgroup of 256 threads: every round looks at 256 places
+// of what is left, so 65 536 ids take two round trips (a binary search: sixteen).  A function of the array and x alone:
+// whatever the order of the ids, two workgroups that ask for the same x get the same answer.  sh: 5 words of LDS.
+__device__ __forceinline__ uint32_t ids_below(const int64_t* __restrict__ ex, uint32_t n, int64_t x, uint32_t* sh) {
+    uint32_t lo = 0, len = n;  // the answer lies in [lo, lo + len]
+    while (len > 0) {
+        const uint32_t step = (len + 255) / 256;
+        const uint32_t at = threadIdx.x * step;
+        const bool below = at < len && ex[lo + at] < x;
+        const uint32_t c = block_sum_256(below ? 1u : 0u, sh);  // places below x: the first c of them, if the ids are sorted
+        if (step == 1) return lo + c;
+        if (c == 0) return lo;
+        lo += (c - 1) * step + 1;
+        len = min(step - 1, n - lo);
     }
+    return lo;
 }
 
-// Forward, step 2: one group of `chunks` threads per (slot, example) sums the rows of the example's
-// lookups in order, divides, and writes the output row (zeros for an example without lookups).
-template <int VEC>
-__global__ __launch_bounds__(256) void k_combine_fwd(const SlotDesc* __restrict__ descs, int N, int dim, int64_t batch,
-                                                     int combiner, const uint32_t* __restrict__ rowptr,
-                                                     DevStatus* status) {
-    if (status->err) return;  // bad example ids: the row pointers are not to be trusted
-    const int chunks = dim / VEC;
-    const int64_t per_slot = batch * chunks;
-    const int64_t total = (int64_t)N * per_slot;
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < total; t += stride) {
-        const int sl = (int)(t / per_slot);
-        const int64_t rest = t - (int64_t)sl * per_slot;
-        const int64_t b = rest / chunks;
-        const int c = (int)(rest - b * chunks);
-        const SlotDesc& d = descs[sl];
-        const uint32_t* rp = rowptr + (size_t)sl * (batch + 1);
-        const uint32_t lo = d.len ? rp[b] : 0, hi = d.len ? rp[b + 1] : 0;
-        const int64_t* ids = d.values;
-        const float* rows = d.grads;
-        const int64_t nrows = d.rows;
-        float acc[VEC];
-#pragma unroll
-        for (int q = 0; q < VEC; q++) acc[q] = 0.f;
-        bool bad_id = false;
-        // windows of COMBINE_WINDOW lookups: ids first, then their rows, all loads independent;
-        // the additions run in lookup order
-        for (uint32_t j0 = lo; j0 < hi; j0 += COMBINE_WINDOW) {
-            int64_t wid[COMBINE_WINDOW];
-#pragma unroll
-            for (int q = 0; q < COMBINE_WINDOW; q++) wid[q] = (j0 + q < hi) ? ids[j0 + q] : -1;
-            float wr[COMBINE_WINDOW][VEC];
-#pragma unroll
-            for (int q = 0; q < COMBINE_WINDOW; q++) {
-                const bool in = j0 + q < hi;
-                const bool ok = in && wid[q] >= 0 && wid[q] < nrows;
-                if (in && !ok) bad_id = true;
-                const float* row = rows + (ok ? wid[q] : 0) * dim + c * VEC;
-                if (VEC == 4) {
-                    const float4 v = ok ? *reinterpret_cast<const float4*>(row) : make_float4(0.f, 0.f, 0.f, 0.f);
-                    wr[q][0] = v.x;
-                    wr[q][1 % VEC] = v.y;
-                    wr[q][2 % VEC] = v.z;
-                    wr[q][3 % VEC] = v.w;
-                } else {
-                    wr[q][0] = ok ? row[0] : 0.f;
-                }
+// Forward: a workgroup takes `per` examples of a slot (items of a call are numbered slot by slot): it finds their
+// lookups, which are consecutive, and every group of LPG lanes sums the rows of an example's lookups in order, divides,
+// and writes the output row (zeros for an example without lookups).  One pass: a kernel that first worked out where the
+// lookups of every example start cost a launch and a pass over the ids of its own (27 us at 5 M lookups).
+//
+// The example ids are checked on the way: the workgroups' shares of a slot's lookups follow each other without a gap
+// whatever the ids are (each ends where ids_below puts the start of the next, the first starts at 0, the last ends at
+// the slot's end), so every lookup is looked at by one workgroup, which wants it to lie among its examples and not
+// before its predecessor.
+//
+// The variable rows of a slot are read again and again: every die of the chip takes a contiguous share of the items, so
+// that a slot's rows (1.3 MB at 20 k distinct signs of 16 elements) are in the L2 of the die that wants them.
+template <int LPG, bool ANY>
+__global__ __launch_bounds__(256) void k_combine_fwd(const SlotDesc* __restrict__ descs, uint32_t items, uint32_t per_slot,
+                                                     uint32_t per, int dim, int64_t batch, int combiner, DevStatus* status) {
+    extern __shared__ uint32_t range[];  // [per] first lookup of an example, [per] the lookup after its last
+    __shared__ uint32_t sh[5];
+    const int sub = threadIdx.x % LPG;
+    const DieShare share(items);
+    uint32_t err = 0;
+    for (uint32_t item = share.first; item < share.end; item += share.step) {
+        const uint32_t sl = item / per_slot;
+        const int64_t b0 = (int64_t)(item - sl * per_slot) * per;
+        const uint32_t nb = (uint32_t)min((int64_t)per, batch - b0);
+        const SlotDesc d = descs[sl];
+        const int64_t* __restrict__ ex = example_of(d);
+        for (uint32_t i = threadIdx.x; i < 2 * per; i += 256) range[i] = 0;
+        const uint32_t lo = b0 == 0 ? 0u : ids_below(ex, d.len, b0, sh);
+        const uint32_t hi = b0 + nb >= batch ? d.len : ids_below(ex, d.len, b0 + nb, sh);
+        __syncthreads();
+        if (hi < lo) err |= DEV_ERR_GRAD_ROWS;
+        for (uint32_t i = lo + threadIdx.x; i < hi; i += 256) {
+            const int64_t x = ex[i], prev = i > 0 ? ex[i - 1] : -1, next = i + 1 < d.len ? ex[i + 1] : batch;
+            if (x < b0 || x >= b0 + nb || prev > x) {
+                err |= DEV_ERR_GRAD_ROWS;
+                continue;
             }
-#pragma unroll
-            for (int q = 0; q < COMBINE_WINDOW; q++)
-                if (j0 + q < hi)
-#pragma unroll
-                    for (int v = 0; v < VEC; v++) acc[v] += wr[q][v];
+            if (prev != x || i == lo) range[x - b0] = i;
+            if (next != x || i + 1 == hi) range[per + (x - b0)] = i + 1;
         }
-        if (bad_id && c == 0) atomicOr(&status->err, DEV_ERR_VAR_CAPACITY);
-        const float div = combine_divisor(hi - lo, combiner);
-        float* o = d.var + b * dim + c * VEC;
-        if (VEC == 4)
-            *reinterpret_cast<float4*>(o) = make_float4(acc[0] / div, acc[1 % VEC] / div, acc[2 % VEC] / div, acc[3 % VEC] / div);
-        else
-            o[0] = acc[0] / div;
+        __syncthreads();
+        const int64_t* __restrict__ ids = d.values;
+        const float* __restrict__ rows = d.grads;
+        for (uint32_t e = threadIdx.x / LPG; e < nb; e += 256 / LPG) {
+            const uint32_t from = range[e], to = max(range[per + e], from);
+            const float div = combine_divisor(to - from, combiner);
+            float* o = d.var + (b0 + e) * dim;
+            for (int c0 = 0; c0 < dim; c0 += 4 * LPG) {  // (rows of more than 128 elements: once more for the next ones)
+                float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+                // windows of COMBINE_WINDOW lookups: ids first, then their rows, all loads independent; the additions
+                // run in lookup order
+                for (uint32_t j0 = from; j0 < to; j0 += COMBINE_WINDOW) {
+                    int64_t wid[COMBINE_WINDOW];
+                    float4 wr[COMBINE_WINDOW];
+#pragma unroll
+                    for (int q = 0; q < COMBINE_WINDOW; q++) wid[q] = j0 + q < to ? ids[j0 + q] : -1;
+#pragma unroll
+                    for (int q = 0; q < COMBINE_WINDOW; q++) {
+                        const bool ok = wid[q] >= 0 && wid[q] < d.rows;
+                        if (j0 + q < to && !ok) err |= DEV_ERR_VAR_CAPACITY;
+                        wr[q] = ok ? row_part<ANY>(rows + wid[q] * dim + c0, sub, dim - c0) : make_float4(0.f, 0.f, 0.f, 0.f);
+                    }
+#pragma unroll
+                    for (int q = 0; q < COMBINE_WINDOW; q++) {
+                        if (j0 + q >= to) break;
+                        acc.x += wr[q].x;
+                        acc.y += wr[q].y;
+                        acc.z += wr[q].z;
+                        acc.w += wr[q].w;
+                    }
+                }
+                put_row_part<ANY>(o + c0, sub, dim - c0, make_float4(acc.x / div, acc.y / div, acc.z / div, acc.w / div));
+            }
+        }
+        __syncthreads();
     }
+    if (err) atomicOr(&status->err, err);
+}
+
+// Behind the last kernel of a call: its error flags to the host, in one word with the number of the call, for which the
+// host polls (a wait on the stream returns about ten microseconds later); the flags start at zero for the next call.
+__global__ void k_report(DevStatus* status, uint64_t* host_word, uint32_t seq) {
+    if (threadIdx.x != 0) return;
+    const unsigned long long w = (unsigned long long)status->err | ((unsigned long long)seq << 32);
+    status->err = 0;
+    __hip_atomic_store(reinterpret_cast<unsigned long long*>(host_word), w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // Backward, step 1: the value of every lookup: its example in the high word, the number of

@@ -36,6 +36,8 @@ constexpr size_t ONE_STREAM_LOOKUPS = 3u << 20;
 constexpr uint32_t SELF_SCAN_TILES = 8192;  // tiles of the ranking pass up to which no scan kernel runs between its launches
 constexpr int GRID_CAP = 256 * 8;                       // 256 CUs x 8 workgroups of 256 threads
 constexpr int TILE_GRID = 256 * 3;                      // workgroups of k_tile_dedup: what the chip holds of it at once
+constexpr uint32_t COMBINE_EXAMPLES = 64;  // examples per workgroup of k_combine_fwd at least
+constexpr int COMBINE_DIRECT = 1024;       // workgroups of it up to which they read the slots' descriptors from pinned host memory
 constexpr size_t LDS_MIN_LOOKUPS = 1024;  // from here on the remap through LDS wins: it also takes fewer launches (cfg1, 8 k lookups: 0.154 -> 0.136 ms)
 
 // Up to this many lookups a batch whose slots are all short (SMALL_SLOT_MAX lookups, SMALL_SLOTS slots) takes the path
@@ -82,6 +84,7 @@ struct SparseTable {
     uint64_t plan_epoch = 0;
     DevStatus* dstatus = nullptr;   // device: status of table-level calls
     DevStatus* dplan = nullptr;     // device: status / counts of the op-level plan
+    DevStatus* dcomb = nullptr;     // device: error flags of a combine op (zero between calls)
     DevStatus* dpush = nullptr;     // device: status of a push that reuses the plan (the plan's counts, flags of its own)
     HostStatus* hpull = nullptr;    // pinned
     HostStatus* hpush = nullptr;    // pinned
@@ -97,6 +100,8 @@ struct SparseTable {
     // per workgroup of a pull's first launch; hseq [0] a large pull's status is on the host, [1] a push's signs are
     // compared) with the numbers the host expects there next, the dynamic LDS its kernels may have.
     uint64_t* hwords = nullptr;
+    uint64_t* hcomb = nullptr;         // pinned: what a combine op reports (k_report)
+    uint32_t seq_comb = 0;
     uint32_t* hseq = nullptr;
     uint32_t seq_pull = 0, seq_verify = 0;
     std::vector<int64_t> plan_counts;  // distinct signs per slot of the small pull that left the plan
@@ -275,10 +280,11 @@ void free_store(Store& s) {
 
 int ensure_side_buffers(SparseTable* t) {
     if (t->dstatus) return TN_OK;
-    TN_HIP(hipMalloc((void**)&t->dstatus, 3 * sizeof(DevStatus)));
-    TN_HIP(hipMemset(t->dstatus, 0, 3 * sizeof(DevStatus)));
+    TN_HIP(hipMalloc((void**)&t->dstatus, 4 * sizeof(DevStatus)));
+    TN_HIP(hipMemset(t->dstatus, 0, 4 * sizeof(DevStatus)));
     t->dplan = t->dstatus + 1;
     t->dpush = t->dstatus + 2;
+    t->dcomb = t->dstatus + 3;
     TN_HIP(hipHostMalloc((void**)&t->hpull, sizeof(HostStatus), hipHostMallocDefault));
     TN_HIP(hipHostMalloc((void**)&t->hpush, sizeof(HostStatus), hipHostMallocDefault));
     std::memset(t->hpull, 0, sizeof(HostStatus));
@@ -288,6 +294,8 @@ int ensure_side_buffers(SparseTable* t) {
     std::memset(t->hseq, 0, 64);
     TN_HIP(hipHostMalloc((void**)&t->hwords, SMALL_WORKGROUPS * sizeof(uint64_t), hipHostMallocDefault));
     std::memset(t->hwords, 0, SMALL_WORKGROUPS * sizeof(uint64_t));
+    TN_HIP(hipHostMalloc((void**)&t->hcomb, 64, hipHostMallocDefault));
+    std::memset(t->hcomb, 0, 64);
     t->hstage_bytes = (size_t)MAX_SLOTS * sizeof(SlotDesc) + (MAX_SLOTS + 1) * sizeof(uint32_t);
     TN_HIP(hipHostMalloc((void**)&t->hstage, t->hstage_bytes, hipHostMallocDefault));
     TN_HIP(hipEventCreateWithFlags(&t->stage_ev, hipEventDisableTiming));
@@ -2426,7 +2434,6 @@ int tn_sparse_table_combine_op(uint32_t table_handle, int N, const int64_t* cons
     hipStream_t st = (hipStream_t)stream;
     TN_TRY(ensure_allocated(t, st));
     std::vector<SlotDesc> descs(N, SlotDesc{});
-    std::vector<uint32_t> lbase(N + 1, 0);
     size_t L = 0;
     bool vec = dim % 4 == 0;
     for (int s = 0; s < N; s++) {
@@ -2440,54 +2447,68 @@ int tn_sparse_table_combine_op(uint32_t table_handle, int N, const int64_t* cons
         d.var = out[s];
         d.rows = var_rows[s];
         d.len = (uint32_t)value_lens[s];
-        d.lbase = (uint32_t)L;
-        lbase[s] = (uint32_t)L;
         L += (size_t)value_lens[s];
         if (L > 0x7FFFFFF0ull) return fail(TN_ERR_UNSUPPORTED, "embedding combine: more than 2^31 lookups in one call");
         vec = vec && aligned16(vars[s]) && aligned16(out[s]);
     }
-    lbase[N] = (uint32_t)L;
-    // an earlier call's status is collected first: this call uses the table's status block
+    // an earlier call's status is collected first
     if (t->push_pending || t->pull_pending) {
         if (t->last_stream && t->last_stream != st) TN_HIP(hipStreamSynchronize(t->last_stream));
         TN_HIP(hipStreamSynchronize(st));
         harvest(t);
     }
     t->last_stream = st;
-    {
-        const size_t db = (size_t)N * sizeof(SlotDesc), lb = (size_t)(N + 1) * sizeof(uint32_t);
-        const size_t rp = (size_t)N * (size_t)(batch + 1) * sizeof(uint32_t);
-        TN_TRY(t->comb_buf.ensure(align_up(db, 256) + align_up(lb, 256) + rp));
-        SlotDesc* ddescs = (SlotDesc*)t->comb_buf.p;
-        uint32_t* dlbase = (uint32_t*)((char*)t->comb_buf.p + align_up(db, 256));
-        uint32_t* rowptr = (uint32_t*)((char*)dlbase + align_up(lb, 256));
-        if (t->stage_pending) {
-            TN_HIP(hipEventSynchronize(t->stage_ev));
-            t->stage_pending = false;
-        }
-        std::memcpy(t->hstage, descs.data(), db);
-        std::memcpy(t->hstage + db, lbase.data(), lb);
-        TN_LAUNCH(k_stage_in, dim3(launch_grid((int64_t)(db + lb) / 4, 256, 64)), dim3(256), st,
-                  reinterpret_cast<const uint32_t*>(t->hstage), reinterpret_cast<uint32_t*>(ddescs), (uint32_t)(db / 4),
-                  dlbase, (uint32_t)(lb / 4), t->dstatus, (int)STATUS_NEW_PLAN, (uint32_t*)nullptr, 0u,
-                  (const DevStatus*)t->dstatus, (const uint32_t*)nullptr, (uint32_t*)nullptr, 0u);
-        TN_HIP(hipEventRecord(t->stage_ev, st));
-        t->stage_pending = true;
-        // where the lookups of every example start, then one thread group per (slot, example)
-        if (L > 0)
-            TN_LAUNCH(k_example_rowptr, dim3(launch_grid(L, 256, GRID_CAP * 2)), dim3(256), st, ddescs, dlbase, N,
-                      (uint32_t)L, batch, rowptr, t->dstatus);
-        if (vec)
-            TN_LAUNCH((k_combine_fwd<4>), dim3(launch_grid((int64_t)N * batch * (dim / 4), 256, GRID_CAP * 4)), dim3(256),
-                      st, ddescs, N, dim, batch, combiner, rowptr, t->dstatus);
-        else
-            TN_LAUNCH((k_combine_fwd<1>), dim3(launch_grid((int64_t)N * batch * dim, 256, GRID_CAP * 4)), dim3(256), st,
-                      ddescs, N, dim, batch, combiner, rowptr, t->dstatus);
+    if (t->stage_pending) {
+        TN_HIP(hipEventSynchronize(t->stage_ev));
+        t->stage_pending = false;
     }
+    // A workgroup per COMBINE_EXAMPLES examples of a slot where that does not fill the chip several times over, else per
+    // more of them: every workgroup pays for finding its lookups.
+    uint32_t per = COMBINE_EXAMPLES;
+    while (per < 1024 && (int64_t)N * ((batch + per - 1) / per) > 4096) per *= 2;
+    const uint32_t per_slot = (uint32_t)((batch + per - 1) / per);
+    const int64_t items = (int64_t)N * per_slot;
+    if (items > 0x7FFFFFF0LL) return fail(TN_ERR_UNSUPPORTED, "embedding combine: too many examples");
+    const int grid = launch_grid(items, 1, GRID_CAP * 4);
+    std::memcpy(t->hstage, descs.data(), (size_t)N * sizeof(SlotDesc));
+    const SlotDesc* ddescs = reinterpret_cast<const SlotDesc*>(t->hstage);
+    if (grid > COMBINE_DIRECT) {  // (few workgroups read their slot's descriptor from the host's buffer themselves: a launch less)
+        const size_t db = (size_t)N * sizeof(SlotDesc);
+        TN_TRY(t->comb_buf.ensure(align_up(db, 256)));
+        TN_LAUNCH(k_stage_in, dim3(launch_grid((int64_t)db / 4, 256, 64)), dim3(256), st,
+                  reinterpret_cast<const uint32_t*>(t->hstage), reinterpret_cast<uint32_t*>(t->comb_buf.p), (uint32_t)(db / 4),
+                  (uint32_t*)nullptr, 0u, (DevStatus*)nullptr, (int)STATUS_KEEP, (uint32_t*)nullptr, 0u,
+                  (const DevStatus*)nullptr, (const uint32_t*)nullptr, (uint32_t*)nullptr, 0u);
+        ddescs = (const SlotDesc*)t->comb_buf.p;
+    }
+    int lanes = 1;
+    while (lanes < 32 && 4 * lanes < dim) lanes *= 2;
+    const bool any = !vec || dim % (4 * lanes) != 0;
+#define TN_LAUNCH_COMBINE_ANY(LPG, ANY)                                                                               \
+    TN_LAUNCH_LDS((k_combine_fwd<LPG, ANY>), dim3(grid), dim3(256), (size_t)per * 8, st, ddescs, (uint32_t)items, per_slot, \
+                  per, dim, batch, combiner, t->dcomb)
+#define TN_LAUNCH_COMBINE(LPG)                  \
+    do {                                        \
+        if (any)                                \
+            TN_LAUNCH_COMBINE_ANY(LPG, true);   \
+        else                                    \
+            TN_LAUNCH_COMBINE_ANY(LPG, false);  \
+    } while (0)
+    switch (lanes) {
+        case 1: TN_LAUNCH_COMBINE(1); break;
+        case 2: TN_LAUNCH_COMBINE(2); break;
+        case 4: TN_LAUNCH_COMBINE(4); break;
+        case 8: TN_LAUNCH_COMBINE(8); break;
+        case 16: TN_LAUNCH_COMBINE(16); break;
+        default: TN_LAUNCH_COMBINE(32); break;
+    }
+#undef TN_LAUNCH_COMBINE
+#undef TN_LAUNCH_COMBINE_ANY
+    const uint32_t seq = ++t->seq_comb;
+    TN_LAUNCH(k_report, dim3(1), dim3(64), st, t->dcomb, t->hcomb, seq);
     TN_HIP(hipGetLastError());
-    TN_HIP(hipMemcpyAsync(&t->hpull->st, t->dstatus, sizeof(DevStatus), hipMemcpyDeviceToHost, st));
-    TN_HIP(hipStreamSynchronize(st));
-    const uint32_t err = t->hpull->st.err;
+    TN_TRY(wait_words(t->hcomb, 1, seq, st, "embedding combine"));
+    const uint32_t err = (uint32_t)*t->hcomb;
     if (err & DEV_ERR_VAR_CAPACITY) return fail(TN_ERR_VAR_CAPACITY, "embedding combine: a mapped id is not a row of its variable");
     if (err & DEV_ERR_GRAD_ROWS)
         return fail(TN_ERR_INVALID_ARGUMENT, "embedding combine: example ids must be non-decreasing and in [0, batch)");
