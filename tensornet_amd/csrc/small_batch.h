@@ -712,14 +712,31 @@ struct SmallSrc {
     __device__ __forceinline__ int click(uint4 m) const { return click_at[m.x]; }
 };
 
+// The records of one sign: entries of the bucket's member list.
+struct SmallGroup {
+    typedef uint4 Entry;
+    SmallSrc src;
+    const uint4* mem;
+    __device__ __forceinline__ Entry entry(uint32_t j) const { return mem[j]; }
+    __device__ __forceinline__ const float* gradient(const Entry& m) const { return src.gradient(m); }
+    __device__ __forceinline__ int show(const Entry& m) const { return (int)m.z; }
+    __device__ __forceinline__ int click(const Entry& m) const { return src.click(m); }
+    __device__ __forceinline__ void taken(uint32_t k, int sub, int lanes) const {
+        for (uint32_t j = sub; j < k; j += lanes) src.click_at[mem[j].x] = 0;
+    }
+};
+
 // One sign with a few records by a group of LPG lanes, AHEAD records at a time: the gradients of the next AHEAD and the
 // member entries of the AHEAD after those are in flight meanwhile, so that a chain of k records costs k / AHEAD round
 // trips instead of 2 k (a small batch's kernels are as long as their longest chain).  Every load is issued whether its
 // record exists or not (past the end: the group's last member again, the row in place of a gradient): a load under a
 // condition makes the compiler wait for all loads where the branches join.
-template <int KIND, int LPG, bool ANY, int AHEAD>
-__device__ __forceinline__ void small_apply_group(const Store& s, const OptDev& o, const SmallSrc& src, uint32_t row,
-                                                  uint32_t k, const uint4* mem, int sub, int lane0, float c1, float c2) {
+// grp: the sign's records -- entry(j) of the j-th (what is fetched ahead), its gradient row (nullptr: it has none) and
+// counts, taken(k, sub, lanes) once all have been applied.
+template <int KIND, int LPG, bool ANY, int AHEAD, typename Group>
+__device__ __forceinline__ void apply_group_ahead(const Store& s, const OptDev& o, const Group& grp, uint32_t row, uint32_t k,
+                                                  int sub, int lane0, float c1, float c2) {
+    typedef typename Group::Entry Entry;
     const int D = s.D;
     float* wp = s.w + (uint64_t)row * s.wstride;
     float* sp = s.st + (uint64_t)row * s.sstride;
@@ -738,32 +755,32 @@ __device__ __forceinline__ void small_apply_group(const Store& s, const OptDev& 
         delta_show = __float_as_int(sp[2 * D + 1]);
     }
     bool any = false;
-    uint4 m1[AHEAD], m2[AHEAD];
+    Entry m1[AHEAD], m2[AHEAD];
     float4 g0[AHEAD], g1[AHEAD];
     int sh0[AHEAD], ck0[AHEAD], sh1[AHEAD], ck1[AHEAD];
     bool ok0[AHEAD], ok1[AHEAD];
-    auto fetch = [&](const uint4 (&m)[AHEAD], uint32_t first, float4 (&g)[AHEAD], int (&sh)[AHEAD], int (&ck)[AHEAD],
+    auto fetch = [&](const Entry (&m)[AHEAD], uint32_t first, float4 (&g)[AHEAD], int (&sh)[AHEAD], int (&ck)[AHEAD],
                      bool (&ok)[AHEAD]) {
 #pragma unroll
         for (int q = 0; q < AHEAD; q++) {
-            const float* gp = src.gradient(m[q]);
+            const float* gp = grp.gradient(m[q]);
             ok[q] = gp != nullptr && first + q < k;
-            sh[q] = (int)m[q].z;
-            ck[q] = KIND == OPT_ADAGRAD ? src.click(m[q]) : 0;
+            sh[q] = grp.show(m[q]);
+            ck[q] = KIND == OPT_ADAGRAD ? grp.click(m[q]) : 0;
             g[q] = row_part<ANY>(ok[q] ? gp : wp, sub, D);
         }
     };
 #pragma unroll
     for (int q = 0; q < AHEAD; q++) {
-        m1[q] = mem[min((uint32_t)q, k - 1)];
-        m2[q] = mem[min((uint32_t)(AHEAD + q), k - 1)];
+        m1[q] = grp.entry(min((uint32_t)q, k - 1));
+        m2[q] = grp.entry(min((uint32_t)(AHEAD + q), k - 1));
     }
     fetch(m1, 0, g0, sh0, ck0, ok0);
 #pragma unroll
     for (int q = 0; q < AHEAD; q++) m1[q] = m2[q];
     for (uint32_t c0 = 0; c0 < k; c0 += AHEAD) {
 #pragma unroll
-        for (int q = 0; q < AHEAD; q++) m2[q] = mem[min(c0 + 2 * AHEAD + q, k - 1)];
+        for (int q = 0; q < AHEAD; q++) m2[q] = grp.entry(min(c0 + 2 * AHEAD + q, k - 1));
         fetch(m1, c0 + AHEAD, g1, sh1, ck1, ok1);
         if constexpr (KIND == OPT_ADAGRAD) {
             // The records of the window depend on each other through g2sum (one rounded addition per record) and
@@ -840,8 +857,7 @@ __device__ __forceinline__ void small_apply_group(const Store& s, const OptDev& 
             m1[q] = m2[q];
         }
     }
-    if (KIND == OPT_ADAGRAD)
-        for (uint32_t j = sub; j < k; j += LPG) src.click_at[mem[j].x] = 0;
+    if (KIND == OPT_ADAGRAD) grp.taken(k, sub, LPG);
     if (!any) return;
     put_row_part<ANY>(wp, sub, D, w);
     if (KIND == OPT_ADAGRAD) {
@@ -861,7 +877,7 @@ __device__ __forceinline__ void small_apply_group(const Store& s, const OptDev& 
 
 // Bytes of dynamic LDS of k_small_apply when its launch includes the workgroups for the signs with many records:
 // per wavefront the staging and the row of apply_big_groups, then its pointer, count, flag and divisor arrays.
-inline size_t small_apply_wave_lds(int D) { return align_up(big_lds_bytes(D), 8) + BIG_CHUNK * (8 + 4 + 4 + 4); }
+inline size_t small_apply_wave_lds(int D) { return align_up(big_lds_bytes(D), 8) + BIG_CHUNK * (8 + 4); }
 
 __host__ __device__ inline size_t small_apply_slots_lds(int N) { return ((size_t)N * 12 + 7) / 8 * 8; }
 
@@ -916,11 +932,9 @@ __global__ __launch_bounds__(256) void k_small_apply(SmallShape b, SmallPlan p, 
         char* base = reinterpret_cast<char*>(apply_lds) + small_apply_slots_lds(flat ? 0 : b.N) + (size_t)wave * wave_lds;
         float* gbuf = reinterpret_cast<float*>(base);
         const float** gptr = reinterpret_cast<const float**>(base + wave_arrays);
-        int* gshow = reinterpret_cast<int*>(gptr + BIG_CHUNK);
-        int* gok = gshow + BIG_CHUNK;
-        float* den = reinterpret_cast<float*>(gok + BIG_CHUNK);
+        float* den = reinterpret_cast<float*>(gptr + BIG_CHUNK);
         apply_big_groups<KIND>(
-            s, o, gbuf_floats, gbuf, gptr, gshow, gok, den, lane, (uint32_t)wave, 4u, head.z,
+            s, o, gbuf_floats, gbuf, gptr, den, lane, (uint32_t)wave, 4u, head.z,
             [&](uint32_t bi, uint32_t& row, uint32_t& off, uint32_t& k) {
                 const uint2 g = p.group[first + b.cap - 1 - bi];
                 row = g.x;
@@ -944,7 +958,8 @@ __global__ __launch_bounds__(256) void k_small_apply(SmallShape b, SmallPlan p, 
         for (uint32_t g = g0; g < head.y; g += 256 / LPG) {
             const uint2 d = p.group[first + head.x + g];
             if (d.x > s.cap) continue;  // no row number at all: never address the table with it
-            small_apply_group<KIND, LPG, ANY, 4>(s, o, src, d.x, d.y >> 16, p.member + first + (d.y & 0xFFFFu), sub, lane0, c1, c2);
+            const SmallGroup grp{src, p.member + first + (d.y & 0xFFFFu)};
+            apply_group_ahead<KIND, LPG, ANY, 4>(s, o, grp, d.x, d.y >> 16, sub, lane0, c1, c2);
         }
         return;
     }

@@ -3,7 +3,7 @@
 // and at operator level (core/kernels/sparse_table_ops.cc:170-265,317-368).
 #include "combine_kernels.h"
 #include "remap_lds.h"
-#include "small_batch.h"
+#include "table_level.h"
 
 #include <algorithm>
 #include <atomic>
@@ -36,6 +36,7 @@ constexpr size_t ONE_STREAM_LOOKUPS = 3u << 20;
 constexpr uint32_t SELF_SCAN_TILES = 8192;  // tiles of the ranking pass up to which no scan kernel runs between its launches
 constexpr int GRID_CAP = 256 * 8;                       // 256 CUs x 8 workgroups of 256 threads
 constexpr int TILE_GRID = 256 * 3;                      // workgroups of k_tile_dedup: what the chip holds of it at once
+constexpr size_t PULL_WORDS = std::max<size_t>(SMALL_WORKGROUPS, TABLE_PULL_WORDS);
 constexpr uint32_t COMBINE_EXAMPLES = 64;  // examples per workgroup of k_combine_fwd at least
 constexpr int COMBINE_DIRECT = 1024;       // workgroups of it up to which they read the slots' descriptors from pinned host memory
 constexpr size_t LDS_MIN_LOOKUPS = 1024;  // from here on the remap through LDS wins: it also takes fewer launches (cfg1, 8 k lookups: 0.154 -> 0.136 ms)
@@ -84,6 +85,7 @@ struct SparseTable {
     uint64_t plan_epoch = 0;
     DevStatus* dstatus = nullptr;   // device: status of table-level calls
     DevStatus* dplan = nullptr;     // device: status / counts of the op-level plan
+    DevStatus* dtpush = nullptr;    // device: error flags of a table-level push (zero between calls)
     DevStatus* dcomb = nullptr;     // device: error flags of a combine op (zero between calls)
     DevStatus* dpush = nullptr;     // device: status of a push that reuses the plan (the plan's counts, flags of its own)
     HostStatus* hpull = nullptr;    // pinned
@@ -97,7 +99,7 @@ struct SparseTable {
     DevBuf pooled_ws;               // scratch of a push of pooled gradients (ordered lookups, reduced rows)
     size_t place_lds = 0, huge_lds = 0;  // dynamic LDS of k_place_lookups / k_order_huge on this device (0: not asked yet)
     // The path of few launches for small batches: the words in pinned memory its kernels report through (hwords: one
-    // per workgroup of a pull's first launch; hseq [0] a large pull's status is on the host, [1] a push's signs are
+    // per workgroup of a small pull's first launch, or of a table-level pull's; hseq [0] a large pull's status is on the host, [1] a push's signs are
     // compared) with the numbers the host expects there next, the dynamic LDS its kernels may have.
     uint64_t* hwords = nullptr;
     uint64_t* hcomb = nullptr;         // pinned: what a combine op reports (k_report)
@@ -107,6 +109,7 @@ struct SparseTable {
     std::vector<int64_t> plan_counts;  // distinct signs per slot of the small pull that left the plan
     SmallShape small_shape{};          // how that pull laid its batch out
     size_t small_lds = 0, small_emit_lds = 0;
+    bool table_lds[2] = {false, false};  // k_table_apply (rows in 16-byte pieces / any) has been told how much it may have
     bool plan_small = false;   // the plan was left by a small pull: a push may take the small path, too
     bool plan_prints = false;  // the plan holds fingerprints of the batch's signs, not a copy of them
     bool exact_verify = false; // pulls that leave fingerprints keep a copy of the signs as well, pushes compare that
@@ -280,11 +283,12 @@ void free_store(Store& s) {
 
 int ensure_side_buffers(SparseTable* t) {
     if (t->dstatus) return TN_OK;
-    TN_HIP(hipMalloc((void**)&t->dstatus, 4 * sizeof(DevStatus)));
-    TN_HIP(hipMemset(t->dstatus, 0, 4 * sizeof(DevStatus)));
+    TN_HIP(hipMalloc((void**)&t->dstatus, 5 * sizeof(DevStatus)));
+    TN_HIP(hipMemset(t->dstatus, 0, 5 * sizeof(DevStatus)));
     t->dplan = t->dstatus + 1;
     t->dpush = t->dstatus + 2;
     t->dcomb = t->dstatus + 3;
+    t->dtpush = t->dstatus + 4;
     TN_HIP(hipHostMalloc((void**)&t->hpull, sizeof(HostStatus), hipHostMallocDefault));
     TN_HIP(hipHostMalloc((void**)&t->hpush, sizeof(HostStatus), hipHostMallocDefault));
     std::memset(t->hpull, 0, sizeof(HostStatus));
@@ -292,8 +296,8 @@ int ensure_side_buffers(SparseTable* t) {
     TN_HIP(hipHostMalloc((void**)&t->hcount, 64, hipHostMallocDefault));
     TN_HIP(hipHostMalloc((void**)&t->hseq, 64, hipHostMallocDefault));
     std::memset(t->hseq, 0, 64);
-    TN_HIP(hipHostMalloc((void**)&t->hwords, SMALL_WORKGROUPS * sizeof(uint64_t), hipHostMallocDefault));
-    std::memset(t->hwords, 0, SMALL_WORKGROUPS * sizeof(uint64_t));
+    TN_HIP(hipHostMalloc((void**)&t->hwords, PULL_WORDS * sizeof(uint64_t), hipHostMallocDefault));
+    std::memset(t->hwords, 0, PULL_WORDS * sizeof(uint64_t));
     TN_HIP(hipHostMalloc((void**)&t->hcomb, 64, hipHostMallocDefault));
     std::memset(t->hcomb, 0, 64);
     t->hstage_bytes = (size_t)MAX_SLOTS * sizeof(SlotDesc) + (MAX_SLOTS + 1) * sizeof(uint32_t);
@@ -1167,6 +1171,52 @@ size_t carve_small(char* base, SmallPlan& p, const SmallShape& b) {
     return align_up(c.off, 256);
 }
 
+// The updates of a table-level push (k_table_apply).
+template <int KIND>
+int launch_table_apply_kind(SparseTable* t, RowShare share, const OptDev& o, const TableShape& b, const tn_sign_info* infos,
+                            const float* grads, int dim, const uint2* recs, const uint16_t* boff, DevStatus* ds, hipStream_t st) {
+    const Store& s = t->store;
+    const size_t wave_lds = small_apply_wave_lds(s.D), lists = table_apply_lists_lds(b.tiles);
+#define TN_LAUNCH_TABLE_ANY(LPG, ANY)                                                                                   \
+    do {                                                                                                                \
+        if (!t->table_lds[ANY]) {                                                                                       \
+            t->table_lds[ANY] = true;                                                                                   \
+            (void)big_lds_bytes_for(reinterpret_cast<const void*>(k_table_apply<KIND, LPG, ANY>));                      \
+        }                                                                                                               \
+        TN_LAUNCH_LDS((k_table_apply<KIND, LPG, ANY>), dim3(b.nb), dim3(256), lists + 4 * wave_lds, st, b, s, o, infos, \
+                      grads, dim, recs, boff, ds, &t->hpush->st.err, big_gbuf_floats(s.D), (uint32_t)wave_lds,          \
+                      (uint32_t)align_up(big_lds_bytes(s.D), 8), (uint32_t)lists);                                      \
+    } while (0)
+#define TN_LAUNCH_TABLE(LPG)                  \
+    do {                                      \
+        if (share.any)                        \
+            TN_LAUNCH_TABLE_ANY(LPG, true);   \
+        else                                  \
+            TN_LAUNCH_TABLE_ANY(LPG, false);  \
+    } while (0)
+    switch (share.lanes) {
+        case 1: TN_LAUNCH_TABLE(1); break;
+        case 2: TN_LAUNCH_TABLE(2); break;
+        case 4: TN_LAUNCH_TABLE(4); break;
+        case 8: TN_LAUNCH_TABLE(8); break;
+        case 16: TN_LAUNCH_TABLE(16); break;
+        default: TN_LAUNCH_TABLE(32); break;
+    }
+#undef TN_LAUNCH_TABLE
+#undef TN_LAUNCH_TABLE_ANY
+    return TN_OK;
+}
+
+int launch_table_apply(SparseTable* t, RowShare share, const TableShape& b, const tn_sign_info* infos, const float* grads,
+                       int dim, const uint2* recs, const uint16_t* boff, DevStatus* ds, hipStream_t st) {
+    const OptDev o = make_optdev(t);
+    switch (o.kind) {
+        case OPT_ADAGRAD: return launch_table_apply_kind<OPT_ADAGRAD>(t, share, o, b, infos, grads, dim, recs, boff, ds, st);
+        case OPT_ADAM: return launch_table_apply_kind<OPT_ADAM>(t, share, o, b, infos, grads, dim, recs, boff, ds, st);
+        default: return launch_table_apply_kind<OPT_FTRL>(t, share, o, b, infos, grads, dim, recs, boff, ds, st);
+    }
+}
+
 // Does the batch qualify for the path of few launches, and how is it laid out on it?
 bool small_batch_shape(SparseTable* t, int N, const int64_t* lens, SmallShape& b) {
     if (!t->small_path || t->async_pull || N <= 0 || N > SMALL_SLOTS || t->dim > 128) return false;
@@ -1589,35 +1639,48 @@ int tn_sparse_table_pull(uint32_t handle, const uint64_t* signs, int64_t n, int 
         return fail(TN_ERR_DIM_MISMATCH,
                     "tn_sparse_table_pull: dim " + std::to_string(dim) + " but table rows hold " + std::to_string(wdim));
     if (n > 0x7FFFFFF0LL) return fail(TN_ERR_UNSUPPORTED, "tn_sparse_table_pull: more than 2^31 signs");
-    t->last_stream = st;
-    if (n == 0) return sync_table(t, st);
-    if (t->push_pending || t->pull_pending) {
+    // a push pending on this stream is collected behind this call's own wait
+    if (t->pull_pending || (t->push_pending && t->last_stream && t->last_stream != st)) {
+        if (t->last_stream && t->last_stream != st) TN_HIP(hipStreamSynchronize(t->last_stream));
         TN_HIP(hipStreamSynchronize(st));
         harvest(t);
     }
+    t->last_stream = st;
+    if (n == 0) return sync_table(t, st);
     TN_TRY(ensure_room(t, (uint64_t)n, st));
-    TN_TRY(t->ws.ensure(2 * align_up((size_t)n * sizeof(uint32_t), 256)));
-    Carver c{(char*)t->ws.p};
-    uint32_t* rows = c.take<uint32_t>(n);
-    uint32_t* newlist = c.take<uint32_t>(n);
+    TN_TRY(t->ws.ensure(align_up((size_t)n * sizeof(uint32_t), 256)));
+    uint32_t* rows = (uint32_t*)t->ws.p;
     const Store& s = t->store;
-    const OptDev o = make_optdev(t);
-    const int blocks = launch_grid(n, 256, GRID_CAP * 2);
-    TN_LAUNCH(k_reset_status, dim3(1), dim3(64), st, t->dstatus, (uint32_t)n, 0u);
-    TN_LAUNCH((k_probe<true>), dim3(blocks), dim3(256), st, s, signs, n, (const DevStatus*)nullptr, 0u, rows, newlist, t->dstatus, (uint32_t)DEV_ERR_TABLE_FULL, make_optdev(t), t->seed);
-    TN_LAUNCH(k_init_rows, dim3(blocks), dim3(256), st, s, o, t->seed, signs, rows, newlist, t->dstatus);
-    TN_LAUNCH(k_finish_insert, dim3(1), dim3(64), st, s, t->dstatus);
-    if (wdim % 4 == 0 && s.wstride % 4 == 0 && aligned16(out))
-        TN_LAUNCH((k_gather_rows<4>), dim3(launch_grid(n * (wdim / 4), 256, GRID_CAP * 4)), dim3(256), st, s, rows, n, out);
-    else
-        TN_LAUNCH((k_gather_rows<1>), dim3(launch_grid(n * wdim, 256, GRID_CAP * 4)), dim3(256), st, s, rows, n, out);
+    const bool vec = wdim % 4 == 0 && s.wstride % 4 == 0 && aligned16(out);
+    const uint32_t per = n > 64 * (int64_t)TABLE_PULL_FEW ? 256 : 64;
+    const uint32_t workgroups = (uint32_t)std::min<int64_t>((n + per - 1) / per, TABLE_PULL_WORDS);
+    const uint32_t seq = ++t->seq_pull;
+    TN_LAUNCH(k_table_pull, dim3(workgroups), dim3(256), st, s, make_optdev(t), t->seed, signs, n, per, vec ? 1 : 0, out, rows,
+              t->hwords, seq);
     TN_HIP(hipGetLastError());
-    TN_HIP(hipMemcpyAsync(&t->hpull->st, t->dstatus, sizeof(DevStatus), hipMemcpyDeviceToHost, st));
-    t->hpull->ubase[0] = 0;
-    t->pull_pending = true;
-    t->pull_slots = 0;
-    t->pending_rows.clear();
-    return sync_table(t, st);
+    TN_TRY(wait_words(t->hwords, workgroups, seq, st, "tn_sparse_table_pull"));
+    uint64_t n_new = 0;
+    uint32_t err = 0;
+    for (uint32_t i = 0; i < workgroups; i++) {
+        n_new += t->hwords[i] & 0x7FFFFFFFu;
+        if ((t->hwords[i] >> 31) & 1u) err = DEV_ERR_TABLE_FULL;
+    }
+    harvest(t);
+    // the call booked room for every sign it could have inserted; keep what it did insert
+    t->count_upper -= t->booked - n_new;
+    t->booked = 0;
+    t->last_counts.clear();
+    latch(t, dev_err_code(err), std::string("sparse pull: ") + dev_err_text(err));
+    if (n_new) {  // a sign that occurs several times may have been copied out before its new row was filled
+        if (vec)
+            TN_LAUNCH((k_gather_rows<4>), dim3(launch_grid(n * (wdim / 4), 256, GRID_CAP * 4)), dim3(256), st, s, rows, n, out);
+        else
+            TN_LAUNCH((k_gather_rows<1>), dim3(launch_grid(n * wdim, 256, GRID_CAP * 4)), dim3(256), st, s, rows, n, out);
+        TN_HIP(hipGetLastError());
+        TN_HIP(hipStreamSynchronize(st));
+    }
+    if (t->upd_pending) return sync_table(t, st);  // (an earlier push's updates on streams of their own)
+    return take_latched(t);
 }
 
 namespace {
@@ -1728,11 +1791,52 @@ int tn_sparse_table_push(uint32_t handle, const tn_sign_info* infos, const float
         return fail(TN_ERR_DIM_MISMATCH,
                     "tn_sparse_table_push: dim " + std::to_string(dim) + " but table rows hold " + std::to_string(wdim));
     if (n > 0x7FFFFFF0LL) return fail(TN_ERR_UNSUPPORTED, "tn_sparse_table_push: more than 2^31 records");
-    t->last_stream = st;
-    if (n == 0) return TN_OK;
-    if (t->push_pending || t->pull_pending) {  // one status block per direction: collect the previous one first
+    if (n > 0 && (t->push_pending || t->pull_pending)) {  // one status block per direction: collect the previous one first
+        if (t->last_stream && t->last_stream != st) TN_HIP(hipStreamSynchronize(t->last_stream));
         TN_HIP(hipStreamSynchronize(st));
         harvest(t);
+    }
+    t->last_stream = st;
+    if (n == 0) return TN_OK;
+    const Store& s = t->store;
+    const RowShare share = row_share(s, aligned16(grads) && dim % 4 == 0 && s.wstride % 4 == 0);
+    DevStatus* ds = t->dtpush;
+    if (share.lanes != 0 && n <= (int64_t)TABLE_TILES * TABLE_THREADS * TABLE_ITEMS_MAX) {
+        // two launches (table_level.h), for rows of up to 128 elements (a wavefront half holds no more) and up to 2 M
+        // records (a bucket's workgroup looks at every tile, and a tile holds what a workgroup keeps in registers)
+        TableShape b{};
+        b.n = (uint32_t)n;
+        b.tile = TABLE_THREADS;
+        while (b.tile < (uint32_t)(TABLE_THREADS * TABLE_ITEMS_MAX) && (n + b.tile - 1) / b.tile > (int64_t)TABLE_TILES) b.tile *= 4;
+        b.tiles = (uint32_t)((n + b.tile - 1) / b.tile);
+        b.nb = (uint32_t)std::min<int64_t>({(n + TABLE_BUCKET_RECORDS - 1) / TABLE_BUCKET_RECORDS, (int64_t)TABLE_BUCKETS,
+                                            (int64_t)(s.cap / 64)});
+        b.scale = (uint32_t)((((uint64_t)b.nb << 32)) / (s.cap + 1));
+        while ((1u << b.bits) < b.nb) b.bits++;
+        auto carve = [&](Carver& c, uint2*& recs, uint16_t*& boff) {
+            recs = c.take<uint2>((size_t)b.tiles * b.tile);
+            boff = c.take<uint16_t>((size_t)b.tiles * (b.nb + 1));
+        };
+        uint2* recs = nullptr;
+        uint16_t* boff = nullptr;
+        Carver room{nullptr};
+        carve(room, recs, boff);
+        TN_TRY(t->ws.ensure(align_up(room.off, 256) + 256));
+        Carver c{(char*)t->ws.p};
+        carve(c, recs, boff);
+        const size_t part_lds = (size_t)b.nb * TABLE_WAVES * sizeof(uint32_t);
+        if (b.tile == TABLE_THREADS)
+            TN_LAUNCH_LDS((k_table_part<1>), dim3(b.tiles), dim3(TABLE_THREADS), part_lds, st, b, s, infos, recs, boff, ds);
+        else if (b.tile == 4 * TABLE_THREADS)
+            TN_LAUNCH_LDS((k_table_part<4>), dim3(b.tiles), dim3(TABLE_THREADS), part_lds, st, b, s, infos, recs, boff, ds);
+        else
+            TN_LAUNCH_LDS((k_table_part<16>), dim3(b.tiles), dim3(TABLE_THREADS), part_lds, st, b, s, infos, recs, boff, ds);
+        t->hpush->st.err = 0;
+        TN_TRY(launch_table_apply(t, share, b, infos, grads, dim, recs, boff, ds, st));
+        TN_HIP(hipGetLastError());
+        t->push_pending = true;
+        t->push_slots = 0;
+        return TN_OK;
     }
     Plan p{};
     Scratch w{};
@@ -1749,7 +1853,7 @@ int tn_sparse_table_push(uint32_t handle, const tn_sign_info* infos, const float
     src.infos = infos;
     src.grads = grads;
     src.dim = dim;
-    DevStatus* ds = t->dstatus;
+    ds = t->dstatus;
     TN_LAUNCH(k_reset_status, dim3(1), dim3(64), st, ds, (uint32_t)n, (uint32_t)group_cap((size_t)n));
     launch_grouping(p, w, src, n, n, big_threshold(t->store), nullptr, ds, st);
     TN_LAUNCH((k_probe<false>), dim3(launch_grid(n, 256, GRID_CAP * 2)), dim3(256), st, t->store, p.grp_sign,
