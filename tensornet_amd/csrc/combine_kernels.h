@@ -140,35 +140,90 @@ __global__ void k_report(DevStatus* status, uint64_t* host_word, uint32_t seq) {
 
 // Backward, step 1: the value of every lookup: its example in the high word, the number of
 // lookups of that example in the low word -- all the reduction needs to know about the lookup, so
-// that it reads them in the order of the distinct signs instead of chasing positions.  The first
-// lookup of an example writes the values of all its lookups.
+// that it reads them in the order of the distinct signs instead of chasing positions.
+//
+// 16 bytes move per lookup; what bounded it were chains of loads (a thread found the slot of a lookup by bisection, then
+// its descriptor, then its id, and the first lookup of an example walked to its last one and wrote all their values).
+// A wavefront now takes KEY_ITEMS runs of 64 lookups, their loads in flight together, and reads the extents of its
+// examples off a ballot of the places where the id changes; an example that goes on beyond the run is followed there by
+// the whole wavefront.  4.9 M lookups: 60 -> 35 us.
+constexpr int KEY_ITEMS = 4;
+constexpr uint32_t KEY_TILE = 256 * KEY_ITEMS;
+
 __global__ __launch_bounds__(256) void k_lookup_keys(const SlotDesc* __restrict__ descs,
                                                      const uint32_t* __restrict__ lbase, int N, uint32_t L,
                                                      int64_t batch, uint64_t* __restrict__ vals, DevStatus* status,
                                                      uint32_t* long_count) {
     __shared__ uint32_t lb[MAX_SLOTS + 1];
     load_lbase(lb, lbase, N);
-    // [0] list of the frequent signs, filled by k_reduce_pooled; [1], [2] lists of k_place_lookups
+    // [1], [2]: entries of the lists of k_place_lookups
     if (blockIdx.x == 0 && threadIdx.x < 3) long_count[threadIdx.x] = 0;
-    const uint32_t stride = gridDim.x * blockDim.x;
-    for (uint32_t gi = blockIdx.x * blockDim.x + threadIdx.x; gi < L; gi += stride) {
-        const int sl = find_slot(lb, N, gi);
-        const SlotDesc& d = descs[sl];
-        const int64_t* ex = example_of(d);
-        const uint32_t i = gi - lb[sl];
-        const int64_t b = ex[i];
-        const int64_t prev = i > 0 ? ex[i - 1] : -1;
-        if (b < 0 || b >= batch || prev > b) {
-            atomicOr(&status->err, DEV_ERR_GRAD_ROWS);
-            status->abort = 1;  // values of later lookups may never be written: nothing downstream may run
-            vals[gi] = ~0ull;
-            continue;
+    const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const uint32_t ntiles = (L + KEY_TILE - 1) / KEY_TILE;
+    for (uint32_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+        const uint32_t g0 = tile * KEY_TILE, g1 = min(L, g0 + KEY_TILE) - 1;
+        const int s0 = find_slot(lb, N, g0);
+        const bool one_slot = g1 < lb[s0 + 1];  // the usual case: the tile lies inside one slot
+        int sl[KEY_ITEMS];
+        int64_t b[KEY_ITEMS], prev[KEY_ITEMS];
+#pragma unroll
+        for (int j = 0; j < KEY_ITEMS; j++) {
+            const uint32_t gi = g0 + (wave * KEY_ITEMS + j) * 64 + lane;
+            sl[j] = s0;
+            b[j] = prev[j] = -1;
+            if (gi <= g1) {
+                if (!one_slot) sl[j] = find_slot(lb, N, gi);
+                const int64_t* ex = example_of(descs[sl[j]]);
+                const uint32_t i = gi - lb[sl[j]];
+                b[j] = ex[i];
+                if (i > 0) prev[j] = ex[i - 1];
+            }
         }
-        if (prev == b) continue;
-        uint32_t j = i;
-        while (j < d.len && ex[j] == b) j++;
-        const uint64_t v = ((uint64_t)b << 32) | (uint64_t)(j - i);
-        for (uint32_t q = i; q < j; q++) vals[lb[sl] + q] = v;
+#pragma unroll
+        for (int j = 0; j < KEY_ITEMS; j++) {
+            const uint32_t base = g0 + (wave * KEY_ITEMS + j) * 64, gi = base + lane;
+            const bool active = gi <= g1;
+            if (active && (b[j] < 0 || b[j] >= batch || prev[j] > b[j])) {
+                atomicOr(&status->err, DEV_ERR_GRAD_ROWS);
+                status->abort = 1;  // nothing downstream may run
+            }
+            // where an example starts (the first lookup of a slot does: prev is -1 there; and what lies behind the last one)
+            const unsigned long long heads = __ballot(!active || b[j] != prev[j]);
+            uint32_t back = 0, ahead = 0;  // lookups of the first / last example of the run before / behind it
+            if (!(heads & 1ull)) {
+                const int64_t x = __shfl(b[j], 0);
+                const int s = __shfl(sl[j], 0);
+                const int64_t* ex = example_of(descs[s]);
+                for (uint32_t i = base - lb[s];; i -= 64) {  // lookups [0, i) of the slot are left
+                    const unsigned long long other = __ballot(lane >= i || ex[i - 1 - lane] != x);
+                    if (other) {
+                        back += (uint32_t)__ffsll((long long)other) - 1;
+                        break;
+                    }
+                    back += 64;
+                }
+            }
+            if (base + 63 <= g1) {
+                const int64_t x = __shfl(b[j], 63);
+                const int s = __shfl(sl[j], 63);
+                const int64_t* ex = example_of(descs[s]);
+                const uint32_t len = lb[s + 1] - lb[s];
+                for (uint32_t i = base + 64 - lb[s];; i += 64) {
+                    const unsigned long long other = __ballot(i + lane >= len || ex[i + lane] != x);
+                    if (other) {
+                        ahead += (uint32_t)__ffsll((long long)other) - 1;
+                        break;
+                    }
+                    ahead += 64;
+                }
+            }
+            if (active) {
+                const unsigned long long below = heads & (~0ull >> (63 - lane)), above = heads & ~(~0ull >> (63 - lane));
+                const uint32_t to_start = below ? lane - (63 - (uint32_t)__clzll((long long)below)) : lane + back;
+                const uint32_t to_end = above ? (uint32_t)__ffsll((long long)above) - 1 - lane : 64 - lane + ahead;
+                vals[gi] = ((uint64_t)b[j] << 32) | (uint64_t)(to_start + to_end);
+            }
+        }
     }
 }
 
@@ -370,30 +425,47 @@ __global__ __launch_bounds__(256) void k_order_huge(const uint32_t* __restrict__
     }
 }
 
-// The share of a lookup in the gradient of its distinct sign: its example's pooled row times
-// 1 / d(lookups of the example), chunk c.
-template <int VEC>
-__device__ __forceinline__ void add_lookup_share(const float* __restrict__ pooled, uint64_t v, int dim, int c,
-                                                 int combiner, float (&acc)[VEC]) {
-    if (v == ~0ull) return;  // flagged by k_lookup_keys
-    const uint32_t b = (uint32_t)(v >> 32);
-    const float scale = combiner == COMBINE_SUM ? 1.f : 1.f / combine_divisor((uint32_t)v, combiner);
-    const float* row = pooled + (uint64_t)b * dim + c * VEC;
-    if (VEC == 4) {
-        const float4 g = *reinterpret_cast<const float4*>(row);
-        acc[0] += g.x * scale;
-        acc[1] += g.y * scale;
-        acc[2] += g.z * scale;
-        acc[3] += g.w * scale;
-    } else {
-        acc[0] += row[0] * scale;
+// The sum of the shares of lookups from, from + step, ... below `to` of one distinct sign, in this order: every lookup
+// has its example's pooled row times 1 / d(lookups of the example); four elements of a row, part c of them.  The
+// values of a window first, then their rows, all loads of a kind independent.
+template <bool ANY>
+__device__ __forceinline__ float4 sum_shares(const float* __restrict__ pooled, const uint64_t* __restrict__ svals, uint32_t from,
+                                             uint32_t to, uint32_t step, int dim, int c, int combiner) {
+    float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (uint32_t j0 = from; j0 < to; j0 += COMBINE_WINDOW * step) {
+        uint64_t v[COMBINE_WINDOW];
+        float4 g[COMBINE_WINDOW];
+#pragma unroll
+        for (int q = 0; q < COMBINE_WINDOW; q++) v[q] = j0 + q * step < to ? svals[j0 + q * step] : 0ull;
+#pragma unroll
+        for (int q = 0; q < COMBINE_WINDOW; q++)
+            g[q] = j0 + q * step < to ? row_part<ANY>(pooled + (v[q] >> 32) * (uint64_t)dim, c, dim)
+                                      : make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+        for (int q = 0; q < COMBINE_WINDOW; q++) {
+            if (j0 + q * step >= to) break;
+            const float scale = combiner == COMBINE_SUM ? 1.f : 1.f / combine_divisor((uint32_t)v[q], combiner);
+            acc.x += g[q].x * scale;
+            acc.y += g[q].y * scale;
+            acc.z += g[q].z * scale;
+            acc.w += g[q].w * scale;
+        }
     }
+    return acc;
 }
 
-// Step 3: one group of `chunks` threads per distinct index sums its lookups' shares of the
-// pooled gradient rows, in position order.  A distinct index with long_min lookups or more (a
-// frequent sign) is left out: k_place_lookups has listed those, one workgroup each sums them (k_reduce_long).
-template <int VEC>
+// Step 3: a group of `chunks` threads per distinct index, four elements of the row each (whatever its length and
+// alignment), sums its lookups' shares of the pooled gradient rows, in position order.  A distinct index with long_min
+// lookups or more (a frequent sign) is left out: k_place_lookups has listed those, one workgroup each sums them
+// (k_reduce_long).
+//
+// Bound by the rows it reads again and again: the pooled rows of a slot (1 MB at 16384 examples of 16 elements) stay in
+// the L2 of a die that works on one slot at a time, so the distinct indices go to the dies in runs of REDUCE_RUN
+// workgroups (DieRuns; a grid-stride loop had every die read the rows of six slots).  4.9 M lookups of 16 elements:
+// 172 -> 138 us, the frequent signs beside it 120 -> 93 us.
+constexpr uint32_t REDUCE_RUN = 256;
+
+template <bool ANY>
 __global__ __launch_bounds__(256) void k_reduce_pooled(const SlotDesc* __restrict__ descs,
                                                        const uint32_t* __restrict__ ubase, int N, int dim,
                                                        int combiner, const DevStatus* status,
@@ -403,39 +475,24 @@ __global__ __launch_bounds__(256) void k_reduce_pooled(const SlotDesc* __restric
     if (status->abort) return;
     __shared__ uint32_t ub[MAX_SLOTS + 1];
     load_lbase(ub, ubase, N);
-    const int chunks = dim / VEC;
-    const int64_t total = (int64_t)status->n_unique * chunks;
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < total; t += stride) {
+    const uint32_t chunks = (uint32_t)(dim + 3) / 4;
+    const uint64_t total = (uint64_t)status->n_unique * chunks;
+    for (DieRuns r((uint32_t)((total + 255) / 256), REDUCE_RUN); r.more(); r.next()) {
+        const uint64_t t = (uint64_t)r.item() * 256 + threadIdx.x;
+        if (t >= total) continue;
         const uint32_t u = (uint32_t)(t / chunks);
-        const int c = (int)(t - (int64_t)u * chunks);
+        const int c = (int)(t - (uint64_t)u * chunks);
         const uint32_t lo = seg_off[u], hi = seg_off[u + 1];
-        if (hi - lo >= long_min) continue;  // (listed by k_place_lookups: k_reduce_long sums those)
-        float acc[VEC];
-#pragma unroll
-        for (int q = 0; q < VEC; q++) acc[q] = 0.f;
+        if (hi - lo >= long_min) continue;
         const float* pooled = descs[find_slot(ub, N, u)].grads;  // the slot whose window of distinct indices holds u
-        for (uint32_t j0 = lo; j0 < hi; j0 += COMBINE_WINDOW) {  // values of a window first, then their rows
-            uint64_t wv[COMBINE_WINDOW];
-#pragma unroll
-            for (int q = 0; q < COMBINE_WINDOW; q++) wv[q] = (j0 + q < hi) ? svals[j0 + q] : ~0ull;
-#pragma unroll
-            for (int q = 0; q < COMBINE_WINDOW; q++) add_lookup_share<VEC>(pooled, wv[q], dim, c, combiner, acc);
-        }
-        float* o = flat + (uint64_t)u * dim + c * VEC;
-        if (VEC == 4)
-            *reinterpret_cast<float4*>(o) = make_float4(acc[0], acc[1], acc[2], acc[3]);
-        else
-            o[0] = acc[0];
+        put_row_part<ANY>(flat + (uint64_t)u * dim, c, dim, sum_shares<ANY>(pooled, svals, lo, hi, 1, dim, c, combiner));
     }
 }
 
 // One workgroup per frequent distinct index: its 256 / chunks thread groups each sum every
 // (256 / chunks)-th lookup in position order, then the partial sums are added in group order.
 // The order of the additions is fixed, so the result does not vary from run to run.
-constexpr int LONG_PART_FLOATS = 1024;  // 256 threads x 4 floats
-
-template <int VEC>
+template <bool ANY>
 __global__ __launch_bounds__(256) void k_reduce_long(const SlotDesc* __restrict__ descs,
                                                      const uint32_t* __restrict__ ubase, int N, int dim, int combiner,
                                                      const uint32_t* __restrict__ seg_off,
@@ -444,8 +501,8 @@ __global__ __launch_bounds__(256) void k_reduce_long(const SlotDesc* __restrict_
                                                      const uint32_t* __restrict__ huge_list,
                                                      const uint32_t* counts, const DevStatus* status) {
     if (status->abort) return;
-    __shared__ float part[LONG_PART_FLOATS];
-    const int chunks = dim / VEC;
+    __shared__ float4 part[256];
+    const int chunks = (dim + 3) / 4;
     const int groups = 256 / chunks;
     const int q = threadIdx.x / chunks, c = threadIdx.x - q * chunks;
     // the frequent ones: the two lists k_place_lookups left (ORDER_MID lookups or more)
@@ -454,33 +511,18 @@ __global__ __launch_bounds__(256) void k_reduce_long(const SlotDesc* __restrict_
         const uint32_t u = k < n_mid ? mid_list[k] : huge_list[k - n_mid];
         const uint32_t lo = seg_off[u], hi = seg_off[u + 1];
         const float* pooled = descs[find_slot(ubase, N, u)].grads;
-        float acc[VEC];
-#pragma unroll
-        for (int v = 0; v < VEC; v++) acc[v] = 0.f;
-        if (q < groups) {
-            for (uint32_t j0 = lo + q; j0 < hi; j0 += COMBINE_WINDOW * groups) {  // values of a window first, then their rows
-                uint64_t wv[COMBINE_WINDOW];
-#pragma unroll
-                for (int w = 0; w < COMBINE_WINDOW; w++) wv[w] = (j0 + w * groups < hi) ? svals[j0 + w * groups] : ~0ull;
-#pragma unroll
-                for (int w = 0; w < COMBINE_WINDOW; w++) add_lookup_share<VEC>(pooled, wv[w], dim, c, combiner, acc);
-            }
-        }
-#pragma unroll
-        for (int v = 0; v < VEC; v++) part[threadIdx.x * VEC + v] = acc[v];
+        if (q < groups) part[threadIdx.x] = sum_shares<ANY>(pooled, svals, lo + q, hi, groups, dim, c, combiner);
         __syncthreads();
         if (q == 0) {
-            float sum[VEC];
-#pragma unroll
-            for (int v = 0; v < VEC; v++) sum[v] = 0.f;
-            for (int g = 0; g < groups; g++)
-#pragma unroll
-                for (int v = 0; v < VEC; v++) sum[v] += part[(g * chunks + c) * VEC + v];
-            float* o = flat + (uint64_t)u * dim + c * VEC;
-            if (VEC == 4)
-                *reinterpret_cast<float4*>(o) = make_float4(sum[0], sum[1], sum[2], sum[3]);
-            else
-                o[0] = sum[0];
+            float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
+            for (int g = 0; g < groups; g++) {
+                const float4 p = part[g * chunks + c];
+                sum.x += p.x;
+                sum.y += p.y;
+                sum.z += p.z;
+                sum.w += p.w;
+            }
+            put_row_part<ANY>(flat + (uint64_t)u * dim, c, dim, sum);
         }
         __syncthreads();
     }

@@ -2322,7 +2322,7 @@ int push_op_impl(uint32_t table_handle, int N, const int64_t* const* values, con
         TN_TRY(t->pooled_ws.ensure(align_up(c.off, 256)));
         Carver c2{(char*)t->pooled_ws.p};
         carve(c2);
-        TN_LAUNCH(k_lookup_keys, dim3(lblocks), dim3(256), st, pd, p.lbase, N, (uint32_t)L, batch, vals, ds, long_count);
+        TN_LAUNCH(k_lookup_keys, dim3(launch_grid((int64_t)(L + KEY_TILE - 1) / KEY_TILE, 1, GRID_CAP * 2)), dim3(256), st, pd, p.lbase, N, (uint32_t)L, batch, vals, ds, long_count);
         // The lookups of every distinct sign side by side, ascending by example (= by position): into their
         // sign's segment first, then ordered inside it.  A few workgroups per slot, each with an LDS counter per
         // distinct index of its share of the slot (a slot has at most as many as lookups).
@@ -2355,7 +2355,7 @@ int push_op_impl(uint32_t table_handle, int N, const int64_t* const* values, con
                       (uint32_t)batch, huge_in_lds ? 1 : 0, gcnt, ds);
         // signs with LONG_SEGMENT lookups or more get a workgroup each instead of one thread group
         static_assert(LONG_SEGMENT == ORDER_MID, "the lists of k_place_lookups are the frequent signs of k_reduce_long");
-        const int chunks = vec ? grad_dim / 4 : grad_dim;
+        const int chunks = (grad_dim + 3) / 4;
         const uint32_t long_min = chunks <= 256 ? LONG_SEGMENT : 0xFFFFFFFFu;
         const int long_blocks = launch_grid((int64_t)L / LONG_SEGMENT + 1, 1, GRID_CAP);
         if (fork) {
@@ -2363,18 +2363,19 @@ int push_op_impl(uint32_t table_handle, int N, const int64_t* const* values, con
             TN_HIP(hipEventRecord(t->join2_ev, t->side2));
             TN_HIP(hipStreamWaitEvent(t->side, t->join2_ev, 0));
         }
+        // (a macro: the profiler names a kernel by the text of its launch)
+#define TN_REDUCE(ANY)                                                                                               \
+    TN_LAUNCH((k_reduce_pooled<ANY>), dim3(launch_grid((int64_t)L * chunks, 256, GRID_CAP * 4)), dim3(256), st, pd,  \
+              p.ubase, N, grad_dim, combiner, ds, seg_off, svals, flat, long_min);                                   \
+    if (long_min != 0xFFFFFFFFu)                                                                                     \
+        TN_LAUNCH((k_reduce_long<ANY>), dim3(long_blocks), dim3(256), s_mid, pd, p.ubase, N, grad_dim, combiner,     \
+                  seg_off, svals, flat, mid_list, huge_list, long_count, ds)
         if (vec) {
-            TN_LAUNCH((k_reduce_pooled<4>), dim3(launch_grid((int64_t)L * chunks, 256, GRID_CAP * 4)), dim3(256), st,
-                      pd, p.ubase, N, grad_dim, combiner, ds, seg_off, svals, flat, long_min);
-            TN_LAUNCH((k_reduce_long<4>), dim3(long_blocks), dim3(256), s_mid, pd, p.ubase, N, grad_dim, combiner,
-                      seg_off, svals, flat, mid_list, huge_list, long_count, ds);
+            TN_REDUCE(false);
         } else {
-            TN_LAUNCH((k_reduce_pooled<1>), dim3(launch_grid((int64_t)L * chunks, 256, GRID_CAP * 4)), dim3(256), st,
-                      pd, p.ubase, N, grad_dim, combiner, ds, seg_off, svals, flat, long_min);
-            if (long_min != 0xFFFFFFFFu)
-                TN_LAUNCH((k_reduce_long<1>), dim3(long_blocks), dim3(256), s_mid, pd, p.ubase, N, grad_dim,
-                          combiner, seg_off, svals, flat, mid_list, huge_list, long_count, ds);
+            TN_REDUCE(true);
         }
+#undef TN_REDUCE
         if (fork) {
             TN_HIP(hipEventRecord(t->join_ev, t->side));
             TN_HIP(hipStreamWaitEvent(st, t->join_ev, 0));
