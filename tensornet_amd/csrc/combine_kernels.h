@@ -10,7 +10,7 @@
 //
 // Both are deterministic: sums run in occurrence order.  The backward pass
 // gets the lookups of every distinct sign side by side, in position order, from a
-// counting sort per slot followed by an ordering of every sign's lookups by example
+// counting sort per slot followed by an ordering of every sign's lookups by position
 // (k_place_lookups, k_rank_short, k_rank_mid, k_order_huge).
 #ifndef TN_COMBINE_KERNELS_H_
 #define TN_COMBINE_KERNELS_H_
@@ -228,16 +228,15 @@ __global__ __launch_bounds__(256) void k_lookup_keys(const SlotDesc* __restrict_
 }
 
 // Step 2: the values of the lookups of every distinct index side by side, in position order:
-// svals[seg_off[u] .. seg_off[u + 1]).  The example ids of a slot ascend with the position and two lookups of
-// one sign in one example carry the same value, so "position order" is "ascending value" and ties do not
-// matter: no stable sort is needed.
+// svals[seg_off[u] .. seg_off[u + 1]).
 //   k_place_lookups  a few workgroups per slot (the distinct indices of a slot's lookups fill a window of their
 //                    own, ascending with the slots): counts the lookups of every index in an LDS array, scans
-//                    the counts into seg_off, and puts every lookup into its index's segment -- in the order the
-//                    atomics arrive; indices with ORDER_MID lookups or more are listed for the kernels below
-//   k_rank_short     a lookup of a short segment finds its place by counting the values of its segment below it
+//                    the counts into seg_off, and puts the position of every lookup into its index's segment -- in
+//                    the order the atomics arrive; indices with ORDER_MID lookups or more are listed for the kernels
+//                    below
+//   k_rank_short     a lookup of a short segment finds its place by counting the positions of its segment below its own
 //   k_rank_mid       a sorting network in LDS, one workgroup per segment of ORDER_MID .. ORDER_HUGE - 1 lookups
-//   k_order_huge     the few longer segments: counting sort over the example ids, one workgroup each
+//   k_order_huge     the few longer segments: a bitmap of their positions in LDS, one workgroup each
 // A slot with more distinct signs than the LDS array holds (lds_cap) keeps its counters in `gcur`.
 constexpr int PLACE_THREADS = 1024;
 constexpr int PLACE_ITEMS = 8;
@@ -245,16 +244,18 @@ constexpr uint32_t ORDER_MID = 64;
 constexpr uint32_t ORDER_HUGE = 1024;
 
 // `parts` workgroups per slot: each of them streams all lookups of the slot (they come out of L2 after the first)
-// and takes those whose distinct index lies in its share of the slot's window of distinct indices -- a workgroup
-// per slot leaves most of the device idle, and what bounds it are the LDS atomics and the stores that depend on
-// them, which a share divides.  The lookups of the indices below its share, which it counts on the way, come
-// before its own in svals.
+// and takes those whose distinct index lies in its share of the slot's window of distinct indices.  The lookups of the
+// indices below its share, which it counts on the way, come before its own.
+//
+// What bounds it are the scattered stores: a die has the windows of a dozen slots in its L2 at a time, and lines that are
+// written out half filled are read and written again.  Only the position is stored, 4 bytes per lookup (a die's windows:
+// 2.5 MB at 49 k lookups a slot), and not the index and the value with it (12 bytes, 7.5 MB: more than its L2).
+// 4.9 M lookups in 100 slots: 168 us before, 135 with one workgroup per slot and 125 with two.
 __global__ __launch_bounds__(PLACE_THREADS) void k_place_lookups(
     const uint32_t* __restrict__ lbase, const uint32_t* __restrict__ ubase, int N, uint32_t L,
-    const uint32_t* __restrict__ u_of_gi, const uint64_t* __restrict__ vals, uint32_t* __restrict__ tkey,
-    uint64_t* __restrict__ tval, uint32_t* __restrict__ seg_off, uint32_t* __restrict__ gcur, uint32_t lds_cap,
-    uint32_t* __restrict__ mid_list, uint32_t* __restrict__ huge_list, uint32_t* counts, const DevStatus* status,
-    uint32_t parts) {
+    const uint32_t* __restrict__ u_of_gi, uint32_t* __restrict__ tpos, uint32_t* __restrict__ seg_off,
+    uint32_t* __restrict__ gcur, uint32_t lds_cap, uint32_t* __restrict__ mid_list, uint32_t* __restrict__ huge_list,
+    uint32_t* counts, const DevStatus* status, uint32_t parts) {
     extern __shared__ uint32_t lcur[];
     __shared__ uint32_t red[PLACE_THREADS / 64];
     __shared__ uint32_t carry_sh;
@@ -315,48 +316,45 @@ __global__ __launch_bounds__(PLACE_THREADS) void k_place_lookups(
     }
     for (uint32_t i0 = threadIdx.x; i0 < len; i0 += PLACE_THREADS * PLACE_ITEMS) {
         uint32_t k[PLACE_ITEMS];
-        uint64_t v[PLACE_ITEMS];
 #pragma unroll
         for (int j = 0; j < PLACE_ITEMS; j++) {
             const uint32_t i = i0 + j * PLACE_THREADS;
             k[j] = i < len ? (keys[i] & ~FIRST_BIT) - ub : 0xFFFFFFFFu;
-            v[j] = (k[j] >= r0 && k[j] < r1) ? vals[l0 + i] : 0ull;
         }
 #pragma unroll
-        for (int j = 0; j < PLACE_ITEMS; j++) {
-            if (k[j] < r0 || k[j] >= r1) continue;
-            const uint32_t at = atomicAdd(&cur[k[j] - r0], 1u);
-            tkey[at] = ub + k[j];
-            tval[at] = v[j];
-        }
+        for (int j = 0; j < PLACE_ITEMS; j++)
+            if (k[j] >= r0 && k[j] < r1) tpos[atomicAdd(&cur[k[j] - r0], 1u)] = l0 + i0 + j * PLACE_THREADS;
     }
 }
 
-__global__ __launch_bounds__(256) void k_rank_short(uint32_t L, const uint32_t* __restrict__ tkey,
-                                                    const uint64_t* __restrict__ tval,
+// The lookups in the order of their segments: the runs of a die (DieRuns) keep to one slot, whose distinct indices and
+// values, read by position, are then in its L2.  4.9 M lookups: 78 -> 62 us.
+constexpr uint32_t RANK_RUN = 128;
+
+__global__ __launch_bounds__(256) void k_rank_short(uint32_t L, const uint32_t* __restrict__ u_of_gi,
+                                                    const uint64_t* __restrict__ vals, const uint32_t* __restrict__ tpos,
                                                     const uint32_t* __restrict__ seg_off, uint64_t* __restrict__ svals,
                                                     const DevStatus* status) {
     if (status->abort) return;
-    const uint32_t stride = gridDim.x * blockDim.x;
-    for (uint32_t t = blockIdx.x * blockDim.x + threadIdx.x; t < L; t += stride) {
-        const uint32_t u = tkey[t];
+    for (DieRuns r((L + 255) / 256, RANK_RUN); r.more(); r.next()) {
+        const uint32_t t = r.item() * 256 + threadIdx.x;
+        if (t >= L) continue;
+        const uint32_t gi = tpos[t];
+        const uint32_t u = u_of_gi[gi] & ~FIRST_BIT;
+        const uint64_t v = vals[gi];
         const uint32_t lo = seg_off[u], hi = seg_off[u + 1];
         if (hi - lo >= ORDER_MID) continue;
-        const uint64_t v = tval[t];
         uint32_t rank = 0;
-        for (uint32_t j = lo; j < hi; j++) {
-            const uint64_t o = tval[j];
-            rank += (o < v || (o == v && j < t)) ? 1u : 0u;
-        }
+        for (uint32_t j = lo; j < hi; j++) rank += tpos[j] < gi ? 1u : 0u;
         svals[lo + rank] = v;
     }
 }
 
 __global__ __launch_bounds__(256) void k_rank_mid(const uint32_t* __restrict__ mid_list, const uint32_t* counts,
-                                                  const uint32_t* __restrict__ seg_off,
-                                                  const uint64_t* __restrict__ tval, uint64_t* __restrict__ svals,
+                                                  const uint32_t* __restrict__ seg_off, const uint64_t* __restrict__ vals,
+                                                  const uint32_t* __restrict__ tpos, uint64_t* __restrict__ svals,
                                                   const DevStatus* status) {
-    __shared__ uint64_t seg[ORDER_HUGE];
+    __shared__ uint32_t seg[ORDER_HUGE];
     if (status->abort) return;
     const uint32_t n_mid = counts[1];
     for (uint32_t k = blockIdx.x; k < n_mid; k += gridDim.x) {
@@ -365,7 +363,7 @@ __global__ __launch_bounds__(256) void k_rank_mid(const uint32_t* __restrict__ m
         uint32_t p2 = ORDER_MID;
         while (p2 < n) p2 <<= 1;
         // bitonic sorting network over the segment padded with the largest value to a power of two
-        for (uint32_t i = threadIdx.x; i < p2; i += 256) seg[i] = i < n ? tval[lo + i] : ~0ull;
+        for (uint32_t i = threadIdx.x; i < p2; i += 256) seg[i] = i < n ? tpos[lo + i] : 0xFFFFFFFFu;
         __syncthreads();
         for (uint32_t size = 2; size <= p2; size <<= 1) {
             for (uint32_t stride = size >> 1; stride > 0; stride >>= 1) {
@@ -373,7 +371,7 @@ __global__ __launch_bounds__(256) void k_rank_mid(const uint32_t* __restrict__ m
                     const uint32_t a = 2 * t - (t & (stride - 1));  // lower element of the t-th pair
                     const uint32_t b = a + stride;
                     const bool up = (a & size) == 0;
-                    const uint64_t x = seg[a], y = seg[b];
+                    const uint32_t x = seg[a], y = seg[b];
                     if ((x > y) == up) {
                         seg[a] = y;
                         seg[b] = x;
@@ -382,46 +380,57 @@ __global__ __launch_bounds__(256) void k_rank_mid(const uint32_t* __restrict__ m
                 __syncthreads();
             }
         }
-        for (uint32_t i = threadIdx.x; i < n; i += 256) svals[lo + i] = seg[i];
+        for (uint32_t i = threadIdx.x; i < n; i += 256) svals[lo + i] = vals[seg[i]];
         __syncthreads();
     }
 }
 
-// cnt: `batch` counters in LDS (in_lds) or in a part of gcnt of the workgroup's own.
+// A segment of many lookups is ordered by a bitmap of their positions in the slot, HUGE_WINDOW of these at a time (the
+// place of a lookup: bits set below its own).  The bitmap of a slot of 49 k lookups with its prefix sums takes 9 KB of LDS,
+// so a CU holds eight workgroups; counters per example, as this had before, took 64 KB at 16384 examples, or memory.
+// Beside k_rank_mid (72 -> 42 us), 4.9 M lookups: 57 -> 34 us.
+constexpr uint32_t HUGE_WINDOW = 1u << 17;
+inline size_t order_huge_lds(size_t max_len) { return (std::min<size_t>(max_len, HUGE_WINDOW) + 63) / 64 * 12; }
+
 __global__ __launch_bounds__(256) void k_order_huge(const uint32_t* __restrict__ huge_list, const uint32_t* counts,
-                                                    const uint32_t* __restrict__ seg_off,
-                                                    const uint64_t* __restrict__ tval, uint64_t* __restrict__ svals,
-                                                    uint32_t batch, int in_lds, uint32_t* __restrict__ gcnt,
-                                                    const DevStatus* status) {
-    extern __shared__ uint32_t lcnt[];
+                                                    const uint32_t* __restrict__ lbase, const uint32_t* __restrict__ ubase,
+                                                    int N, const uint32_t* __restrict__ seg_off,
+                                                    const uint64_t* __restrict__ vals, const uint32_t* __restrict__ tpos,
+                                                    uint64_t* __restrict__ svals, uint32_t room, const DevStatus* status) {
+    extern __shared__ unsigned long long bits[];  // [room], then [room] set bits before the word
     __shared__ uint32_t red[4];
-    __shared__ uint32_t carry_sh;
     if (status->abort) return;
-    uint32_t* const cnt = in_lds ? lcnt : gcnt + (size_t)blockIdx.x * batch;
+    uint32_t* const before = reinterpret_cast<uint32_t*>(bits + room);
     const uint32_t n_huge = counts[2];
     for (uint32_t k = blockIdx.x; k < n_huge; k += gridDim.x) {
         const uint32_t u = huge_list[k];
         const uint32_t lo = seg_off[u], hi = seg_off[u + 1];
-        for (uint32_t i = threadIdx.x; i < batch; i += 256) cnt[i] = 0;
-        if (threadIdx.x == 0) carry_sh = 0;
-        __syncthreads();
-        for (uint32_t j = lo + threadIdx.x; j < hi; j += 256) atomicAdd(&cnt[(uint32_t)(tval[j] >> 32)], 1u);
-        __syncthreads();
-        for (uint32_t i0 = 0; i0 < batch; i0 += 256) {
-            const uint32_t i = i0 + threadIdx.x;
-            const uint32_t c = i < batch ? ld_relaxed(cnt + i) : 0u;
-            uint32_t total;
-            const uint32_t at = carry_sh + block_excl_scan_256<uint32_t>(c, red, &total);
-            if (i < batch) cnt[i] = at;
+        const int sl = find_slot(ubase, N, u);
+        const uint32_t l0 = lbase[sl], len = lbase[sl + 1] - l0;
+        uint32_t done = 0;  // lookups of the windows before
+        for (uint32_t w0 = 0; w0 < len; w0 += HUGE_WINDOW) {
+            const uint32_t span = min(len - w0, HUGE_WINDOW), words = (span + 63) / 64;  // (words <= room)
+            for (uint32_t i = threadIdx.x; i < words; i += 256) bits[i] = 0;
             __syncthreads();
-            if (threadIdx.x == 0) carry_sh += total;
+            for (uint32_t j = lo + threadIdx.x; j < hi; j += 256) {
+                const uint32_t p = tpos[j] - l0 - w0;  // (a position before the window: beyond it)
+                if (p < span) atomicOr(&bits[p >> 6], 1ull << (p & 63));
+            }
+            __syncthreads();
+            for (uint32_t i0 = 0; i0 < words; i0 += 256) {
+                const uint32_t i = i0 + threadIdx.x;
+                uint32_t total;
+                const uint32_t x = block_excl_scan_256<uint32_t>(i < words ? (uint32_t)__popcll(bits[i]) : 0u, red, &total);
+                if (i < words) before[i] = done + x;
+                done += total;
+                __syncthreads();
+            }
+            for (uint32_t j = lo + threadIdx.x; j < hi; j += 256) {
+                const uint32_t gi = tpos[j], p = gi - l0 - w0;
+                if (p < span) svals[lo + before[p >> 6] + (uint32_t)__popcll(bits[p >> 6] & ((1ull << (p & 63)) - 1ull))] = vals[gi];
+            }
             __syncthreads();
         }
-        for (uint32_t j = lo + threadIdx.x; j < hi; j += 256) {
-            const uint64_t v = tval[j];
-            svals[lo + atomicAdd(&cnt[(uint32_t)(v >> 32)], 1u)] = v;
-        }
-        __syncthreads();
     }
 }
 

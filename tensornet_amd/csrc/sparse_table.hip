@@ -97,7 +97,7 @@ struct SparseTable {
     hipEvent_t verify_ev = nullptr; // a push's comparison of the signs has been published
     DevBuf comb_buf;                // slot descriptors of a combine op
     DevBuf pooled_ws;               // scratch of a push of pooled gradients (ordered lookups, reduced rows)
-    size_t place_lds = 0, huge_lds = 0;  // dynamic LDS of k_place_lookups / k_order_huge on this device (0: not asked yet)
+    size_t place_lds = 0;  // dynamic LDS of k_place_lookups on this device (0: not asked yet)
     // The path of few launches for small batches: the words in pinned memory its kernels report through (hwords: one
     // per workgroup of a small pull's first launch, or of a table-level pull's; hseq [0] a large pull's status is on the host, [1] a push's signs are
     // compared) with the numbers the host expects there next, the dynamic LDS its kernels may have.
@@ -2295,28 +2295,21 @@ int push_op_impl(uint32_t table_handle, int N, const int64_t* const* values, con
     auto prepare_src = [&]() -> int {
         src = op_source(p, grad_dim, pd == p.push_descs);
         if (!pooled) return TN_OK;
-        if (!t->place_lds) {
-            t->place_lds = big_lds_bytes_for(reinterpret_cast<const void*>(k_place_lookups));
-            t->huge_lds = big_lds_bytes_for(reinterpret_cast<const void*>(k_order_huge));
-        }
-        const bool huge_in_lds = (size_t)batch * sizeof(uint32_t) <= t->huge_lds;
-        const int huge_grid = huge_in_lds ? GRID_CAP : 64;
+        if (!t->place_lds) t->place_lds = big_lds_bytes_for(reinterpret_cast<const void*>(k_place_lookups));
         Carver c{nullptr};
-        uint32_t *long_count, *gcur, *seg_off, *tkey, *mid_list, *huge_list, *gcnt;
-        uint64_t *vals, *svals, *tval;
+        uint32_t *long_count, *gcur, *seg_off, *tpos, *mid_list, *huge_list;
+        uint64_t *vals, *svals;
         float* flat;
         auto carve = [&](Carver& cv) {
             long_count = cv.take<uint32_t>(4);  // [1], [2]: entries of the lists of k_place_lookups (mid, huge)
             mid_list = cv.take<uint32_t>(L / ORDER_MID + 1);
             huge_list = cv.take<uint32_t>(L / ORDER_HUGE + 1);
             gcur = cv.take<uint32_t>(L);
-            tkey = cv.take<uint32_t>(L);
+            tpos = cv.take<uint32_t>(L);
             vals = cv.take<uint64_t>(L);
-            tval = cv.take<uint64_t>(L);
             svals = cv.take<uint64_t>(L);
             seg_off = cv.take<uint32_t>(L + 1);
             flat = cv.take<float>(L * (size_t)grad_dim);
-            gcnt = cv.take<uint32_t>(huge_in_lds ? 0 : (size_t)huge_grid * (size_t)batch);
         };
         carve(c);
         TN_TRY(t->pooled_ws.ensure(align_up(c.off, 256)));
@@ -2328,14 +2321,16 @@ int push_op_impl(uint32_t table_handle, int N, const int64_t* const* values, con
         // distinct index of its share of the slot (a slot has at most as many as lookups).
         size_t max_len = 0;
         for (int s = 0; s < N; s++) max_len = std::max<size_t>(max_len, (size_t)value_lens[s]);
-        // (one workgroup per slot: with several, each streaming the slot for its share of the distinct indices,
-        // the kernel took longer -- 0.20 against 0.17 ms with five, 0.16 with two -- as did a split by position,
-        // which needs a matrix of counts)
-        const uint32_t parts = 1;
+        // Workgroups per slot: about 200 in all, where the chip is filled (each streams its slot's lookups, so more of them
+        // read more: 100 slots of 49 k lookups 135 / 125 / 163 / 240 us with 1 / 2 / 4 / 8 per slot, 20 of 120 k 602 / 155 /
+        // 150 / 144 / 211 with 1 .. 16, 3 of 120 k 461 / 115 / 103 / 96 / 89); a share whose counters may not fit into LDS
+        // is the slow one.
+        const size_t counters = t->place_lds / sizeof(uint32_t);
+        const uint32_t parts = (uint32_t)std::min<size_t>(16, std::max<size_t>({1, 200 / (size_t)N, (max_len + counters - 1) / counters}));
         const size_t place_bytes = std::min(t->place_lds, align_up((max_len / parts + 2) * sizeof(uint32_t), 256));
         const uint32_t place_cap = (uint32_t)(place_bytes / sizeof(uint32_t));
         TN_LAUNCH_LDS(k_place_lookups, dim3(N * parts), dim3(PLACE_THREADS), place_bytes, st, p.lbase, p.ubase, N, (uint32_t)L,
-                      p.u_of_gi, vals, tkey, tval, seg_off, gcur, place_cap, mid_list, huge_list, long_count, ds, parts);
+                      p.u_of_gi, tpos, seg_off, gcur, place_cap, mid_list, huge_list, long_count, ds, parts);
         // The three kernels that order the segments work on segments of their own (short, middle, huge), the two
         // that sum them likewise (those below LONG_SEGMENT lookups, those from it on): a large batch runs them side
         // by side on the table's streams.
@@ -2346,13 +2341,13 @@ int push_op_impl(uint32_t table_handle, int N, const int64_t* const* values, con
             TN_HIP(hipStreamWaitEvent(t->side, t->fork_ev, 0));
             TN_HIP(hipStreamWaitEvent(t->side2, t->fork_ev, 0));
         }
-        TN_LAUNCH(k_rank_short, dim3(launch_grid(L, 256, GRID_CAP * 4)), dim3(256), st, (uint32_t)L, tkey, tval, seg_off,
-                  svals, ds);
+        TN_LAUNCH(k_rank_short, dim3(launch_grid(L, 256, GRID_CAP * 4)), dim3(256), st, (uint32_t)L, p.u_of_gi, vals, tpos,
+                  seg_off, svals, ds);
         TN_LAUNCH(k_rank_mid, dim3(launch_grid((int64_t)L / ORDER_MID + 1, 1, GRID_CAP * 2)), dim3(256), s_mid, mid_list,
-                  long_count, seg_off, tval, svals, ds);
-        TN_LAUNCH_LDS(k_order_huge, dim3(launch_grid((int64_t)L / ORDER_HUGE + 1, 1, huge_grid)), dim3(256),
-                      huge_in_lds ? (size_t)batch * sizeof(uint32_t) : 0, s_huge, huge_list, long_count, seg_off, tval, svals,
-                      (uint32_t)batch, huge_in_lds ? 1 : 0, gcnt, ds);
+                  long_count, seg_off, vals, tpos, svals, ds);
+        const size_t huge_lds = order_huge_lds(max_len);
+        TN_LAUNCH_LDS(k_order_huge, dim3(launch_grid((int64_t)L / ORDER_HUGE + 1, 1, GRID_CAP)), dim3(256), huge_lds, s_huge,
+                      huge_list, long_count, p.lbase, p.ubase, N, seg_off, vals, tpos, svals, (uint32_t)(huge_lds / 12), ds);
         // signs with LONG_SEGMENT lookups or more get a workgroup each instead of one thread group
         static_assert(LONG_SEGMENT == ORDER_MID, "the lists of k_place_lookups are the frequent signs of k_reduce_long");
         const int chunks = (grad_dim + 3) / 4;
