@@ -23,7 +23,7 @@
 //                  only when there are too many tiles for that)
 //   k_lds_mapped   mapped ids and the per-lookup distinct index
 //
-// With at most 128 slots the groups of equal signs over all slots come out of
+// With at most GRP_SLOTS slots the groups of equal signs over all slots come out of
 // LDS too: k_lds_dedup hands every distinct (slot, sign) record -- sign, first
 // position, occurrences, slot -- to a second level of buckets chosen by the sign's
 // hash alone (fixed room per bucket, one global atomic per touched bucket), and
@@ -63,8 +63,14 @@ static_assert(GRP_CAP % GRP_THREADS == 0 && GRP_CAP % 256 == 0 && GRP_CAP < GRP_
 constexpr int EMIT_THREADS = 512;
 constexpr int EMIT_RECS = GRP_CAP / EMIT_THREADS;  // records per thread of k_group_emit
 constexpr int GRP_ITEMS = (GRP_TABLE + 1 + GRP_THREADS - 1) / GRP_THREADS;
-constexpr int GRP_SLOTS = 128;          // slot masks are 128 bits wide
-static_assert((uint64_t)LDS_MAX_SUB * L1_ROOM <= 0x7FFFFFull && GRP_SLOTS <= 256,
+// A sign has a bit per slot in a mask of two words, or of four where there are more slots than that.  The masks of four
+// words take 85 KB of a CU's LDS (one workgroup instead of three), so the narrow ones stay; with as many slots a frequent
+// sign brings up to 255 records into its bucket, so the buckets are filled to half as much (Zipf 1.02 .. 1.3 over 10^5 ..
+// 10^8 ids in 250 slots: 900 .. 1300 records in the fullest one, 1460 .. 1950 of 1536 when filled like the others).
+constexpr int GRP_NARROW = 128;
+constexpr int GRP_SLOTS = 255;          // a record has eight bits for its slot, its place and the records of its group
+constexpr int GRP_TARGET_WIDE = 512;
+static_assert((uint64_t)LDS_MAX_SUB * L1_ROOM <= 0x7FFFFFull && GRP_SLOTS <= 255,
               "a record's word holds the occurrences of a sign in its slot and the slot");
 
 // Raises DEV_ERR_REMAP_OVERFLOW.  A batch that overflows does so in a million places at once: atomics on the one
@@ -622,21 +628,24 @@ __global__ __launch_bounds__(256) void k_lds_mapped(const SlotDesc* __restrict__
 //   y: bits 0-15 records of the bucket's earlier several-record groups, 16-23 place, 24-31 slot
 // and per bucket the number of groups with one record, with several, the
 // records of the latter, and the big groups.  At most GRP_SLOTS slots.
+// 2039 examples of 211 slots (860 k lookups): the grouping in memory that more than 128 slots took before (insert, compact,
+// fill, rank and the probe of the groups behind it) 162 us, 67 (k_group_count 21, k_probe_recs and k_init_new_recs 19,
+// k_group_emit 17, 10 more in k_lds_dedup).
 // LDS of a workgroup that groups second-level buckets (group_count_bucket).
+template <int WORDS>
 struct GroupCountLds {
     unsigned long long keys[GRP_TABLE + 1];  // entry GRP_TABLE: the sign EMPTY_KEY itself
-    unsigned long long mlo[GRP_TABLE + 1], mhi[GRP_TABLE + 1];
+    unsigned long long mask[WORDS][GRP_TABLE + 1];
     uint16_t rech[GRP_CAP];
     unsigned long long sh[GRP_THREADS / 64];
 };
 
 // One second-level bucket, by a workgroup of GRP_THREADS threads (the caller puts a barrier between two buckets).
-__device__ __forceinline__ void group_count_bucket(uint32_t c, GroupCountLds& lds, const uint32_t* __restrict__ cursor2,
+template <int WORDS>
+__device__ __forceinline__ void group_count_bucket(uint32_t c, GroupCountLds<WORDS>& lds, const uint32_t* __restrict__ cursor2,
                                                    const GroupRec* __restrict__ recs, uint32_t big_k,
                                                    uint2* __restrict__ aux, uint4* __restrict__ bcounts) {
     unsigned long long* const keys = lds.keys;
-    unsigned long long* const mlo = lds.mlo;
-    unsigned long long* const mhi = lds.mhi;
     uint16_t* const rech = lds.rech;
     unsigned long long* const sh = lds.sh;
     // Once every record knows its entry (rech) the keys are dead: the entries' group numbers and offsets
@@ -665,8 +674,8 @@ __device__ __forceinline__ void group_count_bucket(uint32_t c, GroupCountLds& ld
     }
     for (int i = threadIdx.x; i <= GRP_TABLE; i += GRP_THREADS) {
         keys[i] = EMPTY_KEY;
-        mlo[i] = 0;
-        mhi[i] = 0;
+#pragma unroll
+        for (int w = 0; w < WORDS; w++) lds.mask[w][i] = 0;
     }
     __syncthreads();
 #pragma unroll
@@ -683,7 +692,7 @@ __device__ __forceinline__ void group_count_bucket(uint32_t c, GroupCountLds& ld
                 h = (h + 1) & (GRP_TABLE - 1);
             }
         }
-        atomicOr(sl[j] < 64 ? &mlo[h] : &mhi[h], 1ull << (sl[j] & 63));
+        atomicOr(&lds.mask[sl[j] >> 6][h], 1ull << (sl[j] & 63));
         rech[j * GRP_THREADS + threadIdx.x] = (uint16_t)h;
     }
     __syncthreads();
@@ -691,7 +700,11 @@ __device__ __forceinline__ void group_count_bucket(uint32_t c, GroupCountLds& ld
     unsigned long long v = 0;  // 16-bit fields: groups of one record, of several, records of those, big groups
     for (int j = 0; j < GRP_ITEMS; j++) {
         const uint32_t e = j * GRP_THREADS + threadIdx.x;
-        const uint32_t k = (e <= GRP_TABLE) ? (uint32_t)(__popcll(mlo[e]) + __popcll(mhi[e])) : 0;
+        uint32_t k = 0;
+        if (e <= GRP_TABLE) {
+#pragma unroll
+            for (int w = 0; w < WORDS; w++) k += (uint32_t)__popcll(lds.mask[w][e]);
+        }
         ks[j] = k;
         if (k == 1) v += 1ull;
         if (k > 1) v += (1ull << 16) + ((unsigned long long)k << 32) + (is_big(k, big_k) ? 1ull << 48 : 0ull);
@@ -721,20 +734,22 @@ __device__ __forceinline__ void group_count_bucket(uint32_t c, GroupCountLds& ld
         if (s1 == 0xFFFFFFFFu) continue;
         const uint32_t i = j * GRP_THREADS + threadIdx.x;
         const uint32_t h = rech[i];
-        uint32_t place;
-        if (s1 < 64)
-            place = (uint32_t)__popcll(mlo[h] & ((1ull << s1) - 1ull));
-        else
-            place = (uint32_t)__popcll(mlo[h]) + (uint32_t)__popcll(mhi[h] & ((1ull << (s1 - 64)) - 1ull));
+        uint32_t place = 0;
+#pragma unroll
+        for (uint32_t w = 0; w < WORDS; w++) {
+            const unsigned long long lower = w < (s1 >> 6) ? ~0ull : w > (s1 >> 6) ? 0ull : (1ull << (s1 & 63)) - 1ull;
+            place += (uint32_t)__popcll(lds.mask[w][h] & lower);
+        }
         const uint2 ei = einfo[h];
         aux[first + i] = make_uint2(ei.x, ei.y | (place << 16) | (s1 << 24));
     }
 }
 
+template <int WORDS>
 __global__ __launch_bounds__(GRP_THREADS) void k_group_count(uint32_t nb2, const uint32_t* __restrict__ cursor2,
                                                      const GroupRec* __restrict__ recs, uint32_t big_k,
                                                      uint2* __restrict__ aux, uint4* __restrict__ bcounts) {
-    __shared__ GroupCountLds lds;
+    __shared__ GroupCountLds<WORDS> lds;
     for (uint32_t c = blockIdx.x; c < nb2; c += gridDim.x) {
         group_count_bucket(c, lds, cursor2, recs, big_k, aux, bcounts);
         __syncthreads();

@@ -631,9 +631,9 @@ size_t carve_plan(char* base, Plan& p, int N, size_t L, bool exact = false) {
 
 // Second-level buckets of a batch of L lookups: GRP_TARGET records each on average if the batch has the
 // expected share of distinct records plus a quarter (GRP_CAP is the room of a bucket).
-uint32_t second_level_buckets(size_t L, double distinct_est) {
+uint32_t second_level_buckets(size_t L, double distinct_est, size_t target) {
     const double expected = std::min(1.0, distinct_est * 1.25) * (double)L;
-    return (uint32_t)std::max<size_t>(1, ((size_t)expected + GRP_TARGET - 1) / GRP_TARGET);
+    return (uint32_t)std::max<size_t>(1, ((size_t)expected + target - 1) / target);
 }
 
 // dt_entries: entries of the global dedup table, or (use_lds) the number of buckets.
@@ -651,10 +651,11 @@ size_t carve_scratch(char* base, Scratch& w, size_t L, size_t dt_entries, bool u
     Carver c{base};
     if (use_lds) {
         w.nbuckets = (uint32_t)dt_entries;
-        w.nb2 = second_level_buckets(L, distinct_est);
+        const size_t target = N <= GRP_NARROW ? GRP_TARGET : GRP_TARGET_WIDE;
+        w.nb2 = second_level_buckets(L, distinct_est, target);
         // room for the buckets of a batch of distinct signs only: a call that overflows is repeated with that
         // many, and must not pay for a larger buffer then (freeing and allocating waits for the whole device)
-        const size_t nb2_room = std::max<size_t>(w.nb2, (L + GRP_TARGET - 1) / GRP_TARGET);
+        const size_t nb2_room = std::max<size_t>(w.nb2, (L + target - 1) / target);
         const size_t nb1_room = std::max<size_t>(dt_entries, L / L1_FILL + (size_t)N + 1);
         w.bcursor = c.take<uint32_t>(nb1_room + 1 + nb2_room);  // (the part in use is zeroed together)
         w.cursor2 = w.bcursor + dt_entries + 1;
@@ -857,8 +858,12 @@ int launch_build_plan(SparseTable* t, const Plan& p, const Scratch& w, int N, ui
                 TN_HIP(hipEventRecord(t->fork_ev, st));
                 TN_HIP(hipStreamWaitEvent(t->side, t->fork_ev, 0));
             }
-            TN_LAUNCH(k_group_count, dim3(bblocks), dim3(GRP_THREADS), sd, w.nb2, w.cursor2, w.recs,
-                      big_threshold(s), w.aux, w.bcounts);
+            if (N <= GRP_NARROW)
+                TN_LAUNCH((k_group_count<2>), dim3(bblocks), dim3(GRP_THREADS), sd, w.nb2, w.cursor2, w.recs,
+                          big_threshold(s), w.aux, w.bcounts);
+            else
+                TN_LAUNCH((k_group_count<4>), dim3(bblocks), dim3(GRP_THREADS), sd, w.nb2, w.cursor2, w.recs,
+                          big_threshold(s), w.aux, w.bcounts);
             if (!own_offsets) TN_LAUNCH(k_group_offsets, dim3(1), dim3(1024), sd, w.bcounts, w.bbase, w.nb2, ds);
             if (!t->one_stream) {
                 TN_HIP(hipEventRecord(t->join_ev, t->side));
