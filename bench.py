@@ -112,6 +112,7 @@ def kernel_algorithmic_bytes(name, opt, dim, shape):
         "k_apply_big": apply_bytes(shape["Rb"], shape["Gb"]),
         "k_apply_big_adagrad": apply_bytes(shape["Rb"], shape["Gb"]),
         "k_apply_scalar": apply_bytes(U, G),
+        "k_apply_all": apply_bytes(U, G),
     }
     return table.get(name.split("<")[0], 0)
 

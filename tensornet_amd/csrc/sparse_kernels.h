@@ -1554,18 +1554,16 @@ __device__ __forceinline__ void apply_one_record(const Store& s, const OptDev& o
 // Most signs occur in one slot only: one record, no ordering problem, no
 // loop.  LPG lanes update the row of one such sign; its member entry sits at
 // the place of its group number.
+// The workgroups `at`, at + stride, ... of all that do this work.
 template <int KIND, int LPG, bool ANY>
-__global__ __launch_bounds__(256) void k_apply_single(Store s, OptDev o, PushSrc src, DevStatus* status,
-                                                      const uint32_t* __restrict__ grp_row,
-                                                      const Member* __restrict__ list) {
-    // a push launched on a plan that turned out not to be its batch's (the host redoes it), or whose inputs are unusable
-    if (status->mismatch | status->abort) return;
+__device__ __forceinline__ void apply_singles(const Store& s, const OptDev& o, const PushSrc& src, DevStatus* status,
+                                              const uint32_t* __restrict__ grp_row, const Member* __restrict__ list,
+                                              uint32_t at, uint32_t stride) {
     const uint32_t n_single = status->n_single;
     const int sub = threadIdx.x % LPG;
     const int lane0 = (int)__lane_id() - sub;
-    const uint32_t gstride = gridDim.x * (blockDim.x / LPG);
     const float c1 = 1 - o.beta1, c2 = 1 - o.beta2;
-    for (uint32_t g = blockIdx.x * (blockDim.x / LPG) + threadIdx.x / LPG; g < n_single; g += gstride) {
+    for (uint32_t g = at * (256 / LPG) + threadIdx.x / LPG; g < n_single; g += stride * (256 / LPG)) {
         const uint32_t row = grp_row[g];
         if (row > s.cap) continue;  // NO_ROW (unknown sign: flagged by the probe), or no row number at all
         const float* gp;
@@ -1576,6 +1574,15 @@ __global__ __launch_bounds__(256) void k_apply_single(Store s, OptDev o, PushSrc
         }
         apply_one_record<KIND, LPG, ANY>(s, o, row, gp, bshow, bclick, sub, lane0, c1, c2);
     }
+}
+
+template <int KIND, int LPG, bool ANY>
+__global__ __launch_bounds__(256) void k_apply_single(Store s, OptDev o, PushSrc src, DevStatus* status,
+                                                      const uint32_t* __restrict__ grp_row,
+                                                      const Member* __restrict__ list) {
+    // a push launched on a plan that turned out not to be its batch's (the host redoes it), or whose inputs are unusable
+    if (status->mismatch | status->abort) return;
+    apply_singles<KIND, LPG, ANY>(s, o, src, status, grp_row, list, blockIdx.x, gridDim.x);
 }
 
 // One group of LPG lanes owns one distinct sign: it loads the row once, applies
@@ -1681,6 +1688,28 @@ __device__ __forceinline__ void apply_group_vec(const Store& s, const OptDev& o,
     }
 }
 
+// The workgroups `at`, at + stride, ... of all that do this work.
+template <int KIND, int LPG, bool ANY>
+__device__ __forceinline__ void apply_multis(const Store& s, const OptDev& o, const PushSrc& src, DevStatus* status,
+                                             const uint32_t* __restrict__ grp_row, const uint32_t* __restrict__ grp_off,
+                                             const uint32_t* __restrict__ grp_cnt, const Member* __restrict__ list,
+                                             uint32_t big_k, uint32_t ids_cap, const float* const* __restrict__ gaddr,
+                                             uint32_t at, uint32_t stride) {
+    const uint32_t n_multi = status->n_multi;
+    const int sub = threadIdx.x % LPG;                       // my float4 inside the row
+    const int lane0 = (int)__lane_id() - sub;                // first lane of my group in the wavefront
+    const float c1 = 1 - o.beta1, c2 = 1 - o.beta2;
+    for (uint32_t gi = at * (256 / LPG) + threadIdx.x / LPG; gi < n_multi; gi += stride * (256 / LPG)) {
+        const uint32_t g = ids_cap - n_multi + gi;  // groups with several records sit at the top of the id space
+        const uint32_t row = grp_row[g];
+        if (row > s.cap) continue;  // NO_ROW (unknown sign: flagged by the probe), or no row number at all
+        const uint32_t k = grp_cnt[g];
+        if (is_big(k, big_k)) continue;
+        apply_group_vec<KIND, LPG, ANY>(s, o, src, status, row, k, list + grp_off[g],
+                                        gaddr ? gaddr + grp_off[g] : nullptr, sub, lane0, c1, c2);
+    }
+}
+
 template <int KIND, int LPG, bool ANY>
 __global__ __launch_bounds__(256) void k_apply_vec(Store s, OptDev o, PushSrc src, DevStatus* status,
                                                    const uint32_t* __restrict__ grp_row,
@@ -1690,20 +1719,8 @@ __global__ __launch_bounds__(256) void k_apply_vec(Store s, OptDev o, PushSrc sr
                                                    uint32_t ids_cap, const float* const* __restrict__ gaddr) {
     // a push launched on a plan that turned out not to be its batch's (the host redoes it), or whose inputs are unusable
     if (status->mismatch | status->abort) return;
-    const uint32_t n_multi = status->n_multi;
-    const int sub = threadIdx.x % LPG;                       // my float4 inside the row
-    const int lane0 = (int)__lane_id() - sub;                // first lane of my group in the wavefront
-    const uint32_t gstride = gridDim.x * (blockDim.x / LPG);
-    const float c1 = 1 - o.beta1, c2 = 1 - o.beta2;
-    for (uint32_t gi = blockIdx.x * (blockDim.x / LPG) + threadIdx.x / LPG; gi < n_multi; gi += gstride) {
-        const uint32_t g = ids_cap - n_multi + gi;  // groups with several records sit at the top of the id space
-        const uint32_t row = grp_row[g];
-        if (row > s.cap) continue;  // NO_ROW (unknown sign: flagged by the probe), or no row number at all
-        const uint32_t k = grp_cnt[g];
-        if (is_big(k, big_k)) continue;
-        apply_group_vec<KIND, LPG, ANY>(s, o, src, status, row, k, list + grp_off[g],
-                                        gaddr ? gaddr + grp_off[g] : nullptr, sub, lane0, c1, c2);
-    }
+    apply_multis<KIND, LPG, ANY>(s, o, src, status, grp_row, grp_off, grp_cnt, list, big_k, ids_cap, gaddr, blockIdx.x,
+                                 gridDim.x);
 }
 
 // Value of v in lane `src` (the same for the whole wavefront), by register read-out.
@@ -1999,24 +2016,29 @@ struct BigTile {
     static constexpr int CHUNK = R * ROUNDS;
     static constexpr int DP = D + 1;  // padded staging row: lanes walking down a column hit different banks
 };
+// (the signs first, first + stride, ... by the wavefront that calls it, whose own the LDS is; head: the first one's description)
 template <int D>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6, 8))) void k_apply_big_adagrad(
-    Store s, OptDev o, PushSrc src, DevStatus* status, const uint4* __restrict__ big_desc, uint32_t desc_cap,
-    const Member* __restrict__ list, const float* const* __restrict__ gaddr) {
+struct BigTileLds {
+    float gbuf[BigTile<D>::CHUNK * BigTile<D>::DP];
+    const float* gptr[BigTile<D>::CHUNK];
+    float den[BigTile<D>::CHUNK];
+};
+template <int D, typename Sync>
+__device__ __forceinline__ void apply_big_tiles(const Store& s, const OptDev& o, const PushSrc& src, DevStatus* status,
+                                                const uint4* __restrict__ big_desc, const Member* __restrict__ list,
+                                                const float* const* __restrict__ gaddr, BigTileLds<D>& lds, uint4 head,
+                                                uint32_t first, uint32_t stride, Sync sync) {
     using T = BigTile<D>;
     constexpr int R = T::R, DP = T::DP;
-    __shared__ float gbuf[T::CHUNK * DP];
-    __shared__ const float* gptr[T::CHUNK];
-    __shared__ float den[T::CHUNK];
-    const int lane = (int)threadIdx.x;
+    float* const gbuf = lds.gbuf;
+    const float** const gptr = lds.gptr;
+    float* const den = lds.den;
+    const int lane = (int)__lane_id();
     const int li = lane & (D - 1), lm = lane / D;
-    uint4 head = big_desc[blockIdx.x < desc_cap ? blockIdx.x : desc_cap - 1];  // (before the status is known)
-    // a push launched on a plan that turned out not to be its batch's (the host redoes it), or whose inputs are unusable
-    if (status->mismatch | status->abort) return;
     const uint32_t n_big = status->n_big;
     constexpr double inv_d = 1.0 / (double)D;  // exact: D is a power of two
-    for (uint32_t bi = blockIdx.x; bi < n_big; bi += gridDim.x) {
-        if (bi != blockIdx.x) head = big_desc[bi];
+    for (uint32_t bi = first; bi < n_big; bi += stride) {
+        if (bi != first) head = big_desc[bi];
         const uint32_t row = head.x, off = head.y, k = head.z;
         if (row > s.cap) continue;  // NO_ROW, or no row number at all: never address the table with it
         float* wp = s.w + (uint64_t)row * s.wstride;
@@ -2035,7 +2057,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6, 8))) void
             }
             const unsigned long long okmask = __ballot(ok);
             const unsigned long long chunk_mask = cn == 64 ? ~0ull : (1ull << cn) - 1ull;
-            __syncthreads();
+            sync();
             {
                 float v[T::ROUNDS];
 #pragma unroll
@@ -2046,7 +2068,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6, 8))) void
 #pragma unroll
                 for (int q = 0; q < T::ROUNDS; q++) gbuf[(lm + q * R) * DP + li] = v[q];
             }
-            __syncthreads();
+            sync();
             // add_g2sum / dim of record `lane`: double sum of float products in element order
             double mq = 0.0;
             if (lane < cn) {
@@ -2085,7 +2107,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6, 8))) void
                 }
             }
             if (lane < cn) den[lane] = o.eps + sqrtf(myg2);
-            __syncthreads();
+            sync();
             // the steps lr * g / den of all records and elements (independent divisions, the operands of a few
             // rounds fetched together); a record without a gradient row steps by zero, which leaves the weights
             // as they are
@@ -2094,7 +2116,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6, 8))) void
                 const float gv = gbuf[m * DP + li], dn = den[m];
                 gbuf[m * DP + li] = ((okmask >> m) & 1ull) ? o.lr * gv / dn : 0.f;
             }
-            __syncthreads();
+            sync();
             // per element the subtractions in record order
             if (lane < D) {
                 for (int m0 = 0; m0 < cn; m0 += 8) {
@@ -2107,7 +2129,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6, 8))) void
             }
             if (okmask) any = true;
             if (lane == 0 && okmask != chunk_mask) atomicOr(&status->err, DEV_ERR_GRAD_ROWS);
-            __syncthreads();
+            sync();
         }
         if (any) {
             if (lane < D) wp[lane] = w;
@@ -2125,6 +2147,76 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6, 8))) void
     }
 }
 
+template <int D>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6, 8))) void k_apply_big_adagrad(
+    Store s, OptDev o, PushSrc src, DevStatus* status, const uint4* __restrict__ big_desc, uint32_t desc_cap,
+    const Member* __restrict__ list, const float* const* __restrict__ gaddr) {
+    __shared__ BigTileLds<D> lds;
+    const uint4 head = big_desc[blockIdx.x < desc_cap ? blockIdx.x : desc_cap - 1];  // (before the status is known)
+    // a push launched on a plan that turned out not to be its batch's (the host redoes it), or whose inputs are unusable
+    if (status->mismatch | status->abort) return;
+    apply_big_tiles<D>(s, o, src, status, big_desc, list, gaddr, lds, head, blockIdx.x, gridDim.x, [] { __syncthreads(); });
+}
+
+// The updates of a push of up to ONE_STREAM_LOOKUPS lookups by one launch: the workgroups of the three kernels above side
+// by side, those with the longest chains first.  They touch disjoint rows and one alone leaves the chip half idle --
+// k_apply_big and k_apply_vec wait for chains, and a launch for its last workgroups --, but a batch this small does not pay
+// for a second stream (a fork and a join of 15 us).  TILE: the row length k_apply_big_adagrad is made for, 0: the signs with
+// many records the way of k_apply_big, with the staging a wavefront of a workgroup of four can have.
+// 2.1 M lookups of 64 slots, AdaGrad rows of 16: three launches 58 us (19 + 20 + 19), this one 42; 327 k of 40, rows of 64:
+// 77 -> 51, Ftrl rows of 1: 66 -> 38; 286 k of 47, rows of 8 + 2: 32 -> 18.
+struct ApplyAll {
+    uint32_t big_blocks, multi_blocks;  // the first workgroups of the launch, the ones behind them; the rest: one record
+    const uint32_t *grp_row, *grp_off, *grp_cnt, *big_list;
+    const uint4* big_desc;
+    uint32_t big_cap, big_k, ids_cap;
+    const Member* list;
+    const float* const* gaddr;
+    int gbuf_floats;
+    uint32_t wave_lds, wave_arrays;  // bytes of LDS of a wavefront, where in them its arrays are (TILE 0)
+};
+constexpr int ALL_GBUF = 1088;  // floats of gradient staging per wavefront at most: eight workgroups to a CU up to 64 elements
+
+template <int KIND, int LPG, bool ANY, int TILE>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6, 8))) void k_apply_all(Store s, OptDev o, PushSrc src,
+                                                                                              DevStatus* status, ApplyAll a) {
+    // a push launched on a plan that turned out not to be its batch's (the host redoes it), or whose inputs are unusable
+    if (status->mismatch | status->abort) return;
+    if (blockIdx.x < a.big_blocks) {
+        const uint32_t wave = threadIdx.x >> 6, first = blockIdx.x * 4 + wave, stride = a.big_blocks * 4;
+        if constexpr (TILE != 0) {
+            __shared__ BigTileLds<TILE> lds[4];
+            const uint4 head = a.big_desc[first < a.big_cap ? first : a.big_cap - 1];
+            apply_big_tiles<TILE>(s, o, src, status, a.big_desc, a.list, a.gaddr, lds[wave], head, first, stride,
+                                  [] { wave_sync(); });
+        } else {
+            extern __shared__ unsigned long long all_lds[];
+            char* base = reinterpret_cast<char*>(all_lds) + wave * a.wave_lds;
+            const float** gptr = reinterpret_cast<const float**>(base + a.wave_arrays);
+            apply_big_groups<KIND>(
+                s, o, a.gbuf_floats, reinterpret_cast<float*>(base), gptr, reinterpret_cast<float*>(gptr + BIG_CHUNK),
+                (int)(threadIdx.x & 63), first, stride, status->n_big,
+                [&](uint32_t bi, uint32_t& row, uint32_t& off, uint32_t& k) {
+                    const uint32_t g = a.big_list[bi];
+                    row = a.grp_row[g];
+                    off = a.grp_off[g];
+                    k = a.grp_cnt[g];
+                },
+                [&](uint32_t at, const float*& gp, int& sh, int& ck) {
+                    return record_at(src, a.list, a.gaddr, at, gp, sh, ck);
+                },
+                [&] { atomicOr(&status->err, DEV_ERR_GRAD_ROWS); }, [] { wave_sync(); });
+        }
+        return;
+    }
+    const uint32_t at = blockIdx.x - a.big_blocks;
+    if (at < a.multi_blocks)
+        apply_multis<KIND, LPG, ANY>(s, o, src, status, a.grp_row, a.grp_off, a.grp_cnt, a.list, a.big_k, a.ids_cap, a.gaddr, at,
+                                     a.multi_blocks);
+    else
+        apply_singles<KIND, LPG, ANY>(s, o, src, status, a.grp_row, a.list, at - a.multi_blocks,
+                                      gridDim.x - a.big_blocks - a.multi_blocks);
+}
 
 // Rows beyond what a wavefront half holds (more than 128 elements): one thread per distinct sign, scalar loops.
 template <int KIND>

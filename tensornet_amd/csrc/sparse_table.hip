@@ -965,7 +965,11 @@ RowShare row_share(const Store& s, bool aligned) {
     return r;
 }
 
-// The three kernels touch disjoint rows.  k_apply_single saturates the memory system (it runs
+// workgroups of k_apply_all for the signs with many records at most (a wavefront each in turn)
+constexpr int ALL_BIG_GRID = 1024;
+
+// The three kernels touch disjoint rows (a batch that keeps to one stream has them in one launch, k_apply_all).
+// k_apply_single saturates the memory system (it runs
 // at the device's rate for random row updates); k_apply_big and k_apply_vec are bound by
 // dependent chains and instruction issue, so they run one after the other beside it.  The pair is
 // the longer chain: it stays on the caller's stream and k_apply_single goes to the table's side
@@ -989,6 +993,49 @@ int launch_apply_kind(SparseTable* t, RowShare share, const Store& s, const OptD
     if (with_big && gaddr && !addr_ready)
         TN_LAUNCH(k_member_grads, dim3(launch_grid(n_upper, 256, GRID_CAP * 2)), dim3(256), st, src, ds, p.list,
                   p.gaddr, ids_cap);
+    if (with_big && t->one_stream && share.lanes != 0) {
+        ApplyAll a;
+        a.big_blocks = (uint32_t)launch_grid((n_upper / BIG_GROUP + 4) / 4, 1, ALL_BIG_GRID);
+        a.multi_blocks = (uint32_t)launch_grid(n_upper * share.lanes / 2, 256, GRID_CAP * 2);
+        const uint32_t singles = (uint32_t)launch_grid(n_upper * share.lanes, 256, GRID_CAP * 2);
+        a.grp_row = p.grp_row, a.grp_off = p.grp_off, a.grp_cnt = p.grp_cnt, a.big_list = p.big_list;
+        a.big_desc = p.big_desc;
+        a.big_cap = p.big_cap, a.big_k = big_k, a.ids_cap = ids_cap;
+        a.list = p.list;
+        a.gaddr = gaddr;
+        a.gbuf_floats = std::min(big_gbuf_floats(s.D), ALL_GBUF);
+        a.wave_arrays = (uint32_t)align_up((size_t)(a.gbuf_floats + 3 * s.D) * sizeof(float), 8);
+        a.wave_lds = a.wave_arrays + BIG_CHUNK * (8 + 4);
+        // AdaGrad rows of a power-of-two dim on a plan that describes its frequent signs have kernels of their own
+        const bool tiled = KIND == OPT_ADAGRAD && big_desc && s.D == 4 * share.lanes && s.D <= 64;
+#define TN_LAUNCH_ALL_ANY(LPG, ANY)                                                                                        \
+    do {                                                                                                                   \
+        constexpr int TILE = KIND == OPT_ADAGRAD && LPG <= 16 ? 4 * LPG : 0;                                               \
+        const dim3 grid(a.big_blocks + a.multi_blocks + singles);                                                         \
+        if (tiled)                                                                                                         \
+            TN_LAUNCH((k_apply_all<KIND, LPG, ANY, TILE>), grid, dim3(256), st, s, o, src, ds, a);                         \
+        else                                                                                                               \
+            TN_LAUNCH_LDS((k_apply_all<KIND, LPG, ANY, 0>), grid, dim3(256), 4 * a.wave_lds, st, s, o, src, ds, a);        \
+    } while (0)
+#define TN_LAUNCH_ALL(LPG)                    \
+    do {                                      \
+        if (share.any)                        \
+            TN_LAUNCH_ALL_ANY(LPG, true);     \
+        else                                  \
+            TN_LAUNCH_ALL_ANY(LPG, false);    \
+    } while (0)
+        switch (share.lanes) {
+            case 1: TN_LAUNCH_ALL(1); break;
+            case 2: TN_LAUNCH_ALL(2); break;
+            case 4: TN_LAUNCH_ALL(4); break;
+            case 8: TN_LAUNCH_ALL(8); break;
+            case 16: TN_LAUNCH_ALL(16); break;
+            default: TN_LAUNCH_ALL(32); break;
+        }
+#undef TN_LAUNCH_ALL
+#undef TN_LAUNCH_ALL_ANY
+        return TN_OK;
+    }
     if (forked) {
         TN_HIP(hipEventRecord(t->fork_ev, st));
         TN_HIP(hipStreamWaitEvent(t->side, t->fork_ev, 0));
