@@ -2,8 +2,9 @@
 behind the 64 lookups a wavefront looks at, that go on over several of them and take a whole slot; signs with few, many and
 all lookups of a slot; rows of any length.
 
-The examples have powers of two of lookups and the gradients are small multiples of 2^-8: the sums of up to 9000 of them,
-divided or not, are exact in 32 bits in any order, so the order in which long sums are added makes no difference."""
+The examples have powers of two of lookups and the gradients are small multiples of 2^-8: the sums of the lookups of a sign,
+divided or not, are exact in 32 bits in any order (at most 20 bits are in use), so the order in which long sums are added
+makes no difference."""
 import numpy as np
 import pytest
 
@@ -22,7 +23,7 @@ def by_counts(counts, n):
     return np.repeat(np.arange(n), np.resize(counts, n))[:n].astype(np.int64)
 
 
-@pytest.mark.parametrize("dim,slots,n", [(16, 5, 9000), (10, 5, 5001), (1, 3, 4097), (130, 5, 6000), (8, 130, 4160)])
+@pytest.mark.parametrize("dim,slots,n", [(16, 5, 9000), (10, 5, 5001), (1, 3, 4097), (130, 5, 6000), (8, 130, 4160), (4, 3, 150000)])
 def test_pooled_push_of_a_large_batch(tn, oracle, dim, slots, n):
     rng = np.random.default_rng(dim)
     pair = Pair(tn, oracle, "AdaGrad", dim, HP, reserve=200000)
