@@ -11,7 +11,7 @@
 // Both are deterministic: sums run in occurrence order.  The backward pass
 // gets the lookups of every distinct sign side by side, in position order, from a
 // counting sort per slot followed by an ordering of every sign's lookups by position
-// (k_place_lookups, k_rank_short, k_rank_mid, k_order_huge).
+// (k_place_lookups, k_order_segments).
 #ifndef TN_COMBINE_KERNELS_H_
 #define TN_COMBINE_KERNELS_H_
 
@@ -234,9 +234,9 @@ __global__ __launch_bounds__(256) void k_lookup_keys(const SlotDesc* __restrict_
 //                    the counts into seg_off, and puts the position of every lookup into its index's segment -- in
 //                    the order the atomics arrive; indices with ORDER_MID lookups or more are listed for the kernels
 //                    below
-//   k_rank_short     a lookup of a short segment finds its place by counting the positions of its segment below its own
-//   k_rank_mid       a sorting network in LDS, one workgroup per segment of ORDER_MID .. ORDER_HUGE - 1 lookups
-//   k_order_huge     the few longer segments: a bitmap of their positions in LDS, one workgroup each
+//   rank_short       a lookup of a short segment finds its place by counting the positions of its segment below its own
+//   rank_mid         a sorting network in LDS, one workgroup per segment of ORDER_MID .. ORDER_HUGE - 1 lookups
+//   order_huge       the few longer segments: a bitmap of their positions in LDS, one workgroup each
 // A slot with more distinct signs than the LDS array holds (lds_cap) keeps its counters in `gcur`.
 constexpr int PLACE_THREADS = 1024;
 constexpr int PLACE_ITEMS = 8;
@@ -331,12 +331,11 @@ __global__ __launch_bounds__(PLACE_THREADS) void k_place_lookups(
 // values, read by position, are then in its L2.  4.9 M lookups: 78 -> 62 us.
 constexpr uint32_t RANK_RUN = 128;
 
-__global__ __launch_bounds__(256) void k_rank_short(uint32_t L, const uint32_t* __restrict__ u_of_gi,
-                                                    const uint64_t* __restrict__ vals, const uint32_t* __restrict__ tpos,
-                                                    const uint32_t* __restrict__ seg_off, uint64_t* __restrict__ svals,
-                                                    const DevStatus* status) {
-    if (status->abort) return;
-    for (DieRuns r((L + 255) / 256, RANK_RUN); r.more(); r.next()) {
+__device__ __forceinline__ void rank_short(uint32_t L, const uint32_t* __restrict__ u_of_gi,
+                                           const uint64_t* __restrict__ vals, const uint32_t* __restrict__ tpos,
+                                           const uint32_t* __restrict__ seg_off, uint64_t* __restrict__ svals, uint32_t block,
+                                           uint32_t blocks) {
+    for (DieRuns r((L + 255) / 256, RANK_RUN, block, blocks); r.more(); r.next()) {
         const uint32_t t = r.item() * 256 + threadIdx.x;
         if (t >= L) continue;
         const uint32_t gi = tpos[t];
@@ -350,14 +349,12 @@ __global__ __launch_bounds__(256) void k_rank_short(uint32_t L, const uint32_t* 
     }
 }
 
-__global__ __launch_bounds__(256) void k_rank_mid(const uint32_t* __restrict__ mid_list, const uint32_t* counts,
-                                                  const uint32_t* __restrict__ seg_off, const uint64_t* __restrict__ vals,
-                                                  const uint32_t* __restrict__ tpos, uint64_t* __restrict__ svals,
-                                                  const DevStatus* status) {
-    __shared__ uint32_t seg[ORDER_HUGE];
-    if (status->abort) return;
-    const uint32_t n_mid = counts[1];
-    for (uint32_t k = blockIdx.x; k < n_mid; k += gridDim.x) {
+// seg: ORDER_HUGE words of LDS
+__device__ __forceinline__ void rank_mid(const uint32_t* __restrict__ mid_list, uint32_t n_mid,
+                                         const uint32_t* __restrict__ seg_off, const uint64_t* __restrict__ vals,
+                                         const uint32_t* __restrict__ tpos, uint64_t* __restrict__ svals, uint32_t* seg,
+                                         uint32_t block, uint32_t blocks) {
+    for (uint32_t k = block; k < n_mid; k += blocks) {
         const uint32_t u = mid_list[k];
         const uint32_t lo = seg_off[u], n = seg_off[u + 1] - lo;  // ORDER_MID <= n < ORDER_HUGE
         uint32_t p2 = ORDER_MID;
@@ -388,21 +385,19 @@ __global__ __launch_bounds__(256) void k_rank_mid(const uint32_t* __restrict__ m
 // A segment of many lookups is ordered by a bitmap of their positions in the slot, HUGE_WINDOW of these at a time (the
 // place of a lookup: bits set below its own).  The bitmap of a slot of 49 k lookups with its prefix sums takes 9 KB of LDS,
 // so a CU holds eight workgroups; counters per example, as this had before, took 64 KB at 16384 examples, or memory.
-// Beside k_rank_mid (72 -> 42 us), 4.9 M lookups: 57 -> 34 us.
+// Beside rank_mid (72 -> 42 us), 4.9 M lookups: 57 -> 34 us.
 constexpr uint32_t HUGE_WINDOW = 1u << 17;
-inline size_t order_huge_lds(size_t max_len) { return (std::min<size_t>(max_len, HUGE_WINDOW) + 63) / 64 * 12; }
+inline size_t order_huge_room(size_t max_len) { return (std::min<size_t>(max_len, HUGE_WINDOW) + 63) / 64; }
 
-__global__ __launch_bounds__(256) void k_order_huge(const uint32_t* __restrict__ huge_list, const uint32_t* counts,
-                                                    const uint32_t* __restrict__ lbase, const uint32_t* __restrict__ ubase,
-                                                    int N, const uint32_t* __restrict__ seg_off,
-                                                    const uint64_t* __restrict__ vals, const uint32_t* __restrict__ tpos,
-                                                    uint64_t* __restrict__ svals, uint32_t room, const DevStatus* status) {
-    extern __shared__ unsigned long long bits[];  // [room], then [room] set bits before the word
-    __shared__ uint32_t red[4];
-    if (status->abort) return;
+// bits: [room] words of LDS, then [room] numbers of set bits before the word
+__device__ __forceinline__ void order_huge(const uint32_t* __restrict__ huge_list, uint32_t n_huge,
+                                           const uint32_t* __restrict__ lbase, const uint32_t* __restrict__ ubase, int N,
+                                           const uint32_t* __restrict__ seg_off, const uint64_t* __restrict__ vals,
+                                           const uint32_t* __restrict__ tpos, uint64_t* __restrict__ svals,
+                                           unsigned long long* bits, uint32_t room, uint32_t* red, uint32_t block,
+                                           uint32_t blocks) {
     uint32_t* const before = reinterpret_cast<uint32_t*>(bits + room);
-    const uint32_t n_huge = counts[2];
-    for (uint32_t k = blockIdx.x; k < n_huge; k += gridDim.x) {
+    for (uint32_t k = block; k < n_huge; k += blocks) {
         const uint32_t u = huge_list[k];
         const uint32_t lo = seg_off[u], hi = seg_off[u + 1];
         const int sl = find_slot(ubase, N, u);
@@ -432,6 +427,34 @@ __global__ __launch_bounds__(256) void k_order_huge(const uint32_t* __restrict__
             __syncthreads();
         }
     }
+}
+
+// The three side by side in one launch, the longest segments first: each has segments of its own, and waits for chains.
+// 860 k lookups: three launches 34 us, this one 21; 4.9 M: 86, as the three took on three streams, without the events
+// between these.
+constexpr uint32_t ORDER_HUGE_GRID = 1024, ORDER_MID_GRID = 2048;  // workgroups at most, which take their segments in turn
+inline size_t order_lds(size_t room) { return std::max<size_t>(room * 12, ORDER_HUGE * sizeof(uint32_t)); }
+
+__global__ __launch_bounds__(256) void k_order_segments(uint32_t L, const uint32_t* __restrict__ lbase,
+                                                        const uint32_t* __restrict__ ubase, int N,
+                                                        const uint32_t* __restrict__ u_of_gi,
+                                                        const uint32_t* __restrict__ mid_list,
+                                                        const uint32_t* __restrict__ huge_list, const uint32_t* counts,
+                                                        const uint32_t* __restrict__ seg_off,
+                                                        const uint64_t* __restrict__ vals, const uint32_t* __restrict__ tpos,
+                                                        uint64_t* __restrict__ svals, uint32_t room, uint32_t huge_blocks,
+                                                        uint32_t mid_blocks, const DevStatus* status) {
+    extern __shared__ unsigned long long order_sh[];
+    __shared__ uint32_t red[4];
+    if (status->abort) return;
+    const uint32_t b = blockIdx.x, long_blocks = huge_blocks + mid_blocks;
+    if (b < huge_blocks)
+        order_huge(huge_list, counts[2], lbase, ubase, N, seg_off, vals, tpos, svals, order_sh, room, red, b, huge_blocks);
+    else if (b < long_blocks)
+        rank_mid(mid_list, counts[1], seg_off, vals, tpos, svals, reinterpret_cast<uint32_t*>(order_sh), b - huge_blocks,
+                 mid_blocks);
+    else
+        rank_short(L, u_of_gi, vals, tpos, seg_off, svals, b - long_blocks, gridDim.x - long_blocks);
 }
 
 // The sum of the shares of lookups from, from + step, ... below `to` of one distinct sign, in this order: every lookup
@@ -466,7 +489,7 @@ __device__ __forceinline__ float4 sum_shares(const float* __restrict__ pooled, c
 // Step 3: a group of `chunks` threads per distinct index, four elements of the row each (whatever its length and
 // alignment), sums its lookups' shares of the pooled gradient rows, in position order.  A distinct index with long_min
 // lookups or more (a frequent sign) is left out: k_place_lookups has listed those, one workgroup each sums them
-// (k_reduce_long).
+// (reduce_long).
 //
 // Bound by the rows it reads again and again: the pooled rows of a slot (1 MB at 16384 examples of 16 elements) stay in
 // the L2 of a die that works on one slot at a time, so the distinct indices go to the dies in runs of REDUCE_RUN
@@ -475,18 +498,15 @@ __device__ __forceinline__ float4 sum_shares(const float* __restrict__ pooled, c
 constexpr uint32_t REDUCE_RUN = 256;
 
 template <bool ANY>
-__global__ __launch_bounds__(256) void k_reduce_pooled(const SlotDesc* __restrict__ descs,
-                                                       const uint32_t* __restrict__ ubase, int N, int dim,
-                                                       int combiner, const DevStatus* status,
-                                                       const uint32_t* __restrict__ seg_off,
-                                                       const uint64_t* __restrict__ svals, float* __restrict__ flat,
-                                                       uint32_t long_min) {
-    if (status->abort) return;
-    __shared__ uint32_t ub[MAX_SLOTS + 1];
+__device__ __forceinline__ void reduce_short(const SlotDesc* __restrict__ descs, const uint32_t* __restrict__ ubase, int N,
+                                             int dim, int combiner, const DevStatus* status,
+                                             const uint32_t* __restrict__ seg_off, const uint64_t* __restrict__ svals,
+                                             float* __restrict__ flat, uint32_t long_min, uint32_t* ub, uint32_t block,
+                                             uint32_t blocks) {
     load_lbase(ub, ubase, N);
     const uint32_t chunks = (uint32_t)(dim + 3) / 4;
     const uint64_t total = (uint64_t)status->n_unique * chunks;
-    for (DieRuns r((uint32_t)((total + 255) / 256), REDUCE_RUN); r.more(); r.next()) {
+    for (DieRuns r((uint32_t)((total + 255) / 256), REDUCE_RUN, block, blocks); r.more(); r.next()) {
         const uint64_t t = (uint64_t)r.item() * 256 + threadIdx.x;
         if (t >= total) continue;
         const uint32_t u = (uint32_t)(t / chunks);
@@ -502,21 +522,17 @@ __global__ __launch_bounds__(256) void k_reduce_pooled(const SlotDesc* __restric
 // (256 / chunks)-th lookup in position order, then the partial sums are added in group order.
 // The order of the additions is fixed, so the result does not vary from run to run.
 template <bool ANY>
-__global__ __launch_bounds__(256) void k_reduce_long(const SlotDesc* __restrict__ descs,
-                                                     const uint32_t* __restrict__ ubase, int N, int dim, int combiner,
-                                                     const uint32_t* __restrict__ seg_off,
-                                                     const uint64_t* __restrict__ svals, float* __restrict__ flat,
-                                                     const uint32_t* __restrict__ mid_list,
-                                                     const uint32_t* __restrict__ huge_list,
-                                                     const uint32_t* counts, const DevStatus* status) {
-    if (status->abort) return;
-    __shared__ float4 part[256];
+__device__ __forceinline__ void reduce_long(const SlotDesc* __restrict__ descs, const uint32_t* __restrict__ ubase, int N,
+                                            int dim, int combiner, const uint32_t* __restrict__ seg_off,
+                                            const uint64_t* __restrict__ svals, float* __restrict__ flat,
+                                            const uint32_t* __restrict__ mid_list, const uint32_t* __restrict__ huge_list,
+                                            const uint32_t* counts, float4* part, uint32_t block, uint32_t blocks) {
     const int chunks = (dim + 3) / 4;
     const int groups = 256 / chunks;
     const int q = threadIdx.x / chunks, c = threadIdx.x - q * chunks;
     // the frequent ones: the two lists k_place_lookups left (ORDER_MID lookups or more)
     const uint32_t n_mid = counts[1], n_long = n_mid + counts[2];
-    for (uint32_t k = blockIdx.x; k < n_long; k += gridDim.x) {
+    for (uint32_t k = n_long - 1 - block; k < n_long; k -= blocks) {  // (the longest, which are listed last, first; ends by wrapping)
         const uint32_t u = k < n_mid ? mid_list[k] : huge_list[k - n_mid];
         const uint32_t lo = seg_off[u], hi = seg_off[u + 1];
         const float* pooled = descs[find_slot(ubase, N, u)].grads;
@@ -535,6 +551,29 @@ __global__ __launch_bounds__(256) void k_reduce_long(const SlotDesc* __restrict_
         }
         __syncthreads();
     }
+}
+
+// Both side by side in one launch, the frequent signs first.  860 k lookups of 16 elements: 53 us in two launches, 46 in
+// this one; 4.9 M: 140, as on two streams.
+template <bool ANY>
+__global__ __launch_bounds__(256) void k_reduce_pooled(const SlotDesc* __restrict__ descs,
+                                                       const uint32_t* __restrict__ ubase, int N, int dim, int combiner,
+                                                       const DevStatus* status, const uint32_t* __restrict__ seg_off,
+                                                       const uint64_t* __restrict__ svals, float* __restrict__ flat,
+                                                       uint32_t long_min, const uint32_t* __restrict__ mid_list,
+                                                       const uint32_t* __restrict__ huge_list, const uint32_t* counts,
+                                                       uint32_t long_blocks) {
+    __shared__ union {
+        uint32_t ub[MAX_SLOTS + 1];
+        float4 part[256];
+    } sh;
+    if (status->abort) return;
+    if (blockIdx.x < long_blocks)
+        reduce_long<ANY>(descs, ubase, N, dim, combiner, seg_off, svals, flat, mid_list, huge_list, counts, sh.part, blockIdx.x,
+                         long_blocks);
+    else
+        reduce_short<ANY>(descs, ubase, N, dim, combiner, status, seg_off, svals, flat, long_min, sh.ub,
+                          blockIdx.x - long_blocks, gridDim.x - long_blocks);
 }
 
 }  // namespace tn

@@ -2383,50 +2383,27 @@ int push_op_impl(uint32_t table_handle, int N, const int64_t* const* values, con
         const uint32_t place_cap = (uint32_t)(place_bytes / sizeof(uint32_t));
         TN_LAUNCH_LDS(k_place_lookups, dim3(N * parts), dim3(PLACE_THREADS), place_bytes, st, p.lbase, p.ubase, N, (uint32_t)L,
                       p.u_of_gi, tpos, seg_off, gcur, place_cap, mid_list, huge_list, long_count, ds, parts);
-        // The three kernels that order the segments work on segments of their own (short, middle, huge), the two
-        // that sum them likewise (those below LONG_SEGMENT lookups, those from it on): a large batch runs them side
-        // by side on the table's streams.
-        const bool fork = !t->one_stream;
-        hipStream_t s_mid = fork ? t->side : st, s_huge = fork ? t->side2 : st;
-        if (fork) {
-            TN_HIP(hipEventRecord(t->fork_ev, st));
-            TN_HIP(hipStreamWaitEvent(t->side, t->fork_ev, 0));
-            TN_HIP(hipStreamWaitEvent(t->side2, t->fork_ev, 0));
-        }
-        TN_LAUNCH(k_rank_short, dim3(launch_grid(L, 256, GRID_CAP * 4)), dim3(256), st, (uint32_t)L, p.u_of_gi, vals, tpos,
-                  seg_off, svals, ds);
-        TN_LAUNCH(k_rank_mid, dim3(launch_grid((int64_t)L / ORDER_MID + 1, 1, GRID_CAP * 2)), dim3(256), s_mid, mid_list,
-                  long_count, seg_off, vals, tpos, svals, ds);
-        const size_t huge_lds = order_huge_lds(max_len);
-        TN_LAUNCH_LDS(k_order_huge, dim3(launch_grid((int64_t)L / ORDER_HUGE + 1, 1, GRID_CAP)), dim3(256), huge_lds, s_huge,
-                      huge_list, long_count, p.lbase, p.ubase, N, seg_off, vals, tpos, svals, (uint32_t)(huge_lds / 12), ds);
+        const uint32_t room = (uint32_t)order_huge_room(max_len);
+        const uint32_t huge_blocks = (uint32_t)launch_grid((int64_t)L / ORDER_HUGE + 1, 1, ORDER_HUGE_GRID);
+        const uint32_t mid_blocks = (uint32_t)launch_grid((int64_t)L / ORDER_MID + 1, 1, ORDER_MID_GRID);
+        TN_LAUNCH_LDS(k_order_segments, dim3(huge_blocks + mid_blocks + launch_grid(L, 256, GRID_CAP * 4)), dim3(256),
+                      order_lds(room), st, (uint32_t)L, p.lbase, p.ubase, N, p.u_of_gi, mid_list, huge_list, long_count, seg_off,
+                      vals, tpos, svals, room, huge_blocks, mid_blocks, ds);
         // signs with LONG_SEGMENT lookups or more get a workgroup each instead of one thread group
-        static_assert(LONG_SEGMENT == ORDER_MID, "the lists of k_place_lookups are the frequent signs of k_reduce_long");
+        static_assert(LONG_SEGMENT == ORDER_MID, "the lists of k_place_lookups are the frequent signs of reduce_long");
         const int chunks = (grad_dim + 3) / 4;
-        const uint32_t long_min = chunks <= 256 ? LONG_SEGMENT : 0xFFFFFFFFu;
-        const int long_blocks = launch_grid((int64_t)L / LONG_SEGMENT + 1, 1, GRID_CAP);
-        if (fork) {
-            // the frequent signs are summed on the side stream, behind the two kernels that ordered their segments
-            TN_HIP(hipEventRecord(t->join2_ev, t->side2));
-            TN_HIP(hipStreamWaitEvent(t->side, t->join2_ev, 0));
-        }
+        const bool with_long = chunks <= 256;
+        const uint32_t long_blocks = with_long ? (uint32_t)launch_grid((int64_t)L / LONG_SEGMENT + 1, 1, GRID_CAP) : 0;
         // (a macro: the profiler names a kernel by the text of its launch)
-#define TN_REDUCE(ANY)                                                                                               \
-    TN_LAUNCH((k_reduce_pooled<ANY>), dim3(launch_grid((int64_t)L * chunks, 256, GRID_CAP * 4)), dim3(256), st, pd,  \
-              p.ubase, N, grad_dim, combiner, ds, seg_off, svals, flat, long_min);                                   \
-    if (long_min != 0xFFFFFFFFu)                                                                                     \
-        TN_LAUNCH((k_reduce_long<ANY>), dim3(long_blocks), dim3(256), s_mid, pd, p.ubase, N, grad_dim, combiner,     \
-                  seg_off, svals, flat, mid_list, huge_list, long_count, ds)
-        if (vec) {
+#define TN_REDUCE(ANY)                                                                                                 \
+    TN_LAUNCH((k_reduce_pooled<ANY>), dim3(long_blocks + launch_grid((int64_t)L * chunks, 256, GRID_CAP * 4)), dim3(256), \
+              st, pd, p.ubase, N, grad_dim, combiner, ds, seg_off, svals, flat, with_long ? LONG_SEGMENT : 0xFFFFFFFFu,  \
+              mid_list, huge_list, long_count, long_blocks)
+        if (vec)
             TN_REDUCE(false);
-        } else {
+        else
             TN_REDUCE(true);
-        }
 #undef TN_REDUCE
-        if (fork) {
-            TN_HIP(hipEventRecord(t->join_ev, t->side));
-            TN_HIP(hipStreamWaitEvent(st, t->join_ev, 0));
-        }
         src.flat = flat;
         return TN_OK;
     };

@@ -113,10 +113,11 @@ struct DieShare {
 // `for (DieRuns r(n, run); r.more(); r.next()) ... r.item()` covers every item once, whatever the grid.
 struct DieRuns {
     uint32_t n, run, dies, die, k, step;
-    __device__ __forceinline__ DieRuns(uint32_t n_, uint32_t run_) : n(n_), run(run_) {
-        dies = min(XCDS, (uint32_t)gridDim.x), die = blockIdx.x % dies;
-        k = blockIdx.x / dies;
-        step = (gridDim.x - die + dies - 1) / dies;
+    // (block, blocks: the workgroup's number among those of the launch that do this work)
+    __device__ __forceinline__ DieRuns(uint32_t n_, uint32_t run_, uint32_t block, uint32_t blocks) : n(n_), run(run_) {
+        dies = min(XCDS, blocks), die = block % dies;
+        k = block / dies;
+        step = (blocks - die + dies - 1) / dies;
     }
     __device__ __forceinline__ uint32_t item() const { return (k / run * dies + die) * run + k % run; }
     __device__ __forceinline__ bool more() const { return item() < n; }  // (items ascend with k)
