@@ -970,10 +970,12 @@ __global__ __launch_bounds__(256) void k_small_apply(SmallShape b, SmallPlan p, 
         }
         if (gr.x > s.cap) continue;
         const float* gp = src.gradient(mem);
-        if (!gp) continue;
-        int ck = 0;
-        if (KIND == OPT_ADAGRAD) ck = src.click(mem);
-        apply_one_record<KIND, LPG, ANY>(s, o, gr.x, gp, (int)mem.z, ck, sub, lane0, c1, c2);
+        if (gp) {
+            int ck = 0;
+            if (KIND == OPT_ADAGRAD) ck = src.click(mem);
+            apply_one_record<KIND, LPG, ANY>(s, o, gr.x, gp, (int)mem.z, ck, sub, lane0, c1, c2);
+        }
+        // (a record without a gradient row, too: the caller may push the batch again on this plan)
         if (KIND == OPT_ADAGRAD && sub == 0) src.click_at[mem.x] = 0;
     }
 }

@@ -129,6 +129,36 @@ def test_a_gradient_matrix_with_too_few_rows_is_reported(tn, oracle):
     pair.assert_rows_match(all_signs(values))
 
 
+@pytest.mark.parametrize("slots,shared", [(2, False), (3, True), (13, True)])  # a record, three, a wavefront's thirteen
+@pytest.mark.parametrize("small", [True, False])
+def test_a_refused_push_leaves_no_clicks_for_the_next_one(tn, oracle, slots, shared, small):
+    """The last distinct sign of the last slot has no gradient row: the push is refused.  The caller pushes the same
+    batch again, complete: the clicks that sign ends up with are those of the push that had its gradient."""
+    D, per = 8, 41
+    pool = synth.splitmix64(np.arange(1, slots * per + 1, dtype=np.uint64)).view(np.int64)
+    pair = Pair(tn, oracle, "AdaGrad", D, ADAGRAD_HP, use_cvm=True)
+    pair.populate(pool.view(np.uint64))
+    tn.core.set_sparse_table_small_batch_path(pair.h, small)
+    values = [pool[s * per:(s + 1) * per].copy() for s in range(slots)]
+    if shared:
+        for v in values:
+            v[-1] = pool[-1]
+    counts = check_pull(pair, values)
+    assert counts.tolist() == [per] * slots
+    grads = synth.make_grads(counts, pair.wf, 0.01, seed=slots)
+    labels = [np.ones(per, np.int64)] * slots
+    short = grads[:-1] + [grads[-1][:per - 1]]
+    with pytest.raises(tn.TensorNetError) as e:  # (the path of few launches says so at once, the other when it is waited for)
+        tn.ops.sparse_table_push([dev(v) for v in values], [dev(g) for g in short], [dev(l) for l in labels], pair.h)
+        tn.ops.sparse_table_sync(pair.h)
+    assert e.value.code == 1
+    tn.ops.sparse_table_sync(pair.h)
+    rc, _ = pair.o.push_op(values[:-1] + [values[-1][:per - 1]], short, labels[:-1] + [labels[-1][:per - 1]])
+    assert rc == 0
+    pair.push_op(values, grads, labels)
+    pair.assert_rows_match(all_signs(values))
+
+
 def test_small_and_large_batches_alternate_on_one_table(tn, oracle):
     """The two paths share the table's plan and scratch buffers: small, large, small, with a push of each, and
     a push of the small batch after the large pull (another batch than the last pull's)."""
