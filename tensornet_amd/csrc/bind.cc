@@ -52,6 +52,12 @@ public:
     ~Items() { Py_XDECREF(seq_); }
     Py_ssize_t size() const { return PySequence_Fast_GET_SIZE(seq_); }
     PyObject* operator[](Py_ssize_t i) const { return PySequence_Fast_ITEMS(seq_)[i]; }
+    // The items as a tuple (a new reference).
+    PyObject* tuple() const {
+        PyObject* t = PySequence_Tuple(seq_);
+        if (!t) throw PyFailed{};
+        return t;
+    }
 
 private:
     PyObject* seq_;
@@ -114,9 +120,9 @@ private:
 
 // One marshalled call of the library.
 struct Call {
-    virtual ~Call() = default;
+    virtual ~Call() { Py_XDECREF(outputs); }
     virtual int run(void* stream) = 0;
-    PyObject* outputs = nullptr;  // what the operator returns (a new reference held by whoever owns the call); nullptr: None
+    PyObject* outputs = nullptr;  // what a bound operator returns, held by the call; nullptr: None
 };
 
 void finish(int rc) {
@@ -343,7 +349,7 @@ struct PooledCall : Call {
 };
 
 // ------------------------------------------------------------ bound operators
-// A call marshalled once: holds what it reads (the argument sequences as tuples) and its outputs.
+// A call marshalled once: holds what it reads (the items it was marshalled from, as tuples) and its outputs.
 struct Bound {
     PyObject_HEAD
     Call* call;
@@ -352,10 +358,7 @@ struct Bound {
 
 void bound_dealloc(PyObject* self) {
     Bound* b = reinterpret_cast<Bound*>(self);
-    if (b->call) {
-        Py_XDECREF(b->call->outputs);
-        delete b->call;
-    }
+    delete b->call;
     Py_XDECREF(b->keep);
     Py_TYPE(self)->tp_free(self);
 }
@@ -384,26 +387,23 @@ PyGetSetDef bound_getset[] = {{"outputs", bound_outputs, nullptr, "the tensors e
 
 PyTypeObject BoundType = {PyVarObject_HEAD_INIT(nullptr, 0)};
 
-// keep: what must outlive the call (new reference, taken over)
-PyObject* make_bound(std::unique_ptr<Call> call, PyObject* const* args, int n_sequences) {
-    PyObject* keep = PyTuple_New(n_sequences);
-    if (!keep) throw PyFailed{};
-    for (int i = 0; i < n_sequences; i++) {
-        PyObject* t = PySequence_Tuple(args[i]);
-        if (!t) {
-            Py_DECREF(keep);
-            throw PyFailed{};
-        }
-        PyTuple_SET_ITEM(keep, i, t);
-    }
+// sequences: the items the call was marshalled from, which it needs as long as it lives.  (An argument may be an iterator:
+// going over it again would find nothing.)
+PyObject* make_bound(std::unique_ptr<Call> call, std::initializer_list<const Items*> sequences) {
     Bound* b = PyObject_New(Bound, &BoundType);
-    if (!b) {
-        Py_DECREF(keep);
-        throw PyFailed{};
-    }
+    if (!b) throw PyFailed{};
     b->call = call.release();
-    b->keep = keep;
-    return reinterpret_cast<PyObject*>(b);
+    b->keep = PyTuple_New((Py_ssize_t)sequences.size());  // (bound_dealloc takes nullptr, too)
+    PyObject* self = reinterpret_cast<PyObject*>(b);
+    try {
+        if (!b->keep) throw PyFailed{};
+        Py_ssize_t i = 0;
+        for (const Items* s : sequences) PyTuple_SET_ITEM(b->keep, i++, s->tuple());
+    } catch (const PyFailed&) {
+        Py_DECREF(self);
+        throw;
+    }
+    return self;
 }
 
 void arg_count(Py_ssize_t have, Py_ssize_t want, const char* name) {
@@ -443,10 +443,10 @@ PyObject* py_pull(PyObject*, PyObject* const* a, Py_ssize_t na) {
 PyObject* py_bind_pull(PyObject*, PyObject* const* a, Py_ssize_t na) {
     return guarded([&] {
         arg_count(na, 3, "bind_pull");
-        auto c = std::make_unique<PullCall>(Items(a[0]), Items(a[1]), handle_arg(a[2]));
-        PyObject* out = c->views();
-        c->outputs = out;
-        return make_bound(std::move(c), a, 2);
+        const Items resources(a[0]), values(a[1]);
+        auto c = std::make_unique<PullCall>(resources, values, handle_arg(a[2]));
+        c->outputs = c->views();
+        return make_bound(std::move(c), {&resources, &values});
     });
 }
 
@@ -463,7 +463,8 @@ PyObject* py_push(PyObject*, PyObject* const* a, Py_ssize_t na) {
 PyObject* py_bind_push(PyObject*, PyObject* const* a, Py_ssize_t na) {
     return guarded([&] {
         arg_count(na, 4, "bind_push");
-        return make_bound(std::make_unique<PushCall>(Items(a[0]), Items(a[1]), Items(a[2]), handle_arg(a[3])), a, 3);
+        const Items values(a[0]), grads(a[1]), labels(a[2]);
+        return make_bound(std::make_unique<PushCall>(values, grads, labels, handle_arg(a[3])), {&values, &grads, &labels});
     });
 }
 
@@ -480,11 +481,10 @@ PyObject* py_combine(PyObject*, PyObject* const* a, Py_ssize_t na) {
 PyObject* py_bind_combine(PyObject*, PyObject* const* a, Py_ssize_t na) {
     return guarded([&] {
         arg_count(na, 6, "bind_combine");
-        auto c = std::make_unique<CombineCall>(Items(a[0]), Items(a[1]), Items(a[2]), int_arg(a[3]), handle_arg(a[4]),
-                                               (int)int_arg(a[5]));
-        PyObject* out = c->views();
-        c->outputs = out;
-        return make_bound(std::move(c), a, 3);
+        const Items resources(a[0]), mapped(a[1]), examples(a[2]);
+        auto c = std::make_unique<CombineCall>(resources, mapped, examples, int_arg(a[3]), handle_arg(a[4]), (int)int_arg(a[5]));
+        c->outputs = c->views();
+        return make_bound(std::move(c), {&resources, &mapped, &examples});
     });
 }
 
@@ -501,9 +501,9 @@ PyObject* py_push_pooled(PyObject*, PyObject* const* a, Py_ssize_t na) {
 PyObject* py_bind_push_pooled(PyObject*, PyObject* const* a, Py_ssize_t na) {
     return guarded([&] {
         arg_count(na, 6, "bind_push_pooled");
-        return make_bound(std::make_unique<PooledCall>(Items(a[0]), Items(a[1]), Items(a[2]), Items(a[3]),
-                                                       handle_arg(a[4]), (int)int_arg(a[5])),
-                          a, 4);
+        const Items values(a[0]), examples(a[1]), grads(a[2]), labels(a[3]);
+        return make_bound(std::make_unique<PooledCall>(values, examples, grads, labels, handle_arg(a[4]), (int)int_arg(a[5])),
+                          {&values, &examples, &grads, &labels});
     });
 }
 
