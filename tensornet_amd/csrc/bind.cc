@@ -42,25 +42,25 @@ struct PyFailed {};
     throw PyFailed{};
 }
 
-// The items of a sequence argument; keeps the sequence alive.
+// The items of a sequence argument, in a tuple of their own: another thread may clear or refill the caller's list while
+// the library runs without the interpreter's lock.
 class Items {
 public:
-    explicit Items(PyObject* o) : seq_(PySequence_Fast(o, "expected a sequence of tensors")) {
-        if (!seq_) throw PyFailed{};
+    explicit Items(PyObject* o) : items_(PySequence_Tuple(o)) {
+        if (!items_) throw PyFailed{};
     }
     Items(const Items&) = delete;
-    ~Items() { Py_XDECREF(seq_); }
-    Py_ssize_t size() const { return PySequence_Fast_GET_SIZE(seq_); }
-    PyObject* operator[](Py_ssize_t i) const { return PySequence_Fast_ITEMS(seq_)[i]; }
-    // The items as a tuple (a new reference).
+    ~Items() { Py_DECREF(items_); }
+    Py_ssize_t size() const { return PyTuple_GET_SIZE(items_); }
+    PyObject* operator[](Py_ssize_t i) const { return PyTuple_GET_ITEM(items_, i); }
+    // The tuple (a new reference).
     PyObject* tuple() const {
-        PyObject* t = PySequence_Tuple(seq_);
-        if (!t) throw PyFailed{};
-        return t;
+        Py_INCREF(items_);
+        return items_;
     }
 
 private:
-    PyObject* seq_;
+    PyObject* items_;
 };
 
 // A contiguous device tensor of the given type, or a ValueError that names it.

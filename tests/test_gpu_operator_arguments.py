@@ -1,5 +1,7 @@
 """What the operators keep alive of the sequences they are given (tensornet_amd/csrc/bind.cc)."""
 import gc
+import threading
+import time
 import weakref
 
 import numpy as np
@@ -70,4 +72,51 @@ def test_bound_operators_hold_what_an_iterator_hands_out(tn, oracle):
     pair.assert_rows_match(all_signs(values))
     del ops, pull, combine, push, push_pooled
     gc.collect()
+    assert all(r() is None for r in refs)
+
+
+@pytest.mark.parametrize("op", ["pull", "push", "pooled", "combine"])
+def test_an_operator_holds_its_tensors_while_it_runs(tn, oracle, op):
+    """A second thread empties the caller's lists while the call waits for the device: the tensors stay until it ends."""
+    rng, pair, values, examples, labels = setup(tn, oracle, 2)
+    variables = [np.full((2 * BATCH + 1, D), -7.0, np.float32)] * SLOTS
+    gm = tn.ops.sparse_table_pull([dev(v) for v in variables], [dev(v) for v in values], pair.h)
+    counts = tn.ops.sparse_table_last_unique_counts(pair.h, SLOTS)
+    grads = synth.make_grads(counts, D, 0.01, seed=1)
+    pooled = [rng.standard_normal((BATCH, D)).astype(np.float32) * 0.01 for _ in range(SLOTS)]
+    if op == "pull":
+        lists, call = [variables, values], lambda r, v: tn.ops.sparse_table_pull(r, v, pair.h)
+    elif op == "push":
+        lists, call = [values, grads, labels], lambda v, g, l: tn.ops.sparse_table_push(v, g, l, pair.h)
+    elif op == "pooled":
+        lists, call = [values, examples, pooled, labels], lambda *a: tn.ops.sparse_table_push_pooled(*a, pair.h)
+    else:
+        lists = [variables, [m.cpu().numpy() for m in gm], examples]
+        call = lambda r, m, e: tn.ops.embedding_lookup_sparse(r, m, e, BATCH, pair.h)
+    lists = [[dev(a) for a in arrays] for arrays in lists]
+    refs = [weakref.ref(t) for tensors in lists for t in tensors]
+    torch.cuda.synchronize()
+    entered, ended, seen = threading.Event(), threading.Event(), []
+
+    def empty_the_lists():
+        entered.wait()
+        time.sleep(0.02)
+        if ended.is_set():
+            return
+        for tensors in lists:
+            tensors.clear()
+        gone = [r() is None for r in refs]
+        if not ended.is_set():  # (all this time the call was on its way)
+            seen.append(not any(gone))
+
+    other = threading.Thread(target=empty_the_lists)
+    other.start()
+    torch.cuda._sleep(200_000_000)  # the device is busy for a tenth of a second or so
+    entered.set()
+    call(*lists)
+    ended.set()
+    other.join()
+    torch.cuda.synchronize()
+    tn.ops.sparse_table_sync(pair.h)
+    assert seen == [True]
     assert all(r() is None for r in refs)
