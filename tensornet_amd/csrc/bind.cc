@@ -129,13 +129,31 @@ void finish(int rc) {
     if (rc != TN_OK) status_error(rc, tn_last_error());
 }
 
+// The interpreter's lock is released while this lives (an exception that passes it finds the lock held again).
+class Unlocked {
+public:
+    Unlocked() : state_(PyEval_SaveThread()) {}
+    Unlocked(const Unlocked&) = delete;
+    ~Unlocked() { PyEval_RestoreThread(state_); }
+
+private:
+    PyThreadState* state_;
+};
+
+// A call of the library without the interpreter's lock; an error status becomes Python's exception.
+template <typename F>
+void call_library(F f) {
+    int rc;
+    {
+        const Unlocked unlocked;
+        rc = f();
+    }
+    finish(rc);
+}
+
 void run(Call& c) {
     void* stream = current_stream();
-    int rc;
-    Py_BEGIN_ALLOW_THREADS
-    rc = c.run(stream);
-    Py_END_ALLOW_THREADS
-    finish(rc);
+    call_library([&] { return c.run(stream); });
 }
 
 // A list of n tensors that are consecutive parts of `flat` (as torch.split hands them out), without the dispatcher.
@@ -348,6 +366,22 @@ struct PooledCall : Call {
     }
 };
 
+// Every entry point: C++ exceptions (torch's among them) become Python's.
+template <typename F>
+PyObject* guarded(F f) {
+    try {
+        return f();
+    } catch (const PyFailed&) {
+        return nullptr;
+    } catch (const c10::Error& e) {
+        PyErr_SetString(PyExc_RuntimeError, e.what_without_backtrace());
+        return nullptr;
+    } catch (const std::exception& e) {
+        PyErr_SetString(PyExc_RuntimeError, e.what());
+        return nullptr;
+    }
+}
+
 // ------------------------------------------------------------ bound operators
 // A call marshalled once: holds what it reads (the items it was marshalled from, as tuples) and its outputs.
 struct Bound {
@@ -364,15 +398,13 @@ void bound_dealloc(PyObject* self) {
 }
 
 PyObject* bound_call(PyObject* self, PyObject*, PyObject*) {
-    Bound* b = reinterpret_cast<Bound*>(self);
-    try {
+    return guarded([&] {
+        Bound* b = reinterpret_cast<Bound*>(self);
         run(*b->call);
-    } catch (const PyFailed&) {
-        return nullptr;
-    }
-    PyObject* out = b->call->outputs ? b->call->outputs : Py_None;
-    Py_INCREF(out);
-    return out;
+        PyObject* out = b->call->outputs ? b->call->outputs : Py_None;
+        Py_INCREF(out);
+        return out;
+    });
 }
 
 PyObject* bound_outputs(PyObject* self, void*) {
@@ -410,22 +442,6 @@ void arg_count(Py_ssize_t have, Py_ssize_t want, const char* name) {
     if (have == want) return;
     PyErr_Format(PyExc_TypeError, "%s takes %zd arguments, got %zd", name, want, have);
     throw PyFailed{};
-}
-
-// Every entry point: C++ exceptions (torch's among them) become Python's.
-template <typename F>
-PyObject* guarded(F f) {
-    try {
-        return f();
-    } catch (const PyFailed&) {
-        return nullptr;
-    } catch (const c10::Error& e) {
-        PyErr_SetString(PyExc_RuntimeError, e.what_without_backtrace());
-        return nullptr;
-    } catch (const std::exception& e) {
-        PyErr_SetString(PyExc_RuntimeError, e.what());
-        return nullptr;
-    }
 }
 
 PyObject* none() { Py_RETURN_NONE; }
@@ -530,11 +546,9 @@ PyObject* py_dense_push_pull(PyObject*, PyObject* const* a, Py_ssize_t na) {
             w.lens(2)[i] = g.numel();
         }
         void* stream = current_stream();
-        int rc;
-        Py_BEGIN_ALLOW_THREADS
-        rc = tn_dense_table_push_pull(handle, n, w.ptrs<float>(0), w.ptrs<const float>(1), w.lens(2), (float)lr, stream);
-        Py_END_ALLOW_THREADS
-        finish(rc);
+        call_library([&] {
+            return tn_dense_table_push_pull(handle, n, w.ptrs<float>(0), w.ptrs<const float>(1), w.lens(2), (float)lr, stream);
+        });
         return none();
     });
 }
@@ -549,11 +563,7 @@ PyObject* py_table_pull(PyObject*, PyObject* const* a, Py_ssize_t na) {
         const uint64_t* s = (const uint64_t*)signs.data_ptr();
         float* o = (float*)out.data_ptr();
         void* stream = current_stream();
-        int rc;
-        Py_BEGIN_ALLOW_THREADS
-        rc = tn_sparse_table_pull(handle, s, n, (int)dim, o, stream);
-        Py_END_ALLOW_THREADS
-        finish(rc);
+        call_library([&] { return tn_sparse_table_pull(handle, s, n, (int)dim, o, stream); });
         return THPVariable_Wrap(std::move(out));
     });
 }
@@ -572,11 +582,7 @@ PyObject* py_table_push(PyObject*, PyObject* const* a, Py_ssize_t na) {
         const float* g = (const float*)grads.data_ptr();
         const int64_t n = grads.size(0), dim = grads.size(1);
         void* stream = current_stream();
-        int rc;
-        Py_BEGIN_ALLOW_THREADS
-        rc = tn_sparse_table_push(handle, si, g, n, (int)dim, stream);
-        Py_END_ALLOW_THREADS
-        finish(rc);
+        call_library([&] { return tn_sparse_table_push(handle, si, g, n, (int)dim, stream); });
         return none();
     });
 }
