@@ -174,7 +174,8 @@ int tn_sparse_table_row_layout(uint32_t handle, int* weight_floats, int* state_f
  * device signs, in request order, look the row up -- inserting and
  * initialising it if absent (optimizer_kernel.h:299-308) -- and write its
  * `dim` floats to out[i*dim .. i*dim+dim) (device).  dim must equal the
- * table's weight_floats.
+ * table's weight_floats.  Returns when out is written: it may be read on any
+ * stream then.
  */
 int tn_sparse_table_pull(uint32_t handle, const uint64_t* signs, int64_t n, int dim, float* out, void* stream);
 

@@ -130,11 +130,12 @@ __global__ __launch_bounds__(256) void k_combine_fwd(const SlotDesc* __restrict_
 }
 
 // Behind the last kernel of a call: its error flags to the host, in one word with the number of the call, for which the
-// host polls (a wait on the stream returns about ten microseconds later); the flags start at zero for the next call.
+// host polls (a wait on the stream returns about ten microseconds later).  The flags are taken and set to zero for the
+// next call, which may come on another stream as soon as the word is out, by one atomic.
 __global__ void k_report(DevStatus* status, uint64_t* host_word, uint32_t seq) {
     if (threadIdx.x != 0) return;
-    const unsigned long long w = (unsigned long long)status->err | ((unsigned long long)seq << 32);
-    status->err = 0;
+    const uint32_t err = __hip_atomic_exchange(&status->err, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const unsigned long long w = (unsigned long long)err | ((unsigned long long)seq << 32);
     __hip_atomic_store(reinterpret_cast<unsigned long long*>(host_word), w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 

@@ -102,7 +102,7 @@ struct SparseTable {
     // per workgroup of a small pull's first launch, or of a table-level pull's; hseq [0] a large pull's status is on the host, [1] a push's signs are
     // compared) with the numbers the host expects there next, the dynamic LDS its kernels may have.
     uint64_t* hwords = nullptr;
-    uint64_t* hcomb = nullptr;         // pinned: what a combine op reports (k_report)
+    uint64_t* hcomb = nullptr;         // pinned: what a combine op reports (k_report), and that a table-level pull has ended
     uint32_t seq_comb = 0;
     uint32_t* hseq = nullptr;
     uint32_t seq_pull = 0, seq_verify = 0;
@@ -1709,7 +1709,13 @@ int tn_sparse_table_pull(uint32_t handle, const uint64_t* signs, int64_t n, int 
     const uint32_t seq = ++t->seq_pull;
     TN_LAUNCH(k_table_pull, dim3(workgroups), dim3(256), st, s, make_optdev(t), t->seed, signs, n, per, vec ? 1 : 0, out, rows,
               t->hwords, seq);
+    // The rows are written when the call returns, for readers on any stream: a launch behind the pull says that it has
+    // ended.  (A workgroup's own word does not: its other wavefronts' rows may still be on their way.  60 000 signs of 16
+    // elements pushed and pulled: 52 us by the workgroups' words alone, 54 with this, 61 with a wait for the stream.)
+    const uint32_t end_seq = ++t->seq_comb;
+    TN_LAUNCH(k_report, dim3(1), dim3(64), st, t->dcomb, t->hcomb, end_seq);
     TN_HIP(hipGetLastError());
+    TN_TRY(wait_words(t->hcomb, 1, end_seq, st, "tn_sparse_table_pull"));
     TN_TRY(wait_words(t->hwords, workgroups, seq, st, "tn_sparse_table_pull"));
     uint64_t n_new = 0;
     uint32_t err = 0;

@@ -2,12 +2,13 @@
 // records, in which a sign may occur any number of times, in few launches.
 //
 //   pull  k_table_pull   probe or insert every sign, its row to the output, a word to the host per workgroup
+//         k_report       tells the host that the rows are written
 //   push  k_table_part   per tile of records: table row of every record, the records in order of buckets of rows
 //         k_table_apply  per bucket: its records, tile after tile, grouped by row in LDS and applied in record order
 //
 // The push took twelve launches before: a hash table of the records' signs in memory, a compaction of it, arrival
 // order, ranks in arrival order, a probe per sign and three update kernels; the pull five and a wait for a copy.  Both
-// together, at 60 000 records of 16 elements: 147 us before, 51 us now; at 942 570 records of 10 elements 1250 and 325.
+// together, at 60 000 records of 16 elements: 147 us before, 54 us now; at 942 570 records of 10 elements 1250 and 328.
 #ifndef TN_TABLE_LEVEL_H_
 #define TN_TABLE_LEVEL_H_
 

@@ -4,7 +4,7 @@ oracle."""
 import numpy as np
 import torch
 
-from tensornet_amd import synth
+from tensornet_amd import _lib, synth
 
 KINDS = {"AdaGrad": 0, "Adam": 1, "Ftrl": 2}
 
@@ -106,3 +106,18 @@ def check_pull(pair, values, var_rows=None, loose_col=None):
         # bit-exact rows, including the untouched tail of the variable
         assert (g.view(np.int32) == c.view(np.int32)).all(), "var rows of slot %d" % s
     return counts
+
+
+def kernels_of(tn, fn):
+    """Names of the library's kernels that fn() launches."""
+    lib = _lib.load()
+    lib.tn_profile_reset()
+    lib.tn_profile_enable(1)
+    try:
+        fn()
+        torch.cuda.synchronize()
+    finally:
+        lib.tn_profile_enable(0)
+    names = set(_lib.profile_summary())
+    lib.tn_profile_reset()
+    return names

@@ -7,30 +7,15 @@ import numpy as np
 import pytest
 import torch
 
-from tensornet_amd import _lib, synth
+from tensornet_amd import synth
 
-from helpers import Pair, all_signs, check_pull, dev
+from helpers import Pair, all_signs, check_pull, dev, kernels_of
 
 pytestmark = pytest.mark.gpu
 
 ADAGRAD_HP = dict(learning_rate=0.01, initial_g2sum=0.1, epsilon=1e-8)
 ADAM_HP = dict(learning_rate=1e-3, beta1=0.9, beta2=0.999, epsilon=1e-8)
 FTRL_HP = dict(learning_rate=0.05, beta=1.0, lambda1=1.0, lambda2=1.0)
-
-
-def kernels_of(tn, fn):
-    """Names of the library's kernels that fn() launches."""
-    lib = _lib.load()
-    lib.tn_profile_reset()
-    lib.tn_profile_enable(1)
-    try:
-        fn()
-        torch.cuda.synchronize()
-    finally:
-        lib.tn_profile_enable(0)
-    names = set(_lib.profile_summary())
-    lib.tn_profile_reset()
-    return names
 
 
 def batch(rng, slots, per, pool, hot=0, fresh=None):

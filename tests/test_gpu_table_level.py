@@ -3,11 +3,12 @@ record, edges of a tile, of the tile sizes and of what a bucket's workgroup grou
 many and with more than fit at once, unknown signs, new signs that a request repeats."""
 import numpy as np
 import pytest
+import torch
 
 import tensornet_amd
 from tensornet_amd import synth
 
-from helpers import Pair, dev
+from helpers import Pair, dev, kernels_of
 
 pytestmark = pytest.mark.gpu
 
@@ -61,6 +62,34 @@ def test_pull_of_new_signs(tn, oracle, n):
         out = tn.ops.table_pull(pair.h, req, 16)
         rows, _, found = tn.ops.table_export_rows(pair.h, req)  # (normally distributed: no new row is all zero)
         assert bool(found.all()) and bool((out == rows).all()) and bool((out != 0).any(1).all())
+
+
+@pytest.mark.parametrize("n,fresh", [(300, 0), (60000, 0), (60000, 7)])
+def test_pulled_rows_are_written_when_the_call_returns(tn, oracle, n, fresh):
+    """Read on a stream that nothing orders behind the pull's.  (The rows are a moment behind the workgroups' reports, too
+    short for a reader to show it: that the call ends with a launch behind the one that writes them is looked at.)"""
+    rng = np.random.default_rng(n)
+    pair = Pair(tn, oracle, "AdaGrad", 16, HP["AdaGrad"], reserve=200000)
+    base = pair.populate(synth.splitmix64(np.arange(1, 20001, dtype=np.uint64)))
+    req = base[rng.integers(0, len(base), n)]
+    if fresh:
+        req[:fresh] = synth.splitmix64(np.arange(10**6, 10**6 + fresh, dtype=np.uint64))
+    signs = dev(req.view(np.int64))
+    torch.cuda.synchronize()
+    writer, reader = torch.cuda.Stream(), torch.cuda.Stream()
+    host = torch.empty((n, 16), pin_memory=True)
+
+    def pull():
+        with torch.cuda.stream(writer):
+            out = tn.ops.table_pull(pair.h, signs, 16)
+        with torch.cuda.stream(reader):
+            host.copy_(out, non_blocking=True)
+            out.record_stream(reader)
+
+    assert {"k_table_pull", "k_report"} <= kernels_of(tn, pull)
+    torch.cuda.synchronize()
+    want = tn.ops.table_export_rows(pair.h, signs)[0]
+    assert bool((host == want.cpu()).all())
 
 
 def test_push_of_unknown_signs(tn, oracle):
