@@ -24,7 +24,7 @@ namespace tn {
 
 constexpr int SMALL_SLOT_MAX = 4096;         // lookups of a slot at most
 constexpr int SMALL_SLOT_BITS = 13;          // a position in a slot, its rank, its occurrences fit in 13, 13 and 14 bits
-constexpr int SMALL_SLOTS = 512;             // slots at most
+constexpr int SMALL_SLOTS = 512;             // slots at most (the LDS of k_group_emit: 300 slots of 2912 lookups, 512 of 576)
 constexpr int SMALL_PARTS_MAX = 16;          // workgroups of k_small_slots per slot at most
 constexpr int SMALL_SEGMENTS = 256;          // ... and for all slots together where a slot has more than one
 constexpr int SMALL_WORKGROUPS = SMALL_SLOTS > SMALL_SEGMENTS ? SMALL_SLOTS : SMALL_SEGMENTS;  // of k_small_slots at most

@@ -41,9 +41,24 @@ constexpr uint32_t COMBINE_EXAMPLES = 64;  // examples per workgroup of k_combin
 constexpr int COMBINE_DIRECT = 1024;       // workgroups of it up to which they read the slots' descriptors from pinned host memory
 constexpr size_t LDS_MIN_LOOKUPS = 1024;  // from here on the remap through LDS wins: it also takes fewer launches (cfg1, 8 k lookups: 0.154 -> 0.136 ms)
 
-// Up to this many lookups a batch whose slots are all short (SMALL_SLOT_MAX lookups, SMALL_SLOTS slots) takes the path
-// of few launches (small_batch.h).
+// Which batches take the path of few launches (small_batch.h), beside those its arrays have room for (SMALL_SLOT_MAX
+// lookups a slot, SMALL_SLOTS slots, the LDS its kernels may have).  Up to SMALL_MAX_LOOKUPS lookups, and where the other
+// path groups through LDS (GRP_SLOTS slots), up to SMALL_WORK slots x lookups: every bucket's workgroup looks at all
+// slots, and a slot has one workgroup from 129 slots on, so that both grow with slots x lookups where the other path
+// grows with the lookups.  Push and pull of rows of 16 elements under AdaGrad, us, few launches / the other path:
+//   lookups a slot    1024        2048        3072        4096
+//    26 slots        42 / 114    46 / 112    53 / 122    60 / 119   (the limit of 4096 is that of the field widths)
+//    64              54 / 115    68 / 117    78 / 126    85 / 126
+//   128              81 / 132   104 / 135   120 / 152   133 / 151
+//   192             110 / 149   139 / 159   201 / 189   231 / 195
+//   254             148 / 167   220 / 182   275 / 226   339 / 242
+// They cross at 89 to 106 M slots x lookups (160 to 254 slots; rows of 64: 58 to 90, of 8 under Adam: 120; pulls alone: 115).
+// With pooled gradients, whose reduction is shorter here, at 180 M (192 slots, 700 k lookups: 1.08 times as fast, 254 and
+// 700 k: 1.02, 850 k: 0.96).  A pull does not know what push will follow: it goes by the table's last one.
+// With more than GRP_SLOTS slots the other path is 1.2 to 2.2 times as long wherever this one has room (260 slots, 1 M
+// lookups: 1.29; 300, 850 k: 1.24; 400, 400 k: 1.28; 512, 131 k: 1.47).
 constexpr size_t SMALL_MAX_LOOKUPS = 1u << 20;
+constexpr size_t SMALL_WORK = 100'000'000, SMALL_WORK_POOLED = 180'000'000;
 
 // A small batch of at most this many slots leaves every sign to the lane groups of k_small_apply.  With more slots a
 // sign with SMALL_BIG_GROUP records or more is taken by a wavefront of its own: a small batch's kernels are as long as
@@ -165,6 +180,7 @@ struct SparseTable {
     int pull_slots = 0, push_slots = 0;  // N of the pending calls
     std::vector<int64_t> pending_rows;  // var rows of a pending async pull
     int async_pull = 0;
+    bool pooled_pushes = false;     // the last push had pooled gradients
     bool small_path = true;         // small batches take the path of few launches (tn_sparse_table_set_small_batch_path)
     int latched = TN_OK;
     std::string latched_msg;
@@ -1279,6 +1295,7 @@ bool small_batch_shape(SparseTable* t, int N, const int64_t* lens, SmallShape& b
         max_len = std::max<size_t>(max_len, (size_t)lens[s]);
     }
     if (L == 0 || L > SMALL_MAX_LOOKUPS) return false;
+    if (N <= GRP_SLOTS && (size_t)N * L > (t->pooled_pushes ? SMALL_WORK_POOLED : SMALL_WORK)) return false;
     b.N = N;
     b.L = (uint32_t)L;
     b.max_len = (uint32_t)max_len;
@@ -2324,6 +2341,7 @@ int push_op_impl(uint32_t table_handle, int N, const int64_t* const* values, con
     }
     t->last_stream = st;
     if (L == 0) return TN_OK;
+    t->pooled_pushes = pooled;
     t->one_stream = L < ONE_STREAM_LOOKUPS;
     Plan p{};
     Scratch w{};

@@ -1,5 +1,5 @@
-"""The path of few launches that small batches take (every slot within 4096 lookups, at most 128 slots, at
-most 256 k lookups: tensornet_amd/csrc/small_batch.h), through the C ABI against the CPU oracle at the bar of
+"""The path of few launches that small batches take (every slot within 4096 lookups, at most 512 slots, at most 2^20
+lookups and, up to 255 slots, 10^8 slots x lookups: tensornet_amd/csrc/small_batch.h), through the C ABI against the CPU oracle at the bar of
 test_gpu_sparse.py (mapped ids and pulled rows bit for bit, updated rows within 1e-5 / 1e-7): the shapes on
 either side of its limits, several workgroups per slot, signs with many records on either side of the
 threshold from which a wavefront applies them, inserts, and that a batch of its kind does take it."""
@@ -39,8 +39,8 @@ def batch(rng, slots, per, pool, hot=0, fresh=None):
     (3, 4096, "AdaGrad", ADAGRAD_HP, 16),      # the largest slot of the path, eight workgroups per slot
     (3, 4097, "AdaGrad", ADAGRAD_HP, 16),      # one lookup too many: the path of two bucket levels
     (5, 513, "Adam", ADAM_HP, 16),             # two workgroups per slot
-    (128, 40, "AdaGrad", ADAGRAD_HP, 8),       # the most slots of the path
-    (129, 40, "AdaGrad", ADAGRAD_HP, 8),       # one slot too many
+    (128, 40, "AdaGrad", ADAGRAD_HP, 8),       # the most slots with two workgroups each, were they longer
+    (129, 40, "AdaGrad", ADAGRAD_HP, 8),       # one workgroup per slot
     (12, 300, "Ftrl", FTRL_HP, 4),             # the most slots without k_apply_big: signs with up to 12 records by lane groups
     (13, 300, "Ftrl", FTRL_HP, 4),             # ... with it: 5 records or more by a wavefront
     (26, 1024, "Adam", ADAM_HP, 16),
@@ -89,6 +89,27 @@ def test_a_small_batch_takes_the_path_of_few_launches(tn, oracle):
     assert len(pushed) == 2 and "k_small_verify<true>" in pushed and any(k.startswith("k_small_apply") for k in pushed)
     pulled, pushed = step(4097)
     assert "k_lds_dedup<true>" in pulled and not any(k.startswith("k_small") for k in pulled | pushed)
+
+
+@pytest.mark.parametrize("slots,per,small", [(200, 2500, True), (200, 2501, False), (255, 1569, False), (256, 1569, True)])
+def test_the_path_of_a_batch_with_many_slots(tn, oracle, slots, per, small):
+    """10^8 slots x lookups is the limit up to 255 slots; after a push of pooled gradients it is 1.8 x 10^8."""
+    rng = np.random.default_rng(per)
+    pool = synth.splitmix64(np.arange(1, 20001, dtype=np.uint64)).view(np.int64)
+    pair = Pair(tn, oracle, "AdaGrad", 8, ADAGRAD_HP, reserve=100000)
+    pair.populate(pool.view(np.uint64))
+    values = batch(rng, slots, per, pool, hot=2)
+    counts = []
+    launched = kernels_of(tn, lambda: counts.append(check_pull(pair, values)))
+    assert ("k_small_slots" in launched) == small and ("k_tile_dedup" in launched) != small
+    pair.push_op(values, synth.make_grads(counts[0], 8, 0.01, seed=1), [(rng.random(per) < 0.3).astype(np.int64) for _ in values])
+    pair.assert_rows_match(all_signs(values))
+    gvalues = [dev(v) for v in values]
+    zeros = [torch.zeros_like(v) for v in gvalues]  # (example 0 of one, gradients of zero: the rows keep their weights)
+    tn.ops.sparse_table_push_pooled(gvalues, zeros, [torch.zeros((1, 8), device="cuda")] * slots, zeros, pair.h)
+    gvars = [torch.zeros((per + 1, 8), device="cuda") for _ in values]
+    assert "k_small_slots" in kernels_of(tn, lambda: tn.ops.sparse_table_pull(gvars, gvalues, pair.h))
+    tn.ops.sparse_table_sync(pair.h)
 
 
 def test_a_gradient_matrix_with_too_few_rows_is_reported(tn, oracle):
