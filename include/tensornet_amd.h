@@ -233,9 +233,9 @@ int tn_sparse_table_export_rows(uint32_t handle, const uint64_t* signs, int64_t 
  * The call returns when the per-slot counts and the errors of the call are
  * known on the host (the reference op blocks on a semaphore until the pulled
  * rows are there, sparse_table_ops.cc:236).  The outputs are complete in
- * stream order, as the outputs of a GPU op kernel are: on large batches the
- * copy of the pulled rows into vars may still be running on `stream` when the
- * call returns; work enqueued on `stream` afterwards sees them, a host that
+ * stream order, as the outputs of a GPU op kernel are: the copy of the pulled
+ * rows into vars -- on small batches the mapped ids, too -- may still be running
+ * on `stream` when the call returns; work enqueued on `stream` afterwards sees them, a host that
  * reads them synchronises the stream (or calls tn_sparse_table_sync) first.
  */
 int tn_sparse_table_pull_op(uint32_t table_handle, int N, const int64_t* const* values, const int64_t* value_lens,
@@ -257,7 +257,10 @@ int tn_sparse_table_pull_op(uint32_t table_handle, int N, const int64_t* const* 
  * of the same batch reuses what that pull worked out about the batch once the
  * device has confirmed that the signs are the same, and the call returns when
  * that comparison (one pass over the signs, queued ahead of the updates) has
- * reported to the host.
+ * reported to the host.  A push on that plan whose grad_rows[s] is below the
+ * slot's distinct signs applies the records that have a row; a small batch's is
+ * refused with TN_ERR_INVALID_ARGUMENT at once, a larger one's is reported like
+ * the other errors.  Either may be pushed again.
  */
 int tn_sparse_table_push_op(uint32_t table_handle, int N, const int64_t* const* values, const int64_t* value_lens,
                             const float* const* grads, const int64_t* grad_rows, int grad_dim,
@@ -291,9 +294,11 @@ int tn_sparse_table_combine_op(uint32_t table_handle, int N, const int64_t* cons
  * is a device matrix [batch, grad_dim]; the gradient row of the j-th distinct
  * sign of slot s -- what TensorFlow hands the reference's op as grads[s][j, :],
  * core/kernels/sparse_table_ops.cc:336-352 -- is
- *   sum over the lookups of that sign, in order, of pooled_grads[s][example, :] * (1 / d(n_example))
+ *   sum over the lookups of that sign of pooled_grads[s][example, :] * (1 / d(n_example))
  * computed on the device (the segmented reduction of the per-lookup gradients)
- * and applied like a push.  Enqueues and returns like tn_sparse_table_push_op.
+ * and applied like a push.  The sum runs in the order of the lookups; that of a
+ * sign with more than 32 lookups in the slot may be put together from partial
+ * sums, in an order that is the same in every run.  Enqueues and returns like tn_sparse_table_push_op.
  */
 int tn_sparse_table_push_pooled_op(uint32_t table_handle, int N, const int64_t* const* values,
                                    const int64_t* value_lens, const int64_t* const* example_ids,

@@ -6,10 +6,14 @@
 //
 //   forward   out[b, :] = (sum over the lookups i of example b, in order, of var[mapped[i], :]) / d(n_b)
 //             d(n) = 1 (sum), n (mean), sqrt(n) (sqrtn); an example without lookups gives zeros
-//   backward  g[u, :]   = sum over the lookups i of distinct sign u, in order, of dout[b(i), :] * (1 / d(n_b(i)))
+//   backward  g[u, :]   = sum over the lookups i of distinct sign u of dout[b(i), :] * (1 / d(n_b(i)))
 //
-// Both are deterministic: sums run in occurrence order.  The backward pass
-// gets the lookups of every distinct sign side by side, in position order, from a
+// Both are deterministic.  The forward sums run in occurrence order, and so do the backward
+// sums of the signs with few lookups; a sign with ORDER_MID (64) lookups or more in a slot is
+// summed by a workgroup, whose thread groups take every so many of its lookups and whose
+// partial sums are added in group order (k_reduce_pooled).  (On the path of few launches a sign
+// with more than POOL_PIECE (32) lookups is summed in pieces of as many, k_small_pool.)  The
+// backward pass gets the lookups of every distinct sign side by side, in position order, from a
 // counting sort per slot followed by an ordering of every sign's lookups by position
 // (k_place_lookups, k_order_segments).
 #ifndef TN_COMBINE_KERNELS_H_
@@ -238,6 +242,7 @@ __global__ __launch_bounds__(256) void k_lookup_keys(const SlotDesc* __restrict_
 //   rank_short       a lookup of a short segment finds its place by counting the positions of its segment below its own
 //   rank_mid         a sorting network in LDS, one workgroup per segment of ORDER_MID .. ORDER_HUGE - 1 lookups
 //   order_huge       the few longer segments: a bitmap of their positions in LDS, one workgroup each
+//                    (the three are workgroups of one launch, k_order_segments)
 // A slot with more distinct signs than the LDS array holds (lds_cap) keeps its counters in `gcur`.
 constexpr int PLACE_THREADS = 1024;
 constexpr int PLACE_ITEMS = 8;

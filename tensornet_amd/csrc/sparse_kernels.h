@@ -1063,7 +1063,7 @@ __global__ __launch_bounds__(256) void k_group_rank(int64_t n_host, const uint32
     }
 }
 
-// ------------------------------------------ grouping by slot masks (N <= 128)
+// ------------------- grouping by slot masks in memory (N <= 128; a pull's through LDS: remap_lds.h)
 // Within one slot all signs are distinct, so a sign has at most one record per
 // slot and its records in ascending order are its slots in ascending order.
 // With at most 128 slots the set of slots of a sign fits two words: records

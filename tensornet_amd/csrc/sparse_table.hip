@@ -825,8 +825,8 @@ void launch_grouping(const Plan& p, const Scratch& w, const PushSrc& src, int64_
 constexpr int MASK_SLOTS = 128;
 constexpr uint32_t LONG_SEGMENT = 64;  // lookups of one distinct sign from which a workgroup sums them
 
-
-// The same result for the distinct signs of an op with at most 128 slots, from slot masks.
+// The same result for the distinct signs of an op with at most MASK_SLOTS slots, from slot masks.  (Where the signs are not
+// grouped through LDS: a pull that does not wait for its stream, a push that analyses its batch itself.)
 void launch_mask_grouping(const Plan& p, const Scratch& w, int64_t n_upper, uint32_t big_k, const uint32_t* ushow,
                           DevStatus* ds, hipStream_t st) {
     MaskEntry* gt = static_cast<MaskEntry*>(w.gt);

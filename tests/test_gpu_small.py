@@ -36,9 +36,9 @@ def batch(rng, slots, per, pool, hot=0, fresh=None):
 
 @pytest.mark.parametrize("slots,per,opt,hyper,dim", [
     (1, 1, "AdaGrad", ADAGRAD_HP, 8),          # one lookup
-    (3, 4096, "AdaGrad", ADAGRAD_HP, 16),      # the largest slot of the path, eight workgroups per slot
+    (3, 4096, "AdaGrad", ADAGRAD_HP, 16),      # the largest slot of the path, sixteen workgroups per slot
     (3, 4097, "AdaGrad", ADAGRAD_HP, 16),      # one lookup too many: the path of two bucket levels
-    (5, 513, "Adam", ADAM_HP, 16),             # two workgroups per slot
+    (5, 513, "Adam", ADAM_HP, 16),             # five workgroups per slot
     (128, 40, "AdaGrad", ADAGRAD_HP, 8),       # the most slots with two workgroups each, were they longer
     (129, 40, "AdaGrad", ADAGRAD_HP, 8),       # one workgroup per slot
     (12, 300, "Ftrl", FTRL_HP, 4),             # the most slots without k_apply_big: signs with up to 12 records by lane groups
