@@ -65,7 +65,9 @@ __device__ __forceinline__ uint32_t ids_below(const int64_t* __restrict__ ex, ui
 // before its predecessor.
 //
 // The variable rows of a slot are read again and again: every die of the chip takes a contiguous share of the items, so
-// that a slot's rows (1.3 MB at 20 k distinct signs of 16 elements) are in the L2 of the die that wants them.
+// that a slot's rows (1.3 MB at 20 k distinct signs of 16 elements) are in the L2 of the die that wants them.  By the
+// counters they are: 4.9 M lookups read 225 MB from memory where every row and id once are 206, 62 % of the requests to L2
+// hit; 121 us, 2.7 TB/s, the wavefronts wait 61 % of their cycles.
 template <int LPG, bool ANY>
 __global__ __launch_bounds__(256) void k_combine_fwd(const SlotDesc* __restrict__ descs, uint32_t items, uint32_t per_slot,
                                                      uint32_t per, int dim, int64_t batch, int combiner, DevStatus* status) {
@@ -253,9 +255,11 @@ constexpr uint32_t ORDER_HUGE = 1024;
 // and takes those whose distinct index lies in its share of the slot's window of distinct indices.  The lookups of the
 // indices below its share, which it counts on the way, come before its own.
 //
-// What bounds it are the scattered stores: a die has the windows of a dozen slots in its L2 at a time, and lines that are
-// written out half filled are read and written again.  Only the position is stored, 4 bytes per lookup (a die's windows:
-// 2.5 MB at 49 k lookups a slot), and not the index and the value with it (12 bytes, 7.5 MB: more than its L2).
+// What bounds it is the chain of each of its few workgroups (two passes over the slot's lookups with an LDS atomic each, the
+// scan between them): the wavefronts wait 85 % of their cycles while 79 MB are read and 49 written (39 and 28 would do), 1.0
+// TB/s.  Only the position is stored, 4 bytes per lookup, and not the index and the value with it (12 bytes): a die has
+// the windows of a dozen slots in its L2 at a time (2.5 MB at 49 k lookups a slot; 7.5 MB with the value, more than its
+// L2), and lines that are written out half filled are read and written again.
 // 4.9 M lookups in 100 slots: 168 us before, 135 with one workgroup per slot and 125 with two.
 __global__ __launch_bounds__(PLACE_THREADS) void k_place_lookups(
     const uint32_t* __restrict__ lbase, const uint32_t* __restrict__ ubase, int N, uint32_t L,
@@ -334,7 +338,9 @@ __global__ __launch_bounds__(PLACE_THREADS) void k_place_lookups(
 }
 
 // The lookups in the order of their segments: the runs of a die (DieRuns) keep to one slot, whose distinct indices and
-// values, read by position, are then in its L2.  4.9 M lookups: 78 -> 62 us.
+// values, read by position, are then more often in its L2.  4.9 M lookups: 78 -> 62 us.  Bound by the reads by
+// position: with the longer segments beside it 340 MB come from memory where 87 would do (56 % of the L2's requests hit),
+// 4.4 TB/s, about what random granules reach.
 constexpr uint32_t RANK_RUN = 128;
 
 __device__ __forceinline__ void rank_short(uint32_t L, const uint32_t* __restrict__ u_of_gi,
@@ -497,10 +503,11 @@ __device__ __forceinline__ float4 sum_shares(const float* __restrict__ pooled, c
 // lookups or more (a frequent sign) is left out: k_place_lookups has listed those, one workgroup each sums them
 // (reduce_long).
 //
-// Bound by the rows it reads again and again: the pooled rows of a slot (1 MB at 16384 examples of 16 elements) stay in
-// the L2 of a die that works on one slot at a time, so the distinct indices go to the dies in runs of REDUCE_RUN
+// Bound by the rows it reads again and again: the pooled rows of a slot (1 MB at 16384 examples of 16 elements) are more
+// often in the L2 of a die that works on one slot at a time, so the distinct indices go to the dies in runs of REDUCE_RUN
 // workgroups (DieRuns; a grid-stride loop had every die read the rows of six slots).  4.9 M lookups of 16 elements:
-// 172 -> 138 us, the frequent signs beside it 120 -> 93 us.
+// 172 -> 138 us, the frequent signs beside it 120 -> 93 us.  By the counters of both together 30 % of the L2's requests hit:
+// 426 MB are read where each row and value once are 152, with what is written 3.8 TB/s.
 constexpr uint32_t REDUCE_RUN = 256;
 
 template <bool ANY>
