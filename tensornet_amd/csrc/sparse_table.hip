@@ -185,7 +185,8 @@ struct SparseTable {
     int latched = TN_OK;
     std::string latched_msg;
     std::vector<int64_t> last_counts;
-    hipStream_t last_stream = nullptr;
+    hipStream_t last_stream = nullptr;  // of the table's last call, if it had one (nullptr is the default stream)
+    bool had_call = false;
     std::mutex mu;
 };
 
@@ -356,10 +357,18 @@ int order_after_updates(SparseTable* t, hipStream_t st) {
     return TN_OK;
 }
 
+// (The default stream is one like any other here: streams made with hipStreamNonBlocking are not ordered behind it.)
+bool other_stream(const SparseTable* t, hipStream_t st) { return t->had_call && t->last_stream != st; }
+
+void set_last_stream(SparseTable* t, hipStream_t st) {
+    t->last_stream = st;
+    t->had_call = true;
+}
+
 // A call on another stream than the table's last one: what that call left running there (a pull's gather, a small
 // push's updates: tail_ev) is waited for on the device, and a call whose status is still pending on the host.
 int order_after_other_stream(SparseTable* t, hipStream_t st) {
-    if (!t->last_stream || t->last_stream == st) return TN_OK;
+    if (!other_stream(t, st)) return TN_OK;
     if (t->tail_recorded) TN_HIP(hipStreamWaitEvent(st, t->tail_ev, 0));
     if (t->push_pending || t->pull_pending) TN_HIP(hipStreamSynchronize(t->last_stream));
     return TN_OK;
@@ -472,7 +481,7 @@ int sync_table(SparseTable* t, hipStream_t st) {
         t->upd_pending = false;
     }
     TN_HIP(hipStreamSynchronize(st));
-    if (t->last_stream && t->last_stream != st) TN_HIP(hipStreamSynchronize(t->last_stream));
+    if (other_stream(t, st)) TN_HIP(hipStreamSynchronize(t->last_stream));
     harvest(t);
     return take_latched(t);
 }
@@ -1576,7 +1585,7 @@ int tn_sparse_table_clear(uint32_t handle) {
     std::lock_guard<std::mutex> lk(t->mu);
     if (!t->allocated) return TN_OK;
     // everything the table has queued, on whichever stream
-    if (t->last_stream) TN_HIP(hipStreamSynchronize(t->last_stream));
+    TN_HIP(hipStreamSynchronize(t->last_stream));
     TN_HIP(hipStreamSynchronize(t->side));
     TN_HIP(hipStreamSynchronize(t->side2));
     TN_HIP(hipStreamSynchronize(t->aux));
@@ -1709,12 +1718,12 @@ int tn_sparse_table_pull(uint32_t handle, const uint64_t* signs, int64_t n, int 
                     "tn_sparse_table_pull: dim " + std::to_string(dim) + " but table rows hold " + std::to_string(wdim));
     if (n > 0x7FFFFFF0LL) return fail(TN_ERR_UNSUPPORTED, "tn_sparse_table_pull: more than 2^31 signs");
     // a push pending on this stream is collected behind this call's own wait
-    if (t->pull_pending || (t->push_pending && t->last_stream && t->last_stream != st)) {
-        if (t->last_stream && t->last_stream != st) TN_HIP(hipStreamSynchronize(t->last_stream));
+    if (t->pull_pending || (t->push_pending && other_stream(t, st))) {
+        if (other_stream(t, st)) TN_HIP(hipStreamSynchronize(t->last_stream));
         TN_HIP(hipStreamSynchronize(st));
         harvest(t);
     }
-    t->last_stream = st;
+    set_last_stream(t, st);
     if (n == 0) return sync_table(t, st);
     TN_TRY(ensure_room(t, (uint64_t)n, st));
     TN_TRY(t->ws.ensure(align_up((size_t)n * sizeof(uint32_t), 256)));
@@ -1810,11 +1819,11 @@ int tn_sparse_table_pull_static(uint32_t handle, const uint64_t* signs, int64_t 
         return fail(TN_ERR_DIM_MISMATCH, "tn_sparse_table_pull_static: dim " + std::to_string(dim) +
                                              " but table rows hold " + std::to_string(wdim));
     if (t->push_pending || t->pull_pending) {
-        if (t->last_stream && t->last_stream != st) TN_HIP(hipStreamSynchronize(t->last_stream));
+        if (other_stream(t, st)) TN_HIP(hipStreamSynchronize(t->last_stream));
         TN_HIP(hipStreamSynchronize(st));
         harvest(t);
     }
-    t->last_stream = st;
+    set_last_stream(t, st);
     if (n == 0) return sync_table(t, st);
     const Store& s = t->store;
     // every requested sign may be new; a table that would have to grow for them needs a new allocation
@@ -1867,11 +1876,11 @@ int tn_sparse_table_push(uint32_t handle, const tn_sign_info* infos, const float
                     "tn_sparse_table_push: dim " + std::to_string(dim) + " but table rows hold " + std::to_string(wdim));
     if (n > 0x7FFFFFF0LL) return fail(TN_ERR_UNSUPPORTED, "tn_sparse_table_push: more than 2^31 records");
     if (n > 0 && (t->push_pending || t->pull_pending)) {  // one status block per direction: collect the previous one first
-        if (t->last_stream && t->last_stream != st) TN_HIP(hipStreamSynchronize(t->last_stream));
+        if (other_stream(t, st)) TN_HIP(hipStreamSynchronize(t->last_stream));
         TN_HIP(hipStreamSynchronize(st));
         harvest(t);
     }
-    t->last_stream = st;
+    set_last_stream(t, st);
     if (n == 0) return TN_OK;
     const Store& s = t->store;
     const RowShare share = row_share(s, aligned16(grads) && dim % 4 == 0 && s.wstride % 4 == 0);
@@ -1949,7 +1958,7 @@ int tn_sparse_table_load_rows(uint32_t handle, const uint64_t* signs, const floa
     std::lock_guard<std::mutex> lk(t->mu);
     hipStream_t st = (hipStream_t)stream;
     TN_TRY(ensure_allocated(t, st));
-    t->last_stream = st;
+    set_last_stream(t, st);
     if (n == 0) return TN_OK;
     if (n > 0x7FFFFFF0LL) return fail(TN_ERR_UNSUPPORTED, "tn_sparse_table_load_rows: more than 2^31 rows per call");
     if (t->push_pending || t->pull_pending) {
@@ -1983,7 +1992,7 @@ int tn_sparse_table_export_rows(uint32_t handle, const uint64_t* signs, int64_t 
     std::lock_guard<std::mutex> lk(t->mu);
     hipStream_t st = (hipStream_t)stream;
     TN_TRY(ensure_allocated(t, st));
-    t->last_stream = st;
+    set_last_stream(t, st);
     if (n == 0) return TN_OK;
     if (n > 0x7FFFFFF0LL) return fail(TN_ERR_UNSUPPORTED, "tn_sparse_table_export_rows: more than 2^31 rows per call");
     if (t->push_pending || t->pull_pending) {
@@ -2025,11 +2034,11 @@ int tn_sparse_table_export_range(uint32_t handle, uint64_t first_slot, uint64_t 
     hipStream_t st = (hipStream_t)stream;
     TN_TRY(ensure_allocated(t, st));
     if (t->push_pending || t->pull_pending) {
-        if (t->last_stream && t->last_stream != st) TN_HIP(hipStreamSynchronize(t->last_stream));
+        if (other_stream(t, st)) TN_HIP(hipStreamSynchronize(t->last_stream));
         TN_HIP(hipStreamSynchronize(st));
         harvest(t);
     }
-    t->last_stream = st;
+    set_last_stream(t, st);
     *count = 0;
     const Store& s = t->store;
     if (n_slots == 0 || first_slot > s.cap) return TN_OK;
@@ -2066,11 +2075,11 @@ int tn_sparse_table_show_decay(uint32_t handle, int delta_days, void* stream) {
     hipStream_t st = (hipStream_t)stream;
     TN_TRY(ensure_allocated(t, st));
     if (t->push_pending || t->pull_pending) {
-        if (t->last_stream && t->last_stream != st) TN_HIP(hipStreamSynchronize(t->last_stream));
+        if (other_stream(t, st)) TN_HIP(hipStreamSynchronize(t->last_stream));
         TN_HIP(hipStreamSynchronize(st));
         harvest(t);
     }
-    t->last_stream = st;
+    set_last_stream(t, st);
     if (t->opt->kind == OPT_ADAM) return TN_OK;  // adam_kernel.h:67
     const Store& s = t->store;
     TN_LAUNCH(k_show_decay, dim3(launch_grid((int64_t)s.cap + 1, 256, GRID_CAP * 8)), dim3(256), st, s, make_decayconf(t),
@@ -2086,7 +2095,7 @@ int tn_sparse_table_delete_by_show(uint32_t handle, const uint64_t* signs, int64
     std::lock_guard<std::mutex> lk(t->mu);
     hipStream_t st = (hipStream_t)stream;
     TN_TRY(ensure_allocated(t, st));
-    t->last_stream = st;
+    set_last_stream(t, st);
     if (n == 0) return TN_OK;
     if (n > 0x7FFFFFF0LL) return fail(TN_ERR_UNSUPPORTED, "tn_sparse_table_delete_by_show: more than 2^31 rows per call");
     if (t->push_pending || t->pull_pending) {
@@ -2125,14 +2134,14 @@ int tn_sparse_table_pull_op(uint32_t table_handle, int N, const int64_t* const* 
                                              " but table rows hold " + std::to_string(wdim));
     // An earlier push on the same stream need not be waited for: this call runs behind it and
     // collects its status when it waits for its own work.
-    const bool same_stream = !t->last_stream || t->last_stream == st;
+    const bool same_stream = !other_stream(t, st);
     if (!same_stream || t->async_pull) TN_TRY(order_after_updates(t, st));
     if (t->pull_pending || (t->push_pending && (t->async_pull || !same_stream))) {
         if (!same_stream) TN_HIP(hipStreamSynchronize(t->last_stream));
         TN_HIP(hipStreamSynchronize(st));
         harvest(t);
     }
-    t->last_stream = st;
+    set_last_stream(t, st);
     // The remap through LDS needs the call's status on the host to fall back if a
     // bucket overflowed, so it is only used when the pull waits for its stream anyway.
     bool use_lds = !t->async_pull;
@@ -2335,11 +2344,11 @@ int push_op_impl(uint32_t table_handle, int N, const int64_t* const* values, con
     }
     if (t->push_pending || t->pull_pending) {
         // a call pending on another stream (an asynchronous pull) builds the plan this push reads
-        if (t->last_stream && t->last_stream != st) TN_HIP(hipStreamSynchronize(t->last_stream));
+        if (other_stream(t, st)) TN_HIP(hipStreamSynchronize(t->last_stream));
         TN_HIP(hipStreamSynchronize(st));
         harvest(t);
     }
-    t->last_stream = st;
+    set_last_stream(t, st);
     if (L == 0) return TN_OK;
     t->pooled_pushes = pooled;
     t->one_stream = L < ONE_STREAM_LOOKUPS;
@@ -2606,11 +2615,11 @@ int tn_sparse_table_combine_op(uint32_t table_handle, int N, const int64_t* cons
     }
     // an earlier call's status is collected first
     if (t->push_pending || t->pull_pending) {
-        if (t->last_stream && t->last_stream != st) TN_HIP(hipStreamSynchronize(t->last_stream));
+        if (other_stream(t, st)) TN_HIP(hipStreamSynchronize(t->last_stream));
         TN_HIP(hipStreamSynchronize(st));
         harvest(t);
     }
-    t->last_stream = st;
+    set_last_stream(t, st);
     if (t->stage_pending) {
         TN_HIP(hipEventSynchronize(t->stage_ev));
         t->stage_pending = false;
