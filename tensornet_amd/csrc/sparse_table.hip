@@ -366,7 +366,7 @@ void set_last_stream(SparseTable* t, hipStream_t st) {
 }
 
 // A call on another stream than the table's last one: what that call left running there (a pull's gather, a small
-// push's updates: tail_ev) is waited for on the device, and a call whose status is still pending on the host.
+// push's updates, a decay: tail_ev) is waited for on the device, and a call whose status is still pending on the host.
 int order_after_other_stream(SparseTable* t, hipStream_t st) {
     if (!other_stream(t, st)) return TN_OK;
     if (t->tail_recorded) TN_HIP(hipStreamWaitEvent(st, t->tail_ev, 0));
@@ -2084,6 +2084,8 @@ int tn_sparse_table_show_decay(uint32_t handle, int delta_days, void* stream) {
     const Store& s = t->store;
     TN_LAUNCH(k_show_decay, dim3(launch_grid((int64_t)s.cap + 1, 256, GRID_CAP * 8)), dim3(256), st, s, make_decayconf(t),
               delta_days);
+    TN_HIP(hipEventRecord(t->tail_ev, st));  // (still running when this call returns)
+    t->tail_recorded = true;
     TN_HIP(hipGetLastError());
     return TN_OK;
 }

@@ -14,7 +14,7 @@ HP = dict(learning_rate=0.01, initial_g2sum=0.1, epsilon=1e-8)
 
 
 @pytest.mark.parametrize("first", ["default", "own"])
-@pytest.mark.parametrize("what", ["push"])
+@pytest.mark.parametrize("what", ["push", "decay"])
 def test_a_call_waits_for_what_another_stream_still_runs(tn, oracle, first, what):
     """The first stream is busy when the call is queued on it, the second is not.  (Several second streams: one that shares
     a hardware queue with the first would be ordered behind it in any case.)"""
