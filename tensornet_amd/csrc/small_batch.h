@@ -6,9 +6,9 @@
 //                                lookup-or-insert of every distinct sign (sparse_table.cc:52-66), its record filed by
 //                                bucket; every workgroup reports to the host, which returns when it has them all
 //         k_small_group_finish   ranks of the first occurrences -> mapped ids, rows into the variables
-//                                (sparse_table_ops.cc:244-265)
-//         k_group_emit<true>     per bucket: the groups of equal signs over all slots, their records in slot order
-//   push  k_small_verify         comparison with the plan's signs, click sums
+//                                (sparse_table_ops.cc:244-265); beside it, per bucket: the groups of equal signs over all
+//                                slots, their records in slot order
+//   push  k_small_verify         comparison with the plan's signs, click sums; beside it the ranks into the records
 //         k_small_pool           (pooled gradients) the gradient of every distinct sign from those of its examples
 //         k_small_apply          per bucket: every sign's records in order (tells the host that the comparison is complete)
 //
@@ -20,22 +20,24 @@
 
 #include "remap_lds.h"
 
+#include <algorithm>
+
 namespace tn {
 
 constexpr int SMALL_SLOT_MAX = 4096;         // lookups of a slot at most
 constexpr int SMALL_SLOT_BITS = 13;          // a position in a slot, its rank, its occurrences fit in 13, 13 and 14 bits
-constexpr int SMALL_SLOTS = 512;             // slots at most (the LDS of k_group_emit: 300 slots of 2912 lookups, 512 of 576)
+constexpr int SMALL_SLOTS = 512;             // slots at most (the LDS of small_emit_bucket: 300 slots of 2912 lookups, 512 of 576)
 constexpr int SMALL_PARTS_MAX = 16;          // workgroups of k_small_slots per slot at most
 constexpr int SMALL_SEGMENTS = 256;          // ... and for all slots together where a slot has more than one
 constexpr int SMALL_WORKGROUPS = SMALL_SLOTS > SMALL_SEGMENTS ? SMALL_SLOTS : SMALL_SEGMENTS;  // of k_small_slots at most
 constexpr int SMALL_PART_LOOKUPS = 128;      // lookups of a slot per workgroup aimed at
 constexpr int SMALL_BUCKET_RECORDS = 64;     // records per bucket aimed at (if every lookup were distinct)
 constexpr int SMALL_BUCKETS_MAX = 2048;
-constexpr int SMALL_THREADS = 512;           // k_small_slots, k_small_group_finish
+constexpr int SMALL_THREADS = 512;           // k_small_slots
 constexpr int SMALL_ITEMS = SMALL_SLOT_MAX / SMALL_THREADS;
 constexpr int SMALL_WORDS = SMALL_SLOT_MAX / 64;  // 64-lookup words of a slot
 constexpr int SMALL_NEW = 512;               // rows a workgroup of k_small_slots lists to fill them with all its threads
-constexpr int EMIT_SMALL_THREADS = 256;
+constexpr int FINISH_THREADS = 256;          // k_small_group_finish
 constexpr int SMALL_TILE = 1024;             // lookups per workgroup of k_small_verify
 static_assert(SMALL_SLOT_MAX < (1 << SMALL_SLOT_BITS), "positions fit");
 
@@ -65,7 +67,8 @@ struct SmallPlan {
     uint16_t* boff;        // [slot][part][nbp + 1]: where the buckets start in them
     uint4* head;           // per bucket {signs with one record, with a few, with many, records of the latter two}
     uint2* group;          // per bucket, `cap` each: {row, first record | records << 16}; those with many records from the end on
-    uint4* member;         // per bucket, `cap` each: records {gi, rank | slot << 16, occurrences, 0}, those of a sign in slot order
+    uint4* member;         // per bucket, `cap` each: records {gi, rank | slot << 16, occurrences, 0}, those of a sign in slot
+                           // order (the rank comes in with a push, k_small_verify)
     uint32_t* bad;         // != 0: a bucket did not fit, a push has to analyse the batch itself
 };
 
@@ -251,68 +254,11 @@ __global__ __launch_bounds__(SMALL_THREADS) void k_small_slots(SmallShape b, Sma
     }
 }
 
-// Second launch of a small pull: mapped ids (rank of the sign's first lookup) and, for the first lookups, the table row
-// into the variable.  A workgroup takes a run of positions of one slot, a thread per position and part of a row.
-template <int VEC>
-__global__ __launch_bounds__(SMALL_THREADS) void k_small_group_finish(SmallShape b, SmallPlan p,
-                                                                      uint32_t chunks, Store s) {
-    __shared__ unsigned long long bits[SMALL_WORDS];
-    __shared__ uint32_t before[SMALL_WORDS];
-    const int sl = blockIdx.x / chunks;
-    const uint32_t C = (uint32_t)(s.wdim / VEC), per = SMALL_THREADS / C;  // positions per workgroup
-    const uint32_t p0 = (blockIdx.x % chunks) * per;
-    const SlotDesc d = p.descs[sl];
-    if (p0 >= d.len) return;
-    const uint32_t tid = threadIdx.x;
-    const uint32_t pos = p0 + tid / C, c = tid % C;
-    const bool active = tid < per * C && pos < d.len;
-    const uint32_t gi = d.lbase + pos;
-    const uint32_t f = active ? p.first_of[gi] : 0u;
-    const uint32_t row = active ? p.row_at[gi] : NO_ROW;  // (of a first lookup only)
-    const bool first = active && f == pos;
-    if (tid < SMALL_WORDS) {
-        uint64_t v = 0;
-        if (tid < b.words) {
-            const uint64_t* w = p.bits + (size_t)sl * b.parts * b.words + tid;
-            for (uint32_t q = 0; q < b.parts; q++) v |= w[(size_t)q * b.words];
-        }
-        bits[tid] = v;
-        const uint32_t n = (uint32_t)__popcll(v);
-        uint32_t inc = n;
-        for (int x = 1; x < 64; x <<= 1) {
-            const uint32_t y = __shfl_up(inc, x);
-            if ((int)tid >= x) inc += y;
-        }
-        before[tid] = inc - n;
-    }
-    static_assert(SMALL_WORDS == 64, "one wavefront scans the words");
-    const bool copy = first && row <= s.cap;  // NO_ROW (table full): never address the table with it
-    float4 v4 = make_float4(0.f, 0.f, 0.f, 0.f);
-    float v1 = 0.f;
-    if (copy) {
-        if (VEC == 4)
-            v4 = *reinterpret_cast<const float4*>(s.w + (uint64_t)row * s.wstride + c * 4);
-        else
-            v1 = s.w[(uint64_t)row * s.wstride + c];
-    }
-    __syncthreads();
-    if (!active) return;
-    const uint32_t rank = before[f >> 6] + (uint32_t)__popcll(bits[f >> 6] & ((1ull << (f & 63)) - 1ull));
-    if (c == 0) {
-        d.mapped[pos] = (int64_t)rank;
-        if (first) p.rank_at[gi] = (uint16_t)rank;
-    }
-    if (!copy || (int64_t)rank >= d.rows) return;  // (the host reports a variable that is too small)
-    if (VEC == 4)
-        *reinterpret_cast<float4*>(d.var + (uint64_t)rank * s.wdim + c * 4) = v4;
-    else
-        d.var[(uint64_t)rank * s.wdim + c] = v1;
-}
-
-// Third launch of a small pull, a workgroup per bucket: its records, slot after slot, grouped by row in LDS.
+// What is left of a small pull behind its first launch: small_emit_bucket, a workgroup per bucket, and small_finish.
+// Neither needs what the other works out.
 template <>
 struct EmitArgs<true> {
-    static constexpr int THREADS = EMIT_SMALL_THREADS;
+    static constexpr int THREADS = FINISH_THREADS;
     SmallShape b;
     SmallPlan p;
     uint32_t table;  // entries of the LDS hash table of rows at most: a power of two, 5/4 of the room of a bucket
@@ -325,10 +271,11 @@ inline uint32_t small_emit_table(uint32_t cap) {
 }
 inline size_t small_emit_lds(int N, uint32_t cap, uint32_t table) {
     // per slot: records before it, where its records are, its first lookup; table: row, records / number;
-    // per record: row, gi, rank | slot, occurrences | entry, arrival, list
-    return align_up((size_t)(N + 1) * 4 + (size_t)N * 8 + (size_t)table * 12 + (size_t)cap * 22, 8);
+    // per record: row, gi, occurrences | entry, arrival, slot, list
+    return align_up((size_t)(N + 1) * 4 + (size_t)N * 8 + (size_t)table * 12 + (size_t)cap * 20, 8);
 }
 
+// The records of a bucket, slot after slot, grouped by row in LDS.
 __device__ __forceinline__ void small_emit_bucket(const EmitArgs<true>& a, uint32_t* lds) {
     const SmallShape& b = a.b;
     const SmallPlan& p = a.p;
@@ -341,16 +288,16 @@ __device__ __forceinline__ void small_emit_bucket(const EmitArgs<true>& a, uint3
     uint32_t* tinfo = tcnt + a.table;        // [table]: number of the group | first record << 16 (several records)
     uint32_t* rrow = tinfo + a.table;        // [cap]
     uint32_t* rgi = rrow + b.cap;            // [cap]
-    uint32_t* rrs = rgi + b.cap;             // [cap]
-    uint32_t* rce = rrs + b.cap;             // [cap]: occurrences (14 bits) | entry << 14
+    uint32_t* rce = rgi + b.cap;             // [cap]: occurrences (14 bits) | entry << 14
     uint32_t* rarr = rce + b.cap;            // [cap]
-    uint16_t* list = reinterpret_cast<uint16_t*>(rarr + b.cap);  // [cap]
-    __shared__ uint32_t wsum[EMIT_SMALL_THREADS / 64];
+    uint16_t* rsl = reinterpret_cast<uint16_t*>(rarr + b.cap);  // [cap]
+    uint16_t* list = rsl + b.cap;            // [cap]
+    __shared__ uint32_t wsum[FINISH_THREADS / 64];
     __shared__ uint32_t n1, nm, nbig, nmem;
     const uint32_t tid = threadIdx.x, c = blockIdx.x, part = c / b.nbp, cl = c % b.nbp;
     if (tid == 0) n1 = nm = nbig = nmem = 0;
     uint32_t m = 0;
-    for (uint32_t s0 = 0; s0 < N; s0 += EMIT_SMALL_THREADS) {
+    for (uint32_t s0 = 0; s0 < N; s0 += FINISH_THREADS) {
         const uint32_t sl = s0 + tid;
         uint32_t cnt = 0;
         if (sl < N) {
@@ -362,7 +309,7 @@ __device__ __forceinline__ void small_emit_bucket(const EmitArgs<true>& a, uint3
             slb[sl] = lbase;
         }
         uint32_t total;
-        const uint32_t x = m + block_excl_scan<uint32_t, EMIT_SMALL_THREADS / 64>(cnt, wsum, &total);
+        const uint32_t x = m + block_excl_scan<uint32_t, FINISH_THREADS / 64>(cnt, wsum, &total);
         if (sl < N) spre[sl] = x;
         m += total;
     }
@@ -376,16 +323,15 @@ __device__ __forceinline__ void small_emit_bucket(const EmitArgs<true>& a, uint3
     }
     uint32_t table = 64;  // of the records there are
     while (table < m + m / 4) table *= 2;
-    for (uint32_t i = tid; i < table; i += EMIT_SMALL_THREADS) {
+    for (uint32_t i = tid; i < table; i += FINISH_THREADS) {
         trow[i] = NO_ROW;
         tcnt[i] = 0;
     }
     __syncthreads();
-    for (uint32_t i = tid; i < m; i += EMIT_SMALL_THREADS) {
+    for (uint32_t i = tid; i < m; i += FINISH_THREADS) {
         const uint32_t sl = (uint32_t)find_slot(spre, (int)N, i);
         const uint2 r = p.recs[sstart[sl] + i - spre[sl]];
         const uint32_t gi = slb[sl] + (r.y & ((1u << SMALL_SLOT_BITS) - 1u));
-        const uint32_t rank = p.rank_at[gi];
         uint32_t e = 0;
         if (r.x != NO_ROW) {  // (a sign the table had no room for: nothing to update)
             e = (r.x * 2654435761u >> 12) & (table - 1);
@@ -399,38 +345,38 @@ __device__ __forceinline__ void small_emit_bucket(const EmitArgs<true>& a, uint3
         }
         rrow[i] = r.x;
         rgi[i] = gi;
-        rrs[i] = rank | (sl << 16);
+        rsl[i] = (uint16_t)sl;
         rce[i] = (r.y >> SMALL_SLOT_BITS) | (e << 14);
     }
     __syncthreads();
     const size_t first = (size_t)c * b.cap;
     // signs with one record: numbered and written at once; with several: a number and a stretch of the records for each
-    for (uint32_t i = tid; i < m; i += EMIT_SMALL_THREADS) {
+    for (uint32_t i = tid; i < m; i += FINISH_THREADS) {
         if (rrow[i] == NO_ROW) continue;
         const uint32_t e = rce[i] >> 14, k = tcnt[e];
         if (k == 1) {
             const uint32_t g = atomicAdd(&n1, 1u);
             p.group[first + g] = make_uint2(rrow[i], g | (1u << 16));
-            p.member[first + g] = make_uint4(rgi[i], rrs[i], rce[i] & 0x3FFFu, 0u);
+            p.member[first + g] = make_uint4(rgi[i], (uint32_t)rsl[i] << 16, rce[i] & 0x3FFFu, 0u);
         } else if (rarr[i] == 0) {
             tinfo[e] = atomicAdd(is_big(k, a.big_k) ? &nbig : &nm, 1u) | (atomicAdd(&nmem, k) << 16);
         }
     }
     __syncthreads();
-    for (uint32_t i = tid; i < m; i += EMIT_SMALL_THREADS) {
+    for (uint32_t i = tid; i < m; i += FINISH_THREADS) {
         if (rrow[i] == NO_ROW) continue;
         const uint32_t e = rce[i] >> 14, k = tcnt[e];
         if (k > 1) list[(tinfo[e] >> 16) + rarr[i]] = (uint16_t)i;
     }
     __syncthreads();
-    for (uint32_t i = tid; i < m; i += EMIT_SMALL_THREADS) {
+    for (uint32_t i = tid; i < m; i += FINISH_THREADS) {
         if (rrow[i] == NO_ROW) continue;
         const uint32_t e = rce[i] >> 14, k = tcnt[e];
         if (k == 1) continue;
         const uint32_t at = tinfo[e] >> 16;
         uint32_t place = 0;  // records of the sign in earlier slots
         for (uint32_t j = 0; j < k; j++) place += list[at + j] < i ? 1u : 0u;
-        p.member[first + n1 + at + place] = make_uint4(rgi[i], rrs[i], rce[i] & 0x3FFFu, 0u);
+        p.member[first + n1 + at + place] = make_uint4(rgi[i], (uint32_t)rsl[i] << 16, rce[i] & 0x3FFFu, 0u);
         if (rarr[i] == 0) {
             const uint32_t g = tinfo[e] & 0xFFFFu;
             p.group[first + (is_big(k, a.big_k) ? b.cap - 1 - g : n1 + g)] = make_uint2(rrow[i], (n1 + at) | (k << 16));
@@ -439,13 +385,129 @@ __device__ __forceinline__ void small_emit_bucket(const EmitArgs<true>& a, uint3
     if (tid == 0) p.head[c] = make_uint4(n1, nm, nbig, nmem);
 }
 
+// Mapped ids (rank of the sign's first lookup) and, for the first lookups, the table row into the variable: a run of `per`
+// positions of one slot, a thread per position and part of a row, FINISH_ITEMS of them at most.
+constexpr int FINISH_ITEMS = 2;
+template <int VEC>
+__device__ __forceinline__ void small_finish(const SmallShape& b, const SmallPlan& p, uint32_t block, uint32_t chunks,
+                                             uint32_t per, const Store& s) {
+    constexpr uint32_t WAVES = FINISH_THREADS / 64;
+    __shared__ unsigned long long part_bits[WAVES][SMALL_WORDS];
+    __shared__ unsigned long long bits[SMALL_WORDS];
+    __shared__ uint32_t before[SMALL_WORDS];
+    const uint32_t sl = block / chunks;
+    const uint32_t C = (uint32_t)(s.wdim / VEC);
+    const uint32_t p0 = (block % chunks) * per;
+    const SlotDesc d = p.descs[sl];
+    if (p0 >= d.len) return;
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, todo = min(per, d.len - p0) * C;
+    uint32_t pos[FINISH_ITEMS], c[FINISH_ITEMS], f[FINISH_ITEMS], row[FINISH_ITEMS];
+#pragma unroll
+    for (int j = 0; j < FINISH_ITEMS; j++) {
+        const uint32_t q = j * FINISH_THREADS + tid;
+        pos[j] = p0 + q / C;
+        c[j] = q % C;
+        f[j] = q < todo ? p.first_of[d.lbase + pos[j]] : NO_ROW;
+        row[j] = q < todo ? p.row_at[d.lbase + pos[j]] : NO_ROW;  // (of a first lookup only)
+    }
+    {  // the parts' first lookups: a wavefront takes every WAVES-th part, then one puts them together
+        const uint64_t* w = p.bits + (size_t)sl * b.parts * b.words + lane;
+        uint64_t v[SMALL_PARTS_MAX / WAVES];
+#pragma unroll
+        for (uint32_t k = 0; k < SMALL_PARTS_MAX / WAVES; k++) {
+            const uint32_t q = k * WAVES + wave;
+            v[k] = q < b.parts && lane < b.words ? w[(size_t)q * b.words] : 0ull;
+        }
+        uint64_t all = 0;
+#pragma unroll
+        for (uint32_t k = 0; k < SMALL_PARTS_MAX / WAVES; k++) all |= v[k];
+        part_bits[wave][lane] = all;
+    }
+    float4 v4[FINISH_ITEMS];
+    float v1[FINISH_ITEMS];
+#pragma unroll
+    for (int j = 0; j < FINISH_ITEMS; j++) {
+        // (NO_ROW, the table is full: never address the table with it)
+        if (f[j] != pos[j] || row[j] > s.cap) row[j] = NO_ROW;
+        v4[j] = make_float4(0.f, 0.f, 0.f, 0.f);
+        v1[j] = 0.f;
+        if (row[j] != NO_ROW) {
+            if (VEC == 4)
+                v4[j] = *reinterpret_cast<const float4*>(s.w + (uint64_t)row[j] * s.wstride + c[j] * 4);
+            else
+                v1[j] = s.w[(uint64_t)row[j] * s.wstride + c[j]];
+        }
+    }
+    __syncthreads();
+    if (wave == 0) {
+        unsigned long long v = 0;
+        for (uint32_t q = 0; q < WAVES; q++) v |= part_bits[q][lane];
+        const uint32_t n = (uint32_t)__popcll(v);
+        uint32_t inc = n;
+        for (int x = 1; x < 64; x <<= 1) {
+            const uint32_t y = __shfl_up(inc, x);
+            if ((int)lane >= x) inc += y;
+        }
+        bits[lane] = v;
+        before[lane] = inc - n;
+    }
+    static_assert(SMALL_WORDS == 64, "one wavefront scans the words");
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < FINISH_ITEMS; j++) {
+        if (f[j] == NO_ROW) continue;
+        const uint32_t rank = before[f[j] >> 6] + (uint32_t)__popcll(bits[f[j] >> 6] & ((1ull << (f[j] & 63)) - 1ull));
+        if (c[j] == 0) {
+            d.mapped[pos[j]] = (int64_t)rank;
+            if (f[j] == pos[j]) p.rank_at[d.lbase + pos[j]] = (uint16_t)rank;
+        }
+        if (row[j] == NO_ROW || (int64_t)rank >= d.rows) continue;  // (the host reports a variable that is too small)
+        if (VEC == 4)
+            *reinterpret_cast<float4*>(d.var + (uint64_t)rank * s.wdim + c[j] * 4) = v4[j];
+        else
+            d.var[(uint64_t)rank * s.wdim + c[j]] = v1[j];
+    }
+}
+
+template <int VEC>
+__global__ __launch_bounds__(FINISH_THREADS) void k_small_group_finish(SmallShape b, SmallPlan p, uint32_t chunks,
+                                                                       uint32_t per, Store s) {
+    small_finish<VEC>(b, p, blockIdx.x, chunks, per, s);
+}
+
+// Both by one launch: each is a chain of round trips, with the gap between two launches behind it.
+template <int VEC>
+__global__ __launch_bounds__(FINISH_THREADS) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_small_pull_rest(
+    EmitArgs<true> a, uint32_t chunks, uint32_t per, Store s) {
+    extern __shared__ uint32_t emit_lds[];
+    const uint32_t buckets = a.b.buckets();
+    if (blockIdx.x < buckets)
+        small_emit_bucket(a, emit_lds);
+    else
+        small_finish<VEC>(a.b, a.p, blockIdx.x - buckets, chunks, per, s);
+}
+
 // First launch of a small push on the last pull's plan: the signs are compared with the plan's copy, and with CLICKS the
 // non-zero labels are added to the click sums (sparse_table_ops.cc:283-296; a few thousand lookups do not queue up on
 // any entry).  A mismatch also goes to the host (pinned memory); that the comparison is complete, the last launch tells it.
+// The workgroups behind those, a wavefront per bucket, put the ranks of the records' first lookups into the records, which
+// the updates would otherwise read by way of (the pull, which knows both, works them out side by side).
 template <bool CLICKS>
 __global__ __launch_bounds__(256) void k_small_verify(SmallShape b, SmallPlan p, const SlotDesc* host_descs, uint32_t chunks,
                                                       DevStatus* status, uint32_t* host_mismatch) {
     __shared__ SlotDesc sd;
+    if (blockIdx.x >= b.N * chunks) {
+        const uint32_t c = (blockIdx.x - b.N * chunks) * 4 + threadIdx.x / 64;
+        if (c >= b.buckets()) return;
+        const uint4 head = p.head[c];
+        uint4* mem = p.member + (size_t)c * b.cap;
+        const uint32_t n = min(head.x + head.w, b.cap);
+        for (uint32_t i = threadIdx.x & 63; i < n; i += 64) {
+            const uint4 m = mem[i];
+            mem[i].y = (m.y & 0xFFFF0000u) | p.rank_at[m.x];
+        }
+        return;
+    }
     const int sl = blockIdx.x / chunks;
     const uint32_t p0 = (blockIdx.x % chunks) * SMALL_TILE;
     // what the pull left of these positions is on its way while the descriptor comes in from the host's staging buffer
@@ -878,35 +940,36 @@ __device__ __forceinline__ void apply_group_ahead(const Store& s, const OptDev& 
 // Bytes of dynamic LDS of k_small_apply when its launch includes the workgroups for the signs with many records:
 // per wavefront the staging and the row of apply_big_groups, then its pointer, count, flag and divisor arrays.
 inline size_t small_apply_wave_lds(int D) { return align_up(big_lds_bytes(D), 8) + BIG_CHUNK * (8 + 4); }
+// (a sign of a small batch has as many records as the batch has slots at most)
+inline int small_gbuf_floats(int D, int N) { return std::min(big_gbuf_floats(D), std::min(N, BIG_CHUNK) * (D + 1)); }
 
 __host__ __device__ inline size_t small_apply_slots_lds(int N) { return ((size_t)N * 12 + 7) / 8 * 8; }
 
-// The updates of a small push by one launch, `roles` workgroups per bucket: the signs with one record; with a few, by
-// lane groups, several records at a time; with many (four slots' worth and more), by a wavefront each the way
-// k_apply_big does.  Nothing is reported to the host but that this kernel runs, which tells it that the comparison of
-// the signs, launched before, is complete: on the plan of the last pull every sign has its row, and the host has compared
-// the slots' distinct counts with the rows of the gradient matrices itself.
+// The next number of a counter in LDS for the whole wavefront, all of whose lanes call it.
+__device__ __forceinline__ uint32_t wave_draw(uint32_t* counter) {
+    uint32_t r = 0;
+    if (__lane_id() == 0) r = atomicAdd(counter, 1u);
+    return (uint32_t)__builtin_amdgcn_readfirstlane((int)r);
+}
+
+// The updates of a small push by one launch, a workgroup per bucket (three per bucket, one for each kind of sign, were two
+// to five times as many workgroups as the chip holds at once, most of their lanes without a sign: 26 slots of 4096 lookups,
+// Adam rows of 16, 17.9 us, 15.2 now).  What bounds it is the longest chain of a wavefront.  Its wavefronts take the signs with many records (four
+// slots' worth and more) first, one each, the way k_apply_big does; then 64 / LPG signs at a time: those with a few records,
+// several records of a sign in flight, then those with one.  Nothing is reported to the host but that this kernel runs,
+// which tells it that the comparison of the signs, launched before, is complete: on the plan of the last pull every sign has
+// its row, and the host has compared the slots' distinct counts with the rows of the gradient matrices itself.
 template <int KIND, int LPG, bool ANY>
 __global__ __launch_bounds__(256) void k_small_apply(SmallShape b, SmallPlan p, const float* flat, Store s,
                                                      OptDev o, const DevStatus* __restrict__ status, uint32_t* host_seq,
                                                      uint32_t seq, int dim, int gbuf_floats, uint32_t wave_lds,
                                                      uint32_t wave_arrays) {
     extern __shared__ unsigned long long apply_lds[];  // the slots' gradient matrices and their rows; then the wavefronts' staging
+    __shared__ uint32_t next_round;
     if (blockIdx.x == 0 && threadIdx.x == 0) host_store(host_seq, seq);
-    const uint32_t nb = b.buckets();
-    // (the workgroups whose chains are the longest first)
-    const uint32_t c = blockIdx.x % nb, role = gridDim.x / nb - 1 - blockIdx.x / nb;
-    const int sub = threadIdx.x % LPG;
-    const uint32_t g0 = threadIdx.x / LPG;
+    const uint32_t c = blockIdx.x;
     const size_t first = (size_t)c * b.cap;
-    // the first sign and record of a group of lanes before the bucket's counts are known: one round trip less
     const uint4 head = p.head[c];
-    uint2 gr = make_uint2(NO_ROW, 0);
-    uint4 mem = make_uint4(0, 0, 0, 0);
-    if (role == 0) {
-        gr = p.group[first + min(g0, b.cap - 1)];
-        mem = p.member[first + min(g0, b.cap - 1)];
-    }
     const uint32_t stop = status->mismatch | status->abort;
     const float** grads = reinterpret_cast<const float**>(apply_lds);
     uint32_t* rows = reinterpret_cast<uint32_t*>(grads + (flat ? 0 : b.N));
@@ -915,8 +978,9 @@ __global__ __launch_bounds__(256) void k_small_apply(SmallShape b, SmallPlan p, 
             grads[i] = p.push_descs[i].grads;
             rows[i] = (uint32_t)min(p.push_descs[i].rows, (int64_t)SMALL_SLOT_MAX + 1);
         }
-        __syncthreads();
     }
+    if (threadIdx.x == 0) next_round = 0;
+    __syncthreads();
     // a plan that turned out not to be this batch's: nothing to do (the host analyses the batch itself)
     if (stop) return;
     SmallSrc src;
@@ -925,10 +989,9 @@ __global__ __launch_bounds__(256) void k_small_apply(SmallShape b, SmallPlan p, 
     src.flat = flat;
     src.click_at = p.click_at;
     src.dim = dim;
-    const int lane0 = (int)__lane_id() - sub;
     const float c1 = 1 - o.beta1, c2 = 1 - o.beta2;
-    if (role == 2) {
-        const int wave = (int)(threadIdx.x >> 6), lane = (int)(threadIdx.x & 63);
+    const int wave = (int)(threadIdx.x >> 6), lane = (int)(threadIdx.x & 63), sub = lane % LPG, lane0 = lane - sub;
+    if (head.z) {
         char* base = reinterpret_cast<char*>(apply_lds) + small_apply_slots_lds(flat ? 0 : b.N) + (size_t)wave * wave_lds;
         float* gbuf = reinterpret_cast<float*>(base);
         const float** gptr = reinterpret_cast<const float**>(base + wave_arrays);
@@ -952,31 +1015,36 @@ __global__ __launch_bounds__(256) void k_small_apply(SmallShape b, SmallPlan p, 
                 return gp != nullptr;
             },
             [] {}, [] { wave_sync(); });
-        return;
     }
-    if (role == 1) {
-        for (uint32_t g = g0; g < head.y; g += 256 / LPG) {
-            const uint2 d = p.group[first + head.x + g];
-            if (d.x > s.cap) continue;  // no row number at all: never address the table with it
-            const SmallGroup grp{src, p.member + first + (d.y & 0xFFFFu)};
-            apply_group_ahead<KIND, LPG, ANY, 4>(s, o, grp, d.x, d.y >> 16, sub, lane0, c1, c2);
+    constexpr uint32_t PER = 64 / LPG;
+    const uint32_t rounds_multi = (head.y + PER - 1) / PER, rounds = rounds_multi + (head.x + PER - 1) / PER;
+    // (Nothing leaves the loop's body but through its end: with a `continue` under a condition the compiler makes the lanes
+    // that take it a loop of their own, in which lane 0, that draws the next round, does not run.)
+    uint32_t r = wave_draw(&next_round);
+    while (r < rounds) {
+        if (r < rounds_multi) {
+            const uint32_t g = r * PER + lane / LPG;
+            const uint2 d = g < head.y ? p.group[first + head.x + g] : make_uint2(NO_ROW, 0);
+            if (d.x <= s.cap) {  // (no row number at all: never address the table with it)
+                const SmallGroup grp{src, p.member + first + (d.y & 0xFFFFu)};
+                apply_group_ahead<KIND, LPG, ANY, 4>(s, o, grp, d.x, d.y >> 16, sub, lane0, c1, c2);
+            }
+        } else {
+            const uint32_t g = (r - rounds_multi) * PER + lane / LPG, at = min(g, b.cap - 1);
+            const uint2 d = p.group[first + at];
+            const uint4 mem = p.member[first + at];
+            if (g < head.x && d.x <= s.cap) {
+                const float* gp = src.gradient(mem);
+                if (gp) {
+                    int ck = 0;
+                    if (KIND == OPT_ADAGRAD) ck = src.click(mem);
+                    apply_one_record<KIND, LPG, ANY>(s, o, d.x, gp, (int)mem.z, ck, sub, lane0, c1, c2);
+                }
+                // (a record without a gradient row, too: the caller may push the batch again on this plan)
+                if (KIND == OPT_ADAGRAD && sub == 0) src.click_at[mem.x] = 0;
+            }
         }
-        return;
-    }
-    for (uint32_t g = g0; g < head.x; g += 256 / LPG) {
-        if (g != g0) {
-            gr = p.group[first + g];
-            mem = p.member[first + g];
-        }
-        if (gr.x > s.cap) continue;
-        const float* gp = src.gradient(mem);
-        if (gp) {
-            int ck = 0;
-            if (KIND == OPT_ADAGRAD) ck = src.click(mem);
-            apply_one_record<KIND, LPG, ANY>(s, o, gr.x, gp, (int)mem.z, ck, sub, lane0, c1, c2);
-        }
-        // (a record without a gradient row, too: the caller may push the batch again on this plan)
-        if (KIND == OPT_ADAGRAD && sub == 0) src.click_at[mem.x] = 0;
+        r = wave_draw(&next_round);
     }
 }
 

@@ -70,6 +70,16 @@ constexpr int SMALL_NO_BIG_SLOTS = 12;
 constexpr uint32_t SMALL_BIG_GROUP = 5;
 constexpr uint32_t BIG_GROUP_DEFAULT = 16;
 
+// What a small pull has left to do behind its first launch takes one launch (k_small_pull_rest: 26 slots of 4096 lookups
+// 8.7 us, as two launches 7.0 + 7.2 and the gap), unless the buckets' workgroups want so much dynamic LDS, which all
+// workgroups of a launch are given, that fewer than four would be on a CU.  Up to SMALL_SPLIT_SLOTS slots it stays two
+// launches, the sequence tests/test_gpu_small.py pins at 8 slots: a step of 8 slots of 1024 lookups is as long as the host's
+// way from the pull's first launch to the push, 37 us either way.
+constexpr int SMALL_SPLIT_SLOTS = 8;
+// Parts of rows from which a thread of small_finish takes two: up to here more workgroups are the shorter way.
+constexpr size_t FINISH_FULL = 1 << 17;
+constexpr size_t SMALL_SHARED_LDS = 36 * 1024;
+
 enum { FLOW_NONE = 0, FLOW_PULL = 1, FLOW_PUSH = 2 };
 
 struct HostStatus {
@@ -1145,13 +1155,12 @@ int launch_small_apply_kind(SparseTable* t, RowShare share, const OptDev& o, con
     const Store& s = t->store;
     const SmallShape& b = t->small_shape;
     const bool with_big = t->plan_big_k != 0xFFFFFFFFu && (uint32_t)b.N >= t->plan_big_k;
-    const int roles = with_big ? 3 : b.N > 1 ? 2 : 1;
-    const size_t wave_lds = small_apply_wave_lds(s.D);
+    const int gfloats = small_gbuf_floats(s.D, b.N);
+    const size_t arrays = align_up((size_t)(gfloats + 3 * s.D) * sizeof(float), 8), wave_lds = arrays + BIG_CHUNK * (8 + 4);
     const size_t lds = small_apply_slots_lds(flat ? 0 : b.N) + (with_big ? 4 * wave_lds : 0);
 #define TN_LAUNCH_SMALL_ANY(LPG, ANY)                                                                                  \
-    TN_LAUNCH_LDS((k_small_apply<KIND, LPG, ANY>), dim3(b.buckets() * roles), dim3(256), lds, st, b, p, flat, s, o,    \
-                  (const DevStatus*)t->dplan, host_seq, seq, dim, big_gbuf_floats(s.D), (uint32_t)wave_lds,            \
-                  (uint32_t)align_up(big_lds_bytes(s.D), 8))
+    TN_LAUNCH_LDS((k_small_apply<KIND, LPG, ANY>), dim3(b.buckets()), dim3(256), lds, st, b, p, flat, s, o,            \
+                  (const DevStatus*)t->dplan, host_seq, seq, dim, gfloats, (uint32_t)wave_lds, (uint32_t)arrays)
 #define TN_LAUNCH_SMALL(LPG)                  \
     do {                                      \
         if (share.any)                        \
@@ -1398,17 +1407,27 @@ int small_pull(SparseTable* t, const SmallShape& b, const int64_t* const* values
     const uint32_t seq = ++t->seq_pull, workgroups = (uint32_t)b.N * b.parts, entries = small_entries(b.max_len, b.parts);
     TN_LAUNCH_LDS(k_small_slots, dim3(workgroups), dim3(SMALL_THREADS), small_slots_lds(entries, b.max_len, b.nbp), st, b, p,
                   (const SlotDesc*)descs, entries, s, make_optdev(t), t->seed, t->dplan, t->hwords, seq);
-    const uint32_t per = SMALL_THREADS / (uint32_t)(vec ? wdim / 4 : wdim), chunks = (b.max_len + per - 1) / per;
-    if (vec)
-        TN_LAUNCH((k_small_group_finish<4>), dim3((uint32_t)b.N * chunks), dim3(SMALL_THREADS), st, b, p, chunks, s);
-    else
-        TN_LAUNCH((k_small_group_finish<1>), dim3((uint32_t)b.N * chunks), dim3(SMALL_THREADS), st, b, p, chunks, s);
+    const uint32_t C = (uint32_t)(vec ? wdim / 4 : wdim), items = (size_t)b.L * C > FINISH_FULL ? FINISH_ITEMS : 1;
+    const uint32_t per = items * FINISH_THREADS / C, chunks = (b.max_len + per - 1) / per;
     EmitArgs<true> ea;
     ea.b = b;
     ea.p = p;
     ea.table = small_emit_table(b.cap);
     ea.big_k = t->plan_big_k = b.N <= SMALL_NO_BIG_SLOTS ? 0xFFFFFFFFu : SMALL_BIG_GROUP;
-    TN_LAUNCH_LDS((k_group_emit<true>), dim3(b.buckets()), dim3(EMIT_SMALL_THREADS), small_emit_lds(b.N, b.cap, ea.table), st, ea);
+    const size_t emit_lds = small_emit_lds(b.N, b.cap, ea.table);
+    const uint32_t finish = (uint32_t)b.N * chunks;
+    if (b.N > SMALL_SPLIT_SLOTS && emit_lds <= SMALL_SHARED_LDS) {
+        if (vec)
+            TN_LAUNCH_LDS((k_small_pull_rest<4>), dim3(b.buckets() + finish), dim3(FINISH_THREADS), emit_lds, st, ea, chunks, per, s);
+        else
+            TN_LAUNCH_LDS((k_small_pull_rest<1>), dim3(b.buckets() + finish), dim3(FINISH_THREADS), emit_lds, st, ea, chunks, per, s);
+    } else {
+        if (vec)
+            TN_LAUNCH((k_small_group_finish<4>), dim3(finish), dim3(FINISH_THREADS), st, b, p, chunks, per, s);
+        else
+            TN_LAUNCH((k_small_group_finish<1>), dim3(finish), dim3(FINISH_THREADS), st, b, p, chunks, per, s);
+        TN_LAUNCH_LDS((k_group_emit<true>), dim3(b.buckets()), dim3(FINISH_THREADS), emit_lds, st, ea);
+    }
     TN_HIP(hipGetLastError());
     // the call returns when the first launch has reported: what follows is complete in stream order
     TN_HIP(hipEventRecord(t->tail_ev, st));
@@ -1485,11 +1504,13 @@ int small_push(SparseTable* t, const int64_t* const* values, const float* const*
     t->hpush->st.mismatch = 0;
     t->hpush->st.abort = 0;
     const uint32_t seq = ++t->seq_verify, chunks = (b.max_len + SMALL_TILE - 1) / SMALL_TILE;
+    // (the records of pooled gradients go by their first lookups, not by rank)
+    const uint32_t verify_blocks = (uint32_t)b.N * chunks + (pooled ? 0u : (b.buckets() + 3) / 4);
     if (clicks)
-        TN_LAUNCH((k_small_verify<true>), dim3((uint32_t)b.N * chunks), dim3(256), st, b, p, (const SlotDesc*)descs, chunks,
+        TN_LAUNCH((k_small_verify<true>), dim3(verify_blocks), dim3(256), st, b, p, (const SlotDesc*)descs, chunks,
                   t->dplan, &t->hpush->st.mismatch);
     else
-        TN_LAUNCH((k_small_verify<false>), dim3((uint32_t)b.N * chunks), dim3(256), st, b, p, (const SlotDesc*)descs, chunks,
+        TN_LAUNCH((k_small_verify<false>), dim3(verify_blocks), dim3(256), st, b, p, (const SlotDesc*)descs, chunks,
                   t->dplan, &t->hpush->st.mismatch);
     const bool rows16 = dim % 4 == 0 && t->store.wstride % 4 == 0;
     if (pooled)
