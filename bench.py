@@ -634,13 +634,9 @@ def main():
         comb_bytes = {
             # signs' ids + example ids in, one output row per (slot, example) out, variable rows read once
             "k_combine_fwd": 16 * mean_L + 4 * dim * (cfg["batch"] * n_slots + mean_U),
-            # example ids in, value out
-            "k_lookup_keys": 16 * mean_L,
-            # distinct index in (twice: count, place), position out at its place in the sign's segment, segment bounds out
-            "k_place_lookups": 12 * mean_L + 4 * mean_U,
-            # position, distinct index and value in, value out at its rank in the segment, segment bounds in
-            "k_order_segments": 24 * mean_L + 4 * mean_U,
-            # sorted values in, pooled rows read once, one reduced row per distinct sign out
+            # example id and distinct index in, item out
+            "k_lookup_keys": 20 * mean_L,
+            # items in, pooled rows read once, one reduced row per distinct sign out
             "k_reduce_pooled": 8 * mean_L + 4 * dim * (cfg["batch"] * n_slots + mean_U),
         }
         out["combiner_step"] = {
@@ -648,7 +644,7 @@ def main():
             "ms_per_step": cms,
             "keys_per_s": mean_L / (cms * 1e-3),
             "kernels_ms_per_step": {k: round(v, 4) for k, v in cprof.items()
-                                    if k.startswith(("k_combine", "k_lookup_keys", "k_place", "k_order", "k_reduce"))},
+                                    if k.startswith(("k_combine", "k_lookup_keys", "k_reduce"))},
             "kernels_frac_of_hbm_peak": {k: round(comb_bytes[k.split("<")[0]] / (v * 1e-3) / HBM_PEAK, 4)
                                          for k, v in cprof.items() if k.split("<")[0] in comb_bytes},
         }

@@ -9,22 +9,20 @@
 //   backward  g[u, :]   = sum over the lookups i of distinct sign u of dout[b(i), :] * (1 / d(n_b(i)))
 //
 // Both are deterministic.  The forward sums run in occurrence order, and so do the backward
-// sums of the signs with few lookups; a sign with ORDER_MID (64) lookups or more in a slot is
-// summed by a workgroup, whose thread groups take every so many of its lookups and whose
-// partial sums are added in group order (k_reduce_pooled).  (On the path of few launches a sign
-// with more than POOL_PIECE (32) lookups is summed in pieces of as many, k_small_pool.)  The
-// backward pass gets the lookups of every distinct sign side by side, in position order, from a
-// counting sort per slot followed by an ordering of every sign's lookups by position
-// (k_place_lookups, k_order_segments).
+// sums of the signs with few lookups; a sign with many is summed in pieces of POOL_PIECE (16), whose
+// sums are added in order, one with lookups in several rounds of a workgroup round by round
+// (k_reduce_pooled; on the path of few launches k_small_pool).
 #ifndef TN_COMBINE_KERNELS_H_
 #define TN_COMBINE_KERNELS_H_
 
-#include "sparse_kernels.h"
+#include "pool_items.h"
+
+#include <algorithm>
 
 namespace tn {
 
 enum { COMBINE_SUM = 0, COMBINE_MEAN = 1, COMBINE_SQRTN = 2 };
-constexpr int COMBINE_WINDOW = 8;  // lookups of an example / of a distinct sign read ahead with independent loads
+constexpr int COMBINE_WINDOW = 8;  // lookups of an example read ahead with independent loads
 
 // In these kernels a SlotDesc carries: values = mapped ids (forward) / signs (backward),
 // mapped = example index of every lookup, grads = rows to read (variable / pooled gradient),
@@ -145,448 +143,323 @@ __global__ void k_report(DevStatus* status, uint64_t* host_word, uint32_t seq) {
     __hip_atomic_store(reinterpret_cast<unsigned long long*>(host_word), w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-// Backward, step 1: the value of every lookup: its example in the high word, the number of
-// lookups of that example in the low word -- all the reduction needs to know about the lookup, so
-// that it reads them in the order of the distinct signs instead of chasing positions.
-//
-// 16 bytes move per lookup; what bounded it were chains of loads (a thread found the slot of a lookup by bisection, then
-// its descriptor, then its id, and the first lookup of an example walked to its last one and wrote all their values).
-// A wavefront now takes KEY_ITEMS runs of 64 lookups, their loads in flight together, and reads the extents of its
-// examples off a ballot of the places where the id changes; an example that goes on beyond the run is followed there by
-// the whole wavefront.  4.9 M lookups: 60 -> 35 us.
-constexpr int KEY_ITEMS = 4;
-constexpr uint32_t KEY_TILE = 256 * KEY_ITEMS;
+constexpr uint32_t KEY_ITEMS = 8;
+constexpr uint32_t KEY_WAVES = 4;
+constexpr uint32_t POOL_TILE = 64 * KEY_WAVES * KEY_ITEMS;
+constexpr uint32_t POOL_PARTS_LOG2 = 11;
+constexpr uint32_t POOL_FILL = 1600;  // (49 k lookups a slot: 32 parts 176 us, 64 parts 255; of 4 k: 4 parts 42, 8 parts 56)
+constexpr uint32_t POOL_SPREAD = 64;
+constexpr uint32_t POOL_SPREAD_LOG2 = 3;  // 2^3 parts and more: a slot of 12800 lookups (POOL_FILL)
 
-__global__ __launch_bounds__(256) void k_lookup_keys(const SlotDesc* __restrict__ descs,
-                                                     const uint32_t* __restrict__ lbase, int N, uint32_t L,
-                                                     int64_t batch, uint64_t* __restrict__ vals, DevStatus* status,
-                                                     uint32_t* long_count) {
-    __shared__ uint32_t lb[MAX_SLOTS + 1];
-    load_lbase(lb, lbase, N);
-    // [1], [2]: entries of the lists of k_place_lookups
-    if (blockIdx.x == 0 && threadIdx.x < 3) long_count[threadIdx.x] = 0;
-    const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const uint32_t ntiles = (L + KEY_TILE - 1) / KEY_TILE;
-    for (uint32_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-        const uint32_t g0 = tile * KEY_TILE, g1 = min(L, g0 + KEY_TILE) - 1;
-        const int s0 = find_slot(lb, N, g0);
-        const bool one_slot = g1 < lb[s0 + 1];  // the usual case: the tile lies inside one slot
-        int sl[KEY_ITEMS];
-        int64_t b[KEY_ITEMS], prev[KEY_ITEMS];
-#pragma unroll
-        for (int j = 0; j < KEY_ITEMS; j++) {
-            const uint32_t gi = g0 + (wave * KEY_ITEMS + j) * 64 + lane;
-            sl[j] = s0;
-            b[j] = prev[j] = -1;
-            if (gi <= g1) {
-                if (!one_slot) sl[j] = find_slot(lb, N, gi);
-                const int64_t* ex = example_of(descs[sl[j]]);
-                const uint32_t i = gi - lb[sl[j]];
-                b[j] = ex[i];
-                if (i > 0) prev[j] = ex[i - 1];
-            }
-        }
-#pragma unroll
-        for (int j = 0; j < KEY_ITEMS; j++) {
-            const uint32_t base = g0 + (wave * KEY_ITEMS + j) * 64, gi = base + lane;
-            const bool active = gi <= g1;
-            if (active && (b[j] < 0 || b[j] >= batch || prev[j] > b[j])) {
-                atomicOr(&status->err, DEV_ERR_GRAD_ROWS);
-                status->abort = 1;  // nothing downstream may run
-            }
-            // where an example starts (the first lookup of a slot does: prev is -1 there; and what lies behind the last one)
-            const unsigned long long heads = __ballot(!active || b[j] != prev[j]);
-            uint32_t back = 0, ahead = 0;  // lookups of the first / last example of the run before / behind it
-            if (!(heads & 1ull)) {
-                const int64_t x = __shfl(b[j], 0);
-                const int s = __shfl(sl[j], 0);
-                const int64_t* ex = example_of(descs[s]);
-                for (uint32_t i = base - lb[s];; i -= 64) {  // lookups [0, i) of the slot are left
-                    const unsigned long long other = __ballot(lane >= i || ex[i - 1 - lane] != x);
-                    if (other) {
-                        back += (uint32_t)__ffsll((long long)other) - 1;
-                        break;
-                    }
-                    back += 64;
-                }
-            }
-            if (base + 63 <= g1) {
-                const int64_t x = __shfl(b[j], 63);
-                const int s = __shfl(sl[j], 63);
-                const int64_t* ex = example_of(descs[s]);
-                const uint32_t len = lb[s + 1] - lb[s];
-                for (uint32_t i = base + 64 - lb[s];; i += 64) {
-                    const unsigned long long other = __ballot(i + lane >= len || ex[i + lane] != x);
-                    if (other) {
-                        ahead += (uint32_t)__ffsll((long long)other) - 1;
-                        break;
-                    }
-                    ahead += 64;
-                }
-            }
-            if (active) {
-                const unsigned long long below = heads & (~0ull >> (63 - lane)), above = heads & ~(~0ull >> (63 - lane));
-                const uint32_t to_start = below ? lane - (63 - (uint32_t)__clzll((long long)below)) : lane + back;
-                const uint32_t to_end = above ? (uint32_t)__ffsll((long long)above) - 1 - lane : 64 - lane + ahead;
-                vals[gi] = ((uint64_t)b[j] << 32) | (uint64_t)(to_start + to_end);
-            }
-        }
+// How a slot's lookups are shared out to the backward pass's workgroups: in tiles of POOL_TILE for step 1, for step 2 in
+// 2^lp parts of POOL_FILL lookups at most on average.  The distinct indices of the slot ascend with the signs' first occurrences, so
+// that the frequent signs come early.  The lookups of the first `spread` indices of a slot with many parts are dealt to these
+// run by run (64 lookups), and every part leaves a share of those signs' sums (k_reduce_pooled_shares adds them up): a sign
+// with 8 % of a slot's lookups would be three rounds of one part, and the last workgroup's.  The other indices are
+// dealt modulo 2^lp.  Tiles and parts of a call are numbered through the slots so that a slot's
+// first is known from the lookups before it; some numbers are nobody's.
+struct PoolShare {
+    uint32_t lp_max;  // of the longest slot
+    static __host__ __device__ uint32_t parts_log2(uint32_t len) {
+        uint32_t lp = 0;
+        while (lp < POOL_PARTS_LOG2 && (len >> lp) > POOL_FILL) lp++;
+        return lp;
     }
-}
+    static __host__ __device__ uint32_t spread(uint32_t lp) { return lp >= POOL_SPREAD_LOG2 ? POOL_SPREAD : 0u; }
+    static __host__ __device__ uint32_t first_tile(uint32_t slot, uint32_t lookups_before) {
+        return lookups_before / POOL_TILE + slot;
+    }
+    // (2^lp is one, or less than two per POOL_FILL lookups)
+    static __host__ __device__ uint32_t first_part(uint32_t slot, uint32_t lookups_before) {
+        return (uint32_t)(2ull * lookups_before / POOL_FILL) + slot;
+    }
+};
 
-// Step 2: the values of the lookups of every distinct index side by side, in position order:
-// svals[seg_off[u] .. seg_off[u + 1]).
-//   k_place_lookups  a few workgroups per slot (the distinct indices of a slot's lookups fill a window of their
-//                    own, ascending with the slots): counts the lookups of every index in an LDS array, scans
-//                    the counts into seg_off, and puts the position of every lookup into its index's segment -- in
-//                    the order the atomics arrive; indices with ORDER_MID lookups or more are listed for the kernels
-//                    below
-//   rank_short       a lookup of a short segment finds its place by counting the positions of its segment below its own
-//   rank_mid         a sorting network in LDS, one workgroup per segment of ORDER_MID .. ORDER_HUGE - 1 lookups
-//   order_huge       the few longer segments: a bitmap of their positions in LDS, one workgroup each
-//                    (the three are workgroups of one launch, k_order_segments)
-// A slot with more distinct signs than the LDS array holds (lds_cap) keeps its counters in `gcur`.
-constexpr int PLACE_THREADS = 1024;
-constexpr int PLACE_ITEMS = 8;
-constexpr uint32_t ORDER_MID = 64;
-constexpr uint32_t ORDER_HUGE = 1024;
-
-// `parts` workgroups per slot: each of them streams all lookups of the slot (they come out of L2 after the first)
-// and takes those whose distinct index lies in its share of the slot's window of distinct indices.  The lookups of the
-// indices below its share, which it counts on the way, come before its own.
+// Backward, step 1.  A tile of POOL_TILE lookups of a slot leaves an item for every lookup -- example, sign, lookups of the
+// example --, the items of a part side by side in the order of their positions, and where the parts start among them.
 //
-// What bounds it is the chain of each of its few workgroups (two passes over the slot's lookups with an LDS atomic each, the
-// scan between them): the wavefronts wait 85 % of their cycles while 79 MB are read and 49 written (39 and 28 would do), 1.0
-// TB/s.  Only the position is stored, 4 bytes per lookup, and not the index and the value with it (12 bytes): a die has
-// the windows of a dozen slots in its L2 at a time (2.5 MB at 49 k lookups a slot; 7.5 MB with the value, more than its
-// L2), and lines that are written out half filled are read and written again.
-// 4.9 M lookups in 100 slots: 168 us before, 135 with one workgroup per slot and 125 with two.
-__global__ __launch_bounds__(PLACE_THREADS) void k_place_lookups(
-    const uint32_t* __restrict__ lbase, const uint32_t* __restrict__ ubase, int N, uint32_t L,
-    const uint32_t* __restrict__ u_of_gi, uint32_t* __restrict__ tpos, uint32_t* __restrict__ seg_off,
-    uint32_t* __restrict__ gcur, uint32_t lds_cap, uint32_t* __restrict__ mid_list, uint32_t* __restrict__ huge_list,
-    uint32_t* counts, const DevStatus* status, uint32_t parts) {
-    extern __shared__ uint32_t lcur[];
-    __shared__ uint32_t red[PLACE_THREADS / 64];
-    __shared__ uint32_t carry_sh;
-    if (status->abort) return;
-    const int sl = blockIdx.x / parts;
-    const uint32_t part = blockIdx.x % parts;
-    const uint32_t l0 = lbase[sl], len = lbase[sl + 1] - l0;
-    const uint32_t ub = ubase[sl], us = ubase[sl + 1] - ub;
-    if (sl == N - 1 && part == 0 && threadIdx.x == 0) seg_off[ubase[N]] = L;
-    if (len == 0) return;
-    // my share of the slot's distinct indices (relative to ub)
-    const uint32_t r0 = (uint32_t)((uint64_t)us * part / parts), r1 = (uint32_t)((uint64_t)us * (part + 1) / parts);
-    const uint32_t mine = r1 - r0;
-    if (mine == 0) return;
-    uint32_t* const cur = mine <= lds_cap ? lcur : gcur + ub + r0;
-    const uint32_t* const keys = u_of_gi + l0;
-    for (uint32_t i = threadIdx.x; i < mine; i += PLACE_THREADS) cur[i] = 0;
+// 20 bytes move per lookup (4.9 M: 2.1 TB/s).  A wavefront takes KEY_ITEMS runs of 64 lookups, their loads in flight together, and reads the
+// extents of its examples off a ballot of the places where the id changes; an example that goes on beyond the run is
+// followed there by the whole wavefront.  Places in a part come from ballots over the bits of the part's number (as in
+// k_table_part): no atomics whose order of arrival would show.
+// An item: x the example, y bits 0-10 its lookups (POOL_COUNT_MANY: as many or more), 11 the sign's first lookup, 12-31 the
+// key: of the first `spread` distinct indices these themselves, of the others spread + (index - spread) / 2^lp.
+constexpr uint32_t POOL_COUNT_MANY = 0x7FF;
+constexpr uint32_t POOL_FIRST = 0x800;
+constexpr uint32_t POOL_KEY_SHIFT = 12;
+
+inline size_t pool_tile_lds(uint32_t lp) { return ((size_t)KEY_WAVES << lp) * sizeof(uint32_t); }
+
+__global__ __launch_bounds__(256) void k_lookup_keys(const SlotDesc* __restrict__ descs, const uint32_t* __restrict__ lbase,
+                                                     const uint32_t* __restrict__ ubase, uint32_t N,
+                                                     const uint32_t* __restrict__ u_of_gi, int64_t batch,
+                                                     uint2* __restrict__ pool, uint16_t* __restrict__ poff, PoolShare share,
+                                                     DevStatus* status) {
+    extern __shared__ uint32_t cnt[];  // [2^lp][KEY_WAVES]
+    __shared__ uint32_t wsum[KEY_WAVES];
+    __shared__ uint32_t slot;
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    if (tid == 0) slot = N;
     __syncthreads();
-    // (eight lookups per thread at a time, their loads in flight together)
-    uint32_t below = 0;  // lookups of the indices before my share
-    for (uint32_t i0 = threadIdx.x; i0 < len; i0 += PLACE_THREADS * PLACE_ITEMS) {
-        uint32_t k[PLACE_ITEMS];
-#pragma unroll
-        for (int j = 0; j < PLACE_ITEMS; j++) {
-            const uint32_t i = i0 + j * PLACE_THREADS;
-            k[j] = i < len ? (keys[i] & ~FIRST_BIT) - ub : 0xFFFFFFFFu;
-        }
-#pragma unroll
-        for (int j = 0; j < PLACE_ITEMS; j++) {
-            if (k[j] < r0)
-                below++;
-            else if (k[j] < r1)
-                atomicAdd(&cur[k[j] - r0], 1u);
-        }
-    }
-    {
-        uint32_t total;
-        block_excl_scan<uint32_t, PLACE_THREADS / 64>(below, red, &total);
-        if (threadIdx.x == 0) carry_sh = l0 + total;  // the lookups of the slots before, and of the shares before, come first
+    for (uint32_t s = tid; s < N; s += 256) {
+        const uint32_t a = lbase[s], b = lbase[s + 1], t = blockIdx.x - share.first_tile(s, a);  // (wraps before the slot)
+        if (t < (b - a + POOL_TILE - 1) / POOL_TILE) slot = s;
     }
     __syncthreads();
-    for (uint32_t i0 = 0; i0 < mine; i0 += PLACE_THREADS) {
-        const uint32_t i = i0 + threadIdx.x;
-        const uint32_t cnt = i < mine ? ld_relaxed(cur + i) : 0u;  // (counted by atomics: not through the L1 cache)
-        uint32_t total;
-        const uint32_t at = carry_sh + block_excl_scan<uint32_t, PLACE_THREADS / 64>(cnt, red, &total);
-        if (i < mine) {
-            cur[i] = at;
-            seg_off[ub + r0 + i] = at;
-            if (cnt >= ORDER_HUGE)
-                huge_list[atomicAdd(&counts[2], 1u)] = ub + r0 + i;
-            else if (cnt >= ORDER_MID)
-                mid_list[atomicAdd(&counts[1], 1u)] = ub + r0 + i;
-        }
-        __syncthreads();
-        if (threadIdx.x == 0) carry_sh += total;
-        __syncthreads();
-    }
-    for (uint32_t i0 = threadIdx.x; i0 < len; i0 += PLACE_THREADS * PLACE_ITEMS) {
-        uint32_t k[PLACE_ITEMS];
+    if (slot == N) return;
+    const uint32_t sl = slot, l0 = lbase[sl], len = lbase[sl + 1] - l0;
+    const uint32_t t0 = (blockIdx.x - share.first_tile(sl, l0)) * POOL_TILE, lp = share.parts_log2(len);
+    const uint32_t ub = ubase[sl], parts = 1u << lp, spread = share.spread(lp);
+    const int64_t* __restrict__ ex = example_of(descs[sl]);
+    int64_t b[KEY_ITEMS], prev[KEY_ITEMS];
+    uint32_t u[KEY_ITEMS];
 #pragma unroll
-        for (int j = 0; j < PLACE_ITEMS; j++) {
-            const uint32_t i = i0 + j * PLACE_THREADS;
-            k[j] = i < len ? (keys[i] & ~FIRST_BIT) - ub : 0xFFFFFFFFu;
+    for (uint32_t j = 0; j < KEY_ITEMS; j++) {
+        const uint32_t i = t0 + (wave * KEY_ITEMS + j) * 64 + lane;
+        b[j] = prev[j] = -1;
+        u[j] = 0;
+        if (i < len) {
+            b[j] = ex[i];
+            if (i > 0) prev[j] = ex[i - 1];
+            u[j] = u_of_gi[l0 + i];
         }
+    }
+    for (uint32_t i = tid; i < parts * KEY_WAVES; i += 256) cnt[i] = 0;
+    __syncthreads();
+    uint32_t count[KEY_ITEMS], at[KEY_ITEMS];
+    bool bad = false;
 #pragma unroll
-        for (int j = 0; j < PLACE_ITEMS; j++)
-            if (k[j] >= r0 && k[j] < r1) tpos[atomicAdd(&cur[k[j] - r0], 1u)] = l0 + i0 + j * PLACE_THREADS;
-    }
-}
-
-// The lookups in the order of their segments: the runs of a die (DieRuns) keep to one slot, whose distinct indices and
-// values, read by position, are then more often in its L2.  4.9 M lookups: 78 -> 62 us.  Bound by the reads by
-// position: with the longer segments beside it 340 MB come from memory where 87 would do (56 % of the L2's requests hit),
-// 4.4 TB/s, about what random granules reach.
-constexpr uint32_t RANK_RUN = 128;
-
-__device__ __forceinline__ void rank_short(uint32_t L, const uint32_t* __restrict__ u_of_gi,
-                                           const uint64_t* __restrict__ vals, const uint32_t* __restrict__ tpos,
-                                           const uint32_t* __restrict__ seg_off, uint64_t* __restrict__ svals, uint32_t block,
-                                           uint32_t blocks) {
-    for (DieRuns r((L + 255) / 256, RANK_RUN, block, blocks); r.more(); r.next()) {
-        const uint32_t t = r.item() * 256 + threadIdx.x;
-        if (t >= L) continue;
-        const uint32_t gi = tpos[t];
-        const uint32_t u = u_of_gi[gi] & ~FIRST_BIT;
-        const uint64_t v = vals[gi];
-        const uint32_t lo = seg_off[u], hi = seg_off[u + 1];
-        if (hi - lo >= ORDER_MID) continue;
-        uint32_t rank = 0;
-        for (uint32_t j = lo; j < hi; j++) rank += tpos[j] < gi ? 1u : 0u;
-        svals[lo + rank] = v;
-    }
-}
-
-// seg: ORDER_HUGE words of LDS
-__device__ __forceinline__ void rank_mid(const uint32_t* __restrict__ mid_list, uint32_t n_mid,
-                                         const uint32_t* __restrict__ seg_off, const uint64_t* __restrict__ vals,
-                                         const uint32_t* __restrict__ tpos, uint64_t* __restrict__ svals, uint32_t* seg,
-                                         uint32_t block, uint32_t blocks) {
-    for (uint32_t k = block; k < n_mid; k += blocks) {
-        const uint32_t u = mid_list[k];
-        const uint32_t lo = seg_off[u], n = seg_off[u + 1] - lo;  // ORDER_MID <= n < ORDER_HUGE
-        uint32_t p2 = ORDER_MID;
-        while (p2 < n) p2 <<= 1;
-        // bitonic sorting network over the segment padded with the largest value to a power of two
-        for (uint32_t i = threadIdx.x; i < p2; i += 256) seg[i] = i < n ? tpos[lo + i] : 0xFFFFFFFFu;
-        __syncthreads();
-        for (uint32_t size = 2; size <= p2; size <<= 1) {
-            for (uint32_t stride = size >> 1; stride > 0; stride >>= 1) {
-                for (uint32_t t = threadIdx.x; t < p2 / 2; t += 256) {
-                    const uint32_t a = 2 * t - (t & (stride - 1));  // lower element of the t-th pair
-                    const uint32_t b = a + stride;
-                    const bool up = (a & size) == 0;
-                    const uint32_t x = seg[a], y = seg[b];
-                    if ((x > y) == up) {
-                        seg[a] = y;
-                        seg[b] = x;
-                    }
+    for (uint32_t j = 0; j < KEY_ITEMS; j++) {
+        const uint32_t base = t0 + (wave * KEY_ITEMS + j) * 64, i = base + lane;
+        const bool active = i < len;
+        bad |= active && (b[j] < 0 || b[j] >= batch || prev[j] > b[j]);
+        // where an example starts (the first lookup of a slot does: prev is -1 there; and what lies behind the last one)
+        const unsigned long long heads = __ballot(!active || b[j] != prev[j]);
+        uint32_t back = 0, ahead = 0;  // lookups of the first / last example of the run before / behind it
+        if (!(heads & 1ull)) {
+            const int64_t x = __shfl(b[j], 0);
+            for (uint32_t e = base;; e -= 64) {  // lookups [0, e) of the slot are left
+                const unsigned long long other = __ballot(lane >= e || ex[e - 1 - lane] != x);
+                if (other) {
+                    back += (uint32_t)__ffsll((long long)other) - 1;
+                    break;
                 }
+                back += 64;
+            }
+        }
+        if (base + 64 < len) {
+            const int64_t x = __shfl(b[j], 63);
+            for (uint32_t e = base + 64;; e += 64) {
+                const unsigned long long other = __ballot(e + lane >= len || ex[e + lane] != x);
+                if (other) {
+                    ahead += (uint32_t)__ffsll((long long)other) - 1;
+                    break;
+                }
+                ahead += 64;
+            }
+        }
+        const unsigned long long below = heads & (~0ull >> (63 - lane)), above = heads & ~(~0ull >> (63 - lane));
+        const uint32_t to_start = below ? lane - (63 - (uint32_t)__clzll((long long)below)) : lane + back;
+        const uint32_t to_end = above ? (uint32_t)__ffsll((long long)above) - 1 - lane : 64 - lane + ahead;
+        count[j] = min(to_start + to_end, POOL_COUNT_MANY);
+        // its place among the tile's lookups of its part: behind those of earlier runs and lanes
+        const uint32_t index = (u[j] & ~FIRST_BIT) - ub;
+        const uint32_t part = (index < spread ? i >> 6 : index - spread) & (parts - 1u), k = part * KEY_WAVES + wave;
+        unsigned long long same = __ballot(active);
+        for (uint32_t q = 0; q < lp; q++) {
+            const unsigned long long m = __ballot((part >> q) & 1u);
+            same &= ((part >> q) & 1u) ? m : ~m;
+        }
+        at[j] = 0;
+        if (active) at[j] = cnt[k] + (uint32_t)__popcll(same & ((1ull << lane) - 1ull));
+        wave_sync();
+        if (active && (uint32_t)__ffsll((long long)same) - 1 == lane) cnt[k] += (uint32_t)__popcll(same);
+        wave_sync();
+    }
+    if (bad) {
+        atomicOr(&status->err, DEV_ERR_GRAD_ROWS);
+        status->abort = 1;  // nothing downstream may run
+    }
+    __syncthreads();
+    const uint32_t total = parts * KEY_WAVES, each = (total + 255) / 256;
+    uint32_t sum = 0;
+    for (uint32_t q = 0; q < each; q++) sum += tid * each + q < total ? cnt[tid * each + q] : 0u;
+    uint32_t x = block_excl_scan_256<uint32_t>(sum, wsum, nullptr);
+    uint16_t* off = poff + (size_t)blockIdx.x * ((1u << share.lp_max) + 1);
+    for (uint32_t q = 0; q < each; q++) {
+        const uint32_t k = tid * each + q;
+        if (k >= total) break;
+        const uint32_t c = cnt[k];
+        cnt[k] = x;
+        if (k % KEY_WAVES == 0) off[k / KEY_WAVES] = (uint16_t)x;
+        x += c;
+    }
+    if (tid == 0) off[parts] = (uint16_t)min(POOL_TILE, len - t0);
+    __syncthreads();
+#pragma unroll
+    for (uint32_t j = 0; j < KEY_ITEMS; j++) {
+        const uint32_t i = t0 + (wave * KEY_ITEMS + j) * 64 + lane, index = (u[j] & ~FIRST_BIT) - ub;
+        if (i >= len) continue;
+        const uint32_t part = (index < spread ? i >> 6 : index - spread) & (parts - 1u);
+        const uint32_t key = index < spread ? index : spread + ((index - spread) >> lp);
+        pool[l0 + t0 + cnt[part * KEY_WAVES + wave] + at[j]] =
+            make_uint2((uint32_t)b[j], count[j] | (u[j] & FIRST_BIT ? POOL_FIRST : 0u) | (key << POOL_KEY_SHIFT));
+    }
+}
+
+// The lookups of example x in a slot's sorted ids.
+__device__ __forceinline__ uint32_t lookups_of(const int64_t* __restrict__ ex, uint32_t n, int64_t x) {
+    uint32_t bound[2];
+    for (int k = 0; k < 2; k++) {  // the first id >= x, then > x
+        uint32_t lo = 0, len = n;
+        while (len > 0) {
+            const uint32_t half = len / 2;
+            if (ex[lo + half] < x + k) {
+                lo += half + 1;
+                len -= half + 1;
+            } else {
+                len = half;
+            }
+        }
+        bound[k] = lo;
+    }
+    return bound[1] - bound[0];
+}
+
+// Step 2: the gradient of every distinct sign, a workgroup per part of a slot: the part's items, tile after tile,
+// POOL_ITEMS_MAX at a time, sorted and summed in LDS (pool_items).  What a further round has of a sign is added to what the
+// round before left; the round that meets a sign's first lookup writes its row.  The sums of the signs that are spread over
+// the parts go to the part's own rows of `shares`, `has` tells which there are.  The order of all additions is fixed.
+//
+// What bounds it is a workgroup's chain (slot, tiles, items; sort; rows; shares: 20 us, 27 with the chip full), so it wants
+// three workgroups on a CU.  4.9 M lookups in 100 slots, rows of 16: 175 us, with k_lookup_keys (46) and the shares (6) 227,
+// where a counting sort of the lookups through memory, an ordering pass and a reduction by sign took 390; 860 k in 211 slots:
+// 58 for 103.
+static_assert((1u << POOL_SPREAD_LOG2) % 8 == 0 && POOL_SPREAD == 64, "k_reduce_pooled_shares");
+template <int LPG, bool ANY>
+__global__ __launch_bounds__(POOL_THREADS) __attribute__((amdgpu_waves_per_eu(6, 6))) void k_reduce_pooled(const SlotDesc* __restrict__ descs,
+                                                                const uint32_t* __restrict__ lbase,
+                                                                const uint32_t* __restrict__ ubase, uint32_t N,
+                                                                const uint2* __restrict__ pool,
+                                                                const uint16_t* __restrict__ poff, int dim, int D, int combiner,
+                                                                const DevStatus* status, float* __restrict__ flat,
+                                                                PoolShare share, float* __restrict__ shares,
+                                                                uint64_t* __restrict__ has) {
+    __shared__ PoolLds lds;
+    __shared__ uint32_t slot;
+    __shared__ unsigned long long have, had;  // spread signs with a sum so far, before the round
+    // the workgroups of a slot, which read the same rows, on one die (DieShare, an item per workgroup)
+    const uint32_t item = blockIdx.x % XCDS * (gridDim.x / XCDS) + blockIdx.x / XCDS;  // (the grid is a multiple of XCDS)
+    if (status->abort | status->mismatch) return;
+    const uint32_t tid = threadIdx.x;
+    if (tid == 0) {
+        slot = N;
+        have = had = 0;
+    }
+    __syncthreads();
+    for (uint32_t s = tid; s < N; s += POOL_THREADS) {
+        const uint32_t a = lbase[s], b = lbase[s + 1], q = item - share.first_part(s, a);  // (wraps before the slot)
+        if (b > a && q < (1u << share.parts_log2(b - a))) slot = s;
+    }
+    __syncthreads();
+    if (slot == N) return;
+    const uint32_t sl = slot, l0 = lbase[sl], len = lbase[sl + 1] - l0, ub = ubase[sl], us = ubase[sl + 1] - ub;
+    const uint32_t lp = share.parts_log2(len), part = item - share.first_part(sl, l0), tile0 = share.first_tile(sl, l0);
+    const uint32_t spread = share.spread(lp);
+    if (!spread && part >= us) return;
+    const uint32_t top = us > spread ? spread + ((us - 1 - spread) >> lp) : us - 1, bits = top ? 32 - (uint32_t)__clz((int)top) : 0u;
+    const float* pooled = descs[sl].grads;
+    const int64_t* ex = example_of(descs[sl]);
+    const uint32_t mine = (len + POOL_TILE - 1) / POOL_TILE;
+    uint32_t* const before = lds.list;                   // [POOL_THREADS + 1]: items of my part in the tiles before
+    uint32_t* const start = before + POOL_THREADS + 1;   // [POOL_THREADS]: where they are in a tile
+    for (uint32_t g0 = 0; g0 < mine; g0 += POOL_THREADS) {  // tiles, as many at a time as there are threads
+        uint32_t total = 1;
+        for (uint32_t done = 0; done < total; done += POOL_ITEMS_MAX) {
+            {  // (again in a further round: the sums of the one before took the list's place)
+                uint32_t c = 0, lo = 0;
+                if (g0 + tid < mine) {
+                    const uint16_t* off = poff + (size_t)(tile0 + g0 + tid) * ((1u << share.lp_max) + 1) + part;
+                    lo = off[0];
+                    c = off[1] - lo;
+                }
+                const uint32_t x = block_excl_scan<uint32_t, POOL_WAVES>(c, lds.wsum, &total);
+                before[tid] = x;
+                start[tid] = (g0 + tid) * POOL_TILE + lo;
+                if (tid == 0) before[POOL_THREADS] = total;
+            }
+            __syncthreads();
+            const uint32_t n = min(POOL_ITEMS_MAX, total - done);  // (total < done: a part without items here, no round)
+#pragma unroll
+            for (uint32_t j = 0; j < POOL_ITEMS; j++) {
+                const uint32_t i = j * POOL_THREADS + tid;
+                if (i < n && done < total) {
+                    const uint32_t t = (uint32_t)find_slot(before, (int)min(mine - g0, (uint32_t)POOL_THREADS), done + i);
+                    const uint2 v = pool[l0 + start[t] + (done + i - before[t])];
+                    uint32_t count = v.y & POOL_COUNT_MANY;
+                    if (combiner != COMBINE_SUM && count == POOL_COUNT_MANY) count = lookups_of(ex, len, (int64_t)v.x);
+                    const float scale = pool_scale((float)count, combiner);
+                    lds.key[i] = v.y >> POOL_KEY_SHIFT;
+                    lds.example[i] = v.x;
+                    lds.scale[i] = v.y & POOL_FIRST ? scale : -scale;
+                }
+            }
+            if (done < total)
+                pool_items<LPG, ANY>(lds, n, bits, pooled, dim, D, [&](uint32_t key, bool first, bool& add) {
+                    if (key < spread) {
+                        add = ((had >> key) & 1ull) != 0;
+                        atomicOr(&have, 1ull << key);
+                        return shares + ((uint64_t)item * POOL_SPREAD + key) * dim;
+                    }
+                    add = !first;
+                    return flat + (uint64_t)(ub + spread + (((key - spread) << lp) | part)) * dim;
+                });
+            else
+                __syncthreads();
+            if (spread) {
+                if (tid == 0) had = have;
                 __syncthreads();
             }
         }
-        for (uint32_t i = threadIdx.x; i < n; i += 256) svals[lo + i] = vals[seg[i]];
-        __syncthreads();
     }
+    if (spread && tid == 0) has[item] = have;
 }
 
-// A segment of many lookups is ordered by a bitmap of their positions in the slot, HUGE_WINDOW of these at a time (the
-// place of a lookup: bits set below its own).  The bitmap of a slot of 49 k lookups with its prefix sums takes 9 KB of LDS,
-// so a CU holds eight workgroups; counters per example, as this had before, took 64 KB at 16384 examples, or memory.
-// Beside rank_mid (72 -> 42 us), 4.9 M lookups: 57 -> 34 us.
-constexpr uint32_t HUGE_WINDOW = 1u << 17;
-inline size_t order_huge_room(size_t max_len) { return (std::min<size_t>(max_len, HUGE_WINDOW) + 63) / 64; }
-
-// bits: [room] words of LDS, then [room] numbers of set bits before the word
-__device__ __forceinline__ void order_huge(const uint32_t* __restrict__ huge_list, uint32_t n_huge,
-                                           const uint32_t* __restrict__ lbase, const uint32_t* __restrict__ ubase, int N,
-                                           const uint32_t* __restrict__ seg_off, const uint64_t* __restrict__ vals,
-                                           const uint32_t* __restrict__ tpos, uint64_t* __restrict__ svals,
-                                           unsigned long long* bits, uint32_t room, uint32_t* red, uint32_t block,
-                                           uint32_t blocks) {
-    uint32_t* const before = reinterpret_cast<uint32_t*>(bits + room);
-    for (uint32_t k = block; k < n_huge; k += blocks) {
-        const uint32_t u = huge_list[k];
-        const uint32_t lo = seg_off[u], hi = seg_off[u + 1];
-        const int sl = find_slot(ubase, N, u);
-        const uint32_t l0 = lbase[sl], len = lbase[sl + 1] - l0;
-        uint32_t done = 0;  // lookups of the windows before
-        for (uint32_t w0 = 0; w0 < len; w0 += HUGE_WINDOW) {
-            const uint32_t span = min(len - w0, HUGE_WINDOW), words = (span + 63) / 64;  // (words <= room)
-            for (uint32_t i = threadIdx.x; i < words; i += 256) bits[i] = 0;
-            __syncthreads();
-            for (uint32_t j = lo + threadIdx.x; j < hi; j += 256) {
-                const uint32_t p = tpos[j] - l0 - w0;  // (a position before the window: beyond it)
-                if (p < span) atomicOr(&bits[p >> 6], 1ull << (p & 63));
-            }
-            __syncthreads();
-            for (uint32_t i0 = 0; i0 < words; i0 += 256) {
-                const uint32_t i = i0 + threadIdx.x;
-                uint32_t total;
-                const uint32_t x = block_excl_scan_256<uint32_t>(i < words ? (uint32_t)__popcll(bits[i]) : 0u, red, &total);
-                if (i < words) before[i] = done + x;
-                done += total;
-                __syncthreads();
-            }
-            for (uint32_t j = lo + threadIdx.x; j < hi; j += 256) {
-                const uint32_t gi = tpos[j], p = gi - l0 - w0;
-                if (p < span) svals[lo + before[p >> 6] + (uint32_t)__popcll(bits[p >> 6] & ((1ull << (p & 63)) - 1ull))] = vals[gi];
-            }
-            __syncthreads();
+// The sums of the spread signs: a wavefront per sign, whose groups of LPG lanes take every so many of the slot's parts in turn
+// and then add their sums up by halves.
+template <int LPG, bool ANY>
+__global__ __launch_bounds__(256) void k_reduce_pooled_shares(const uint32_t* __restrict__ lbase,
+                                                              const uint32_t* __restrict__ ubase, int dim, int D,
+                                                              const DevStatus* status, const float* __restrict__ shares,
+                                                              const uint64_t* __restrict__ has, float* __restrict__ flat,
+                                                              PoolShare share) {
+    if (status->abort | status->mismatch) return;
+    constexpr uint32_t PER = 256 / 64;
+    const uint32_t sl = blockIdx.x / (POOL_SPREAD / PER), key = blockIdx.x % (POOL_SPREAD / PER) * PER + threadIdx.x / 64;
+    const uint32_t group = threadIdx.x % 64 / LPG;
+    const int sub = threadIdx.x % LPG;
+    const uint32_t l0 = lbase[sl], len = lbase[sl + 1] - l0, ub = ubase[sl], us = ubase[sl + 1] - ub;
+    const uint32_t lp = share.parts_log2(len), parts = 1u << lp, p0 = share.first_part(sl, l0);
+    if (len == 0 || share.spread(lp) == 0 || key >= us) return;  // (the same for a whole wavefront)
+    for (int c0 = 0; c0 < D; c0 += 4 * LPG) {
+        float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+        for (uint32_t q = group; q < parts; q += 64 / LPG) {
+            if (!((has[p0 + q] >> key) & 1ull)) continue;
+            const float4 v = row_part<ANY>(shares + ((uint64_t)(p0 + q) * POOL_SPREAD + key) * dim + c0, sub, D - c0);
+            acc.x += v.x;
+            acc.y += v.y;
+            acc.z += v.z;
+            acc.w += v.w;
         }
-    }
-}
-
-// The three side by side in one launch, the longest segments first: each has segments of its own, and waits for chains.
-// 860 k lookups: three launches 34 us, this one 21; 4.9 M: 86, as the three took on three streams, without the events
-// between these.
-constexpr uint32_t ORDER_HUGE_GRID = 1024, ORDER_MID_GRID = 2048;  // workgroups at most, which take their segments in turn
-inline size_t order_lds(size_t room) { return std::max<size_t>(room * 12, ORDER_HUGE * sizeof(uint32_t)); }
-
-__global__ __launch_bounds__(256) void k_order_segments(uint32_t L, const uint32_t* __restrict__ lbase,
-                                                        const uint32_t* __restrict__ ubase, int N,
-                                                        const uint32_t* __restrict__ u_of_gi,
-                                                        const uint32_t* __restrict__ mid_list,
-                                                        const uint32_t* __restrict__ huge_list, const uint32_t* counts,
-                                                        const uint32_t* __restrict__ seg_off,
-                                                        const uint64_t* __restrict__ vals, const uint32_t* __restrict__ tpos,
-                                                        uint64_t* __restrict__ svals, uint32_t room, uint32_t huge_blocks,
-                                                        uint32_t mid_blocks, const DevStatus* status) {
-    extern __shared__ unsigned long long order_sh[];
-    __shared__ uint32_t red[4];
-    if (status->abort) return;
-    const uint32_t b = blockIdx.x, long_blocks = huge_blocks + mid_blocks;
-    if (b < huge_blocks)
-        order_huge(huge_list, counts[2], lbase, ubase, N, seg_off, vals, tpos, svals, order_sh, room, red, b, huge_blocks);
-    else if (b < long_blocks)
-        rank_mid(mid_list, counts[1], seg_off, vals, tpos, svals, reinterpret_cast<uint32_t*>(order_sh), b - huge_blocks,
-                 mid_blocks);
-    else
-        rank_short(L, u_of_gi, vals, tpos, seg_off, svals, b - long_blocks, gridDim.x - long_blocks);
-}
-
-// The sum of the shares of lookups from, from + step, ... below `to` of one distinct sign, in this order: every lookup
-// has its example's pooled row times 1 / d(lookups of the example); four elements of a row, part c of them.  The
-// values of a window first, then their rows, all loads of a kind independent.
-template <bool ANY>
-__device__ __forceinline__ float4 sum_shares(const float* __restrict__ pooled, const uint64_t* __restrict__ svals, uint32_t from,
-                                             uint32_t to, uint32_t step, int dim, int c, int combiner) {
-    float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
-    for (uint32_t j0 = from; j0 < to; j0 += COMBINE_WINDOW * step) {
-        uint64_t v[COMBINE_WINDOW];
-        float4 g[COMBINE_WINDOW];
 #pragma unroll
-        for (int q = 0; q < COMBINE_WINDOW; q++) v[q] = j0 + q * step < to ? svals[j0 + q * step] : 0ull;
-#pragma unroll
-        for (int q = 0; q < COMBINE_WINDOW; q++)
-            g[q] = j0 + q * step < to ? row_part<ANY>(pooled + (v[q] >> 32) * (uint64_t)dim, c, dim)
-                                      : make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll
-        for (int q = 0; q < COMBINE_WINDOW; q++) {
-            if (j0 + q * step >= to) break;
-            const float scale = combiner == COMBINE_SUM ? 1.f : 1.f / combine_divisor((uint32_t)v[q], combiner);
-            acc.x += g[q].x * scale;
-            acc.y += g[q].y * scale;
-            acc.z += g[q].z * scale;
-            acc.w += g[q].w * scale;
+        for (int o = 32; o >= LPG; o >>= 1) {
+            acc.x += __shfl_xor(acc.x, o);
+            acc.y += __shfl_xor(acc.y, o);
+            acc.z += __shfl_xor(acc.z, o);
+            acc.w += __shfl_xor(acc.w, o);
         }
+        if (group == 0) put_row_part<ANY>(flat + (uint64_t)(ub + key) * dim + c0, sub, D - c0, acc);
     }
-    return acc;
-}
-
-// Step 3: a group of `chunks` threads per distinct index, four elements of the row each (whatever its length and
-// alignment), sums its lookups' shares of the pooled gradient rows, in position order.  A distinct index with long_min
-// lookups or more (a frequent sign) is left out: k_place_lookups has listed those, one workgroup each sums them
-// (reduce_long).
-//
-// Bound by the rows it reads again and again: the pooled rows of a slot (1 MB at 16384 examples of 16 elements) are more
-// often in the L2 of a die that works on one slot at a time, so the distinct indices go to the dies in runs of REDUCE_RUN
-// workgroups (DieRuns; a grid-stride loop had every die read the rows of six slots).  4.9 M lookups of 16 elements:
-// 172 -> 138 us, the frequent signs beside it 120 -> 93 us.  By the counters of both together 30 % of the L2's requests hit:
-// 426 MB are read where each row and value once are 152, with what is written 3.8 TB/s.
-constexpr uint32_t REDUCE_RUN = 256;
-
-template <bool ANY>
-__device__ __forceinline__ void reduce_short(const SlotDesc* __restrict__ descs, const uint32_t* __restrict__ ubase, int N,
-                                             int dim, int combiner, const DevStatus* status,
-                                             const uint32_t* __restrict__ seg_off, const uint64_t* __restrict__ svals,
-                                             float* __restrict__ flat, uint32_t long_min, uint32_t* ub, uint32_t block,
-                                             uint32_t blocks) {
-    load_lbase(ub, ubase, N);
-    const uint32_t chunks = (uint32_t)(dim + 3) / 4;
-    const uint64_t total = (uint64_t)status->n_unique * chunks;
-    for (DieRuns r((uint32_t)((total + 255) / 256), REDUCE_RUN, block, blocks); r.more(); r.next()) {
-        const uint64_t t = (uint64_t)r.item() * 256 + threadIdx.x;
-        if (t >= total) continue;
-        const uint32_t u = (uint32_t)(t / chunks);
-        const int c = (int)(t - (uint64_t)u * chunks);
-        const uint32_t lo = seg_off[u], hi = seg_off[u + 1];
-        if (hi - lo >= long_min) continue;
-        const float* pooled = descs[find_slot(ub, N, u)].grads;  // the slot whose window of distinct indices holds u
-        put_row_part<ANY>(flat + (uint64_t)u * dim, c, dim, sum_shares<ANY>(pooled, svals, lo, hi, 1, dim, c, combiner));
-    }
-}
-
-// One workgroup per frequent distinct index: its 256 / chunks thread groups each sum every
-// (256 / chunks)-th lookup in position order, then the partial sums are added in group order.
-// The order of the additions is fixed, so the result does not vary from run to run.
-template <bool ANY>
-__device__ __forceinline__ void reduce_long(const SlotDesc* __restrict__ descs, const uint32_t* __restrict__ ubase, int N,
-                                            int dim, int combiner, const uint32_t* __restrict__ seg_off,
-                                            const uint64_t* __restrict__ svals, float* __restrict__ flat,
-                                            const uint32_t* __restrict__ mid_list, const uint32_t* __restrict__ huge_list,
-                                            const uint32_t* counts, float4* part, uint32_t block, uint32_t blocks) {
-    const int chunks = (dim + 3) / 4;
-    const int groups = 256 / chunks;
-    const int q = threadIdx.x / chunks, c = threadIdx.x - q * chunks;
-    // the frequent ones: the two lists k_place_lookups left (ORDER_MID lookups or more)
-    const uint32_t n_mid = counts[1], n_long = n_mid + counts[2];
-    for (uint32_t k = n_long - 1 - block; k < n_long; k -= blocks) {  // (the longest, which are listed last, first; ends by wrapping)
-        const uint32_t u = k < n_mid ? mid_list[k] : huge_list[k - n_mid];
-        const uint32_t lo = seg_off[u], hi = seg_off[u + 1];
-        const float* pooled = descs[find_slot(ubase, N, u)].grads;
-        if (q < groups) part[threadIdx.x] = sum_shares<ANY>(pooled, svals, lo + q, hi, groups, dim, c, combiner);
-        __syncthreads();
-        if (q == 0) {
-            float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
-            for (int g = 0; g < groups; g++) {
-                const float4 p = part[g * chunks + c];
-                sum.x += p.x;
-                sum.y += p.y;
-                sum.z += p.z;
-                sum.w += p.w;
-            }
-            put_row_part<ANY>(flat + (uint64_t)u * dim, c, dim, sum);
-        }
-        __syncthreads();
-    }
-}
-
-// Both side by side in one launch, the frequent signs first.  860 k lookups of 16 elements: 53 us in two launches, 46 in
-// this one; 4.9 M: 140, as on two streams.
-template <bool ANY>
-__global__ __launch_bounds__(256) void k_reduce_pooled(const SlotDesc* __restrict__ descs,
-                                                       const uint32_t* __restrict__ ubase, int N, int dim, int combiner,
-                                                       const DevStatus* status, const uint32_t* __restrict__ seg_off,
-                                                       const uint64_t* __restrict__ svals, float* __restrict__ flat,
-                                                       uint32_t long_min, const uint32_t* __restrict__ mid_list,
-                                                       const uint32_t* __restrict__ huge_list, const uint32_t* counts,
-                                                       uint32_t long_blocks) {
-    __shared__ union {
-        uint32_t ub[MAX_SLOTS + 1];
-        float4 part[256];
-    } sh;
-    if (status->abort) return;
-    if (blockIdx.x < long_blocks)
-        reduce_long<ANY>(descs, ubase, N, dim, combiner, seg_off, svals, flat, mid_list, huge_list, counts, sh.part, blockIdx.x,
-                         long_blocks);
-    else
-        reduce_short<ANY>(descs, ubase, N, dim, combiner, status, seg_off, svals, flat, long_min, sh.ub,
-                          blockIdx.x - long_blocks, gridDim.x - long_blocks);
 }
 
 }  // namespace tn

@@ -1,0 +1,224 @@
+// The backward half of the combiner in LDS: up to POOL_ITEMS_MAX lookups of a slot, in the order of their positions, are
+// sorted by their sign and every sign's pooled rows summed.  What both paths of a push of pooled gradients are made of
+// (k_reduce_pooled, k_small_pool).
+#ifndef TN_POOL_ITEMS_H_
+#define TN_POOL_ITEMS_H_
+
+#include "sparse_kernels.h"
+
+namespace tn {
+
+constexpr int POOL_THREADS = 512;
+constexpr uint32_t POOL_ITEMS_MAX = 2048;
+constexpr uint32_t POOL_ITEMS = POOL_ITEMS_MAX / POOL_THREADS;
+constexpr uint32_t POOL_WAVES = POOL_THREADS / 64;
+constexpr uint32_t POOL_RUN = POOL_ITEMS_MAX / POOL_WAVES;  // consecutive lookups a wavefront sorts
+constexpr uint32_t POOL_WORDS = POOL_ITEMS_MAX / 64;
+constexpr uint32_t POOL_PIECE = 16;
+constexpr uint32_t POOL_PIECES = POOL_ITEMS_MAX / POOL_PIECE;
+constexpr uint32_t POOL_AHEAD = 4;  // rows of a group of lanes in flight (eight: the registers of three workgroups do not hold them)
+constexpr uint32_t POOL_DIGIT = 7;  // (10, one pass for most slots, whose 8192 counters take longer: 44 -> 47 us, 175 -> 184)
+enum { POOL_SUM = 0, POOL_MEAN = 1, POOL_SQRTN = 2 };  // (the combiners of the C ABI)
+static_assert(POOL_RUN == 64 * POOL_ITEMS && 64 % POOL_PIECE == 0, "whole wavefronts, pieces inside a word");
+
+// 47 KB: three workgroups of eight wavefronts to a CU (twice the size in workgroups of sixteen: one to a CU, and 4.9 M
+// lookups took 2.5 times as long)
+struct PoolLds {
+    uint32_t key[POOL_ITEMS_MAX];      // the lookup's sign
+    uint32_t example[POOL_ITEMS_MAX];  // its example
+    float scale[POOL_ITEMS_MAX];       // 1 / d(lookups of the example); negative: not its sign's first lookup
+    uint16_t ord[POOL_ITEMS_MAX];      // the lookups in the order of their signs
+    union {
+        struct {
+            uint16_t half[POOL_ITEMS_MAX];             // while sorting: the order after every other pass,
+            uint16_t digit[POOL_WAVES << POOL_DIGIT];  // counters
+        };
+        float4 part[POOL_PIECES][2][4];  // then: what a piece has of a sign that began before it / goes on behind it
+        uint32_t list[2 * POOL_THREADS + 1];  // (before: k_reduce_pooled's tiles)
+    };
+    unsigned long long heads[POOL_WORDS];  // starts of the signs in the order
+    uint32_t wsum[POOL_WAVES];
+};
+
+// Last set bit at or below i, first one above it (or `none`), in a bitmap in LDS.
+__device__ __forceinline__ uint32_t bit_at_or_below(const unsigned long long* bm, uint32_t i) {
+    uint32_t w = i >> 6;
+    unsigned long long v = bm[w] & (~0ull >> (63 - (i & 63)));
+    while (v == 0) v = bm[--w];  // (bit 0 is set)
+    return w * 64 + 63 - (uint32_t)__clzll((long long)v);
+}
+__device__ __forceinline__ uint32_t bit_above(const unsigned long long* bm, uint32_t i, uint32_t words, uint32_t none) {
+    uint32_t w = i >> 6;
+    unsigned long long v = (i & 63) == 63 ? 0ull : bm[w] & (~0ull << ((i & 63) + 1));
+    while (v == 0) {
+        if (++w >= words) return none;
+        v = bm[w];
+    }
+    return w * 64 + (uint32_t)__ffsll((long long)v) - 1;
+}
+
+__device__ __forceinline__ float pool_scale(float count, int combiner) {
+    return combiner == POOL_SUM ? 1.f : 1.f / (combiner == POOL_MEAN ? count : sqrtf(count));
+}
+
+// lds.key, example, scale [0, n) are filled, keys of `bits` bits, n > 0.  A stable radix sort (passes of up to 7 bits,
+// a wavefront's lanes told apart by ballots); then every group of LPG lanes takes POOL_PIECE consecutive places of the order,
+// whatever signs they hold, POOL_AHEAD rows in flight, sixteen elements of them at a time (LPG 4).  (A group per sign has one
+// row in flight where most signs have one lookup, and waits for the longest of its wavefront: twice as long.)  A sign
+// with lookups in several pieces: their shares are added in order.  row(key, first, add): where its sum goes, and whether it
+// is added to what stands there; first: the sign's first lookup is among those summed.
+template <int LPG, bool ANY, typename Row>
+__device__ __forceinline__ void pool_items(PoolLds& lds, uint32_t n, uint32_t bits, const float* __restrict__ pooled, int dim,
+                                           int D, Row row) {
+    static_assert(LPG <= 4, "PoolLds::part");
+    uint32_t tid = threadIdx.x;
+    // (addresses worked out from here on stay inside the round: held in registers across the caller's loop they cost a
+    // workgroup of the three)
+    asm volatile("" : "+v"(tid));
+    const uint32_t lane = tid & 63, wave = tid >> 6;
+    const uint32_t passes = (bits + POOL_DIGIT - 1) / POOL_DIGIT, width = passes ? (bits + passes - 1) / passes : 0u;
+    __syncthreads();
+    if (passes == 0) {
+        for (uint32_t i = tid; i < n; i += POOL_THREADS) lds.ord[i] = (uint16_t)i;
+        __syncthreads();
+    }
+    for (uint32_t pass = 0; pass < passes; pass++) {
+        uint16_t* const to = (passes - 1 - pass) & 1u ? lds.half : lds.ord;
+        const uint16_t* const from = (passes - 1 - pass) & 1u ? lds.ord : lds.half;  // (the first pass takes them as they are)
+        for (uint32_t i = tid; i < POOL_WAVES << width >> 1; i += POOL_THREADS) reinterpret_cast<uint32_t*>(lds.digit)[i] = 0;
+        __syncthreads();
+        uint32_t item[POOL_ITEMS], dg[POOL_ITEMS], at[POOL_ITEMS];
+#pragma unroll
+        for (uint32_t j = 0; j < POOL_ITEMS; j++) {
+            const uint32_t i = wave * POOL_RUN + j * 64 + lane;
+            item[j] = i < n ? (pass == 0 ? i : (uint32_t)from[i]) : 0u;
+        }
+#pragma unroll
+        for (uint32_t j = 0; j < POOL_ITEMS; j++) {
+            const bool valid = wave * POOL_RUN + j * 64 + lane < n;
+            dg[j] = (lds.key[item[j]] >> (pass * width)) & ((1u << width) - 1u);
+            unsigned long long same = __ballot(valid);
+            for (uint32_t q = 0; q < width; q++) {
+                const unsigned long long m = __ballot((dg[j] >> q) & 1u);
+                same &= ((dg[j] >> q) & 1u) ? m : ~m;
+            }
+            at[j] = 0;
+            const uint32_t k = dg[j] * POOL_WAVES + wave;
+            if (valid) at[j] = lds.digit[k] + (uint32_t)__popcll(same & ((1ull << lane) - 1ull));  // (before this round)
+            wave_sync();
+            if (valid && (uint32_t)__ffsll((long long)same) - 1 == lane) lds.digit[k] += (uint16_t)__popcll(same);
+            wave_sync();
+        }
+        __syncthreads();
+        {  // digit by digit and wavefront by wavefront: where they go
+            const uint32_t all = POOL_WAVES << width, each = (all + POOL_THREADS - 1) / POOL_THREADS, k0 = tid * each;
+            uint32_t sum = 0;
+            for (uint32_t k = k0; k < min(k0 + each, all); k++) sum += lds.digit[k];
+            uint32_t x = block_excl_scan<uint32_t, POOL_WAVES>(sum, lds.wsum, nullptr);
+            for (uint32_t k = k0; k < min(k0 + each, all); k++) {
+                const uint32_t c = lds.digit[k];
+                lds.digit[k] = (uint16_t)x;
+                x += c;
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (uint32_t j = 0; j < POOL_ITEMS; j++)
+            if (wave * POOL_RUN + j * 64 + lane < n) to[lds.digit[dg[j] * POOL_WAVES + wave] + at[j]] = (uint16_t)item[j];
+        __syncthreads();
+    }
+    // starts of the signs in the order (and what lies behind it)
+#pragma unroll
+    for (uint32_t j = 0; j < POOL_ITEMS; j++) {
+        const uint32_t i = wave * POOL_RUN + j * 64 + lane;
+        const bool head = i >= n || i == 0 || lds.key[lds.ord[i]] != lds.key[lds.ord[i - 1]];
+        const unsigned long long m = __ballot(head);
+        if (lane == 0) lds.heads[i >> 6] = m;
+    }
+    __syncthreads();
+    const uint32_t pieces = (n + POOL_PIECE - 1) / POOL_PIECE;
+    asm volatile("" : "+v"(tid));
+    const int sub = tid % LPG;
+    auto put = [&](uint32_t key, bool first, int c0, float4 v) {
+        bool add;
+        float* out = row(key, first, add) + c0;
+        if (add) {
+            const float4 w = row_part<ANY>(out, sub, D - c0);
+            v = make_float4(w.x + v.x, w.y + v.y, w.z + v.z, w.w + v.w);
+        }
+        put_row_part<ANY>(out, sub, D - c0, v);
+    };
+    for (int c0 = 0; c0 < D; c0 += 4 * LPG) {
+        for (uint32_t q = tid / LPG; q < pieces; q += POOL_THREADS / LPG) {
+            const uint32_t lo = q * POOL_PIECE, hi = lo + POOL_PIECE;
+            // which places start a sign, and the one behind the piece (those behind the last lookup do)
+            uint32_t hb = (uint32_t)(lds.heads[lo >> 6] >> (lo & 63)) & ((1u << POOL_PIECE) - 1u);
+            if (hi >= n || ((lds.heads[hi >> 6] >> (hi & 63)) & 1ull)) hb |= 1u << POOL_PIECE;
+            bool began = false, first = false;  // the running sum's sign: here, with its first lookup
+            float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll 1
+            for (uint32_t j0 = 0; j0 < POOL_PIECE && lo + j0 < n; j0 += POOL_AHEAD, hb >>= POOL_AHEAD) {
+                float4 g[POOL_AHEAD];
+                float sc[POOL_AHEAD];
+                uint32_t key[POOL_AHEAD];
+#pragma unroll
+                for (uint32_t w = 0; w < POOL_AHEAD; w++) {
+                    const uint32_t i = lds.ord[min(lo + j0 + w, n - 1)];
+                    sc[w] = lds.scale[i];
+                    key[w] = lds.key[i];
+                    g[w] = row_part<ANY>(pooled + (uint64_t)lds.example[i] * dim + c0, sub, D - c0);
+                }
+#pragma unroll
+                for (uint32_t w = 0; w < POOL_AHEAD; w++) {
+                    if (lo + j0 + w >= n) break;
+                    if ((hb >> w) & 1u) {
+                        acc = make_float4(0.f, 0.f, 0.f, 0.f);
+                        began = true;
+                        first = sc[w] > 0.f;
+                    }
+                    const float scale = fabsf(sc[w]);
+                    acc.x += g[w].x * scale;
+                    acc.y += g[w].y * scale;
+                    acc.z += g[w].z * scale;
+                    acc.w += g[w].w * scale;
+                    if ((hb >> (w + 1)) & 1u) {  // the sign ends here
+                        if (began)
+                            put(key[w], first, c0, acc);
+                        else
+                            lds.part[q][0][sub] = acc;
+                    }
+                }
+            }
+            if (!(hb & 1u)) lds.part[q][began ? 1 : 0][sub] = acc;  // it goes on
+        }
+        __syncthreads();
+        for (uint32_t q = tid / LPG; q < pieces; q += POOL_THREADS / LPG) {
+            const uint32_t hi = (q + 1) * POOL_PIECE;
+            if (hi >= n || ((lds.heads[hi >> 6] >> (hi & 63)) & 1ull)) continue;  // no sign goes on behind this piece
+            const uint32_t from = bit_at_or_below(lds.heads, hi - 1);
+            if (from < q * POOL_PIECE) continue;  // it began before it
+            const uint32_t end = bit_above(lds.heads, hi, POOL_WORDS, n), last = (end - 1) / POOL_PIECE;
+            float4 acc = lds.part[q][1][sub];
+            for (uint32_t r = q + 1; r <= last; r += 4) {
+                float4 g[4];
+#pragma unroll
+                for (uint32_t w = 0; w < 4; w++) g[w] = lds.part[min(r + w, last)][0][sub];
+#pragma unroll
+                for (uint32_t w = 0; w < 4; w++) {
+                    if (r + w > last) break;
+                    acc.x += g[w].x;
+                    acc.y += g[w].y;
+                    acc.z += g[w].z;
+                    acc.w += g[w].w;
+                }
+            }
+            const uint32_t i = lds.ord[from];
+            put(lds.key[i], lds.scale[i] > 0.f, c0, acc);
+        }
+        __syncthreads();
+    }
+}
+
+}  // namespace tn
+
+#endif  // TN_POOL_ITEMS_H_

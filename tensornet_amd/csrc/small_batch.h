@@ -18,6 +18,7 @@
 #ifndef TN_SMALL_BATCH_H_
 #define TN_SMALL_BATCH_H_
 
+#include "pool_items.h"
 #include "remap_lds.h"
 
 #include <algorithm>
@@ -551,76 +552,55 @@ __global__ __launch_bounds__(256) void k_small_verify(SmallShape b, SmallPlan p,
 }
 
 // Pooled gradients: the gradient of every distinct sign of a slot is the sum over its lookups, in order, of their
-// examples' rows times 1 / d(lookups of the example); a workgroup per slot.  The lookups are ordered by their sign's
-// first position with a stable radix sort in LDS (two passes of 7 bits, a wavefront's lanes told apart by ballots) and
-// every stretch of POOL_PIECE lookups of one sign is summed by a group of lanes; the sums of a sign with several
-// stretches are added in order.  The order of all additions is fixed.  flat[gi of the sign's first lookup, :] = sum, over
-// the D elements the updates read (rows of `dim`: with the cvm columns).
-constexpr int POOL_THREADS = 1024;
-constexpr int POOL_ITEMS = SMALL_SLOT_MAX / POOL_THREADS;
-constexpr int POOL_WAVES = POOL_THREADS / 64;
-constexpr int POOL_RUN = SMALL_SLOT_MAX / POOL_WAVES;  // consecutive lookups a wavefront sorts
-constexpr uint32_t POOL_PIECE = 32;
-constexpr int POOL_DIGIT = 7;
-enum { POOL_SUM = 0, POOL_MEAN = 1, POOL_SQRTN = 2 };  // (the combiners of the C ABI)
-static_assert(2 * POOL_DIGIT >= SMALL_SLOT_BITS && POOL_RUN == 64 * POOL_ITEMS, "two passes sort a slot");
-
-// Last set bit at or below i, first one above it (or `none`), in a bitmap in LDS.
-__device__ __forceinline__ uint32_t bit_at_or_below(const unsigned long long* bm, uint32_t i) {
-    uint32_t w = i >> 6;
-    unsigned long long v = bm[w] & (~0ull >> (63 - (i & 63)));
-    while (v == 0) v = bm[--w];  // (bit 0 is set)
-    return w * 64 + 63 - (uint32_t)__clzll((long long)v);
+// examples' rows times 1 / d(lookups of the example).  2^lp workgroups per slot, each of which looks at the whole slot and
+// takes the signs whose first position is its own modulo 2^lp, POOL_ITEMS_MAX lookups at a time (pool_items).
+// flat[gi of the sign's first lookup, :] = sum, over the D elements the updates read (rows of `dim`: with the cvm columns).
+// 50 slots of 3100 lookups: 39 us (a workgroup of 1024 threads per slot: 43), a push and pull with 512, 1024, 2048 lookups a
+// workgroup 142, 136, 136 us.
+constexpr uint32_t SMALL_POOL_FILL = 1024;
+inline uint32_t small_pool_parts_log2(uint32_t max_len) {
+    uint32_t lp = 0;
+    while ((max_len >> lp) > SMALL_POOL_FILL) lp++;
+    return lp;
 }
-__device__ __forceinline__ uint32_t bit_above(const unsigned long long* bm, uint32_t i, uint32_t words, uint32_t none) {
-    uint32_t w = i >> 6;
-    unsigned long long v = (i & 63) == 63 ? 0ull : bm[w] & (~0ull << ((i & 63) + 1));
-    while (v == 0) {
-        if (++w >= words) return none;
-        v = bm[w];
-    }
-    return w * 64 + (uint32_t)__ffsll((long long)v) - 1;
-}
+constexpr uint32_t SMALL_POOL_ITEMS = SMALL_SLOT_MAX / POOL_THREADS;  // lookups of a thread
 
 template <int LPG, bool ANY>
-__global__ __launch_bounds__(POOL_THREADS) void k_small_pool(SmallShape b, SmallPlan p, const SlotDesc* __restrict__ descs,
+__global__ __launch_bounds__(POOL_THREADS) __attribute__((amdgpu_waves_per_eu(6, 6))) void k_small_pool(SmallShape b, SmallPlan p, const SlotDesc* __restrict__ descs,
                                                              int64_t batch, int dim, int D, int combiner,
-                                                             float* __restrict__ flat, float* __restrict__ partial,
-                                                             DevStatus* status,
-                                                             uint32_t* host_err) {
-    __shared__ uint16_t fo[SMALL_SLOT_MAX];             // first position of the lookup's sign
-    __shared__ uint32_t xb[SMALL_SLOT_MAX];             // example of the lookup
-    __shared__ uint16_t ord[SMALL_SLOT_MAX];            // the lookups in the order of their signs
-    __shared__ uint16_t piece[SMALL_SLOT_MAX + 1];      // where the pieces start in it
-    __shared__ uint32_t work[SMALL_SLOT_MAX];           // while sorting: the order after the first pass, counters; then the scales
-    __shared__ unsigned long long heads[SMALL_WORDS];   // starts: of the examples by position, then of the signs in the order
-    __shared__ uint32_t wsum[POOL_WAVES];
+                                                             float* __restrict__ flat, DevStatus* status, uint32_t* host_err,
+                                                             uint32_t lp) {
+    __shared__ PoolLds lds;
+    __shared__ unsigned long long starts[SMALL_WORDS];  // of the examples
     __shared__ uint32_t bad;
-    uint16_t* const half = reinterpret_cast<uint16_t*>(work);                          // [SMALL_SLOT_MAX]
-    uint32_t* const digit = work + SMALL_SLOT_MAX / 2;                                 // [1 << POOL_DIGIT][POOL_WAVES]
-    float* const scale = reinterpret_cast<float*>(work);                               // [SMALL_SLOT_MAX], by position
-    static_assert((POOL_WAVES << POOL_DIGIT) <= SMALL_SLOT_MAX / 2, "the counters fit");
-    const SlotDesc d = descs[blockIdx.x];
+    const uint32_t sl = blockIdx.x >> lp, part = blockIdx.x & ((1u << lp) - 1u);
+    const SlotDesc d = descs[sl];
     const uint32_t n = d.len, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     if (n == 0 || status->mismatch) return;
     const int64_t* ex = d.mapped;
     if (tid == 0) bad = 0;
-    for (uint32_t i = tid; i < SMALL_WORDS; i += POOL_THREADS) heads[i] = 0;
     __syncthreads();
+    uint32_t f[SMALL_POOL_ITEMS], x[SMALL_POOL_ITEMS];
+    uint32_t cnt = 0;
 #pragma unroll
-    for (int j = 0; j < POOL_ITEMS; j++) {
-        const uint32_t i = wave * POOL_RUN + j * 64 + lane;
+    for (uint32_t j = 0; j < SMALL_POOL_ITEMS; j++) {
+        const uint32_t i = (wave * SMALL_POOL_ITEMS + j) * 64 + lane;
         bool head = false;
+        x[j] = 0;
+        f[j] = NO_ROW;
         if (i < n) {
-            const int64_t x = ex[i], prev = i > 0 ? ex[i - 1] : -1;
-            if (x < 0 || x >= batch || prev > x) bad = 1;
-            fo[i] = p.first_of[d.lbase + i];
-            xb[i] = (uint32_t)x;
-            head = x != prev;
+            const int64_t e = ex[i], prev = i > 0 ? ex[i - 1] : -1;
+            if (e < 0 || e >= batch || prev > e) bad = 1;
+            head = e != prev;
+            x[j] = (uint32_t)e;
+            f[j] = p.first_of[d.lbase + i];
+            if ((f[j] & ((1u << lp) - 1u)) != part) f[j] = NO_ROW;
         }
         const unsigned long long m = __ballot(head);
-        if (lane == 0) heads[i >> 6] = m;
+        if (lane == 0) starts[i >> 6] = m;
+        cnt += (uint32_t)__popcll(__ballot(f[j] != NO_ROW));
     }
+    if (lane == 0) lds.wsum[wave] = cnt;
     __syncthreads();
     if (bad) {  // unsorted or out-of-range example ids: nothing of this push is applied
         if (tid == 0) {
@@ -629,131 +609,34 @@ __global__ __launch_bounds__(POOL_THREADS) void k_small_pool(SmallShape b, Small
         }
         return;
     }
-    const uint32_t words = (n + 63) / 64;
-    float mine[POOL_ITEMS];  // 1 / d(lookups of the example) of my lookups
+    uint32_t first = 0, total = 0;  // of my part: lookups of the wavefronts before, of all
 #pragma unroll
-    for (int j = 0; j < POOL_ITEMS; j++) {
-        const uint32_t i = wave * POOL_RUN + j * 64 + lane;
-        mine[j] = 1.f;
-        if (i < n && combiner != POOL_SUM) {
-            const float cnt = (float)(bit_above(heads, i, words, n) - bit_at_or_below(heads, i));
-            mine[j] = 1.f / (combiner == POOL_MEAN ? cnt : sqrtf(cnt));
-        }
+    for (uint32_t w = 0; w < POOL_WAVES; w++) {
+        if (w < wave) first += lds.wsum[w];
+        total += lds.wsum[w];
     }
-    // stable sort by fo: pass 0 takes the lookups in order, pass 1 the order of pass 0
-    for (int pass = 0; pass < 2; pass++) {
-        for (uint32_t i = tid; i < POOL_WAVES << POOL_DIGIT; i += POOL_THREADS) digit[i] = 0;
-        __syncthreads();
-        uint32_t item[POOL_ITEMS], dg[POOL_ITEMS], at[POOL_ITEMS];
+    const uint32_t words = (n + 63) / 64, bits = (n - 1) >> lp ? 32 - (uint32_t)__clz((int)((n - 1) >> lp)) : 0u;
+    for (uint32_t done = 0; done < total; done += POOL_ITEMS_MAX) {
+        uint32_t at = first - done;  // (of a round before: wraps)
 #pragma unroll
-        for (int j = 0; j < POOL_ITEMS; j++) {
-            const uint32_t i = wave * POOL_RUN + j * 64 + lane;
-            const bool valid = i < n;
-            item[j] = valid ? (pass == 0 ? i : (uint32_t)half[i]) : 0u;
-            dg[j] = valid ? ((uint32_t)fo[item[j]] >> (pass * POOL_DIGIT)) & ((1u << POOL_DIGIT) - 1u) : 0u;
-            unsigned long long same = __ballot(valid);
-#pragma unroll
-            for (int q = 0; q < POOL_DIGIT; q++) {
-                const unsigned long long m = __ballot((dg[j] >> q) & 1u);
-                same &= ((dg[j] >> q) & 1u) ? m : ~m;
+        for (uint32_t j = 0; j < SMALL_POOL_ITEMS; j++) {
+            const uint32_t i = (wave * SMALL_POOL_ITEMS + j) * 64 + lane;
+            const unsigned long long own = __ballot(f[j] != NO_ROW);
+            const uint32_t q = at + (uint32_t)__popcll(own & ((1ull << lane) - 1ull));
+            if (f[j] != NO_ROW && q < POOL_ITEMS_MAX) {
+                const float count = combiner == POOL_SUM ? 1.f : (float)(bit_above(starts, i, words, n) - bit_at_or_below(starts, i));
+                const float scale = pool_scale(count, combiner);
+                lds.key[q] = f[j] >> lp;
+                lds.example[q] = x[j];
+                lds.scale[q] = f[j] == i ? scale : -scale;
             }
-            at[j] = 0;
-            const uint32_t k = dg[j] * POOL_WAVES + wave;
-            if (valid) at[j] = digit[k] + (uint32_t)__popcll(same & ((1ull << lane) - 1ull));  // (before this round)
-            wave_sync();
-            if (valid && (uint32_t)__ffsll((long long)same) - 1 == lane) digit[k] += (uint32_t)__popcll(same);
-            wave_sync();
+            at += (uint32_t)__popcll(own);
         }
-        __syncthreads();
-        {  // digit by digit and wavefront by wavefront: where they go
-            constexpr uint32_t EACH = (POOL_WAVES << POOL_DIGIT) / POOL_THREADS;
-            uint32_t c[EACH], sum = 0;
-#pragma unroll
-            for (uint32_t q = 0; q < EACH; q++) {
-                c[q] = digit[tid * EACH + q];
-                sum += c[q];
-            }
-            uint32_t x = block_excl_scan<uint32_t, POOL_WAVES>(sum, wsum, nullptr);
-#pragma unroll
-            for (uint32_t q = 0; q < EACH; q++) {
-                digit[tid * EACH + q] = x;
-                x += c[q];
-            }
-        }
-        __syncthreads();
-#pragma unroll
-        for (int j = 0; j < POOL_ITEMS; j++)
-            if (wave * POOL_RUN + j * 64 + lane < n)
-                (pass == 0 ? half : ord)[digit[dg[j] * POOL_WAVES + wave] + at[j]] = (uint16_t)item[j];
-        __syncthreads();
-    }
-    // starts of the signs in the order; the scales in the counters' place
-#pragma unroll
-    for (int j = 0; j < POOL_ITEMS; j++) {
-        const uint32_t i = wave * POOL_RUN + j * 64 + lane;
-        const bool head = i < n && (i == 0 || fo[ord[i]] != fo[ord[i - 1]]);
-        const unsigned long long m = __ballot(head);
-        if (lane == 0) heads[i >> 6] = m;
-        if (i < n) scale[i] = mine[j];
-    }
-    __syncthreads();
-    // pieces: every POOL_PIECE lookups of a sign
-    uint32_t starts = 0;
-#pragma unroll
-    for (int j = 0; j < POOL_ITEMS; j++) {
-        const uint32_t i = tid * POOL_ITEMS + j;
-        if (i < n && ((i - bit_at_or_below(heads, i)) % POOL_PIECE) == 0) starts |= 1u << j;
-    }
-    uint32_t pieces;
-    uint32_t k = block_excl_scan<uint32_t, POOL_WAVES>(__popc(starts), wsum, &pieces);
-#pragma unroll
-    for (int j = 0; j < POOL_ITEMS; j++)
-        if (starts & (1u << j)) piece[k++] = (uint16_t)(tid * POOL_ITEMS + j);
-    if (tid == 0) piece[pieces] = (uint16_t)n;
-    __syncthreads();
-    const float* pooled = d.grads;
-    const int sub = tid % LPG;
-    for (uint32_t q = tid / LPG; q < pieces; q += POOL_THREADS / LPG) {
-        const uint32_t lo = piece[q], hi = piece[q + 1];
-        float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
-        for (uint32_t j0 = lo; j0 < hi; j0 += 8) {  // eight rows in flight
-            float4 g[8];
-            float sc[8];
-#pragma unroll
-            for (uint32_t w = 0; w < 8; w++) {
-                const uint32_t i = ord[min(j0 + w, hi - 1)];
-                sc[w] = scale[i];
-                g[w] = row_part<ANY>(pooled + (uint64_t)xb[i] * dim, sub, D);
-            }
-#pragma unroll
-            for (uint32_t w = 0; w < 8; w++) {
-                if (j0 + w >= hi) break;
-                acc.x += g[w].x * sc[w];
-                acc.y += g[w].y * sc[w];
-                acc.z += g[w].z * sc[w];
-                acc.w += g[w].w * sc[w];
-            }
-        }
-        const uint32_t head = bit_at_or_below(heads, lo);
-        const bool whole = head == lo && (hi == n || ((heads[hi >> 6] >> (hi & 63)) & 1ull));
-        float* out = whole ? flat + (uint64_t)(d.lbase + fo[ord[lo]]) * dim : partial + (uint64_t)(d.lbase + q) * dim;
-        put_row_part<ANY>(out, sub, D, acc);
-    }
-    __syncthreads();
-    for (uint32_t q = tid / LPG; q < pieces; q += POOL_THREADS / LPG) {
-        const uint32_t lo = piece[q], hi = piece[q + 1];
-        if (bit_at_or_below(heads, lo) != lo || hi == n || ((heads[hi >> 6] >> (hi & 63)) & 1ull)) continue;
-        float4 acc = row_part<ANY>(partial + (uint64_t)(d.lbase + q) * dim, sub, D);
-        for (uint32_t r = q + 1; r < pieces; r++) {
-            const uint32_t at = piece[r];
-            if ((heads[at >> 6] >> (at & 63)) & 1ull) break;  // the next sign
-            const float4 g = row_part<ANY>(partial + (uint64_t)(d.lbase + r) * dim, sub, D);
-            acc.x += g.x;
-            acc.y += g.y;
-            acc.z += g.z;
-            acc.w += g.w;
-        }
-        put_row_part<ANY>(flat + (uint64_t)(d.lbase + fo[ord[lo]]) * dim, sub, D, acc);
+        pool_items<LPG, ANY>(lds, min(POOL_ITEMS_MAX, total - done), bits, d.grads, dim, D,
+                             [&](uint32_t key, bool first, bool& add) {
+                                 add = !first;
+                                 return flat + (uint64_t)(d.lbase + ((key << lp) | part)) * dim;
+                             });
     }
 }
 

@@ -121,8 +121,7 @@ struct SparseTable {
     hipEvent_t stage_ev = nullptr;  // staging buffer free again
     hipEvent_t verify_ev = nullptr; // a push's comparison of the signs has been published
     DevBuf comb_buf;                // slot descriptors of a combine op
-    DevBuf pooled_ws;               // scratch of a push of pooled gradients (ordered lookups, reduced rows)
-    size_t place_lds = 0;  // dynamic LDS of k_place_lookups on this device (0: not asked yet)
+    DevBuf pooled_ws;               // scratch of a push of pooled gradients (items of the lookups, reduced rows)
     // The path of few launches for small batches: the words in pinned memory its kernels report through (hwords: one
     // per workgroup of a small pull's first launch, or of a table-level pull's; hseq [0] a large pull's status is on the host, [1] a push's signs are
     // compared) with the numbers the host expects there next, the dynamic LDS its kernels may have.
@@ -842,7 +841,6 @@ void launch_grouping(const Plan& p, const Scratch& w, const PushSrc& src, int64_
 }
 
 constexpr int MASK_SLOTS = 128;
-constexpr uint32_t LONG_SEGMENT = 64;  // lookups of one distinct sign from which a workgroup sums them
 
 // The same result for the distinct signs of an op with at most MASK_SLOTS slots, from slot masks.  (Where the signs are not
 // grouped through LDS: a pull that does not wait for its stream, a push that analyses its batch itself.)
@@ -1191,31 +1189,31 @@ int launch_small_apply(SparseTable* t, RowShare share, const SmallPlan& p, const
     }
 }
 
+// LAUNCH(lanes, any) for the kernels that reduce pooled rows by pool_items: rows of up to 4, 8 or more elements; any: they do
+// not fill the lanes, or stand at other than 16-byte boundaries (row_part<true>).
+#define TN_POOL_LANES(LAUNCH, D, ALIGNED)                          \
+    do {                                                           \
+        const int lanes = (D) <= 4 ? 1 : (D) <= 8 ? 2 : 4;         \
+        const bool any = !(ALIGNED) || (D) % (4 * lanes) != 0;     \
+        if (any && lanes == 1) LAUNCH(1, true);                    \
+        else if (any && lanes == 2) LAUNCH(2, true);               \
+        else if (any) LAUNCH(4, true);                             \
+        else if (lanes == 1) LAUNCH(1, false);                     \
+        else if (lanes == 2) LAUNCH(2, false);                     \
+        else LAUNCH(4, false);                                     \
+    } while (0)
+
 // The gradients of a small push's distinct signs from pooled ones (k_small_pool).
-int launch_small_pool(SparseTable* t, RowShare share, const SmallPlan& p, int64_t batch, int dim, int combiner, float* flat,
-                      float* partial, hipStream_t st, uint32_t* host_err) {
+int launch_small_pool(SparseTable* t, bool aligned, const SmallPlan& p, int64_t batch, int dim, int combiner, float* flat,
+                      hipStream_t st, uint32_t* host_err) {
     static_assert((int)POOL_SUM == (int)COMBINE_SUM && (int)POOL_MEAN == (int)COMBINE_MEAN && (int)POOL_SQRTN == (int)COMBINE_SQRTN, "");
     const SmallShape& b = t->small_shape;
-#define TN_LAUNCH_POOL_ANY(LPG, ANY)                                                                                 \
-    TN_LAUNCH((k_small_pool<LPG, ANY>), dim3(b.N), dim3(POOL_THREADS), st, b, p, p.push_descs, batch, dim, t->store.D, \
-              combiner, flat, partial, t->dplan, host_err)
-#define TN_LAUNCH_POOL(LPG)                  \
-    do {                                     \
-        if (share.any)                       \
-            TN_LAUNCH_POOL_ANY(LPG, true);   \
-        else                                 \
-            TN_LAUNCH_POOL_ANY(LPG, false);  \
-    } while (0)
-    switch (share.lanes) {
-        case 1: TN_LAUNCH_POOL(1); break;
-        case 2: TN_LAUNCH_POOL(2); break;
-        case 4: TN_LAUNCH_POOL(4); break;
-        case 8: TN_LAUNCH_POOL(8); break;
-        case 16: TN_LAUNCH_POOL(16); break;
-        default: TN_LAUNCH_POOL(32); break;
-    }
+    const uint32_t lp = small_pool_parts_log2(b.max_len);
+#define TN_LAUNCH_POOL(LPG, ANY)                                                                                           \
+    TN_LAUNCH((k_small_pool<LPG, ANY>), dim3((uint32_t)b.N << lp), dim3(POOL_THREADS), st, b, p, p.push_descs, batch, dim, \
+              t->store.D, combiner, flat, t->dplan, host_err, lp)
+    TN_POOL_LANES(TN_LAUNCH_POOL, t->store.D, aligned);
 #undef TN_LAUNCH_POOL
-#undef TN_LAUNCH_POOL_ANY
     return TN_OK;
 }
 
@@ -1476,12 +1474,10 @@ int small_push(SparseTable* t, const int64_t* const* values, const float* const*
     const bool pooled = example_ids != nullptr, clicks = t->opt->kind == OPT_ADAGRAD;  // (the only optimizer that reads batch_click)
     SmallPlan p{};
     carve_small((char*)t->plan_buf.p, p, b);
-    float *flat = nullptr, *partial = nullptr;
+    float* flat = nullptr;
     if (pooled) {
-        TN_TRY(t->pooled_ws.ensure(2 * align_up((size_t)b.L * dim * sizeof(float), 256)));
-        Carver c{(char*)t->pooled_ws.p};
-        flat = c.take<float>((size_t)b.L * dim);
-        partial = c.take<float>((size_t)b.L * dim);
+        TN_TRY(t->pooled_ws.ensure(align_up((size_t)b.L * dim * sizeof(float), 256)));
+        flat = (float*)t->pooled_ws.p;
     }
     if (t->stage_pending) {
         TN_HIP(hipEventSynchronize(t->stage_ev));
@@ -1514,8 +1510,7 @@ int small_push(SparseTable* t, const int64_t* const* values, const float* const*
                   t->dplan, &t->hpush->st.mismatch);
     const bool rows16 = dim % 4 == 0 && t->store.wstride % 4 == 0;
     if (pooled)
-        TN_TRY(launch_small_pool(t, row_share(t->store, vec && rows16), p, batch, dim, combiner, flat, partial, st,
-                                 &t->hpush->st.abort));
+        TN_TRY(launch_small_pool(t, vec, p, batch, dim, combiner, flat, st, &t->hpush->st.abort));
     TN_TRY(launch_small_apply(t, row_share(t->store, (pooled || vec) && rows16), p, flat, dim, st, t->hseq + 1, seq));
     // what a call on another stream has to wait for: the updates are still running when this call returns
     TN_HIP(hipEventRecord(t->tail_ev, st));
@@ -2396,70 +2391,48 @@ int push_op_impl(uint32_t table_handle, int N, const int64_t* const* values, con
         return TN_OK;
     };
     // Where the apply kernels find the gradient of a record.  Pooled gradients are first reduced
-    // to one row per distinct sign: stable sort of (distinct index, position) pairs, then one
-    // ordered sum per distinct index.
+    // to one row per distinct sign.
     PushSrc src{};
     const uint32_t* pub_ubase = nullptr;  // a push on the pull's plan publishes its own copy of the distinct counts
     auto prepare_src = [&]() -> int {
         src = op_source(p, grad_dim, pd == p.push_descs);
         if (!pooled) return TN_OK;
-        if (!t->place_lds) t->place_lds = big_lds_bytes_for(reinterpret_cast<const void*>(k_place_lookups));
+        size_t max_len = 0;
+        for (int s = 0; s < N; s++) max_len = std::max<size_t>(max_len, (size_t)value_lens[s]);
+        const PoolShare share{PoolShare::parts_log2((uint32_t)max_len)};
+        const uint32_t tiles = PoolShare::first_tile((uint32_t)N, (uint32_t)L);
+        const uint32_t blocks = (PoolShare::first_part((uint32_t)N, (uint32_t)L) + XCDS - 1) / XCDS * XCDS;
         Carver c{nullptr};
-        uint32_t *long_count, *gcur, *seg_off, *tpos, *mid_list, *huge_list;
-        uint64_t *vals, *svals;
-        float* flat;
+        uint2* pool;
+        uint16_t* poff;
+        float *flat, *shares;
+        uint64_t* has;
+        const bool spread = PoolShare::spread(share.lp_max) != 0;
         auto carve = [&](Carver& cv) {
-            long_count = cv.take<uint32_t>(4);  // [1], [2]: entries of the lists of k_place_lookups (mid, huge)
-            mid_list = cv.take<uint32_t>(L / ORDER_MID + 1);
-            huge_list = cv.take<uint32_t>(L / ORDER_HUGE + 1);
-            gcur = cv.take<uint32_t>(L);
-            tpos = cv.take<uint32_t>(L);
-            vals = cv.take<uint64_t>(L);
-            svals = cv.take<uint64_t>(L);
-            seg_off = cv.take<uint32_t>(L + 1);
+            pool = cv.take<uint2>(L);
+            poff = cv.take<uint16_t>((size_t)tiles * ((1u << share.lp_max) + 1));
             flat = cv.take<float>(L * (size_t)grad_dim);
+            shares = cv.take<float>(spread ? (size_t)blocks * POOL_SPREAD * grad_dim : 0);
+            has = cv.take<uint64_t>(spread ? blocks : 0);
         };
         carve(c);
         TN_TRY(t->pooled_ws.ensure(align_up(c.off, 256)));
         Carver c2{(char*)t->pooled_ws.p};
         carve(c2);
-        TN_LAUNCH(k_lookup_keys, dim3(launch_grid((int64_t)(L + KEY_TILE - 1) / KEY_TILE, 1, GRID_CAP * 2)), dim3(256), st, pd, p.lbase, N, (uint32_t)L, batch, vals, ds, long_count);
-        // The lookups of every distinct sign side by side, ascending by example (= by position): into their
-        // sign's segment first, then ordered inside it.  A few workgroups per slot, each with an LDS counter per
-        // distinct index of its share of the slot (a slot has at most as many as lookups).
-        size_t max_len = 0;
-        for (int s = 0; s < N; s++) max_len = std::max<size_t>(max_len, (size_t)value_lens[s]);
-        // Workgroups per slot: about 200 in all, where the chip is filled (each streams its slot's lookups, so more of them
-        // read more: 100 slots of 49 k lookups 135 / 125 / 163 / 240 us with 1 / 2 / 4 / 8 per slot, 20 of 120 k 602 / 155 /
-        // 150 / 144 / 211 with 1 .. 16, 3 of 120 k 461 / 115 / 103 / 96 / 89); a share whose counters may not fit into LDS
-        // is the slow one.
-        const size_t counters = t->place_lds / sizeof(uint32_t);
-        const uint32_t parts = (uint32_t)std::min<size_t>(16, std::max<size_t>({1, 200 / (size_t)N, (max_len + counters - 1) / counters}));
-        const size_t place_bytes = std::min(t->place_lds, align_up((max_len / parts + 2) * sizeof(uint32_t), 256));
-        const uint32_t place_cap = (uint32_t)(place_bytes / sizeof(uint32_t));
-        TN_LAUNCH_LDS(k_place_lookups, dim3(N * parts), dim3(PLACE_THREADS), place_bytes, st, p.lbase, p.ubase, N, (uint32_t)L,
-                      p.u_of_gi, tpos, seg_off, gcur, place_cap, mid_list, huge_list, long_count, ds, parts);
-        const uint32_t room = (uint32_t)order_huge_room(max_len);
-        const uint32_t huge_blocks = (uint32_t)launch_grid((int64_t)L / ORDER_HUGE + 1, 1, ORDER_HUGE_GRID);
-        const uint32_t mid_blocks = (uint32_t)launch_grid((int64_t)L / ORDER_MID + 1, 1, ORDER_MID_GRID);
-        TN_LAUNCH_LDS(k_order_segments, dim3(huge_blocks + mid_blocks + launch_grid(L, 256, GRID_CAP * 4)), dim3(256),
-                      order_lds(room), st, (uint32_t)L, p.lbase, p.ubase, N, p.u_of_gi, mid_list, huge_list, long_count, seg_off,
-                      vals, tpos, svals, room, huge_blocks, mid_blocks, ds);
-        // signs with LONG_SEGMENT lookups or more get a workgroup each instead of one thread group
-        static_assert(LONG_SEGMENT == ORDER_MID, "the lists of k_place_lookups are the frequent signs of reduce_long");
-        const int chunks = (grad_dim + 3) / 4;
-        const bool with_long = chunks <= 256;
-        const uint32_t long_blocks = with_long ? (uint32_t)launch_grid((int64_t)L / LONG_SEGMENT + 1, 1, GRID_CAP) : 0;
-        // (a macro: the profiler names a kernel by the text of its launch)
-#define TN_REDUCE(ANY)                                                                                                 \
-    TN_LAUNCH((k_reduce_pooled<ANY>), dim3(long_blocks + launch_grid((int64_t)L * chunks, 256, GRID_CAP * 4)), dim3(256), \
-              st, pd, p.ubase, N, grad_dim, combiner, ds, seg_off, svals, flat, with_long ? LONG_SEGMENT : 0xFFFFFFFFu,  \
-              mid_list, huge_list, long_count, long_blocks)
-        if (vec)
-            TN_REDUCE(false);
-        else
-            TN_REDUCE(true);
+        TN_LAUNCH_LDS(k_lookup_keys, dim3(tiles), dim3(256), pool_tile_lds(share.lp_max), st, pd, p.lbase, p.ubase, (uint32_t)N,
+                      p.u_of_gi, batch, pool, poff, share, ds);
+#define TN_REDUCE(LPG, ANY)                                                                                                \
+    TN_LAUNCH((k_reduce_pooled<LPG, ANY>), dim3(blocks), dim3(POOL_THREADS), st, pd, p.lbase, p.ubase, (uint32_t)N, pool,  \
+              poff, grad_dim, t->store.D, combiner, ds, flat, share, shares, has)
+        TN_POOL_LANES(TN_REDUCE, t->store.D, vec);
 #undef TN_REDUCE
+        if (spread) {
+#define TN_REDUCE(LPG, ANY)                                                                                                \
+    TN_LAUNCH((k_reduce_pooled_shares<LPG, ANY>), dim3((uint32_t)N * (POOL_SPREAD / 4)), dim3(256), st, p.lbase, p.ubase,  \
+              grad_dim, t->store.D, ds, shares, has, flat, share)
+            TN_POOL_LANES(TN_REDUCE, t->store.D, grad_dim % 4 == 0);
+#undef TN_REDUCE
+        }
         src.flat = flat;
         return TN_OK;
     };
