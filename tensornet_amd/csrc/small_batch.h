@@ -25,7 +25,8 @@
 
 namespace tn {
 
-constexpr int SMALL_SLOT_MAX = 4096;         // lookups of a slot at most
+constexpr int SMALL_SLOT_MAX = 8192;         // lookups of a slot at most
+constexpr int SMALL_SLOT_SHORT = 4096;       // ... that a workgroup of SMALL_THREADS holds in registers
 constexpr int SMALL_SLOT_BITS = 13;          // a position in a slot, its rank, its occurrences fit in 13, 13 and 14 bits
 constexpr int SMALL_SLOTS = 512;             // slots at most (the LDS of small_emit_bucket: 300 slots of 2912 lookups, 512 of 576)
 constexpr int SMALL_PARTS_MAX = 16;          // workgroups of k_small_slots per slot at most
@@ -34,13 +35,13 @@ constexpr int SMALL_WORKGROUPS = SMALL_SLOTS > SMALL_SEGMENTS ? SMALL_SLOTS : SM
 constexpr int SMALL_PART_LOOKUPS = 128;      // lookups of a slot per workgroup aimed at
 constexpr int SMALL_BUCKET_RECORDS = 64;     // records per bucket aimed at (if every lookup were distinct)
 constexpr int SMALL_BUCKETS_MAX = 2048;
-constexpr int SMALL_THREADS = 512;           // k_small_slots
-constexpr int SMALL_ITEMS = SMALL_SLOT_MAX / SMALL_THREADS;
+constexpr int SMALL_THREADS = 512;           // k_small_slots; twice as many for slots of more than SMALL_SLOT_SHORT lookups
+constexpr int SMALL_ITEMS = SMALL_SLOT_SHORT / SMALL_THREADS;
 constexpr int SMALL_WORDS = SMALL_SLOT_MAX / 64;  // 64-lookup words of a slot
 constexpr int SMALL_NEW = 512;               // rows a workgroup of k_small_slots lists to fill them with all its threads
 constexpr int FINISH_THREADS = 256;          // k_small_group_finish
 constexpr int SMALL_TILE = 1024;             // lookups per workgroup of k_small_verify
-static_assert(SMALL_SLOT_MAX < (1 << SMALL_SLOT_BITS), "positions fit");
+static_assert(SMALL_SLOT_MAX <= (1 << SMALL_SLOT_BITS) && SMALL_SLOT_MAX == 2 * SMALL_SLOT_SHORT, "positions fit");
 
 // How a small batch is laid out: worked out by the pull, kept with its plan.
 struct SmallShape {
@@ -101,9 +102,10 @@ inline size_t small_slots_lds(uint32_t entries, uint32_t max_len, uint32_t nbp) 
 // and then took a share of the probes repeated the slot's remap up to eight times).  What bounds it is a chain of
 // round trips -- descriptor, signs, probe, second probe -- and a CU's rate of random 64-byte reads (0.2 per ns), hence
 // many workgroups with about a hundred signs each.
-__global__ __launch_bounds__(SMALL_THREADS) void k_small_slots(SmallShape b, SmallPlan p, const SlotDesc* host_descs,
-                                                               uint32_t entries, Store s, OptDev o, uint64_t seed,
-                                                               DevStatus* status, uint64_t* host_words, uint32_t seq) {
+template <int THREADS>
+__device__ __forceinline__ void small_slots(const SmallShape& b, const SmallPlan& p, const SlotDesc* host_descs, uint32_t entries,
+                                            const Store& s, const OptDev& o, uint64_t seed, DevStatus* status,
+                                            uint64_t* host_words, uint32_t seq) {
     extern __shared__ unsigned long long smem64[];
     unsigned long long* keys = smem64;
     uint32_t* word = reinterpret_cast<uint32_t*>(keys + entries + 1);  // bits 16-31 smallest position, 0-15 occurrences
@@ -111,7 +113,7 @@ __global__ __launch_bounds__(SMALL_THREADS) void k_small_slots(SmallShape b, Sma
     uint16_t* used = reinterpret_cast<uint16_t*>(hist + b.nbp + 1);   // [max_len]: the entries in use
     __shared__ SlotDesc sd;
     __shared__ unsigned long long bits[SMALL_WORDS];
-    __shared__ uint32_t wsum[SMALL_THREADS / 64];
+    __shared__ uint32_t wsum[THREADS / 64];
     __shared__ uint32_t sh_first, sh_new, sh_full;
     __shared__ uint32_t new_row[SMALL_NEW];
     __shared__ uint16_t new_ent[SMALL_NEW];
@@ -122,12 +124,12 @@ __global__ __launch_bounds__(SMALL_THREADS) void k_small_slots(SmallShape b, Sma
     // while the tables are cleared)
     uint32_t dword = 0;
     if (tid < sizeof(SlotDesc) / 4) dword = reinterpret_cast<const uint32_t*>(host_descs + sl)[tid];
-    for (uint32_t i = tid; i <= entries; i += SMALL_THREADS) {
+    for (uint32_t i = tid; i <= entries; i += THREADS) {
         keys[i] = EMPTY_KEY;
         word[i] = 0xFFFF0000u;
     }
-    for (uint32_t i = tid; i <= b.nbp; i += SMALL_THREADS) hist[i] = 0;
-    for (uint32_t i = tid; i < SMALL_WORDS; i += SMALL_THREADS) bits[i] = 0;
+    for (uint32_t i = tid; i <= b.nbp; i += THREADS) hist[i] = 0;
+    for (uint32_t i = tid; i < SMALL_WORDS; i += THREADS) bits[i] = 0;
     if (tid == 0) sh_first = sh_new = sh_full = 0;
     if (blockIdx.x == 0) {
         if (tid < sizeof(DevStatus) / 4) reinterpret_cast<uint32_t*>(status)[tid] = 0;
@@ -143,14 +145,14 @@ __global__ __launch_bounds__(SMALL_THREADS) void k_small_slots(SmallShape b, Sma
     uint64_t sg[SMALL_ITEMS];
 #pragma unroll
     for (int j = 0; j < SMALL_ITEMS; j++) {
-        const uint32_t pos = j * SMALL_THREADS + tid;
+        const uint32_t pos = j * THREADS + tid;
         sg[j] = pos < len ? (uint64_t)values[pos] : 0;
     }
     // the lookups of my share: entry of the sign, smallest position
     uint32_t ent[SMALL_ITEMS];
 #pragma unroll
     for (int j = 0; j < SMALL_ITEMS; j++) {
-        const uint32_t pos = j * SMALL_THREADS + tid;
+        const uint32_t pos = j * THREADS + tid;
         ent[j] = 0xFFFFFFFFu;
         if (pos >= len) continue;
         if (part == 0) p.vals_copy[lbase + pos] = sg[j];
@@ -173,7 +175,7 @@ __global__ __launch_bounds__(SMALL_THREADS) void k_small_slots(SmallShape b, Sma
 #pragma unroll
     for (int j = 0; j < SMALL_ITEMS; j++) {
         if (ent[j] == 0xFFFFFFFFu) continue;
-        const uint32_t pos = j * SMALL_THREADS + tid;
+        const uint32_t pos = j * THREADS + tid;
         const uint32_t f = atomicAdd(&word[ent[j]], 1u) >> 16;
         p.first_of[lbase + pos] = (uint16_t)f;
         if (f == pos) {
@@ -189,7 +191,7 @@ __global__ __launch_bounds__(SMALL_THREADS) void k_small_slots(SmallShape b, Sma
     uint32_t row[SMALL_ITEMS], place[SMALL_ITEMS], bk[SMALL_ITEMS];
 #pragma unroll
     for (int r = 0; r < SMALL_ITEMS; r++) {
-        const uint32_t i = r * SMALL_THREADS + tid;
+        const uint32_t i = r * THREADS + tid;
         row[r] = NO_ROW;
         place[r] = bk[r] = 0;
         if (i < n_first) {
@@ -220,10 +222,10 @@ __global__ __launch_bounds__(SMALL_THREADS) void k_small_slots(SmallShape b, Sma
     }
     // where the buckets start among the part's records
     uint32_t at = 0;
-    for (uint32_t i0 = 0; i0 < b.nbp; i0 += SMALL_THREADS) {
+    for (uint32_t i0 = 0; i0 < b.nbp; i0 += THREADS) {
         const uint32_t c = i0 + tid < b.nbp ? hist[i0 + tid] : 0u;
         uint32_t total;
-        const uint32_t x = at + block_excl_scan<uint32_t, SMALL_THREADS / 64>(c, wsum, &total);
+        const uint32_t x = at + block_excl_scan<uint32_t, THREADS / 64>(c, wsum, &total);
         if (i0 + tid < b.nbp) {
             hist[i0 + tid] = x;
             p.boff[(size_t)blockIdx.x * (b.nbp + 1) + i0 + tid] = (uint16_t)x;
@@ -235,7 +237,7 @@ __global__ __launch_bounds__(SMALL_THREADS) void k_small_slots(SmallShape b, Sma
     const uint32_t rbase = b.parts * lbase + part * len;
 #pragma unroll
     for (int r = 0; r < SMALL_ITEMS; r++) {
-        const uint32_t i = r * SMALL_THREADS + tid;
+        const uint32_t i = r * THREADS + tid;
         if (i < n_first) {
             const uint32_t w = word[used[i]], pos = w >> 16, cnt = w & 0xFFFFu;
             // batch_show = occurrences (sparse_table_ops.cc:290-293)
@@ -244,15 +246,26 @@ __global__ __launch_bounds__(SMALL_THREADS) void k_small_slots(SmallShape b, Sma
             p.click_at[lbase + pos] = 0;
         }
     }
-    for (uint32_t i = tid; i < b.words; i += SMALL_THREADS) p.bits[(size_t)blockIdx.x * b.words + i] = bits[i];
+    for (uint32_t i = tid; i < b.words; i += THREADS) p.bits[(size_t)blockIdx.x * b.words + i] = bits[i];
     if (sh_new) {
         const uint32_t pairs = (uint32_t)(s.D + 1) / 2, work = min(sh_new, (uint32_t)SMALL_NEW) * pairs;
         const float stddev = (float)(1.0 / sqrt((double)s.D));
-        for (uint32_t q = tid; q < work; q += SMALL_THREADS) {
+        for (uint32_t q = tid; q < work; q += THREADS) {
             const uint32_t k = q / pairs;
             init_row_pair(s, o, seed, (uint64_t)keys[new_ent[k]], new_row[k], q - k * pairs, stddev);
         }
     }
+}
+
+__global__ __launch_bounds__(SMALL_THREADS) void k_small_slots(SmallShape b, SmallPlan p, const SlotDesc* host_descs,
+                                                               uint32_t entries, Store s, OptDev o, uint64_t seed,
+                                                               DevStatus* status, uint64_t* host_words, uint32_t seq) {
+    small_slots<SMALL_THREADS>(b, p, host_descs, entries, s, o, seed, status, host_words, seq);
+}
+__global__ __launch_bounds__(2 * SMALL_THREADS) void k_small_slots_long(SmallShape b, SmallPlan p, const SlotDesc* host_descs,
+                                                                        uint32_t entries, Store s, OptDev o, uint64_t seed,
+                                                                        DevStatus* status, uint64_t* host_words, uint32_t seq) {
+    small_slots<2 * SMALL_THREADS>(b, p, host_descs, entries, s, o, seed, status, host_words, seq);
 }
 
 // What is left of a small pull behind its first launch: small_emit_bucket, a workgroup per bucket, and small_finish.
@@ -411,18 +424,21 @@ __device__ __forceinline__ void small_finish(const SmallShape& b, const SmallPla
         f[j] = q < todo ? p.first_of[d.lbase + pos[j]] : NO_ROW;
         row[j] = q < todo ? p.row_at[d.lbase + pos[j]] : NO_ROW;  // (of a first lookup only)
     }
-    {  // the parts' first lookups: a wavefront takes every WAVES-th part, then one puts them together
-        const uint64_t* w = p.bits + (size_t)sl * b.parts * b.words + lane;
+    // the parts' first lookups: a wavefront takes every WAVES-th part, then one puts them together
+    constexpr uint32_t RUNS = SMALL_WORDS / 64;
+#pragma unroll
+    for (uint32_t r = 0; r < RUNS; r++) {
+        const uint64_t* w = p.bits + (size_t)sl * b.parts * b.words + r * 64 + lane;
         uint64_t v[SMALL_PARTS_MAX / WAVES];
 #pragma unroll
         for (uint32_t k = 0; k < SMALL_PARTS_MAX / WAVES; k++) {
             const uint32_t q = k * WAVES + wave;
-            v[k] = q < b.parts && lane < b.words ? w[(size_t)q * b.words] : 0ull;
+            v[k] = q < b.parts && r * 64 + lane < b.words ? w[(size_t)q * b.words] : 0ull;
         }
         uint64_t all = 0;
 #pragma unroll
         for (uint32_t k = 0; k < SMALL_PARTS_MAX / WAVES; k++) all |= v[k];
-        part_bits[wave][lane] = all;
+        part_bits[wave][r * 64 + lane] = all;
     }
     float4 v4[FINISH_ITEMS];
     float v1[FINISH_ITEMS];
@@ -441,18 +457,22 @@ __device__ __forceinline__ void small_finish(const SmallShape& b, const SmallPla
     }
     __syncthreads();
     if (wave == 0) {
-        unsigned long long v = 0;
-        for (uint32_t q = 0; q < WAVES; q++) v |= part_bits[q][lane];
-        const uint32_t n = (uint32_t)__popcll(v);
-        uint32_t inc = n;
-        for (int x = 1; x < 64; x <<= 1) {
-            const uint32_t y = __shfl_up(inc, x);
-            if ((int)lane >= x) inc += y;
+        uint32_t done = 0;
+#pragma unroll
+        for (uint32_t r = 0; r < RUNS; r++) {
+            unsigned long long v = 0;
+            for (uint32_t q = 0; q < WAVES; q++) v |= part_bits[q][r * 64 + lane];
+            const uint32_t n = (uint32_t)__popcll(v);
+            uint32_t inc = n;
+            for (int x = 1; x < 64; x <<= 1) {
+                const uint32_t y = __shfl_up(inc, x);
+                if ((int)lane >= x) inc += y;
+            }
+            bits[r * 64 + lane] = v;
+            before[r * 64 + lane] = done + inc - n;
+            done += __shfl(inc, 63);
         }
-        bits[lane] = v;
-        before[lane] = inc - n;
     }
-    static_assert(SMALL_WORDS == 64, "one wavefront scans the words");
     __syncthreads();
 #pragma unroll
     for (int j = 0; j < FINISH_ITEMS; j++) {
@@ -678,7 +698,8 @@ struct SmallGroup {
 // condition makes the compiler wait for all loads where the branches join.
 // grp: the sign's records -- entry(j) of the j-th (what is fetched ahead), its gradient row (nullptr: it has none) and
 // counts, taken(k, sub, lanes) once all have been applied.
-template <int KIND, int LPG, bool ANY, int AHEAD, typename Group>
+// ONCE: the caller says that k <= AHEAD, so nothing is fetched ahead (and registers for 32 words are free).
+template <int KIND, int LPG, bool ANY, int AHEAD, bool ONCE, typename Group>
 __device__ __forceinline__ void apply_group_ahead(const Store& s, const OptDev& o, const Group& grp, uint32_t row, uint32_t k,
                                                   int sub, int lane0, float c1, float c2) {
     typedef typename Group::Entry Entry;
@@ -718,15 +739,19 @@ __device__ __forceinline__ void apply_group_ahead(const Store& s, const OptDev& 
 #pragma unroll
     for (int q = 0; q < AHEAD; q++) {
         m1[q] = grp.entry(min((uint32_t)q, k - 1));
-        m2[q] = grp.entry(min((uint32_t)(AHEAD + q), k - 1));
+        if (!ONCE) m2[q] = grp.entry(min((uint32_t)(AHEAD + q), k - 1));
     }
     fetch(m1, 0, g0, sh0, ck0, ok0);
+    if (!ONCE) {
 #pragma unroll
-    for (int q = 0; q < AHEAD; q++) m1[q] = m2[q];
-    for (uint32_t c0 = 0; c0 < k; c0 += AHEAD) {
+        for (int q = 0; q < AHEAD; q++) m1[q] = m2[q];
+    }
+    for (uint32_t c0 = 0; c0 < (ONCE ? 1 : k); c0 += AHEAD) {
+        if (!ONCE) {
 #pragma unroll
-        for (int q = 0; q < AHEAD; q++) m2[q] = grp.entry(min(c0 + 2 * AHEAD + q, k - 1));
-        fetch(m1, c0 + AHEAD, g1, sh1, ck1, ok1);
+            for (int q = 0; q < AHEAD; q++) m2[q] = grp.entry(min(c0 + 2 * AHEAD + q, k - 1));
+            fetch(m1, c0 + AHEAD, g1, sh1, ck1, ok1);
+        }
         if constexpr (KIND == OPT_ADAGRAD) {
             // The records of the window depend on each other through g2sum (one rounded addition per record) and
             // through the row (one subtraction per element and record) only.  Everything else -- the sums of squares
@@ -793,6 +818,7 @@ __device__ __forceinline__ void apply_group_ahead(const Store& s, const OptDev& 
                 }
             }
         }
+        if (ONCE) break;
 #pragma unroll
         for (int q = 0; q < AHEAD; q++) {
             g0[q] = g1[q];
@@ -820,6 +846,271 @@ __device__ __forceinline__ void apply_group_ahead(const Store& s, const OptDev& 
     }
 }
 
+// One sign with many records by a wavefront, rows of D elements, D a power of two up to 64.  A small batch's updates are as
+// long as their longest sign (its records: one per slot), so this is made for the length of the chain: what the chain itself
+// does not need is worked out for all records of a chunk side by side.  The lanes tile (record, element) as lane = record * D +
+// element, R records a round, and hold the gradients of a chunk's rounds in registers, all loads in flight; the next chunk's
+// are on their way while this one's records are applied, its member entries a chunk before that.  In LDS, a lane per
+// element walks the records in their order three times at most, with what depends on the record before only:
+//   AdaGrad  g2sum (a lane per record, double sum of squares first) | steps lr g / den by all lanes | subtractions
+//   Adam     m and v | steps lr m / (eps + sqrt(v)) by all lanes | subtractions
+//   Ftrl     n | sqrt(n), the quotient of the weight and the factor of z by all lanes | z and w
+// The same operations on the same operands as record after record.  300 slots of 300 lookups, AdaGrad rows of 32 (signs with
+// 300 records): k_small_apply 78 -> 60 us; 40 slots of 8192, Ftrl rows of 1: 32 -> 26.
+template <int KIND, int D>
+struct BigWave {
+    static constexpr int R = 64 / D, DP = D + 1;  // records a round; padded row: lanes walking down a column hit different banks
+    static constexpr int BUFS = KIND == OPT_ADAGRAD ? 1 : KIND == OPT_ADAM ? 2 : 3;
+    static constexpr int fit(int chunk) {
+        return chunk > R && (chunk * DP * BUFS > 2304 || chunk > 16 * R) ? fit(chunk / 2) : chunk;
+    }
+    static constexpr int CHUNK = fit(64), ROUNDS = CHUNK / R;
+    static_assert(CHUNK >= R && CHUNK % R == 0, "whole rounds");
+    float buf[BUFS][CHUNK * DP];  // gradients, then steps (Ftrl: gradients) | Adam v, Ftrl n, then its factor | Ftrl quotient
+    const float* gptr[CHUNK];
+    float den[CHUNK];
+};
+
+// x0 + the sum of `v` over the lanes below n, added one after the other; many at once where that is exact (whole numbers).
+__device__ __forceinline__ float ordered_sum(float x0, int v, int n, unsigned long long okmask) {
+    if (n <= 16) {
+        const float few = (float)v;
+        for (int m = 0; m < n; m++)
+            if ((okmask >> m) & 1ull) x0 += lane_value(few, m);
+        return x0;
+    }
+    int all = v;
+#pragma unroll
+    for (int o = 1; o < 64; o *= 2) all += __shfl_xor(all, o);
+    const float most = 16777216.f;
+    if (x0 == truncf(x0) && x0 >= 0.f && x0 < most / 2 && all >= 0 && all < (1 << 23) && !__any(v < 0)) return x0 + (float)all;
+    const float f = (float)v;
+    for (int m = 0; m < n; m++)
+        if ((okmask >> m) & 1ull) x0 += lane_value(f, m);
+    return x0;
+}
+
+// The signs bi0, bi0 + stride, ... below n_big; head: {row, first member, records} of the first, describe(bi): of another;
+// entry(at): member `at`; record(entry, gradient, show, click): whether it has a gradient; missing(): one had none.
+template <int KIND, int D, typename Describe, typename Member, typename Record, typename Missing>
+__device__ __forceinline__ void apply_big_wave(const Store& s, const OptDev& o, BigWave<KIND, D>& lds, uint4 head, uint32_t bi0,
+                                               uint32_t stride, uint32_t n_big, Describe describe, Member entry, Record record,
+                                               Missing missing) {
+    using T = BigWave<KIND, D>;
+    constexpr int R = T::R, DP = T::DP, CHUNK = T::CHUNK, ROUNDS = T::ROUNDS;
+    float* const gbuf = lds.buf[0];
+    float* const vbuf = lds.buf[T::BUFS > 1 ? 1 : 0];
+    float* const qbuf = lds.buf[T::BUFS > 2 ? 2 : 0];
+    const int lane = (int)__lane_id(), li = lane & (D - 1), lm = lane / D;
+    const float c1 = 1 - o.beta1, c2 = 1 - o.beta2;
+    for (uint32_t bi = bi0; bi < n_big; bi += stride) {
+        if (bi != bi0) head = describe(bi);
+        const uint32_t row = head.x, off = head.y, k = head.z;
+        if (row > s.cap || k == 0) continue;  // NO_ROW, or no row number at all: never address the table with it
+        float* wp = s.w + (uint64_t)row * s.wstride;
+        float* sp = s.st + (uint64_t)row * s.sstride;
+        float w = lane < D ? wp[lane] : 0.f;
+        float a = 0.f, b = 0.f, show = 0.f, click = 0.f, g2sum = 0.f;
+        int delta_show = 0;
+        if (KIND == OPT_ADAGRAD) {
+            g2sum = sp[0];
+            show = sp[1];
+            click = sp[2];
+        } else {
+            a = lane < D ? sp[lane] : 0.f;
+            b = lane < D ? sp[D + lane] : 0.f;
+            delta_show = __float_as_int(sp[2 * D + 1]);
+        }
+        auto chunk_entry = [&](uint32_t c0) { return entry(off + min(c0 + (uint32_t)lane, k - 1)); };
+        auto now = chunk_entry(0);
+        auto next = chunk_entry(CHUNK);
+        float v[ROUNDS];
+        int sh = 0, ck = 0;
+        unsigned long long okmask = 0;
+        // gradients of the chunk from c0 on, whose entries are e, on their way
+        auto fetch = [&](uint32_t c0, const auto& e) {
+            const int cn = (int)min(k - c0, (uint32_t)CHUNK);
+            bool ok = false;
+            sh = ck = 0;
+            if (lane < cn) {
+                const float* gp = nullptr;
+                ok = record(e, gp, sh, ck);
+                lds.gptr[lane] = gp;
+            }
+            okmask = __ballot(ok);
+            if (!ok) sh = ck = 0;
+            wave_sync();
+#pragma unroll
+            for (int q = 0; q < ROUNDS; q++) {
+                const int m = lm + q * R;
+                v[q] = (m < cn && ((okmask >> m) & 1ull)) ? lds.gptr[m][li] : 0.f;
+            }
+        };
+        fetch(0, now);
+        bool any = false;
+        for (uint32_t c0 = 0; c0 < k; c0 += CHUNK) {
+            const int cn = (int)min(k - c0, (uint32_t)CHUNK), csh = sh, cck = ck;
+            const unsigned long long mask = okmask, all = cn == 64 ? ~0ull : (1ull << cn) - 1ull;
+#pragma unroll
+            for (int q = 0; q < ROUNDS; q++) gbuf[(lm + q * R) * DP + li] = v[q];
+            wave_sync();
+            if (c0 + CHUNK < k) {
+                now = next;
+                next = chunk_entry(c0 + 2 * CHUNK);
+                fetch(c0 + CHUNK, now);
+            }
+            if (KIND == OPT_ADAGRAD) {
+                // add_g2sum / dim of record `lane`: double sum of float products in element order
+                double mq = 0.0;
+                if (lane < cn) {
+                    const float* gr = gbuf + lane * DP;
+                    constexpr int AT_ONCE = D < 16 ? D : 16;
+                    double tot = 0.0;
+#pragma unroll
+                    for (int i0 = 0; i0 < D; i0 += AT_ONCE) {
+                        float x[AT_ONCE];
+#pragma unroll
+                        for (int i = 0; i < AT_ONCE; i++) x[i] = gr[i0 + i];
+#pragma unroll
+                        for (int i = 0; i < AT_ONCE; i++) tot += (double)(x[i] * x[i]);
+                    }
+                    mq = tot * (1.0 / (double)D);  // (exact: D is a power of two)
+                }
+                show = ordered_sum(show, csh, cn, mask);
+                click = ordered_sum(click, cck, cn, mask);
+                // g2sum after every record (float += double, rounded each time): every lane runs the chain on values read
+                // out of the records' lanes, lane m keeps the g2sum its record meets
+                float myg2 = 0.f;
+                for (int m0 = 0; m0 < cn; m0 += 8) {
+                    double x[8];
+#pragma unroll
+                    for (int j = 0; j < 8; j++) x[j] = lane_value(mq, min(m0 + j, 63));
+#pragma unroll
+                    for (int j = 0; j < 8; j++) {
+                        if (m0 + j < cn && ((mask >> (m0 + j)) & 1ull)) g2sum = (float)((double)g2sum + x[j]);
+                        if (lane == m0 + j) myg2 = g2sum;
+                    }
+                }
+                if (lane < cn) lds.den[lane] = o.eps + sqrtf(myg2);
+                wave_sync();
+#pragma unroll 4
+                for (int m = lm; m < cn; m += R) {  // a record without a gradient row steps by zero
+                    const float gv = gbuf[m * DP + li], dn = lds.den[m];
+                    gbuf[m * DP + li] = ((mask >> m) & 1ull) ? o.lr * gv / dn : 0.f;
+                }
+            } else {
+                int shown = csh;
+#pragma unroll
+                for (int x = 1; x < 64; x *= 2) shown += __shfl_xor(shown, x);
+                delta_show += shown;
+                const float n0 = b;
+                if (lane < D) {
+                    for (int m0 = 0; m0 < cn; m0 += 8) {
+                        float g[8];
+#pragma unroll
+                        for (int j = 0; j < 8; j++) g[j] = gbuf[min(m0 + j, cn - 1) * DP + lane];
+#pragma unroll
+                        for (int j = 0; j < 8; j++) {
+                            if (m0 + j >= cn) break;
+                            if ((mask >> (m0 + j)) & 1ull) {
+                                if (KIND == OPT_ADAM) {
+                                    a = o.beta1 * a + c1 * g[j];
+                                    b = o.beta2 * b + c2 * g[j] * g[j];
+                                } else {
+                                    b += g[j] * g[j];
+                                }
+                            }
+                            if (KIND == OPT_ADAM) gbuf[(m0 + j) * DP + lane] = a;
+                            vbuf[(m0 + j) * DP + lane] = b;
+                        }
+                    }
+                }
+                wave_sync();
+                if (KIND == OPT_ADAM) {
+#pragma unroll 4
+                    for (int m = lm; m < cn; m += R) {
+                        const float am = gbuf[m * DP + li], bm = vbuf[m * DP + li];
+                        gbuf[m * DP + li] = ((mask >> m) & 1ull) ? o.lr * am / (o.eps + sqrtf(bm)) : 0.f;
+                    }
+                } else {
+                    const float first = __shfl(n0, li);
+                    float t[ROUNDS];
+#pragma unroll
+                    for (int q = 0; q < ROUNDS; q++) {
+                        const int m = lm + q * R;
+                        t[q] = 0.f;
+                        if (m >= cn) continue;
+                        const float nm = vbuf[m * DP + li], before = m > 0 ? vbuf[(m - 1) * DP + li] : first, root = sqrtf(nm);
+                        t[q] = o.lr * (root - sqrtf(before));
+                        qbuf[m * DP + li] = -1 / ((o.beta + root) * o.lr + o.lambda2);
+                    }
+                    wave_sync();
+#pragma unroll
+                    for (int q = 0; q < ROUNDS; q++) {
+                        const int m = lm + q * R;
+                        if (m < cn) vbuf[m * DP + li] = t[q];
+                    }
+                }
+            }
+            wave_sync();
+            if (lane < D) {
+                for (int m0 = 0; m0 < cn; m0 += 8) {
+                    if (KIND != OPT_FTRL) {
+                        float t[8];
+#pragma unroll
+                        for (int j = 0; j < 8; j++) t[j] = m0 + j < cn ? gbuf[(m0 + j) * DP + lane] : 0.f;
+#pragma unroll
+                        for (int j = 0; j < 8; j++) w -= t[j];
+                    } else {
+                        float g[8], t[8], f[8];
+#pragma unroll
+                        for (int j = 0; j < 8; j++) {
+                            const int at = min(m0 + j, cn - 1) * DP + lane;
+                            g[j] = gbuf[at];
+                            t[j] = vbuf[at];
+                            f[j] = qbuf[at];
+                        }
+#pragma unroll
+                        for (int j = 0; j < 8; j++) {
+                            if (m0 + j >= cn || !((mask >> (m0 + j)) & 1ull)) continue;
+                            a += g[j] - t[j] * w;
+                            const float z = a > 0 ? a - o.lambda1 : a + o.lambda1;
+                            w = fabsf(a) <= o.lambda1 ? 0.f : f[j] * z;
+                        }
+                    }
+                }
+            }
+            if (mask) any = true;
+            if (lane == 0 && mask != all) missing();
+            wave_sync();
+        }
+        if (any) {
+            if (lane < D) {
+                wp[lane] = w;
+                if (KIND != OPT_ADAGRAD) {
+                    sp[lane] = a;
+                    sp[D + lane] = b;
+                }
+            }
+            if (lane == 0) {
+                if (KIND == OPT_ADAGRAD) {
+                    sp[0] = g2sum;
+                    sp[1] = show;
+                    sp[2] = click;
+                    sp[3] = 0.f;  // no_show_days = 0
+                    if (o.use_cvm) {
+                        wp[D] = show;
+                        wp[D + 1] = logf(click + 1) - logf(show + 1);
+                    }
+                } else {
+                    sp[2 * D + 1] = __int_as_float(delta_show);
+                }
+            }
+        }
+        wave_sync();
+    }
+}
+
 // Bytes of dynamic LDS of k_small_apply when its launch includes the workgroups for the signs with many records:
 // per wavefront the staging and the row of apply_big_groups, then its pointer, count, flag and divisor arrays.
 inline size_t small_apply_wave_lds(int D) { return align_up(big_lds_bytes(D), 8) + BIG_CHUNK * (8 + 4); }
@@ -842,7 +1133,10 @@ __device__ __forceinline__ uint32_t wave_draw(uint32_t* counter) {
 // several records of a sign in flight, then those with one.  Nothing is reported to the host but that this kernel runs,
 // which tells it that the comparison of the signs, launched before, is complete: on the plan of the last pull every sign has
 // its row, and the host has compared the slots' distinct counts with the rows of the gradient matrices itself.
-template <int KIND, int LPG, bool ANY>
+// BIG: how the signs with many records are applied -- BIG_NONE, the plan lists none; BIG_GROUPS, rows of any length
+// (apply_big_groups); else rows of as many elements (apply_big_wave).
+enum { BIG_NONE = 0, BIG_GROUPS = -1 };
+template <int KIND, int LPG, bool ANY, int BIG>
 __global__ __launch_bounds__(256) void k_small_apply(SmallShape b, SmallPlan p, const float* flat, Store s,
                                                      OptDev o, const DevStatus* __restrict__ status, uint32_t* host_seq,
                                                      uint32_t seq, int dim, int gbuf_floats, uint32_t wave_lds,
@@ -853,6 +1147,7 @@ __global__ __launch_bounds__(256) void k_small_apply(SmallShape b, SmallPlan p, 
     const uint32_t c = blockIdx.x;
     const size_t first = (size_t)c * b.cap;
     const uint4 head = p.head[c];
+    const uint2 big0 = p.group[first + b.cap - 1 - (threadIdx.x >> 6)];  // (if there are so many: one round trip less)
     const uint32_t stop = status->mismatch | status->abort;
     const float** grads = reinterpret_cast<const float**>(apply_lds);
     uint32_t* rows = reinterpret_cast<uint32_t*>(grads + (flat ? 0 : b.N));
@@ -874,7 +1169,22 @@ __global__ __launch_bounds__(256) void k_small_apply(SmallShape b, SmallPlan p, 
     src.dim = dim;
     const float c1 = 1 - o.beta1, c2 = 1 - o.beta2;
     const int wave = (int)(threadIdx.x >> 6), lane = (int)(threadIdx.x & 63), sub = lane % LPG, lane0 = lane - sub;
-    if (head.z) {
+    auto describe = [](uint2 g) { return make_uint4(g.x, g.y & 0xFFFFu, g.y >> 16, 0u); };
+    auto group = [&](uint32_t bi) { return describe(p.group[first + b.cap - 1 - bi]); };
+    auto record = [&](const uint4& m, const float*& gp, int& sh, int& ck) {
+        gp = src.gradient(m);
+        sh = (int)m.z;
+        if (KIND == OPT_ADAGRAD) {
+            ck = src.click(m);
+            src.click_at[m.x] = 0;
+        }
+        return gp != nullptr;
+    };
+    if constexpr (BIG > 0) {
+        __shared__ BigWave<KIND, BIG> tiles[4];
+        apply_big_wave<KIND, BIG>(s, o, tiles[wave], describe(big0), (uint32_t)wave, 4u, head.z, group,
+                                  [&](uint32_t at) { return p.member[first + at]; }, record, [] {});
+    } else if (BIG == BIG_GROUPS && head.z) {
         char* base = reinterpret_cast<char*>(apply_lds) + small_apply_slots_lds(flat ? 0 : b.N) + (size_t)wave * wave_lds;
         float* gbuf = reinterpret_cast<float*>(base);
         const float** gptr = reinterpret_cast<const float**>(base + wave_arrays);
@@ -882,25 +1192,17 @@ __global__ __launch_bounds__(256) void k_small_apply(SmallShape b, SmallPlan p, 
         apply_big_groups<KIND>(
             s, o, gbuf_floats, gbuf, gptr, den, lane, (uint32_t)wave, 4u, head.z,
             [&](uint32_t bi, uint32_t& row, uint32_t& off, uint32_t& k) {
-                const uint2 g = p.group[first + b.cap - 1 - bi];
+                const uint4 g = group(bi);
                 row = g.x;
-                off = g.y & 0xFFFFu;
-                k = g.y >> 16;
+                off = g.y;
+                k = g.z;
             },
-            [&](uint32_t at, const float*& gp, int& sh, int& ck) {
-                const uint4 m = p.member[first + at];
-                gp = src.gradient(m);
-                sh = (int)m.z;
-                if (KIND == OPT_ADAGRAD) {
-                    ck = src.click(m);
-                    src.click_at[m.x] = 0;
-                }
-                return gp != nullptr;
-            },
-            [] {}, [] { wave_sync(); });
+            [&](uint32_t at, const float*& gp, int& sh, int& ck) { return record(p.member[first + at], gp, sh, ck); }, [] {},
+            [] { wave_sync(); });
     }
-    constexpr uint32_t PER = 64 / LPG;
-    const uint32_t rounds_multi = (head.y + PER - 1) / PER, rounds = rounds_multi + (head.x + PER - 1) / PER;
+    // signs with one record: several rounds of a wavefront on their way at a time where a round has few
+    constexpr uint32_t PER = 64 / LPG, AT_ONCE = LPG >= 16 ? 4 : LPG >= 4 ? 2 : 1;
+    const uint32_t rounds_multi = (head.y + PER - 1) / PER, rounds = rounds_multi + (head.x + AT_ONCE * PER - 1) / (AT_ONCE * PER);
     // (Nothing leaves the loop's body but through its end: with a `continue` under a condition the compiler makes the lanes
     // that take it a loop of their own, in which lane 0, that draws the next round, does not run.)
     uint32_t r = wave_draw(&next_round);
@@ -910,21 +1212,40 @@ __global__ __launch_bounds__(256) void k_small_apply(SmallShape b, SmallPlan p, 
             const uint2 d = g < head.y ? p.group[first + head.x + g] : make_uint2(NO_ROW, 0);
             if (d.x <= s.cap) {  // (no row number at all: never address the table with it)
                 const SmallGroup grp{src, p.member + first + (d.y & 0xFFFFu)};
-                apply_group_ahead<KIND, LPG, ANY, 4>(s, o, grp, d.x, d.y >> 16, sub, lane0, c1, c2);
+                apply_group_ahead<KIND, LPG, ANY, 4, BIG != BIG_NONE>(s, o, grp, d.x, d.y >> 16, sub, lane0, c1, c2);
             }
         } else {
-            const uint32_t g = (r - rounds_multi) * PER + lane / LPG, at = min(g, b.cap - 1);
-            const uint2 d = p.group[first + at];
-            const uint4 mem = p.member[first + at];
-            if (g < head.x && d.x <= s.cap) {
-                const float* gp = src.gradient(mem);
-                if (gp) {
-                    int ck = 0;
-                    if (KIND == OPT_ADAGRAD) ck = src.click(mem);
-                    apply_one_record<KIND, LPG, ANY>(s, o, d.x, gp, (int)mem.z, ck, sub, lane0, c1, c2);
+            uint2 d[AT_ONCE];
+            uint4 mem[AT_ONCE];
+            const float* gp[AT_ONCE];
+            RecordRow row[AT_ONCE];
+            int ck[AT_ONCE];
+            bool ok[AT_ONCE];
+#pragma unroll
+            for (uint32_t q = 0; q < AT_ONCE; q++) {
+                const uint32_t g = ((r - rounds_multi) * AT_ONCE + q) * PER + lane / LPG, at = min(g, b.cap - 1);
+                d[q] = p.group[first + at];
+                mem[q] = p.member[first + at];
+                ok[q] = g < head.x;
+            }
+            // (what lies behind the last sign is nobody's: row 0 in its place, and nothing written)
+#pragma unroll
+            for (uint32_t q = 0; q < AT_ONCE; q++) {
+                ok[q] = ok[q] && d[q].x <= s.cap;
+                if (!ok[q]) {
+                    d[q].x = 0;
+                    mem[q].x = 0;
                 }
+                gp[q] = ok[q] ? src.gradient(mem[q]) : nullptr;
+                row[q] = fetch_record<KIND, ANY>(s, d[q].x, gp[q] ? gp[q] : s.w, sub);
+                ck[q] = KIND == OPT_ADAGRAD ? src.click(mem[q]) : 0;
+            }
+#pragma unroll
+            for (uint32_t q = 0; q < AT_ONCE; q++) {
+                if (gp[q])
+                    finish_record<KIND, LPG, ANY>(s, o, d[q].x, row[q], (int)mem[q].z, ck[q], sub, lane0, c1, c2);
                 // (a record without a gradient row, too: the caller may push the batch again on this plan)
-                if (KIND == OPT_ADAGRAD && sub == 0) src.click_at[mem.x] = 0;
+                if (KIND == OPT_ADAGRAD && ok[q] && sub == 0) src.click_at[mem[q].x] = 0;
             }
         }
         r = wave_draw(&next_round);

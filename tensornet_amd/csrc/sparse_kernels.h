@@ -1494,18 +1494,37 @@ __device__ __forceinline__ void put_row_part(float* p, int sub, int D, float4 v)
     }
 }
 
-// One record applied to its sign's row by LPG lanes: gradient, row and state once.
+// One record applied to its sign's row by LPG lanes: gradient, row and state once.  In two halves, for callers that have
+// several records on their way at a time.
+struct RecordRow {
+    float4 g, w, a, b;  // a: AdaGrad's state; a, b: Adam m, v / Ftrl z, n
+    int delta_show;
+};
+template <int KIND, bool ANY>
+__device__ __forceinline__ RecordRow fetch_record(const Store& s, uint32_t row, const float* gp, int sub) {
+    const int D = s.D;
+    const float* wp = s.w + (uint64_t)row * s.wstride;
+    const float* sp = s.st + (uint64_t)row * s.sstride;
+    RecordRow r;
+    r.g = row_part<ANY>(gp, sub, D);
+    r.w = row_part<ANY>(wp, sub, D);
+    if (KIND == OPT_ADAGRAD) {
+        r.a = *reinterpret_cast<const float4*>(sp);
+    } else {
+        r.a = row_part<ANY>(sp, sub, D);
+        r.b = row_part<ANY>(sp + D, sub, D);
+        r.delta_show = __float_as_int(sp[2 * D + 1]);
+    }
+    return r;
+}
 template <int KIND, int LPG, bool ANY>
-__device__ __forceinline__ void apply_one_record(const Store& s, const OptDev& o, uint32_t row, const float* gp, int bshow,
-                                                 int bclick, int sub, int lane0, float c1, float c2) {
+__device__ __forceinline__ void finish_record(const Store& s, const OptDev& o, uint32_t row, RecordRow& r, int bshow, int bclick,
+                                              int sub, int lane0, float c1, float c2) {
     const int D = s.D;
     float* wp = s.w + (uint64_t)row * s.wstride;
     float* sp = s.st + (uint64_t)row * s.sstride;
-    const float4 gr = row_part<ANY>(gp, sub, D);
-    float4 w = row_part<ANY>(wp, sub, D);
     if (KIND == OPT_ADAGRAD) {
-        const float4 h = *reinterpret_cast<const float4*>(sp);
-        const float p0 = gr.x * gr.x, p1 = gr.y * gr.y, p2 = gr.z * gr.z, p3 = gr.w * gr.w;
+        const float p0 = r.g.x * r.g.x, p1 = r.g.y * r.g.y, p2 = r.g.z * r.g.z, p3 = r.g.w * r.g.w;
         double tot = 0.0;  // add_g2sum: double accumulator over the float products, element order 0..D-1
         for (int l = 0; l < LPG; l++) {
             double cand = tot;
@@ -1515,15 +1534,15 @@ __device__ __forceinline__ void apply_one_record(const Store& s, const OptDev& o
             cand += (double)p3;
             tot = __shfl(cand, lane0 + l);
         }
-        const float g2sum = (float)((double)h.x + tot / (double)D);
+        const float g2sum = (float)((double)r.a.x + tot / (double)D);
         const float den = o.eps + sqrtf(g2sum);
-        w.x -= o.lr * gr.x / den;
-        w.y -= o.lr * gr.y / den;
-        w.z -= o.lr * gr.z / den;
-        w.w -= o.lr * gr.w / den;
-        put_row_part<ANY>(wp, sub, D, w);
+        r.w.x -= o.lr * r.g.x / den;
+        r.w.y -= o.lr * r.g.y / den;
+        r.w.z -= o.lr * r.g.z / den;
+        r.w.w -= o.lr * r.g.w / den;
+        put_row_part<ANY>(wp, sub, D, r.w);
         if (sub == 0) {
-            const float show = h.y + (float)bshow, click = h.z + (float)bclick;
+            const float show = r.a.y + (float)bshow, click = r.a.z + (float)bclick;
             *reinterpret_cast<float4*>(sp) = make_float4(g2sum, show, click, 0.f);  // no_show_days = 0
             if (o.use_cvm) {
                 wp[D] = show;
@@ -1531,24 +1550,28 @@ __device__ __forceinline__ void apply_one_record(const Store& s, const OptDev& o
             }
         }
     } else {
-        float4 a = row_part<ANY>(sp, sub, D);
-        float4 b = row_part<ANY>(sp + D, sub, D);
         if (KIND == OPT_ADAM) {
-            adam_elem(o, c1, c2, gr.x, w.x, a.x, b.x);
-            adam_elem(o, c1, c2, gr.y, w.y, a.y, b.y);
-            adam_elem(o, c1, c2, gr.z, w.z, a.z, b.z);
-            adam_elem(o, c1, c2, gr.w, w.w, a.w, b.w);
+            adam_elem(o, c1, c2, r.g.x, r.w.x, r.a.x, r.b.x);
+            adam_elem(o, c1, c2, r.g.y, r.w.y, r.a.y, r.b.y);
+            adam_elem(o, c1, c2, r.g.z, r.w.z, r.a.z, r.b.z);
+            adam_elem(o, c1, c2, r.g.w, r.w.w, r.a.w, r.b.w);
         } else {
-            ftrl_elem(o, gr.x, w.x, a.x, b.x);
-            ftrl_elem(o, gr.y, w.y, a.y, b.y);
-            ftrl_elem(o, gr.z, w.z, a.z, b.z);
-            ftrl_elem(o, gr.w, w.w, a.w, b.w);
+            ftrl_elem(o, r.g.x, r.w.x, r.a.x, r.b.x);
+            ftrl_elem(o, r.g.y, r.w.y, r.a.y, r.b.y);
+            ftrl_elem(o, r.g.z, r.w.z, r.a.z, r.b.z);
+            ftrl_elem(o, r.g.w, r.w.w, r.a.w, r.b.w);
         }
-        put_row_part<ANY>(wp, sub, D, w);
-        put_row_part<ANY>(sp, sub, D, a);
-        put_row_part<ANY>(sp + D, sub, D, b);
-        if (sub == 0) sp[2 * D + 1] = __int_as_float(__float_as_int(sp[2 * D + 1]) + bshow);
+        put_row_part<ANY>(wp, sub, D, r.w);
+        put_row_part<ANY>(sp, sub, D, r.a);
+        put_row_part<ANY>(sp + D, sub, D, r.b);
+        if (sub == 0) sp[2 * D + 1] = __int_as_float(r.delta_show + bshow);
     }
+}
+template <int KIND, int LPG, bool ANY>
+__device__ __forceinline__ void apply_one_record(const Store& s, const OptDev& o, uint32_t row, const float* gp, int bshow,
+                                                 int bclick, int sub, int lane0, float c1, float c2) {
+    RecordRow r = fetch_record<KIND, ANY>(s, row, gp, sub);
+    finish_record<KIND, LPG, ANY>(s, o, row, r, bshow, bclick, sub, lane0, c1, c2);
 }
 
 // Most signs occur in one slot only: one record, no ordering problem, no
@@ -2016,18 +2039,18 @@ struct BigTile {
     static constexpr int CHUNK = R * ROUNDS;
     static constexpr int DP = D + 1;  // padded staging row: lanes walking down a column hit different banks
 };
-// (the signs first, first + stride, ... by the wavefront that calls it, whose own the LDS is; head: the first one's description)
+// (the signs first, first + stride, ... below n_big by the wavefront that calls it, whose own the LDS is; head: the first one's
+// description, describe(bi): another's; record, missing, sync: as apply_big_groups')
 template <int D>
 struct BigTileLds {
     float gbuf[BigTile<D>::CHUNK * BigTile<D>::DP];
     const float* gptr[BigTile<D>::CHUNK];
     float den[BigTile<D>::CHUNK];
 };
-template <int D, typename Sync>
-__device__ __forceinline__ void apply_big_tiles(const Store& s, const OptDev& o, const PushSrc& src, DevStatus* status,
-                                                const uint4* __restrict__ big_desc, const Member* __restrict__ list,
-                                                const float* const* __restrict__ gaddr, BigTileLds<D>& lds, uint4 head,
-                                                uint32_t first, uint32_t stride, Sync sync) {
+template <int D, typename Describe, typename Record, typename Missing, typename Sync>
+__device__ __forceinline__ void apply_big_tiles(const Store& s, const OptDev& o, BigTileLds<D>& lds, uint4 head, uint32_t first,
+                                                uint32_t stride, uint32_t n_big, Describe describe, Record record,
+                                                Missing missing, Sync sync) {
     using T = BigTile<D>;
     constexpr int R = T::R, DP = T::DP;
     float* const gbuf = lds.gbuf;
@@ -2035,10 +2058,9 @@ __device__ __forceinline__ void apply_big_tiles(const Store& s, const OptDev& o,
     float* const den = lds.den;
     const int lane = (int)__lane_id();
     const int li = lane & (D - 1), lm = lane / D;
-    const uint32_t n_big = status->n_big;
     constexpr double inv_d = 1.0 / (double)D;  // exact: D is a power of two
     for (uint32_t bi = first; bi < n_big; bi += stride) {
-        if (bi != first) head = big_desc[bi];
+        if (bi != first) head = describe(bi);
         const uint32_t row = head.x, off = head.y, k = head.z;
         if (row > s.cap) continue;  // NO_ROW, or no row number at all: never address the table with it
         float* wp = s.w + (uint64_t)row * s.wstride;
@@ -2052,7 +2074,7 @@ __device__ __forceinline__ void apply_big_tiles(const Store& s, const OptDev& o,
             int sh = 0, ck = 0;
             if (lane < cn) {
                 const float* gp = nullptr;
-                ok = record_at(src, list + off + c0, gaddr ? gaddr + off + c0 : nullptr, lane, gp, sh, ck);
+                ok = record(off + c0 + (uint32_t)lane, gp, sh, ck);
                 gptr[lane] = gp;
             }
             const unsigned long long okmask = __ballot(ok);
@@ -2128,7 +2150,7 @@ __device__ __forceinline__ void apply_big_tiles(const Store& s, const OptDev& o,
                 }
             }
             if (okmask) any = true;
-            if (lane == 0 && okmask != chunk_mask) atomicOr(&status->err, DEV_ERR_GRAD_ROWS);
+            if (lane == 0 && okmask != chunk_mask) missing();
             sync();
         }
         if (any) {
@@ -2155,7 +2177,10 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6, 8))) void
     const uint4 head = big_desc[blockIdx.x < desc_cap ? blockIdx.x : desc_cap - 1];  // (before the status is known)
     // a push launched on a plan that turned out not to be its batch's (the host redoes it), or whose inputs are unusable
     if (status->mismatch | status->abort) return;
-    apply_big_tiles<D>(s, o, src, status, big_desc, list, gaddr, lds, head, blockIdx.x, gridDim.x, [] { __syncthreads(); });
+    apply_big_tiles<D>(
+        s, o, lds, head, blockIdx.x, gridDim.x, status->n_big, [&](uint32_t bi) { return big_desc[bi]; },
+        [&](uint32_t at, const float*& gp, int& sh, int& ck) { return record_at(src, list, gaddr, at, gp, sh, ck); },
+        [&] { atomicOr(&status->err, DEV_ERR_GRAD_ROWS); }, [] { __syncthreads(); });
 }
 
 // The updates of a push of up to ONE_STREAM_LOOKUPS lookups by one launch: the workgroups of the three kernels above side
@@ -2187,8 +2212,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6, 8))) voi
         if constexpr (TILE != 0) {
             __shared__ BigTileLds<TILE> lds[4];
             const uint4 head = a.big_desc[first < a.big_cap ? first : a.big_cap - 1];
-            apply_big_tiles<TILE>(s, o, src, status, a.big_desc, a.list, a.gaddr, lds[wave], head, first, stride,
-                                  [] { wave_sync(); });
+            apply_big_tiles<TILE>(
+                s, o, lds[wave], head, first, stride, status->n_big, [&](uint32_t bi) { return a.big_desc[bi]; },
+                [&](uint32_t at, const float*& gp, int& sh, int& ck) { return record_at(src, a.list, a.gaddr, at, gp, sh, ck); },
+                [&] { atomicOr(&status->err, DEV_ERR_GRAD_ROWS); }, [] { wave_sync(); });
         } else {
             extern __shared__ unsigned long long all_lds[];
             char* base = reinterpret_cast<char*>(all_lds) + wave * a.wave_lds;

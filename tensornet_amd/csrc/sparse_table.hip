@@ -52,6 +52,9 @@ constexpr size_t LDS_MIN_LOOKUPS = 1024;  // from here on the remap through LDS 
 //   128              81 / 132   104 / 135   120 / 152   133 / 151
 //   192             110 / 149   139 / 159   201 / 189   231 / 195
 //   254             148 / 167   220 / 182   275 / 226   339 / 242
+// Slots of more than 4096 lookups (k_small_slots_long; more than SMALL_SPLIT_SLOTS of them, tests/test_gpu_small.py pins 8 slots
+// of 4097 to the other path): 20 slots of 6000, AdaGrad rows of 16, 52 / 128 us, 40 of 8192, Ftrl rows of 1, 71 / 142,
+// 100 of 8000, Adam rows of 16, 138 / 171.
 // They cross at 89 to 106 M slots x lookups (160 to 254 slots; rows of 64: 58 to 90, of 8 under Adam: 120; pulls alone: 115).
 // With pooled gradients, whose reduction is shorter here, at 180 M (192 slots, 700 k lookups: 1.08 times as fast, 254 and
 // 700 k: 1.02, 850 k: 0.96).  A pull does not know what push will follow: it goes by the table's last one.
@@ -67,7 +70,7 @@ constexpr size_t SMALL_WORK = 100'000'000, SMALL_WORK_POOLED = 180'000'000;
 // 0.040 ms with every sign left to the lane groups, 0.020 ms with the threshold at 5; 1024 x 8 slots: no difference
 // between 4 and 12 slots here).
 constexpr int SMALL_NO_BIG_SLOTS = 12;
-constexpr uint32_t SMALL_BIG_GROUP = 5;
+constexpr uint32_t SMALL_BIG_GROUP = 5;  // (k_small_apply takes the signs with fewer in one go)
 constexpr uint32_t BIG_GROUP_DEFAULT = 16;
 
 // What a small pull has left to do behind its first launch takes one launch (k_small_pull_rest: 26 slots of 4096 lookups
@@ -75,7 +78,7 @@ constexpr uint32_t BIG_GROUP_DEFAULT = 16;
 // workgroups of a launch are given, that fewer than four would be on a CU.  Up to SMALL_SPLIT_SLOTS slots it stays two
 // launches, the sequence tests/test_gpu_small.py pins at 8 slots: a step of 8 slots of 1024 lookups is as long as the host's
 // way from the pull's first launch to the push, 37 us either way.
-constexpr int SMALL_SPLIT_SLOTS = 8;
+constexpr int SMALL_SPLIT_SLOTS = 8;  // (up to as many, slots are short, too: small_batch_shape)
 // Parts of rows from which a thread of small_finish takes two: up to here more workgroups are the shorter way.
 constexpr size_t FINISH_FULL = 1 << 17;
 constexpr size_t SMALL_SHARED_LDS = 36 * 1024;
@@ -1155,27 +1158,33 @@ int launch_small_apply_kind(SparseTable* t, RowShare share, const OptDev& o, con
     const bool with_big = t->plan_big_k != 0xFFFFFFFFu && (uint32_t)b.N >= t->plan_big_k;
     const int gfloats = small_gbuf_floats(s.D, b.N);
     const size_t arrays = align_up((size_t)(gfloats + 3 * s.D) * sizeof(float), 8), wave_lds = arrays + BIG_CHUNK * (8 + 4);
-    const size_t lds = small_apply_slots_lds(flat ? 0 : b.N) + (with_big ? 4 * wave_lds : 0);
-#define TN_LAUNCH_SMALL_ANY(LPG, ANY)                                                                                  \
-    TN_LAUNCH_LDS((k_small_apply<KIND, LPG, ANY>), dim3(b.buckets()), dim3(256), lds, st, b, p, flat, s, o,            \
+    const bool lds_big = with_big && (s.D > 64 || (s.D & (s.D - 1)) != 0);  // (others keep their staging in static LDS)
+    const size_t lds = small_apply_slots_lds(flat ? 0 : b.N) + (lds_big ? 4 * wave_lds : 0);
+#define TN_LAUNCH_SMALL_BIG(LPG, ANY, BIG)                                                                             \
+    TN_LAUNCH_LDS((k_small_apply<KIND, LPG, ANY, BIG>), dim3(b.buckets()), dim3(256), lds, st, b, p, flat, s, o,       \
                   (const DevStatus*)t->dplan, host_seq, seq, dim, gfloats, (uint32_t)wave_lds, (uint32_t)arrays)
-#define TN_LAUNCH_SMALL(LPG)                  \
-    do {                                      \
-        if (share.any)                        \
-            TN_LAUNCH_SMALL_ANY(LPG, true);   \
-        else                                  \
-            TN_LAUNCH_SMALL_ANY(LPG, false);  \
+// (aligned rows that fill their lanes have 4, 8 .. 128 elements; of these the last are too long for apply_big_wave)
+#define TN_LAUNCH_SMALL_ROWS(LPG)                                                                     \
+    do {                                                                                              \
+        constexpr int WAVE = LPG <= 16 ? 4 * LPG : BIG_GROUPS;                                        \
+        if (!with_big && share.any) TN_LAUNCH_SMALL_BIG(LPG, true, BIG_NONE);                         \
+        else if (!with_big) TN_LAUNCH_SMALL_BIG(LPG, false, BIG_NONE);                                \
+        else if (!share.any) TN_LAUNCH_SMALL_BIG(LPG, false, WAVE);                                   \
+        else if (lds_big) TN_LAUNCH_SMALL_BIG(LPG, true, BIG_GROUPS);                                 \
+        else if (s.D == 1) TN_LAUNCH_SMALL_BIG(LPG, true, (LPG == 1 ? 1 : WAVE));                     \
+        else if (s.D == 2) TN_LAUNCH_SMALL_BIG(LPG, true, (LPG == 1 ? 2 : WAVE));                     \
+        else TN_LAUNCH_SMALL_BIG(LPG, true, WAVE);                                                    \
     } while (0)
     switch (share.lanes) {
-        case 1: TN_LAUNCH_SMALL(1); break;
-        case 2: TN_LAUNCH_SMALL(2); break;
-        case 4: TN_LAUNCH_SMALL(4); break;
-        case 8: TN_LAUNCH_SMALL(8); break;
-        case 16: TN_LAUNCH_SMALL(16); break;
-        default: TN_LAUNCH_SMALL(32); break;
+        case 1: TN_LAUNCH_SMALL_ROWS(1); break;
+        case 2: TN_LAUNCH_SMALL_ROWS(2); break;
+        case 4: TN_LAUNCH_SMALL_ROWS(4); break;
+        case 8: TN_LAUNCH_SMALL_ROWS(8); break;
+        case 16: TN_LAUNCH_SMALL_ROWS(16); break;
+        default: TN_LAUNCH_SMALL_ROWS(32); break;
     }
-#undef TN_LAUNCH_SMALL
-#undef TN_LAUNCH_SMALL_ANY
+#undef TN_LAUNCH_SMALL_ROWS
+#undef TN_LAUNCH_SMALL_BIG
     return TN_OK;
 }
 
@@ -1305,8 +1314,9 @@ int launch_table_apply(SparseTable* t, RowShare share, const TableShape& b, cons
 bool small_batch_shape(SparseTable* t, int N, const int64_t* lens, SmallShape& b) {
     if (!t->small_path || t->async_pull || N <= 0 || N > SMALL_SLOTS || t->dim > 128) return false;
     size_t L = 0, max_len = 0;
+    const int64_t longest = N > SMALL_SPLIT_SLOTS ? SMALL_SLOT_MAX : SMALL_SLOT_SHORT;
     for (int s = 0; s < N; s++) {
-        if (lens[s] < 0 || lens[s] > SMALL_SLOT_MAX) return false;
+        if (lens[s] < 0 || lens[s] > longest) return false;
         L += (size_t)lens[s];
         max_len = std::max<size_t>(max_len, (size_t)lens[s]);
     }
@@ -1326,6 +1336,7 @@ bool small_batch_shape(SparseTable* t, int N, const int64_t* lens, SmallShape& b
     b.cap = (uint32_t)align_up(2 * (L / b.buckets()) + 64 + 4 * (size_t)N, 64);
     if (!t->small_lds) {
         t->small_lds = big_lds_bytes_for(reinterpret_cast<const void*>(k_small_slots), 144 * 1024);
+        t->small_lds = std::min(t->small_lds, big_lds_bytes_for(reinterpret_cast<const void*>(k_small_slots_long), 144 * 1024));
         t->small_emit_lds = big_lds_bytes_for(reinterpret_cast<const void*>(k_group_emit<true>), 144 * 1024);
     }
     return small_slots_lds(small_entries(b.max_len, b.parts), b.max_len, b.nbp) <= t->small_lds &&
@@ -1403,8 +1414,13 @@ int small_pull(SparseTable* t, const SmallShape& b, const int64_t* const* values
         vec = vec && aligned16(vars[i]);
     }
     const uint32_t seq = ++t->seq_pull, workgroups = (uint32_t)b.N * b.parts, entries = small_entries(b.max_len, b.parts);
-    TN_LAUNCH_LDS(k_small_slots, dim3(workgroups), dim3(SMALL_THREADS), small_slots_lds(entries, b.max_len, b.nbp), st, b, p,
-                  (const SlotDesc*)descs, entries, s, make_optdev(t), t->seed, t->dplan, t->hwords, seq);
+    const size_t slots_lds = small_slots_lds(entries, b.max_len, b.nbp);
+    if (b.max_len <= SMALL_SLOT_SHORT)
+        TN_LAUNCH_LDS(k_small_slots, dim3(workgroups), dim3(SMALL_THREADS), slots_lds, st, b, p, (const SlotDesc*)descs, entries,
+                      s, make_optdev(t), t->seed, t->dplan, t->hwords, seq);
+    else
+        TN_LAUNCH_LDS(k_small_slots_long, dim3(workgroups), dim3(2 * SMALL_THREADS), slots_lds, st, b, p, (const SlotDesc*)descs,
+                      entries, s, make_optdev(t), t->seed, t->dplan, t->hwords, seq);
     const uint32_t C = (uint32_t)(vec ? wdim / 4 : wdim), items = (size_t)b.L * C > FINISH_FULL ? FINISH_ITEMS : 1;
     const uint32_t per = items * FINISH_THREADS / C, chunks = (b.max_len + per - 1) / per;
     EmitArgs<true> ea;

@@ -343,7 +343,7 @@ __global__ __launch_bounds__(256) void k_table_apply(TableShape b, Store s, OptD
                 if (g < n_multi) {
                     const uint32_t e = multi[g];
                     grp.sorted = sorted + toff[e];
-                    apply_group_ahead<KIND, LPG, ANY, 4>(s, o, grp, trow[e], tcnt[e], sub, lane0, c1, c2);
+                    apply_group_ahead<KIND, LPG, ANY, 4, false>(s, o, grp, trow[e], tcnt[e], sub, lane0, c1, c2);
                 }
             } else {
                 const uint32_t g = (r - rounds_multi) * (64 / LPG) + lane / LPG;
