@@ -27,7 +27,7 @@ constexpr int COMBINE_WINDOW = 8;  // lookups of an example read ahead with inde
 // In these kernels a SlotDesc carries: values = mapped ids (forward) / signs (backward),
 // mapped = example index of every lookup, grads = rows to read (variable / pooled gradient),
 // var = rows to write (forward: out[batch, dim]), rows = rows of `grads`, len = lookups.
-__device__ __forceinline__ const int64_t* example_of(const SlotDesc& d) { return d.mapped; }
+__device__ __forceinline__ Global<const int64_t> example_of(const SlotDesc& d) { return as_global((const int64_t*)d.mapped); }
 
 __device__ __forceinline__ float combine_divisor(uint32_t n, int combiner) {
     if (combiner == COMBINE_SUM || n == 0) return 1.f;
@@ -37,7 +37,7 @@ __device__ __forceinline__ float combine_divisor(uint32_t n, int combiner) {
 // How many of the sorted ids ex[0 .. n) lie below `x`, by a workgroup of 256 threads: every round looks at 256 places
 // of what is left, so 65 536 ids take two round trips (a binary search: sixteen).  A function of the array and x alone:
 // whatever the order of the ids, two workgroups that ask for the same x get the same answer.  sh: 5 words of LDS.
-__device__ __forceinline__ uint32_t ids_below(const int64_t* __restrict__ ex, uint32_t n, int64_t x, uint32_t* sh) {
+__device__ __forceinline__ uint32_t ids_below(Global<const int64_t> ex, uint32_t n, int64_t x, uint32_t* sh) {
     uint32_t lo = 0, len = n;  // the answer lies in [lo, lo + len]
     while (len > 0) {
         const uint32_t step = (len + 255) / 256;
@@ -79,7 +79,7 @@ __global__ __launch_bounds__(256) void k_combine_fwd(const SlotDesc* __restrict_
         const int64_t b0 = (int64_t)(item - sl * per_slot) * per;
         const uint32_t nb = (uint32_t)min((int64_t)per, batch - b0);
         const SlotDesc d = descs[sl];
-        const int64_t* __restrict__ ex = example_of(d);
+        const Global<const int64_t> ex = example_of(d);
         for (uint32_t i = threadIdx.x; i < 2 * per; i += 256) range[i] = 0;
         const uint32_t lo = b0 == 0 ? 0u : ids_below(ex, d.len, b0, sh);
         const uint32_t hi = b0 + nb >= batch ? d.len : ids_below(ex, d.len, b0 + nb, sh);
@@ -95,7 +95,7 @@ __global__ __launch_bounds__(256) void k_combine_fwd(const SlotDesc* __restrict_
             if (next != x || i + 1 == hi) range[per + (x - b0)] = i + 1;
         }
         __syncthreads();
-        const int64_t* __restrict__ ids = d.values;
+        const Global<const int64_t> ids = as_global(d.values);
         const float* __restrict__ rows = d.grads;
         for (uint32_t e = threadIdx.x / LPG; e < nb; e += 256 / LPG) {
             const uint32_t from = range[e], to = max(range[per + e], from);
@@ -210,7 +210,7 @@ __global__ __launch_bounds__(256) void k_lookup_keys(const SlotDesc* __restrict_
     const uint32_t sl = slot, l0 = lbase[sl], len = lbase[sl + 1] - l0;
     const uint32_t t0 = (blockIdx.x - share.first_tile(sl, l0)) * POOL_TILE, lp = share.parts_log2(len);
     const uint32_t ub = ubase[sl], parts = 1u << lp, spread = share.spread(lp);
-    const int64_t* __restrict__ ex = example_of(descs[sl]);
+    const Global<const int64_t> ex = example_of(descs[sl]);
     int64_t b[KEY_ITEMS], prev[KEY_ITEMS];
     uint32_t u[KEY_ITEMS];
 #pragma unroll
@@ -308,7 +308,7 @@ __global__ __launch_bounds__(256) void k_lookup_keys(const SlotDesc* __restrict_
 }
 
 // The lookups of example x in a slot's sorted ids.
-__device__ __forceinline__ uint32_t lookups_of(const int64_t* __restrict__ ex, uint32_t n, int64_t x) {
+__device__ __forceinline__ uint32_t lookups_of(Global<const int64_t> ex, uint32_t n, int64_t x) {
     uint32_t bound[2];
     for (int k = 0; k < 2; k++) {  // the first id >= x, then > x
         uint32_t lo = 0, len = n;
@@ -369,7 +369,7 @@ __global__ __launch_bounds__(POOL_THREADS) __attribute__((amdgpu_waves_per_eu(6,
     if (!spread && part >= us) return;
     const uint32_t top = us > spread ? spread + ((us - 1 - spread) >> lp) : us - 1, bits = top ? 32 - (uint32_t)__clz((int)top) : 0u;
     const float* pooled = descs[sl].grads;
-    const int64_t* ex = example_of(descs[sl]);
+    const Global<const int64_t> ex = example_of(descs[sl]);
     const uint32_t mine = (len + POOL_TILE - 1) / POOL_TILE;
     uint32_t* const before = lds.list;                   // [POOL_THREADS + 1]: items of my part in the tiles before
     uint32_t* const start = before + POOL_THREADS + 1;   // [POOL_THREADS]: where they are in a tile

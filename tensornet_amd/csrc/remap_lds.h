@@ -173,7 +173,7 @@ __global__ __launch_bounds__(TILE_THREADS) __attribute__((amdgpu_waves_per_eu(6,
         const uint32_t n_tile = g1 - g0 + 1;
         const int s0 = find_slot(lb, N, g0);
         const bool one_slot = g1 < lb[s0 + 1];  // the usual case: the slot's values and buckets sit in registers
-        const int64_t* v0 = slot_values(s0) - lb[s0];
+        const Global<const int64_t> v0 = as_global(slot_values(s0)) - lb[s0];
         uint64_t sg[TILE_ITEMS];
         int sl[TILE_ITEMS];
 #pragma unroll
@@ -186,7 +186,7 @@ __global__ __launch_bounds__(TILE_THREADS) __attribute__((amdgpu_waves_per_eu(6,
                     sg[j] = (uint64_t)v0[gi];
                 } else {
                     sl[j] = find_slot(lb, N, gi);
-                    sg[j] = (uint64_t)slot_values(sl[j])[gi - lb[sl[j]]];
+                    sg[j] = (uint64_t)as_global(slot_values(sl[j]))[gi - lb[sl[j]]];
                 }
             }
         }
@@ -538,7 +538,7 @@ __global__ __launch_bounds__(REMAP_THREADS) void k_lds_assign(
             while (gi >= lb[sl + 1]) sl++;
             sls[j] = sl;
             if (LISTS && (bits & (1u << j))) {
-                vals[j] = (uint64_t)descs[sl].values[gi - lb[sl]];
+                vals[j] = (uint64_t)as_global(descs[sl].values)[gi - lb[sl]];
                 cnts[j] = cnt_at[gi];
             }
         }
@@ -603,7 +603,7 @@ __global__ __launch_bounds__(256) void k_lds_mapped(const SlotDesc* __restrict__
                 if (g0 + j < L) u_of_gi[g0 + j] = u[j] | (f[j] == g0 + j ? FIRST_BIT : 0u);
         }
         int sl = find_slot(lb, N, g0);
-        int64_t* out = descs[sl].mapped - lb[sl];
+        Global<int64_t> out = as_global(descs[sl].mapped) - lb[sl];
         uint32_t ub = ubase[sl];
 #pragma unroll
         for (int j = 0; j < 4; j++) {
@@ -611,7 +611,7 @@ __global__ __launch_bounds__(256) void k_lds_mapped(const SlotDesc* __restrict__
             if (gi >= L) break;
             if (gi >= lb[sl + 1]) {
                 do sl++; while (gi >= lb[sl + 1]);
-                out = descs[sl].mapped - lb[sl];
+                out = as_global(descs[sl].mapped) - lb[sl];
                 ub = ubase[sl];
             }
             out[gi] = (int64_t)(u[j] - ub);

@@ -140,7 +140,7 @@ __device__ __forceinline__ void small_slots(const SmallShape& b, const SmallPlan
         if (part == 0) reinterpret_cast<uint32_t*>(p.descs + sl)[tid] = dword;  // for the launches after this one
     }
     __syncthreads();
-    const int64_t* values = sd.values;
+    const Global<const int64_t> values = as_global(sd.values);
     const uint32_t len = sd.len, lbase = sd.lbase;
     uint64_t sg[SMALL_ITEMS];
 #pragma unroll
@@ -479,14 +479,14 @@ __device__ __forceinline__ void small_finish(const SmallShape& b, const SmallPla
         if (f[j] == NO_ROW) continue;
         const uint32_t rank = before[f[j] >> 6] + (uint32_t)__popcll(bits[f[j] >> 6] & ((1ull << (f[j] & 63)) - 1ull));
         if (c[j] == 0) {
-            d.mapped[pos[j]] = (int64_t)rank;
+            as_global(d.mapped)[pos[j]] = (int64_t)rank;
             if (f[j] == pos[j]) p.rank_at[d.lbase + pos[j]] = (uint16_t)rank;
         }
         if (row[j] == NO_ROW || (int64_t)rank >= d.rows) continue;  // (the host reports a variable that is too small)
         if (VEC == 4)
-            *reinterpret_cast<float4*>(d.var + (uint64_t)rank * s.wdim + c[j] * 4) = v4[j];
+            put_row_part<false>(d.var + (uint64_t)rank * s.wdim, c[j], 0, v4[j]);
         else
-            d.var[(uint64_t)rank * s.wdim + c[j]] = v1[j];
+            as_global(d.var)[(uint64_t)rank * s.wdim + c[j]] = v1[j];
     }
 }
 
@@ -557,8 +557,8 @@ __global__ __launch_bounds__(256) void k_small_verify(SmallShape b, SmallPlan p,
 #pragma unroll
     for (int j = 0; j < PER; j++) {
         const uint32_t pos = p0 + j * 256 + threadIdx.x;
-        now[j] = pos < len ? (uint64_t)sd.values[pos] : 0;
-        label[j] = CLICKS && pos < len ? (int)sd.labels[pos] : 0;
+        now[j] = pos < len ? (uint64_t)as_global(sd.values)[pos] : 0;
+        label[j] = CLICKS && pos < len ? (int)as_global(sd.labels)[pos] : 0;
     }
 #pragma unroll
     for (int j = 0; j < PER; j++) {
@@ -597,7 +597,7 @@ __global__ __launch_bounds__(POOL_THREADS) __attribute__((amdgpu_waves_per_eu(6,
     const SlotDesc d = descs[sl];
     const uint32_t n = d.len, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     if (n == 0 || status->mismatch) return;
-    const int64_t* ex = d.mapped;
+    const Global<const int64_t> ex = as_global((const int64_t*)d.mapped);
     if (tid == 0) bad = 0;
     __syncthreads();
     uint32_t f[SMALL_POOL_ITEMS], x[SMALL_POOL_ITEMS];
@@ -943,7 +943,7 @@ __device__ __forceinline__ void apply_big_wave(const Store& s, const OptDev& o, 
 #pragma unroll
             for (int q = 0; q < ROUNDS; q++) {
                 const int m = lm + q * R;
-                v[q] = (m < cn && ((okmask >> m) & 1ull)) ? lds.gptr[m][li] : 0.f;
+                v[q] = (m < cn && ((okmask >> m) & 1ull)) ? as_global(lds.gptr[m])[li] : 0.f;
             }
         };
         fetch(0, now);

@@ -573,6 +573,53 @@ __global__ __launch_bounds__(256) void k_rehash(Store from, Store to, DevStatus*
     }
 }
 
+// The update kernels' view of a row: lane `sub` of the LPG lanes that share it owns elements [4 sub, 4 sub + 4).  With
+// ANY the row has any length up to 4 LPG and stands at any 4-byte boundary -- rows of 1, 6 or 10 elements, gradients
+// of rows with the two cvm columns (10 floats apart for 8 elements): a lane whose part is whole moves it with one
+// unaligned 16-byte access, which gfx950 takes, the last one element by element, lanes beyond the row hold zeros
+// (which change neither a sum of squares nor anything that is stored).  One thread per sign, as such rows had before,
+// cost 78 us for 282 k lookups of 8 + 2 elements (k_apply_scalar); this way it is 28 (k_apply_single 10, k_apply_vec 18).
+typedef float any_float4 __attribute__((ext_vector_type(4), aligned(4)));
+template <bool ANY>
+__device__ __forceinline__ float4 row_part(const float* p, int sub, int D) {
+    if (!ANY) {
+        const native_float4 q = ((Global<const native_float4>)p)[sub];
+        return make_float4(q.x, q.y, q.z, q.w);
+    }
+    const int left = D - 4 * sub;
+    const Global<const float> e = as_global(p + 4 * sub);
+    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (left >= 4) {
+        const any_float4 q = *(Global<const any_float4>)e;
+        v = make_float4(q.x, q.y, q.z, q.w);
+    } else if (left > 0) {
+        v.x = e[0];
+        if (left > 1) v.y = e[1];
+        if (left > 2) v.z = e[2];
+    }
+    return v;
+}
+template <bool ANY>
+__device__ __forceinline__ void put_row_part(float* p, int sub, int D, float4 v) {
+    if (!ANY) {
+        native_float4 q;
+        q.x = v.x, q.y = v.y, q.z = v.z, q.w = v.w;
+        ((Global<native_float4>)p)[sub] = q;
+        return;
+    }
+    const int left = D - 4 * sub;
+    const Global<float> e = as_global(p + 4 * sub);
+    if (left >= 4) {
+        any_float4 q;
+        q.x = v.x, q.y = v.y, q.z = v.z, q.w = v.w;
+        *(Global<any_float4>)e = q;
+    } else if (left > 0) {
+        e[0] = v.x;
+        if (left > 1) e[1] = v.y;
+        if (left > 2) e[2] = v.z;
+    }
+}
+
 // -------------------------------------------------------------------- remap
 // Slot of a lookup: last s with lbase[s] <= gi (lbase[N] = L), skipping empty slots.
 __device__ __forceinline__ int find_slot(const uint32_t* lb, int N, uint32_t gi) {
@@ -611,7 +658,7 @@ __global__ __launch_bounds__(256) void k_remap_insert(const SlotDesc* __restrict
         const int sl = find_slot(lb, N, gi);
         const SlotDesc& d = descs[sl];
         const uint32_t li = gi - lb[sl];
-        const uint64_t sign = (uint64_t)d.values[li];
+        const uint64_t sign = (uint64_t)as_global(d.values)[li];
         vals_copy[gi] = sign;
         const uint32_t tbase = d.tbase, tcap = d.tcap;
         uint32_t e;
@@ -786,7 +833,7 @@ __global__ __launch_bounds__(REMAP_THREADS) void k_assign_rank(
         }
         if (bits & (1u << j)) {
             dt[tidx[gi]].rank = u;
-            uniq_sign[u] = (uint64_t)descs[sl].values[gi - lb[sl]];
+            uniq_sign[u] = (uint64_t)as_global(descs[sl].values)[gi - lb[sl]];
             uniq_slot[u] = (uint32_t)sl;
             u++;
         }
@@ -814,7 +861,7 @@ __global__ __launch_bounds__(256) void k_write_mapped(const SlotDesc* __restrict
         u_of_gi[gi] = u | (first ? FIRST_BIT : 0u);
         if (write_ids) {
             const int sl = find_slot(lb, N, gi);
-            descs[sl].mapped[gi - lb[sl]] = (int64_t)(u - ubase[sl]);
+            as_global(descs[sl].mapped)[gi - lb[sl]] = (int64_t)(u - ubase[sl]);
         }
     }
 }
@@ -865,7 +912,7 @@ __global__ __launch_bounds__(256) void k_count_show(const SlotDesc* __restrict__
             int label = 0;
             if (with_click) {
                 const int sl = find_slot(lb, N, gi);
-                label = (int)descs[sl].labels[gi - lb[sl]];
+                label = (int)as_global(descs[sl].labels)[gi - lb[sl]];
             }
             const bool repeat = (v & FIRST_BIT) == 0;
             if (!repeat && label == 0) continue;
@@ -1201,10 +1248,9 @@ __global__ __launch_bounds__(256) void k_gather_vars(Store s, DevStatus* status,
         }
         if (row > s.cap) continue;  // NO_ROW, or no row number at all: never address the table with it
         if (VEC == 4) {
-            float4 v = *reinterpret_cast<const float4*>(s.w + (uint64_t)row * s.wstride + c * 4);
-            *reinterpret_cast<float4*>(d.var + r * s.wdim + c * 4) = v;
+            put_row_part<false>(d.var + r * s.wdim, c, 0, row_part<false>(s.w + (uint64_t)row * s.wstride, c, 0));
         } else {
-            d.var[r * s.wdim + c] = s.w[(uint64_t)row * s.wstride + c];
+            as_global(d.var)[r * s.wdim + c] = s.w[(uint64_t)row * s.wstride + c];
         }
     }
 }
@@ -1351,10 +1397,10 @@ __global__ __launch_bounds__(256) void k_verify_values(const SlotDesc* __restric
             if (gi <= g1) {
                 const int sl = one_slot ? s0 : find_slot(lb, N, gi);
                 const SlotDesc& d = descs[sl];
-                now[j] = (uint64_t)d.values[gi - lb[sl]];
+                now[j] = (uint64_t)as_global(d.values)[gi - lb[sl]];
                 if (COPY) then[j] = vals_copy[gi];
                 if (CLICKS) {
-                    label[j] = (int)d.labels[gi - lb[sl]];
+                    label[j] = (int)as_global(d.labels)[gi - lb[sl]];
                     u[j] = u_of_gi[gi] & ~FIRST_BIT;
                 }
                 if (gi < n_members) {  // the member lists of the groups with several records fill the top of the array
@@ -1449,48 +1495,6 @@ __device__ __forceinline__ void ftrl_elem(const OptDev& o, float g, float& w, fl
             w *= z - o.lambda1;
         else
             w *= z + o.lambda1;
-    }
-}
-
-// The update kernels' view of a row: lane `sub` of the LPG lanes that share it owns elements [4 sub, 4 sub + 4).  With
-// ANY the row has any length up to 4 LPG and stands at any 4-byte boundary -- rows of 1, 6 or 10 elements, gradients
-// of rows with the two cvm columns (10 floats apart for 8 elements): a lane whose part is whole moves it with one
-// unaligned 16-byte access, which gfx950 takes, the last one element by element, lanes beyond the row hold zeros
-// (which change neither a sum of squares nor anything that is stored).  One thread per sign, as such rows had before,
-// cost 78 us for 282 k lookups of 8 + 2 elements (k_apply_scalar); this way it is 28 (k_apply_single 10, k_apply_vec 18).
-typedef float any_float4 __attribute__((ext_vector_type(4), aligned(4)));
-template <bool ANY>
-__device__ __forceinline__ float4 row_part(const float* p, int sub, int D) {
-    if (!ANY) return reinterpret_cast<const float4*>(p)[sub];
-    const int left = D - 4 * sub;
-    p += 4 * sub;
-    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (left >= 4) {
-        const any_float4 q = *reinterpret_cast<const any_float4*>(p);
-        v = make_float4(q.x, q.y, q.z, q.w);
-    } else if (left > 0) {
-        v.x = p[0];
-        if (left > 1) v.y = p[1];
-        if (left > 2) v.z = p[2];
-    }
-    return v;
-}
-template <bool ANY>
-__device__ __forceinline__ void put_row_part(float* p, int sub, int D, float4 v) {
-    if (!ANY) {
-        reinterpret_cast<float4*>(p)[sub] = v;
-        return;
-    }
-    const int left = D - 4 * sub;
-    p += 4 * sub;
-    if (left >= 4) {
-        any_float4 q;
-        q.x = v.x, q.y = v.y, q.z = v.z, q.w = v.w;
-        *reinterpret_cast<any_float4*>(p) = q;
-    } else if (left > 0) {
-        p[0] = v.x;
-        if (left > 1) p[1] = v.y;
-        if (left > 2) p[2] = v.z;
     }
 }
 
@@ -1845,7 +1849,7 @@ __device__ __forceinline__ void apply_big_groups(const Store& s, const OptDev& o
 #pragma unroll
                     for (int q = 0; q < BIG_LOADS; q++) {
                         const int m = m0 + q * mstep;
-                        v[q] = (m < cn && ((okmask >> m) & 1ull)) ? gptr[m][li] : 0.f;
+                        v[q] = (m < cn && ((okmask >> m) & 1ull)) ? as_global(gptr[m])[li] : 0.f;
                     }
 #pragma unroll
                     for (int q = 0; q < BIG_LOADS; q++) {
@@ -1862,7 +1866,7 @@ __device__ __forceinline__ void apply_big_groups(const Store& s, const OptDev& o
                         v[q] = 0.f;
                         if (t < cn * D) {
                             const int m = t / D, i = t - m * D;
-                            if ((okmask >> m) & 1ull) v[q] = gptr[m][i];
+                            if ((okmask >> m) & 1ull) v[q] = as_global(gptr[m])[i];
                         }
                     }
 #pragma unroll
@@ -2085,7 +2089,7 @@ __device__ __forceinline__ void apply_big_tiles(const Store& s, const OptDev& o,
 #pragma unroll
                 for (int q = 0; q < T::ROUNDS; q++) {
                     const int m = lm + q * R;
-                    v[q] = (m < cn && ((okmask >> m) & 1ull)) ? gptr[m][li] : 0.f;
+                    v[q] = (m < cn && ((okmask >> m) & 1ull)) ? as_global(gptr[m])[li] : 0.f;
                 }
 #pragma unroll
                 for (int q = 0; q < T::ROUNDS; q++) gbuf[(lm + q * R) * DP + li] = v[q];

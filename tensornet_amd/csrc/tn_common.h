@@ -143,6 +143,16 @@ __device__ __forceinline__ uint32_t ld_relaxed(const uint32_t* p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// A pointer that came out of memory (a slot's tensor out of its descriptor, a gradient row out of LDS) as one to global memory,
+// which is all it can be.  The compiler has to take it for a generic one, and a generic (flat) load counts as an LDS access, too:
+// the next wait for LDS waits for the memory as well, so nothing stays in flight across a barrier or an LDS read.
+template <typename T>
+using Global = T __attribute__((address_space(1)))*;
+template <typename T>
+__device__ __forceinline__ Global<T> as_global(T* p) {
+    return (Global<T>)p;
+}
+
 // 16-byte accesses marked non-temporal, for data that is read once or written once per call and
 // should not displace what the caches hold.
 typedef float native_float4 __attribute__((ext_vector_type(4)));
