@@ -136,7 +136,7 @@ __global__ __launch_bounds__(256) void k_combine_fwd(const SlotDesc* __restrict_
 // Behind the last kernel of a call: its error flags to the host, in one word with the number of the call, for which the
 // host polls (a wait on the stream returns about ten microseconds later).  The flags are taken and set to zero for the
 // next call, which may come on another stream as soon as the word is out, by one atomic.
-__global__ void k_report(DevStatus* status, uint64_t* host_word, uint32_t seq) {
+static __global__ void k_report(DevStatus* status, uint64_t* host_word, uint32_t seq) {
     if (threadIdx.x != 0) return;
     const uint32_t err = __hip_atomic_exchange(&status->err, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     const unsigned long long w = (unsigned long long)err | ((unsigned long long)seq << 32);
@@ -190,7 +190,7 @@ constexpr uint32_t POOL_KEY_SHIFT = 12;
 
 inline size_t pool_tile_lds(uint32_t lp) { return ((size_t)KEY_WAVES << lp) * sizeof(uint32_t); }
 
-__global__ __launch_bounds__(256) void k_lookup_keys(const SlotDesc* __restrict__ descs, const uint32_t* __restrict__ lbase,
+static __global__ __launch_bounds__(256) void k_lookup_keys(const SlotDesc* __restrict__ descs, const uint32_t* __restrict__ lbase,
                                                      const uint32_t* __restrict__ ubase, uint32_t N,
                                                      const uint32_t* __restrict__ u_of_gi, int64_t batch,
                                                      uint2* __restrict__ pool, uint16_t* __restrict__ poff, PoolShare share,

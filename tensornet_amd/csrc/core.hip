@@ -4,6 +4,7 @@
 // (py_wrapper.cc:112).
 #include "tn_common.h"
 
+#include <algorithm>
 #include <cstring>
 
 namespace tn {
@@ -13,6 +14,20 @@ thread_local std::string t_last_error;
 std::mutex g_opt_mu;
 std::vector<std::shared_ptr<OptConf>> g_opts;
 }  // namespace
+
+size_t big_lds_bytes_for(const void* kernel, size_t cap) {
+    int dev = 0, most = 0;
+    size_t bytes = 48 * 1024;
+    if (hipGetDevice(&dev) == hipSuccess &&
+        hipDeviceGetAttribute(&most, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) == hipSuccess && most > 2048)
+        bytes = std::min<size_t>((size_t)most - 2048, cap);  // (room for the kernel's static arrays)
+    if (bytes > 48 * 1024 &&
+        hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        bytes = 48 * 1024;
+    }
+    return bytes;
+}
 
 void set_error(const std::string& msg) { t_last_error = msg; }
 

@@ -138,7 +138,7 @@ inline size_t tile_dedup_lds(int N, uint32_t span_cap) {
     const size_t lb = align_up(((size_t)N + 1) * sizeof(uint32_t), 8);
     return (N <= TILE_LDS_SLOTS ? lb + (size_t)N * (sizeof(uint64_t) + sizeof(uint2)) : lb) + (size_t)span_cap * sizeof(uint32_t);
 }
-__global__ __launch_bounds__(TILE_THREADS) __attribute__((amdgpu_waves_per_eu(6, 8))) void k_tile_dedup(const SlotDesc* __restrict__ descs,
+static __global__ __launch_bounds__(TILE_THREADS) __attribute__((amdgpu_waves_per_eu(6, 8))) void k_tile_dedup(const SlotDesc* __restrict__ descs,
                                                              const uint32_t* __restrict__ lbase, int N, uint32_t L,
                                                              uint32_t* bcursor, ulonglong2* __restrict__ prec,
                                                              ulonglong2* __restrict__ prints,
@@ -441,7 +441,7 @@ __device__ __forceinline__ uint32_t rank_of(const uint8_t* __restrict__ flag8, c
 // what the first-level buckets of every slot were handed: status->tile_share_q16 = the largest share
 // records / lookups among the slots with more than one bucket's worth of lookups, in 1 / 65536 (the host sizes
 // the next call's buckets from it).
-__global__ __launch_bounds__(REMAP_THREADS) void k_lds_flags(uint32_t L, const uint32_t* __restrict__ first_of,
+static __global__ __launch_bounds__(REMAP_THREADS) void k_lds_flags(uint32_t L, const uint32_t* __restrict__ first_of,
                                                              uint8_t* __restrict__ flag8,
                                                              uint32_t* __restrict__ tilesum,
                                                              const SlotDesc* __restrict__ descs, int N,
@@ -564,7 +564,7 @@ __global__ __launch_bounds__(REMAP_THREADS) void k_lds_assign(
 }
 
 // mapped id = rank of the sign's first occurrence, relative to the slot.
-__global__ __launch_bounds__(256) void k_lds_mapped(const SlotDesc* __restrict__ descs,
+static __global__ __launch_bounds__(256) void k_lds_mapped(const SlotDesc* __restrict__ descs,
                                                     const uint32_t* __restrict__ lbase,
                                                     const uint32_t* __restrict__ ubase, int N, uint32_t L,
                                                     const uint32_t* __restrict__ first_of,
@@ -757,7 +757,7 @@ __global__ __launch_bounds__(GRP_THREADS) void k_group_count(uint32_t nb2, const
 }
 
 // Exclusive scan of the per-bucket counts (one workgroup); also the totals.
-__global__ __launch_bounds__(1024) void k_group_offsets(const uint4* __restrict__ bcounts, uint4* __restrict__ bbase,
+static __global__ __launch_bounds__(1024) void k_group_offsets(const uint4* __restrict__ bcounts, uint4* __restrict__ bbase,
                                                         uint32_t nb2, DevStatus* status) {
     constexpr int ITEMS = 8;
     __shared__ uint4 wsum[16];
@@ -815,7 +815,7 @@ __global__ __launch_bounds__(1024) void k_group_offsets(const uint4* __restrict_
 // newcnt[c] entries -- not one list of the call: places in one list are handed out by atomics on one counter,
 // which take about 11 ns each one after the other (one per wavefront, tens of thousands, took longer than all the
 // probes together; one per bucket still kept every workgroup waiting for its turn among a thousand).
-__global__ __launch_bounds__(256) void k_probe_recs(uint32_t nb2, const uint32_t* __restrict__ cursor2,
+static __global__ __launch_bounds__(256) void k_probe_recs(uint32_t nb2, const uint32_t* __restrict__ cursor2,
                                                     const GroupRec* __restrict__ recs, uint32_t* __restrict__ rrow,
                                                     uint32_t* __restrict__ newrec, uint32_t* __restrict__ newcnt,
                                                     Store s, DevStatus* status) {
@@ -865,7 +865,7 @@ __device__ __forceinline__ void init_row_pair(const Store& s, const OptDev& o, u
 // Fills the rows k_probe_recs inserted, `parts` workgroups per bucket's list (a batch of few buckets and many new
 // signs still fills the device) and one lane per pair of elements; the first workgroup also adds up the lists'
 // lengths: the call's number of new rows.
-__global__ __launch_bounds__(256) void k_init_new_recs(Store s, OptDev o, uint64_t seed,
+static __global__ __launch_bounds__(256) void k_init_new_recs(Store s, OptDev o, uint64_t seed,
                                                        const GroupRec* __restrict__ recs,
                                                        const uint32_t* __restrict__ rrow, uint32_t nb2,
                                                        const uint32_t* __restrict__ newrec,

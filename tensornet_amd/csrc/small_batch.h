@@ -257,12 +257,12 @@ __device__ __forceinline__ void small_slots(const SmallShape& b, const SmallPlan
     }
 }
 
-__global__ __launch_bounds__(SMALL_THREADS) void k_small_slots(SmallShape b, SmallPlan p, const SlotDesc* host_descs,
+static __global__ __launch_bounds__(SMALL_THREADS) void k_small_slots(SmallShape b, SmallPlan p, const SlotDesc* host_descs,
                                                                uint32_t entries, Store s, OptDev o, uint64_t seed,
                                                                DevStatus* status, uint64_t* host_words, uint32_t seq) {
     small_slots<SMALL_THREADS>(b, p, host_descs, entries, s, o, seed, status, host_words, seq);
 }
-__global__ __launch_bounds__(2 * SMALL_THREADS) void k_small_slots_long(SmallShape b, SmallPlan p, const SlotDesc* host_descs,
+static __global__ __launch_bounds__(2 * SMALL_THREADS) void k_small_slots_long(SmallShape b, SmallPlan p, const SlotDesc* host_descs,
                                                                         uint32_t entries, Store s, OptDev o, uint64_t seed,
                                                                         DevStatus* status, uint64_t* host_words, uint32_t seq) {
     small_slots<2 * SMALL_THREADS>(b, p, host_descs, entries, s, o, seed, status, host_words, seq);

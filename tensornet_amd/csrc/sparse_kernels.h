@@ -104,14 +104,14 @@ __device__ __forceinline__ uint32_t wave_alloc(bool flag, uint32_t* counter) {
 }
 
 // ------------------------------------------------------------------ fills
-__global__ __launch_bounds__(256) void k_fill_ff(uint4* p, size_t n16) {
+static __global__ __launch_bounds__(256) void k_fill_ff(uint4* p, size_t n16) {
     size_t stride = (size_t)gridDim.x * blockDim.x;
     uint4 v = make_uint4(0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu);
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n16; i += stride) p[i] = v;
 }
 
 // fills the first (status->gcap + 1) group entries
-__global__ __launch_bounds__(256) void k_fill_groups(GroupEntry* gt, const DevStatus* status) {
+static __global__ __launch_bounds__(256) void k_fill_groups(GroupEntry* gt, const DevStatus* status) {
     size_t n16 = (size_t)status->gcap + 1;
     size_t stride = (size_t)gridDim.x * blockDim.x;
     uint4 v = make_uint4(0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu);
@@ -119,7 +119,7 @@ __global__ __launch_bounds__(256) void k_fill_groups(GroupEntry* gt, const DevSt
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n16; i += stride) p[i] = v;
 }
 
-__global__ void k_reset_status(DevStatus* status, uint32_t n_unique, uint32_t gcap) {
+static __global__ void k_reset_status(DevStatus* status, uint32_t n_unique, uint32_t gcap) {
     if (threadIdx.x == 0 && blockIdx.x == 0) {
         status->err = 0;
         status->n_unique = n_unique;
@@ -142,7 +142,7 @@ __global__ void k_reset_status(DevStatus* status, uint32_t n_unique, uint32_t gc
 // the flags), clears `zero[0 .. n_zero)` and copies copy_n words from copy_src to copy_dst.
 enum { STATUS_KEEP = 0, STATUS_NEW_PLAN = 1, STATUS_REUSE_PLAN = 2 };
 
-__global__ __launch_bounds__(256) void k_stage_in(const uint32_t* __restrict__ host_src, uint32_t* __restrict__ dst_a,
+static __global__ __launch_bounds__(256) void k_stage_in(const uint32_t* __restrict__ host_src, uint32_t* __restrict__ dst_a,
                                                   uint32_t words_a, uint32_t* __restrict__ dst_b, uint32_t words_b,
                                                   DevStatus* status, int status_mode, uint32_t* __restrict__ zero,
                                                   uint32_t n_zero, const DevStatus* plan_status,
@@ -181,7 +181,7 @@ __global__ __launch_bounds__(256) void k_stage_in(const uint32_t* __restrict__ h
 // inserted are added to the table's number of resident keys.  With host_seq != nullptr the word seq is written
 // there once everything else is on the host: a host that polls that word has the status a few microseconds
 // after this kernel, well before a wait on the stream would return.
-__global__ __launch_bounds__(256) void k_publish(const DevStatus* __restrict__ status,
+static __global__ __launch_bounds__(256) void k_publish(const DevStatus* __restrict__ status,
                                                  const uint32_t* __restrict__ ubase, uint32_t n_ubase,
                                                  uint32_t* __restrict__ host_dst, unsigned long long* count,
                                                  uint32_t* host_seq, uint32_t seq) {
@@ -197,7 +197,7 @@ __global__ __launch_bounds__(256) void k_publish(const DevStatus* __restrict__ s
     }
 }
 
-__global__ void k_finish_insert(Store s, const DevStatus* status) {
+static __global__ void k_finish_insert(Store s, const DevStatus* status) {
     if (threadIdx.x == 0 && blockIdx.x == 0) *s.count += status->n_new;
 }
 
@@ -369,7 +369,7 @@ __device__ __forceinline__ void init_row(const Store& s, const OptDev& o, uint64
     init_state(s, o, s.st + row * s.sstride);
 }
 
-__global__ __launch_bounds__(256) void k_init_rows(Store s, OptDev o, uint64_t seed, const uint64_t* __restrict__ signs,
+static __global__ __launch_bounds__(256) void k_init_rows(Store s, OptDev o, uint64_t seed, const uint64_t* __restrict__ signs,
                                                    const uint32_t* __restrict__ rows,
                                                    const uint32_t* __restrict__ newlist, const DevStatus* status) {
     const uint32_t n_new = status->n_new;
@@ -394,7 +394,7 @@ struct DecayConf {
 //   AdaGrad  show *= rate; click *= rate; no_show_days += delta_days   (ada_grad_kernel.cc:191-195)
 //   Ftrl     show *= rate                                              (ftrl_kernel.cc:124)
 //   Adam     nothing                                                   (adam_kernel.h:67)
-__global__ __launch_bounds__(256) void k_show_decay(Store s, DecayConf c, int delta_days) {
+static __global__ __launch_bounds__(256) void k_show_decay(Store s, DecayConf c, int delta_days) {
     const uint64_t n = s.cap + 1;
     const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
@@ -414,7 +414,7 @@ __global__ __launch_bounds__(256) void k_show_decay(Store s, DecayConf c, int de
 // Value::DeleteByShow for the rows of given signs: out[i] = 1 if the row would be left out of a
 // saved table (optimizer_kernel.h:332,345; ada_grad_kernel.cc:197-204, ftrl_kernel.cc:126,
 // adam_kernel.h:69), 0 otherwise and for absent signs.
-__global__ __launch_bounds__(256) void k_delete_by_show(Store s, DecayConf c, const uint32_t* __restrict__ rows,
+static __global__ __launch_bounds__(256) void k_delete_by_show(Store s, DecayConf c, const uint32_t* __restrict__ rows,
                                                         int64_t n, uint8_t* __restrict__ out) {
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
@@ -437,7 +437,7 @@ __global__ __launch_bounds__(256) void k_delete_by_show(Store s, DecayConf c, co
 // the row of the sign 0xFFFF...F), compacted into signs / w / state in no particular order;
 // with skip_eliminated rows for which DeleteByShow holds are left out (what a saved table
 // holds, optimizer_kernel.h:332,345).  *count = rows written.
-__global__ __launch_bounds__(256) void k_export_range(Store s, DecayConf c, uint64_t first, uint64_t n_slots,
+static __global__ __launch_bounds__(256) void k_export_range(Store s, DecayConf c, uint64_t first, uint64_t n_slots,
                                                       int skip_eliminated, uint64_t* __restrict__ signs,
                                                       float* __restrict__ w, float* __restrict__ state,
                                                       uint32_t* count) {
@@ -500,7 +500,7 @@ __global__ __launch_bounds__(256) void k_gather_rows(Store s, const uint32_t* __
 }
 
 // Snapshot load: table row <- caller row (+ given or fresh state).
-__global__ __launch_bounds__(256) void k_load_rows(Store s, OptDev o, const uint32_t* __restrict__ rows, int64_t n,
+static __global__ __launch_bounds__(256) void k_load_rows(Store s, OptDev o, const uint32_t* __restrict__ rows, int64_t n,
                                                    const float* __restrict__ w, const float* __restrict__ state) {
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
@@ -520,7 +520,7 @@ __global__ __launch_bounds__(256) void k_load_rows(Store s, OptDev o, const uint
     }
 }
 
-__global__ __launch_bounds__(256) void k_export_rows(Store s, OptDev o, const uint32_t* __restrict__ rows, int64_t n,
+static __global__ __launch_bounds__(256) void k_export_rows(Store s, OptDev o, const uint32_t* __restrict__ rows, int64_t n,
                                                      float* __restrict__ w, float* __restrict__ state,
                                                      uint8_t* __restrict__ found) {
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
@@ -538,7 +538,7 @@ __global__ __launch_bounds__(256) void k_export_rows(Store s, OptDev o, const ui
 }
 
 // Re-insertion of every resident row into a larger table.
-__global__ __launch_bounds__(256) void k_rehash(Store from, Store to, DevStatus* status) {
+static __global__ __launch_bounds__(256) void k_rehash(Store from, Store to, DevStatus* status) {
     const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i <= from.cap; i += stride) {
         uint64_t dst;
@@ -647,7 +647,7 @@ __device__ __forceinline__ void load_lbase(uint32_t* sh, const uint32_t* lbase, 
 // Entries only ever change from EMPTY_KEY to a sign and minpos only decreases,
 // so ordinary (possibly stale) loads are safe: a stale value costs one atomic,
 // whose return value is the truth.
-__global__ __launch_bounds__(256) void k_remap_insert(const SlotDesc* __restrict__ descs,
+static __global__ __launch_bounds__(256) void k_remap_insert(const SlotDesc* __restrict__ descs,
                                                       const uint32_t* __restrict__ lbase, int N, uint32_t L,
                                                       DedupEntry* dt, uint32_t* __restrict__ tidx,
                                                       uint64_t* __restrict__ vals_copy) {
@@ -722,7 +722,7 @@ __device__ __forceinline__ T block_excl_scan_256(T v, T* sh /*4*/, T* total) {
 
 // Step 2: a lookup is a first occurrence iff its position equals its entry's
 // minpos.  One flag bit per lookup (8 per thread), one count per tile.
-__global__ __launch_bounds__(REMAP_THREADS) void k_flag_count(const uint32_t* __restrict__ lbase, int N, uint32_t L,
+static __global__ __launch_bounds__(REMAP_THREADS) void k_flag_count(const uint32_t* __restrict__ lbase, int N, uint32_t L,
                                                               const DedupEntry* __restrict__ dt,
                                                               const uint32_t* __restrict__ tidx,
                                                               uint8_t* __restrict__ flag8,
@@ -791,7 +791,7 @@ __device__ __forceinline__ uint32_t scan_u32_1024(const uint32_t* __restrict__ i
 
 // Step 3 (one workgroup): exclusive scan of the tile counts; total distinct
 // count U; size of the group table; ubase of trailing empty slots.
-__global__ __launch_bounds__(1024) void k_scan_tiles(const uint32_t* __restrict__ tilesum,
+static __global__ __launch_bounds__(1024) void k_scan_tiles(const uint32_t* __restrict__ tilesum,
                                                      uint32_t* __restrict__ tileoff, uint32_t ntiles,
                                                      const uint32_t* __restrict__ lbase, uint32_t* __restrict__ ubase,
                                                      int N, uint32_t L, DevStatus* status) {
@@ -809,7 +809,7 @@ __global__ __launch_bounds__(1024) void k_scan_tiles(const uint32_t* __restrict_
 
 // Step 4: rank of every first occurrence = number of first occurrences before
 // it in the concatenated order; the compact lists of distinct signs follow.
-__global__ __launch_bounds__(REMAP_THREADS) void k_assign_rank(
+static __global__ __launch_bounds__(REMAP_THREADS) void k_assign_rank(
     const SlotDesc* __restrict__ descs, const uint32_t* __restrict__ lbase, int N, uint32_t L, DedupEntry* dt,
     const uint32_t* __restrict__ tidx, const uint8_t* __restrict__ flag8, const uint32_t* __restrict__ tileoff,
     uint32_t* __restrict__ ubase, uint64_t* __restrict__ uniq_sign, uint32_t* __restrict__ uniq_slot) {
@@ -845,7 +845,7 @@ constexpr uint32_t FIRST_BIT = 0x80000000u;
 // Step 5: mapped id = rank within the slot (sparse_table_ops.cc:130).  The
 // index of each lookup's distinct sign is kept for the push (u_of_gi, top bit
 // set on first occurrences).
-__global__ __launch_bounds__(256) void k_write_mapped(const SlotDesc* __restrict__ descs,
+static __global__ __launch_bounds__(256) void k_write_mapped(const SlotDesc* __restrict__ descs,
                                                       const uint32_t* __restrict__ lbase,
                                                       const uint32_t* __restrict__ ubase, int N, uint32_t L,
                                                       const DedupEntry* __restrict__ dt,
@@ -869,7 +869,7 @@ __global__ __launch_bounds__(256) void k_write_mapped(const SlotDesc* __restrict
 // Push: batch_show = occurrences, batch_click = sum of labels per distinct sign
 // (sparse_table_ops.cc:283-296; labels are narrowed to int as there), kept in
 // the member lists.  Every sign starts at show 1 / click 0 ...
-__global__ __launch_bounds__(256) void k_reset_counts(Member* __restrict__ list, const DevStatus* status,
+static __global__ __launch_bounds__(256) void k_reset_counts(Member* __restrict__ list, const DevStatus* status,
                                                       uint32_t ids_cap, int keep_show) {
     const uint32_t n_single = status->n_single, n_members = status->n_members;
     const uint32_t stride = gridDim.x * blockDim.x;
@@ -886,7 +886,7 @@ constexpr int COUNT_SLOTS = 4096;  // LDS table entries per tile (load factor <=
 // ... and the repeated lookups and the non-zero labels are added.  Repeats
 // are concentrated on few signs, so each tile of 2048 lookups first adds them
 // up in an LDS hash table and issues one global atomic per sign it saw.
-__global__ __launch_bounds__(256) void k_count_show(const SlotDesc* __restrict__ descs,
+static __global__ __launch_bounds__(256) void k_count_show(const SlotDesc* __restrict__ descs,
                                                     const uint32_t* __restrict__ lbase, int N, uint32_t L,
                                                     const uint32_t* __restrict__ u_of_gi,
                                                     const uint2* __restrict__ where_u, Member* list,
@@ -959,7 +959,7 @@ __device__ __forceinline__ uint64_t src_sign(const PushSrc& p, uint32_t u) {
 
 // Records with the same sign must be applied one after the other in record
 // order (sparse_table.cc:72-82).  Every record joins the group of its sign...
-__global__ __launch_bounds__(256) void k_group_insert(PushSrc src, int64_t n_host, DevStatus* status, GroupEntry* gt,
+static __global__ __launch_bounds__(256) void k_group_insert(PushSrc src, int64_t n_host, DevStatus* status, GroupEntry* gt,
                                                       uint32_t* __restrict__ gidx, uint32_t* __restrict__ ord) {
     const int64_t n = src.infos ? n_host : (int64_t)status->n_unique;
     const uint32_t gcap = status->gcap;
@@ -1044,7 +1044,7 @@ __device__ __forceinline__ void compact_span(DevStatus* status, const uint32_t (
 }
 
 // ...every group gets a number and a slice of the member array...
-__global__ __launch_bounds__(256) void k_group_compact(DevStatus* status, GroupEntry* gt,
+static __global__ __launch_bounds__(256) void k_group_compact(DevStatus* status, GroupEntry* gt,
                                                        uint64_t* __restrict__ grp_sign,
                                                        uint32_t* __restrict__ grp_off,
                                                        uint32_t* __restrict__ grp_cnt,
@@ -1070,7 +1070,7 @@ __global__ __launch_bounds__(256) void k_group_compact(DevStatus* status, GroupE
 }
 
 // ...the members are written into it in arrival order...
-__global__ __launch_bounds__(256) void k_group_fill(int64_t n_host, const uint32_t* n_dev, const GroupEntry* gt,
+static __global__ __launch_bounds__(256) void k_group_fill(int64_t n_host, const uint32_t* n_dev, const GroupEntry* gt,
                                                     const uint32_t* __restrict__ grp_off,
                                                     const uint32_t* __restrict__ gidx,
                                                     const uint32_t* __restrict__ ord, uint32_t* __restrict__ arrival) {
@@ -1082,7 +1082,7 @@ __global__ __launch_bounds__(256) void k_group_fill(int64_t n_host, const uint32
 
 // ...and finally put in ascending record order: the place of a record is the
 // number of members of its group that precede it.
-__global__ __launch_bounds__(256) void k_group_rank(int64_t n_host, const uint32_t* n_dev, const GroupEntry* gt,
+static __global__ __launch_bounds__(256) void k_group_rank(int64_t n_host, const uint32_t* n_dev, const GroupEntry* gt,
                                                     const uint32_t* __restrict__ grp_off,
                                                     const uint32_t* __restrict__ gidx,
                                                     const uint32_t* __restrict__ arrival,
@@ -1125,7 +1125,7 @@ struct MaskEntry {
     uint64_t nlo, nhi;  // complemented slot masks (16-byte aligned)
 };
 
-__global__ __launch_bounds__(256) void k_fill_masks(MaskEntry* gt, const DevStatus* status) {
+static __global__ __launch_bounds__(256) void k_fill_masks(MaskEntry* gt, const DevStatus* status) {
     size_t n16 = ((size_t)status->gcap + 1) * 2;
     size_t stride = (size_t)gridDim.x * blockDim.x;
     uint4 v = make_uint4(0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu);
@@ -1133,7 +1133,7 @@ __global__ __launch_bounds__(256) void k_fill_masks(MaskEntry* gt, const DevStat
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n16; i += stride) p[i] = v;
 }
 
-__global__ __launch_bounds__(256) void k_mask_insert(const uint64_t* __restrict__ uniq_sign,
+static __global__ __launch_bounds__(256) void k_mask_insert(const uint64_t* __restrict__ uniq_sign,
                                                      const uint32_t* __restrict__ uniq_slot, DevStatus* status,
                                                      MaskEntry* gt, uint32_t* __restrict__ gidx) {
     const uint32_t n = status->n_unique;
@@ -1163,7 +1163,7 @@ __global__ __launch_bounds__(256) void k_mask_insert(const uint64_t* __restrict_
     }
 }
 
-__global__ __launch_bounds__(256) void k_mask_compact(DevStatus* status, MaskEntry* gt,
+static __global__ __launch_bounds__(256) void k_mask_compact(DevStatus* status, MaskEntry* gt,
                                                       uint64_t* __restrict__ grp_sign,
                                                       uint32_t* __restrict__ grp_off,
                                                       uint32_t* __restrict__ grp_cnt,
@@ -1191,7 +1191,7 @@ __global__ __launch_bounds__(256) void k_mask_compact(DevStatus* status, MaskEnt
     }
 }
 
-__global__ __launch_bounds__(256) void k_mask_fill(const DevStatus* status, const MaskEntry* gt,
+static __global__ __launch_bounds__(256) void k_mask_fill(const DevStatus* status, const MaskEntry* gt,
                                                    const uint32_t* __restrict__ gidx,
                                                    const uint32_t* __restrict__ uniq_slot,
                                                    const uint32_t* __restrict__ ushow, Member* __restrict__ list,
@@ -1299,7 +1299,7 @@ __device__ __forceinline__ bool record_at(const PushSrc& p, const Member* mem, c
 // top of the member array): gaddr[place], nullptr where the op's gradient matrix has no such row.
 // One coalesced pass that takes the slot descriptor out of the per-record chains of the apply
 // kernels for those groups.
-__global__ __launch_bounds__(256) void k_member_grads(PushSrc src, const DevStatus* status,
+static __global__ __launch_bounds__(256) void k_member_grads(PushSrc src, const DevStatus* status,
                                                       const Member* __restrict__ list,
                                                       const float** __restrict__ gaddr, uint32_t ids_cap) {
     if (status->mismatch | status->abort) return;

@@ -1,6 +1,7 @@
 // SparseTable host side: registry, HBM storage management and the launch
 // sequences of pull / push at table level (core/ps/table/sparse_table.cc:52-83)
 // and at operator level (core/kernels/sparse_table_ops.cc:170-265,317-368).
+#include "apply_launch.h"
 #include "combine_kernels.h"
 #include "remap_lds.h"
 #include "table_level.h"
@@ -987,20 +988,6 @@ int launch_build_plan(SparseTable* t, const Plan& p, const Scratch& w, int N, ui
     return TN_OK;
 }
 
-// How the update kernels share a row out: `lanes` lanes, four elements each (0: the row is too long for that).
-// any: the rows do not fill the lanes, or stand at other than 16-byte boundaries (row_part<true>).
-struct RowShare {
-    int lanes;
-    bool any;
-};
-RowShare row_share(const Store& s, bool aligned) {
-    RowShare r{1, !aligned || s.D % 4 != 0};
-    while (4 * r.lanes < s.D) r.lanes *= 2;
-    if (4 * r.lanes != s.D) r.any = true;
-    if (r.lanes > 32) r.lanes = 0;
-    return r;
-}
-
 // workgroups of k_apply_all for the signs with many records at most (a wavefront each in turn)
 constexpr int ALL_BIG_GRID = 1024;
 
@@ -1148,53 +1135,17 @@ int launch_apply(SparseTable* t, const Plan& p, const PushSrc& src, DevStatus* d
     }
 }
 
-// The updates of a small push, one launch (k_small_apply), with the workgroups for the signs with many records if the
-// plan lists such.  flat: the reduced rows of pooled gradients, else nullptr.
-template <int KIND>
-int launch_small_apply_kind(SparseTable* t, RowShare share, const OptDev& o, const SmallPlan& p, const float* flat, int dim,
-                            hipStream_t st, uint32_t* host_seq, uint32_t seq) {
-    const Store& s = t->store;
+// The updates of a small push, one launch (k_small_apply), with the signs with many records if the plan lists such.  flat: the
+// reduced rows of pooled gradients, else nullptr.
+void launch_small_apply(SparseTable* t, RowShare share, const SmallPlan& p, const float* flat, int dim, hipStream_t st,
+                        uint32_t* host_seq, uint32_t seq) {
     const SmallShape& b = t->small_shape;
     const bool with_big = t->plan_big_k != 0xFFFFFFFFu && (uint32_t)b.N >= t->plan_big_k;
-    const int gfloats = small_gbuf_floats(s.D, b.N);
-    const size_t arrays = align_up((size_t)(gfloats + 3 * s.D) * sizeof(float), 8), wave_lds = arrays + BIG_CHUNK * (8 + 4);
-    const bool lds_big = with_big && (s.D > 64 || (s.D & (s.D - 1)) != 0);  // (others keep their staging in static LDS)
-    const size_t lds = small_apply_slots_lds(flat ? 0 : b.N) + (lds_big ? 4 * wave_lds : 0);
-#define TN_LAUNCH_SMALL_BIG(LPG, ANY, BIG)                                                                             \
-    TN_LAUNCH_LDS((k_small_apply<KIND, LPG, ANY, BIG>), dim3(b.buckets()), dim3(256), lds, st, b, p, flat, s, o,       \
-                  (const DevStatus*)t->dplan, host_seq, seq, dim, gfloats, (uint32_t)wave_lds, (uint32_t)arrays)
-// (aligned rows that fill their lanes have 4, 8 .. 128 elements; of these the last are too long for apply_big_wave)
-#define TN_LAUNCH_SMALL_ROWS(LPG)                                                                     \
-    do {                                                                                              \
-        constexpr int WAVE = LPG <= 16 ? 4 * LPG : BIG_GROUPS;                                        \
-        if (!with_big && share.any) TN_LAUNCH_SMALL_BIG(LPG, true, BIG_NONE);                         \
-        else if (!with_big) TN_LAUNCH_SMALL_BIG(LPG, false, BIG_NONE);                                \
-        else if (!share.any) TN_LAUNCH_SMALL_BIG(LPG, false, WAVE);                                   \
-        else if (lds_big) TN_LAUNCH_SMALL_BIG(LPG, true, BIG_GROUPS);                                 \
-        else if (s.D == 1) TN_LAUNCH_SMALL_BIG(LPG, true, (LPG == 1 ? 1 : WAVE));                     \
-        else if (s.D == 2) TN_LAUNCH_SMALL_BIG(LPG, true, (LPG == 1 ? 2 : WAVE));                     \
-        else TN_LAUNCH_SMALL_BIG(LPG, true, WAVE);                                                    \
-    } while (0)
-    switch (share.lanes) {
-        case 1: TN_LAUNCH_SMALL_ROWS(1); break;
-        case 2: TN_LAUNCH_SMALL_ROWS(2); break;
-        case 4: TN_LAUNCH_SMALL_ROWS(4); break;
-        case 8: TN_LAUNCH_SMALL_ROWS(8); break;
-        case 16: TN_LAUNCH_SMALL_ROWS(16); break;
-        default: TN_LAUNCH_SMALL_ROWS(32); break;
-    }
-#undef TN_LAUNCH_SMALL_ROWS
-#undef TN_LAUNCH_SMALL_BIG
-    return TN_OK;
-}
-
-int launch_small_apply(SparseTable* t, RowShare share, const SmallPlan& p, const float* flat, int dim, hipStream_t st,
-                       uint32_t* host_seq, uint32_t seq) {
-    const OptDev o = make_optdev(t);
-    switch (o.kind) {
-        case OPT_ADAGRAD: return launch_small_apply_kind<OPT_ADAGRAD>(t, share, o, p, flat, dim, st, host_seq, seq);
-        case OPT_ADAM: return launch_small_apply_kind<OPT_ADAM>(t, share, o, p, flat, dim, st, host_seq, seq);
-        default: return launch_small_apply_kind<OPT_FTRL>(t, share, o, p, flat, dim, st, host_seq, seq);
+    const SmallApplyCall c{b, p, flat, t->store, make_optdev(t), t->dplan, host_seq, seq, dim, share, with_big, st};
+    switch (c.o.kind) {
+        case OPT_ADAGRAD: return tn::launch_small_apply<OPT_ADAGRAD>(c);
+        case OPT_ADAM: return tn::launch_small_apply<OPT_ADAM>(c);
+        default: return tn::launch_small_apply<OPT_FTRL>(c);
     }
 }
 
@@ -1226,22 +1177,6 @@ int launch_small_pool(SparseTable* t, bool aligned, const SmallPlan& p, int64_t 
     return TN_OK;
 }
 
-// Bytes of dynamic LDS a workgroup of `kernel` may have on this device (128 KB at most), after telling the
-// runtime that the kernel wants them.
-size_t big_lds_bytes_for(const void* kernel, size_t cap = 128 * 1024) {
-    int dev = 0, most = 0;
-    size_t bytes = 48 * 1024;
-    if (hipGetDevice(&dev) == hipSuccess &&
-        hipDeviceGetAttribute(&most, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) == hipSuccess && most > 2048)
-        bytes = std::min<size_t>((size_t)most - 2048, cap);  // (room for the kernel's static arrays)
-    if (bytes > 48 * 1024 &&
-        hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) != hipSuccess) {
-        (void)hipGetLastError();
-        bytes = 48 * 1024;
-    }
-    return bytes;
-}
-
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 size_t carve_small(char* base, SmallPlan& p, const SmallShape& b) {
@@ -1265,48 +1200,14 @@ size_t carve_small(char* base, SmallPlan& p, const SmallShape& b) {
 }
 
 // The updates of a table-level push (k_table_apply).
-template <int KIND>
-int launch_table_apply_kind(SparseTable* t, RowShare share, const OptDev& o, const TableShape& b, const tn_sign_info* infos,
-                            const float* grads, int dim, const uint2* recs, const uint16_t* boff, DevStatus* ds, hipStream_t st) {
-    const Store& s = t->store;
-    const size_t wave_lds = small_apply_wave_lds(s.D), lists = table_apply_lists_lds(b.tiles);
-#define TN_LAUNCH_TABLE_ANY(LPG, ANY)                                                                                   \
-    do {                                                                                                                \
-        if (!t->table_lds[ANY]) {                                                                                       \
-            t->table_lds[ANY] = true;                                                                                   \
-            (void)big_lds_bytes_for(reinterpret_cast<const void*>(k_table_apply<KIND, LPG, ANY>));                      \
-        }                                                                                                               \
-        TN_LAUNCH_LDS((k_table_apply<KIND, LPG, ANY>), dim3(b.nb), dim3(256), lists + 4 * wave_lds, st, b, s, o, infos, \
-                      grads, dim, recs, boff, ds, &t->hpush->st.err, big_gbuf_floats(s.D), (uint32_t)wave_lds,          \
-                      (uint32_t)align_up(big_lds_bytes(s.D), 8), (uint32_t)lists);                                      \
-    } while (0)
-#define TN_LAUNCH_TABLE(LPG)                  \
-    do {                                      \
-        if (share.any)                        \
-            TN_LAUNCH_TABLE_ANY(LPG, true);   \
-        else                                  \
-            TN_LAUNCH_TABLE_ANY(LPG, false);  \
-    } while (0)
-    switch (share.lanes) {
-        case 1: TN_LAUNCH_TABLE(1); break;
-        case 2: TN_LAUNCH_TABLE(2); break;
-        case 4: TN_LAUNCH_TABLE(4); break;
-        case 8: TN_LAUNCH_TABLE(8); break;
-        case 16: TN_LAUNCH_TABLE(16); break;
-        default: TN_LAUNCH_TABLE(32); break;
-    }
-#undef TN_LAUNCH_TABLE
-#undef TN_LAUNCH_TABLE_ANY
-    return TN_OK;
-}
-
-int launch_table_apply(SparseTable* t, RowShare share, const TableShape& b, const tn_sign_info* infos, const float* grads,
-                       int dim, const uint2* recs, const uint16_t* boff, DevStatus* ds, hipStream_t st) {
-    const OptDev o = make_optdev(t);
-    switch (o.kind) {
-        case OPT_ADAGRAD: return launch_table_apply_kind<OPT_ADAGRAD>(t, share, o, b, infos, grads, dim, recs, boff, ds, st);
-        case OPT_ADAM: return launch_table_apply_kind<OPT_ADAM>(t, share, o, b, infos, grads, dim, recs, boff, ds, st);
-        default: return launch_table_apply_kind<OPT_FTRL>(t, share, o, b, infos, grads, dim, recs, boff, ds, st);
+void launch_table_apply(SparseTable* t, RowShare share, const TableShape& b, const tn_sign_info* infos, const float* grads,
+                        int dim, const uint2* recs, const uint16_t* boff, DevStatus* ds, hipStream_t st) {
+    const TableApplyCall c{b, t->store, make_optdev(t), infos, grads, dim, recs, boff, ds, &t->hpush->st.err, share, st,
+                           t->table_lds};
+    switch (c.o.kind) {
+        case OPT_ADAGRAD: return tn::launch_table_apply<OPT_ADAGRAD>(c);
+        case OPT_ADAM: return tn::launch_table_apply<OPT_ADAM>(c);
+        default: return tn::launch_table_apply<OPT_FTRL>(c);
     }
 }
 
@@ -1527,7 +1428,7 @@ int small_push(SparseTable* t, const int64_t* const* values, const float* const*
     const bool rows16 = dim % 4 == 0 && t->store.wstride % 4 == 0;
     if (pooled)
         TN_TRY(launch_small_pool(t, vec, p, batch, dim, combiner, flat, st, &t->hpush->st.abort));
-    TN_TRY(launch_small_apply(t, row_share(t->store, (pooled || vec) && rows16), p, flat, dim, st, t->hseq + 1, seq));
+    launch_small_apply(t, row_share(t->store, (pooled || vec) && rows16), p, flat, dim, st, t->hseq + 1, seq);
     // what a call on another stream has to wait for: the updates are still running when this call returns
     TN_HIP(hipEventRecord(t->tail_ev, st));
     t->tail_recorded = true;
@@ -1948,7 +1849,7 @@ int tn_sparse_table_push(uint32_t handle, const tn_sign_info* infos, const float
         else
             TN_LAUNCH_LDS((k_table_part<16>), dim3(b.tiles), dim3(TABLE_THREADS), part_lds, st, b, s, infos, recs, boff, ds);
         t->hpush->st.err = 0;
-        TN_TRY(launch_table_apply(t, share, b, infos, grads, dim, recs, boff, ds, st));
+        launch_table_apply(t, share, b, infos, grads, dim, recs, boff, ds, st);
         TN_HIP(hipGetLastError());
         t->push_pending = true;
         t->push_slots = 0;

@@ -25,7 +25,7 @@ constexpr uint32_t TABLE_PULL_FEW = 256;     // ... as many as there are CUs: wi
 // workgroup that holds the same sign may copy it too early, so a request that inserted anything is copied out once more
 // (k_gather_rows, from rows[]).  Every workgroup tells the host itself: rows inserted | out of slots << 31 | seq << 32.
 // Bound by the two dependent reads of a row (keys, then weights).
-__global__ __launch_bounds__(256) void k_table_pull(Store s, OptDev o, uint64_t seed, const uint64_t* __restrict__ signs,
+static __global__ __launch_bounds__(256) void k_table_pull(Store s, OptDev o, uint64_t seed, const uint64_t* __restrict__ signs,
                                                     int64_t n, uint32_t per, int vec, float* __restrict__ out,
                                                     uint32_t* __restrict__ rows, uint64_t* host_words, uint32_t seq) {
     __shared__ uint32_t row[256];

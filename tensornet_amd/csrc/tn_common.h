@@ -181,6 +181,10 @@ struct DevBuf {
 
 int launch_grid(int64_t work_items, int threads, int max_blocks);
 
+// Bytes of dynamic LDS a workgroup of `kernel` may have on this device (cap at most), after telling the runtime that the
+// kernel wants them.
+size_t big_lds_bytes_for(const void* kernel, size_t cap = 128 * 1024);
+
 // Host-side access to a dense table for the checkpoint code (defined beside the table).
 struct DenseMeta {
     int kind;  // OPT_ADAM / OPT_ADAGRAD
