@@ -855,8 +855,11 @@ __device__ __forceinline__ void apply_group_ahead(const Store& s, const OptDev& 
 //   AdaGrad  g2sum (a lane per record, double sum of squares first) | steps lr g / den by all lanes | subtractions
 //   Adam     m and v | steps lr m / (eps + sqrt(v)) by all lanes | subtractions
 //   Ftrl     n | sqrt(n), the quotient of the weight and the factor of z by all lanes | z and w
-// The same operations on the same operands as record after record.  300 slots of 300 lookups, AdaGrad rows of 32 (signs with
-// 300 records): k_small_apply 78 -> 60 us; 40 slots of 8192, Ftrl rows of 1: 32 -> 26.
+// The same operations on the same operands as record after record.  What a chunk of 64 records takes at D = 16 under AdaGrad was
+// 9 us, 3.3 of them the g2sum chain (a branch per record), 1.4 each the divisions (one round after the other) and the
+// subtractions (LDS reads between them): the chain now runs on zeros where there is no gradient, the divisions of four rounds
+// and the reads of the next subtractions are under way together.  300 slots of 300 lookups, AdaGrad rows of 32 (signs with 300
+// records): k_small_apply 78 -> 41 us (60 before the latter); 40 slots of 8192, rows of 64: 66 -> 55; Ftrl rows of 1: 32 -> 23.
 template <int KIND, int D>
 struct BigWave {
     static constexpr int R = 64 / D, DP = D + 1;  // records a round; padded row: lanes walking down a column hit different banks
@@ -871,27 +874,28 @@ struct BigWave {
     float den[CHUNK];
 };
 
-// x0 + the sum of `v` over the lanes below n, added one after the other; many at once where that is exact (whole numbers).
-__device__ __forceinline__ float ordered_sum(float x0, int v, int n, unsigned long long okmask) {
-    if (n <= 16) {
-        const float few = (float)v;
-        for (int m = 0; m < n; m++)
-            if ((okmask >> m) & 1ull) x0 += lane_value(few, m);
-        return x0;
-    }
-    int all = v;
-#pragma unroll
-    for (int o = 1; o < 64; o *= 2) all += __shfl_xor(all, o);
-    const float most = 16777216.f;
-    if (x0 == truncf(x0) && x0 >= 0.f && x0 < most / 2 && all >= 0 && all < (1 << 23) && !__any(v < 0)) return x0 + (float)all;
+// The sum of v over the wavefront, in every lane (all of them call it).
+__device__ __forceinline__ int wave_sum(int v) {
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, false);  // row_shr:1, 2, 4, 8: lane 15 of a row has the row's
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xA, 0xF, false);  // row_bcast:15 into rows 1 and 3
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xC, 0xF, false);  // row_bcast:31 into rows 2 and 3
+    return __builtin_amdgcn_readlane(v, 63);
+}
+
+// x0 + v of the lanes 0, 1, ... below n, added one after the other; at once where that is exact (whole numbers).
+__device__ __forceinline__ float ordered_sum(float x0, int v, int n) {
+    if (x0 == truncf(x0) && x0 >= 0.f && x0 < 8388608.f && !__any(v < 0 || v >= (1 << 16))) return x0 + (float)wave_sum(v);
     const float f = (float)v;
-    for (int m = 0; m < n; m++)
-        if ((okmask >> m) & 1ull) x0 += lane_value(f, m);
+    for (int m = 0; m < n; m++) x0 += lane_value(f, m);
     return x0;
 }
 
 // The signs bi0, bi0 + stride, ... below n_big; head: {row, first member, records} of the first, describe(bi): of another;
-// entry(at): member `at`; record(entry, gradient, show, click): whether it has a gradient; missing(): one had none.
+// entry(at): member `at`; record(entry, gradient, show, click, there): whether it has a gradient (there: the lane's record is
+// one of the chunk's, and not a later chunk's or the last one again); missing(): one had none.
 template <int KIND, int D, typename Describe, typename Member, typename Record, typename Missing>
 __device__ __forceinline__ void apply_big_wave(const Store& s, const OptDev& o, BigWave<KIND, D>& lds, uint4 head, uint32_t bi0,
                                                uint32_t stride, uint32_t n_big, Describe describe, Member entry, Record record,
@@ -927,32 +931,30 @@ __device__ __forceinline__ void apply_big_wave(const Store& s, const OptDev& o, 
         float v[ROUNDS];
         int sh = 0, ck = 0;
         unsigned long long okmask = 0;
-        // gradients of the chunk from c0 on, whose entries are e, on their way
+        // Gradients of the chunk from c0 on, whose entries are e, on their way.  (Every load is issued, the row's in the place
+        // of a gradient there is not: under a condition each they are a branch each.)
         auto fetch = [&](uint32_t c0, const auto& e) {
-            const int cn = (int)min(k - c0, (uint32_t)CHUNK);
-            bool ok = false;
-            sh = ck = 0;
-            if (lane < cn) {
-                const float* gp = nullptr;
-                ok = record(e, gp, sh, ck);
-                lds.gptr[lane] = gp;
-            }
+            const float* gp = nullptr;
+            const bool there = lane < CHUNK && c0 + (uint32_t)lane < k;
+            const bool ok = record(e, gp, sh, ck, there) && there;
             okmask = __ballot(ok);
-            if (!ok) sh = ck = 0;
+            if (lane < CHUNK) lds.gptr[lane] = ok ? gp : wp;
             wave_sync();
+            const float* from[ROUNDS];
 #pragma unroll
-            for (int q = 0; q < ROUNDS; q++) {
-                const int m = lm + q * R;
-                v[q] = (m < cn && ((okmask >> m) & 1ull)) ? as_global(lds.gptr[m])[li] : 0.f;
-            }
+            for (int q = 0; q < ROUNDS; q++) from[q] = lds.gptr[lm + q * R];
+#pragma unroll
+            for (int q = 0; q < ROUNDS; q++) v[q] = as_global(from[q])[li];
         };
         fetch(0, now);
         bool any = false;
         for (uint32_t c0 = 0; c0 < k; c0 += CHUNK) {
-            const int cn = (int)min(k - c0, (uint32_t)CHUNK), csh = sh, cck = ck;
+            const int cn = (int)min(k - c0, (uint32_t)CHUNK);
             const unsigned long long mask = okmask, all = cn == 64 ? ~0ull : (1ull << cn) - 1ull;
+            const bool mine = (mask >> lane) & 1ull;
+            const int csh = mine ? sh : 0, cck = KIND == OPT_ADAGRAD && mine ? ck : 0;
 #pragma unroll
-            for (int q = 0; q < ROUNDS; q++) gbuf[(lm + q * R) * DP + li] = v[q];
+            for (int q = 0; q < ROUNDS; q++) gbuf[(lm + q * R) * DP + li] = (mask >> (lm + q * R)) & 1ull ? v[q] : 0.f;
             wave_sync();
             if (c0 + CHUNK < k) {
                 now = next;
@@ -960,7 +962,7 @@ __device__ __forceinline__ void apply_big_wave(const Store& s, const OptDev& o, 
                 fetch(c0 + CHUNK, now);
             }
             if (KIND == OPT_ADAGRAD) {
-                // add_g2sum / dim of record `lane`: double sum of float products in element order
+                // add_g2sum / dim of record `lane`: double sum of float products in element order (no gradient: zero)
                 double mq = 0.0;
                 if (lane < cn) {
                     const float* gr = gbuf + lane * DP;
@@ -976,33 +978,43 @@ __device__ __forceinline__ void apply_big_wave(const Store& s, const OptDev& o, 
                     }
                     mq = tot * (1.0 / (double)D);  // (exact: D is a power of two)
                 }
-                show = ordered_sum(show, csh, cn, mask);
-                click = ordered_sum(click, cck, cn, mask);
+                show = ordered_sum(show, csh, cn);
+                click = ordered_sum(click, cck, cn);
                 // g2sum after every record (float += double, rounded each time): every lane runs the chain on values read
-                // out of the records' lanes, lane m keeps the g2sum its record meets
+                // out of the records' lanes, lane m keeps the g2sum its record meets.  (Behind the last record and for one
+                // without a gradient zeros are added, which changes nothing.)
                 float myg2 = 0.f;
                 for (int m0 = 0; m0 < cn; m0 += 8) {
                     double x[8];
 #pragma unroll
-                    for (int j = 0; j < 8; j++) x[j] = lane_value(mq, min(m0 + j, 63));
+                    for (int j = 0; j < 8; j++) x[j] = lane_value(mq, m0 + j);
 #pragma unroll
                     for (int j = 0; j < 8; j++) {
-                        if (m0 + j < cn && ((mask >> (m0 + j)) & 1ull)) g2sum = (float)((double)g2sum + x[j]);
-                        if (lane == m0 + j) myg2 = g2sum;
+                        g2sum = (float)((double)g2sum + x[j]);
+                        myg2 = lane == m0 + j ? g2sum : myg2;
                     }
                 }
-                if (lane < cn) lds.den[lane] = o.eps + sqrtf(myg2);
+                if (lane < CHUNK) lds.den[lane] = o.eps + sqrtf(myg2);
                 wave_sync();
-#pragma unroll 4
-                for (int m = lm; m < cn; m += R) {  // a record without a gradient row steps by zero
-                    const float gv = gbuf[m * DP + li], dn = lds.den[m];
-                    gbuf[m * DP + li] = ((mask >> m) & 1ull) ? o.lr * gv / dn : 0.f;
+                constexpr int SIDE = ROUNDS < 4 ? ROUNDS : 4;  // rounds side by side
+                for (int q0 = 0; q0 * R < cn; q0 += SIDE) {
+                    float gv[SIDE], dn[SIDE];
+#pragma unroll
+                    for (int q = 0; q < SIDE; q++) {
+                        gv[q] = gbuf[(lm + (q0 + q) * R) * DP + li];
+                        dn[q] = lds.den[lm + (q0 + q) * R];
+                    }
+#pragma unroll
+                    for (int q = 0; q < SIDE; q++) gv[q] = o.lr * gv[q] / dn[q];
+                    // (a record without a gradient row has zeros, and a step of zero or, on a fresh row, no number: set to zero)
+#pragma unroll
+                    for (int q = 0; q < SIDE; q++) {
+                        const int m = lm + (q0 + q) * R;
+                        gbuf[m * DP + li] = (mask >> m) & 1ull ? gv[q] : 0.f;
+                    }
                 }
             } else {
-                int shown = csh;
-#pragma unroll
-                for (int x = 1; x < 64; x *= 2) shown += __shfl_xor(shown, x);
-                delta_show += shown;
+                delta_show += wave_sum(csh);
                 const float n0 = b;
                 if (lane < D) {
                     for (int m0 = 0; m0 < cn; m0 += 8) {
@@ -1027,10 +1039,21 @@ __device__ __forceinline__ void apply_big_wave(const Store& s, const OptDev& o, 
                 }
                 wave_sync();
                 if (KIND == OPT_ADAM) {
-#pragma unroll 4
-                    for (int m = lm; m < cn; m += R) {
-                        const float am = gbuf[m * DP + li], bm = vbuf[m * DP + li];
-                        gbuf[m * DP + li] = ((mask >> m) & 1ull) ? o.lr * am / (o.eps + sqrtf(bm)) : 0.f;
+                    constexpr int SIDE = ROUNDS < 4 ? ROUNDS : 4;
+                    for (int q0 = 0; q0 * R < cn; q0 += SIDE) {
+                        float am[SIDE], bm[SIDE];
+#pragma unroll
+                        for (int q = 0; q < SIDE; q++) {
+                            am[q] = gbuf[(lm + (q0 + q) * R) * DP + li];
+                            bm[q] = vbuf[(lm + (q0 + q) * R) * DP + li];
+                        }
+#pragma unroll
+                        for (int q = 0; q < SIDE; q++) am[q] = o.lr * am[q] / (o.eps + sqrtf(bm[q]));
+#pragma unroll
+                        for (int q = 0; q < SIDE; q++) {
+                            const int m = lm + (q0 + q) * R;
+                            gbuf[m * DP + li] = (mask >> m) & 1ull ? am[q] : 0.f;
+                        }
                     }
                 } else {
                     const float first = __shfl(n0, li);
@@ -1053,30 +1076,39 @@ __device__ __forceinline__ void apply_big_wave(const Store& s, const OptDev& o, 
                 }
             }
             wave_sync();
-            if (lane < D) {
+            if (KIND != OPT_FTRL) {
+                // (what lies behind the last record steps by nothing)
+                constexpr int AHEAD = CHUNK < 16 ? CHUNK : 16;
+                if (lane < D) {
+                    float t[AHEAD], u[AHEAD];
+#pragma unroll
+                    for (int j = 0; j < AHEAD; j++) t[j] = gbuf[j * DP + lane];
+                    for (int m0 = 0; m0 < cn; m0 += AHEAD) {
+#pragma unroll
+                        for (int j = 0; j < AHEAD; j++) u[j] = gbuf[min(m0 + AHEAD + j, CHUNK - 1) * DP + lane];
+#pragma unroll
+                        for (int j = 0; j < AHEAD; j++) w -= m0 + j < cn ? t[j] : 0.f;
+#pragma unroll
+                        for (int j = 0; j < AHEAD; j++) t[j] = u[j];
+                    }
+                }
+            } else if (lane < D) {
                 for (int m0 = 0; m0 < cn; m0 += 8) {
-                    if (KIND != OPT_FTRL) {
-                        float t[8];
+                    float g[8], t[8], f[8];
 #pragma unroll
-                        for (int j = 0; j < 8; j++) t[j] = m0 + j < cn ? gbuf[(m0 + j) * DP + lane] : 0.f;
+                    for (int j = 0; j < 8; j++) {
+                        const int at = min(m0 + j, cn - 1) * DP + lane;
+                        g[j] = gbuf[at];
+                        t[j] = vbuf[at];
+                        f[j] = qbuf[at];
+                    }
 #pragma unroll
-                        for (int j = 0; j < 8; j++) w -= t[j];
-                    } else {
-                        float g[8], t[8], f[8];
-#pragma unroll
-                        for (int j = 0; j < 8; j++) {
-                            const int at = min(m0 + j, cn - 1) * DP + lane;
-                            g[j] = gbuf[at];
-                            t[j] = vbuf[at];
-                            f[j] = qbuf[at];
-                        }
-#pragma unroll
-                        for (int j = 0; j < 8; j++) {
-                            if (m0 + j >= cn || !((mask >> (m0 + j)) & 1ull)) continue;
-                            a += g[j] - t[j] * w;
-                            const float z = a > 0 ? a - o.lambda1 : a + o.lambda1;
-                            w = fabsf(a) <= o.lambda1 ? 0.f : f[j] * z;
-                        }
+                    for (int j = 0; j < 8; j++) {
+                        const bool now_ = m0 + j < cn && ((mask >> (m0 + j)) & 1ull);
+                        const float z1 = a + (g[j] - t[j] * w), z = z1 > 0 ? z1 - o.lambda1 : z1 + o.lambda1;
+                        const float w1 = fabsf(z1) <= o.lambda1 ? 0.f : f[j] * z;
+                        a = now_ ? z1 : a;
+                        w = now_ ? w1 : w;
                     }
                 }
             }
@@ -1171,12 +1203,12 @@ __global__ __launch_bounds__(256) void k_small_apply(SmallShape b, SmallPlan p, 
     const int wave = (int)(threadIdx.x >> 6), lane = (int)(threadIdx.x & 63), sub = lane % LPG, lane0 = lane - sub;
     auto describe = [](uint2 g) { return make_uint4(g.x, g.y & 0xFFFFu, g.y >> 16, 0u); };
     auto group = [&](uint32_t bi) { return describe(p.group[first + b.cap - 1 - bi]); };
-    auto record = [&](const uint4& m, const float*& gp, int& sh, int& ck) {
+    auto record = [&](const uint4& m, const float*& gp, int& sh, int& ck, bool there) {
         gp = src.gradient(m);
         sh = (int)m.z;
         if (KIND == OPT_ADAGRAD) {
             ck = src.click(m);
-            src.click_at[m.x] = 0;
+            if (there) src.click_at[m.x] = 0;
         }
         return gp != nullptr;
     };
@@ -1197,7 +1229,7 @@ __global__ __launch_bounds__(256) void k_small_apply(SmallShape b, SmallPlan p, 
                 off = g.y;
                 k = g.z;
             },
-            [&](uint32_t at, const float*& gp, int& sh, int& ck) { return record(p.member[first + at], gp, sh, ck); }, [] {},
+            [&](uint32_t at, const float*& gp, int& sh, int& ck) { return record(p.member[first + at], gp, sh, ck, true); }, [] {},
             [] { wave_sync(); });
     }
     // signs with one record: several rounds of a wavefront on their way at a time where a round has few
