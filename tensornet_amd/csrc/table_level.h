@@ -198,8 +198,10 @@ inline size_t table_apply_lists_lds(uint32_t tiles) {
 // LPG lanes, several records in flight.  A sign's records in the next chunk find the row as this chunk left it (the
 // workgroup's own stores, behind a barrier), so any number of records of a sign is taken in order.  Bound by chains of
 // dependent reads (12 us to group a bucket's records, then the longest sign); the lists are short so that three
-// workgroups fit on a CU (a chunk of 1536 records left room for one: 59 us for 34 at 60 000 records).
-template <int KIND, int LPG, bool ANY>
+// workgroups fit on a CU (a chunk of 1536 records left room for one: 59 us for 34 at 60 000 records).  Rows of a power of two up to
+// 64 elements have the long signs taken by apply_big_wave (BIG > 0), the others by apply_big_groups (60 000 records of 40 times
+// 1500 signs, AdaGrad rows of 16: 28 us by the latter, 19.5 by the former).
+template <int KIND, int LPG, bool ANY, int BIG>
 __global__ __launch_bounds__(256) void k_table_apply(TableShape b, Store s, OptDev o, const tn_sign_info* __restrict__ infos,
                                                      const float* __restrict__ grads, int dim, const uint2* __restrict__ recs,
                                                      const uint16_t* __restrict__ boff, DevStatus* status, uint32_t* host_err,
@@ -309,7 +311,23 @@ __global__ __launch_bounds__(256) void k_table_apply(TableShape b, Store s, OptD
         // The wavefronts take the long signs first, then 64 / LPG short ones at a time: those that have no long sign
         // (10 us for 40 records) go on meanwhile.
         const int wave = (int)(tid >> 6), lane = (int)(tid & 63);
-        if (n_big) {
+        if constexpr (BIG > 0) {
+            __shared__ BigWave<KIND, BIG> tiles[TABLE_WAVES];
+            auto group = [&](uint32_t bi) {
+                const uint32_t e = big[bi];
+                return make_uint4(trow[e], toff[e], tcnt[e], 0u);
+            };
+            apply_big_wave<KIND, BIG>(
+                s, o, tiles[wave], (uint32_t)wave < n_big ? group((uint32_t)wave) : make_uint4(NO_ROW, 0, 0, 0), (uint32_t)wave,
+                (uint32_t)TABLE_WAVES, n_big, group, [&](uint32_t at) { return ridx[sorted[at]]; },
+                [&](uint32_t e, const float*& gp, int& sh, int& ck, bool) {
+                    gp = grads + (uint64_t)e * dim;
+                    sh = infos[e].batch_show;
+                    ck = infos[e].batch_click;
+                    return true;
+                },
+                [] {});
+        } else if (n_big) {
             char* base = reinterpret_cast<char*>(lds) + lists_lds + (size_t)wave * wave_lds;
             float* gbuf = reinterpret_cast<float*>(base);
             const float** gptr = reinterpret_cast<const float**>(base + wave_arrays);

@@ -49,6 +49,23 @@ def test_push_and_pull(tn, oracle, opt, dim, cvm, n, spread):
     pair.assert_rows_match(base)
 
 
+@pytest.mark.parametrize("opt", ["AdaGrad", "Adam", "Ftrl"])
+@pytest.mark.parametrize("dim", [1, 2, 4, 8, 16, 32, 64])
+@pytest.mark.parametrize("cvm", [False, True])
+def test_signs_with_many_records(tn, oracle, opt, dim, cvm):
+    """As many records as a wavefront takes up, as a chunk of it holds, one less and one more, and more than are grouped at
+    a time, among signs with one or two."""
+    rng = np.random.default_rng(dim)
+    pair = Pair(tn, oracle, opt, dim, HP[opt], use_cvm=cvm, reserve=2000)
+    base = pair.populate(synth.splitmix64(np.arange(1, 601, dtype=np.uint64)))
+    times = [15, 16, 17, 31, 32, 33, 63, 64, 65, 127, 128, 129, 511, 512, 513, 1100]
+    req = rng.permutation(np.concatenate([np.repeat(base[:len(times)], times), base[100:], base[100:200]]))
+    for _ in range(2):
+        infos, grads = pushed(tn, oracle, pair, req, rng)
+        assert pair.o.push(infos, grads) == 0
+    pair.assert_rows_match(base)
+
+
 @pytest.mark.parametrize("n", [1, 64, 65, 1000, 65536])
 def test_pull_of_new_signs(tn, oracle, n):
     """Most signs of the request are new and come up several times; every place gets the filled row."""
