@@ -846,303 +846,6 @@ __device__ __forceinline__ void apply_group_ahead(const Store& s, const OptDev& 
     }
 }
 
-// One sign with many records by a wavefront, rows of D elements, D a power of two up to 64.  A small batch's updates are as
-// long as their longest sign (its records: one per slot), so this is made for the length of the chain: what the chain itself
-// does not need is worked out for all records of a chunk side by side.  The lanes tile (record, element) as lane = record * D +
-// element, R records a round, and hold the gradients of a chunk's rounds in registers, all loads in flight; the next chunk's
-// are on their way while this one's records are applied, its member entries a chunk before that.  In LDS, a lane per
-// element walks the records in their order three times at most, with what depends on the record before only:
-//   AdaGrad  g2sum (a lane per record, double sum of squares first) | steps lr g / den by all lanes | subtractions
-//   Adam     m and v | steps lr m / (eps + sqrt(v)) by all lanes | subtractions
-//   Ftrl     n | sqrt(n), the quotient of the weight and the factor of z by all lanes | z and w
-// The same operations on the same operands as record after record.  What a chunk of 64 records takes at D = 16 under AdaGrad was
-// 9 us, 3.3 of them the g2sum chain (a branch per record), 1.4 each the divisions (one round after the other) and the
-// subtractions (LDS reads between them): the chain now runs on zeros where there is no gradient, the divisions of four rounds
-// and the reads of the next subtractions are under way together.  300 slots of 300 lookups, AdaGrad rows of 32 (signs with 300
-// records): k_small_apply 78 -> 41 us (60 before the latter); 40 slots of 8192, rows of 64: 66 -> 55; Ftrl rows of 1: 32 -> 23.
-template <int KIND, int D>
-struct BigWave {
-    static constexpr int R = 64 / D, DP = D + 1;  // records a round; padded row: lanes walking down a column hit different banks
-    static constexpr int BUFS = KIND == OPT_ADAGRAD ? 1 : KIND == OPT_ADAM ? 2 : 3;
-    static constexpr int fit(int chunk) {
-        return chunk > R && (chunk * DP * BUFS > 2304 || chunk > 16 * R) ? fit(chunk / 2) : chunk;
-    }
-    static constexpr int CHUNK = fit(64), ROUNDS = CHUNK / R;
-    static_assert(CHUNK >= R && CHUNK % R == 0, "whole rounds");
-    float buf[BUFS][CHUNK * DP];  // gradients, then steps (Ftrl: gradients) | Adam v, Ftrl n, then its factor | Ftrl quotient
-    const float* gptr[CHUNK];
-    float den[CHUNK];
-};
-
-// The sum of v over the wavefront, in every lane (all of them call it).
-__device__ __forceinline__ int wave_sum(int v) {
-    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, false);  // row_shr:1, 2, 4, 8: lane 15 of a row has the row's
-    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, false);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, false);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, false);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xA, 0xF, false);  // row_bcast:15 into rows 1 and 3
-    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xC, 0xF, false);  // row_bcast:31 into rows 2 and 3
-    return __builtin_amdgcn_readlane(v, 63);
-}
-
-// x0 + v of the lanes 0, 1, ... below n, added one after the other; at once where that is exact (whole numbers).
-__device__ __forceinline__ float ordered_sum(float x0, int v, int n) {
-    if (x0 == truncf(x0) && x0 >= 0.f && x0 < 8388608.f && !__any(v < 0 || v >= (1 << 16))) return x0 + (float)wave_sum(v);
-    const float f = (float)v;
-    for (int m = 0; m < n; m++) x0 += lane_value(f, m);
-    return x0;
-}
-
-// The signs bi0, bi0 + stride, ... below n_big; head: {row, first member, records} of the first, describe(bi): of another;
-// entry(at): member `at`; record(entry, gradient, show, click, there): whether it has a gradient (there: the lane's record is
-// one of the chunk's, and not a later chunk's or the last one again); missing(): one had none.
-template <int KIND, int D, typename Describe, typename Member, typename Record, typename Missing>
-__device__ __forceinline__ void apply_big_wave(const Store& s, const OptDev& o, BigWave<KIND, D>& lds, uint4 head, uint32_t bi0,
-                                               uint32_t stride, uint32_t n_big, Describe describe, Member entry, Record record,
-                                               Missing missing) {
-    using T = BigWave<KIND, D>;
-    constexpr int R = T::R, DP = T::DP, CHUNK = T::CHUNK, ROUNDS = T::ROUNDS;
-    float* const gbuf = lds.buf[0];
-    float* const vbuf = lds.buf[T::BUFS > 1 ? 1 : 0];
-    float* const qbuf = lds.buf[T::BUFS > 2 ? 2 : 0];
-    const int lane = (int)__lane_id(), li = lane & (D - 1), lm = lane / D;
-    const float c1 = 1 - o.beta1, c2 = 1 - o.beta2;
-    for (uint32_t bi = bi0; bi < n_big; bi += stride) {
-        if (bi != bi0) head = describe(bi);
-        const uint32_t row = head.x, off = head.y, k = head.z;
-        if (row > s.cap || k == 0) continue;  // NO_ROW, or no row number at all: never address the table with it
-        float* wp = s.w + (uint64_t)row * s.wstride;
-        float* sp = s.st + (uint64_t)row * s.sstride;
-        float w = lane < D ? wp[lane] : 0.f;
-        float a = 0.f, b = 0.f, show = 0.f, click = 0.f, g2sum = 0.f;
-        int delta_show = 0;
-        if (KIND == OPT_ADAGRAD) {
-            g2sum = sp[0];
-            show = sp[1];
-            click = sp[2];
-        } else {
-            a = lane < D ? sp[lane] : 0.f;
-            b = lane < D ? sp[D + lane] : 0.f;
-            delta_show = __float_as_int(sp[2 * D + 1]);
-        }
-        auto chunk_entry = [&](uint32_t c0) { return entry(off + min(c0 + (uint32_t)lane, k - 1)); };
-        auto now = chunk_entry(0);
-        auto next = chunk_entry(CHUNK);
-        float v[ROUNDS];
-        int sh = 0, ck = 0;
-        unsigned long long okmask = 0;
-        // Gradients of the chunk from c0 on, whose entries are e, on their way.  (Every load is issued, the row's in the place
-        // of a gradient there is not: under a condition each they are a branch each.)
-        auto fetch = [&](uint32_t c0, const auto& e) {
-            const float* gp = nullptr;
-            const bool there = lane < CHUNK && c0 + (uint32_t)lane < k;
-            const bool ok = record(e, gp, sh, ck, there) && there;
-            okmask = __ballot(ok);
-            if (lane < CHUNK) lds.gptr[lane] = ok ? gp : wp;
-            wave_sync();
-            const float* from[ROUNDS];
-#pragma unroll
-            for (int q = 0; q < ROUNDS; q++) from[q] = lds.gptr[lm + q * R];
-#pragma unroll
-            for (int q = 0; q < ROUNDS; q++) v[q] = as_global(from[q])[li];
-        };
-        fetch(0, now);
-        bool any = false;
-        for (uint32_t c0 = 0; c0 < k; c0 += CHUNK) {
-            const int cn = (int)min(k - c0, (uint32_t)CHUNK);
-            const unsigned long long mask = okmask, all = cn == 64 ? ~0ull : (1ull << cn) - 1ull;
-            const bool mine = (mask >> lane) & 1ull;
-            const int csh = mine ? sh : 0, cck = KIND == OPT_ADAGRAD && mine ? ck : 0;
-#pragma unroll
-            for (int q = 0; q < ROUNDS; q++) gbuf[(lm + q * R) * DP + li] = (mask >> (lm + q * R)) & 1ull ? v[q] : 0.f;
-            wave_sync();
-            if (c0 + CHUNK < k) {
-                now = next;
-                next = chunk_entry(c0 + 2 * CHUNK);
-                fetch(c0 + CHUNK, now);
-            }
-            if (KIND == OPT_ADAGRAD) {
-                // add_g2sum / dim of record `lane`: double sum of float products in element order (no gradient: zero)
-                double mq = 0.0;
-                if (lane < cn) {
-                    const float* gr = gbuf + lane * DP;
-                    constexpr int AT_ONCE = D < 16 ? D : 16;
-                    double tot = 0.0;
-#pragma unroll
-                    for (int i0 = 0; i0 < D; i0 += AT_ONCE) {
-                        float x[AT_ONCE];
-#pragma unroll
-                        for (int i = 0; i < AT_ONCE; i++) x[i] = gr[i0 + i];
-#pragma unroll
-                        for (int i = 0; i < AT_ONCE; i++) tot += (double)(x[i] * x[i]);
-                    }
-                    mq = tot * (1.0 / (double)D);  // (exact: D is a power of two)
-                }
-                show = ordered_sum(show, csh, cn);
-                click = ordered_sum(click, cck, cn);
-                // g2sum after every record (float += double, rounded each time): every lane runs the chain on values read
-                // out of the records' lanes, lane m keeps the g2sum its record meets.  (Behind the last record and for one
-                // without a gradient zeros are added, which changes nothing.)
-                float myg2 = 0.f;
-                for (int m0 = 0; m0 < cn; m0 += 8) {
-                    double x[8];
-#pragma unroll
-                    for (int j = 0; j < 8; j++) x[j] = lane_value(mq, m0 + j);
-#pragma unroll
-                    for (int j = 0; j < 8; j++) {
-                        g2sum = (float)((double)g2sum + x[j]);
-                        myg2 = lane == m0 + j ? g2sum : myg2;
-                    }
-                }
-                if (lane < CHUNK) lds.den[lane] = o.eps + sqrtf(myg2);
-                wave_sync();
-                constexpr int SIDE = ROUNDS < 4 ? ROUNDS : 4;  // rounds side by side
-                for (int q0 = 0; q0 * R < cn; q0 += SIDE) {
-                    float gv[SIDE], dn[SIDE];
-#pragma unroll
-                    for (int q = 0; q < SIDE; q++) {
-                        gv[q] = gbuf[(lm + (q0 + q) * R) * DP + li];
-                        dn[q] = lds.den[lm + (q0 + q) * R];
-                    }
-#pragma unroll
-                    for (int q = 0; q < SIDE; q++) gv[q] = o.lr * gv[q] / dn[q];
-                    // (a record without a gradient row has zeros, and a step of zero or, on a fresh row, no number: set to zero)
-#pragma unroll
-                    for (int q = 0; q < SIDE; q++) {
-                        const int m = lm + (q0 + q) * R;
-                        gbuf[m * DP + li] = (mask >> m) & 1ull ? gv[q] : 0.f;
-                    }
-                }
-            } else {
-                delta_show += wave_sum(csh);
-                const float n0 = b;
-                if (lane < D) {
-                    for (int m0 = 0; m0 < cn; m0 += 8) {
-                        float g[8];
-#pragma unroll
-                        for (int j = 0; j < 8; j++) g[j] = gbuf[min(m0 + j, cn - 1) * DP + lane];
-#pragma unroll
-                        for (int j = 0; j < 8; j++) {
-                            if (m0 + j >= cn) break;
-                            if ((mask >> (m0 + j)) & 1ull) {
-                                if (KIND == OPT_ADAM) {
-                                    a = o.beta1 * a + c1 * g[j];
-                                    b = o.beta2 * b + c2 * g[j] * g[j];
-                                } else {
-                                    b += g[j] * g[j];
-                                }
-                            }
-                            if (KIND == OPT_ADAM) gbuf[(m0 + j) * DP + lane] = a;
-                            vbuf[(m0 + j) * DP + lane] = b;
-                        }
-                    }
-                }
-                wave_sync();
-                if (KIND == OPT_ADAM) {
-                    constexpr int SIDE = ROUNDS < 4 ? ROUNDS : 4;
-                    for (int q0 = 0; q0 * R < cn; q0 += SIDE) {
-                        float am[SIDE], bm[SIDE];
-#pragma unroll
-                        for (int q = 0; q < SIDE; q++) {
-                            am[q] = gbuf[(lm + (q0 + q) * R) * DP + li];
-                            bm[q] = vbuf[(lm + (q0 + q) * R) * DP + li];
-                        }
-#pragma unroll
-                        for (int q = 0; q < SIDE; q++) am[q] = o.lr * am[q] / (o.eps + sqrtf(bm[q]));
-#pragma unroll
-                        for (int q = 0; q < SIDE; q++) {
-                            const int m = lm + (q0 + q) * R;
-                            gbuf[m * DP + li] = (mask >> m) & 1ull ? am[q] : 0.f;
-                        }
-                    }
-                } else {
-                    const float first = __shfl(n0, li);
-                    float t[ROUNDS];
-#pragma unroll
-                    for (int q = 0; q < ROUNDS; q++) {
-                        const int m = lm + q * R;
-                        t[q] = 0.f;
-                        if (m >= cn) continue;
-                        const float nm = vbuf[m * DP + li], before = m > 0 ? vbuf[(m - 1) * DP + li] : first, root = sqrtf(nm);
-                        t[q] = o.lr * (root - sqrtf(before));
-                        qbuf[m * DP + li] = -1 / ((o.beta + root) * o.lr + o.lambda2);
-                    }
-                    wave_sync();
-#pragma unroll
-                    for (int q = 0; q < ROUNDS; q++) {
-                        const int m = lm + q * R;
-                        if (m < cn) vbuf[m * DP + li] = t[q];
-                    }
-                }
-            }
-            wave_sync();
-            if (KIND != OPT_FTRL) {
-                // (what lies behind the last record steps by nothing)
-                constexpr int AHEAD = CHUNK < 16 ? CHUNK : 16;
-                if (lane < D) {
-                    float t[AHEAD], u[AHEAD];
-#pragma unroll
-                    for (int j = 0; j < AHEAD; j++) t[j] = gbuf[j * DP + lane];
-                    for (int m0 = 0; m0 < cn; m0 += AHEAD) {
-#pragma unroll
-                        for (int j = 0; j < AHEAD; j++) u[j] = gbuf[min(m0 + AHEAD + j, CHUNK - 1) * DP + lane];
-#pragma unroll
-                        for (int j = 0; j < AHEAD; j++) w -= m0 + j < cn ? t[j] : 0.f;
-#pragma unroll
-                        for (int j = 0; j < AHEAD; j++) t[j] = u[j];
-                    }
-                }
-            } else if (lane < D) {
-                for (int m0 = 0; m0 < cn; m0 += 8) {
-                    float g[8], t[8], f[8];
-#pragma unroll
-                    for (int j = 0; j < 8; j++) {
-                        const int at = min(m0 + j, cn - 1) * DP + lane;
-                        g[j] = gbuf[at];
-                        t[j] = vbuf[at];
-                        f[j] = qbuf[at];
-                    }
-#pragma unroll
-                    for (int j = 0; j < 8; j++) {
-                        const bool now_ = m0 + j < cn && ((mask >> (m0 + j)) & 1ull);
-                        const float z1 = a + (g[j] - t[j] * w), z = z1 > 0 ? z1 - o.lambda1 : z1 + o.lambda1;
-                        const float w1 = fabsf(z1) <= o.lambda1 ? 0.f : f[j] * z;
-                        a = now_ ? z1 : a;
-                        w = now_ ? w1 : w;
-                    }
-                }
-            }
-            if (mask) any = true;
-            if (lane == 0 && mask != all) missing();
-            wave_sync();
-        }
-        if (any) {
-            if (lane < D) {
-                wp[lane] = w;
-                if (KIND != OPT_ADAGRAD) {
-                    sp[lane] = a;
-                    sp[D + lane] = b;
-                }
-            }
-            if (lane == 0) {
-                if (KIND == OPT_ADAGRAD) {
-                    sp[0] = g2sum;
-                    sp[1] = show;
-                    sp[2] = click;
-                    sp[3] = 0.f;  // no_show_days = 0
-                    if (o.use_cvm) {
-                        wp[D] = show;
-                        wp[D + 1] = logf(click + 1) - logf(show + 1);
-                    }
-                } else {
-                    sp[2 * D + 1] = __int_as_float(delta_show);
-                }
-            }
-        }
-        wave_sync();
-    }
-}
-
 // Bytes of dynamic LDS of k_small_apply when its launch includes the workgroups for the signs with many records:
 // per wavefront the staging and the row of apply_big_groups, then its pointer, count, flag and divisor arrays.
 inline size_t small_apply_wave_lds(int D) { return align_up(big_lds_bytes(D), 8) + BIG_CHUNK * (8 + 4); }

@@ -2026,165 +2026,345 @@ __global__ __launch_bounds__(64) void k_apply_big(Store s, OptDev o, PushSrc src
         [&] { atomicOr(&status->err, DEV_ERR_GRAD_ROWS); }, [] { __syncthreads(); });
 }
 
-// k_apply_big for AdaGrad rows of D elements, D a power of two from 4 to 64, on a plan whose big_desc lists
-// {row, first member, records, group} of every sign with many records (written by k_group_emit): one wavefront
-// per sign, its records up to BigTile<D>::CHUNK at a time.  The lanes tile (record, element) as
-// lane = record * D + element, 64 / D records a round, and keep the gradients of their rounds in registers, so
-// every gradient load of a chunk is in flight at once; the sign's description is asked for together with the
-// status, the row together with the first records.  The staging in LDS only turns the tile round -- a lane per
-// record for the sum of squares (double, in element order), a lane per element for the subtractions (in record
-// order) -- and every loop over it fetches several entries before it uses the first, so that no step of a chain
-// waits for LDS.  Operation for operation the arithmetic of apply_big_groups.
-template <int D>
-struct BigTile {
-    static constexpr int R = 64 / D;                                            // records a round
-    static constexpr int MOST = D == 32 ? 8 : 16;                               // (what the register file takes without spilling)
-    static constexpr int ROUNDS = BIG_CHUNK / R < MOST ? BIG_CHUNK / R : MOST;  // gradient registers of a lane
-    static constexpr int CHUNK = R * ROUNDS;
-    static constexpr int DP = D + 1;  // padded staging row: lanes walking down a column hit different banks
+// One sign with many records by a wavefront, rows of D elements, D a power of two up to 64.  A small batch's updates are as
+// long as their longest sign (its records: one per slot), so this is made for the length of the chain: what the chain itself
+// does not need is worked out for all records of a chunk side by side.  The lanes tile (record, element) as lane = record * D +
+// element, R records a round, and hold the gradients of a chunk's rounds in registers, all loads in flight; the next chunk's
+// are on their way while this one's records are applied, its member entries a chunk before that.  In LDS, a lane per
+// element walks the records in their order three times at most, with what depends on the record before only:
+//   AdaGrad  g2sum (a lane per record, double sum of squares first) | steps lr g / den by all lanes | subtractions
+//   Adam     m and v | steps lr m / (eps + sqrt(v)) by all lanes | subtractions
+//   Ftrl     n | sqrt(n), the quotient of the weight and the factor of z by all lanes | z and w
+// The same operations on the same operands as record after record.  What a chunk of 64 records takes at D = 16 under AdaGrad was
+// 9 us, 3.3 of them the g2sum chain (a branch per record), 1.4 each the divisions (one round after the other) and the
+// subtractions (LDS reads between them): the chain now runs on zeros where there is no gradient, the divisions of four rounds
+// and the reads of the next subtractions are under way together.  300 slots of 300 lookups, AdaGrad rows of 32 (signs with 300
+// records): k_small_apply 78 -> 41 us (60 before the latter); 40 slots of 8192, rows of 64: 66 -> 55; Ftrl rows of 1: 32 -> 23.
+template <int KIND, int D, int MOST = 16>
+struct BigWave {
+    static constexpr int R = 64 / D, DP = D + 1;  // records a round; padded row: lanes walking down a column hit different banks
+    static constexpr int BUFS = KIND == OPT_ADAGRAD ? 1 : KIND == OPT_ADAM ? 2 : 3;
+    static constexpr int fit(int chunk) {
+        return chunk > R && (chunk * DP * BUFS > 2304 || chunk > MOST * R) ? fit(chunk / 2) : chunk;
+    }
+    static constexpr int CHUNK = fit(64), ROUNDS = CHUNK / R;
+    static_assert(CHUNK >= R && CHUNK % R == 0, "whole rounds");
+    float buf[BUFS][CHUNK * DP];  // gradients, then steps (Ftrl: gradients) | Adam v, Ftrl n, then its factor | Ftrl quotient
+    const float* gptr[CHUNK];
+    float den[CHUNK];
 };
-// (the signs first, first + stride, ... below n_big by the wavefront that calls it, whose own the LDS is; head: the first one's
-// description, describe(bi): another's; record, missing, sync: as apply_big_groups')
-template <int D>
-struct BigTileLds {
-    float gbuf[BigTile<D>::CHUNK * BigTile<D>::DP];
-    const float* gptr[BigTile<D>::CHUNK];
-    float den[BigTile<D>::CHUNK];
-};
-template <int D, typename Describe, typename Record, typename Missing, typename Sync>
-__device__ __forceinline__ void apply_big_tiles(const Store& s, const OptDev& o, BigTileLds<D>& lds, uint4 head, uint32_t first,
-                                                uint32_t stride, uint32_t n_big, Describe describe, Record record,
-                                                Missing missing, Sync sync) {
-    using T = BigTile<D>;
-    constexpr int R = T::R, DP = T::DP;
-    float* const gbuf = lds.gbuf;
-    const float** const gptr = lds.gptr;
-    float* const den = lds.den;
-    const int lane = (int)__lane_id();
-    const int li = lane & (D - 1), lm = lane / D;
-    constexpr double inv_d = 1.0 / (double)D;  // exact: D is a power of two
-    for (uint32_t bi = first; bi < n_big; bi += stride) {
-        if (bi != first) head = describe(bi);
+
+// The sum of v over the wavefront, in every lane (all of them call it).
+__device__ __forceinline__ int wave_sum(int v) {
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, false);  // row_shr:1, 2, 4, 8: lane 15 of a row has the row's
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xA, 0xF, false);  // row_bcast:15 into rows 1 and 3
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xC, 0xF, false);  // row_bcast:31 into rows 2 and 3
+    return __builtin_amdgcn_readlane(v, 63);
+}
+
+// x0 + v of the lanes 0, 1, ... below n, added one after the other; at once where that is exact (whole numbers).
+__device__ __forceinline__ float ordered_sum(float x0, int v, int n) {
+    if (x0 == truncf(x0) && x0 >= 0.f && x0 < 8388608.f && !__any(v < 0 || v >= (1 << 16))) return x0 + (float)wave_sum(v);
+    const float f = (float)v;
+    for (int m = 0; m < n; m++) x0 += lane_value(f, m);
+    return x0;
+}
+
+// The signs bi0, bi0 + stride, ... below n_big; head: {row, first member, records} of the first, describe(bi): of another;
+// entry(at): member `at`; record(entry, gradient, show, click, there): whether it has a gradient (there: the lane's record is
+// one of the chunk's, and not a later chunk's or the last one again); missing(): one had none.
+template <int KIND, int D, int MOST, typename Describe, typename Entry, typename Record, typename Missing>
+__device__ __forceinline__ void apply_big_wave(const Store& s, const OptDev& o, BigWave<KIND, D, MOST>& lds, uint4 head, uint32_t bi0,
+                                               uint32_t stride, uint32_t n_big, Describe describe, Entry entry, Record record,
+                                               Missing missing) {
+    using T = BigWave<KIND, D, MOST>;
+    constexpr int R = T::R, DP = T::DP, CHUNK = T::CHUNK, ROUNDS = T::ROUNDS;
+    float* const gbuf = lds.buf[0];
+    float* const vbuf = lds.buf[T::BUFS > 1 ? 1 : 0];
+    float* const qbuf = lds.buf[T::BUFS > 2 ? 2 : 0];
+    const int lane = (int)__lane_id(), li = lane & (D - 1), lm = lane / D;
+    const float c1 = 1 - o.beta1, c2 = 1 - o.beta2;
+    for (uint32_t bi = bi0; bi < n_big; bi += stride) {
+        if (bi != bi0) head = describe(bi);
         const uint32_t row = head.x, off = head.y, k = head.z;
-        if (row > s.cap) continue;  // NO_ROW, or no row number at all: never address the table with it
+        if (row > s.cap || k == 0) continue;  // NO_ROW, or no row number at all: never address the table with it
         float* wp = s.w + (uint64_t)row * s.wstride;
         float* sp = s.st + (uint64_t)row * s.sstride;
         float w = lane < D ? wp[lane] : 0.f;
-        float g2sum = sp[0], show = sp[1], click = sp[2];
+        float a = 0.f, b = 0.f, show = 0.f, click = 0.f, g2sum = 0.f;
+        int delta_show = 0;
+        if (KIND == OPT_ADAGRAD) {
+            g2sum = sp[0];
+            show = sp[1];
+            click = sp[2];
+        } else {
+            a = lane < D ? sp[lane] : 0.f;
+            b = lane < D ? sp[D + lane] : 0.f;
+            delta_show = __float_as_int(sp[2 * D + 1]);
+        }
+        auto chunk_entry = [&](uint32_t c0) { return entry(off + min(c0 + (uint32_t)lane, k - 1)); };
+        auto now = chunk_entry(0);
+        auto next = chunk_entry(CHUNK);
+        float v[ROUNDS];
+        int sh = 0, ck = 0;
+        unsigned long long okmask = 0;
+        // Gradients of the chunk from c0 on, whose entries are e, on their way.  (Every load is issued, the row's in the place
+        // of a gradient there is not: under a condition each they are a branch each.)
+        auto fetch = [&](uint32_t c0, const auto& e) {
+            const float* gp = nullptr;
+            const bool there = lane < CHUNK && c0 + (uint32_t)lane < k;
+            const bool ok = record(e, gp, sh, ck, there) && there;
+            okmask = __ballot(ok);
+            if (lane < CHUNK) lds.gptr[lane] = ok ? gp : wp;
+            wave_sync();
+            const float* from[ROUNDS];
+#pragma unroll
+            for (int q = 0; q < ROUNDS; q++) from[q] = lds.gptr[lm + q * R];
+#pragma unroll
+            for (int q = 0; q < ROUNDS; q++) v[q] = as_global(from[q])[li];
+        };
+        fetch(0, now);
         bool any = false;
-        for (uint32_t c0 = 0; c0 < k; c0 += T::CHUNK) {
-            const int cn = (int)((k - c0) < (uint32_t)T::CHUNK ? (k - c0) : (uint32_t)T::CHUNK);
-            bool ok = false;
-            int sh = 0, ck = 0;
-            if (lane < cn) {
-                const float* gp = nullptr;
-                ok = record(off + c0 + (uint32_t)lane, gp, sh, ck);
-                gptr[lane] = gp;
-            }
-            const unsigned long long okmask = __ballot(ok);
-            const unsigned long long chunk_mask = cn == 64 ? ~0ull : (1ull << cn) - 1ull;
-            sync();
-            {
-                float v[T::ROUNDS];
+        for (uint32_t c0 = 0; c0 < k; c0 += CHUNK) {
+            const int cn = (int)min(k - c0, (uint32_t)CHUNK);
+            const unsigned long long mask = okmask, all = cn == 64 ? ~0ull : (1ull << cn) - 1ull;
+            const bool mine = (mask >> lane) & 1ull;
+            const int csh = mine ? sh : 0, cck = KIND == OPT_ADAGRAD && mine ? ck : 0;
 #pragma unroll
-                for (int q = 0; q < T::ROUNDS; q++) {
-                    const int m = lm + q * R;
-                    v[q] = (m < cn && ((okmask >> m) & 1ull)) ? as_global(gptr[m])[li] : 0.f;
+            for (int q = 0; q < ROUNDS; q++) gbuf[(lm + q * R) * DP + li] = (mask >> (lm + q * R)) & 1ull ? v[q] : 0.f;
+            wave_sync();
+            if (c0 + CHUNK < k) {
+                now = next;
+                next = chunk_entry(c0 + 2 * CHUNK);
+                fetch(c0 + CHUNK, now);
+            }
+            if (KIND == OPT_ADAGRAD) {
+                // add_g2sum / dim of record `lane`: double sum of float products in element order (no gradient: zero)
+                double mq = 0.0;
+                if (lane < cn) {
+                    const float* gr = gbuf + lane * DP;
+                    constexpr int AT_ONCE = D < 16 ? D : 16;
+                    double tot = 0.0;
+#pragma unroll
+                    for (int i0 = 0; i0 < D; i0 += AT_ONCE) {
+                        float x[AT_ONCE];
+#pragma unroll
+                        for (int i = 0; i < AT_ONCE; i++) x[i] = gr[i0 + i];
+#pragma unroll
+                        for (int i = 0; i < AT_ONCE; i++) tot += (double)(x[i] * x[i]);
+                    }
+                    mq = tot * (1.0 / (double)D);  // (exact: D is a power of two)
                 }
+                show = ordered_sum(show, csh, cn);
+                click = ordered_sum(click, cck, cn);
+                // g2sum after every record (float += double, rounded each time): every lane runs the chain on values read
+                // out of the records' lanes, lane m keeps the g2sum its record meets.  (Behind the last record and for one
+                // without a gradient zeros are added, which changes nothing.)
+                float myg2 = 0.f;
+                for (int m0 = 0; m0 < cn; m0 += 8) {
+                    double x[8];
 #pragma unroll
-                for (int q = 0; q < T::ROUNDS; q++) gbuf[(lm + q * R) * DP + li] = v[q];
-            }
-            sync();
-            // add_g2sum / dim of record `lane`: double sum of float products in element order
-            double mq = 0.0;
-            if (lane < cn) {
-                const float* gr = gbuf + lane * DP;
-                constexpr int AT_ONCE = D < 16 ? D : 16;
-                double tot = 0.0;
+                    for (int j = 0; j < 8; j++) x[j] = lane_value(mq, m0 + j);
 #pragma unroll
-                for (int i0 = 0; i0 < D; i0 += AT_ONCE) {
-                    float a[AT_ONCE];
-#pragma unroll
-                    for (int i = 0; i < AT_ONCE; i++) a[i] = gr[i0 + i];
-#pragma unroll
-                    for (int i = 0; i < AT_ONCE; i++) tot += (double)(a[i] * a[i]);
+                    for (int j = 0; j < 8; j++) {
+                        g2sum = (float)((double)g2sum + x[j]);
+                        myg2 = lane == m0 + j ? g2sum : myg2;
+                    }
                 }
-                mq = tot * inv_d;
-            }
-            // g2sum after every record (float += double, rounded each time), show and click in record order:
-            // every lane runs the same chain on values read out of the records' lanes, lane m keeps the g2sum
-            // its record meets
-            const float fsh = (float)sh, fck = (float)ck;
-            float myg2 = 0.f;
-            if (okmask == chunk_mask) {
-                for (int m = 0; m < cn; m++) {
-                    show += lane_value(fsh, m);
-                    click += lane_value(fck, m);
-                    g2sum = (float)((double)g2sum + lane_value(mq, m));
-                    if (lane == m) myg2 = g2sum;
+                if (lane < CHUNK) lds.den[lane] = o.eps + sqrtf(myg2);
+                wave_sync();
+                constexpr int SIDE = ROUNDS < 4 ? ROUNDS : 4;  // rounds side by side
+                for (int q0 = 0; q0 * R < cn; q0 += SIDE) {
+                    float gv[SIDE], dn[SIDE];
+#pragma unroll
+                    for (int q = 0; q < SIDE; q++) {
+                        gv[q] = gbuf[(lm + (q0 + q) * R) * DP + li];
+                        dn[q] = lds.den[lm + (q0 + q) * R];
+                    }
+#pragma unroll
+                    for (int q = 0; q < SIDE; q++) gv[q] = o.lr * gv[q] / dn[q];
+                    // (a record without a gradient row has zeros, and a step of zero or, on a fresh row, no number: set to zero)
+#pragma unroll
+                    for (int q = 0; q < SIDE; q++) {
+                        const int m = lm + (q0 + q) * R;
+                        gbuf[m * DP + li] = (mask >> m) & 1ull ? gv[q] : 0.f;
+                    }
                 }
             } else {
-                for (int m = 0; m < cn; m++) {
-                    if (!((okmask >> m) & 1ull)) continue;
-                    show += lane_value(fsh, m);
-                    click += lane_value(fck, m);
-                    g2sum = (float)((double)g2sum + lane_value(mq, m));
-                    if (lane == m) myg2 = g2sum;
+                delta_show += wave_sum(csh);
+                const float n0 = b;
+                if (lane < D) {
+                    for (int m0 = 0; m0 < cn; m0 += 8) {
+                        float g[8];
+#pragma unroll
+                        for (int j = 0; j < 8; j++) g[j] = gbuf[min(m0 + j, cn - 1) * DP + lane];
+#pragma unroll
+                        for (int j = 0; j < 8; j++) {
+                            if (m0 + j >= cn) break;
+                            if ((mask >> (m0 + j)) & 1ull) {
+                                if (KIND == OPT_ADAM) {
+                                    a = o.beta1 * a + c1 * g[j];
+                                    b = o.beta2 * b + c2 * g[j] * g[j];
+                                } else {
+                                    b += g[j] * g[j];
+                                }
+                            }
+                            if (KIND == OPT_ADAM) gbuf[(m0 + j) * DP + lane] = a;
+                            vbuf[(m0 + j) * DP + lane] = b;
+                        }
+                    }
+                }
+                wave_sync();
+                if (KIND == OPT_ADAM) {
+                    constexpr int SIDE = ROUNDS < 4 ? ROUNDS : 4;
+                    for (int q0 = 0; q0 * R < cn; q0 += SIDE) {
+                        float am[SIDE], bm[SIDE];
+#pragma unroll
+                        for (int q = 0; q < SIDE; q++) {
+                            am[q] = gbuf[(lm + (q0 + q) * R) * DP + li];
+                            bm[q] = vbuf[(lm + (q0 + q) * R) * DP + li];
+                        }
+#pragma unroll
+                        for (int q = 0; q < SIDE; q++) am[q] = o.lr * am[q] / (o.eps + sqrtf(bm[q]));
+#pragma unroll
+                        for (int q = 0; q < SIDE; q++) {
+                            const int m = lm + (q0 + q) * R;
+                            gbuf[m * DP + li] = (mask >> m) & 1ull ? am[q] : 0.f;
+                        }
+                    }
+                } else {
+                    const float first = __shfl(n0, li);
+                    float t[ROUNDS];
+#pragma unroll
+                    for (int q = 0; q < ROUNDS; q++) {
+                        const int m = lm + q * R;
+                        t[q] = 0.f;
+                        if (m >= cn) continue;
+                        const float nm = vbuf[m * DP + li], before = m > 0 ? vbuf[(m - 1) * DP + li] : first, root = sqrtf(nm);
+                        t[q] = o.lr * (root - sqrtf(before));
+                        qbuf[m * DP + li] = -1 / ((o.beta + root) * o.lr + o.lambda2);
+                    }
+                    wave_sync();
+#pragma unroll
+                    for (int q = 0; q < ROUNDS; q++) {
+                        const int m = lm + q * R;
+                        if (m < cn) vbuf[m * DP + li] = t[q];
+                    }
                 }
             }
-            if (lane < cn) den[lane] = o.eps + sqrtf(myg2);
-            sync();
-            // the steps lr * g / den of all records and elements (independent divisions, the operands of a few
-            // rounds fetched together); a record without a gradient row steps by zero, which leaves the weights
-            // as they are
-#pragma unroll 4
-            for (int m = lm; m < cn; m += R) {
-                const float gv = gbuf[m * DP + li], dn = den[m];
-                gbuf[m * DP + li] = ((okmask >> m) & 1ull) ? o.lr * gv / dn : 0.f;
-            }
-            sync();
-            // per element the subtractions in record order
-            if (lane < D) {
+            wave_sync();
+            if (KIND != OPT_FTRL) {
+                // (what lies behind the last record steps by nothing)
+                constexpr int AHEAD = CHUNK < 16 ? CHUNK : 16;
+                if (lane < D) {
+                    float t[AHEAD], u[AHEAD];
+#pragma unroll
+                    for (int j = 0; j < AHEAD; j++) t[j] = gbuf[j * DP + lane];
+                    for (int m0 = 0; m0 < cn; m0 += AHEAD) {
+#pragma unroll
+                        for (int j = 0; j < AHEAD; j++) u[j] = gbuf[min(m0 + AHEAD + j, CHUNK - 1) * DP + lane];
+#pragma unroll
+                        for (int j = 0; j < AHEAD; j++) w -= m0 + j < cn ? t[j] : 0.f;
+#pragma unroll
+                        for (int j = 0; j < AHEAD; j++) t[j] = u[j];
+                    }
+                }
+            } else if (lane < D) {
                 for (int m0 = 0; m0 < cn; m0 += 8) {
-                    float t[8];
+                    float g[8], t[8], f[8];
 #pragma unroll
-                    for (int j = 0; j < 8; j++) t[j] = m0 + j < cn ? gbuf[(m0 + j) * DP + lane] : 0.f;
+                    for (int j = 0; j < 8; j++) {
+                        const int at = min(m0 + j, cn - 1) * DP + lane;
+                        g[j] = gbuf[at];
+                        t[j] = vbuf[at];
+                        f[j] = qbuf[at];
+                    }
 #pragma unroll
-                    for (int j = 0; j < 8; j++) w -= t[j];
+                    for (int j = 0; j < 8; j++) {
+                        const bool now_ = m0 + j < cn && ((mask >> (m0 + j)) & 1ull);
+                        const float z1 = a + (g[j] - t[j] * w), z = z1 > 0 ? z1 - o.lambda1 : z1 + o.lambda1;
+                        const float w1 = fabsf(z1) <= o.lambda1 ? 0.f : f[j] * z;
+                        a = now_ ? z1 : a;
+                        w = now_ ? w1 : w;
+                    }
                 }
             }
-            if (okmask) any = true;
-            if (lane == 0 && okmask != chunk_mask) missing();
-            sync();
+            if (mask) any = true;
+            if (lane == 0 && mask != all) missing();
+            wave_sync();
         }
         if (any) {
-            if (lane < D) wp[lane] = w;
+            if (lane < D) {
+                wp[lane] = w;
+                if (KIND != OPT_ADAGRAD) {
+                    sp[lane] = a;
+                    sp[D + lane] = b;
+                }
+            }
             if (lane == 0) {
-                sp[0] = g2sum;
-                sp[1] = show;
-                sp[2] = click;
-                sp[3] = 0.f;  // no_show_days = 0
-                if (o.use_cvm) {
-                    wp[D] = show;
-                    wp[D + 1] = logf(click + 1) - logf(show + 1);
+                if (KIND == OPT_ADAGRAD) {
+                    sp[0] = g2sum;
+                    sp[1] = show;
+                    sp[2] = click;
+                    sp[3] = 0.f;  // no_show_days = 0
+                    if (o.use_cvm) {
+                        wp[D] = show;
+                        wp[D + 1] = logf(click + 1) - logf(show + 1);
+                    }
+                } else {
+                    sp[2 * D + 1] = __int_as_float(delta_show);
                 }
             }
         }
+        wave_sync();
     }
 }
 
+// A record of a sign with many records by its place in the member lists: its entry, and where its gradient row is if that was
+// worked out beforehand (k_member_grads).
+struct BigSrc {
+    PushSrc src;
+    const Member* list;
+    const float* const* ga;
+    struct Entry {
+        Member m;
+        const float* g;
+    };
+    __device__ __forceinline__ Entry entry(uint32_t at) const { return {list[at], ga ? ga[at] : nullptr}; }
+    __device__ __forceinline__ bool record(const Entry& e, const float*& g, int& show, int& click) const {
+        if (!ga) return src_record(src, e.m, g, show, click);
+        g = e.g;
+        show = e.m.show;
+        click = e.m.click;
+        return g != nullptr;
+    }
+};
+
+// apply_big_wave's rounds in the general path's kernels: a chunk of half the records, which takes 123 registers at D = 16 where 16
+// rounds take 150 and more.  In k_apply_all (beside the other signs' workgroups, so four wavefronts a SIMD are wanted) 2.1 M lookups
+// of 64 slots: 212 us a step with 8 rounds, 217 with 16; 430 k pooled of 211, signs of 211 records: 361 against 364.
+constexpr int BIG_MOST = 8;
+
+// k_apply_big for AdaGrad rows of D elements, D a power of two from 4 to 64, on a plan whose big_desc lists {row, first member,
+// records, group} of every sign with many records (written by k_group_emit): one wavefront per sign, by apply_big_wave.  (Adam and
+// Ftrl the same way: 800 k lookups, Adam rows of 16, 136 us a step with and without; not worth their kernels.)
 template <int D>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6, 8))) void k_apply_big_adagrad(
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_apply_big_adagrad(
     Store s, OptDev o, PushSrc src, DevStatus* status, const uint4* __restrict__ big_desc, uint32_t desc_cap,
     const Member* __restrict__ list, const float* const* __restrict__ gaddr) {
-    __shared__ BigTileLds<D> lds;
+    __shared__ BigWave<OPT_ADAGRAD, D, BIG_MOST> lds;
     const uint4 head = big_desc[blockIdx.x < desc_cap ? blockIdx.x : desc_cap - 1];  // (before the status is known)
     // a push launched on a plan that turned out not to be its batch's (the host redoes it), or whose inputs are unusable
     if (status->mismatch | status->abort) return;
-    apply_big_tiles<D>(
+    const BigSrc from{src, list, gaddr};
+    apply_big_wave<OPT_ADAGRAD, D>(
         s, o, lds, head, blockIdx.x, gridDim.x, status->n_big, [&](uint32_t bi) { return big_desc[bi]; },
-        [&](uint32_t at, const float*& gp, int& sh, int& ck) { return record_at(src, list, gaddr, at, gp, sh, ck); },
-        [&] { atomicOr(&status->err, DEV_ERR_GRAD_ROWS); }, [] { __syncthreads(); });
+        [&](uint32_t at) { return from.entry(at); },
+        [&](const BigSrc::Entry& e, const float*& gp, int& sh, int& ck, bool) { return from.record(e, gp, sh, ck); },
+        [&] { atomicOr(&status->err, DEV_ERR_GRAD_ROWS); });
 }
 
 // The updates of a push of up to ONE_STREAM_LOOKUPS lookups by one launch: the workgroups of the three kernels above side
@@ -2207,19 +2387,21 @@ struct ApplyAll {
 constexpr int ALL_GBUF = 1088;  // floats of gradient staging per wavefront at most: eight workgroups to a CU up to 64 elements
 
 template <int KIND, int LPG, bool ANY, int TILE>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6, 8))) void k_apply_all(Store s, OptDev o, PushSrc src,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_apply_all(Store s, OptDev o, PushSrc src,
                                                                                               DevStatus* status, ApplyAll a) {
     // a push launched on a plan that turned out not to be its batch's (the host redoes it), or whose inputs are unusable
     if (status->mismatch | status->abort) return;
     if (blockIdx.x < a.big_blocks) {
         const uint32_t wave = threadIdx.x >> 6, first = blockIdx.x * 4 + wave, stride = a.big_blocks * 4;
         if constexpr (TILE != 0) {
-            __shared__ BigTileLds<TILE> lds[4];
+            __shared__ BigWave<KIND, TILE, BIG_MOST> lds[4];
+            const BigSrc from{src, a.list, a.gaddr};
             const uint4 head = a.big_desc[first < a.big_cap ? first : a.big_cap - 1];
-            apply_big_tiles<TILE>(
+            apply_big_wave<KIND, TILE>(
                 s, o, lds[wave], head, first, stride, status->n_big, [&](uint32_t bi) { return a.big_desc[bi]; },
-                [&](uint32_t at, const float*& gp, int& sh, int& ck) { return record_at(src, a.list, a.gaddr, at, gp, sh, ck); },
-                [&] { atomicOr(&status->err, DEV_ERR_GRAD_ROWS); }, [] { wave_sync(); });
+                [&](uint32_t at) { return from.entry(at); },
+                [&](const BigSrc::Entry& e, const float*& gp, int& sh, int& ck, bool) { return from.record(e, gp, sh, ck); },
+                [&] { atomicOr(&status->err, DEV_ERR_GRAD_ROWS); });
         } else {
             extern __shared__ unsigned long long all_lds[];
             char* base = reinterpret_cast<char*>(all_lds) + wave * a.wave_lds;
