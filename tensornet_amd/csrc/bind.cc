@@ -16,9 +16,12 @@
 #include <torch/csrc/DynamicTypes.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <array>
 #include <memory>
 #include <string>
+#include <vector>
 
+#include "host_work.h"
 #include "tensornet_amd.h"
 
 namespace {
@@ -156,34 +159,73 @@ void run(Call& c) {
     call_library([&] { return c.run(stream); });
 }
 
-// A list of n tensors that are consecutive parts of `flat` (as torch.split hands them out), without the dispatcher.
+// n tensors that are consecutive parts of `flat` (as torch.split hands them out), without the dispatcher.  Half of what a view
+// takes is the tensor, which needs no interpreter (build), the other half its Python object (take).
 class Views {
 public:
-    Views(const at::Tensor& flat, Py_ssize_t n) : flat_(flat), list_(PyList_New(n)) {
-        if (!list_) throw PyFailed{};
-    }
+    Views(const at::Tensor& flat, Py_ssize_t n) : flat_(flat), n_((size_t)n) { made_.reserve(n_); }
     Views(const Views&) = delete;
-    ~Views() { Py_XDECREF(list_); }
-    void add(Py_ssize_t i, at::IntArrayRef sizes, int64_t offset) {
-        auto impl = c10::make_intrusive<c10::TensorImpl>(c10::TensorImpl::VIEW, c10::Storage(flat_.storage()),
-                                                         flat_.key_set(), flat_.dtype());
-        impl->set_storage_offset(offset);
-        impl->set_sizes_contiguous(sizes);
-        impl->set_version_counter(flat_.unsafeGetTensorImpl()->version_counter());
-        PyObject* o = THPVariable_Wrap(at::Tensor(std::move(impl)));
-        if (!o) throw PyFailed{};
-        PyList_SET_ITEM(list_, i, o);
+    // sizes(i): the next view's; those that build() has not come to are made by take().
+    template <typename Sizes>
+    void build(Sizes sizes) {
+        while (made_.size() < n_) {
+            const auto dims = sizes(made_.size());
+            auto impl = c10::make_intrusive<c10::TensorImpl>(c10::TensorImpl::VIEW, c10::Storage(flat_.storage()),
+                                                             flat_.key_set(), flat_.dtype());
+            impl->set_storage_offset(offset_);
+            impl->set_sizes_contiguous(dims);
+            impl->set_version_counter(flat_.unsafeGetTensorImpl()->version_counter());
+            offset_ += impl->numel();
+            made_.emplace_back(std::move(impl));
+        }
     }
-    PyObject* take() {
-        PyObject* l = list_;
-        list_ = nullptr;
-        return l;
+    template <typename Sizes>
+    PyObject* take(Sizes sizes) {
+        build(sizes);
+        PyObject* list = PyList_New((Py_ssize_t)n_);
+        if (!list) throw PyFailed{};
+        for (size_t i = 0; i < n_; i++) {
+            PyObject* o = THPVariable_Wrap(std::move(made_[i]));
+            if (!o) {
+                Py_DECREF(list);
+                throw PyFailed{};
+            }
+            PyList_SET_ITEM(list, (Py_ssize_t)i, o);
+        }
+        return list;
     }
 
 private:
     const at::Tensor& flat_;
-    PyObject* list_;
+    const size_t n_;
+    std::vector<at::Tensor> made_;
+    int64_t offset_ = 0;
 };
+
+// A call with outputs: their tensors are made while it waits for the device, which has nothing to do once it has reported.
+// (The tensors only, without the interpreter's lock: taking it in the middle of a call would have the call wait for other
+// Python threads.)  Pull and combine of 26 slots 46.4 -> 44.3 us; with the pooled push, 211 slots, 361 -> 354.
+template <typename C>
+PyObject* run_for_views(C& c) {
+    struct Work {
+        C& call;
+        Views views;
+    } work{c, Views(c.flat, c.n)};
+    tn_while_waiting(
+        [](void* p) {
+            Work& w = *static_cast<Work*>(p);
+            try {
+                w.views.build([&](size_t i) { return w.call.view_sizes(i); });
+            } catch (...) {  // (out of memory: take() tries again, and reports it)
+            }
+        },
+        &work);
+    struct TakeBack {
+        ~TakeBack() { tn_while_waiting(nullptr, nullptr); }
+    } take_back;
+    run(c);
+    return work.views.take([&](size_t i) { return c.view_sizes(i); });
+}
 
 struct PullCall : Call {
     uint32_t handle;
@@ -226,15 +268,7 @@ struct PullCall : Call {
             p += w.lens(1)[i];
         }
     }
-    PyObject* views() {
-        Views list(flat, n);
-        int64_t at = 0;
-        for (int i = 0; i < n; i++) {
-            list.add(i, {w.lens(1)[i]}, at);
-            at += w.lens(1)[i];
-        }
-        return list.take();
-    }
+    std::array<int64_t, 1> view_sizes(size_t i) { return {w.lens(1)[i]}; }
     int run(void* stream) override {
         return tn_sparse_table_pull_op(handle, n, w.ptrs<const int64_t>(0), w.lens(1), w.ptrs<float>(2), w.lens(3), dim,
                                        w.ptrs<int64_t>(4), stream);
@@ -314,11 +348,7 @@ struct CombineCall : Call {
         flat = at::empty({n, batch, dim}, r0.options().requires_grad(false));
         for (int i = 0; i < n; i++) w.ptrs<float>(5)[i] = (float*)flat.data_ptr() + (int64_t)i * batch * dim;
     }
-    PyObject* views() {
-        Views list(flat, n);
-        for (int i = 0; i < n; i++) list.add(i, {batch, (int64_t)dim}, (int64_t)i * batch * dim);
-        return list.take();
-    }
+    std::array<int64_t, 2> view_sizes(size_t) { return {batch, (int64_t)dim}; }
     int run(void* stream) override {
         return tn_sparse_table_combine_op(handle, n, w.ptrs<const int64_t>(0), w.lens(1), w.ptrs<const int64_t>(2),
                                           w.ptrs<const float>(3), w.lens(4), dim, batch, combiner, w.ptrs<float>(5), stream);
@@ -451,8 +481,7 @@ PyObject* py_pull(PyObject*, PyObject* const* a, Py_ssize_t na) {
         arg_count(na, 3, "sparse_table_pull");
         const Items resources(a[0]), values(a[1]);
         PullCall c(resources, values, handle_arg(a[2]));
-        run(c);
-        return c.views();
+        return run_for_views(c);
     });
 }
 
@@ -461,7 +490,7 @@ PyObject* py_bind_pull(PyObject*, PyObject* const* a, Py_ssize_t na) {
         arg_count(na, 3, "bind_pull");
         const Items resources(a[0]), values(a[1]);
         auto c = std::make_unique<PullCall>(resources, values, handle_arg(a[2]));
-        c->outputs = c->views();
+        c->outputs = Views(c->flat, c->n).take([&](size_t i) { return c->view_sizes(i); });
         return make_bound(std::move(c), {&resources, &values});
     });
 }
@@ -489,8 +518,7 @@ PyObject* py_combine(PyObject*, PyObject* const* a, Py_ssize_t na) {
         arg_count(na, 6, "embedding_lookup_sparse");
         const Items resources(a[0]), mapped(a[1]), examples(a[2]);
         CombineCall c(resources, mapped, examples, int_arg(a[3]), handle_arg(a[4]), (int)int_arg(a[5]));
-        run(c);
-        return c.views();
+        return run_for_views(c);
     });
 }
 
@@ -499,7 +527,7 @@ PyObject* py_bind_combine(PyObject*, PyObject* const* a, Py_ssize_t na) {
         arg_count(na, 6, "bind_combine");
         const Items resources(a[0]), mapped(a[1]), examples(a[2]);
         auto c = std::make_unique<CombineCall>(resources, mapped, examples, int_arg(a[3]), handle_arg(a[4]), (int)int_arg(a[5]));
-        c->outputs = c->views();
+        c->outputs = Views(c->flat, c->n).take([&](size_t i) { return c->view_sizes(i); });
         return make_bound(std::move(c), {&resources, &mapped, &examples});
     });
 }

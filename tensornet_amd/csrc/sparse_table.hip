@@ -3,6 +3,7 @@
 // and at operator level (core/kernels/sparse_table_ops.cc:170-265,317-368).
 #include "apply_launch.h"
 #include "combine_kernels.h"
+#include "host_work.h"
 #include "remap_lds.h"
 #include "table_level.h"
 
@@ -1244,6 +1245,17 @@ bool small_batch_shape(SparseTable* t, int N, const int64_t* lens, SmallShape& b
            small_emit_lds(N, b.cap, small_emit_table(b.cap)) <= t->small_emit_lds;
 }
 
+thread_local void (*waiting_fn)(void*) = nullptr;
+thread_local void* waiting_arg = nullptr;
+
+// The launches are queued and the host is about to wait for them.
+void do_host_work() {
+    if (void (*fn)(void*) = waiting_fn) {
+        waiting_fn = nullptr;
+        fn(waiting_arg);
+    }
+}
+
 // Waits for a kernel of the small path to report through pinned memory: *flag == want.  The word is polled for a
 // while (it arrives a few microseconds after the kernel's end, well before a wait on the stream or on an event
 // returns), then the stream is waited for, which also brings a failed launch to light.
@@ -1269,6 +1281,7 @@ int wait_reported(const uint32_t* flag, uint32_t want, hipStream_t st, const cha
 
 // The same for the words of a small pull's first launch: hwords[0 .. n) all carry `seq`.
 int wait_words(const uint64_t* words, uint32_t n, uint32_t seq, hipStream_t st, const char* what) {
+    do_host_work();
     const volatile uint64_t* w = words;
     const auto t0 = std::chrono::steady_clock::now();
     uint32_t i = 0;
@@ -2196,6 +2209,7 @@ int tn_sparse_table_pull_op(uint32_t table_handle, int N, const int64_t* const* 
         t->plan_lens.assign(value_lens, value_lens + N);
         t->plan_epoch = t->epoch;
         if (t->async_pull) return TN_OK;
+        do_host_work();
         if (early)
             TN_HIP(hipEventSynchronize(t->pub_ev));
         else if (early_inline)
@@ -2588,6 +2602,11 @@ int tn_sparse_table_combine_op(uint32_t table_handle, int N, const int64_t* cons
     if (err & DEV_ERR_GRAD_ROWS)
         return fail(TN_ERR_INVALID_ARGUMENT, "embedding combine: example ids must be non-decreasing and in [0, batch)");
     return TN_OK;
+}
+
+void tn_while_waiting(void (*fn)(void*), void* arg) {
+    waiting_fn = fn;
+    waiting_arg = arg;
 }
 
 }  // extern "C"
