@@ -1313,7 +1313,7 @@ int small_pull(SparseTable* t, const SmallShape& b, const int64_t* const* values
         t->stage_pending = false;
     }
     SlotDesc* descs = reinterpret_cast<SlotDesc*>(t->hstage);
-    bool vec = wdim % 4 == 0 && s.wstride % 4 == 0;
+    int width = (wdim | s.wstride) % 4 == 0 ? 4 : (wdim | s.wstride) % 2 == 0 ? 2 : 1;  // elements of a row moved together
     uint32_t at = 0;
     for (int i = 0; i < b.N; i++) {
         SlotDesc d{};
@@ -1325,7 +1325,7 @@ int small_pull(SparseTable* t, const SmallShape& b, const int64_t* const* values
         d.lbase = at;
         descs[i] = d;
         at += d.len;
-        vec = vec && aligned16(vars[i]);
+        while ((uintptr_t)vars[i] % (width * sizeof(float)) != 0) width /= 2;
     }
     const uint32_t seq = ++t->seq_pull, workgroups = (uint32_t)b.N * b.parts, entries = small_entries(b.max_len, b.parts);
     const size_t slots_lds = small_slots_lds(entries, b.max_len, b.nbp);
@@ -1335,7 +1335,7 @@ int small_pull(SparseTable* t, const SmallShape& b, const int64_t* const* values
     else
         TN_LAUNCH_LDS(k_small_slots_long, dim3(workgroups), dim3(2 * SMALL_THREADS), slots_lds, st, b, p, (const SlotDesc*)descs,
                       entries, s, make_optdev(t), t->seed, t->dplan, t->hwords, seq);
-    const uint32_t C = (uint32_t)(vec ? wdim / 4 : wdim), items = (size_t)b.L * C > FINISH_FULL ? FINISH_ITEMS : 1;
+    const uint32_t C = (uint32_t)(wdim / width), items = (size_t)b.L * C > FINISH_FULL ? FINISH_ITEMS : 1;
     const uint32_t per = items * FINISH_THREADS / C, chunks = (b.max_len + per - 1) / per;
     EmitArgs<true> ea;
     ea.b = b;
@@ -1345,15 +1345,19 @@ int small_pull(SparseTable* t, const SmallShape& b, const int64_t* const* values
     const size_t emit_lds = small_emit_lds(b.N, b.cap, ea.table);
     const uint32_t finish = (uint32_t)b.N * chunks;
     if (b.N > SMALL_SPLIT_SLOTS && emit_lds <= SMALL_SHARED_LDS) {
-        if (vec)
-            TN_LAUNCH_LDS((k_small_pull_rest<4>), dim3(b.buckets() + finish), dim3(FINISH_THREADS), emit_lds, st, ea, chunks, per, s);
-        else
-            TN_LAUNCH_LDS((k_small_pull_rest<1>), dim3(b.buckets() + finish), dim3(FINISH_THREADS), emit_lds, st, ea, chunks, per, s);
+#define TN_LAUNCH_REST(VEC)                                                                                              \
+    TN_LAUNCH_LDS((k_small_pull_rest<VEC>), dim3(b.buckets() + finish), dim3(FINISH_THREADS), emit_lds, st, ea, chunks, per, s)
+        if (width == 4) TN_LAUNCH_REST(4);
+        else if (width == 2) TN_LAUNCH_REST(2);
+        else TN_LAUNCH_REST(1);
+#undef TN_LAUNCH_REST
     } else {
-        if (vec)
-            TN_LAUNCH((k_small_group_finish<4>), dim3(finish), dim3(FINISH_THREADS), st, b, p, chunks, per, s);
-        else
-            TN_LAUNCH((k_small_group_finish<1>), dim3(finish), dim3(FINISH_THREADS), st, b, p, chunks, per, s);
+#define TN_LAUNCH_FINISH(VEC) \
+    TN_LAUNCH((k_small_group_finish<VEC>), dim3(finish), dim3(FINISH_THREADS), st, b, p, chunks, per, s)
+        if (width == 4) TN_LAUNCH_FINISH(4);
+        else if (width == 2) TN_LAUNCH_FINISH(2);
+        else TN_LAUNCH_FINISH(1);
+#undef TN_LAUNCH_FINISH
         TN_LAUNCH_LDS((k_group_emit<true>), dim3(b.buckets()), dim3(FINISH_THREADS), emit_lds, st, ea);
     }
     TN_HIP(hipGetLastError());
