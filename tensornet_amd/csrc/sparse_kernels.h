@@ -2343,16 +2343,18 @@ struct BigSrc {
     }
 };
 
-// apply_big_wave's rounds in the general path's kernels: a chunk of half the records, which takes 123 registers at D = 16 where 16
-// rounds take 150 and more.  In k_apply_all (beside the other signs' workgroups, so four wavefronts a SIMD are wanted) 2.1 M lookups
-// of 64 slots: 212 us a step with 8 rounds, 217 with 16; 430 k pooled of 211, signs of 211 records: 361 against 364.
-constexpr int BIG_MOST = 8;
+// apply_big_wave's rounds in the general path's kernels: chunks of a quarter of the records, which fit the 80 registers of six
+// wavefronts a SIMD at D = 16 (12 to 28 bytes spilled at 8, 32, 64) where 8 rounds take 123 and 16 take 150.  The other signs'
+// workgroups beside them wait for memory and want the wavefronts.  2.1 M lookups of 64 slots: 208.8 us a step with 4 rounds and
+// six wavefronts, 214.9 with 8 and four, 217 with 8 and six (88 bytes spilled) or 16 and four; 430 k pooled lookups of 211 slots,
+// signs of 211 records: 352.9, 352.1, 361.7, 364.
+constexpr int BIG_MOST = 4;
 
 // k_apply_big for AdaGrad rows of D elements, D a power of two from 4 to 64, on a plan whose big_desc lists {row, first member,
 // records, group} of every sign with many records (written by k_group_emit): one wavefront per sign, by apply_big_wave.  (Adam and
 // Ftrl the same way: 800 k lookups, Adam rows of 16, 136 us a step with and without; not worth their kernels.)
 template <int D>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_apply_big_adagrad(
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6, 8))) void k_apply_big_adagrad(
     Store s, OptDev o, PushSrc src, DevStatus* status, const uint4* __restrict__ big_desc, uint32_t desc_cap,
     const Member* __restrict__ list, const float* const* __restrict__ gaddr) {
     __shared__ BigWave<OPT_ADAGRAD, D, BIG_MOST> lds;
@@ -2387,7 +2389,7 @@ struct ApplyAll {
 constexpr int ALL_GBUF = 1088;  // floats of gradient staging per wavefront at most: eight workgroups to a CU up to 64 elements
 
 template <int KIND, int LPG, bool ANY, int TILE>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_apply_all(Store s, OptDev o, PushSrc src,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6, 8))) void k_apply_all(Store s, OptDev o, PushSrc src,
                                                                                               DevStatus* status, ApplyAll a) {
     // a push launched on a plan that turned out not to be its batch's (the host redoes it), or whose inputs are unusable
     if (status->mismatch | status->abort) return;
