@@ -362,7 +362,7 @@ int tn_sparse_table_last_unique_counts(uint32_t handle, int N, int64_t* counts);
  * stream themselves); its errors are then latched like push_op's. */
 int tn_sparse_table_set_async(uint32_t handle, int async_pull);
 
-/* Whether small batches (every slot at most 4096 lookups, at most 512 slots, 1048576 lookups in all and, up to 255
+/* Whether small batches (every slot at most 8192 lookups -- 4096 with eight slots or fewer --, at most 512 slots, 1048576 lookups in all and, up to 255
  * slots, 100 million slots x lookups -- 180 million if the table's last push had pooled gradients --, as far as a
  * workgroup's LDS goes) take the path of few launches (the default) or the one every other batch takes.  Same
  * results either way; a switch for measurements and tests, without a counterpart in the reference. */

@@ -518,8 +518,8 @@ __global__ __launch_bounds__(FINISH_THREADS) __attribute__((amdgpu_waves_per_eu(
 // First launch of a small push on the last pull's plan: the signs are compared with the plan's copy, and with CLICKS the
 // non-zero labels are added to the click sums (sparse_table_ops.cc:283-296; a few thousand lookups do not queue up on
 // any entry).  A mismatch also goes to the host (pinned memory); that the comparison is complete, the last launch tells it.
-// The workgroups behind those, a wavefront per bucket, put the ranks of the records' first lookups into the records, which
-// the updates would otherwise read by way of (the pull, which knows both, works them out side by side).
+// The workgroups behind those, a wavefront per bucket, put the ranks of the records' first lookups into the records: the
+// updates would otherwise read them through rank_at, a round trip more (the pull works ranks and records out side by side).
 template <bool CLICKS>
 __global__ __launch_bounds__(256) void k_small_verify(SmallShape b, SmallPlan p, const SlotDesc* host_descs, uint32_t chunks,
                                                       DevStatus* status, uint32_t* host_mismatch) {
