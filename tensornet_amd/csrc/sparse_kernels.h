@@ -2344,11 +2344,14 @@ struct BigSrc {
 };
 
 // apply_big_wave's rounds in the general path's kernels: chunks of a quarter of the records, which fit the 80 registers of six
-// wavefronts a SIMD at D = 16 (12 to 28 bytes spilled at 8, 32, 64) where 8 rounds take 123 and 16 take 150.  The other signs'
+// wavefronts a SIMD at D = 16 (8 to 16 bytes spilled at 32, 64) where 8 rounds take 123 and 16 take 150.  The other signs'
 // workgroups beside them wait for memory and want the wavefronts.  2.1 M lookups of 64 slots: 208.8 us a step with 4 rounds and
 // six wavefronts, 214.9 with 8 and four, 217 with 8 and six (88 bytes spilled) or 16 and four; 430 k pooled lookups of 211 slots,
 // signs of 211 records: 352.9, 352.1, 361.7, 364.
-constexpr int BIG_MOST = 4;
+// Rows of 4 and 8: two rounds, 32 and 16 records (four spill 17 and 13 registers, and the signs with few records, which are
+// the same kernel's, pay for it).  2.05 M lookups of 88 slots, 250 k signs, k_apply_all: rows of 4 46.5 us with four rounds,
+// 35.4 with two, rows of 8 45.4 and 38.9.
+constexpr int big_most(int D) { return D <= 8 ? 2 : 4; }
 
 // k_apply_big for AdaGrad rows of D elements, D a power of two from 4 to 64, on a plan whose big_desc lists {row, first member,
 // records, group} of every sign with many records (written by k_group_emit): one wavefront per sign, by apply_big_wave.  (Adam and
@@ -2357,7 +2360,7 @@ template <int D>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6, 8))) void k_apply_big_adagrad(
     Store s, OptDev o, PushSrc src, DevStatus* status, const uint4* __restrict__ big_desc, uint32_t desc_cap,
     const Member* __restrict__ list, const float* const* __restrict__ gaddr) {
-    __shared__ BigWave<OPT_ADAGRAD, D, BIG_MOST> lds;
+    __shared__ BigWave<OPT_ADAGRAD, D, big_most(D)> lds;
     const uint4 head = big_desc[blockIdx.x < desc_cap ? blockIdx.x : desc_cap - 1];  // (before the status is known)
     // a push launched on a plan that turned out not to be its batch's (the host redoes it), or whose inputs are unusable
     if (status->mismatch | status->abort) return;
@@ -2396,7 +2399,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6, 8))) voi
     if (blockIdx.x < a.big_blocks) {
         const uint32_t wave = threadIdx.x >> 6, first = blockIdx.x * 4 + wave, stride = a.big_blocks * 4;
         if constexpr (TILE != 0) {
-            __shared__ BigWave<KIND, TILE, BIG_MOST> lds[4];
+            __shared__ BigWave<KIND, TILE, big_most(TILE)> lds[4];
             const BigSrc from{src, a.list, a.gaddr};
             const uint4 head = a.big_desc[first < a.big_cap ? first : a.big_cap - 1];
             apply_big_wave<KIND, TILE>(
