@@ -5,6 +5,7 @@
 #include "combine_kernels.h"
 #include "host_work.h"
 #include "remap_lds.h"
+#include "row_width.h"
 #include "table_level.h"
 
 #include <algorithm>
@@ -1313,7 +1314,7 @@ int small_pull(SparseTable* t, const SmallShape& b, const int64_t* const* values
         t->stage_pending = false;
     }
     SlotDesc* descs = reinterpret_cast<SlotDesc*>(t->hstage);
-    int width = (wdim | s.wstride) % 4 == 0 ? 4 : (wdim | s.wstride) % 2 == 0 ? 2 : 1;  // elements of a row moved together
+    int width = row_width(wdim, s.wstride);
     uint32_t at = 0;
     for (int i = 0; i < b.N; i++) {
         SlotDesc d{};
@@ -1325,7 +1326,7 @@ int small_pull(SparseTable* t, const SmallShape& b, const int64_t* const* values
         d.lbase = at;
         descs[i] = d;
         at += d.len;
-        while ((uintptr_t)vars[i] % (width * sizeof(float)) != 0) width /= 2;
+        width = row_width_at(width, vars[i]);
     }
     const uint32_t seq = ++t->seq_pull, workgroups = (uint32_t)b.N * b.parts, entries = small_entries(b.max_len, b.parts);
     const size_t slots_lds = small_slots_lds(entries, b.max_len, b.nbp);
