@@ -219,6 +219,33 @@ __device__ __forceinline__ void pool_items(PoolLds& lds, uint32_t n, uint32_t bi
     }
 }
 
+// The sum of a sign whose lookups were dealt to `parts` workgroups, by a wavefront: its groups of LPG lanes take every so many of
+// the parts in turn and then add their sums up by halves.  has(q): part q has a share; share(q): its row.
+template <int LPG, bool ANY, typename Has, typename Share>
+__device__ __forceinline__ void add_shares(uint32_t parts, int D, Has has, Share share, float* __restrict__ out) {
+    const uint32_t group = (uint32_t)__lane_id() / LPG;
+    const int sub = (int)__lane_id() % LPG;
+    for (int c0 = 0; c0 < D; c0 += 4 * LPG) {
+        float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+        for (uint32_t q = group; q < parts; q += 64 / LPG) {
+            if (!has(q)) continue;
+            const float4 v = row_part<ANY>(share(q) + c0, sub, D - c0);
+            acc.x += v.x;
+            acc.y += v.y;
+            acc.z += v.z;
+            acc.w += v.w;
+        }
+#pragma unroll
+        for (int o = 32; o >= LPG; o >>= 1) {
+            acc.x += __shfl_xor(acc.x, o);
+            acc.y += __shfl_xor(acc.y, o);
+            acc.z += __shfl_xor(acc.z, o);
+            acc.w += __shfl_xor(acc.w, o);
+        }
+        if (group == 0) put_row_part<ANY>(out + c0, sub, D - c0, acc);
+    }
+}
+
 }  // namespace tn
 
 #endif  // TN_POOL_ITEMS_H_

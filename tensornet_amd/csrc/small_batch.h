@@ -38,6 +38,8 @@ constexpr int SMALL_BUCKETS_MAX = 2048;
 constexpr int SMALL_THREADS = 512;           // k_small_slots; twice as many for slots of more than SMALL_SLOT_SHORT lookups
 constexpr int SMALL_ITEMS = SMALL_SLOT_SHORT / SMALL_THREADS;
 constexpr int SMALL_WORDS = SMALL_SLOT_MAX / 64;  // 64-lookup words of a slot
+constexpr uint32_t SMALL_HEAVY_MAX = SMALL_SLOT_MAX / HEAVY_LOOKUPS;  // heavy signs of a slot at most
+constexpr uint32_t SMALL_NONE = 0xFFFFu;     // no position
 constexpr int SMALL_NEW = 512;               // rows a workgroup of k_small_slots lists to fill them with all its threads
 constexpr int FINISH_THREADS = 256;          // k_small_group_finish
 constexpr int SMALL_TILE = 1024;             // lookups per workgroup of k_small_verify
@@ -71,6 +73,7 @@ struct SmallPlan {
     uint2* group;          // per bucket, `cap` each: {row, first record | records << 16}; those with many records from the end on
     uint4* member;         // per bucket, `cap` each: records {gi, rank | slot << 16, occurrences, 0}, those of a sign in slot
                            // order (the rank comes in with a push, k_small_verify)
+    uint16_t* heavy;       // [slot][part][SMALL_HEAVY_MAX]: first lookups of the heavy signs (HEAVY_LOOKUPS), then SMALL_NONE
     uint32_t* bad;         // != 0: a bucket did not fit, a push has to analyse the batch itself
 };
 
@@ -79,11 +82,11 @@ __device__ __forceinline__ void host_store(uint32_t* p, uint32_t v) {
 }
 
 // What a workgroup of k_small_slots tells the host, in one word: its distinct signs, the rows it inserted, whether the
-// table is full, and the number of the call, which says that the word is this call's.
+// table is full, whether it has a heavy sign, and the number of the call, which says that the word is this call's.
 constexpr int SMALL_REPORT_BITS = 14;
-__host__ __device__ inline uint64_t small_report(uint32_t n_first, uint32_t n_new, bool full, uint32_t seq) {
+__host__ __device__ inline uint64_t small_report(uint32_t n_first, uint32_t n_new, bool full, bool heavy, uint32_t seq) {
     return (uint64_t)n_first | ((uint64_t)n_new << SMALL_REPORT_BITS) | ((uint64_t)(full ? 1 : 0) << (2 * SMALL_REPORT_BITS)) |
-           ((uint64_t)seq << 32);
+           ((uint64_t)(heavy ? 2 : 0) << (2 * SMALL_REPORT_BITS)) | ((uint64_t)seq << 32);
 }
 
 // Entries of the LDS table of k_small_slots: room for a slot of distinct signs that all fall into one part, and two
@@ -114,7 +117,8 @@ __device__ __forceinline__ void small_slots(const SmallShape& b, const SmallPlan
     __shared__ SlotDesc sd;
     __shared__ unsigned long long bits[SMALL_WORDS];
     __shared__ uint32_t wsum[THREADS / 64];
-    __shared__ uint32_t sh_first, sh_new, sh_full;
+    __shared__ uint32_t sh_first, sh_new, sh_full, sh_heavy;
+    __shared__ uint16_t heavy[SMALL_HEAVY_MAX];
     __shared__ uint32_t new_row[SMALL_NEW];
     __shared__ uint16_t new_ent[SMALL_NEW];
     const int sl = blockIdx.x / b.parts;
@@ -130,7 +134,8 @@ __device__ __forceinline__ void small_slots(const SmallShape& b, const SmallPlan
     }
     for (uint32_t i = tid; i <= b.nbp; i += THREADS) hist[i] = 0;
     for (uint32_t i = tid; i < SMALL_WORDS; i += THREADS) bits[i] = 0;
-    if (tid == 0) sh_first = sh_new = sh_full = 0;
+    if (tid == 0) sh_first = sh_new = sh_full = sh_heavy = 0;
+    if (tid < SMALL_HEAVY_MAX) heavy[tid] = SMALL_NONE;
     if (blockIdx.x == 0) {
         if (tid < sizeof(DevStatus) / 4) reinterpret_cast<uint32_t*>(status)[tid] = 0;
         if (tid == 0) *p.bad = 0;
@@ -197,6 +202,8 @@ __device__ __forceinline__ void small_slots(const SmallShape& b, const SmallPlan
         if (i < n_first) {
             const uint32_t e = used[i];
             const uint64_t sign = (uint64_t)keys[e];
+            const uint32_t w = word[e];
+            if ((w & 0xFFFFu) >= HEAVY_LOOKUPS) heavy[atomicAdd(&sh_heavy, 1u)] = (uint16_t)(w >> 16);
             bool is_new = false;
             row[r] = probe_slot<true>(s, sign, is_new);
             if (is_new) {
@@ -216,7 +223,7 @@ __device__ __forceinline__ void small_slots(const SmallShape& b, const SmallPlan
     __syncthreads();
     if (tid == 0) {
         __hip_atomic_store(reinterpret_cast<unsigned long long*>(host_words + blockIdx.x),
-                           (unsigned long long)small_report(n_first, sh_new, sh_full != 0, seq), __ATOMIC_RELAXED,
+                           (unsigned long long)small_report(n_first, sh_new, sh_full != 0, sh_heavy != 0, seq), __ATOMIC_RELAXED,
                            __HIP_MEMORY_SCOPE_SYSTEM);
         if (sh_new) atomicAdd(s.count, (unsigned long long)sh_new);
     }
@@ -233,6 +240,7 @@ __device__ __forceinline__ void small_slots(const SmallShape& b, const SmallPlan
         at += total;
     }
     if (tid == 0) p.boff[(size_t)blockIdx.x * (b.nbp + 1) + b.nbp] = (uint16_t)at;
+    if (tid < SMALL_HEAVY_MAX) p.heavy[blockIdx.x * SMALL_HEAVY_MAX + tid] = heavy[tid];
     __syncthreads();
     const uint32_t rbase = b.parts * lbase + part * len;
 #pragma unroll
@@ -590,42 +598,97 @@ inline uint32_t small_pool_parts_log2(uint32_t max_len) {
     while ((max_len >> lp) > SMALL_POOL_FILL) lp++;
     return lp;
 }
-constexpr uint32_t SMALL_POOL_ITEMS = SMALL_SLOT_MAX / POOL_THREADS;  // lookups of a thread
+constexpr uint32_t SMALL_POOL_AHEAD = 4;  // runs of 64 lookups of a wavefront in flight
 
-template <int LPG, bool ANY>
+// The heavy signs of a slot, by position: `heavy` (SMALL_HEAVY_MAX words of LDS), their number.  The workgroups that deal its
+// lookups out, and those that add the shares up, all have to have them in the same order.  Ends with a barrier.
+__device__ __forceinline__ uint32_t small_heavy(const SmallShape& b, const SmallPlan& p, uint32_t sl, uint32_t* heavy,
+                                                uint32_t* found) {
+    const uint32_t tid = threadIdx.x;
+    if (tid == 0) *found = 0;
+    __syncthreads();
+    if (tid < b.parts * SMALL_HEAVY_MAX) {
+        const uint32_t f = p.heavy[sl * b.parts * SMALL_HEAVY_MAX + tid];
+        if (f != SMALL_NONE) heavy[atomicAdd(found, 1u)] = f;
+    }
+    __syncthreads();
+    const uint32_t n = *found, f = tid < n ? heavy[tid] : 0u;
+    uint32_t rank = 0;
+    for (uint32_t e = 0; e < n; e++) rank += heavy[e] < f ? 1u : 0u;
+    __syncthreads();
+    if (tid < n) heavy[rank] = f;
+    __syncthreads();
+    return n;
+}
+static_assert(SMALL_PARTS_MAX * SMALL_HEAVY_MAX <= POOL_THREADS && SMALL_HEAVY_MAX * 64 == POOL_THREADS, "small_heavy");
+
+// HEAVY: the lookups of the slot's heavy signs are dealt to its workgroups run by run (64 lookups), each of which leaves a share
+// of their sums (k_small_pool_shares adds them up).  As one workgroup's such a sign is a chain of rounds (25 us each at 16
+// elements a row): 100 slots of 8000 lookups, 80 % of them one sign, a step with rows of 16 237 us, of 64 475;
+// so 163 and 266.
+template <int LPG, bool ANY, bool HEAVY>
 __global__ __launch_bounds__(POOL_THREADS) __attribute__((amdgpu_waves_per_eu(6, 6))) void k_small_pool(SmallShape b, SmallPlan p, const SlotDesc* __restrict__ descs,
                                                              int64_t batch, int dim, int D, int combiner,
                                                              float* __restrict__ flat, DevStatus* status, uint32_t* host_err,
-                                                             uint32_t lp) {
+                                                             uint32_t lp, float* __restrict__ shares,
+                                                             uint32_t* __restrict__ has) {
     __shared__ PoolLds lds;
+    __shared__ uint32_t heavy[HEAVY ? SMALL_HEAVY_MAX : 1], found, have, had;  // have: heavy signs with a sum so far
     __shared__ unsigned long long starts[SMALL_WORDS];  // of the examples
     __shared__ uint32_t bad;
-    const uint32_t sl = blockIdx.x >> lp, part = blockIdx.x & ((1u << lp) - 1u);
+    // The workgroups of a slot, which read the same lookups and rows, on one die (DieShare, an item per workgroup).  Dealt out
+    // in turn, the first part of every slot of eight parts, which has the sign that begins it, was the first die's.
+    const uint32_t item = blockIdx.x % XCDS * (gridDim.x / XCDS) + blockIdx.x / XCDS;  // (the grid is a multiple of XCDS)
+    const uint32_t sl = item >> lp, part = item & ((1u << lp) - 1u);
+    if (sl >= (uint32_t)b.N) return;
     const SlotDesc d = descs[sl];
     const uint32_t n = d.len, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     if (n == 0 || status->mismatch) return;
     const Global<const int64_t> ex = as_global((const int64_t*)d.mapped);
-    if (tid == 0) bad = 0;
-    __syncthreads();
-    uint32_t f[SMALL_POOL_ITEMS], x[SMALL_POOL_ITEMS];
+    const Global<const uint16_t> first_of = as_global((const uint16_t*)p.first_of + d.lbase);
+    if (tid == 0) bad = have = had = 0;
+    const uint32_t n_heavy = HEAVY ? small_heavy(b, p, sl, heavy, &found) : 0u;
+    if (!HEAVY) __syncthreads();
+    // a wavefront's runs, one behind the other
+    const uint32_t words = (n + 63) / 64, per = (words + POOL_WAVES - 1) / POOL_WAVES;
+    const uint32_t w0 = wave * per, w1 = min(words, w0 + per), mask = (1u << lp) - 1u;
+    const uint32_t others = ((n - 1) >> lp) + 1;  // keys of the signs that are not heavy; the heavy ones' behind them
+    // the key of a lookup of sign f at position i, if it is my part's
+    auto key_of = [&](uint32_t f, uint32_t i, bool& mine) {
+        mine = (f & mask) == part;
+        uint32_t key = f >> lp;
+        if (HEAVY)
+            for (uint32_t e = 0; e < n_heavy; e++)
+                if (f == heavy[e]) {
+                    mine = ((i >> 6) & mask) == part;
+                    key = others + e;
+                }
+        mine = mine && f != NO_ROW;
+        return key;
+    };
     uint32_t cnt = 0;
+#pragma unroll 1
+    for (uint32_t w = w0; w < w1; w += SMALL_POOL_AHEAD) {
+        int64_t e[SMALL_POOL_AHEAD], prev[SMALL_POOL_AHEAD];
+        uint32_t f[SMALL_POOL_AHEAD];
 #pragma unroll
-    for (uint32_t j = 0; j < SMALL_POOL_ITEMS; j++) {
-        const uint32_t i = (wave * SMALL_POOL_ITEMS + j) * 64 + lane;
-        bool head = false;
-        x[j] = 0;
-        f[j] = NO_ROW;
-        if (i < n) {
-            const int64_t e = ex[i], prev = i > 0 ? ex[i - 1] : -1;
-            if (e < 0 || e >= batch || prev > e) bad = 1;
-            head = e != prev;
-            x[j] = (uint32_t)e;
-            f[j] = p.first_of[d.lbase + i];
-            if ((f[j] & ((1u << lp) - 1u)) != part) f[j] = NO_ROW;
+        for (uint32_t j = 0; j < SMALL_POOL_AHEAD; j++) {
+            const uint32_t i = (w + j) * 64 + lane;
+            const bool there = w + j < w1 && i < n;
+            e[j] = there ? ex[i] : -1;
+            prev[j] = there && i > 0 ? ex[i - 1] : -1;
+            f[j] = there ? (uint32_t)first_of[i] : NO_ROW;
         }
-        const unsigned long long m = __ballot(head);
-        if (lane == 0) starts[i >> 6] = m;
-        cnt += (uint32_t)__popcll(__ballot(f[j] != NO_ROW));
+#pragma unroll
+        for (uint32_t j = 0; j < SMALL_POOL_AHEAD; j++) {
+            const bool there = f[j] != NO_ROW;
+            if (there && (e[j] < 0 || e[j] >= batch || prev[j] > e[j])) bad = 1;
+            const unsigned long long m = __ballot(there && e[j] != prev[j]);
+            if (lane == 0 && w + j < w1) starts[w + j] = m;
+            bool mine;
+            key_of(f[j], (w + j) * 64 + lane, mine);
+            cnt += (uint32_t)__popcll(__ballot(mine));
+        }
     }
     if (lane == 0) lds.wsum[wave] = cnt;
     __syncthreads();
@@ -642,29 +705,72 @@ __global__ __launch_bounds__(POOL_THREADS) __attribute__((amdgpu_waves_per_eu(6,
         if (w < wave) first += lds.wsum[w];
         total += lds.wsum[w];
     }
-    const uint32_t words = (n + 63) / 64, bits = (n - 1) >> lp ? 32 - (uint32_t)__clz((int)((n - 1) >> lp)) : 0u;
+    const uint32_t top = others - 1 + n_heavy, bits = top ? 32 - (uint32_t)__clz((int)top) : 0u;
+#pragma unroll 1
     for (uint32_t done = 0; done < total; done += POOL_ITEMS_MAX) {
         uint32_t at = first - done;  // (of a round before: wraps)
+#pragma unroll 1
+        for (uint32_t w = w0; w < w1; w += SMALL_POOL_AHEAD) {
+            // (read again: kept across the rounds in registers, of which 187 were spilled, 100 slots of 6000 lookups took 151 us
+            // here; so 54, and 50 with a slot's workgroups on one die)
+            int64_t e[SMALL_POOL_AHEAD];
+            uint32_t f[SMALL_POOL_AHEAD];
 #pragma unroll
-        for (uint32_t j = 0; j < SMALL_POOL_ITEMS; j++) {
-            const uint32_t i = (wave * SMALL_POOL_ITEMS + j) * 64 + lane;
-            const unsigned long long own = __ballot(f[j] != NO_ROW);
-            const uint32_t q = at + (uint32_t)__popcll(own & ((1ull << lane) - 1ull));
-            if (f[j] != NO_ROW && q < POOL_ITEMS_MAX) {
-                const float count = combiner == POOL_SUM ? 1.f : (float)(bit_above(starts, i, words, n) - bit_at_or_below(starts, i));
-                const float scale = pool_scale(count, combiner);
-                lds.key[q] = f[j] >> lp;
-                lds.example[q] = x[j];
-                lds.scale[q] = f[j] == i ? scale : -scale;
+            for (uint32_t j = 0; j < SMALL_POOL_AHEAD; j++) {
+                const uint32_t i = (w + j) * 64 + lane;
+                const bool there = w + j < w1 && i < n;
+                e[j] = there ? ex[i] : 0;
+                f[j] = there ? (uint32_t)first_of[i] : NO_ROW;
             }
-            at += (uint32_t)__popcll(own);
+#pragma unroll
+            for (uint32_t j = 0; j < SMALL_POOL_AHEAD; j++) {
+                const uint32_t i = (w + j) * 64 + lane;
+                bool mine;
+                const uint32_t key = key_of(f[j], i, mine);
+                const unsigned long long own = __ballot(mine);
+                const uint32_t q = at + (uint32_t)__popcll(own & ((1ull << lane) - 1ull));
+                if (mine && q < POOL_ITEMS_MAX) {
+                    const float count = combiner == POOL_SUM ? 1.f : (float)(bit_above(starts, i, words, n) - bit_at_or_below(starts, i));
+                    const float scale = pool_scale(count, combiner);
+                    lds.key[q] = key;
+                    lds.example[q] = (uint32_t)e[j];
+                    lds.scale[q] = f[j] == i ? scale : -scale;
+                }
+                at += (uint32_t)__popcll(own);
+            }
         }
         pool_items<LPG, ANY>(lds, min(POOL_ITEMS_MAX, total - done), bits, d.grads, dim, D,
                              [&](uint32_t key, bool first, bool& add) {
+                                 if (HEAVY && key >= others) {
+                                     add = ((had >> (key - others)) & 1u) != 0;
+                                     atomicOr(&have, 1u << (key - others));
+                                     return shares + ((uint64_t)item * SMALL_HEAVY_MAX + (key - others)) * dim;
+                                 }
                                  add = !first;
                                  return flat + (uint64_t)(d.lbase + ((key << lp) | part)) * dim;
                              });
+        if (HEAVY) {
+            if (tid == 0) had = have;
+            __syncthreads();
+        }
     }
+    if (HEAVY && tid == 0) has[item] = have;
+}
+
+// The sums of the heavy signs: a workgroup per slot, a wavefront per sign.
+template <int LPG, bool ANY>
+__global__ __launch_bounds__(64 * SMALL_HEAVY_MAX) void k_small_pool_shares(SmallShape b, SmallPlan p, int dim, int D,
+                                                                            float* __restrict__ flat, const DevStatus* status,
+                                                                            uint32_t lp, const float* __restrict__ shares,
+                                                                            const uint32_t* __restrict__ has) {
+    __shared__ uint32_t heavy[SMALL_HEAVY_MAX], found;
+    if (status->abort | status->mismatch) return;
+    const uint32_t sl = blockIdx.x, e = threadIdx.x / 64, item0 = sl << lp;
+    if (e >= small_heavy(b, p, sl, heavy, &found)) return;
+    add_shares<LPG, ANY>(
+        1u << lp, D, [&](uint32_t q) { return ((has[item0 + q] >> e) & 1u) != 0; },
+        [&](uint32_t q) { return shares + ((uint64_t)(item0 + q) * SMALL_HEAVY_MAX + e) * dim; },
+        flat + (uint64_t)(p.descs[sl].lbase + heavy[e]) * dim);
 }
 
 // Where the update kernels find the gradient of a record: the slots' matrices (in LDS), or the reduced rows of a push

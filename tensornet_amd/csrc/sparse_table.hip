@@ -136,6 +136,7 @@ struct SparseTable {
     uint32_t seq_comb = 0;
     uint32_t* hseq = nullptr;
     uint32_t seq_pull = 0, seq_verify = 0;
+    bool plan_heavy = false;        // the pull that left the plan (small, or through LDS) found a sign with HEAVY_LOOKUPS lookups in a slot
     std::vector<int64_t> plan_counts;  // distinct signs per slot of the small pull that left the plan
     SmallShape small_shape{};          // how that pull laid its batch out
     size_t small_lds = 0, small_emit_lds = 0;
@@ -1165,18 +1166,53 @@ void launch_small_apply(SparseTable* t, RowShare share, const SmallPlan& p, cons
         else LAUNCH(4, false);                                     \
     } while (0)
 
+// Where the reduction of a small push's pooled gradients leaves its sums.
+struct SmallPool {
+    uint32_t lp, blocks;  // workgroups of a slot (2^lp), of the launch
+    bool spread;          // heavy signs are dealt to all of a slot's (in one round's lookups none is a chain)
+    float *flat, *shares;
+    uint32_t* has;
+};
+int small_pool_room(SparseTable* t, int dim, SmallPool& r) {
+    const SmallShape& b = t->small_shape;
+    r.lp = small_pool_parts_log2(b.max_len);
+    r.blocks = (uint32_t)align_up((size_t)b.N << r.lp, XCDS);
+    r.spread = t->plan_heavy && b.max_len > POOL_ITEMS_MAX;
+    auto carve = [&](char* base) {
+        Carver c{base};
+        r.flat = c.take<float>((size_t)b.L * dim);
+        r.shares = c.take<float>(r.spread ? (size_t)r.blocks * SMALL_HEAVY_MAX * dim : 0);
+        r.has = c.take<uint32_t>(r.spread ? r.blocks : 0);
+        return align_up(c.off, 256);
+    };
+    TN_TRY(t->pooled_ws.ensure(carve(nullptr)));
+    carve((char*)t->pooled_ws.p);
+    return TN_OK;
+}
+
 // The gradients of a small push's distinct signs from pooled ones (k_small_pool).
-int launch_small_pool(SparseTable* t, bool aligned, const SmallPlan& p, int64_t batch, int dim, int combiner, float* flat,
-                      hipStream_t st, uint32_t* host_err) {
+void launch_small_pool(SparseTable* t, bool aligned, const SmallPlan& p, int64_t batch, int dim, int combiner, const SmallPool& r,
+                       hipStream_t st, uint32_t* host_err) {
     static_assert((int)POOL_SUM == (int)COMBINE_SUM && (int)POOL_MEAN == (int)COMBINE_MEAN && (int)POOL_SQRTN == (int)COMBINE_SQRTN, "");
     const SmallShape& b = t->small_shape;
-    const uint32_t lp = small_pool_parts_log2(b.max_len);
 #define TN_LAUNCH_POOL(LPG, ANY)                                                                                           \
-    TN_LAUNCH((k_small_pool<LPG, ANY>), dim3((uint32_t)b.N << lp), dim3(POOL_THREADS), st, b, p, p.push_descs, batch, dim, \
-              t->store.D, combiner, flat, t->dplan, host_err, lp)
-    TN_POOL_LANES(TN_LAUNCH_POOL, t->store.D, aligned);
+    TN_LAUNCH((k_small_pool<LPG, ANY, false>), dim3(r.blocks), dim3(POOL_THREADS), st, b, p, p.push_descs, batch, dim,     \
+              t->store.D, combiner, r.flat, t->dplan, host_err, r.lp, r.shares, r.has)
+#define TN_LAUNCH_SPREAD(LPG, ANY)                                                                                         \
+    TN_LAUNCH((k_small_pool<LPG, ANY, true>), dim3(r.blocks), dim3(POOL_THREADS), st, b, p, p.push_descs, batch, dim,      \
+              t->store.D, combiner, r.flat, t->dplan, host_err, r.lp, r.shares, r.has)
+#define TN_LAUNCH_SHARES(LPG, ANY)                                                                                         \
+    TN_LAUNCH((k_small_pool_shares<LPG, ANY>), dim3((uint32_t)b.N), dim3(64 * SMALL_HEAVY_MAX), st, b, p, dim, t->store.D, \
+              r.flat, t->dplan, r.lp, r.shares, r.has)
+    if (r.spread) {
+        TN_POOL_LANES(TN_LAUNCH_SPREAD, t->store.D, aligned);
+        TN_POOL_LANES(TN_LAUNCH_SHARES, t->store.D, dim % 4 == 0);
+    } else {
+        TN_POOL_LANES(TN_LAUNCH_POOL, t->store.D, aligned);
+    }
+#undef TN_LAUNCH_SHARES
+#undef TN_LAUNCH_SPREAD
 #undef TN_LAUNCH_POOL
-    return TN_OK;
 }
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
@@ -1197,6 +1233,7 @@ size_t carve_small(char* base, SmallPlan& p, const SmallShape& b) {
     p.head = c.take<uint4>(b.buckets());
     p.group = c.take<uint2>((size_t)b.buckets() * b.cap);
     p.member = c.take<uint4>((size_t)b.buckets() * b.cap);
+    p.heavy = c.take<uint16_t>(segments * SMALL_HEAVY_MAX);
     p.bad = c.take<uint32_t>(1);
     return align_up(c.off, 256);
 }
@@ -1380,6 +1417,7 @@ int small_pull(SparseTable* t, const SmallShape& b, const int64_t* const* values
     harvest(t);  // (a push before this call)
     uint64_t n_new = 0, n_distinct = 0;
     bool full = false;
+    t->plan_heavy = false;
     constexpr uint64_t MASK = (1u << SMALL_REPORT_BITS) - 1u;
     t->last_counts.assign(b.N, 0);
     for (uint32_t i = 0; i < workgroups; i++) {
@@ -1387,6 +1425,7 @@ int small_pull(SparseTable* t, const SmallShape& b, const int64_t* const* values
         t->last_counts[i / b.parts] += (int64_t)(w & MASK);
         n_new += (w >> SMALL_REPORT_BITS) & MASK;
         full |= ((w >> (2 * SMALL_REPORT_BITS)) & 1u) != 0;
+        t->plan_heavy |= ((w >> (2 * SMALL_REPORT_BITS)) & 2u) != 0;
     }
     // the call booked room for every sign it could have inserted; keep what it did insert
     t->count_upper -= t->booked - n_new;
@@ -1409,11 +1448,8 @@ int small_push(SparseTable* t, const int64_t* const* values, const float* const*
     const bool pooled = example_ids != nullptr, clicks = t->opt->kind == OPT_ADAGRAD;  // (the only optimizer that reads batch_click)
     SmallPlan p{};
     carve_small((char*)t->plan_buf.p, p, b);
-    float* flat = nullptr;
-    if (pooled) {
-        TN_TRY(t->pooled_ws.ensure(align_up((size_t)b.L * dim * sizeof(float), 256)));
-        flat = (float*)t->pooled_ws.p;
-    }
+    SmallPool pool{};
+    if (pooled) TN_TRY(small_pool_room(t, dim, pool));
     if (t->stage_pending) {
         TN_HIP(hipEventSynchronize(t->stage_ev));
         t->stage_pending = false;
@@ -1445,8 +1481,8 @@ int small_push(SparseTable* t, const int64_t* const* values, const float* const*
                   t->dplan, &t->hpush->st.mismatch);
     const bool rows16 = dim % 4 == 0 && t->store.wstride % 4 == 0;
     if (pooled)
-        TN_TRY(launch_small_pool(t, vec, p, batch, dim, combiner, flat, st, &t->hpush->st.abort));
-    launch_small_apply(t, row_share(t->store, (pooled || vec) && rows16), p, flat, dim, st, t->hseq + 1, seq);
+        launch_small_pool(t, vec, p, batch, dim, combiner, pool, st, &t->hpush->st.abort);
+    launch_small_apply(t, row_share(t->store, (pooled || vec) && rows16), p, pool.flat, dim, st, t->hseq + 1, seq);
     // what a call on another stream has to wait for: the updates are still running when this call returns
     TN_HIP(hipEventRecord(t->tail_ev, st));
     t->tail_recorded = true;

@@ -92,6 +92,8 @@ struct DevStatus {
     uint32_t tile_share_q16;  // remap through LDS: records handed to the first-level buckets per lookup, largest share of a slot, in 1 / 65536
     uint32_t pad[1];
 };
+// Lookups of a sign in its slot from which a push of pooled gradients deals them to several workgroups.
+constexpr uint32_t HEAVY_LOOKUPS = 1024;
 
 // The chip is eight dies, each with an L2 of its own, and the workgroups of a launch go to the dies in turn
 // (workgroup i to die i % 8).  A kernel whose neighbouring work items touch the same memory gives every die a
