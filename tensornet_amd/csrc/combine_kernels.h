@@ -149,22 +149,32 @@ constexpr uint32_t POOL_TILE = 64 * KEY_WAVES * KEY_ITEMS;
 constexpr uint32_t POOL_PARTS_LOG2 = 11;
 constexpr uint32_t POOL_FILL = 1600;  // (49 k lookups a slot: 32 parts 176 us, 64 parts 255; of 4 k: 4 parts 42, 8 parts 56)
 constexpr uint32_t POOL_SPREAD = 64;
-constexpr uint32_t POOL_SPREAD_LOG2 = 3;  // 2^3 parts and more: a slot of 12800 lookups (POOL_FILL)
+constexpr uint32_t POOL_EXTRA = 64;
+constexpr uint32_t POOL_SHARES = POOL_SPREAD + POOL_EXTRA;
+// Slots of 2^3 parts and more have spread signs: from 6404 lookups on.  Shorter ones of several parts have extra ones only, and
+// only if the pull has found a heavy sign in the batch (DevStatus::heavy), or did not look for one: it is up to three further
+// rounds there, and finding it and adding up the shares are two launches.
+constexpr uint32_t POOL_SPREAD_LOG2 = 3, POOL_SPREAD_LOG2_HEAVY = 1;
 
 // How a slot's lookups are shared out to the backward pass's workgroups: in tiles of POOL_TILE for step 1, for step 2 in
 // 2^lp parts of POOL_FILL lookups at most on average.  The distinct indices of the slot ascend with the signs' first occurrences, so
 // that the frequent signs come early.  The lookups of the first `spread` indices of a slot with many parts are dealt to these
 // run by run (64 lookups), and every part leaves a share of those signs' sums (k_reduce_pooled_shares adds them up): a sign
-// with 8 % of a slot's lookups would be three rounds of one part, and the last workgroup's.  The other indices are
+// with 8 % of a slot's lookups would be three rounds of one part, and the last workgroup's.  So are those of up to POOL_EXTRA
+// further ones with half as many lookups as a part or more (k_pool_frequent).  The other indices are
 // dealt modulo 2^lp.  Tiles and parts of a call are numbered through the slots so that a slot's
 // first is known from the lookups before it; some numbers are nobody's.
 struct PoolShare {
     uint32_t lp_max;  // of the longest slot
+    uint32_t spread_log2;
+    PoolShare(uint32_t max_len, bool heavy)
+        : lp_max(parts_log2(max_len)), spread_log2(heavy ? POOL_SPREAD_LOG2_HEAVY : POOL_SPREAD_LOG2) {}
     static __host__ __device__ uint32_t parts_log2(uint32_t len) {
         uint32_t lp = 0;
         while (lp < POOL_PARTS_LOG2 && (len >> lp) > POOL_FILL) lp++;
         return lp;
     }
+    __host__ __device__ bool spreads(uint32_t lp) const { return lp >= spread_log2; }  // has extra ones, maybe
     static __host__ __device__ uint32_t spread(uint32_t lp) { return lp >= POOL_SPREAD_LOG2 ? POOL_SPREAD : 0u; }
     static __host__ __device__ uint32_t first_tile(uint32_t slot, uint32_t lookups_before) {
         return lookups_before / POOL_TILE + slot;
@@ -175,6 +185,74 @@ struct PoolShare {
     }
 };
 
+// Which signs of a slot that has spread ones are frequent although they come late -- behind the first distinct ones, or where
+// the lookups are grouped: `extra`, per slot the number of them, then their indices.  Left to one part such a sign is a chain
+// of rounds: 100 slots of 49 k lookups, 80 % of them a sign that comes 101st, k_reduce_pooled 632 us, so 155; a step of one
+// slot of a million 9.2 ms, so 0.27.  The counts of a sample decide: 128 runs of sixteen lookups (in a short slot fewer) at places that are even but for a
+// jitter (positions with a period would all look alike).  A workgroup per slot; what is chosen depends on the lookups alone, not on the order of atomics.
+constexpr uint32_t FREQUENT_RUN = 16, FREQUENT_SAMPLES = 2048, FREQUENT_TABLE = 4096;
+constexpr uint32_t FREQUENT_LEAST = 8;  // of the sample, however long the slot: fewer are chance
+constexpr uint32_t FREQUENT_LISTED = FREQUENT_SAMPLES / FREQUENT_LEAST;
+static __global__ __launch_bounds__(POOL_THREADS) void k_pool_frequent(const uint32_t* __restrict__ lbase,
+                                                                       const uint32_t* __restrict__ ubase,
+                                                                       const uint32_t* __restrict__ u_of_gi, PoolShare share,
+                                                                       uint32_t* __restrict__ extra) {
+    __shared__ uint32_t index[FREQUENT_TABLE], count[FREQUENT_TABLE];
+    __shared__ uint32_t listed[FREQUENT_LISTED], times[FREQUENT_LISTED], n_listed;
+    const uint32_t sl = blockIdx.x, tid = threadIdx.x, l0 = lbase[sl], len = lbase[sl + 1] - l0, ub = ubase[sl];
+    uint32_t* const out = extra + sl * (POOL_EXTRA + 1);
+    const uint32_t lp = share.parts_log2(len), spread = share.spread(lp);
+    if (!share.spreads(lp)) {
+        if (tid == 0) out[0] = 0;
+        return;
+    }
+    constexpr uint32_t PER = FREQUENT_SAMPLES / POOL_THREADS;
+    const uint32_t runs = min(FREQUENT_SAMPLES / FREQUENT_RUN, len / (2 * FREQUENT_RUN));  // (several parts: len is POOL_FILL and more)
+    uint32_t x[PER];
+#pragma unroll
+    for (uint32_t j = 0; j < PER; j++) {
+        const uint32_t r = (j * POOL_THREADS + tid) / FREQUENT_RUN;
+        x[j] = NO_ROW;
+        if (r >= runs) continue;
+        const uint32_t from = (uint32_t)((uint64_t)len * r / runs), room = (uint32_t)((uint64_t)len * (r + 1) / runs) - from;
+        const uint32_t jitter = (uint32_t)(((uint64_t)((r + 1) * 2654435761u) * (room - FREQUENT_RUN + 1)) >> 32);
+        x[j] = (u_of_gi[l0 + from + jitter + tid % FREQUENT_RUN] & ~FIRST_BIT) - ub;  // (room: two runs' at least)
+    }
+    for (uint32_t i = tid; i < FREQUENT_TABLE; i += POOL_THREADS) {
+        index[i] = NO_ROW;
+        count[i] = 0;
+    }
+    if (tid == 0) n_listed = 0;
+    __syncthreads();
+#pragma unroll
+    for (uint32_t j = 0; j < PER; j++) {
+        if (x[j] < spread || x[j] == NO_ROW) continue;
+        for (uint32_t h = (x[j] * 2654435761u) / (uint32_t)(0x100000000ull / FREQUENT_TABLE);; h = (h + 1) % FREQUENT_TABLE) {
+            const uint32_t old = atomicCAS(&index[h], NO_ROW, x[j]);
+            if (old != NO_ROW && old != x[j]) continue;  // (half of the entries stay free)
+            atomicAdd(&count[h], 1u);
+            break;
+        }
+    }
+    __syncthreads();
+    const uint32_t least = max(FREQUENT_LEAST, (uint32_t)((uint64_t)runs * FREQUENT_RUN * (POOL_FILL / 2) / len));
+    for (uint32_t i = tid; i < FREQUENT_TABLE; i += POOL_THREADS) {
+        if (count[i] < least) continue;
+        const uint32_t k = atomicAdd(&n_listed, 1u);
+        listed[k] = index[i];
+        times[k] = count[i];
+    }
+    __syncthreads();
+    const uint32_t n = n_listed;
+    if (tid == 0) out[0] = min(n, POOL_EXTRA);
+    if (tid >= n) return;
+    uint32_t rank = 0;  // the most frequent first, of those alike the one that comes first
+    for (uint32_t i = 0; i < n; i++)
+        rank += times[i] > times[tid] || (times[i] == times[tid] && listed[i] < listed[tid]) ? 1u : 0u;
+    if (rank < POOL_EXTRA) out[1 + rank] = listed[tid];
+}
+static_assert(FREQUENT_LISTED <= POOL_THREADS && FREQUENT_SAMPLES % POOL_THREADS == 0 && 2 * FREQUENT_SAMPLES <= FREQUENT_TABLE, "");
+
 // Backward, step 1.  A tile of POOL_TILE lookups of a slot leaves an item for every lookup -- example, sign, lookups of the
 // example --, the items of a part side by side in the order of their positions, and where the parts start among them.
 //
@@ -183,7 +261,8 @@ struct PoolShare {
 // followed there by the whole wavefront.  Places in a part come from ballots over the bits of the part's number (as in
 // k_table_part): no atomics whose order of arrival would show.
 // An item: x the example, y bits 0-10 its lookups (POOL_COUNT_MANY: as many or more), 11 the sign's first lookup, 12-31 the
-// key: of the first `spread` distinct indices these themselves, of the others spread + (index - spread) / 2^lp.
+// key: of the first `spread` distinct indices these themselves, of the extra ones spread + their place among them, of the
+// others (index - spread) / 2^lp behind those.
 constexpr uint32_t POOL_COUNT_MANY = 0x7FF;
 constexpr uint32_t POOL_FIRST = 0x800;
 constexpr uint32_t POOL_KEY_SHIFT = 12;
@@ -194,8 +273,9 @@ static __global__ __launch_bounds__(256) void k_lookup_keys(const SlotDesc* __re
                                                      const uint32_t* __restrict__ ubase, uint32_t N,
                                                      const uint32_t* __restrict__ u_of_gi, int64_t batch,
                                                      uint2* __restrict__ pool, uint16_t* __restrict__ poff, PoolShare share,
-                                                     DevStatus* status) {
+                                                     const uint32_t* __restrict__ extra, DevStatus* status) {
     extern __shared__ uint32_t cnt[];  // [2^lp][KEY_WAVES]
+    __shared__ uint32_t more[POOL_EXTRA];
     __shared__ uint32_t wsum[KEY_WAVES];
     __shared__ uint32_t slot;
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -210,6 +290,7 @@ static __global__ __launch_bounds__(256) void k_lookup_keys(const SlotDesc* __re
     const uint32_t sl = slot, l0 = lbase[sl], len = lbase[sl + 1] - l0;
     const uint32_t t0 = (blockIdx.x - share.first_tile(sl, l0)) * POOL_TILE, lp = share.parts_log2(len);
     const uint32_t ub = ubase[sl], parts = 1u << lp, spread = share.spread(lp);
+    const uint32_t extras = share.spreads(lp) ? extra[sl * (POOL_EXTRA + 1)] : 0u, spread_all = spread + extras;
     const Global<const int64_t> ex = example_of(descs[sl]);
     int64_t b[KEY_ITEMS], prev[KEY_ITEMS];
     uint32_t u[KEY_ITEMS];
@@ -225,7 +306,27 @@ static __global__ __launch_bounds__(256) void k_lookup_keys(const SlotDesc* __re
         }
     }
     for (uint32_t i = tid; i < parts * KEY_WAVES; i += 256) cnt[i] = 0;
+    if (tid < extras) more[tid] = extra[sl * (POOL_EXTRA + 1) + 1 + tid];
     __syncthreads();
+    // numbered through: the spread indices first, then the others
+    if (extras == 0) {
+#pragma unroll
+        for (uint32_t j = 0; j < KEY_ITEMS; j++) u[j] -= ub;
+    } else {
+        uint32_t to[KEY_ITEMS];
+#pragma unroll
+        for (uint32_t j = 0; j < KEY_ITEMS; j++) {
+            const uint32_t index = (u[j] & ~FIRST_BIT) - ub;
+            to[j] = index < spread ? index : index + extras;
+        }
+        for (uint32_t e = 0; e < extras; e++) {
+            const uint32_t x = more[e] + extras;
+#pragma unroll
+            for (uint32_t j = 0; j < KEY_ITEMS; j++) to[j] = to[j] == x ? ~(spread + e) : to[j];
+        }
+#pragma unroll
+        for (uint32_t j = 0; j < KEY_ITEMS; j++) u[j] = (u[j] & FIRST_BIT) | ((int)to[j] < 0 ? ~to[j] : to[j]);
+    }
     uint32_t count[KEY_ITEMS], at[KEY_ITEMS];
     bool bad = false;
 #pragma unroll
@@ -263,8 +364,8 @@ static __global__ __launch_bounds__(256) void k_lookup_keys(const SlotDesc* __re
         const uint32_t to_end = above ? (uint32_t)__ffsll((long long)above) - 1 - lane : 64 - lane + ahead;
         count[j] = min(to_start + to_end, POOL_COUNT_MANY);
         // its place among the tile's lookups of its part: behind those of earlier runs and lanes
-        const uint32_t index = (u[j] & ~FIRST_BIT) - ub;
-        const uint32_t part = (index < spread ? i >> 6 : index - spread) & (parts - 1u), k = part * KEY_WAVES + wave;
+        const uint32_t index = u[j] & ~FIRST_BIT;
+        const uint32_t part = (index < spread_all ? i >> 6 : index - spread_all) & (parts - 1u), k = part * KEY_WAVES + wave;
         unsigned long long same = __ballot(active);
         for (uint32_t q = 0; q < lp; q++) {
             const unsigned long long m = __ballot((part >> q) & 1u);
@@ -298,10 +399,10 @@ static __global__ __launch_bounds__(256) void k_lookup_keys(const SlotDesc* __re
     __syncthreads();
 #pragma unroll
     for (uint32_t j = 0; j < KEY_ITEMS; j++) {
-        const uint32_t i = t0 + (wave * KEY_ITEMS + j) * 64 + lane, index = (u[j] & ~FIRST_BIT) - ub;
+        const uint32_t i = t0 + (wave * KEY_ITEMS + j) * 64 + lane, index = u[j] & ~FIRST_BIT;
         if (i >= len) continue;
-        const uint32_t part = (index < spread ? i >> 6 : index - spread) & (parts - 1u);
-        const uint32_t key = index < spread ? index : spread + ((index - spread) >> lp);
+        const uint32_t part = (index < spread_all ? i >> 6 : index - spread_all) & (parts - 1u);
+        const uint32_t key = index < spread_all ? index : spread_all + ((index - spread_all) >> lp);
         pool[l0 + t0 + cnt[part * KEY_WAVES + wave] + at[j]] =
             make_uint2((uint32_t)b[j], count[j] | (u[j] & FIRST_BIT ? POOL_FIRST : 0u) | (key << POOL_KEY_SHIFT));
     }
@@ -335,7 +436,7 @@ __device__ __forceinline__ uint32_t lookups_of(Global<const int64_t> ex, uint32_
 // three workgroups on a CU.  4.9 M lookups in 100 slots, rows of 16: 175 us, with k_lookup_keys (46) and the shares (6) 227,
 // where a counting sort of the lookups through memory, an ordering pass and a reduction by sign took 390; 860 k in 211 slots:
 // 58 for 103.
-static_assert((1u << POOL_SPREAD_LOG2) % 8 == 0 && POOL_SPREAD == 64, "k_reduce_pooled_shares");
+static_assert(POOL_SPREAD == 64 && POOL_EXTRA <= POOL_SPREAD, "k_reduce_pooled_shares");
 template <int LPG, bool ANY>
 __global__ __launch_bounds__(POOL_THREADS) __attribute__((amdgpu_waves_per_eu(6, 6))) void k_reduce_pooled(const SlotDesc* __restrict__ descs,
                                                                 const uint32_t* __restrict__ lbase,
@@ -343,19 +444,17 @@ __global__ __launch_bounds__(POOL_THREADS) __attribute__((amdgpu_waves_per_eu(6,
                                                                 const uint2* __restrict__ pool,
                                                                 const uint16_t* __restrict__ poff, int dim, int D, int combiner,
                                                                 const DevStatus* status, float* __restrict__ flat,
-                                                                PoolShare share, float* __restrict__ shares,
-                                                                uint64_t* __restrict__ has) {
+                                                                PoolShare share, const uint32_t* __restrict__ extra,
+                                                                float* __restrict__ shares, uint64_t* __restrict__ has) {
     __shared__ PoolLds lds;
     __shared__ uint32_t slot;
-    __shared__ unsigned long long have, had;  // spread signs with a sum so far, before the round
+    __shared__ unsigned long long have[POOL_SHARES / 64], had[POOL_SHARES / 64];  // spread signs with a sum so far, before the round
     // the workgroups of a slot, which read the same rows, on one die (DieShare, an item per workgroup)
     const uint32_t item = blockIdx.x % XCDS * (gridDim.x / XCDS) + blockIdx.x / XCDS;  // (the grid is a multiple of XCDS)
     if (status->abort | status->mismatch) return;
     const uint32_t tid = threadIdx.x;
-    if (tid == 0) {
-        slot = N;
-        have = had = 0;
-    }
+    if (tid == 0) slot = N;
+    if (tid < POOL_SHARES / 64) have[tid] = had[tid] = 0;
     __syncthreads();
     for (uint32_t s = tid; s < N; s += POOL_THREADS) {
         const uint32_t a = lbase[s], b = lbase[s + 1], q = item - share.first_part(s, a);  // (wraps before the slot)
@@ -365,9 +464,10 @@ __global__ __launch_bounds__(POOL_THREADS) __attribute__((amdgpu_waves_per_eu(6,
     if (slot == N) return;
     const uint32_t sl = slot, l0 = lbase[sl], len = lbase[sl + 1] - l0, ub = ubase[sl], us = ubase[sl + 1] - ub;
     const uint32_t lp = share.parts_log2(len), part = item - share.first_part(sl, l0), tile0 = share.first_tile(sl, l0);
-    const uint32_t spread = share.spread(lp);
-    if (!spread && part >= us) return;
-    const uint32_t top = us > spread ? spread + ((us - 1 - spread) >> lp) : us - 1, bits = top ? 32 - (uint32_t)__clz((int)top) : 0u;
+    const uint32_t spread = share.spread(lp), spread_all = spread + (share.spreads(lp) ? extra[sl * (POOL_EXTRA + 1)] : 0u);
+    if (!spread_all && part >= us) return;
+    const uint32_t rest = ub + spread + part;  // the part's first row of an index that is not spread
+    const uint32_t top = us > spread ? spread_all + ((us - 1 - spread) >> lp) : us - 1, bits = top ? 32 - (uint32_t)__clz((int)top) : 0u;
     const float* pooled = descs[sl].grads;
     const Global<const int64_t> ex = example_of(descs[sl]);
     const uint32_t mine = (len + POOL_TILE - 1) / POOL_TILE;
@@ -406,59 +506,48 @@ __global__ __launch_bounds__(POOL_THREADS) __attribute__((amdgpu_waves_per_eu(6,
             }
             if (done < total)
                 pool_items<LPG, ANY>(lds, n, bits, pooled, dim, D, [&](uint32_t key, bool first, bool& add) {
-                    if (key < spread) {
-                        add = ((had >> key) & 1ull) != 0;
-                        atomicOr(&have, 1ull << key);
-                        return shares + ((uint64_t)item * POOL_SPREAD + key) * dim;
+                    if (key < spread_all) {
+                        add = ((had[key / 64] >> (key % 64)) & 1ull) != 0;
+                        atomicOr(&have[key / 64], 1ull << (key % 64));
+                        return shares + ((uint64_t)item * POOL_SHARES + key) * dim;
                     }
                     add = !first;
-                    return flat + (uint64_t)(ub + spread + (((key - spread) << lp) | part)) * dim;
+                    return flat + (uint64_t)(rest + ((key - spread_all) << lp)) * dim;
                 });
             else
                 __syncthreads();
-            if (spread) {
-                if (tid == 0) had = have;
+            if (spread_all) {
+                if (tid < POOL_SHARES / 64) had[tid] = have[tid];
                 __syncthreads();
             }
         }
     }
-    if (spread && tid == 0) has[item] = have;
+    if (spread_all && tid < POOL_SHARES / 64) has[(uint64_t)item * (POOL_SHARES / 64) + tid] = have[tid];
 }
 
-// The sums of the spread signs: a wavefront per sign, whose groups of LPG lanes take every so many of the slot's parts in turn
-// and then add their sums up by halves.
+// The sums of the spread signs, a wavefront per sign.
 template <int LPG, bool ANY>
 __global__ __launch_bounds__(256) void k_reduce_pooled_shares(const uint32_t* __restrict__ lbase,
                                                               const uint32_t* __restrict__ ubase, int dim, int D,
                                                               const DevStatus* status, const float* __restrict__ shares,
                                                               const uint64_t* __restrict__ has, float* __restrict__ flat,
-                                                              PoolShare share) {
+                                                              PoolShare share, const uint32_t* __restrict__ extra) {
     if (status->abort | status->mismatch) return;
     constexpr uint32_t PER = 256 / 64;
-    const uint32_t sl = blockIdx.x / (POOL_SPREAD / PER), key = blockIdx.x % (POOL_SPREAD / PER) * PER + threadIdx.x / 64;
-    const uint32_t group = threadIdx.x % 64 / LPG;
-    const int sub = threadIdx.x % LPG;
+    const uint32_t sl = blockIdx.x / (POOL_SPREAD / PER), key0 = blockIdx.x % (POOL_SPREAD / PER) * PER + threadIdx.x / 64;
     const uint32_t l0 = lbase[sl], len = lbase[sl + 1] - l0, ub = ubase[sl], us = ubase[sl + 1] - ub;
-    const uint32_t lp = share.parts_log2(len), parts = 1u << lp, p0 = share.first_part(sl, l0);
-    if (len == 0 || share.spread(lp) == 0 || key >= us) return;  // (the same for a whole wavefront)
-    for (int c0 = 0; c0 < D; c0 += 4 * LPG) {
-        float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
-        for (uint32_t q = group; q < parts; q += 64 / LPG) {
-            if (!((has[p0 + q] >> key) & 1ull)) continue;
-            const float4 v = row_part<ANY>(shares + ((uint64_t)(p0 + q) * POOL_SPREAD + key) * dim + c0, sub, D - c0);
-            acc.x += v.x;
-            acc.y += v.y;
-            acc.z += v.z;
-            acc.w += v.w;
-        }
-#pragma unroll
-        for (int o = 32; o >= LPG; o >>= 1) {
-            acc.x += __shfl_xor(acc.x, o);
-            acc.y += __shfl_xor(acc.y, o);
-            acc.z += __shfl_xor(acc.z, o);
-            acc.w += __shfl_xor(acc.w, o);
-        }
-        if (group == 0) put_row_part<ANY>(flat + (uint64_t)(ub + key) * dim + c0, sub, D - c0, acc);
+    const uint32_t lp = share.parts_log2(len), p0 = share.first_part(sl, l0);
+    if (len == 0 || !share.spreads(lp)) return;
+    const uint32_t* const more = extra + sl * (POOL_EXTRA + 1);
+    const uint32_t spread = share.spread(lp), spread_all = spread + more[0];
+    for (uint32_t key = key0; key < spread_all; key += POOL_SPREAD) {  // (the same for a whole wavefront)
+        const uint32_t index = key < spread ? key : more[1 + key - spread];
+        if (index >= us) return;
+        add_shares<LPG, ANY>(
+            1u << lp, D,
+            [&](uint32_t q) { return ((has[(uint64_t)(p0 + q) * (POOL_SHARES / 64) + key / 64] >> (key % 64)) & 1ull) != 0; },
+            [&](uint32_t q) { return shares + ((uint64_t)(p0 + q) * POOL_SHARES + key) * dim; },
+            flat + (uint64_t)(ub + index) * dim);
     }
 }
 

@@ -327,6 +327,7 @@ __global__ __launch_bounds__(DEDUP_THREADS) void k_lds_dedup(const uint32_t* __r
     // The buckets of a slot scatter four-byte words over the same stretch of first_of and cnt_at (the slot's
     // positions): on one die they meet in one L2 and leave it as whole lines.
     const DieShare share(nbuckets);
+    bool heavy = false;
     for (uint32_t b = share.first; b < share.end; b += share.step) {
         const uint32_t n = min(bcursor[b], (uint32_t)L1_ROOM);
         if (n == 0) continue;
@@ -391,9 +392,10 @@ __global__ __launch_bounds__(DEDUP_THREADS) void k_lds_dedup(const uint32_t* __r
             const uint32_t f = minpos[h];
             if (f != gi) {
                 first_of[gi] = f;  // k_tile_dedup left first_of[gi] = gi
-            } else {
+            } else {  // one record per occupied entry gets here
+                heavy |= cnts[h] >= HEAVY_LOOKUPS;
                 if (!EMIT) cnt_at[gi] = cnts[h];  // with EMIT the record carries the count
-                if (EMIT) {  // one record per occupied entry gets here
+                if (EMIT) {
                     // the sign's only record: all its lookups lie in one tile (what a push makes of it: the tile's
                     // click sum for the sign is the whole sum)
                     if (cnts[h] == mu[j]) cnts[h] |= REC_ONE_TILE;
@@ -425,6 +427,7 @@ __global__ __launch_bounds__(DEDUP_THREADS) void k_lds_dedup(const uint32_t* __r
         }
         __syncthreads();
     }
+    if (heavy) status->heavy = 1;  // (all that write, write this)
 }
 
 // Rank of the first occurrence at position gi = number of first occurrences before it: the

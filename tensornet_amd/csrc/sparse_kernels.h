@@ -132,6 +132,7 @@ static __global__ void k_reset_status(DevStatus* status, uint32_t n_unique, uint
         status->abort = 0;
         status->n_big = 0;
         status->tile_share_q16 = 0;
+        status->heavy = 0;
     }
 }
 
@@ -173,6 +174,7 @@ static __global__ __launch_bounds__(256) void k_stage_in(const uint32_t* __restr
             status->n_members = 0;
             status->n_big = 0;
             status->tile_share_q16 = 0;
+            status->heavy = 0;
         }
     }
 }

@@ -463,6 +463,7 @@ void harvest(SparseTable* t) {
         t->pull_pending = false;
         const HostStatus& h = *t->hpull;
         int N = t->pull_slots;
+        t->plan_heavy = h.st.heavy != 0;
         // the call booked room for every sign it could have inserted; keep what it did insert
         if (t->booked >= h.st.n_new) t->count_upper -= t->booked - h.st.n_new;
         t->booked = 0;
@@ -2371,7 +2372,7 @@ int push_op_impl(uint32_t table_handle, int N, const int64_t* const* values, con
         if (!pooled) return TN_OK;
         size_t max_len = 0;
         for (int s = 0; s < N; s++) max_len = std::max<size_t>(max_len, (size_t)value_lens[s]);
-        const PoolShare share{PoolShare::parts_log2((uint32_t)max_len)};
+        const PoolShare share((uint32_t)max_len, !reuse || !t->plan_has_show || t->plan_heavy);
         const uint32_t tiles = PoolShare::first_tile((uint32_t)N, (uint32_t)L);
         const uint32_t blocks = (PoolShare::first_part((uint32_t)N, (uint32_t)L) + XCDS - 1) / XCDS * XCDS;
         Carver c{nullptr};
@@ -2379,29 +2380,32 @@ int push_op_impl(uint32_t table_handle, int N, const int64_t* const* values, con
         uint16_t* poff;
         float *flat, *shares;
         uint64_t* has;
-        const bool spread = PoolShare::spread(share.lp_max) != 0;
+        uint32_t* extra;
+        const bool spread = share.spreads(share.lp_max);
         auto carve = [&](Carver& cv) {
             pool = cv.take<uint2>(L);
             poff = cv.take<uint16_t>((size_t)tiles * ((1u << share.lp_max) + 1));
             flat = cv.take<float>(L * (size_t)grad_dim);
-            shares = cv.take<float>(spread ? (size_t)blocks * POOL_SPREAD * grad_dim : 0);
-            has = cv.take<uint64_t>(spread ? blocks : 0);
+            shares = cv.take<float>(spread ? (size_t)blocks * POOL_SHARES * grad_dim : 0);
+            has = cv.take<uint64_t>(spread ? (size_t)blocks * (POOL_SHARES / 64) : 0);
+            extra = cv.take<uint32_t>(spread ? (size_t)N * (POOL_EXTRA + 1) : 0);
         };
         carve(c);
         TN_TRY(t->pooled_ws.ensure(align_up(c.off, 256)));
         Carver c2{(char*)t->pooled_ws.p};
         carve(c2);
+        if (spread) TN_LAUNCH(k_pool_frequent, dim3((uint32_t)N), dim3(POOL_THREADS), st, p.lbase, p.ubase, p.u_of_gi, share, extra);
         TN_LAUNCH_LDS(k_lookup_keys, dim3(tiles), dim3(256), pool_tile_lds(share.lp_max), st, pd, p.lbase, p.ubase, (uint32_t)N,
-                      p.u_of_gi, batch, pool, poff, share, ds);
+                      p.u_of_gi, batch, pool, poff, share, extra, ds);
 #define TN_REDUCE(LPG, ANY)                                                                                                \
     TN_LAUNCH((k_reduce_pooled<LPG, ANY>), dim3(blocks), dim3(POOL_THREADS), st, pd, p.lbase, p.ubase, (uint32_t)N, pool,  \
-              poff, grad_dim, t->store.D, combiner, ds, flat, share, shares, has)
+              poff, grad_dim, t->store.D, combiner, ds, flat, share, extra, shares, has)
         TN_POOL_LANES(TN_REDUCE, t->store.D, vec);
 #undef TN_REDUCE
         if (spread) {
 #define TN_REDUCE(LPG, ANY)                                                                                                \
     TN_LAUNCH((k_reduce_pooled_shares<LPG, ANY>), dim3((uint32_t)N * (POOL_SPREAD / 4)), dim3(256), st, p.lbase, p.ubase,  \
-              grad_dim, t->store.D, ds, shares, has, flat, share)
+              grad_dim, t->store.D, ds, shares, has, flat, share, extra)
             TN_POOL_LANES(TN_REDUCE, t->store.D, grad_dim % 4 == 0);
 #undef TN_REDUCE
         }

@@ -90,7 +90,7 @@ struct DevStatus {
     uint32_t n_big;      // groups with many records (handled one wavefront each)
     uint32_t abort;      // the call's inputs are unusable (flagged in err): later kernels of the call do nothing
     uint32_t tile_share_q16;  // remap through LDS: records handed to the first-level buckets per lookup, largest share of a slot, in 1 / 65536
-    uint32_t pad[1];
+    uint32_t heavy;  // remap through LDS: a slot has a sign with HEAVY_LOOKUPS lookups or more
 };
 // Lookups of a sign in its slot from which a push of pooled gradients deals them to several workgroups.
 constexpr uint32_t HEAVY_LOOKUPS = 1024;

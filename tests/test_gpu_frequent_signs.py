@@ -1,6 +1,7 @@
 """Pooled gradients of slots in which a few signs have most of the lookups: signs with as many lookups as are dealt to several
-workgroups and one fewer, as many of them as a slot can have, the only sign there is; rows of one and of several runs of sixteen
-elements.  Sums are exact in 32 bits in any order (test_gpu_pooled_edges.py says why)."""
+workgroups and one fewer, as many of them as a slot can have, the only sign there is, frequent signs behind many others and in
+one run, more of them than are dealt out; rows of one and of several runs of sixteen elements, on both paths.  Sums are exact in
+32 bits in any order (test_gpu_pooled_edges.py says why)."""
 import numpy as np
 import pytest
 
@@ -58,3 +59,34 @@ def test_small_batches(tn, oracle, dim, slots, n, counts, spread):
     assert spread == (most >= 1024 and n > 2048)
     assert any(k.startswith("k_small_pool") for k in names)
     assert any(k.startswith("k_small_pool_shares") for k in names) == spread
+
+
+@pytest.mark.parametrize("dim,lens", [(16, [6405, 1, 30002]), (20, [1603, 1596, 3206]), (64, [6405, 4004]), (4, [200004])])
+@pytest.mark.parametrize("kind", ["late", "late, several", "more than are dealt out", "in one run", "one sign", "none"])
+def test_large_batches(tn, oracle, dim, lens, kind):
+    rng = np.random.default_rng(dim * 7 + len(kind))
+    pair = Pair(tn, oracle, "AdaGrad", dim, HP, reserve=400000)
+    tn.core.set_sparse_table_small_batch_path(pair.h, False)
+    pool = synth.splitmix64(np.arange(1, 3002, dtype=np.uint64)).view(np.int64)
+    pair.populate(pool.view(np.uint64))
+    values = []
+    for n in lens:
+        v = pool[200 + rng.integers(0, 2800, n)]
+        if kind == "late":
+            v[rng.random(n) < 0.8] = pool[0]
+            v[:min(n, 100)] = pool[200:][:min(n, 100)]
+        elif kind == "late, several":
+            m = rng.random(n) < 0.7
+            v[m] = pool[rng.integers(0, 5, m.sum())]
+            v[:min(n, 100)] = pool[200:][:min(n, 100)]
+        elif kind == "more than are dealt out":  # (200 k lookups: 2 k of each)
+            v = pool[100 + rng.integers(0, 80, n)]
+            v[:min(n, 90)] = pool[200:][:min(n, 90)]
+        elif kind == "in one run":
+            v[n // 2:] = np.sort(pool[rng.integers(0, 4, n - n // 2)])
+        elif kind == "one sign":
+            v[:] = pool[0]
+        values.append(v)
+    names, most = step(tn, pair, rng, values, C.SUM if kind == "one sign" else C.MEAN)
+    spread = max(lens) > 6403 or most >= 1024  # (a slot of eight parts, or a heavy sign)
+    assert any(k.startswith("k_reduce_pooled_shares") for k in names) == ("k_pool_frequent" in names) == spread
