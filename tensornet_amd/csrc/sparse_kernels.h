@@ -2345,15 +2345,23 @@ struct BigSrc {
     }
 };
 
-// apply_big_wave's rounds in the general path's kernels: chunks of a quarter of the records, which fit the 80 registers of six
-// wavefronts a SIMD at D = 16 (8 to 16 bytes spilled at 32, 64) where 8 rounds take 123 and 16 take 150.  The other signs'
-// workgroups beside them wait for memory and want the wavefronts.  2.1 M lookups of 64 slots: 208.8 us a step with 4 rounds and
-// six wavefronts, 214.9 with 8 and four, 217 with 8 and six (88 bytes spilled) or 16 and four; 430 k pooled lookups of 211 slots,
-// signs of 211 records: 352.9, 352.1, 361.7, 364.
-// Rows of 4 and 8: two rounds, 32 and 16 records (four spill 17 and 13 registers, and the signs with few records, which are
-// the same kernel's, pay for it).  2.05 M lookups of 88 slots, 250 k signs, k_apply_all: rows of 4 46.5 us with four rounds,
-// 35.4 with two, rows of 8 45.4 and 38.9.
-constexpr int big_most(int D) { return D <= 8 ? 2 : 4; }
+// apply_big_wave's rounds in the general path's kernels.  More rounds a chunk are fewer chunks in a sign's chain and more
+// registers; the other signs' workgroups, beside them or in the same kernel, wait for memory and want the wavefronts.
+//
+// k_apply_all by rounds, median us, six wavefronts a SIMD unless it says otherwise, registers spilled in parentheses; 2.05 M
+// lookups of 88 slots over 250 k signs:
+//   rows of 4: one 34.8, two 35.5 (3), four 46.5 (17); of 8: two 38.1, four 44.8 (13); of 16: four 47.8 (2.1 M lookups of 64
+//   slots, a step: four 208.8, eight with four wavefronts 214.9, with six 217 (24))
+// rows of 32, 1.7 M of 211 slots over 10^8 ids: two 151, four 104.3 (4), eight with five 102.2; 600 k of 20 slots, few frequent
+// signs: four 26.7, eight with five 28.8
+// rows of 64, 860 k of 211 slots over 10^6 ids: two 206, four 122.5 (2), eight with six 136.5 (27), with five 91.0; over 10^8:
+// four 123.9, eight with five 110.0, with four 124.6; 600 k of 20 slots: 59.5, 63.0, 69.8
+constexpr int big_most(int D) { return D <= 8 ? 2 : D <= 32 ? 4 : 8; }
+constexpr int big_waves(int D) { return D == 64 ? 5 : 6; }
+// k_apply_big_adagrad, a kernel of its own, has room for more at six wavefronts a SIMD.  3.5 M lookups of 88 slots: rows of 4 two
+// rounds 30.6 us (2 registers spilled), four 29.6; of 8 two 33.5, four 35.7 (8), eight 31.9; of 32 four 57.5, eight 51.7; of 64
+// four 121.7 (and k_apply_single beside it 100), eight 86.3 (78).  Rows of 16: four 38.8, eight spill 5.
+constexpr int big_most_alone(int D) { return D == 4 || D == 16 ? 4 : 8; }
 
 // k_apply_big for AdaGrad rows of D elements, D a power of two from 4 to 64, on a plan whose big_desc lists {row, first member,
 // records, group} of every sign with many records (written by k_group_emit): one wavefront per sign, by apply_big_wave.  (Adam and
@@ -2362,7 +2370,7 @@ template <int D>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6, 8))) void k_apply_big_adagrad(
     Store s, OptDev o, PushSrc src, DevStatus* status, const uint4* __restrict__ big_desc, uint32_t desc_cap,
     const Member* __restrict__ list, const float* const* __restrict__ gaddr) {
-    __shared__ BigWave<OPT_ADAGRAD, D, big_most(D)> lds;
+    __shared__ BigWave<OPT_ADAGRAD, D, big_most_alone(D)> lds;
     const uint4 head = big_desc[blockIdx.x < desc_cap ? blockIdx.x : desc_cap - 1];  // (before the status is known)
     // a push launched on a plan that turned out not to be its batch's (the host redoes it), or whose inputs are unusable
     if (status->mismatch | status->abort) return;
@@ -2394,7 +2402,7 @@ struct ApplyAll {
 constexpr int ALL_GBUF = 1088;  // floats of gradient staging per wavefront at most: eight workgroups to a CU up to 64 elements
 
 template <int KIND, int LPG, bool ANY, int TILE>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6, 8))) void k_apply_all(Store s, OptDev o, PushSrc src,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(big_waves(TILE), 8))) void k_apply_all(Store s, OptDev o, PushSrc src,
                                                                                               DevStatus* status, ApplyAll a) {
     // a push launched on a plan that turned out not to be its batch's (the host redoes it), or whose inputs are unusable
     if (status->mismatch | status->abort) return;

@@ -1,7 +1,7 @@
 """Signs with many records -- one in most slots of the batch -- on the large-batch path, where a wavefront
-owns each of them: AdaGrad rows of every power-of-two dim from 4 to 64 (k_apply_big_adagrad<D>: its chunk is 64
-records for dims up to 16, 16 for 32 and 64, so 70 records are several chunks, the last one partial), a dim with
-its own general kernel (12), Adam; with the two cvm columns; all against the CPU oracle, record by record in slot
+owns each of them: AdaGrad rows of every power-of-two dim from 4 to 64 (apply_big_wave, in chunks of 8 to 64 records,
+so 70 records are several chunks, the last one partial; k_apply_all, and k_apply_big_adagrad<D> for batches of millions of
+lookups), a dim with its own general kernel (12), Adam; with the two cvm columns; all against the CPU oracle, record by record in slot
 order (core/kernels/sparse_table_ops.cc:336-367, core/ps/table/sparse_table.cc:68-83,
 core/ps/optimizer/ada_grad_kernel.cc:105-129): rows within 1e-5 relative / 1e-7 absolute, more than 99 % of them
 bit for bit."""
@@ -10,7 +10,7 @@ import pytest
 
 from tensornet_amd import synth
 
-from helpers import Pair, all_signs, check_pull
+from helpers import Pair, all_signs, check_pull, kernels_of
 
 pytestmark = pytest.mark.gpu
 
@@ -62,3 +62,23 @@ def test_signs_in_most_slots_on_the_large_batch_path(tn, oracle, opt, hyper, dim
         pair.push_op(values, grads, labels)
         # (with cvm a tenth or so of the columns is the logarithm column, which follows the libm in use)
         assert pair.assert_rows_match(all_signs(values)) > (0.9 if cvm else 0.99)
+
+
+@pytest.mark.parametrize("dim", [4, 8, 16, 32, 64])
+def test_signs_in_most_slots_of_millions_of_lookups(tn, oracle, dim):
+    """Signs with one record and with every number of records up to one in each of the 70 slots, 45 200 lookups a slot."""
+    rng = np.random.default_rng(dim)
+    pair = Pair(tn, oracle, "AdaGrad", dim, ADAGRAD_HP, reserve=100000, zero_init=True)
+    pool = synth.splitmix64(np.arange(1, 2001, dtype=np.uint64)).view(np.int64)
+    pair.populate(pool[:1500].view(np.uint64))
+    values = []
+    for s in range(SLOTS):
+        own = np.concatenate([pool[s:SLOTS], pool[SLOTS + s::SLOTS][:20], pool[200 + rng.integers(0, 1800, 100)]])
+        values.append(rng.permutation(np.concatenate([own, own[rng.integers(0, len(own), 45200 - len(own))]])))
+    for step in range(2):
+        counts = check_pull(pair, values)
+        grads = synth.make_grads(counts, pair.wf, 0.05, seed=step)
+        labels = [(rng.random(len(v)) < 0.3).astype(np.int64) for v in values]
+        names = kernels_of(tn, lambda: pair.push_op(values, grads, labels))
+        assert any(k.startswith("k_apply_big_adagrad") for k in names)
+        assert pair.assert_rows_match(all_signs(values)) > 0.99
