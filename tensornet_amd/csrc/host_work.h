@@ -5,8 +5,11 @@
 
 extern "C" {
 
-// The calling thread's next operator calls fn(arg) once, with its launches queued, before it waits for what they report; not at
-// all if it does not get there.  fn: nullptr takes it back.  fn must not throw, nor call this library.
+// The calling thread's next call that waits for the device -- a pull, of a batch or of the table, or a combine -- calls fn(arg)
+// once, with its launches queued, before it waits for what they report.  Other calls (a push, a pull that does not wait, one
+// that is refused) leave it for the next one.  fn: nullptr takes it back.
+// fn runs under the lock of the call's table: other threads' calls on that table wait for it.  It must not throw, nor call
+// this library, nor wait for a thread that may be in it.
 __attribute__((visibility("default"))) void tn_while_waiting(void (*fn)(void*), void* arg);
 }
 
