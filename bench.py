@@ -644,7 +644,7 @@ def main():
             "ms_per_step": cms,
             "keys_per_s": mean_L / (cms * 1e-3),
             "kernels_ms_per_step": {k: round(v, 4) for k, v in cprof.items()
-                                    if k.startswith(("k_combine", "k_lookup_keys", "k_reduce"))},
+                                    if k.startswith(("k_combine", "k_pool", "k_lookup_keys", "k_reduce"))},
             "kernels_frac_of_hbm_peak": {k: round(comb_bytes[k.split("<")[0]] / (v * 1e-3) / HBM_PEAK, 4)
                                          for k, v in cprof.items() if k.split("<")[0] in comb_bytes},
         }

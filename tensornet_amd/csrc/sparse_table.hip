@@ -55,9 +55,10 @@ constexpr size_t LDS_MIN_LOOKUPS = 1024;  // from here on the remap through LDS 
 //   128              81 / 132   104 / 135   120 / 152   133 / 151
 //   192             110 / 149   139 / 159   201 / 189   231 / 195
 //   254             148 / 167   220 / 182   275 / 226   339 / 242
-// Slots of more than 4096 lookups (k_small_slots_long; more than SMALL_SPLIT_SLOTS of them, tests/test_gpu_small.py pins 8 slots
-// of 4097 to the other path): 20 slots of 6000, AdaGrad rows of 16, 52 / 128 us, 40 of 8192, Ftrl rows of 1, 71 / 142,
-// 100 of 8000, Adam rows of 16, 138 / 171.
+// Slots of more than 4096 lookups (k_small_slots_long): 20 slots of 6000, AdaGrad rows of 16, 52 / 128 us, 40 of 8192, Ftrl rows
+// of 1, 71 / 142, 100 of 8000, Adam rows of 16, 138 / 171.  Up to SMALL_SPLIT_SLOTS of them stay with the other path, where
+// tests/test_gpu_small.py wants 3 and 8 slots of 4097.  They lose by it: AdaGrad rows of 16, one slot of 4097 to 8192 lookups
+// 32 to 37 us here and 92 to 96 there, two 34 to 40 and 95 to 113, four 35 to 43 and 100 to 115, eight 38 to 48 and 101 to 115.
 // They cross at 89 to 106 M slots x lookups (160 to 254 slots; rows of 64: 58 to 90, of 8 under Adam: 120; pulls alone: 115).
 // With pooled gradients, whose reduction is shorter here, at 180 M (192 slots, 700 k lookups: 1.08 times as fast, 254 and
 // 700 k: 1.02, 850 k: 0.96).  A pull does not know what push will follow: it goes by the table's last one.
@@ -79,8 +80,8 @@ constexpr uint32_t BIG_GROUP_DEFAULT = 16;
 // What a small pull has left to do behind its first launch takes one launch (k_small_pull_rest: 26 slots of 4096 lookups
 // 8.7 us, as two launches 7.0 + 7.2 and the gap), unless the buckets' workgroups want so much dynamic LDS, which all
 // workgroups of a launch are given, that fewer than four would be on a CU.  Up to SMALL_SPLIT_SLOTS slots it stays two
-// launches, the sequence tests/test_gpu_small.py pins at 8 slots: a step of 8 slots of 1024 lookups is as long as the host's
-// way from the pull's first launch to the push, 37 us either way.
+// launches, the sequence tests/test_gpu_small.py wants at 8 slots, which one would beat there, too: a step of 4 slots of 256
+// lookups 32.8 us as two launches, 32.0 as one, of 8 of 1024 36.3 and 34.4, of 8 of 4096 42.0 and 39.4.
 constexpr int SMALL_SPLIT_SLOTS = 8;  // (up to as many, slots are short, too: small_batch_shape)
 // Parts of rows from which a thread of small_finish takes two: up to here more workgroups are the shorter way.
 constexpr size_t FINISH_FULL = 1 << 17;

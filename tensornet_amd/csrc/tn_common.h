@@ -111,21 +111,6 @@ struct DieShare {
     }
 };
 
-// The same in runs of `run` items, dealt to the dies in turn, where the work of an item varies along the array:
-// `for (DieRuns r(n, run); r.more(); r.next()) ... r.item()` covers every item once, whatever the grid.
-struct DieRuns {
-    uint32_t n, run, dies, die, k, step;
-    // (block, blocks: the workgroup's number among those of the launch that do this work)
-    __device__ __forceinline__ DieRuns(uint32_t n_, uint32_t run_, uint32_t block, uint32_t blocks) : n(n_), run(run_) {
-        dies = min(XCDS, blocks), die = block % dies;
-        k = block / dies;
-        step = (blocks - die + dies - 1) / dies;
-    }
-    __device__ __forceinline__ uint32_t item() const { return (k / run * dies + die) * run + k % run; }
-    __device__ __forceinline__ bool more() const { return item() < n; }  // (items ascend with k)
-    __device__ __forceinline__ void next() { k += step; }
-};
-
 __device__ __forceinline__ uint64_t mix64(uint64_t x) {
     x ^= x >> 33;
     x *= 0xff51afd7ed558ccdull;

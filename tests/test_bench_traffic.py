@@ -13,8 +13,7 @@ import bench  # noqa: E402
 
 SHAPE = dict(L=5000000, U=2000000, G=1080000, G1=917000, Rm=550000, Gm=149000, Rb=548000, Gb=13500, T=2940000)
 # side measurements of bench.py (combiner, ShowDecay, dense): profiled in the same runs, not part of the step
-SIDE = ("k_show_decay", "k_reduce_pooled", "k_combine_fwd", "k_lookup_keys", "k_place_lookups", "k_order_segments",
-        "k_report", "k_dense_adam_v4", "k_dense_adagrad_v4", "k_probe", "k_load_rows", "k_export_rows", "k_finish_insert",
+SIDE = ("k_show_decay", "k_pool_frequent", "k_reduce_pooled", "k_combine_fwd", "k_lookup_keys", "k_report", "k_dense_adam_v4", "k_dense_adagrad_v4", "k_probe", "k_load_rows", "k_export_rows", "k_finish_insert",
         "k_reset_status", "k_fill_f32")
 
 
