@@ -113,6 +113,13 @@ def kernel_algorithmic_bytes(name, opt, dim, shape):
         "k_apply_big_adagrad": apply_bytes(shape["Rb"], shape["Gb"]),
         "k_apply_scalar": apply_bytes(U, G),
         "k_apply_all": apply_bytes(U, G),
+        # the path of few launches
+        "k_small_slots": 18 * L + 24 * U,      # signs in, their copy and first positions out; a stored-key compare, record and
+        "k_small_slots_long": 18 * L + 24 * U, # row of every distinct sign
+        "k_small_group_finish": 10 * L + U * (2 * row + 4),       # first position in, mapped id out; rows into the variables
+        "k_small_pull_rest": 10 * L + U * (2 * row + 4) + 24 * U, # the same; the records in, by sign out
+        "k_small_verify": 26 * L,              # signs, their copy, labels, first positions
+        "k_small_apply": apply_bytes(U, G),
     }
     return table.get(name.split("<")[0], 0)
 

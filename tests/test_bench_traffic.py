@@ -40,3 +40,14 @@ def test_a_kernel_without_a_figure_is_refused():
     with pytest.raises(SystemExit) as e:
         bench.measured_traffic(["k_tile_dedup", "k_some_new_kernel<4>"])
     assert "k_some_new_kernel" in str(e.value)
+
+
+@pytest.mark.parametrize("step", [
+    ["k_small_slots", "k_small_group_finish<4>", "k_group_emit<true>", "k_small_verify<true>", "k_small_apply<KIND, LPG, ANY, BIG>"],
+    ["k_small_slots", "k_small_pull_rest<4>", "k_small_verify<false>", "k_small_apply<KIND, LPG, ANY, BIG>"],
+    ["k_small_slots_long", "k_small_pull_rest<1>", "k_small_verify<true>", "k_small_apply<KIND, LPG, ANY, BIG>"]])
+def test_the_small_path_has_a_dominant_kernel(step):
+    """`bench.py --config cfg1 / cfg2` price their dominant kernel: one with algorithmic bytes is there, whichever launches the
+    batch takes."""
+    for k in step:
+        assert bench.kernel_algorithmic_bytes(k, "Adam", 16, SHAPE) > 0
