@@ -8,10 +8,10 @@
 //             d(n) = 1 (sum), n (mean), sqrt(n) (sqrtn); an example without lookups gives zeros
 //   backward  g[u, :]   = sum over the lookups i of distinct sign u of dout[b(i), :] * (1 / d(n_b(i)))
 //
-// Both are deterministic.  The forward sums run in occurrence order, and so do the backward
-// sums of the signs with few lookups; a sign with many is summed in pieces of POOL_PIECE (16), whose
-// sums are added in order, one with lookups in several rounds of a workgroup round by round
-// (k_reduce_pooled; on the path of few launches k_small_pool).
+// Both are deterministic.  The forward sums run in occurrence order.  So do the backward sums, but cut up: a workgroup's
+// lookups, in the order of their signs, every POOL_PIECE (16) places; what a sign has in several pieces is added in order,
+// what it has in several rounds of a workgroup round by round, what a frequent one has in several workgroups by halves
+// (k_reduce_pooled, on the path of few launches k_small_pool; add_shares).
 #ifndef TN_COMBINE_KERNELS_H_
 #define TN_COMBINE_KERNELS_H_
 
@@ -162,8 +162,8 @@ constexpr uint32_t POOL_SPREAD_LOG2 = 3, POOL_SPREAD_LOG2_HEAVY = 1;
 // run by run (64 lookups), and every part leaves a share of those signs' sums (k_reduce_pooled_shares adds them up): a sign
 // with 8 % of a slot's lookups would be three rounds of one part, and the last workgroup's.  So are those of up to POOL_EXTRA
 // further ones with half as many lookups as a part or more (k_pool_frequent).  The other indices are
-// dealt modulo 2^lp.  Tiles and parts of a call are numbered through the slots so that a slot's
-// first is known from the lookups before it; some numbers are nobody's.
+// dealt modulo 2^lp.  Tiles and parts of a call are numbered through the slots so that a slot's first is known from the
+// lookups before it; some numbers are nobody's.
 struct PoolShare {
     uint32_t lp_max;  // of the longest slot
     uint32_t spread_log2;
@@ -188,8 +188,9 @@ struct PoolShare {
 // Which signs of a slot that has spread ones are frequent although they come late -- behind the first distinct ones, or where
 // the lookups are grouped: `extra`, per slot the number of them, then their indices.  Left to one part such a sign is a chain
 // of rounds: 100 slots of 49 k lookups, 80 % of them a sign that comes 101st, k_reduce_pooled 632 us, so 155; a step of one
-// slot of a million 9.2 ms, so 0.27.  The counts of a sample decide: 128 runs of sixteen lookups (in a short slot fewer) at places that are even but for a
-// jitter (positions with a period would all look alike).  A workgroup per slot; what is chosen depends on the lookups alone, not on the order of atomics.
+// slot of a million 9.2 ms, so 0.27.  The counts of a sample decide: 128 runs of sixteen lookups (in a short slot fewer) at
+// places that are even but for a jitter (positions with a period would all look alike).  A workgroup per slot, a chain of one
+// round trip and LDS: 6.7 us for 100 slots of 49 k.  What is chosen depends on the lookups alone, not on the order of atomics.
 constexpr uint32_t FREQUENT_RUN = 16, FREQUENT_SAMPLES = 2048, FREQUENT_TABLE = 4096;
 constexpr uint32_t FREQUENT_LEAST = 8;  // of the sample, however long the slot: fewer are chance
 constexpr uint32_t FREQUENT_LISTED = FREQUENT_SAMPLES / FREQUENT_LEAST;

@@ -9,7 +9,8 @@
 //                                (sparse_table_ops.cc:244-265); beside it, per bucket: the groups of equal signs over all
 //                                slots, their records in slot order
 //   push  k_small_verify         comparison with the plan's signs, click sums; beside it the ranks into the records
-//         k_small_pool           (pooled gradients) the gradient of every distinct sign from those of its examples
+//         k_small_pool           (pooled gradients) the gradient of every distinct sign from those of its examples; with
+//                                heavy signs k_small_pool_shares, which adds up what a slot's workgroups have of them
 //         k_small_apply          per bucket: every sign's records in order (tells the host that the comparison is complete)
 //
 // Workgroups of one launch never wait for each other, and none needs another's results: what needs them runs in the

@@ -2,9 +2,9 @@
 embedding_lookup_sparse on the pulled rows; backward: push fed with pooled
 gradients, reduced per distinct sign on the device) against oracle/combine.py
 and the table oracle, through the C ABI.  Tolerance 1e-5 relative / 1e-7
-absolute (sums run in the same order on both sides but for signs with more than
-32 lookups in a slot, whose partial sums are associated differently; the scale
-factors may differ in the last bit)."""
+absolute (both sides add the same terms, the kernels in pieces and shares of a
+fixed order, i.e. associated differently; the scale factors may differ in the
+last bit)."""
 import numpy as np
 import pytest
 import torch
