@@ -16,8 +16,8 @@ void launch_small_apply(const SmallApplyCall& c) {
     const bool lds_big = c.with_big && (s.D > 64 || (s.D & (s.D - 1)) != 0);  // (others keep their staging in static LDS)
     const size_t lds = small_apply_slots_lds(c.flat ? 0 : b.N) + (lds_big ? 4 * wave_lds : 0);
 #define TN_LAUNCH_SMALL_BIG(LPG, ANY, BIG)                                                                               \
-    TN_LAUNCH_LDS((k_small_apply<KIND, LPG, ANY, BIG>), dim3(b.buckets()), dim3(256), lds, c.st, b, c.p, c.flat, s, c.o, \
-                  c.status, c.host_seq, c.seq, c.dim, gfloats, (uint32_t)wave_lds, (uint32_t)arrays)
+    TN_LAUNCH_LDS_EVENT(c.done, (k_small_apply<KIND, LPG, ANY, BIG>), dim3(b.buckets()), dim3(256), lds, c.st, b, c.p,   \
+                        c.flat, s, c.o, c.status, c.host_seq, c.seq, c.dim, gfloats, (uint32_t)wave_lds, (uint32_t)arrays)
 // (aligned rows that fill their lanes have 4, 8 .. 128 elements; of these the last are too long for apply_big_wave)
 #define TN_LAUNCH_SMALL_ROWS(LPG)                                                 \
     do {                                                                          \

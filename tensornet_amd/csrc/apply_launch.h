@@ -34,6 +34,7 @@ struct SmallApplyCall {
     RowShare share;
     bool with_big;  // the plan lists signs with many records
     hipStream_t st;
+    hipEvent_t done;
 };
 template <int KIND>
 void launch_small_apply(const SmallApplyCall& c);

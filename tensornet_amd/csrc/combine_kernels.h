@@ -274,12 +274,14 @@ static __global__ __launch_bounds__(256) void k_lookup_keys(const SlotDesc* __re
                                                      const uint32_t* __restrict__ ubase, uint32_t N,
                                                      const uint32_t* __restrict__ u_of_gi, int64_t batch,
                                                      uint2* __restrict__ pool, uint16_t* __restrict__ poff, PoolShare share,
-                                                     const uint32_t* __restrict__ extra, DevStatus* status) {
+                                                     const uint32_t* __restrict__ extra, DevStatus* status,
+                                                     HostWord compared) {
     extern __shared__ uint32_t cnt[];  // [2^lp][KEY_WAVES]
     __shared__ uint32_t more[POOL_EXTRA];
     __shared__ uint32_t wsum[KEY_WAVES];
     __shared__ uint32_t slot;
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    compared.tell();
     if (tid == 0) slot = N;
     __syncthreads();
     for (uint32_t s = tid; s < N; s += 256) {

@@ -101,6 +101,11 @@ void prof_end(hipStream_t st) {
     if (!g_prof_recs.empty()) (void)hipEventRecord(g_prof_recs.back().b, st);
 }
 
+bool records_events(hipStream_t st) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(st, &status) != hipSuccess || status != hipStreamCaptureStatusNone;
+}
+
 void DevBuf::release() {
     if (p) (void)hipFree(p);
     p = nullptr;

@@ -939,6 +939,16 @@ static __global__ __launch_bounds__(256) void k_count_show(const SlotDesc* __res
     }
 }
 
+// A word in pinned memory that tells the host a kernel has come this far (nullptr: none): what ran ahead of the kernel is
+// complete.
+struct HostWord {
+    uint32_t* word;
+    uint32_t seq;
+    __device__ __forceinline__ void tell() const {
+        if (word && blockIdx.x == 0 && threadIdx.x == 0) __hip_atomic_store(word, seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+};
+
 // ------------------------------------------------------------ push grouping
 // Where the sign / gradient / counts of record u of a push come from.
 struct PushSrc {
@@ -953,6 +963,8 @@ struct PushSrc {
     int dim;
     // op-level push of pooled gradients: one reduced gradient row per distinct sign, record order
     const float* flat;
+    // op-level push on the last pull's plan: the comparison of its signs, ahead of the update kernels, is complete
+    HostWord compared;
 };
 
 __device__ __forceinline__ uint64_t src_sign(const PushSrc& p, uint32_t u) {
@@ -1609,6 +1621,7 @@ template <int KIND, int LPG, bool ANY>
 __global__ __launch_bounds__(256) void k_apply_single(Store s, OptDev o, PushSrc src, DevStatus* status,
                                                       const uint32_t* __restrict__ grp_row,
                                                       const Member* __restrict__ list) {
+    src.compared.tell();
     // a push launched on a plan that turned out not to be its batch's (the host redoes it), or whose inputs are unusable
     if (status->mismatch | status->abort) return;
     apply_singles<KIND, LPG, ANY>(s, o, src, status, grp_row, list, blockIdx.x, gridDim.x);
@@ -1746,6 +1759,7 @@ __global__ __launch_bounds__(256) void k_apply_vec(Store s, OptDev o, PushSrc sr
                                                    const uint32_t* __restrict__ grp_cnt,
                                                    const Member* __restrict__ list, uint32_t big_k,
                                                    uint32_t ids_cap, const float* const* __restrict__ gaddr) {
+    src.compared.tell();
     // a push launched on a plan that turned out not to be its batch's (the host redoes it), or whose inputs are unusable
     if (status->mismatch | status->abort) return;
     apply_multis<KIND, LPG, ANY>(s, o, src, status, grp_row, grp_off, grp_cnt, list, big_k, ids_cap, gaddr, blockIdx.x,
@@ -2014,6 +2028,7 @@ __global__ __launch_bounds__(64) void k_apply_big(Store s, OptDev o, PushSrc src
     extern __shared__ float gbuf[];  // gbuf_floats floats of staging, then the row: rw[D], ra[D], rb[D]
     __shared__ const float* gptr[BIG_CHUNK];
     __shared__ float den[BIG_CHUNK];
+    src.compared.tell();
     // a push launched on a plan that turned out not to be its batch's (the host redoes it), or whose inputs are unusable
     if (status->mismatch | status->abort) return;
     apply_big_groups<KIND>(
@@ -2372,6 +2387,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6, 8))) void
     const Member* __restrict__ list, const float* const* __restrict__ gaddr) {
     __shared__ BigWave<OPT_ADAGRAD, D, big_most_alone(D)> lds;
     const uint4 head = big_desc[blockIdx.x < desc_cap ? blockIdx.x : desc_cap - 1];  // (before the status is known)
+    src.compared.tell();
     // a push launched on a plan that turned out not to be its batch's (the host redoes it), or whose inputs are unusable
     if (status->mismatch | status->abort) return;
     const BigSrc from{src, list, gaddr};
@@ -2404,6 +2420,7 @@ constexpr int ALL_GBUF = 1088;  // floats of gradient staging per wavefront at m
 template <int KIND, int LPG, bool ANY, int TILE>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(big_waves(TILE), 8))) void k_apply_all(Store s, OptDev o, PushSrc src,
                                                                                               DevStatus* status, ApplyAll a) {
+    src.compared.tell();
     // a push launched on a plan that turned out not to be its batch's (the host redoes it), or whose inputs are unusable
     if (status->mismatch | status->abort) return;
     if (blockIdx.x < a.big_blocks) {
@@ -2454,6 +2471,7 @@ __global__ __launch_bounds__(256) void k_apply_scalar(Store s, OptDev o, PushSrc
                                                       const uint32_t* __restrict__ grp_cnt,
                                                       const Member* __restrict__ list, uint32_t big_k,
                                                       uint32_t ids_cap) {
+    src.compared.tell();
     // a push launched on a plan that turned out not to be its batch's (the host redoes it), or whose inputs are unusable
     if (status->mismatch | status->abort) return;
     const uint32_t n_single = status->n_single, n_multi = status->n_multi;

@@ -12,6 +12,7 @@
 #include <atomic>
 #include <chrono>
 #include <cstring>
+#include <thread>
 
 // Device memory of tn_sparse_table_pull_static, the one entry point that allocates nothing: the call's
 // status block, then the row number and the new-row list of every requested sign.  Every GPU the library
@@ -126,7 +127,6 @@ struct SparseTable {
     char* hstage = nullptr;         // pinned staging of slot descriptors
     size_t hstage_bytes = 0;
     hipEvent_t stage_ev = nullptr;  // staging buffer free again
-    hipEvent_t verify_ev = nullptr; // a push's comparison of the signs has been published
     DevBuf comb_buf;                // slot descriptors of a combine op
     DevBuf pooled_ws;               // scratch of a push of pooled gradients (items of the lookups, reduced rows)
     // The path of few launches for small batches: the words in pinned memory its kernels report through (hwords: one
@@ -176,9 +176,9 @@ struct SparseTable {
     hipStream_t flow_stream = nullptr;
     bool push_pub_on_side = false;  // the pending push's status is published on the side stream
     // A pull whose status is final before its last kernel (the gather) publishes it on the side stream
-    // meanwhile and returns when it is there: ready_ev = the status can be published, pub_ev = it is on
-    // the host, tail_ev = the gather is done (what a call on another stream has to wait for).
-    hipEvent_t ready_ev = nullptr, pub_ev = nullptr, tail_ev = nullptr;
+    // meanwhile and returns when it is there: ready_ev = the status can be published,
+    // tail_ev = the gather is done (what a call on another stream has to wait for).
+    hipEvent_t ready_ev = nullptr, tail_ev = nullptr;
     bool tail_recorded = false;
     bool one_stream = false;        // the running call is small: its kernels all go to the caller's stream
     bool plan_clicks_dirty = false;  // a push has added clicks to the member lists of the current plan
@@ -191,7 +191,9 @@ struct SparseTable {
     // whose room is fixed, with the same fallback as above.
     double tile_est = 1.0;
     uint64_t pull_lookups = 0;  // lookups of the pull whose status is pending
-    bool stage_pending = false;
+    // The staging buffer is being read by a call that has not waited for that: stage_ev has been recorded behind it, or
+    // (a call that was to wait and failed before) not.
+    bool stage_pending = false, stage_recorded = false;
     bool push_pending = false;      // hpush holds an unchecked status
     bool pull_pending = false;
     int pull_slots = 0, push_slots = 0;  // N of the pending calls
@@ -337,12 +339,10 @@ int ensure_side_buffers(SparseTable* t) {
     t->hstage_bytes = (size_t)MAX_SLOTS * sizeof(SlotDesc) + (MAX_SLOTS + 1) * sizeof(uint32_t);
     TN_HIP(hipHostMalloc((void**)&t->hstage, t->hstage_bytes, hipHostMallocDefault));
     TN_HIP(hipEventCreateWithFlags(&t->stage_ev, hipEventDisableTiming));
-    TN_HIP(hipEventCreateWithFlags(&t->verify_ev, hipEventDisableTiming));
     TN_HIP(hipEventCreateWithFlags(&t->fork_ev, hipEventDisableTiming));
     TN_HIP(hipEventCreateWithFlags(&t->join_ev, hipEventDisableTiming));
     TN_HIP(hipEventCreateWithFlags(&t->join2_ev, hipEventDisableTiming));
     TN_HIP(hipEventCreateWithFlags(&t->ready_ev, hipEventDisableTiming));
-    TN_HIP(hipEventCreateWithFlags(&t->pub_ev, hipEventDisableTiming));
     TN_HIP(hipEventCreateWithFlags(&t->tail_ev, hipEventDisableTiming));
     TN_HIP(hipEventCreateWithFlags(&t->apply_ev, hipEventDisableTiming));
     TN_HIP(hipEventCreateWithFlags(&t->upd_ev, hipEventDisableTiming));
@@ -795,25 +795,32 @@ int stage_slots(SparseTable* t, int N, const int64_t* const* values, const int64
     return TN_OK;
 }
 
+// The staging buffer may be written again.
+int staging_free(SparseTable* t) {
+    if (t->stage_pending) TN_HIP(t->stage_recorded ? hipEventSynchronize(t->stage_ev) : hipDeviceSynchronize());
+    t->stage_pending = false;
+    return TN_OK;
+}
+
 // Slot descriptors to the device (dst_descs; the slots' first lookups to dst_lbase unless nullptr); the same
 // launch prepares the call's status block `ds` (status_mode) and clears `zero[0 .. n_zero)`.  It runs on `run_on`.
+// waited: the caller waits for something behind it, and then says that the staging buffer is free; else an event says so.
+// joined: an event for other streams to wait for.
 int upload_slots(SparseTable* t, SlotDesc* dst_descs, uint32_t* dst_lbase, DevStatus* ds,
                  const std::vector<SlotDesc>& descs, const std::vector<uint32_t>& lbase, hipStream_t run_on,
-                 int status_mode, uint32_t* zero = nullptr, uint32_t n_zero = 0, const uint32_t* copy_src = nullptr,
-                 uint32_t* copy_dst = nullptr, uint32_t copy_n = 0) {
-    if (t->stage_pending) {
-        TN_HIP(hipEventSynchronize(t->stage_ev));
-        t->stage_pending = false;
-    }
+                 bool waited, hipEvent_t joined, int status_mode, uint32_t* zero = nullptr, uint32_t n_zero = 0,
+                 const uint32_t* copy_src = nullptr, uint32_t* copy_dst = nullptr, uint32_t copy_n = 0) {
+    TN_TRY(staging_free(t));
     const size_t db = descs.size() * sizeof(SlotDesc);
     const size_t lb = dst_lbase ? lbase.size() * sizeof(uint32_t) : 0;
     std::memcpy(t->hstage, descs.data(), db);
     if (lb) std::memcpy(t->hstage + db, lbase.data(), lb);
-    TN_LAUNCH(k_stage_in, dim3(launch_grid((int64_t)std::max<size_t>((db + lb) / 4, n_zero), 256, 64)), dim3(256),
-              run_on, reinterpret_cast<const uint32_t*>(t->hstage), reinterpret_cast<uint32_t*>(dst_descs),
-              (uint32_t)(db / 4), dst_lbase, (uint32_t)(lb / 4), ds, status_mode, zero, n_zero,
-              (const DevStatus*)t->dplan, copy_src, copy_dst, copy_n);
-    TN_HIP(hipEventRecord(t->stage_ev, run_on));
+    TN_LAUNCH_EVENT(joined, k_stage_in, dim3(launch_grid((int64_t)std::max<size_t>((db + lb) / 4, n_zero), 256, 64)),
+                    dim3(256), run_on, reinterpret_cast<const uint32_t*>(t->hstage), reinterpret_cast<uint32_t*>(dst_descs),
+                    (uint32_t)(db / 4), dst_lbase, (uint32_t)(lb / 4), ds, status_mode, zero, n_zero,
+                    (const DevStatus*)t->dplan, copy_src, copy_dst, copy_n);
+    if (!waited) TN_HIP(hipEventRecord(t->stage_ev, run_on));
+    t->stage_recorded = !waited;
     t->stage_pending = true;
     return TN_OK;
 }
@@ -885,8 +892,9 @@ int launch_build_plan(SparseTable* t, const Plan& p, const Scratch& w, int N, ui
         TN_LAUNCH_LDS(k_tile_dedup, dim3(tiles), dim3(TILE_THREADS), tile_lds, st, p.descs, p.lbase, N, L, w.bcursor, w.prec,
                       reinterpret_cast<ulonglong2*>(p.vals_copy), p.vals_exact, w.first_of, ds, w.span_cap);
         if (lds_groups)
-            TN_LAUNCH((k_lds_dedup<true>), dim3(launch_grid(w.nbuckets, 1, GRID_CAP * 2)), dim3(DEDUP_THREADS), st, w.bcursor,
-                      w.nbuckets, w.prec, w.first_of, w.cnt_at, ds, w.nb2, w.cursor2, w.recs);
+            TN_LAUNCH_EVENT(t->one_stream ? nullptr : t->fork_ev, (k_lds_dedup<true>), dim3(launch_grid(w.nbuckets, 1, GRID_CAP * 2)),
+                            dim3(DEDUP_THREADS), st, w.bcursor, w.nbuckets, w.prec, w.first_of, w.cnt_at, ds, w.nb2, w.cursor2,
+                            w.recs);
         else
             TN_LAUNCH((k_lds_dedup<false>), dim3(launch_grid(w.nbuckets, 1, GRID_CAP * 2)), dim3(DEDUP_THREADS), st, w.bcursor,
                       w.nbuckets, w.prec, w.first_of, w.cnt_at, ds, w.nb2, w.cursor2, w.recs);
@@ -896,29 +904,24 @@ int launch_build_plan(SparseTable* t, const Plan& p, const Scratch& w, int N, ui
             // against streaming kernels) and joins before the member lists are written.
             const int bblocks = launch_grid(w.nb2, 1, GRID_CAP * 4);
             hipStream_t sd = t->one_stream ? st : t->side, sd2 = t->one_stream ? st : t->side2;
-            if (!t->one_stream) {
-                TN_HIP(hipEventRecord(t->fork_ev, st));
-                TN_HIP(hipStreamWaitEvent(t->side, t->fork_ev, 0));
-            }
+            hipEvent_t joined = t->one_stream ? nullptr : t->join_ev, joined2 = t->one_stream ? nullptr : t->join2_ev;
+            if (!t->one_stream) TN_HIP(hipStreamWaitEvent(t->side, t->fork_ev, 0));
             if (N <= GRP_NARROW)
-                TN_LAUNCH((k_group_count<2>), dim3(bblocks), dim3(GRP_THREADS), sd, w.nb2, w.cursor2, w.recs,
-                          big_threshold(s), w.aux, w.bcounts);
+                TN_LAUNCH_EVENT(own_offsets ? joined : nullptr, (k_group_count<2>), dim3(bblocks), dim3(GRP_THREADS), sd, w.nb2,
+                                w.cursor2, w.recs, big_threshold(s), w.aux, w.bcounts);
             else
-                TN_LAUNCH((k_group_count<4>), dim3(bblocks), dim3(GRP_THREADS), sd, w.nb2, w.cursor2, w.recs,
-                          big_threshold(s), w.aux, w.bcounts);
-            if (!own_offsets) TN_LAUNCH(k_group_offsets, dim3(1), dim3(1024), sd, w.bcounts, w.bbase, w.nb2, ds);
-            if (!t->one_stream) {
-                TN_HIP(hipEventRecord(t->join_ev, t->side));
-                // ... and so do the rows of the records' signs, on a stream of their own
-                TN_HIP(hipStreamWaitEvent(t->side2, t->fork_ev, 0));
-            }
+                TN_LAUNCH_EVENT(own_offsets ? joined : nullptr, (k_group_count<4>), dim3(bblocks), dim3(GRP_THREADS), sd, w.nb2,
+                                w.cursor2, w.recs, big_threshold(s), w.aux, w.bcounts);
+            if (!own_offsets)
+                TN_LAUNCH_EVENT(joined, k_group_offsets, dim3(1), dim3(1024), sd, w.bcounts, w.bbase, w.nb2, ds);
+            // ... and so do the rows of the records' signs, on a stream of their own
+            if (!t->one_stream) TN_HIP(hipStreamWaitEvent(t->side2, t->fork_ev, 0));
             // few workgroups: enough probes in flight for the memory system, most of every CU left to the grouping
             TN_LAUNCH(k_probe_recs, dim3(std::min(bblocks, PROBE_RECS_GRID)), dim3(256), sd2, w.nb2, w.cursor2, w.recs, w.rrow,
                       w.newrec, w.newcnt, s, ds);
             const uint32_t init_parts = std::max<uint32_t>(1, (uint32_t)GRID_CAP / w.nb2);
-            TN_LAUNCH(k_init_new_recs, dim3(launch_grid((int64_t)w.nb2 * init_parts, 1, GRID_CAP)), dim3(256), sd2, s,
-                      make_optdev(t), t->seed, w.recs, w.rrow, w.nb2, w.newrec, w.newcnt, ds, init_parts);
-            if (!t->one_stream) TN_HIP(hipEventRecord(t->join2_ev, t->side2));
+            TN_LAUNCH_EVENT(joined2, k_init_new_recs, dim3(launch_grid((int64_t)w.nb2 * init_parts, 1, GRID_CAP)), dim3(256), sd2,
+                            s, make_optdev(t), t->seed, w.recs, w.rrow, w.nb2, w.newrec, w.newcnt, ds, init_parts);
         }
         TN_LAUNCH(k_lds_flags, dim3(w.ntiles), dim3(REMAP_THREADS), st, L, w.first_of, w.flag8, w.tilesum, p.descs, N,
                   w.bcursor, ds);
@@ -977,7 +980,7 @@ int launch_build_plan(SparseTable* t, const Plan& p, const Scratch& w, int N, ui
         ea.rrow = w.rrow;
         ea.grp_row = p.grp_row;
         ea.status = ds;
-        TN_LAUNCH((k_group_emit<false>), dim3(bblocks), dim3(EMIT_THREADS), st, ea);
+        TN_LAUNCH_EVENT(t->one_stream ? nullptr : t->ready_ev, (k_group_emit<false>), dim3(bblocks), dim3(EMIT_THREADS), st, ea);
         t->plan_big_desc = true;
         return TN_OK;  // the rows were found beside the grouping
     } else if (N <= MASK_SLOTS)
@@ -1009,7 +1012,7 @@ constexpr int ALL_BIG_GRID = 1024;
 template <int KIND>
 int launch_apply_kind(SparseTable* t, RowShare share, const Store& s, const OptDev& o, const PushSrc& src, DevStatus* ds,
                       const Plan& p, int64_t n_upper, hipStream_t st, bool addr_ready, uint32_t big_k, bool detach,
-                      bool big_desc) {
+                      bool big_desc, hipEvent_t behind) {
     const uint32_t ids_cap = (uint32_t)n_upper;
     const bool with_big = big_k != 0xFFFFFFFFu;
     const float* const* gaddr = (with_big && !src.infos && !src.flat) ? p.gaddr : nullptr;
@@ -1018,9 +1021,11 @@ int launch_apply_kind(SparseTable* t, RowShare share, const Store& s, const OptD
     const bool forked = (with_big || detach) && !t->one_stream;
     // op-level gradients: their addresses for the records of the groups with several records, once, in a
     // coalesced pass ahead of everything (beside k_apply_single it would take several times as long)
-    if (with_big && gaddr && !addr_ready)
-        TN_LAUNCH(k_member_grads, dim3(launch_grid(n_upper, 256, GRID_CAP * 2)), dim3(256), st, src, ds, p.list,
-                  p.gaddr, ids_cap);
+    if (with_big && gaddr && !addr_ready) {
+        behind = forked ? t->fork_ev : nullptr;
+        TN_LAUNCH_EVENT(behind, k_member_grads, dim3(launch_grid(n_upper, 256, GRID_CAP * 2)), dim3(256), st, src, ds, p.list,
+                        p.gaddr, ids_cap);
+    }
     if (with_big && t->one_stream && share.lanes != 0) {
         ApplyAll a;
         a.big_blocks = (uint32_t)launch_grid((n_upper / BIG_GROUP + 4) / 4, 1, ALL_BIG_GRID);
@@ -1065,10 +1070,17 @@ int launch_apply_kind(SparseTable* t, RowShare share, const Store& s, const OptD
         return TN_OK;
     }
     if (forked) {
-        TN_HIP(hipEventRecord(t->fork_ev, st));
-        TN_HIP(hipStreamWaitEvent(t->side, t->fork_ev, 0));
-        if (detach) TN_HIP(hipStreamWaitEvent(t->aux, t->fork_ev, 0));
+        if (!behind) {
+            behind = t->fork_ev;
+            TN_HIP(hipEventRecord(behind, st));
+        }
+        TN_HIP(hipStreamWaitEvent(t->side, behind, 0));
+        if (detach) TN_HIP(hipStreamWaitEvent(t->aux, behind, 0));
     }
+    // What the status of the push and the caller's stream wait for: the end of k_apply_single where that has a stream of its
+    // own, and of the last kernel on the caller's stream (detached: on the auxiliary and the side stream).
+    hipEvent_t single_done = detach ? t->apply_ev : forked ? t->join_ev : nullptr;
+    hipEvent_t last_done = detach || t->one_stream ? nullptr : t->apply_ev;
     if (with_big) {
         const int gfloats = big_gbuf_floats(s.D);
         const int big_blocks = launch_grid(n_upper / BIG_GROUP + 1, 1, 16384);
@@ -1090,11 +1102,11 @@ int launch_apply_kind(SparseTable* t, RowShare share, const Store& s, const OptD
     }
 #define TN_LAUNCH_VEC_ANY(LPG, ANY)                                                                                \
     do {                                                                                                          \
-        TN_LAUNCH((k_apply_single<KIND, LPG, ANY>), dim3(launch_grid(n_upper * LPG, 256, GRID_CAP * 4)), dim3(256), \
-                  detach ? t->aux : (forked ? t->side : st), s, o, src, ds, p.grp_row, p.list);                   \
-        TN_LAUNCH((k_apply_vec<KIND, LPG, ANY>), dim3(launch_grid(n_upper * LPG / 2, 256, GRID_CAP * 4)), dim3(256), \
-                  detach ? t->side : st, s, o, src, ds, p.grp_row, p.grp_off, p.grp_cnt, p.list, big_k, ids_cap,  \
-                  gaddr);                                                                                         \
+        TN_LAUNCH_EVENT(single_done, (k_apply_single<KIND, LPG, ANY>), dim3(launch_grid(n_upper * LPG, 256, GRID_CAP * 4)), \
+                        dim3(256), detach ? t->aux : (forked ? t->side : st), s, o, src, ds, p.grp_row, p.list);   \
+        TN_LAUNCH_EVENT(last_done, (k_apply_vec<KIND, LPG, ANY>), dim3(launch_grid(n_upper * LPG / 2, 256, GRID_CAP * 4)), \
+                        dim3(256), detach ? t->side : st, s, o, src, ds, p.grp_row, p.grp_off, p.grp_cnt, p.list,  \
+                        big_k, ids_cap, gaddr);                                                                    \
     } while (0)
 #define TN_LAUNCH_VEC(LPG)                        \
     do {                                          \
@@ -1111,15 +1123,13 @@ int launch_apply_kind(SparseTable* t, RowShare share, const Store& s, const OptD
         case 16: TN_LAUNCH_VEC(16); break;
         case 32: TN_LAUNCH_VEC(32); break;
         default:
-            TN_LAUNCH((k_apply_scalar<KIND>), dim3(launch_grid(n_upper, 256, GRID_CAP * 2)), dim3(256), st, s, o, src, ds,
-                      p.grp_row, p.grp_off, p.grp_cnt, p.list, big_k, ids_cap);
+            if (forked) TN_HIP(hipEventRecord(t->join_ev, t->side));  // (nothing of this push is there)
+            TN_LAUNCH_EVENT(last_done, (k_apply_scalar<KIND>), dim3(launch_grid(n_upper, 256, GRID_CAP * 2)), dim3(256), st, s, o,
+                            src, ds, p.grp_row, p.grp_off, p.grp_cnt, p.list, big_k, ids_cap);
     }
 #undef TN_LAUNCH_VEC
 #undef TN_LAUNCH_VEC_ANY
-    if (forked && !detach) {
-        TN_HIP(hipEventRecord(t->join_ev, t->side));
-        TN_HIP(hipStreamWaitEvent(st, t->join_ev, 0));
-    }
+    if (forked && !detach) TN_HIP(hipStreamWaitEvent(st, t->join_ev, 0));
     return TN_OK;
 }
 
@@ -1127,26 +1137,28 @@ int launch_apply_kind(SparseTable* t, RowShare share, const Store& s, const OptD
 // addr_ready: p.gaddr already holds the gradient addresses of the multi-record groups' records.
 // big_k: the number of records from which the plan's grouping listed a sign for k_apply_big (0: the table's default).
 // big_desc: p.big_desc describes the signs of p.big_list (the plan of a pull that grouped through LDS).
+// behind: an event that the last kernel on `st` signals, if it signals one.
 int launch_apply(SparseTable* t, const Plan& p, const PushSrc& src, DevStatus* ds, int64_t n_upper, bool vec_ok,
-                 hipStream_t st, bool addr_ready = false, uint32_t big_k = 0, bool detach = false, bool big_desc = false) {
+                 hipStream_t st, bool addr_ready = false, uint32_t big_k = 0, bool detach = false, bool big_desc = false,
+                 hipEvent_t behind = nullptr) {
     const Store& s = t->store;
     const OptDev o = make_optdev(t);
     const RowShare share = row_share(s, vec_ok);
     if (big_k == 0) big_k = big_threshold(s);
     switch (o.kind) {
-        case OPT_ADAGRAD: return launch_apply_kind<OPT_ADAGRAD>(t, share, s, o, src, ds, p, n_upper, st, addr_ready, big_k, detach, big_desc);
-        case OPT_ADAM: return launch_apply_kind<OPT_ADAM>(t, share, s, o, src, ds, p, n_upper, st, addr_ready, big_k, detach, big_desc);
-        default: return launch_apply_kind<OPT_FTRL>(t, share, s, o, src, ds, p, n_upper, st, addr_ready, big_k, detach, big_desc);
+        case OPT_ADAGRAD: return launch_apply_kind<OPT_ADAGRAD>(t, share, s, o, src, ds, p, n_upper, st, addr_ready, big_k, detach, big_desc, behind);
+        case OPT_ADAM: return launch_apply_kind<OPT_ADAM>(t, share, s, o, src, ds, p, n_upper, st, addr_ready, big_k, detach, big_desc, behind);
+        default: return launch_apply_kind<OPT_FTRL>(t, share, s, o, src, ds, p, n_upper, st, addr_ready, big_k, detach, big_desc, behind);
     }
 }
 
 // The updates of a small push, one launch (k_small_apply), with the signs with many records if the plan lists such.  flat: the
 // reduced rows of pooled gradients, else nullptr.
 void launch_small_apply(SparseTable* t, RowShare share, const SmallPlan& p, const float* flat, int dim, hipStream_t st,
-                        uint32_t* host_seq, uint32_t seq) {
+                        uint32_t* host_seq, uint32_t seq, hipEvent_t done) {
     const SmallShape& b = t->small_shape;
     const bool with_big = t->plan_big_k != 0xFFFFFFFFu && (uint32_t)b.N >= t->plan_big_k;
-    const SmallApplyCall c{b, p, flat, t->store, make_optdev(t), t->dplan, host_seq, seq, dim, share, with_big, st};
+    const SmallApplyCall c{b, p, flat, t->store, make_optdev(t), t->dplan, host_seq, seq, dim, share, with_big, st, done};
     switch (c.o.kind) {
         case OPT_ADAGRAD: return tn::launch_small_apply<OPT_ADAGRAD>(c);
         case OPT_ADAM: return tn::launch_small_apply<OPT_ADAM>(c);
@@ -1296,44 +1308,45 @@ void do_host_work() {
     }
 }
 
-// Waits for a kernel of the small path to report through pinned memory: *flag == want.  The word is polled for a
-// while (it arrives a few microseconds after the kernel's end, well before a wait on the stream or on an event
-// returns), then the stream is waited for, which also brings a failed launch to light.
+// Waits for kernels on `st` to report through pinned memory: there() looks whether they have.  It is polled for a
+// while (a word arrives a few microseconds after it is written, well before a wait on the stream or on an event
+// returns).  A caller's stream with much else to do ahead of the call is looked at now and then from there on: until the
+// report is there, whatever is queued behind it, or the stream has ended without, which also brings a failed launch to light.
+template <typename There>
+int wait_until(There there, hipStream_t st, const char* what) {
+    const auto t0 = std::chrono::steady_clock::now();
+    for (uint32_t spins = 1;; spins++) {
+        if (there()) break;
+        __builtin_ia32_pause();
+        if ((spins & 255u) || std::chrono::steady_clock::now() - t0 < std::chrono::milliseconds(2)) continue;
+        const hipError_t state = hipStreamQuery(st);
+        if (state == hipErrorNotReady) {
+            std::this_thread::sleep_for(std::chrono::microseconds(20));
+            continue;
+        }
+        TN_HIP(state);
+        if (!there()) return fail(TN_ERR_HIP, std::string(what) + ": the device did not report");
+        break;
+    }
+    std::atomic_thread_fence(std::memory_order_acquire);  // what the device wrote before the report is read after it
+    return TN_OK;
+}
 int wait_reported(const uint32_t* flag, uint32_t want, hipStream_t st, const char* what) {
     const volatile uint32_t* f = flag;
-    const auto t0 = std::chrono::steady_clock::now();
-    for (;;) {
-        for (int i = 0; i < 256; i++) {
-            if (*f == want) {
-                // what the device wrote before the word (the status block) is read after it
-                std::atomic_thread_fence(std::memory_order_acquire);
-                return TN_OK;
-            }
-            __builtin_ia32_pause();
-        }
-        if (std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(2)) break;
-    }
-    TN_HIP(hipStreamSynchronize(st));
-    if (*f != want) return fail(TN_ERR_HIP, std::string(what) + ": the device did not report");
-    std::atomic_thread_fence(std::memory_order_acquire);
-    return TN_OK;
+    return wait_until([&] { return *f == want; }, st, what);
 }
 
 // The same for the words of a small pull's first launch: hwords[0 .. n) all carry `seq`.
 int wait_words(const uint64_t* words, uint32_t n, uint32_t seq, hipStream_t st, const char* what) {
     do_host_work();
     const volatile uint64_t* w = words;
-    const auto t0 = std::chrono::steady_clock::now();
     uint32_t i = 0;
-    for (uint32_t spins = 0;; spins++) {
-        while (i < n && (uint32_t)(w[i] >> 32) == seq) i++;
-        if (i == n) return TN_OK;
-        __builtin_ia32_pause();
-        if ((spins & 255u) == 255u && std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(2)) break;
-    }
-    TN_HIP(hipStreamSynchronize(st));
-    while (i < n && (uint32_t)(w[i] >> 32) == seq) i++;
-    return i == n ? TN_OK : fail(TN_ERR_HIP, std::string(what) + ": the device did not report");
+    return wait_until(
+        [&] {
+            while (i < n && (uint32_t)(w[i] >> 32) == seq) i++;
+            return i == n;
+        },
+        st, what);
 }
 
 // SparseTablePull of a small batch laid out as `b` (the caller has validated the call and made room in the table).
@@ -1348,10 +1361,7 @@ int small_pull(SparseTable* t, const SmallShape& b, const int64_t* const* values
     TN_TRY(t->plan_buf.ensure(bytes));
     carve_small((char*)t->plan_buf.p, p, b);
     t->plan_valid = false;
-    if (t->stage_pending) {
-        TN_HIP(hipEventSynchronize(t->stage_ev));
-        t->stage_pending = false;
-    }
+    TN_TRY(staging_free(t));
     SlotDesc* descs = reinterpret_cast<SlotDesc*>(t->hstage);
     int width = row_width(wdim, s.wstride);
     uint32_t at = 0;
@@ -1386,7 +1396,8 @@ int small_pull(SparseTable* t, const SmallShape& b, const int64_t* const* values
     const uint32_t finish = (uint32_t)b.N * chunks;
     if (b.N > SMALL_SPLIT_SLOTS && emit_lds <= SMALL_SHARED_LDS) {
 #define TN_LAUNCH_REST(VEC)                                                                                              \
-    TN_LAUNCH_LDS((k_small_pull_rest<VEC>), dim3(b.buckets() + finish), dim3(FINISH_THREADS), emit_lds, st, ea, chunks, per, s)
+    TN_LAUNCH_LDS_EVENT(t->tail_ev, (k_small_pull_rest<VEC>), dim3(b.buckets() + finish), dim3(FINISH_THREADS), emit_lds, st, \
+                        ea, chunks, per, s)
         if (width == 4) TN_LAUNCH_REST(4);
         else if (width == 2) TN_LAUNCH_REST(2);
         else TN_LAUNCH_REST(1);
@@ -1398,11 +1409,10 @@ int small_pull(SparseTable* t, const SmallShape& b, const int64_t* const* values
         else if (width == 2) TN_LAUNCH_FINISH(2);
         else TN_LAUNCH_FINISH(1);
 #undef TN_LAUNCH_FINISH
-        TN_LAUNCH_LDS((k_group_emit<true>), dim3(b.buckets()), dim3(FINISH_THREADS), emit_lds, st, ea);
+        TN_LAUNCH_LDS_EVENT(t->tail_ev, (k_group_emit<true>), dim3(b.buckets()), dim3(FINISH_THREADS), emit_lds, st, ea);
     }
     TN_HIP(hipGetLastError());
     // the call returns when the first launch has reported: what follows is complete in stream order
-    TN_HIP(hipEventRecord(t->tail_ev, st));
     t->tail_recorded = true;
     t->small_shape = b;
     t->plan_valid = true;
@@ -1452,10 +1462,7 @@ int small_push(SparseTable* t, const int64_t* const* values, const float* const*
     carve_small((char*)t->plan_buf.p, p, b);
     SmallPool pool{};
     if (pooled) TN_TRY(small_pool_room(t, dim, pool));
-    if (t->stage_pending) {
-        TN_HIP(hipEventSynchronize(t->stage_ev));
-        t->stage_pending = false;
-    }
+    TN_TRY(staging_free(t));
     SlotDesc* descs = reinterpret_cast<SlotDesc*>(t->hstage);
     uint32_t at = 0;
     for (int i = 0; i < b.N; i++) {
@@ -1484,9 +1491,8 @@ int small_push(SparseTable* t, const int64_t* const* values, const float* const*
     const bool rows16 = dim % 4 == 0 && t->store.wstride % 4 == 0;
     if (pooled)
         launch_small_pool(t, vec, p, batch, dim, combiner, pool, st, &t->hpush->st.abort);
-    launch_small_apply(t, row_share(t->store, (pooled || vec) && rows16), p, pool.flat, dim, st, t->hseq + 1, seq);
-    // what a call on another stream has to wait for: the updates are still running when this call returns
-    TN_HIP(hipEventRecord(t->tail_ev, st));
+    // (tail_ev is what a call on another stream has to wait for: the updates are still running when this call returns)
+    launch_small_apply(t, row_share(t->store, (pooled || vec) && rows16), p, pool.flat, dim, st, t->hseq + 1, seq, t->tail_ev);
     t->tail_recorded = true;
     TN_HIP(hipGetLastError());
     // the outcome of the comparison: the updates are queued behind it and do nothing on a mismatch
@@ -2200,8 +2206,9 @@ int tn_sparse_table_pull_op(uint32_t table_handle, int N, const int64_t* const* 
         const bool hoist = behind_push && attempt == 0 && !t->one_stream && N == t->plan_N && !t->upd_pending;
         behind_push = false;
         if (hoist && t->tail_recorded) TN_HIP(hipStreamWaitEvent(t->aux, t->tail_ev, 0));  // the gather that read p.descs
-        TN_TRY(upload_slots(t, p.descs, p.lbase, t->dplan, descs, lbase, hoist ? t->aux : st, STATUS_NEW_PLAN,
-                            use_lds ? w.bcursor : nullptr, use_lds ? w.nbuckets + 1 + w.nb2 : 0));
+        TN_TRY(upload_slots(t, p.descs, p.lbase, t->dplan, descs, lbase, hoist ? t->aux : st, !t->async_pull,
+                            hoist ? t->stage_ev : nullptr, STATUS_NEW_PLAN, use_lds ? w.bcursor : nullptr,
+                            use_lds ? w.nbuckets + 1 + w.nb2 : 0));
         if (hoist) TN_HIP(hipStreamWaitEvent(st, t->stage_ev, 0));
 
         const Store& s = t->store;
@@ -2213,31 +2220,27 @@ int tn_sparse_table_pull_op(uint32_t table_handle, int N, const int64_t* const* 
         // variables are complete in stream order, as the outputs of any call that takes a stream.
         const bool final_early = use_lds && N <= GRP_SLOTS && !t->async_pull;
         const bool early = final_early && !t->one_stream;
-        // A call that keeps to the caller's stream publishes there, ahead of the gather, and tells the host through
+        // A call that keeps to the caller's stream publishes there, ahead of the gather.  Either tells the host through
         // a word in pinned memory: the host prepares the push while the gather runs.
         const bool early_inline = final_early && t->one_stream;
-        const uint32_t seq = early_inline ? ++t->seq_pull : 0;
+        const uint32_t seq = final_early ? ++t->seq_pull : 0;
         const uint32_t* rows_of_groups = (use_lds && N <= GRP_SLOTS) ? nullptr : p.grp_row;
-        if (early) TN_HIP(hipEventRecord(t->ready_ev, st));
         if (early_inline)
             TN_LAUNCH(k_publish, dim3(1), dim3(256), st, ds, p.ubase, (uint32_t)(N + 1),
                       reinterpret_cast<uint32_t*>(t->hpull), s.count, t->hseq + 0, seq);
+        hipEvent_t tail = early || early_inline ? t->tail_ev : nullptr;
         if (vec)
-            TN_LAUNCH((k_gather_vars<4>), dim3(launch_grid((int64_t)L * (wdim / 4), 256, GRID_CAP * 4)), dim3(256), st, s,
-                      ds, rows_of_groups, p.where_u, p.ubase, N, p.descs);
+            TN_LAUNCH_EVENT(tail, (k_gather_vars<4>), dim3(launch_grid((int64_t)L * (wdim / 4), 256, GRID_CAP * 4)), dim3(256),
+                            st, s, ds, rows_of_groups, p.where_u, p.ubase, N, p.descs);
         else
-            TN_LAUNCH((k_gather_vars<1>), dim3(launch_grid((int64_t)L * wdim, 256, GRID_CAP * 4)), dim3(256), st, s, ds,
-                      rows_of_groups, p.where_u, p.ubase, N, p.descs);
+            TN_LAUNCH_EVENT(tail, (k_gather_vars<1>), dim3(launch_grid((int64_t)L * wdim, 256, GRID_CAP * 4)), dim3(256), st, s,
+                            ds, rows_of_groups, p.where_u, p.ubase, N, p.descs);
         TN_HIP(hipGetLastError());
-        if (early || early_inline) {
-            TN_HIP(hipEventRecord(t->tail_ev, st));
-            t->tail_recorded = true;
-        }
-        if (early) TN_HIP(hipStreamWaitEvent(t->side, t->ready_ev, 0));
+        if (tail) t->tail_recorded = true;
+        if (early) TN_HIP(hipStreamWaitEvent(t->side, t->ready_ev, 0));  // (k_group_emit's end)
         if (!early_inline)
             TN_LAUNCH(k_publish, dim3(1), dim3(256), early ? t->side : st, ds, p.ubase, (uint32_t)(N + 1),
-                      reinterpret_cast<uint32_t*>(t->hpull), s.count, (uint32_t*)nullptr, 0u);
-        if (early) TN_HIP(hipEventRecord(t->pub_ev, t->side));
+                      reinterpret_cast<uint32_t*>(t->hpull), s.count, early ? t->hseq + 0 : nullptr, seq);
         t->pull_pending = true;
         t->pull_slots = N;
         t->pull_lookups = (uint64_t)L;
@@ -2253,12 +2256,11 @@ int tn_sparse_table_pull_op(uint32_t table_handle, int N, const int64_t* const* 
         t->plan_epoch = t->epoch;
         if (t->async_pull) return TN_OK;
         do_host_work();
-        if (early)
-            TN_HIP(hipEventSynchronize(t->pub_ev));
-        else if (early_inline)
-            TN_TRY(wait_reported(t->hseq + 0, seq, st, "SparseTablePull"));
+        if (final_early)
+            TN_TRY(wait_reported(t->hseq + 0, seq, early ? t->side : st, "SparseTablePull"));
         else
             TN_HIP(hipStreamSynchronize(st));
+        t->stage_pending = false;
         if (use_lds && (t->hpull->st.err & DEV_ERR_REMAP_OVERFLOW)) {
             // rows the failed attempt inserted belong to signs of this batch; keep them counted
             t->hpull->st.err &= ~DEV_ERR_REMAP_OVERFLOW;
@@ -2367,10 +2369,16 @@ int push_op_impl(uint32_t table_handle, int N, const int64_t* const* values, con
     // Where the apply kernels find the gradient of a record.  Pooled gradients are first reduced
     // to one row per distinct sign.
     PushSrc src{};
+    hipEvent_t behind = nullptr;  // what the last kernel ahead of the updates signals, if anything
+    uint32_t compared_seq = 0;    // with a plan of the last pull's: what the host waits for in hseq[1]
     const uint32_t* pub_ubase = nullptr;  // a push on the pull's plan publishes its own copy of the distinct counts
     auto prepare_src = [&]() -> int {
         src = op_source(p, grad_dim, pd == p.push_descs);
-        if (!pooled) return TN_OK;
+        const HostWord compared{reuse ? t->hseq + 1 : nullptr, compared_seq};
+        if (!pooled) {
+            src.compared = compared;
+            return TN_OK;
+        }
         size_t max_len = 0;
         for (int s = 0; s < N; s++) max_len = std::max<size_t>(max_len, (size_t)value_lens[s]);
         const PoolShare share((uint32_t)max_len, !reuse || !t->plan_has_show || t->plan_heavy);
@@ -2397,16 +2405,18 @@ int push_op_impl(uint32_t table_handle, int N, const int64_t* const* values, con
         carve(c2);
         if (spread) TN_LAUNCH(k_pool_frequent, dim3((uint32_t)N), dim3(POOL_THREADS), st, p.lbase, p.ubase, p.u_of_gi, share, extra);
         TN_LAUNCH_LDS(k_lookup_keys, dim3(tiles), dim3(256), pool_tile_lds(share.lp_max), st, pd, p.lbase, p.ubase, (uint32_t)N,
-                      p.u_of_gi, batch, pool, poff, share, extra, ds);
+                      p.u_of_gi, batch, pool, poff, share, extra, ds, compared);
+        behind = t->one_stream ? nullptr : t->fork_ev;
+        hipEvent_t reduced = spread ? nullptr : behind;
 #define TN_REDUCE(LPG, ANY)                                                                                                \
-    TN_LAUNCH((k_reduce_pooled<LPG, ANY>), dim3(blocks), dim3(POOL_THREADS), st, pd, p.lbase, p.ubase, (uint32_t)N, pool,  \
-              poff, grad_dim, t->store.D, combiner, ds, flat, share, extra, shares, has)
+    TN_LAUNCH_EVENT(reduced, (k_reduce_pooled<LPG, ANY>), dim3(blocks), dim3(POOL_THREADS), st, pd, p.lbase, p.ubase,      \
+                    (uint32_t)N, pool, poff, grad_dim, t->store.D, combiner, ds, flat, share, extra, shares, has)
         TN_POOL_LANES(TN_REDUCE, t->store.D, vec);
 #undef TN_REDUCE
         if (spread) {
 #define TN_REDUCE(LPG, ANY)                                                                                                \
-    TN_LAUNCH((k_reduce_pooled_shares<LPG, ANY>), dim3((uint32_t)N * (POOL_SPREAD / 4)), dim3(256), st, p.lbase, p.ubase,  \
-              grad_dim, t->store.D, ds, shares, has, flat, share, extra)
+    TN_LAUNCH_EVENT(behind, (k_reduce_pooled_shares<LPG, ANY>), dim3((uint32_t)N * (POOL_SPREAD / 4)), dim3(256), st,      \
+                    p.lbase, p.ubase, grad_dim, t->store.D, ds, shares, has, flat, share, extra)
             TN_POOL_LANES(TN_REDUCE, t->store.D, grad_dim % 4 == 0);
 #undef TN_REDUCE
         }
@@ -2426,8 +2436,8 @@ int push_op_impl(uint32_t table_handle, int N, const int64_t* const* values, con
         // that gather (the plan's counts are final from ready_ev on)
         const bool hoist = behind_pull && !t->one_stream;
         if (hoist) TN_HIP(hipStreamWaitEvent(t->aux, t->ready_ev, 0));
-        TN_TRY(upload_slots(t, p.push_descs, nullptr, ds, descs, lbase, hoist ? t->aux : st, STATUS_REUSE_PLAN, nullptr, 0,
-                            p.ubase, p.push_ubase, (uint32_t)(N + 1)));
+        TN_TRY(upload_slots(t, p.push_descs, nullptr, ds, descs, lbase, hoist ? t->aux : st, true, hoist ? t->stage_ev : nullptr,
+                            STATUS_REUSE_PLAN, nullptr, 0, p.ubase, p.push_ubase, (uint32_t)(N + 1)));
         pub_ubase = p.push_ubase;
         if (hoist) TN_HIP(hipStreamWaitEvent(st, t->stage_ev, 0));
         // On a plan with show counts the verify pass also sums the clicks; they start at zero
@@ -2435,7 +2445,10 @@ int push_op_impl(uint32_t table_handle, int N, const int64_t* const* values, con
         const bool clicks = t->plan_has_show && with_click;
         const int vblocks = launch_grid((int64_t)(L + VERIFY_TILE - 1) / VERIFY_TILE, 1, GRID_CAP * 2);
         const size_t vlds = ((size_t)N + 1) * sizeof(uint32_t);
-        // the outcome comes back through pinned host memory, written by the verify kernel itself
+        // the outcome comes back through pinned host memory, written by the verify kernel itself; that it has come, by a
+        // word from the kernels behind it
+        compared_seq = ++t->seq_verify;
+        behind = t->one_stream || pooled ? nullptr : t->fork_ev;
         t->hpush->st.mismatch = 0;
         uint32_t* host_mismatch = &t->hpush->st.mismatch;
         // op-level gradients (not pooled): the verify pass also works out the gradient addresses of the records
@@ -2445,8 +2458,8 @@ int push_op_impl(uint32_t table_handle, int N, const int64_t* const* values, con
         const float** vgaddr = addr_in_verify ? p.gaddr : nullptr;
         // (a macro: the profiler names a kernel by the text of its launch)
 #define TN_VERIFY(CLICKS, COPY)                                                                                      \
-    TN_LAUNCH_LDS((k_verify_values<CLICKS, COPY>), dim3(vblocks), dim3(256), vlds, st, pd, p.lbase, N, (uint32_t)L, \
-                  then_vals, ds, p.u_of_gi, p.where_u, p.list, host_mismatch, vsrc, vgaddr)
+    TN_LAUNCH_LDS_EVENT(behind, (k_verify_values<CLICKS, COPY>), dim3(vblocks), dim3(256), vlds, st, pd, p.lbase, N,  \
+                        (uint32_t)L, then_vals, ds, p.u_of_gi, p.where_u, p.list, host_mismatch, vsrc, vgaddr)
         const bool copy = !t->plan_prints || t->plan_exact;
         const uint64_t* then_vals = t->plan_exact ? p.vals_exact : p.vals_copy;
         if (clicks) {
@@ -2463,20 +2476,20 @@ int push_op_impl(uint32_t table_handle, int N, const int64_t* const* values, con
             TN_VERIFY(false, false);
         }
 #undef TN_VERIFY
-        TN_HIP(hipEventRecord(t->verify_ev, st));
         // Counts and apply kernels are queued before the host knows the outcome: the counts only
         // touch the plan's member lists, which a mismatch discards anyway, and the apply kernels
         // return at once when the mismatch flag is set.  The device never waits for the host.
-        if (!t->plan_has_show) TN_TRY(launch_counts());
+        if (!t->plan_has_show) {
+            TN_TRY(launch_counts());
+            behind = nullptr;
+        }
         TN_TRY(prepare_src());
         TN_TRY(launch_apply(t, p, src, ds, (int64_t)L, vec, st, addr_in_verify, t->plan_big_k,
-                            t->detach_updates && !pooled, t->plan_big_desc));
-        if (t->detached_now) {
-            // their end, for whoever touches the table next; the status goes out behind them (below)
-            TN_HIP(hipEventRecord(t->apply_ev, t->aux));
-            TN_HIP(hipStreamWaitEvent(t->side, t->apply_ev, 0));
-        }
-        TN_HIP(hipEventSynchronize(t->verify_ev));
+                            t->detach_updates && !pooled, t->plan_big_desc, behind));
+        // their end, for whoever touches the table next; the status goes out behind them (below)
+        if (t->detached_now) TN_HIP(hipStreamWaitEvent(t->side, t->apply_ev, 0));
+        TN_TRY(wait_reported(t->hseq + 1, compared_seq, t->detached_now ? t->side : st, "SparseTablePush"));
+        t->stage_pending = false;
         reuse = t->hpush->st.mismatch == 0;
         if (t->detached_now && !reuse) {
             // (the update kernels return at once on a mismatch; what follows works on the caller's stream)
@@ -2497,7 +2510,7 @@ int push_op_impl(uint32_t table_handle, int N, const int64_t* const* values, con
         pd = p.descs;
         TN_TRY(t->ws.ensure(carve_scratch(nullptr, w, L, dt_entries, false)));
         carve_scratch((char*)t->ws.p, w, L, dt_entries, false);
-        TN_TRY(upload_slots(t, p.descs, p.lbase, ds, descs, lbase, st, STATUS_NEW_PLAN));
+        TN_TRY(upload_slots(t, p.descs, p.lbase, ds, descs, lbase, st, false, nullptr, STATUS_NEW_PLAN));
         TN_TRY(launch_build_plan(t, p, w, N, (uint32_t)L, false, false, st));
         TN_TRY(launch_counts());
         TN_TRY(prepare_src());
@@ -2509,14 +2522,11 @@ int push_op_impl(uint32_t table_handle, int N, const int64_t* const* values, con
     const bool pub_on_side = reuse && !t->one_stream;
     const bool detached = reuse && t->detached_now;  // (the side stream is behind all update kernels already)
     t->detached_now = false;
-    if (pub_on_side && !detached) {
-        TN_HIP(hipEventRecord(t->apply_ev, st));
-        TN_HIP(hipStreamWaitEvent(t->side, t->apply_ev, 0));
-    }
-    TN_LAUNCH(k_publish, dim3(1), dim3(256), pub_on_side ? t->side : st, ds, pub_ubase ? pub_ubase : p.ubase,
-              (uint32_t)(N + 1), reinterpret_cast<uint32_t*>(t->hpush), (unsigned long long*)nullptr, (uint32_t*)nullptr, 0u);
+    if (pub_on_side && !detached) TN_HIP(hipStreamWaitEvent(t->side, t->apply_ev, 0));  // (k_apply_single is ahead on that stream)
+    TN_LAUNCH_EVENT(detached ? t->upd_ev : nullptr, k_publish, dim3(1), dim3(256), pub_on_side ? t->side : st, ds,
+                    pub_ubase ? pub_ubase : p.ubase, (uint32_t)(N + 1), reinterpret_cast<uint32_t*>(t->hpush),
+                    (unsigned long long*)nullptr, (uint32_t*)nullptr, 0u);
     if (detached) {
-        TN_HIP(hipEventRecord(t->upd_ev, t->side));
         t->upd_pending = true;
         t->upd_N = N;
         t->upd_groups_off = (size_t)((const char*)p.grp_sign - (const char*)t->plan_buf.p);
@@ -2593,10 +2603,7 @@ int tn_sparse_table_combine_op(uint32_t table_handle, int N, const int64_t* cons
         harvest(t);
     }
     set_last_stream(t, st);
-    if (t->stage_pending) {
-        TN_HIP(hipEventSynchronize(t->stage_ev));
-        t->stage_pending = false;
-    }
+    TN_TRY(staging_free(t));
     // A workgroup per COMBINE_EXAMPLES examples of a slot where that does not fill the chip several times over, else per
     // more of them: every workgroup pays for finding its lookups.
     uint32_t per = COMBINE_EXAMPLES;

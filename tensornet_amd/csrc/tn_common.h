@@ -3,6 +3,7 @@
 #ifndef TN_COMMON_H_
 #define TN_COMMON_H_
 
+#include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -206,6 +207,31 @@ void prof_end(hipStream_t st);
     } while (0)
 
 #define TN_LAUNCH(KERNEL, GRID, BLOCK, STREAM, ...) TN_LAUNCH_LDS(KERNEL, GRID, BLOCK, 0, STREAM, __VA_ARGS__)
+
+// A launch whose end is what `event` waits for (nullptr: an ordinary one).  The kernel's own completion is the event's signal; an
+// event recorded behind it is a packet of its own in the queue, which holds the next kernel up: kernels of 30 us one after the
+// other 30.5 us each, with an event recorded behind each 33.5, with the event as their signal 30.5; with a second stream that
+// waits for it 36.2 and 32.6.  (A stream that is being captured gets a recorded event, which a graph knows.)
+bool records_events(hipStream_t st);
+template <typename... P, typename... A>
+void launch_signalling(hipEvent_t event, void (*kernel)(P...), dim3 grid, dim3 block, size_t lds, hipStream_t st, A... args) {
+    if (event && !records_events(st)) {
+        hipExtLaunchKernelGGL(kernel, grid, block, (uint32_t)lds, st, nullptr, event, 0, args...);
+        return;
+    }
+    hipLaunchKernelGGL(kernel, grid, block, lds, st, args...);
+    if (event) (void)hipEventRecord(event, st);
+}
+
+#define TN_LAUNCH_LDS_EVENT(EVENT, KERNEL, GRID, BLOCK, LDS_BYTES, STREAM, ...)                  \
+    do {                                                                                        \
+        if (::tn::g_profile_on) ::tn::prof_begin(#KERNEL, STREAM);                              \
+        ::tn::launch_signalling(EVENT, KERNEL, GRID, BLOCK, LDS_BYTES, STREAM, __VA_ARGS__);    \
+        if (::tn::g_profile_on) ::tn::prof_end(STREAM);                                         \
+    } while (0)
+
+#define TN_LAUNCH_EVENT(EVENT, KERNEL, GRID, BLOCK, STREAM, ...) \
+    TN_LAUNCH_LDS_EVENT(EVENT, KERNEL, GRID, BLOCK, 0, STREAM, __VA_ARGS__)
 
 }  // namespace tn
 
