@@ -32,7 +32,7 @@ def log(msg):
 # profiles/cfg3_adagrad_dim16_pull_push.md (counters cannot be read from inside this script).
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "cfg3_traffic.json")
 # launched by a step, a few microseconds each, no traffic worth counting
-SMALL_STEP_KERNELS = ("k_stage_in", "k_publish", "k_init_new_recs", "k_group_offsets", "k_scan_tiles")
+SMALL_STEP_KERNELS = ("k_stage_in", "k_publish", "k_init_new_recs", "k_assign_init", "k_group_offsets", "k_scan_tiles")
 
 
 def measured_traffic(step_kernels):
@@ -64,9 +64,9 @@ def step_algorithmic_bytes(opt, dim, L, U):
     return 32 * L + U * (8 + 8 * dim + 4 * dim + 8 + 8 * dim + state_bytes(opt, dim))
 
 
-# Launched on the table's side streams, concurrently with kernels of the caller's stream (the other
-# update kernels; the ranking kernels of the remap).
-SIDE_STREAM_KERNELS = ("k_apply_single", "k_group_count", "k_group_offsets", "k_probe_recs")
+# Launched on the table's side stream, concurrently with kernels of the caller's stream (the other
+# update kernels).
+SIDE_STREAM_KERNELS = ("k_apply_single",)
 BIG_GROUP = 16  # records from which a sign is applied by k_apply_big (sparse_table.hip)
 
 
@@ -102,6 +102,9 @@ def kernel_algorithmic_bytes(name, opt, dim, shape):
         # table
         "k_probe": 8 * G + 4 * G,              # one stored-key compare per distinct sign, row number out
         "k_probe_recs": 8 * U + 8 * U + 4 * U, # the record's sign in, one stored-key compare, row number out
+        "k_group_probe": 24 * U + 20 * U + 4 * L,      # placement of the records, their probes, the lookups' flags
+        "k_assign_init": 4 * U,
+        "k_emit_mapped": 52 * U + 20 * G + 12 * L,     # member lists; mapped ids
         "k_gather_vars": U * (2 * row + 4),    # row read + variable row write
         # push
         # the op's signs and labels, against the pull's copy of the signs (COPY) or its fingerprints of them

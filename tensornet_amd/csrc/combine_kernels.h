@@ -275,7 +275,7 @@ static __global__ __launch_bounds__(256) void k_lookup_keys(const SlotDesc* __re
                                                      const uint32_t* __restrict__ u_of_gi, int64_t batch,
                                                      uint2* __restrict__ pool, uint16_t* __restrict__ poff, PoolShare share,
                                                      const uint32_t* __restrict__ extra, DevStatus* status,
-                                                     HostWord compared) {
+                                                     HostWord compared, uint32_t* host_err) {
     extern __shared__ uint32_t cnt[];  // [2^lp][KEY_WAVES]
     __shared__ uint32_t more[POOL_EXTRA];
     __shared__ uint32_t wsum[KEY_WAVES];
@@ -382,6 +382,7 @@ static __global__ __launch_bounds__(256) void k_lookup_keys(const SlotDesc* __re
     }
     if (bad) {
         atomicOr(&status->err, DEV_ERR_GRAD_ROWS);
+        if (host_err) *host_err = DEV_ERR_GRAD_ROWS;
         status->abort = 1;  // nothing downstream may run
     }
     __syncthreads();

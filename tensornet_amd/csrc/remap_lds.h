@@ -17,20 +17,23 @@
 //   k_tile_dedup   per tile of 2048 lookups: LDS hash table -> first position of every sign inside the tile,
 //                  one record per distinct sign of the tile handed to its bucket (+ fingerprints of the signs)
 //   k_lds_dedup    per bucket: LDS hash table -> first position in the slot, occurrence counts
-//   k_lds_flags    first-occurrence flags per tile (coalesced: first_of[gi] == gi)
-//   k_lds_assign   ranks, distinct lists, show counts; the tiles' offsets come from a sum over the
+//   tile_flags     first-occurrence flags per tile (coalesced: first_of[gi] == gi)
+//   assign_tile    ranks, distinct lists, show counts; the tiles' offsets come from a sum over the
 //                  counts of the tiles before (k_scan_tiles, shared with the global-table path,
 //                  only when there are too many tiles for that)
-//   k_lds_mapped   mapped ids and the per-lookup distinct index
+//   map_lookups    mapped ids and the per-lookup distinct index
 //
 // With at most GRP_SLOTS slots the groups of equal signs over all slots come out of
 // LDS too: k_lds_dedup hands every distinct (slot, sign) record -- sign, first
 // position, occurrences, slot -- to a second level of buckets chosen by the sign's
 // hash alone (fixed room per bucket, one global atomic per touched bucket), and
-// one workgroup per such bucket (k_group_count) finds the signs shared between
-// slots with an LDS table of slot masks; k_group_emit numbers the groups from the
+// one workgroup per such bucket (group_count_bucket) finds the signs shared between
+// slots with an LDS table of slot masks; emit_buckets numbers the groups from the
 // counts of the buckets before its own (summed by itself, or by the scan
 // k_group_offsets when there are too many buckets) and writes their member lists.
+// The grouping and the ranking do not need each other until then, so they share
+// launches: k_group_probe (counts, probes, flags), k_assign_init (ranks, new rows),
+// k_emit_mapped (member lists, mapped ids).
 //
 // If an LDS table ever overflows (more distinct signs in a bucket than it has
 // room for) DEV_ERR_REMAP_OVERFLOW is raised; every index written stays in
@@ -57,12 +60,14 @@ constexpr int LDS_SPAN2 = 512;          // second-level buckets whose counts one
 constexpr int GRP_TARGET = 1024;        // records per second-level bucket if every lookup were distinct
 constexpr int GRP_CAP = 1536;           // room of a second-level bucket
 constexpr int GRP_TABLE = 2048;         // entries of its LDS hash table (> GRP_CAP: an insert always ends)
-constexpr int GRP_THREADS = 512;        // threads of k_group_count
+constexpr int GRP_THREADS = 512;        // threads of k_group_probe
 constexpr int GRP_RECS = GRP_CAP / GRP_THREADS;  // records per thread of a second-level bucket's workgroup
 static_assert(GRP_CAP % GRP_THREADS == 0 && GRP_CAP % 256 == 0 && GRP_CAP < GRP_TABLE, "a bucket fits its table and the registers of one workgroup");
 constexpr int EMIT_THREADS = 512;
-constexpr int EMIT_RECS = GRP_CAP / EMIT_THREADS;  // records per thread of k_group_emit
-constexpr int GRP_ITEMS = (GRP_TABLE + 1 + GRP_THREADS - 1) / GRP_THREADS;
+constexpr int EMIT_RECS = GRP_CAP / EMIT_THREADS;  // records per thread of emit_buckets
+// (four-word masks: with 1792 entries two workgroups share a CU's LDS, with 2048 it holds one)
+constexpr int grp_table(int words) { return words == 2 ? GRP_TABLE : 1792; }
+static_assert(grp_table(4) > GRP_CAP, "an insert always ends");
 // A sign has a bit per slot in a mask of two words, or of four where there are more slots than that.  The masks of four
 // words take 85 KB of a CU's LDS (one workgroup instead of three), so the narrow ones stay; with as many slots a frequent
 // sign brings up to 255 records into its bucket, so the buckets are filled to half as much (Zipf 1.02 .. 1.3 over 10^5 ..
@@ -431,7 +436,7 @@ __global__ __launch_bounds__(DEDUP_THREADS) void k_lds_dedup(const uint32_t* __r
 }
 
 // Rank of the first occurrence at position gi = number of first occurrences before it: the
-// count up to its 64-lookup word (wordpre, written by k_lds_assign) plus the flags below it
+// count up to its 64-lookup word (wordpre, written by assign_tile) plus the flags below it
 // in the word.  Both arrays are small enough to stay in L2 (L / 8 and L / 16 bytes), so a
 // rank costs two cache hits instead of a random read of a 4-byte-per-lookup array.
 __device__ __forceinline__ uint32_t rank_of(const uint8_t* __restrict__ flag8, const uint32_t* __restrict__ wordpre,
@@ -444,26 +449,21 @@ __device__ __forceinline__ uint32_t rank_of(const uint8_t* __restrict__ flag8, c
 // what the first-level buckets of every slot were handed: status->tile_share_q16 = the largest share
 // records / lookups among the slots with more than one bucket's worth of lookups, in 1 / 65536 (the host sizes
 // the next call's buckets from it).
-static __global__ __launch_bounds__(REMAP_THREADS) void k_lds_flags(uint32_t L, const uint32_t* __restrict__ first_of,
-                                                             uint8_t* __restrict__ flag8,
-                                                             uint32_t* __restrict__ tilesum,
-                                                             const SlotDesc* __restrict__ descs, int N,
-                                                             const uint32_t* __restrict__ bcursor,
-                                                             DevStatus* status) {
-    __shared__ uint32_t red[4];
-    for (int sl = blockIdx.x; sl < N; sl += gridDim.x) {
-        const SlotDesc& d = descs[sl];
-        if (d.len <= (uint32_t)L1_ROOM) continue;  // (the same for the whole workgroup)
-        uint32_t mine = 0;
-        for (uint32_t b = threadIdx.x; b < d.tcap; b += REMAP_THREADS) mine += bcursor[d.tbase + b];
-        const uint32_t all = block_sum_256(mine, red);
-        if (threadIdx.x == 0) {
-            const uint64_t q = ((uint64_t)all << 16) / d.len + 1;
-            atomicMax(&status->tile_share_q16, (uint32_t)(q < 65536 ? q : 65536));
-        }
-        __syncthreads();
+// Both by wavefronts: a slot's share by one, a tile's flags by four (REMAP_THREADS lookups times eight; `tid` of them).
+__device__ __forceinline__ void slot_tile_share(const SlotDesc& d, const uint32_t* __restrict__ bcursor, DevStatus* status) {
+    if (d.len <= (uint32_t)L1_ROOM) return;
+    const uint32_t lane = (uint32_t)__lane_id();
+    uint32_t all = 0;
+    for (uint32_t b = lane; b < d.tcap; b += 64) all += bcursor[d.tbase + b];
+    for (int o = 32; o > 0; o >>= 1) all += __shfl_xor(all, o);
+    if (lane == 0) {
+        const uint64_t q = ((uint64_t)all << 16) / d.len + 1;
+        atomicMax(&status->tile_share_q16, (uint32_t)(q < 65536 ? q : 65536));
     }
-    const uint32_t base = blockIdx.x * REMAP_TILE + threadIdx.x * REMAP_ITEMS;
+}
+__device__ __forceinline__ uint32_t tile_flags(uint32_t tile, uint32_t tid, uint32_t L, const uint32_t* __restrict__ first_of,
+                                               uint8_t* __restrict__ flag8) {
+    const uint32_t base = tile * REMAP_TILE + tid * REMAP_ITEMS;
     uint32_t bits = 0;
     static_assert(REMAP_ITEMS == 8, "a thread's lookups are two 16-byte loads");
     if (base + REMAP_ITEMS <= L) {
@@ -481,24 +481,44 @@ static __global__ __launch_bounds__(REMAP_THREADS) void k_lds_flags(uint32_t L, 
         }
         flag8[base / REMAP_ITEMS] = (uint8_t)bits;
     }
-    uint32_t total = block_sum_256(__popc(bits), red);
-    if (threadIdx.x == 0) tilesum[blockIdx.x] = total;
+    return __popc(bits);
+}
+// The tiles from `tile0` on, `waves` / 4 of them, by a workgroup of that many wavefronts.  red: a word per wavefront.
+__device__ __forceinline__ void flag_tiles(uint32_t tile0, uint32_t ntiles, uint32_t L, const uint32_t* __restrict__ first_of,
+                                           uint8_t* __restrict__ flag8, uint32_t* __restrict__ tilesum, uint32_t* red) {
+    const uint32_t tile = tile0 + threadIdx.x / REMAP_THREADS, tid = threadIdx.x % REMAP_THREADS;
+    uint32_t n = tile < ntiles ? tile_flags(tile, tid, L, first_of, flag8) : 0u;
+    for (int o = 32; o > 0; o >>= 1) n += __shfl_xor(n, o);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = n;
+    __syncthreads();
+    const uint32_t w = threadIdx.x / 64;
+    if (tid == 0 && tile < ntiles) tilesum[tile] = red[w] + red[w + 1] + red[w + 2] + red[w + 3];
+}
+static_assert(REMAP_THREADS == 256, "four wavefronts a tile");
+
+static __global__ __launch_bounds__(REMAP_THREADS) void k_lds_flags(uint32_t L, const uint32_t* __restrict__ first_of,
+                                                             uint8_t* __restrict__ flag8,
+                                                             uint32_t* __restrict__ tilesum,
+                                                             const SlotDesc* __restrict__ descs, int N,
+                                                             const uint32_t* __restrict__ bcursor,
+                                                             DevStatus* status) {
+    __shared__ uint32_t red[4];
+    if (threadIdx.x < 64)
+        for (int sl = blockIdx.x; sl < N; sl += gridDim.x) slot_tile_share(descs[sl], bcursor, status);
+    flag_tiles(blockIdx.x, gridDim.x, L, first_of, flag8, tilesum, red);
 }
 
 // Ranks of the first occurrences (per 64-lookup word: wordpre, see rank_of) and, with LISTS, the distinct
 // lists and show counts.  Each thread owns 8 consecutive lookups; all loads are
 // issued before any dependent store.
 template <bool LISTS>
-__global__ __launch_bounds__(REMAP_THREADS) void k_lds_assign(
+__device__ __forceinline__ void assign_tile(
+    uint32_t* lb, uint32_t* red, uint32_t ntiles,
     const SlotDesc* __restrict__ descs, const uint32_t* __restrict__ lbase, int N, uint32_t L,
     const uint8_t* __restrict__ flag8, const uint32_t* __restrict__ tileoff, const uint32_t* __restrict__ cnt_at,
     uint32_t* __restrict__ wordpre, uint32_t* __restrict__ ubase, uint64_t* __restrict__ uniq_sign,
     uint32_t* __restrict__ uniq_slot, uint32_t* __restrict__ ushow, const uint32_t* __restrict__ tilesum,
     DevStatus* status) {
-    // lb[N + 1], sized by the launch: a fixed array for the largest slot count would take 16 KB of LDS per
-    // workgroup away from the grouping kernel that runs beside this one
-    extern __shared__ uint32_t lb[];
-    __shared__ uint32_t red[4];
     load_lbase(lb, lbase, N);
     const uint32_t base = blockIdx.x * REMAP_TILE + threadIdx.x * REMAP_ITEMS;
     uint32_t bits = 0;
@@ -515,7 +535,7 @@ __global__ __launch_bounds__(REMAP_THREADS) void k_lds_assign(
     }
     uint32_t total;
     uint32_t u = off + block_excl_scan_256<uint32_t>(__popc(bits), red, &total);
-    if (tilesum && blockIdx.x == gridDim.x - 1) {  // what k_scan_tiles leaves besides the offsets
+    if (tilesum && blockIdx.x == ntiles - 1) {  // what k_scan_tiles leaves besides the offsets
         const uint32_t U = off + total;
         if (threadIdx.x == 0) {
             status->n_unique = U;
@@ -566,20 +586,29 @@ __global__ __launch_bounds__(REMAP_THREADS) void k_lds_assign(
     }
 }
 
-// mapped id = rank of the sign's first occurrence, relative to the slot.
-static __global__ __launch_bounds__(256) void k_lds_mapped(const SlotDesc* __restrict__ descs,
-                                                    const uint32_t* __restrict__ lbase,
-                                                    const uint32_t* __restrict__ ubase, int N, uint32_t L,
-                                                    const uint32_t* __restrict__ first_of,
-                                                    const uint8_t* __restrict__ flag8,
-                                                    const uint32_t* __restrict__ wordpre,
-                                                    uint32_t* __restrict__ u_of_gi) {
-    extern __shared__ uint32_t lb[];  // lb[N + 1], sized by the launch (see k_lds_assign)
+template <bool LISTS>
+__global__ __launch_bounds__(REMAP_THREADS) void k_lds_assign(
+    const SlotDesc* __restrict__ descs, const uint32_t* __restrict__ lbase, int N, uint32_t L,
+    const uint8_t* __restrict__ flag8, const uint32_t* __restrict__ tileoff, const uint32_t* __restrict__ cnt_at,
+    uint32_t* __restrict__ wordpre, uint32_t* __restrict__ ubase, uint64_t* __restrict__ uniq_sign,
+    uint32_t* __restrict__ uniq_slot, uint32_t* __restrict__ ushow, const uint32_t* __restrict__ tilesum,
+    DevStatus* status) {
+    extern __shared__ uint32_t lb[];  // lb[N + 1], sized by the launch
+    __shared__ uint32_t red[4];
+    assign_tile<LISTS>(lb, red, gridDim.x, descs, lbase, N, L, flag8, tileoff, cnt_at, wordpre, ubase, uniq_sign, uniq_slot, ushow,
+                       tilesum, status);
+}
+
+// mapped id = rank of the sign's first occurrence, relative to the slot.  By workgroup `at` of `of`.
+__device__ __forceinline__ void map_lookups(uint32_t* lb, uint32_t at, uint32_t of, const SlotDesc* __restrict__ descs,
+                                            const uint32_t* __restrict__ lbase, const uint32_t* __restrict__ ubase, int N,
+                                            uint32_t L, const uint32_t* __restrict__ first_of, const uint8_t* __restrict__ flag8,
+                                            const uint32_t* __restrict__ wordpre, uint32_t* __restrict__ u_of_gi) {
     load_lbase(lb, lbase, N);
     // four consecutive lookups per thread: one 16-byte load and store, one slot search
-    const uint32_t stride = gridDim.x * blockDim.x;
+    const uint32_t stride = of * blockDim.x;
     const uint32_t quads = (L + 3) / 4;
-    for (uint32_t q = blockIdx.x * blockDim.x + threadIdx.x; q < quads; q += stride) {
+    for (uint32_t q = at * blockDim.x + threadIdx.x; q < quads; q += stride) {
         const uint32_t g0 = q * 4;
         uint32_t f[4], u[4];
         if (g0 + 4 <= L) {
@@ -622,6 +651,17 @@ static __global__ __launch_bounds__(256) void k_lds_mapped(const SlotDesc* __res
     }
 }
 
+static __global__ __launch_bounds__(256) void k_lds_mapped(const SlotDesc* __restrict__ descs,
+                                                    const uint32_t* __restrict__ lbase,
+                                                    const uint32_t* __restrict__ ubase, int N, uint32_t L,
+                                                    const uint32_t* __restrict__ first_of,
+                                                    const uint8_t* __restrict__ flag8,
+                                                    const uint32_t* __restrict__ wordpre,
+                                                    uint32_t* __restrict__ u_of_gi) {
+    extern __shared__ uint32_t lb[];  // lb[N + 1], sized by the launch
+    map_lookups(lb, blockIdx.x, gridDim.x, descs, lbase, ubase, N, L, first_of, flag8, wordpre, u_of_gi);
+}
+
 // One workgroup per second-level bucket: groups its records by sign (all slots
 // of a sign meet here) with an LDS table of slot masks.  The place of a record
 // among its group's members (ascending slot order) is the number of lower
@@ -632,13 +672,13 @@ static __global__ __launch_bounds__(256) void k_lds_mapped(const SlotDesc* __res
 // and per bucket the number of groups with one record, with several, the
 // records of the latter, and the big groups.  At most GRP_SLOTS slots.
 // 2039 examples of 211 slots (860 k lookups): the grouping in memory that more than 128 slots took before (insert, compact,
-// fill, rank and the probe of the groups behind it) 162 us, 67 (k_group_count 21, k_probe_recs and k_init_new_recs 19,
-// k_group_emit 17, 10 more in k_lds_dedup).
+// fill, rank and the probe of the groups behind it) 162 us, 67 as launches of their own (counts 21, probes and new rows 19,
+// member lists 17, 10 more in k_lds_dedup).
 // LDS of a workgroup that groups second-level buckets (group_count_bucket).
 template <int WORDS>
 struct GroupCountLds {
-    unsigned long long keys[GRP_TABLE + 1];  // entry GRP_TABLE: the sign EMPTY_KEY itself
-    unsigned long long mask[WORDS][GRP_TABLE + 1];
+    unsigned long long keys[grp_table(WORDS) + 1];  // entry grp_table: the sign EMPTY_KEY itself
+    unsigned long long mask[WORDS][grp_table(WORDS) + 1];
     uint16_t rech[GRP_CAP];
     unsigned long long sh[GRP_THREADS / 64];
 };
@@ -648,6 +688,7 @@ template <int WORDS>
 __device__ __forceinline__ void group_count_bucket(uint32_t c, GroupCountLds<WORDS>& lds, const uint32_t* __restrict__ cursor2,
                                                    const GroupRec* __restrict__ recs, uint32_t big_k,
                                                    uint2* __restrict__ aux, uint4* __restrict__ bcounts) {
+    constexpr int TABLE = grp_table(WORDS), ITEMS = (TABLE + 1 + GRP_THREADS - 1) / GRP_THREADS;
     unsigned long long* const keys = lds.keys;
     uint16_t* const rech = lds.rech;
     unsigned long long* const sh = lds.sh;
@@ -675,7 +716,7 @@ __device__ __forceinline__ void group_count_bucket(uint32_t c, GroupCountLds<WOR
             sl[j] = r.cnt >> 24;
         }
     }
-    for (int i = threadIdx.x; i <= GRP_TABLE; i += GRP_THREADS) {
+    for (int i = threadIdx.x; i <= TABLE; i += GRP_THREADS) {
         keys[i] = EMPTY_KEY;
 #pragma unroll
         for (int w = 0; w < WORDS; w++) lds.mask[w][i] = 0;
@@ -685,26 +726,26 @@ __device__ __forceinline__ void group_count_bucket(uint32_t c, GroupCountLds<WOR
     for (int j = 0; j < GRP_RECS; j++) {
         if (sl[j] == 0xFFFFFFFFu) continue;
         const uint64_t sign = sg[j];
-        uint32_t h = GRP_TABLE;
+        uint32_t h = TABLE;
         if (sign != EMPTY_KEY) {
-            h = (uint32_t)(mix64(sign) >> 9) & (GRP_TABLE - 1);
-            for (;;) {  // n <= GRP_CAP < GRP_TABLE: a free entry exists
+            h = scale32((uint32_t)mix64(sign), TABLE);  // (the hash's lower half: the bucket was chosen by the upper one)
+            for (;;) {  // n <= GRP_CAP < TABLE: a free entry exists
                 unsigned long long old = keys[h];
                 if (old == EMPTY_KEY) old = atomicCAS(&keys[h], (unsigned long long)EMPTY_KEY, sign);
                 if (old == EMPTY_KEY || old == sign) break;
-                h = (h + 1) & (GRP_TABLE - 1);
+                h = h + 1 == (uint32_t)TABLE ? 0 : h + 1;
             }
         }
         atomicOr(&lds.mask[sl[j] >> 6][h], 1ull << (sl[j] & 63));
         rech[j * GRP_THREADS + threadIdx.x] = (uint16_t)h;
     }
     __syncthreads();
-    uint32_t ks[GRP_ITEMS];
+    uint32_t ks[ITEMS];
     unsigned long long v = 0;  // 16-bit fields: groups of one record, of several, records of those, big groups
-    for (int j = 0; j < GRP_ITEMS; j++) {
+    for (int j = 0; j < ITEMS; j++) {
         const uint32_t e = j * GRP_THREADS + threadIdx.x;
         uint32_t k = 0;
-        if (e <= GRP_TABLE) {
+        if (e <= TABLE) {
 #pragma unroll
             for (int w = 0; w < WORDS; w++) k += (uint32_t)__popcll(lds.mask[w][e]);
         }
@@ -717,7 +758,7 @@ __device__ __forceinline__ void group_count_bucket(uint32_t c, GroupCountLds<WOR
     if (threadIdx.x == 0)
         bcounts[c] = make_uint4((uint32_t)(total & 0xFFFF), (uint32_t)((total >> 16) & 0xFFFF),
                                 (uint32_t)((total >> 32) & 0xFFFF), (uint32_t)(total >> 48));
-    for (int j = 0; j < GRP_ITEMS; j++) {
+    for (int j = 0; j < ITEMS; j++) {
         const uint32_t k = ks[j];
         if (k == 0) continue;
         const uint32_t e = j * GRP_THREADS + threadIdx.x;
@@ -745,17 +786,6 @@ __device__ __forceinline__ void group_count_bucket(uint32_t c, GroupCountLds<WOR
         }
         const uint2 ei = einfo[h];
         aux[first + i] = make_uint2(ei.x, ei.y | (place << 16) | (s1 << 24));
-    }
-}
-
-template <int WORDS>
-__global__ __launch_bounds__(GRP_THREADS) void k_group_count(uint32_t nb2, const uint32_t* __restrict__ cursor2,
-                                                     const GroupRec* __restrict__ recs, uint32_t big_k,
-                                                     uint2* __restrict__ aux, uint4* __restrict__ bcounts) {
-    __shared__ GroupCountLds<WORDS> lds;
-    for (uint32_t c = blockIdx.x; c < nb2; c += gridDim.x) {
-        group_count_bucket(c, lds, cursor2, recs, big_k, aux, bcounts);
-        __syncthreads();
     }
 }
 
@@ -808,39 +838,86 @@ static __global__ __launch_bounds__(1024) void k_group_offsets(const uint4* __re
 
 // The table row of every distinct record, found or, for an absent sign, inserted and filled
 // (SparseKernelBlock::GetWeight, optimizer_kernel.h:299-308): rrow[record] = row, NO_ROW if the
-// table is full.  It needs nothing but the records the dedup handed over, so it runs on a
-// stream of its own beside the grouping and the ranking (random reads of the table against LDS
+// table is full.  It needs nothing but the records the dedup handed over, so its workgroups stand
+// beside the grouping's and the flags' (random reads of the table against LDS
 // and streaming work).  A sign present in several slots is probed once per slot; whichever
 // thread claims a free slot first owns the insertion, the others find the key there.
 // A new row is not filled here: one or two lanes of a wavefront drawing sixteen normal deviates would hold up
 // the other sixty (with 1 % of the lookups new, most wavefronts have such a lane); the record is listed and
-// k_init_new_recs fills the rows with every lane busy.  The list is the bucket's own -- newrec[c * GRP_CAP ...],
+// init_new_recs fills the rows with every lane busy.  The list is the bucket's own -- newrec[c * GRP_CAP ...],
 // newcnt[c] entries -- not one list of the call: places in one list are handed out by atomics on one counter,
 // which take about 11 ns each one after the other (one per wavefront, tens of thousands, took longer than all the
 // probes together; one per bucket still kept every workgroup waiting for its turn among a thousand).
-static __global__ __launch_bounds__(256) void k_probe_recs(uint32_t nb2, const uint32_t* __restrict__ cursor2,
-                                                    const GroupRec* __restrict__ recs, uint32_t* __restrict__ rrow,
-                                                    uint32_t* __restrict__ newrec, uint32_t* __restrict__ newcnt,
-                                                    Store s, DevStatus* status) {
-    __shared__ uint32_t s_count;
-    for (uint32_t c = blockIdx.x; c < nb2; c += gridDim.x) {
-        const uint32_t n = min(cursor2[c], (uint32_t)GRP_CAP);
-        const size_t first = (size_t)c * GRP_CAP;
-        if (threadIdx.x == 0) s_count = 0;
-        __syncthreads();
-        for (uint32_t i0 = 0; i0 < n; i0 += 256) {
-            const uint32_t i = i0 + threadIdx.x;
-            bool is_new = false;
-            if (i < n) {
-                const uint64_t sign = recs[first + i].sign;
-                const uint32_t row = probe_slot<true>(s, sign, is_new);
-                rrow[first + i] = row;
-                if (row == NO_ROW) atomicOr(&status->err, DEV_ERR_TABLE_FULL);
-            }
-            if (is_new) newrec[first + atomicAdd(&s_count, 1u)] = i;  // rare: about one record in forty (at most n)
+__device__ __forceinline__ void probe_bucket(uint32_t c, uint32_t* s_count, const uint32_t* __restrict__ cursor2,
+                                             const GroupRec* __restrict__ recs, uint32_t* __restrict__ rrow,
+                                             uint32_t* __restrict__ newrec, uint32_t* __restrict__ newcnt, const Store& s,
+                                             DevStatus* status) {
+    const uint32_t n = min(cursor2[c], (uint32_t)GRP_CAP);
+    const size_t first = (size_t)c * GRP_CAP;
+    uint64_t sign[GRP_RECS];
+#pragma unroll
+    for (int j = 0; j < GRP_RECS; j++) {
+        const uint32_t i = j * GRP_THREADS + threadIdx.x;
+        sign[j] = i < n ? recs[first + i].sign : 0;
+    }
+    if (threadIdx.x == 0) *s_count = 0;
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < GRP_RECS; j++) {
+        const uint32_t i = j * GRP_THREADS + threadIdx.x;
+        if (i >= n) break;
+        bool is_new = false;
+        const uint32_t row = probe_slot<true>(s, sign[j], is_new);
+        rrow[first + i] = row;
+        if (row == NO_ROW) atomicOr(&status->err, DEV_ERR_TABLE_FULL);
+        if (is_new) newrec[first + atomicAdd(s_count, 1u)] = i;  // rare: about one record in forty (at most n)
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) newcnt[c] = *s_count;
+}
+
+// What the dedup's records and first positions are wanted for first, by one launch: the groups of equal signs (a workgroup per
+// second-level bucket, LDS), the signs' rows (a workgroup per bucket, random reads: every other workgroup, so that a CU has some
+// of both), the first-occurrence flags (two tiles a workgroup) and what the slots' buckets were handed (a wavefront per slot).
+// Three launches on a stream take the sum of their times; three streams beside each other left most of it in the hand-overs.
+// 2.1 M lookups of 64 slots: 28 us as three launches, 21.5; 4.9 M of 100: 86 alone, about 90 with the hand-overs of three
+// streams, 68.  It wants six wavefronts a SIMD (three workgroups to a CU; two, 83 registers: 82 us).
+struct GroupProbeArgs {
+    uint32_t nb2, ntiles, L;
+    const uint32_t* cursor2;
+    const GroupRec* recs;
+    uint32_t big_k;
+    uint2* aux;
+    uint4* bcounts;
+    uint32_t *rrow, *newrec, *newcnt;
+    const uint32_t* first_of;
+    uint8_t* flag8;
+    uint32_t* tilesum;
+    const SlotDesc* descs;
+    int N;
+    const uint32_t* bcursor;
+};
+template <int WORDS>
+__global__ __launch_bounds__(GRP_THREADS) __attribute__((amdgpu_waves_per_eu(WORDS == 2 ? 6 : 4, 8))) void k_group_probe(GroupProbeArgs a, Store s, DevStatus* status) {
+    __shared__ union {
+        GroupCountLds<WORDS> group;
+        uint32_t red[GRP_THREADS / 64];
+    } lds;
+    constexpr uint32_t TILES = GRP_THREADS / REMAP_THREADS, SLOTS = GRP_THREADS / 64;
+    const uint32_t flags0 = 2 * a.nb2, slots0 = flags0 + (a.ntiles + TILES - 1) / TILES;
+    const uint32_t items = slots0 + ((uint32_t)a.N + SLOTS - 1) / SLOTS;
+    for (uint32_t item = blockIdx.x; item < items; item += gridDim.x) {
+        if (item < flags0) {
+            if (item & 1u)
+                group_count_bucket(item / 2, lds.group, a.cursor2, a.recs, a.big_k, a.aux, a.bcounts);
+            else
+                probe_bucket(item / 2, lds.red, a.cursor2, a.recs, a.rrow, a.newrec, a.newcnt, s, status);
+        } else if (item < slots0) {
+            flag_tiles((item - flags0) * TILES, a.ntiles, a.L, a.first_of, a.flag8, a.tilesum, lds.red);
+        } else {
+            const uint32_t sl = (item - slots0) * SLOTS + threadIdx.x / 64;
+            if (sl < (uint32_t)a.N) slot_tile_share(a.descs[sl], a.bcursor, status);
         }
-        __syncthreads();
-        if (threadIdx.x == 0) newcnt[c] = s_count;
         __syncthreads();
     }
 }
@@ -865,35 +942,52 @@ __device__ __forceinline__ void init_row_pair(const Store& s, const OptDev& o, u
     }
 }
 
-// Fills the rows k_probe_recs inserted, `parts` workgroups per bucket's list (a batch of few buckets and many new
+// Fills the rows probe_bucket inserted, `parts` workgroups per bucket's list (a batch of few buckets and many new
 // signs still fills the device) and one lane per pair of elements; the first workgroup also adds up the lists'
 // lengths: the call's number of new rows.
-static __global__ __launch_bounds__(256) void k_init_new_recs(Store s, OptDev o, uint64_t seed,
-                                                       const GroupRec* __restrict__ recs,
-                                                       const uint32_t* __restrict__ rrow, uint32_t nb2,
-                                                       const uint32_t* __restrict__ newrec,
-                                                       const uint32_t* __restrict__ newcnt, DevStatus* status,
-                                                       uint32_t parts) {
-    __shared__ uint32_t red[4];
-    if (blockIdx.x == 0) {
+struct InitArgs {
+    uint64_t seed;
+    const GroupRec* recs;
+    const uint32_t* rrow;
+    uint32_t nb2;
+    const uint32_t *newrec, *newcnt;
+    uint32_t parts;
+};
+__device__ __forceinline__ void init_new_recs(const Store& s, const OptDev& o, const InitArgs& a, uint32_t at, uint32_t of,
+                                              uint32_t* red, DevStatus* status) {
+    if (at == 0) {
         uint32_t mine = 0;
-        for (uint32_t c = threadIdx.x; c < nb2; c += 256) mine += min(newcnt[c], (uint32_t)GRP_CAP);
+        for (uint32_t c = threadIdx.x; c < a.nb2; c += 256) mine += min(a.newcnt[c], (uint32_t)GRP_CAP);
         uint32_t total;
         block_excl_scan_256<uint32_t>(mine, red, &total);
         if (threadIdx.x == 0) status->n_new = total;
     }
     const uint32_t pairs = (uint32_t)(s.D + 1) / 2;
     const float stddev = (float)(1.0 / sqrt((double)s.D));
-    for (uint32_t w = blockIdx.x; w < nb2 * parts; w += gridDim.x) {
-        const uint32_t c = w / parts, part = w - c * parts;
-        const uint32_t cnt = min(newcnt[c], (uint32_t)GRP_CAP);
+    for (uint32_t w = at; w < a.nb2 * a.parts; w += of) {
+        const uint32_t c = w / a.parts, part = w - c * a.parts;
+        const uint32_t cnt = min(a.newcnt[c], (uint32_t)GRP_CAP);
         const size_t first = (size_t)c * GRP_CAP;
-        for (uint32_t t = part * 256 + threadIdx.x; t < cnt * pairs; t += parts * 256) {
+        for (uint32_t t = part * 256 + threadIdx.x; t < cnt * pairs; t += a.parts * 256) {
             const uint32_t j = t / pairs, q = t - j * pairs;
-            const size_t i = first + min(newrec[first + j], (uint32_t)GRP_CAP - 1);
-            init_row_pair(s, o, seed, recs[i].sign, rrow[i], q, stddev);
+            const size_t i = first + min(a.newrec[first + j], (uint32_t)GRP_CAP - 1);
+            init_row_pair(s, o, a.seed, a.recs[i].sign, a.rrow[i], q, stddev);
         }
     }
+}
+
+// The ranks, then the new rows (as two launches of 2.1 M lookups 5.5 + 4.0 us, so 5.4).
+static __global__ __launch_bounds__(REMAP_THREADS) void k_assign_init(
+    const SlotDesc* __restrict__ descs, const uint32_t* __restrict__ lbase, int N, uint32_t L, uint32_t ntiles,
+    const uint8_t* __restrict__ flag8, const uint32_t* __restrict__ tileoff, uint32_t* __restrict__ wordpre,
+    uint32_t* __restrict__ ubase, const uint32_t* __restrict__ tilesum, Store s, OptDev o, InitArgs init, DevStatus* status) {
+    extern __shared__ uint32_t lb[];  // lb[N + 1], sized by the launch
+    __shared__ uint32_t red[4];
+    if (blockIdx.x < ntiles)
+        assign_tile<false>(lb, red, ntiles, descs, lbase, N, L, flag8, tileoff, nullptr, wordpre, ubase, nullptr, nullptr, nullptr,
+                           tilesum, status);
+    else
+        init_new_recs(s, o, init, blockIdx.x - ntiles, gridDim.x - ntiles, red, status);
 }
 
 // Numbers the groups and writes the member lists: groups with one record get
@@ -907,7 +1001,7 @@ static __global__ __launch_bounds__(256) void k_init_new_recs(Store s, OptDev o,
 // the arrays is first put together in LDS and then copied out in order; only where_u, indexed
 // by the distinct index of the record, stays a scattered store.  where_u[u] = {place in the member
 // list (with WHERE_ONE_TILE if all lookups of the record lie in one tile), table row of the record's sign
-// (rrow, from k_probe_recs)}; the groups get the rows too.  A group with big_k records or more is listed in
+// (rrow, from probe_bucket)}; the groups get the rows too.  A group with big_k records or more is listed in
 // big_list and, with {row, first member, records, group}, in big_desc.
 //
 template <bool SMALL>
@@ -933,7 +1027,7 @@ struct EmitArgs<false> {
     uint32_t* grp_row;
     DevStatus* status;
 };
-__device__ __forceinline__ void emit_buckets(uint32_t nb2, const uint32_t* __restrict__ cursor2,
+__device__ __forceinline__ void emit_buckets(uint32_t of, uint32_t nb2, const uint32_t* __restrict__ cursor2,
                                              const GroupRec* __restrict__ recs, const uint2* __restrict__ aux,
                                              const uint4* __restrict__ bbase, const uint4* __restrict__ bcounts,
                                              const uint8_t* __restrict__ flag8, const uint32_t* __restrict__ wordpre,
@@ -953,7 +1047,7 @@ __device__ __forceinline__ void emit_buckets(uint32_t nb2, const uint32_t* __res
     __shared__ uint32_t s_off[GRP_CAP / 2];
     __shared__ uint16_t s_cnt[GRP_CAP / 2];  // at most GRP_SLOTS records per group
     __shared__ uint4 s_part[EMIT_THREADS / 64];
-    for (uint32_t c = blockIdx.x; c < nb2; c += gridDim.x) {
+    for (uint32_t c = blockIdx.x; c < nb2; c += of) {
         const uint32_t n = min(cursor2[c], (uint32_t)GRP_CAP);
         const size_t first = (size_t)c * GRP_CAP;
         // the bucket's records first: their loads are in flight while the bucket's offsets are worked out
@@ -1076,13 +1170,29 @@ __device__ __forceinline__ void emit_buckets(uint32_t nb2, const uint32_t* __res
 template <bool SMALL>
 __global__ __launch_bounds__(EmitArgs<SMALL>::THREADS) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_group_emit(
     EmitArgs<SMALL> a) {
-    if constexpr (SMALL) {
-        extern __shared__ uint32_t emit_lds[];
-        small_emit_bucket(a, emit_lds);
-    } else {
-        emit_buckets(a.nb2, a.cursor2, a.recs, a.aux, a.bbase, a.bcounts, a.flag8, a.wordpre, a.ids_cap, a.big_k, a.grp_sign,
-                     a.grp_off, a.grp_cnt, a.big_list, a.big_desc, a.list, a.where_u, a.rrow, a.grp_row, a.status);
-    }
+    extern __shared__ uint32_t emit_lds[];
+    small_emit_bucket(a, emit_lds);
+}
+
+// The member lists, whose workgroups are chains of round trips, and the mapped ids, a stream, by one launch: 2.1 M lookups of 64
+// slots 26 us for 31, 4.9 M of 100 slots 77 for 100.
+struct MapArgs {
+    const SlotDesc* descs;
+    const uint32_t *lbase, *ubase;
+    int N;
+    uint32_t L;
+    const uint32_t* first_of;
+    uint32_t* u_of_gi;
+};
+static __global__ __launch_bounds__(EMIT_THREADS) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_emit_mapped(
+    EmitArgs<false> a, MapArgs m, uint32_t emit_blocks) {
+    extern __shared__ uint32_t lb[];  // lb[N + 1], sized by the launch
+    if (blockIdx.x < emit_blocks)
+        emit_buckets(emit_blocks, a.nb2, a.cursor2, a.recs, a.aux, a.bbase, a.bcounts, a.flag8, a.wordpre, a.ids_cap, a.big_k,
+                     a.grp_sign, a.grp_off, a.grp_cnt, a.big_list, a.big_desc, a.list, a.where_u, a.rrow, a.grp_row, a.status);
+    else
+        map_lookups(lb, blockIdx.x - emit_blocks, gridDim.x - emit_blocks, m.descs, m.lbase, m.ubase, m.N, m.L, m.first_of, a.flag8,
+                    a.wordpre, m.u_of_gi);
 }
 
 }  // namespace tn

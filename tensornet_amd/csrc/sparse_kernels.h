@@ -182,11 +182,10 @@ static __global__ __launch_bounds__(256) void k_stage_in(const uint32_t* __restr
 // host_dst: a DevStatus followed by n_ubase words.  With count != nullptr the rows the call
 // inserted are added to the table's number of resident keys.  With host_seq != nullptr the word seq is written
 // there once everything else is on the host: a host that polls that word has the status a few microseconds
-// after this kernel, well before a wait on the stream would return.
-static __global__ __launch_bounds__(256) void k_publish(const DevStatus* __restrict__ status,
-                                                 const uint32_t* __restrict__ ubase, uint32_t n_ubase,
-                                                 uint32_t* __restrict__ host_dst, unsigned long long* count,
-                                                 uint32_t* host_seq, uint32_t seq) {
+// after this kernel, well before a wait on the stream would return.  By one workgroup.
+__device__ __forceinline__ void publish(const DevStatus* __restrict__ status, const uint32_t* __restrict__ ubase, uint32_t n_ubase,
+                                        uint32_t* __restrict__ host_dst, unsigned long long* count, uint32_t* host_seq,
+                                        uint32_t seq) {
     if (count && threadIdx.x == 0) *count += status->n_new;
     const uint32_t sw = sizeof(DevStatus) / 4;
     const uint32_t* sp = reinterpret_cast<const uint32_t*>(status);
@@ -198,6 +197,18 @@ static __global__ __launch_bounds__(256) void k_publish(const DevStatus* __restr
         if (threadIdx.x == 0) __hip_atomic_store(host_seq, seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
 }
+static __global__ __launch_bounds__(256) void k_publish(const DevStatus* __restrict__ status,
+                                                 const uint32_t* __restrict__ ubase, uint32_t n_ubase,
+                                                 uint32_t* __restrict__ host_dst, unsigned long long* count) {
+    publish(status, ubase, n_ubase, host_dst, count, nullptr, 0);
+}
+// The same as the first workgroup of another kernel (host_dst == nullptr: nothing to publish).
+struct Publish {
+    uint32_t* host_dst;
+    unsigned long long* count;
+    uint32_t* host_seq;
+    uint32_t seq;
+};
 
 static __global__ void k_finish_insert(Store s, const DevStatus* status) {
     if (threadIdx.x == 0 && blockIdx.x == 0) *s.count += status->n_new;
@@ -965,6 +976,13 @@ struct PushSrc {
     const float* flat;
     // op-level push on the last pull's plan: the comparison of its signs, ahead of the update kernels, is complete
     HostWord compared;
+    // ... and where in pinned memory the host finds an error of theirs (such a push publishes no status)
+    uint32_t* host_err;
+    // a slot's gradient matrix has no row for one of its distinct signs
+    __device__ __forceinline__ void no_gradient(DevStatus* status) const {
+        atomicOr(&status->err, DEV_ERR_GRAD_ROWS);
+        if (host_err) *host_err = DEV_ERR_GRAD_ROWS;
+    }
 };
 
 __device__ __forceinline__ uint64_t src_sign(const PushSrc& p, uint32_t u) {
@@ -1236,20 +1254,28 @@ static __global__ __launch_bounds__(256) void k_mask_fill(const DevStatus* statu
 // vars[slot][rank, :] = table row of the sign, for every distinct sign u of
 // every slot (PopulatePulledVariable_, sparse_table_ops.cc:244-265).
 // grp_row == nullptr: where_u[u].y is the row itself instead of the group that has it.
+// pub: a call whose status is final by now publishes it here, by a workgroup of its own, the first: the host has it while the
+// others still copy (a launch of its own took 4.6 us of a pull that keeps to one stream, and where it ran on a second one, the
+// hand-over).
 template <int VEC>
 __global__ __launch_bounds__(256) void k_gather_vars(Store s, DevStatus* status, const uint32_t* __restrict__ grp_row,
                                                      const uint2* __restrict__ where_u,
                                                      const uint32_t* __restrict__ ubase, int N,
-                                                     const SlotDesc* __restrict__ descs) {
+                                                     const SlotDesc* __restrict__ descs, Publish pub) {
     __shared__ uint32_t ub[MAX_SLOTS + 1];
+    const uint32_t first = pub.host_dst ? 1u : 0u;
+    if (blockIdx.x < first) {
+        publish(status, ubase, (uint32_t)(N + 1), pub.host_dst, pub.count, pub.host_seq, pub.seq);
+        return;
+    }
     // A remap whose LDS tables overflowed dropped records: their where_u entries were never written (the
     // host repeats the call on the other path).  The flag is final before this kernel starts.
     if (status->err & DEV_ERR_REMAP_OVERFLOW) return;
     load_lbase(ub, ubase, N);
     const int chunks = s.wdim / VEC;
     const int64_t total = (int64_t)status->n_unique * chunks;
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < total; t += stride) {
+    const int64_t stride = (int64_t)(gridDim.x - first) * blockDim.x;
+    for (int64_t t = (int64_t)(blockIdx.x - first) * blockDim.x + threadIdx.x; t < total; t += stride) {
         const int64_t u = t / chunks;
         const int c = (int)(t - u * chunks);
         const uint32_t row = grp_row ? grp_row[where_u[u].y] : where_u[u].y;
@@ -1610,7 +1636,7 @@ __device__ __forceinline__ void apply_singles(const Store& s, const OptDev& o, c
         const float* gp;
         int bshow, bclick;
         if (!src_record(src, list[g], gp, bshow, bclick)) {
-            if (sub == 0) atomicOr(&status->err, DEV_ERR_GRAD_ROWS);
+            if (sub == 0) src.no_gradient(status);
             continue;
         }
         apply_one_record<KIND, LPG, ANY>(s, o, row, gp, bshow, bclick, sub, lane0, c1, c2);
@@ -1692,7 +1718,7 @@ __device__ __forceinline__ void apply_group_vec(const Store& s, const OptDev& o,
         }
     };
     auto no_gradient = [&]() {
-        if (sub == 0) atomicOr(&status->err, DEV_ERR_GRAD_ROWS);
+        if (sub == 0) src.no_gradient(status);
     };
     const float* gp;
     int nshow = 0, nclick = 0;
@@ -2040,7 +2066,7 @@ __global__ __launch_bounds__(64) void k_apply_big(Store s, OptDev o, PushSrc src
             k = grp_cnt[g];
         },
         [&](uint32_t at, const float*& gp, int& sh, int& ck) { return record_at(src, list, gaddr, at, gp, sh, ck); },
-        [&] { atomicOr(&status->err, DEV_ERR_GRAD_ROWS); }, [] { __syncthreads(); });
+        [&] { src.no_gradient(status); }, [] { __syncthreads(); });
 }
 
 // One sign with many records by a wavefront, rows of D elements, D a power of two up to 64.  A small batch's updates are as
@@ -2379,7 +2405,7 @@ constexpr int big_waves(int D) { return D == 64 ? 5 : 6; }
 constexpr int big_most_alone(int D) { return D == 4 || D == 16 ? 4 : 8; }
 
 // k_apply_big for AdaGrad rows of D elements, D a power of two from 4 to 64, on a plan whose big_desc lists {row, first member,
-// records, group} of every sign with many records (written by k_group_emit): one wavefront per sign, by apply_big_wave.  (Adam and
+// records, group} of every sign with many records (written by k_emit_mapped): one wavefront per sign, by apply_big_wave.  (Adam and
 // Ftrl the same way: 800 k lookups, Adam rows of 16, 136 us a step with and without; not worth their kernels.)
 template <int D>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6, 8))) void k_apply_big_adagrad(
@@ -2395,7 +2421,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6, 8))) void
         s, o, lds, head, blockIdx.x, gridDim.x, status->n_big, [&](uint32_t bi) { return big_desc[bi]; },
         [&](uint32_t at) { return from.entry(at); },
         [&](const BigSrc::Entry& e, const float*& gp, int& sh, int& ck, bool) { return from.record(e, gp, sh, ck); },
-        [&] { atomicOr(&status->err, DEV_ERR_GRAD_ROWS); });
+        [&] { src.no_gradient(status); });
 }
 
 // The updates of a push of up to ONE_STREAM_LOOKUPS lookups by one launch: the workgroups of the three kernels above side
@@ -2433,7 +2459,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(big_waves(T
                 s, o, lds[wave], head, first, stride, status->n_big, [&](uint32_t bi) { return a.big_desc[bi]; },
                 [&](uint32_t at) { return from.entry(at); },
                 [&](const BigSrc::Entry& e, const float*& gp, int& sh, int& ck, bool) { return from.record(e, gp, sh, ck); },
-                [&] { atomicOr(&status->err, DEV_ERR_GRAD_ROWS); });
+                [&] { src.no_gradient(status); });
         } else {
             extern __shared__ unsigned long long all_lds[];
             char* base = reinterpret_cast<char*>(all_lds) + wave * a.wave_lds;
@@ -2450,7 +2476,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(big_waves(T
                 [&](uint32_t at, const float*& gp, int& sh, int& ck) {
                     return record_at(src, a.list, a.gaddr, at, gp, sh, ck);
                 },
-                [&] { atomicOr(&status->err, DEV_ERR_GRAD_ROWS); }, [] { wave_sync(); });
+                [&] { src.no_gradient(status); }, [] { wave_sync(); });
         }
         return;
     }
@@ -2490,7 +2516,7 @@ __global__ __launch_bounds__(256) void k_apply_scalar(Store s, OptDev o, PushSrc
             const float* gp;
             int bshow, bclick;
             if (!src_record(src, mem[j], gp, bshow, bclick)) {
-                atomicOr(&status->err, DEV_ERR_GRAD_ROWS);
+                src.no_gradient(status);
                 continue;
             }
             if (KIND == OPT_ADAGRAD) {

@@ -31,7 +31,6 @@ constexpr double MAX_LOAD = 0.75;                       // optimizer_kernel.h:26
 constexpr double RESERVE_LOAD = 0.5;                    // what a reservation is sized for where memory allows
 constexpr uint64_t DEFAULT_SLOTS = 8ull * 15485863ull;  // optimizer_kernel.h:43,263
 constexpr uint64_t MAX_SLOTS_PER_TABLE = 0xFFFFFFF0ull; // rows are addressed with 32 bits
-constexpr int PROBE_RECS_GRID = 1024;  // workgroups of k_probe_recs (measured: 512-1024 are best)
 // Below this many lookups a call keeps all its kernels on the caller's stream.  The kernels of a smaller
 // batch are too short for the overlap on the side streams to win back what the events that fork and
 // join them cost the host (measured: 106 k lookups 0.22 -> 0.17 ms per pull + push, 2.1 M 0.33 -> 0.31 ms,
@@ -138,7 +137,7 @@ struct SparseTable {
     uint32_t* hseq = nullptr;
     uint32_t seq_pull = 0, seq_verify = 0;
     bool plan_heavy = false;        // the pull that left the plan (small, or through LDS) found a sign with HEAVY_LOOKUPS lookups in a slot
-    std::vector<int64_t> plan_counts;  // distinct signs per slot of the small pull that left the plan
+    std::vector<int64_t> plan_counts;  // distinct signs per slot of the pull that left the plan
     SmallShape small_shape{};          // how that pull laid its batch out
     size_t small_lds = 0, small_emit_lds = 0;
     bool table_lds[2] = {false, false};  // k_table_apply (rows in 16-byte pieces / any) has been told how much it may have
@@ -149,13 +148,12 @@ struct SparseTable {
     uint32_t plan_big_k = BIG_GROUP_DEFAULT;  // records from which the plan lists a sign as one for k_apply_big
     bool plan_big_desc = false;               // the plan's big_desc goes with its big_list (a pull grouped through LDS)
     hipStream_t side = nullptr;     // the signs with many records are applied here, beside the others
-    hipStream_t side2 = nullptr;    // a pull probes the table here, beside the grouping of its distinct records
     // The slot descriptors of a call reach the device here while the caller's stream still runs the tail of the
     // call before (a pull's gather, a push's updates): the kernel reads pinned host memory, whose round trips
     // would otherwise stand at the head of every call.
     hipStream_t aux = nullptr;
-    hipEvent_t fork_ev = nullptr, join_ev = nullptr, join2_ev = nullptr;
-    hipEvent_t apply_ev = nullptr;  // a push's updates are done (its status is published beside what follows)
+    hipEvent_t fork_ev = nullptr, join_ev = nullptr;
+    hipEvent_t apply_ev = nullptr;  // the detached updates on the auxiliary stream are done
     // Detached updates (tn_sparse_table_set_detached_updates): the update kernels of a large push run on the
     // table's own streams and the caller's stream does not wait for them, so that whatever the caller queues next
     // -- above all the analysis of the next pull's batch, which touches no table row -- runs beside them.
@@ -174,9 +172,9 @@ struct SparseTable {
     // on that pull's plan.  Every entry point clears it (ensure_allocated); pull and push set it again.
     int flow = 0;
     hipStream_t flow_stream = nullptr;
-    bool push_pub_on_side = false;  // the pending push's status is published on the side stream
-    // A pull whose status is final before its last kernel (the gather) publishes it on the side stream
-    // meanwhile and returns when it is there: ready_ev = the status can be published,
+    bool push_on_side = false;  // the pending push's updates end on the side stream (detached)
+    // A pull whose status is final before its last kernel (the gather) publishes it by that kernel's first workgroup
+    // and returns when it is there: ready_ev = what the gather works on is complete,
     // tail_ev = the gather is done (what a call on another stream has to wait for).
     hipEvent_t ready_ev = nullptr, tail_ev = nullptr;
     bool tail_recorded = false;
@@ -341,13 +339,11 @@ int ensure_side_buffers(SparseTable* t) {
     TN_HIP(hipEventCreateWithFlags(&t->stage_ev, hipEventDisableTiming));
     TN_HIP(hipEventCreateWithFlags(&t->fork_ev, hipEventDisableTiming));
     TN_HIP(hipEventCreateWithFlags(&t->join_ev, hipEventDisableTiming));
-    TN_HIP(hipEventCreateWithFlags(&t->join2_ev, hipEventDisableTiming));
     TN_HIP(hipEventCreateWithFlags(&t->ready_ev, hipEventDisableTiming));
     TN_HIP(hipEventCreateWithFlags(&t->tail_ev, hipEventDisableTiming));
     TN_HIP(hipEventCreateWithFlags(&t->apply_ev, hipEventDisableTiming));
     TN_HIP(hipEventCreateWithFlags(&t->upd_ev, hipEventDisableTiming));
     TN_HIP(hipStreamCreateWithFlags(&t->side, hipStreamNonBlocking));  // default priority
-    TN_HIP(hipStreamCreateWithFlags(&t->side2, hipStreamNonBlocking));
     TN_HIP(hipStreamCreateWithFlags(&t->aux, hipStreamNonBlocking));
     return TN_OK;
 }
@@ -446,11 +442,11 @@ void harvest(SparseTable* t) {
     // a pending push is older than a pending pull (a push collects everything before it starts)
     if (t->push_pending) {
         t->push_pending = false;
-        if (t->push_pub_on_side) {  // its status went out on the side stream, behind its updates
-            t->push_pub_on_side = false;
+        if (t->push_on_side) {
+            t->push_on_side = false;
             const hipError_t e = hipStreamSynchronize(t->side);
             if (e != hipSuccess) latch(t, TN_ERR_HIP, std::string("sparse push: ") + hipGetErrorString(e));
-            t->upd_pending = false;  // (detached updates end on that stream, ahead of the status)
+            t->upd_pending = false;
         }
         const HostStatus& h = *t->hpush;
         int N = t->push_slots;
@@ -470,6 +466,7 @@ void harvest(SparseTable* t) {
         t->booked = 0;
         t->last_counts.assign(N, 0);
         for (int s = 0; s < N; s++) t->last_counts[s] = (int64_t)h.ubase[s + 1] - (int64_t)h.ubase[s];
+        t->plan_counts = t->last_counts;
         if (t->pull_lookups > 0) {
             note_distinct_share(t, (double)h.ubase[N] / (double)t->pull_lookups);
             if (h.st.tile_share_q16 != 0) {  // (a pull through LDS with a slot of more than one bucket)
@@ -589,7 +586,7 @@ struct Plan {
     Member* list;          // members of every group, ascending (with their show / click counts)
     uint2* where_u;        // record -> {its place in `list`, its group}
     uint32_t* big_list;    // groups with BIG_GROUP records or more
-    uint4* big_desc;       // {row, first member, records, group} of those groups (k_group_emit writes it, the other groupings do not)
+    uint4* big_desc;       // {row, first member, records, group} of those groups (emit_buckets writes it, the other groupings do not)
     uint32_t big_cap;      // entries of big_list / big_desc
     const float** gaddr;   // gradient row of every record of the groups with several records (a push fills it)
     uint64_t* vals_exact;  // copy of the signs beside their fingerprints (tn_sparse_table_set_exact_verify), else nullptr
@@ -883,7 +880,7 @@ int launch_build_plan(SparseTable* t, const Plan& p, const Scratch& w, int N, ui
     const Store& s = t->store;
     const int lblocks = launch_grid(L, 256, GRID_CAP * 2);
     const bool lds_groups = use_lds && N <= GRP_SLOTS;
-    // second-level buckets up to which k_group_emit adds up the bucket counts itself (one bucket per workgroup)
+    // second-level buckets up to which emit_buckets adds up the bucket counts itself (one bucket per workgroup)
     const bool own_offsets = w.nb2 <= (uint32_t)GRID_CAP * 4;
     if (use_lds) {
         // (as many workgroups as the chip holds of this kernel at once -- three per CU --, each taking its tiles in turn)
@@ -892,52 +889,58 @@ int launch_build_plan(SparseTable* t, const Plan& p, const Scratch& w, int N, ui
         TN_LAUNCH_LDS(k_tile_dedup, dim3(tiles), dim3(TILE_THREADS), tile_lds, st, p.descs, p.lbase, N, L, w.bcursor, w.prec,
                       reinterpret_cast<ulonglong2*>(p.vals_copy), p.vals_exact, w.first_of, ds, w.span_cap);
         if (lds_groups)
-            TN_LAUNCH_EVENT(t->one_stream ? nullptr : t->fork_ev, (k_lds_dedup<true>), dim3(launch_grid(w.nbuckets, 1, GRID_CAP * 2)),
-                            dim3(DEDUP_THREADS), st, w.bcursor, w.nbuckets, w.prec, w.first_of, w.cnt_at, ds, w.nb2, w.cursor2,
-                            w.recs);
+            TN_LAUNCH((k_lds_dedup<true>), dim3(launch_grid(w.nbuckets, 1, GRID_CAP * 2)), dim3(DEDUP_THREADS), st, w.bcursor,
+                      w.nbuckets, w.prec, w.first_of, w.cnt_at, ds, w.nb2, w.cursor2, w.recs);
         else
             TN_LAUNCH((k_lds_dedup<false>), dim3(launch_grid(w.nbuckets, 1, GRID_CAP * 2)), dim3(DEDUP_THREADS), st, w.bcursor,
                       w.nbuckets, w.prec, w.first_of, w.cnt_at, ds, w.nb2, w.cursor2, w.recs);
-        if (lds_groups) {
-            // The grouping of the distinct records only needs what the dedup handed over: it runs on
-            // the side stream beside the ranking of the first occurrences (LDS / latency bound
-            // against streaming kernels) and joins before the member lists are written.
-            const int bblocks = launch_grid(w.nb2, 1, GRID_CAP * 4);
-            hipStream_t sd = t->one_stream ? st : t->side, sd2 = t->one_stream ? st : t->side2;
-            hipEvent_t joined = t->one_stream ? nullptr : t->join_ev, joined2 = t->one_stream ? nullptr : t->join2_ev;
-            if (!t->one_stream) TN_HIP(hipStreamWaitEvent(t->side, t->fork_ev, 0));
-            if (N <= GRP_NARROW)
-                TN_LAUNCH_EVENT(own_offsets ? joined : nullptr, (k_group_count<2>), dim3(bblocks), dim3(GRP_THREADS), sd, w.nb2,
-                                w.cursor2, w.recs, big_threshold(s), w.aux, w.bcounts);
-            else
-                TN_LAUNCH_EVENT(own_offsets ? joined : nullptr, (k_group_count<4>), dim3(bblocks), dim3(GRP_THREADS), sd, w.nb2,
-                                w.cursor2, w.recs, big_threshold(s), w.aux, w.bcounts);
-            if (!own_offsets)
-                TN_LAUNCH_EVENT(joined, k_group_offsets, dim3(1), dim3(1024), sd, w.bcounts, w.bbase, w.nb2, ds);
-            // ... and so do the rows of the records' signs, on a stream of their own
-            if (!t->one_stream) TN_HIP(hipStreamWaitEvent(t->side2, t->fork_ev, 0));
-            // few workgroups: enough probes in flight for the memory system, most of every CU left to the grouping
-            TN_LAUNCH(k_probe_recs, dim3(std::min(bblocks, PROBE_RECS_GRID)), dim3(256), sd2, w.nb2, w.cursor2, w.recs, w.rrow,
-                      w.newrec, w.newcnt, s, ds);
-            const uint32_t init_parts = std::max<uint32_t>(1, (uint32_t)GRID_CAP / w.nb2);
-            TN_LAUNCH_EVENT(joined2, k_init_new_recs, dim3(launch_grid((int64_t)w.nb2 * init_parts, 1, GRID_CAP)), dim3(256), sd2,
-                            s, make_optdev(t), t->seed, w.recs, w.rrow, w.nb2, w.newrec, w.newcnt, ds, init_parts);
-        }
-        TN_LAUNCH(k_lds_flags, dim3(w.ntiles), dim3(REMAP_THREADS), st, L, w.first_of, w.flag8, w.tilesum, p.descs, N,
-                  w.bcursor, ds);
         // up to SELF_SCAN_TILES tiles the ranking pass adds up the tile counts itself
         const uint32_t* own_sums = w.ntiles <= SELF_SCAN_TILES ? w.tilesum : nullptr;
+        const size_t lb_lds = ((size_t)N + 1) * sizeof(uint32_t);
+        if (lds_groups) {
+            GroupProbeArgs ga;
+            ga.nb2 = w.nb2, ga.ntiles = w.ntiles, ga.L = L;
+            ga.cursor2 = w.cursor2;
+            ga.recs = w.recs;
+            ga.big_k = big_threshold(s);
+            ga.aux = w.aux;
+            ga.bcounts = w.bcounts;
+            ga.rrow = w.rrow, ga.newrec = w.newrec, ga.newcnt = w.newcnt;
+            ga.first_of = w.first_of;
+            ga.flag8 = w.flag8;
+            ga.tilesum = w.tilesum;
+            ga.descs = p.descs;
+            ga.N = N;
+            ga.bcursor = w.bcursor;
+            const int gblocks = launch_grid(2 * (int64_t)w.nb2 + (w.ntiles + 1) / 2 + (N + 7) / 8, 1, GRID_CAP * 16);
+            if (N <= GRP_NARROW)
+                TN_LAUNCH((k_group_probe<2>), dim3(gblocks), dim3(GRP_THREADS), st, ga, s, ds);
+            else
+                TN_LAUNCH((k_group_probe<4>), dim3(gblocks), dim3(GRP_THREADS), st, ga, s, ds);
+            if (!own_offsets) TN_LAUNCH(k_group_offsets, dim3(1), dim3(1024), st, w.bcounts, w.bbase, w.nb2, ds);
+        } else {
+            TN_LAUNCH(k_lds_flags, dim3(w.ntiles), dim3(REMAP_THREADS), st, L, w.first_of, w.flag8, w.tilesum, p.descs, N,
+                      w.bcursor, ds);
+        }
         if (!own_sums)
             TN_LAUNCH(k_scan_tiles, dim3(1), dim3(1024), st, w.tilesum, w.tileoff, w.ntiles, p.lbase, p.ubase, N, L, ds);
-        const size_t lb_lds = ((size_t)N + 1) * sizeof(uint32_t);
-        if (lds_groups)
-            TN_LAUNCH_LDS((k_lds_assign<false>), dim3(w.ntiles), dim3(REMAP_THREADS), lb_lds, st, p.descs, p.lbase, N, L,
-                          w.flag8, w.tileoff, w.cnt_at, w.wordpre, p.ubase, p.uniq_sign, p.uniq_slot, p.ushow, own_sums, ds);
-        else
+        if (lds_groups) {
+            InitArgs ia;
+            ia.seed = t->seed;
+            ia.recs = w.recs;
+            ia.rrow = w.rrow;
+            ia.nb2 = w.nb2;
+            ia.newrec = w.newrec, ia.newcnt = w.newcnt;
+            ia.parts = std::max<uint32_t>(1, (uint32_t)GRID_CAP / w.nb2);
+            const int iblocks = launch_grid((int64_t)w.nb2 * ia.parts, 1, GRID_CAP);
+            TN_LAUNCH_LDS(k_assign_init, dim3(w.ntiles + iblocks), dim3(REMAP_THREADS), lb_lds, st, p.descs, p.lbase, N, L, w.ntiles,
+                          w.flag8, w.tileoff, w.wordpre, p.ubase, own_sums, s, make_optdev(t), ia, ds);
+        } else {
             TN_LAUNCH_LDS((k_lds_assign<true>), dim3(w.ntiles), dim3(REMAP_THREADS), lb_lds, st, p.descs, p.lbase, N, L,
                           w.flag8, w.tileoff, w.cnt_at, w.wordpre, p.ubase, p.uniq_sign, p.uniq_slot, p.ushow, own_sums, ds);
-        TN_LAUNCH_LDS(k_lds_mapped, dim3(lblocks), dim3(256), lb_lds, st, p.descs, p.lbase, p.ubase, N, L, w.first_of,
-                      w.flag8, w.wordpre, p.u_of_gi);
+            TN_LAUNCH_LDS(k_lds_mapped, dim3(lblocks), dim3(256), lb_lds, st, p.descs, p.lbase, p.ubase, N, L, w.first_of,
+                          w.flag8, w.wordpre, p.u_of_gi);
+        }
     } else {
         TN_LAUNCH(k_fill_ff, dim3(launch_grid((int64_t)w.dt_entries, 256, GRID_CAP * 2)), dim3(256), st,
                   reinterpret_cast<uint4*>(w.dt), w.dt_entries);
@@ -955,10 +958,6 @@ int launch_build_plan(SparseTable* t, const Plan& p, const Scratch& w, int N, ui
     TN_TRY(order_after_updates(t, st));
     if (lds_groups) {
         const int bblocks = launch_grid(w.nb2, 1, GRID_CAP * 4);
-        if (!t->one_stream) {
-            TN_HIP(hipStreamWaitEvent(st, t->join_ev, 0));
-            TN_HIP(hipStreamWaitEvent(st, t->join2_ev, 0));
-        }
         EmitArgs<false> ea;
         ea.nb2 = w.nb2;
         ea.cursor2 = w.cursor2;
@@ -980,7 +979,10 @@ int launch_build_plan(SparseTable* t, const Plan& p, const Scratch& w, int N, ui
         ea.rrow = w.rrow;
         ea.grp_row = p.grp_row;
         ea.status = ds;
-        TN_LAUNCH_EVENT(t->one_stream ? nullptr : t->ready_ev, (k_group_emit<false>), dim3(bblocks), dim3(EMIT_THREADS), st, ea);
+        const MapArgs ma{p.descs, p.lbase, p.ubase, N, L, w.first_of, p.u_of_gi};
+        const int mblocks = launch_grid(((int64_t)L + 3) / 4, EMIT_THREADS, GRID_CAP);
+        TN_LAUNCH_LDS_EVENT(t->one_stream ? nullptr : t->ready_ev, k_emit_mapped, dim3(bblocks + mblocks), dim3(EMIT_THREADS),
+                            ((size_t)N + 1) * sizeof(uint32_t), st, ea, ma, (uint32_t)bblocks);
         t->plan_big_desc = true;
         return TN_OK;  // the rows were found beside the grouping
     } else if (N <= MASK_SLOTS)
@@ -1077,10 +1079,8 @@ int launch_apply_kind(SparseTable* t, RowShare share, const Store& s, const OptD
         TN_HIP(hipStreamWaitEvent(t->side, behind, 0));
         if (detach) TN_HIP(hipStreamWaitEvent(t->aux, behind, 0));
     }
-    // What the status of the push and the caller's stream wait for: the end of k_apply_single where that has a stream of its
-    // own, and of the last kernel on the caller's stream (detached: on the auxiliary and the side stream).
+    // the end of k_apply_single, for the caller's stream (detached: for the side stream)
     hipEvent_t single_done = detach ? t->apply_ev : forked ? t->join_ev : nullptr;
-    hipEvent_t last_done = detach || t->one_stream ? nullptr : t->apply_ev;
     if (with_big) {
         const int gfloats = big_gbuf_floats(s.D);
         const int big_blocks = launch_grid(n_upper / BIG_GROUP + 1, 1, 16384);
@@ -1104,9 +1104,9 @@ int launch_apply_kind(SparseTable* t, RowShare share, const Store& s, const OptD
     do {                                                                                                          \
         TN_LAUNCH_EVENT(single_done, (k_apply_single<KIND, LPG, ANY>), dim3(launch_grid(n_upper * LPG, 256, GRID_CAP * 4)), \
                         dim3(256), detach ? t->aux : (forked ? t->side : st), s, o, src, ds, p.grp_row, p.list);   \
-        TN_LAUNCH_EVENT(last_done, (k_apply_vec<KIND, LPG, ANY>), dim3(launch_grid(n_upper * LPG / 2, 256, GRID_CAP * 4)), \
-                        dim3(256), detach ? t->side : st, s, o, src, ds, p.grp_row, p.grp_off, p.grp_cnt, p.list,  \
-                        big_k, ids_cap, gaddr);                                                                    \
+        TN_LAUNCH((k_apply_vec<KIND, LPG, ANY>), dim3(launch_grid(n_upper * LPG / 2, 256, GRID_CAP * 4)), dim3(256), \
+                  detach ? t->side : st, s, o, src, ds, p.grp_row, p.grp_off, p.grp_cnt, p.list, big_k, ids_cap,  \
+                  gaddr);                                                                                         \
     } while (0)
 #define TN_LAUNCH_VEC(LPG)                        \
     do {                                          \
@@ -1124,8 +1124,8 @@ int launch_apply_kind(SparseTable* t, RowShare share, const Store& s, const OptD
         case 32: TN_LAUNCH_VEC(32); break;
         default:
             if (forked) TN_HIP(hipEventRecord(t->join_ev, t->side));  // (nothing of this push is there)
-            TN_LAUNCH_EVENT(last_done, (k_apply_scalar<KIND>), dim3(launch_grid(n_upper, 256, GRID_CAP * 2)), dim3(256), st, s, o,
-                            src, ds, p.grp_row, p.grp_off, p.grp_cnt, p.list, big_k, ids_cap);
+            TN_LAUNCH((k_apply_scalar<KIND>), dim3(launch_grid(n_upper, 256, GRID_CAP * 2)), dim3(256), st, s, o, src, ds,
+                      p.grp_row, p.grp_off, p.grp_cnt, p.list, big_k, ids_cap);
     }
 #undef TN_LAUNCH_VEC
 #undef TN_LAUNCH_VEC_ANY
@@ -1582,7 +1582,6 @@ int tn_sparse_table_clear(uint32_t handle) {
     // everything the table has queued, on whichever stream
     TN_HIP(hipStreamSynchronize(t->last_stream));
     TN_HIP(hipStreamSynchronize(t->side));
-    TN_HIP(hipStreamSynchronize(t->side2));
     TN_HIP(hipStreamSynchronize(t->aux));
     harvest(t);
     free_store(t->store);
@@ -2216,31 +2215,26 @@ int tn_sparse_table_pull_op(uint32_t table_handle, int N, const int64_t* const* 
         TN_TRY(launch_build_plan(t, p, w, N, (uint32_t)L, true, use_lds, st));
         // The grouping through LDS leaves the row of every distinct record in where_u itself, and the
         // call's status (counts, new rows, errors) is final before the gather starts: it is published
-        // on the side stream beside the gather, and the call returns when the host has it.  The
+        // by the gather's first workgroup, and the call returns when the host has it, through a word in pinned memory: the
+        // host prepares the push while the gather runs.  The
         // variables are complete in stream order, as the outputs of any call that takes a stream.
         const bool final_early = use_lds && N <= GRP_SLOTS && !t->async_pull;
-        const bool early = final_early && !t->one_stream;
-        // A call that keeps to the caller's stream publishes there, ahead of the gather.  Either tells the host through
-        // a word in pinned memory: the host prepares the push while the gather runs.
-        const bool early_inline = final_early && t->one_stream;
         const uint32_t seq = final_early ? ++t->seq_pull : 0;
         const uint32_t* rows_of_groups = (use_lds && N <= GRP_SLOTS) ? nullptr : p.grp_row;
-        if (early_inline)
-            TN_LAUNCH(k_publish, dim3(1), dim3(256), st, ds, p.ubase, (uint32_t)(N + 1),
-                      reinterpret_cast<uint32_t*>(t->hpull), s.count, t->hseq + 0, seq);
-        hipEvent_t tail = early || early_inline ? t->tail_ev : nullptr;
+        Publish pub{};
+        if (final_early) pub = {reinterpret_cast<uint32_t*>(t->hpull), s.count, t->hseq + 0, seq};
+        hipEvent_t tail = final_early ? t->tail_ev : nullptr;
         if (vec)
-            TN_LAUNCH_EVENT(tail, (k_gather_vars<4>), dim3(launch_grid((int64_t)L * (wdim / 4), 256, GRID_CAP * 4)), dim3(256),
-                            st, s, ds, rows_of_groups, p.where_u, p.ubase, N, p.descs);
+            TN_LAUNCH_EVENT(tail, (k_gather_vars<4>), dim3(1 + launch_grid((int64_t)L * (wdim / 4), 256, GRID_CAP * 4)), dim3(256),
+                            st, s, ds, rows_of_groups, p.where_u, p.ubase, N, p.descs, pub);
         else
-            TN_LAUNCH_EVENT(tail, (k_gather_vars<1>), dim3(launch_grid((int64_t)L * wdim, 256, GRID_CAP * 4)), dim3(256), st, s,
-                            ds, rows_of_groups, p.where_u, p.ubase, N, p.descs);
+            TN_LAUNCH_EVENT(tail, (k_gather_vars<1>), dim3(1 + launch_grid((int64_t)L * wdim, 256, GRID_CAP * 4)), dim3(256), st,
+                            s, ds, rows_of_groups, p.where_u, p.ubase, N, p.descs, pub);
         TN_HIP(hipGetLastError());
         if (tail) t->tail_recorded = true;
-        if (early) TN_HIP(hipStreamWaitEvent(t->side, t->ready_ev, 0));  // (k_group_emit's end)
-        if (!early_inline)
-            TN_LAUNCH(k_publish, dim3(1), dim3(256), early ? t->side : st, ds, p.ubase, (uint32_t)(N + 1),
-                      reinterpret_cast<uint32_t*>(t->hpull), s.count, early ? t->hseq + 0 : nullptr, seq);
+        if (!final_early)
+            TN_LAUNCH(k_publish, dim3(1), dim3(256), st, ds, p.ubase, (uint32_t)(N + 1), reinterpret_cast<uint32_t*>(t->hpull),
+                      s.count);
         t->pull_pending = true;
         t->pull_slots = N;
         t->pull_lookups = (uint64_t)L;
@@ -2257,7 +2251,7 @@ int tn_sparse_table_pull_op(uint32_t table_handle, int N, const int64_t* const* 
         if (t->async_pull) return TN_OK;
         do_host_work();
         if (final_early)
-            TN_TRY(wait_reported(t->hseq + 0, seq, early ? t->side : st, "SparseTablePull"));
+            TN_TRY(wait_reported(t->hseq + 0, seq, st, "SparseTablePull"));
         else
             TN_HIP(hipStreamSynchronize(st));
         t->stage_pending = false;
@@ -2277,15 +2271,12 @@ int tn_sparse_table_pull_op(uint32_t table_handle, int N, const int64_t* const* 
             t->latched_msg.clear();
             continue;
         }
-        if (early) {
-            t->push_pub_on_side = false;  // a push's status went out on the side stream ahead of this call's
+        if (final_early) {
             harvest(t);
-            t->flow = FLOW_PULL;
-            t->flow_stream = st;
-            return take_latched(t);
-        }
-        if (early_inline) {
-            harvest(t);
+            if (!t->one_stream) {
+                t->flow = FLOW_PULL;
+                t->flow_stream = st;
+            }
             return take_latched(t);
         }
         return sync_table(t, st);
@@ -2371,12 +2362,13 @@ int push_op_impl(uint32_t table_handle, int N, const int64_t* const* values, con
     PushSrc src{};
     hipEvent_t behind = nullptr;  // what the last kernel ahead of the updates signals, if anything
     uint32_t compared_seq = 0;    // with a plan of the last pull's: what the host waits for in hseq[1]
-    const uint32_t* pub_ubase = nullptr;  // a push on the pull's plan publishes its own copy of the distinct counts
     auto prepare_src = [&]() -> int {
         src = op_source(p, grad_dim, pd == p.push_descs);
         const HostWord compared{reuse ? t->hseq + 1 : nullptr, compared_seq};
+        uint32_t* host_err = reuse ? &t->hpush->st.err : nullptr;
         if (!pooled) {
             src.compared = compared;
+            src.host_err = host_err;
             return TN_OK;
         }
         size_t max_len = 0;
@@ -2405,7 +2397,7 @@ int push_op_impl(uint32_t table_handle, int N, const int64_t* const* values, con
         carve(c2);
         if (spread) TN_LAUNCH(k_pool_frequent, dim3((uint32_t)N), dim3(POOL_THREADS), st, p.lbase, p.ubase, p.u_of_gi, share, extra);
         TN_LAUNCH_LDS(k_lookup_keys, dim3(tiles), dim3(256), pool_tile_lds(share.lp_max), st, pd, p.lbase, p.ubase, (uint32_t)N,
-                      p.u_of_gi, batch, pool, poff, share, extra, ds, compared);
+                      p.u_of_gi, batch, pool, poff, share, extra, ds, compared, host_err);
         behind = t->one_stream ? nullptr : t->fork_ev;
         hipEvent_t reduced = spread ? nullptr : behind;
 #define TN_REDUCE(LPG, ANY)                                                                                                \
@@ -2438,7 +2430,6 @@ int push_op_impl(uint32_t table_handle, int N, const int64_t* const* values, con
         if (hoist) TN_HIP(hipStreamWaitEvent(t->aux, t->ready_ev, 0));
         TN_TRY(upload_slots(t, p.push_descs, nullptr, ds, descs, lbase, hoist ? t->aux : st, true, hoist ? t->stage_ev : nullptr,
                             STATUS_REUSE_PLAN, nullptr, 0, p.ubase, p.push_ubase, (uint32_t)(N + 1)));
-        pub_ubase = p.push_ubase;
         if (hoist) TN_HIP(hipStreamWaitEvent(st, t->stage_ev, 0));
         // On a plan with show counts the verify pass also sums the clicks; they start at zero
         // after the pull, a further push on the same plan clears them first.
@@ -2450,6 +2441,7 @@ int push_op_impl(uint32_t table_handle, int N, const int64_t* const* values, con
         compared_seq = ++t->seq_verify;
         behind = t->one_stream || pooled ? nullptr : t->fork_ev;
         t->hpush->st.mismatch = 0;
+        t->hpush->st.err = 0;
         uint32_t* host_mismatch = &t->hpush->st.mismatch;
         // op-level gradients (not pooled): the verify pass also works out the gradient addresses of the records
         // of the groups with several records (see k_member_grads)
@@ -2504,7 +2496,6 @@ int push_op_impl(uint32_t table_handle, int N, const int64_t* const* values, con
         // (its status cannot be waited for, a push only enqueues)
         t->plan_valid = false;
         ds = t->dplan;
-        pub_ubase = nullptr;
         TN_TRY(t->plan_buf.ensure(carve_plan(nullptr, p, N, L)));
         carve_plan((char*)t->plan_buf.p, p, N, L);
         pd = p.descs;
@@ -2517,24 +2508,23 @@ int push_op_impl(uint32_t table_handle, int N, const int64_t* const* values, con
         TN_TRY(launch_apply(t, p, src, ds, (int64_t)L, vec, st));
     }
     TN_HIP(hipGetLastError());
-    // The status of a large push goes out on the side stream, behind the updates and beside whatever the caller's
-    // stream runs next (a pull's status follows it on that stream, so whoever has that one has this one too).
-    const bool pub_on_side = reuse && !t->one_stream;
     const bool detached = reuse && t->detached_now;  // (the side stream is behind all update kernels already)
     t->detached_now = false;
-    if (pub_on_side && !detached) TN_HIP(hipStreamWaitEvent(t->side, t->apply_ev, 0));  // (k_apply_single is ahead on that stream)
-    TN_LAUNCH_EVENT(detached ? t->upd_ev : nullptr, k_publish, dim3(1), dim3(256), pub_on_side ? t->side : st, ds,
-                    pub_ubase ? pub_ubase : p.ubase, (uint32_t)(N + 1), reinterpret_cast<uint32_t*>(t->hpush),
-                    (unsigned long long*)nullptr, (uint32_t*)nullptr, 0u);
+    if (reuse)
+        t->last_counts = t->plan_counts;  // (its errors reach the host by themselves)
+    else
+        TN_LAUNCH(k_publish, dim3(1), dim3(256), st, ds, p.ubase, (uint32_t)(N + 1), reinterpret_cast<uint32_t*>(t->hpush),
+                  (unsigned long long*)nullptr);
     if (detached) {
+        TN_HIP(hipEventRecord(t->upd_ev, t->side));
         t->upd_pending = true;
         t->upd_N = N;
         t->upd_groups_off = (size_t)((const char*)p.grp_sign - (const char*)t->plan_buf.p);
         t->upd_slack = (size_t)((const char*)p.grp_row - (const char*)p.grp_sign);
     }
     t->push_pending = true;
-    t->push_pub_on_side = pub_on_side;
-    t->push_slots = N;
+    t->push_on_side = detached;
+    t->push_slots = reuse ? 0 : N;
     // (the reduction of pooled gradients reads the plan's slot layout until the end of the call: nothing of the
     // next pull may run beside it)
     if (reuse && !pooled) {
