@@ -34,22 +34,37 @@ __device__ __forceinline__ float combine_divisor(uint32_t n, int combiner) {
     return combiner == COMBINE_MEAN ? (float)n : sqrtf((float)n);
 }
 
-// How many of the sorted ids ex[0 .. n) lie below `x`, by a workgroup of 256 threads: every round looks at 256 places
-// of what is left, so 65 536 ids take two round trips (a binary search: sixteen).  A function of the array and x alone:
-// whatever the order of the ids, two workgroups that ask for the same x get the same answer.  sh: 5 words of LDS.
-__device__ __forceinline__ uint32_t ids_below(Global<const int64_t> ex, uint32_t n, int64_t x, uint32_t* sh) {
-    uint32_t lo = 0, len = n;  // the answer lies in [lo, lo + len]
-    while (len > 0) {
-        const uint32_t step = (len + 255) / 256;
-        const uint32_t at = threadIdx.x * step;
-        const bool below = at < len && ex[lo + at] < x;
-        const uint32_t c = block_sum_256(below ? 1u : 0u, sh);  // places below x: the first c of them, if the ids are sorted
-        if (step == 1) return lo + c;
-        if (c == 0) return lo;
-        lo += (c - 1) * step + 1;
-        len = min(step - 1, n - lo);
+// How many of the sorted ids ex[0 .. n) lie below x0 and how many below x1, by a workgroup of 256 threads: every round looks at
+// 256 places of what is left, so 65 536 ids take two round trips (a binary search: sixteen).  Either is a function of the array
+// and its x alone: whatever the order of the ids, two workgroups that ask for the same x get the same answer.  sh: 5 words of LDS.
+__device__ __forceinline__ uint2 ids_below(Global<const int64_t> ex, uint32_t n, int64_t x0, int64_t x1, uint32_t* sh) {
+    uint32_t lo[2] = {0, 0}, len[2] = {n, n};  // the answers lie in [lo, lo + len]
+    const int64_t x[2] = {x0, x1};
+    while (len[0] | len[1]) {
+        uint32_t step[2], below = 0;
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+            step[k] = (len[k] + 255) / 256;
+            const uint32_t at = threadIdx.x * step[k];
+            if (at < len[k] && ex[lo[k] + at] < x[k]) below += 1u << (16 * k);
+        }
+        const uint32_t both = block_sum_256(below, sh);  // places below x: the first c of them, if the ids are sorted
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+            const uint32_t c = both >> (16 * k) & 0xFFFFu;
+            if (len[k] == 0) continue;
+            if (step[k] == 1) {
+                lo[k] += c;
+                len[k] = 0;
+            } else if (c == 0) {
+                len[k] = 0;
+            } else {
+                lo[k] += (c - 1) * step[k] + 1;
+                len[k] = min(step[k] - 1, n - lo[k]);
+            }
+        }
     }
-    return lo;
+    return make_uint2(lo[0], lo[1]);
 }
 
 // Forward: a workgroup takes `per` examples of a slot (items of a call are numbered slot by slot): it finds their
@@ -60,16 +75,20 @@ __device__ __forceinline__ uint32_t ids_below(Global<const int64_t> ex, uint32_t
 // The example ids are checked on the way: the workgroups' shares of a slot's lookups follow each other without a gap
 // whatever the ids are (each ends where ids_below puts the start of the next, the first starts at 0, the last ends at
 // the slot's end), so every lookup is looked at by one workgroup, which wants it to lie among its examples and not
-// before its predecessor.
+// before its predecessor.  The same pass checks the mapped ids and leaves them in LDS where they fit (COMBINE_IDS): read where
+// they are used, by every lane of a group, they were a round trip in front of every example's rows.  Rows of 16, 4.9 M lookups
+// 121 -> 100 us, 860 k 29 -> 21, 20 k (104 workgroups) 7.9 -> 7.1.
 //
 // The variable rows of a slot are read again and again: every die of the chip takes a contiguous share of the items, so
-// that a slot's rows (1.3 MB at 20 k distinct signs of 16 elements) are in the L2 of the die that wants them.  By the
-// counters they are: 4.9 M lookups read 225 MB from memory where every row and id once are 206, 62 % of the requests to L2
-// hit; 121 us, 2.7 TB/s, the wavefronts wait 61 % of their cycles.
+// that a slot's rows (1.3 MB at 20 k distinct signs of 16 elements) are in the L2 of the die that wants them.  The 4.9 M lookups
+// read 225 MB and write 105 in the 100 us, 3.3 TB/s.
+constexpr uint32_t COMBINE_IDS = 2048;
+constexpr uint32_t COMBINE_AHEAD = 2;  // lookups of a thread in flight while they are checked
 template <int LPG, bool ANY>
-__global__ __launch_bounds__(256) void k_combine_fwd(const SlotDesc* __restrict__ descs, uint32_t items, uint32_t per_slot,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ANY ? 6 : 7, 8))) void k_combine_fwd(const SlotDesc* __restrict__ descs, uint32_t items, uint32_t per_slot,
                                                      uint32_t per, int dim, int64_t batch, int combiner, DevStatus* status) {
     extern __shared__ uint32_t range[];  // [per] first lookup of an example, [per] the lookup after its last
+    __shared__ uint32_t row[COMBINE_IDS];
     __shared__ uint32_t sh[5];
     const int sub = threadIdx.x % LPG;
     const DieShare share(items);
@@ -80,22 +99,46 @@ __global__ __launch_bounds__(256) void k_combine_fwd(const SlotDesc* __restrict_
         const uint32_t nb = (uint32_t)min((int64_t)per, batch - b0);
         const SlotDesc d = descs[sl];
         const Global<const int64_t> ex = example_of(d);
+        const Global<const int64_t> ids = as_global(d.values);
         for (uint32_t i = threadIdx.x; i < 2 * per; i += 256) range[i] = 0;
-        const uint32_t lo = b0 == 0 ? 0u : ids_below(ex, d.len, b0, sh);
-        const uint32_t hi = b0 + nb >= batch ? d.len : ids_below(ex, d.len, b0 + nb, sh);
+        uint32_t lo = 0, hi = d.len;
+        if (b0 > 0 || b0 + nb < batch) {
+            const uint2 bound = ids_below(ex, d.len, b0, b0 + nb, sh);
+            if (b0 > 0) lo = bound.x;
+            if (b0 + nb < batch) hi = bound.y;
+        }
+        const bool narrow = d.rows < (int64_t)NO_ROW, kept = narrow && hi - lo <= COMBINE_IDS;
         __syncthreads();
         if (hi < lo) err |= DEV_ERR_GRAD_ROWS;
-        for (uint32_t i = lo + threadIdx.x; i < hi; i += 256) {
-            const int64_t x = ex[i], prev = i > 0 ? ex[i - 1] : -1, next = i + 1 < d.len ? ex[i + 1] : batch;
-            if (x < b0 || x >= b0 + nb || prev > x) {
-                err |= DEV_ERR_GRAD_ROWS;
-                continue;
+        for (uint32_t i0 = lo + threadIdx.x; i0 < hi; i0 += 256 * COMBINE_AHEAD) {
+            int64_t x[COMBINE_AHEAD], prev[COMBINE_AHEAD], next[COMBINE_AHEAD], id[COMBINE_AHEAD];
+#pragma unroll
+            for (uint32_t q = 0; q < COMBINE_AHEAD; q++) {
+                const uint32_t i = i0 + 256 * q;
+                if (i >= hi) continue;
+                x[q] = ex[i];
+                prev[q] = i > 0 ? ex[i - 1] : -1;
+                next[q] = i + 1 < d.len ? ex[i + 1] : batch;
+                id[q] = kept ? ids[i] : 0;
             }
-            if (prev != x || i == lo) range[x - b0] = i;
-            if (next != x || i + 1 == hi) range[per + (x - b0)] = i + 1;
+#pragma unroll
+            for (uint32_t q = 0; q < COMBINE_AHEAD; q++) {
+                const uint32_t i = i0 + 256 * q;
+                if (i >= hi) continue;
+                if (kept) {
+                    const bool ok = id[q] >= 0 && id[q] < d.rows;
+                    row[i - lo] = ok ? (uint32_t)id[q] : NO_ROW;
+                    if (!ok) err |= DEV_ERR_VAR_CAPACITY;
+                }
+                if (x[q] < b0 || x[q] >= b0 + nb || prev[q] > x[q]) {
+                    err |= DEV_ERR_GRAD_ROWS;
+                    continue;
+                }
+                if (prev[q] != x[q] || i == lo) range[x[q] - b0] = i;
+                if (next[q] != x[q] || i + 1 == hi) range[per + (x[q] - b0)] = i + 1;
+            }
         }
         __syncthreads();
-        const Global<const int64_t> ids = as_global(d.values);
         const float* __restrict__ rows = d.grads;
         for (uint32_t e = threadIdx.x / LPG; e < nb; e += 256 / LPG) {
             const uint32_t from = range[e], to = max(range[per + e], from);
@@ -103,19 +146,38 @@ __global__ __launch_bounds__(256) void k_combine_fwd(const SlotDesc* __restrict_
             float* o = d.var + (b0 + e) * dim;
             for (int c0 = 0; c0 < dim; c0 += 4 * LPG) {  // (rows of more than 128 elements: once more for the next ones)
                 float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
-                // windows of COMBINE_WINDOW lookups: ids first, then their rows, all loads independent; the additions
-                // run in lookup order
+                // windows of COMBINE_WINDOW lookups, their rows' loads independent; the additions run in lookup order
                 for (uint32_t j0 = from; j0 < to; j0 += COMBINE_WINDOW) {
-                    int64_t wid[COMBINE_WINDOW];
+                    uint32_t r[COMBINE_WINDOW];
                     float4 wr[COMBINE_WINDOW];
+                    if (kept) {
 #pragma unroll
-                    for (int q = 0; q < COMBINE_WINDOW; q++) wid[q] = j0 + q < to ? ids[j0 + q] : -1;
+                        for (uint32_t q = 0; q < COMBINE_WINDOW; q++) r[q] = j0 + q < to ? row[j0 + q - lo] : NO_ROW;
+                    } else if (narrow) {
 #pragma unroll
-                    for (int q = 0; q < COMBINE_WINDOW; q++) {
-                        const bool ok = wid[q] >= 0 && wid[q] < d.rows;
-                        if (j0 + q < to && !ok) err |= DEV_ERR_VAR_CAPACITY;
-                        wr[q] = ok ? row_part<ANY>(rows + wid[q] * dim + c0, sub, dim - c0) : make_float4(0.f, 0.f, 0.f, 0.f);
+                        for (uint32_t q = 0; q < COMBINE_WINDOW; q++) {
+                            const int64_t id = j0 + q < to ? ids[j0 + q] : -1;
+                            const bool ok = id >= 0 && id < d.rows;
+                            if (j0 + q < to && !ok) err |= DEV_ERR_VAR_CAPACITY;
+                            r[q] = ok ? (uint32_t)id : NO_ROW;
+                        }
+                    } else {  // (a variable of four billion rows)
+#pragma unroll 1
+                        for (uint32_t j = j0; j < min(j0 + COMBINE_WINDOW, to); j++) {
+                            const int64_t id = ids[j];
+                            if (id < 0 || id >= d.rows) {
+                                err |= DEV_ERR_VAR_CAPACITY;
+                                continue;
+                            }
+                            const float4 v = row_part<ANY>(rows + id * dim + c0, sub, dim - c0);
+                            acc = make_float4(acc.x + v.x, acc.y + v.y, acc.z + v.z, acc.w + v.w);
+                        }
+                        continue;
                     }
+#pragma unroll
+                    for (uint32_t q = 0; q < COMBINE_WINDOW; q++)
+                        wr[q] = r[q] != NO_ROW ? row_part<ANY>(rows + (uint64_t)r[q] * dim + c0, sub, dim - c0)
+                                               : make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
                     for (int q = 0; q < COMBINE_WINDOW; q++) {
                         if (j0 + q >= to) break;

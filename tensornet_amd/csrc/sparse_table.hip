@@ -2570,6 +2570,7 @@ int tn_sparse_table_combine_op(uint32_t table_handle, int N, const int64_t* cons
     TN_TRY(ensure_allocated(t, st));
     std::vector<SlotDesc> descs(N, SlotDesc{});
     size_t L = 0;
+    int64_t max_len = 0;
     bool vec = dim % 4 == 0;
     for (int s = 0; s < N; s++) {
         if (value_lens[s] < 0 || var_rows[s] < 0 || !out[s] ||
@@ -2583,6 +2584,7 @@ int tn_sparse_table_combine_op(uint32_t table_handle, int N, const int64_t* cons
         d.rows = var_rows[s];
         d.len = (uint32_t)value_lens[s];
         L += (size_t)value_lens[s];
+        max_len = std::max<int64_t>(max_len, value_lens[s]);
         if (L > 0x7FFFFFF0ull) return fail(TN_ERR_UNSUPPORTED, "embedding combine: more than 2^31 lookups in one call");
         vec = vec && aligned16(vars[s]) && aligned16(out[s]);
     }
@@ -2594,10 +2596,13 @@ int tn_sparse_table_combine_op(uint32_t table_handle, int N, const int64_t* cons
     }
     set_last_stream(t, st);
     TN_TRY(staging_free(t));
-    // A workgroup per COMBINE_EXAMPLES examples of a slot where that does not fill the chip several times over, else per
-    // more of them: every workgroup pays for finding its lookups.
+    // A workgroup per COMBINE_EXAMPLES examples of a slot where the chip holds them all at once, else per more of them, as long
+    // as their lookups' rows fit in LDS: every workgroup pays for finding its lookups.  (211 slots of 2039 examples, 256 a
+    // workgroup 21 us, 128 25, 64 32; 100 slots of 16384: 1024, which do not fit 167, 512 100, 256 108, 128 127.)
     uint32_t per = COMBINE_EXAMPLES;
-    while (per < 1024 && (int64_t)N * ((batch + per - 1) / per) > 4096) per *= 2;
+    while (per < 512 && (int64_t)N * ((batch + per - 1) / per) > GRID_CAP &&
+           (double)max_len * (2 * per) <= 0.8 * COMBINE_IDS * (double)batch)
+        per *= 2;
     const uint32_t per_slot = (uint32_t)((batch + per - 1) / per);
     const int64_t items = (int64_t)N * per_slot;
     if (items > 0x7FFFFFF0LL) return fail(TN_ERR_UNSUPPORTED, "embedding combine: too many examples");
