@@ -124,12 +124,15 @@ static_assert(LDS_TILE < (1 << 12) && MAX_SLOTS < (1 << 12), "a tile record's fi
 //
 // The table has two entries per lookup of the tile.  The lookups of a slot own the entries [2 a, 2 b) if they sit
 // at the tile's positions [a, b): tiles that span slots (any number of them) keep the slots apart without a pass
-// per slot.  The last entry of a slot's range belongs to the sign that equals EMPTY_KEY; the others are filled by
-// linear probing.  The lookup that turns out to be its sign's first in the tile hands the record on: it holds the
+// per slot.  They are filled by linear probing.  An entry names a position of its sign, not the sign, which stands in LDS once
+// for every lookup.  The lookup that turns out to be its sign's first in the tile hands the record on: it holds the
 // sign and its hash in registers already, so the table is never walked (most of its entries are free, and a walk
 // pays for every one of them).  Places in the buckets: an LDS counter per bucket the tile can touch gives a
 // record its place among the tile's records for the bucket, one global atomic per touched bucket reserves the
 // tile's slice of it.
+//
+// 33 KB of LDS and 64 registers: four workgroups to a CU.  (With the signs as the table's keys, 49 KB, three: 4.9 M lookups of 100
+// slots 48.6 us, so 44.6; 2.1 M of 64 20.5 and 17.9, a round of workgroups instead of one and a third.)
 //
 // It also leaves the fingerprints of the batch's signs, which a push compares its own with (k_verify_values: one
 // per 64 strided lookups of a tile of 256 x 8, which are the lookups of the wavefronts w and w + 4 here), and,
@@ -143,7 +146,7 @@ inline size_t tile_dedup_lds(int N, uint32_t span_cap) {
     const size_t lb = align_up(((size_t)N + 1) * sizeof(uint32_t), 8);
     return (N <= TILE_LDS_SLOTS ? lb + (size_t)N * (sizeof(uint64_t) + sizeof(uint2)) : lb) + (size_t)span_cap * sizeof(uint32_t);
 }
-static __global__ __launch_bounds__(TILE_THREADS) __attribute__((amdgpu_waves_per_eu(6, 8))) void k_tile_dedup(const SlotDesc* __restrict__ descs,
+static __global__ __launch_bounds__(TILE_THREADS) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_tile_dedup(const SlotDesc* __restrict__ descs,
                                                              const uint32_t* __restrict__ lbase, int N, uint32_t L,
                                                              uint32_t* bcursor, ulonglong2* __restrict__ prec,
                                                              ulonglong2* __restrict__ prints,
@@ -151,8 +154,9 @@ static __global__ __launch_bounds__(TILE_THREADS) __attribute__((amdgpu_waves_pe
                                                              uint32_t* __restrict__ first_of, DevStatus* status,
                                                              uint32_t span_cap) {
     extern __shared__ uint32_t lb[];  // lb[N + 1], sized by the launch; then vals[N], tb[N], hist[span_cap] (see tile_dedup_lds)
-    __shared__ unsigned long long keys[TILE_TABLE];
-    __shared__ uint32_t word[TILE_TABLE];  // bits 16-31 smallest position in the tile, 0-15 occurrences
+    __shared__ uint64_t signs[LDS_TILE];
+    __shared__ uint32_t word[TILE_TABLE];  // bits 16-31 a position of the entry's sign, at last the smallest, 0-15 its occurrences
+    constexpr uint32_t FREE = 0xFFFF0000u;
     __shared__ ulonglong2 fp[TILE_THREADS / 64];
     // With few slots everything a tile needs of its slots' descriptors comes in with the slots' first lookups, in
     // one round trip, instead of in a second one once the tile knows its slot.
@@ -204,11 +208,10 @@ static __global__ __launch_bounds__(TILE_THREADS) __attribute__((amdgpu_waves_pe
             span = bl.x + bl.y - b0.x;
         }
         span = min(span, span_cap);
-        for (int i = threadIdx.x; i < TILE_TABLE; i += TILE_THREADS) {
-            keys[i] = EMPTY_KEY;
-            word[i] = 0xFFFF0000u;
-        }
+        for (int i = threadIdx.x; i < TILE_TABLE; i += TILE_THREADS) word[i] = FREE;
         for (uint32_t i = threadIdx.x; i < span; i += TILE_THREADS) hist[i] = 0;
+#pragma unroll
+        for (int j = 0; j < TILE_ITEMS; j++) signs[j * TILE_THREADS + threadIdx.x] = sg[j];
         // the hash of every sign once: fingerprint, place in the table, bucket
         uint32_t hs[TILE_ITEMS];
         {
@@ -242,17 +245,17 @@ static __global__ __launch_bounds__(TILE_THREADS) __attribute__((amdgpu_waves_pe
                 a = max(lb[sl[j]], g0) - g0;
                 m = min(lb[sl[j] + 1], g1 + 1) - g0 - a;
             }
-            const uint32_t lo = 2 * a, size = 2 * m - 1;
-            uint32_t e = lo + size;  // the entry of the sign EMPTY_KEY
-            if (sg[j] != EMPTY_KEY) {
-                e = lo + scale32(hs[j], size);
-                for (;;) {  // at most m distinct signs in 2 m - 1 entries: a free one exists
-                    const unsigned long long old = atomicCAS(&keys[e], (unsigned long long)EMPTY_KEY, sg[j]);
-                    if (old == EMPTY_KEY || old == sg[j]) break;
-                    e = (e + 1 == lo + size) ? lo : e + 1;
+            const uint32_t lo = 2 * a, size = 2 * m;
+            uint32_t e = lo + scale32(hs[j], size);
+            for (;;) {  // at most m distinct signs in 2 m entries: a free one exists
+                const uint32_t old = atomicCAS(&word[e], FREE, pos << 16);
+                if (old == FREE) break;
+                if (signs[old >> 16] == sg[j]) {
+                    if (old > pos << 16) atomicMin(&word[e], pos << 16);
+                    break;
                 }
+                e = (e + 1 == lo + size) ? lo : e + 1;
             }
-            atomicMin(&word[e], pos << 16);
             ent[j] = e;
         }
         __syncthreads();

@@ -38,7 +38,7 @@ constexpr uint64_t MAX_SLOTS_PER_TABLE = 0xFFFFFFF0ull; // rows are addressed wi
 constexpr size_t ONE_STREAM_LOOKUPS = 3u << 20;
 constexpr uint32_t SELF_SCAN_TILES = 8192;  // tiles of the ranking pass up to which no scan kernel runs between its launches
 constexpr int GRID_CAP = 256 * 8;                       // 256 CUs x 8 workgroups of 256 threads
-constexpr int TILE_GRID = 256 * 3;                      // workgroups of k_tile_dedup: what the chip holds of it at once
+constexpr int TILE_GRID = 256 * 4;                      // workgroups of k_tile_dedup: what the chip holds of it at once
 constexpr size_t PULL_WORDS = std::max<size_t>(SMALL_WORKGROUPS, TABLE_PULL_WORDS);
 constexpr uint32_t COMBINE_EXAMPLES = 64;  // examples per workgroup of k_combine_fwd at least
 constexpr int COMBINE_DIRECT = 1024;       // workgroups of it up to which they read the slots' descriptors from pinned host memory
@@ -883,7 +883,7 @@ int launch_build_plan(SparseTable* t, const Plan& p, const Scratch& w, int N, ui
     // second-level buckets up to which emit_buckets adds up the bucket counts itself (one bucket per workgroup)
     const bool own_offsets = w.nb2 <= (uint32_t)GRID_CAP * 4;
     if (use_lds) {
-        // (as many workgroups as the chip holds of this kernel at once -- three per CU --, each taking its tiles in turn)
+        // (as many workgroups as the chip holds of this kernel at once -- four per CU --, each taking its tiles in turn)
         const int tiles = launch_grid((int64_t)(L + LDS_TILE - 1) / LDS_TILE, 1, TILE_GRID);
         const size_t tile_lds = tile_dedup_lds(N, w.span_cap);
         TN_LAUNCH_LDS(k_tile_dedup, dim3(tiles), dim3(TILE_THREADS), tile_lds, st, p.descs, p.lbase, N, L, w.bcursor, w.prec,
