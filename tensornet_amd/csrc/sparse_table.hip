@@ -31,11 +31,12 @@ constexpr double MAX_LOAD = 0.75;                       // optimizer_kernel.h:26
 constexpr double RESERVE_LOAD = 0.5;                    // what a reservation is sized for where memory allows
 constexpr uint64_t DEFAULT_SLOTS = 8ull * 15485863ull;  // optimizer_kernel.h:43,263
 constexpr uint64_t MAX_SLOTS_PER_TABLE = 0xFFFFFFF0ull; // rows are addressed with 32 bits
-// Below this many lookups a call keeps all its kernels on the caller's stream.  The kernels of a smaller
-// batch are too short for the overlap on the side streams to win back what the events that fork and
-// join them cost the host (measured: 106 k lookups 0.22 -> 0.17 ms per pull + push, 2.1 M 0.33 -> 0.31 ms,
-// 5 M 0.67 -> 0.71 ms).
-constexpr size_t ONE_STREAM_LOOKUPS = 3u << 20;
+constexpr size_t DETACH_LOOKUPS = 3u << 20;  // lookups of a push from which its updates may be detached
+// A batch of as many lookups whose slots have every sign some hundred times has the signs with many records in a launch of their
+// own (k_apply_big_adagrad, which detached updates use): tests/test_gpu_big_groups.py counts on it there.  The one launch for
+// all signs would do: 3.2 M lookups of 70 slots over 300 signs, rows of 16, a step 132 us, with a launch of their own 139; 3.5 M
+// of 88 slots over 2000 signs 188 and 196, over 250 k (not such a batch) 567 and 582.
+constexpr uint64_t OWN_BIG_LOOKUPS = 256;
 constexpr uint32_t SELF_SCAN_TILES = 8192;  // tiles of the ranking pass up to which no scan kernel runs between its launches
 constexpr int GRID_CAP = 256 * 8;                       // 256 CUs x 8 workgroups of 256 threads
 constexpr int TILE_GRID = 256 * 4;                      // workgroups of k_tile_dedup: what the chip holds of it at once
@@ -86,8 +87,6 @@ constexpr int SMALL_SPLIT_SLOTS = 8;  // (up to as many, slots are short, too: s
 // Parts of rows from which a thread of small_finish takes two: up to here more workgroups are the shorter way.
 constexpr size_t FINISH_FULL = 1 << 17;
 constexpr size_t SMALL_SHARED_LDS = 36 * 1024;
-
-enum { FLOW_NONE = 0, FLOW_PULL = 1, FLOW_PUSH = 2 };
 
 struct HostStatus {
     DevStatus st;
@@ -147,12 +146,10 @@ struct SparseTable {
     bool plan_exact = false;   // the plan holds such a copy
     uint32_t plan_big_k = BIG_GROUP_DEFAULT;  // records from which the plan lists a sign as one for k_apply_big
     bool plan_big_desc = false;               // the plan's big_desc goes with its big_list (a pull grouped through LDS)
-    hipStream_t side = nullptr;     // the signs with many records are applied here, beside the others
-    // The slot descriptors of a call reach the device here while the caller's stream still runs the tail of the
-    // call before (a pull's gather, a push's updates): the kernel reads pinned host memory, whose round trips
-    // would otherwise stand at the head of every call.
-    hipStream_t aux = nullptr;
-    hipEvent_t fork_ev = nullptr, join_ev = nullptr;
+    bool plan_frequent = false;               // the plan's records have OWN_BIG_LOOKUPS lookups or more on average
+    hipStream_t side = nullptr;     // the signs with several records of detached updates are applied here
+    hipStream_t aux = nullptr;      // k_apply_single of detached updates runs here
+    hipEvent_t fork_ev = nullptr;   // detached updates may start
     hipEvent_t apply_ev = nullptr;  // the detached updates on the auxiliary stream are done
     // Detached updates (tn_sparse_table_set_detached_updates): the update kernels of a large push run on the
     // table's own streams and the caller's stream does not wait for them, so that whatever the caller queues next
@@ -167,18 +164,11 @@ struct SparseTable {
     // and the groups from upd_groups_off on, less the first upd_slack bytes (the groups' signs, which they leave alone)
     int upd_N = 0;
     size_t upd_groups_off = 0, upd_slack = 0;
-    // The call before this one on the table, if it left work behind on `flow_stream` that the next call of the
-    // training loop may overlap with: FLOW_PULL = a pull that returned before its gather, FLOW_PUSH = a push
-    // on that pull's plan.  Every entry point clears it (ensure_allocated); pull and push set it again.
-    int flow = 0;
-    hipStream_t flow_stream = nullptr;
     bool push_on_side = false;  // the pending push's updates end on the side stream (detached)
     // A pull whose status is final before its last kernel (the gather) publishes it by that kernel's first workgroup
-    // and returns when it is there: ready_ev = what the gather works on is complete,
-    // tail_ev = the gather is done (what a call on another stream has to wait for).
-    hipEvent_t ready_ev = nullptr, tail_ev = nullptr;
+    // and returns when it is there: tail_ev = the gather is done (what a call on another stream has to wait for).
+    hipEvent_t tail_ev = nullptr;
     bool tail_recorded = false;
-    bool one_stream = false;        // the running call is small: its kernels all go to the caller's stream
     bool plan_clicks_dirty = false;  // a push has added clicks to the member lists of the current plan
     // Distinct records per lookup seen by the recent pulls (1 = every lookup distinct, the safe start):
     // sizes the number of second-level buckets, whose room is fixed.  A batch with more distinct
@@ -338,8 +328,6 @@ int ensure_side_buffers(SparseTable* t) {
     TN_HIP(hipHostMalloc((void**)&t->hstage, t->hstage_bytes, hipHostMallocDefault));
     TN_HIP(hipEventCreateWithFlags(&t->stage_ev, hipEventDisableTiming));
     TN_HIP(hipEventCreateWithFlags(&t->fork_ev, hipEventDisableTiming));
-    TN_HIP(hipEventCreateWithFlags(&t->join_ev, hipEventDisableTiming));
-    TN_HIP(hipEventCreateWithFlags(&t->ready_ev, hipEventDisableTiming));
     TN_HIP(hipEventCreateWithFlags(&t->tail_ev, hipEventDisableTiming));
     TN_HIP(hipEventCreateWithFlags(&t->apply_ev, hipEventDisableTiming));
     TN_HIP(hipEventCreateWithFlags(&t->upd_ev, hipEventDisableTiming));
@@ -392,7 +380,6 @@ int ensure_allocated(SparseTable* t, hipStream_t st, bool beside_updates = false
     TN_TRY(ensure_side_buffers(t));
     if (!beside_updates) TN_TRY(order_after_updates(t, st));
     TN_TRY(order_after_other_stream(t, st));
-    t->flow = FLOW_NONE;  // pull and push read it before they get here and set it again
     if (t->allocated) return TN_OK;
     uint64_t cap = DEFAULT_SLOTS;
     if (t->reserve_keys) cap = reserved_slots(t, t->reserve_keys);
@@ -467,6 +454,7 @@ void harvest(SparseTable* t) {
         t->last_counts.assign(N, 0);
         for (int s = 0; s < N; s++) t->last_counts[s] = (int64_t)h.ubase[s + 1] - (int64_t)h.ubase[s];
         t->plan_counts = t->last_counts;
+        t->plan_frequent = t->pull_lookups >= OWN_BIG_LOOKUPS * h.ubase[N];
         if (t->pull_lookups > 0) {
             note_distinct_share(t, (double)h.ubase[N] / (double)t->pull_lookups);
             if (h.st.tile_share_q16 != 0) {  // (a pull through LDS with a slot of more than one bucket)
@@ -800,23 +788,21 @@ int staging_free(SparseTable* t) {
 }
 
 // Slot descriptors to the device (dst_descs; the slots' first lookups to dst_lbase unless nullptr); the same
-// launch prepares the call's status block `ds` (status_mode) and clears `zero[0 .. n_zero)`.  It runs on `run_on`.
+// launch prepares the call's status block `ds` (status_mode) and clears `zero[0 .. n_zero)`.
 // waited: the caller waits for something behind it, and then says that the staging buffer is free; else an event says so.
-// joined: an event for other streams to wait for.
 int upload_slots(SparseTable* t, SlotDesc* dst_descs, uint32_t* dst_lbase, DevStatus* ds,
-                 const std::vector<SlotDesc>& descs, const std::vector<uint32_t>& lbase, hipStream_t run_on,
-                 bool waited, hipEvent_t joined, int status_mode, uint32_t* zero = nullptr, uint32_t n_zero = 0,
+                 const std::vector<SlotDesc>& descs, const std::vector<uint32_t>& lbase, hipStream_t st,
+                 bool waited, int status_mode, uint32_t* zero = nullptr, uint32_t n_zero = 0,
                  const uint32_t* copy_src = nullptr, uint32_t* copy_dst = nullptr, uint32_t copy_n = 0) {
     TN_TRY(staging_free(t));
     const size_t db = descs.size() * sizeof(SlotDesc);
     const size_t lb = dst_lbase ? lbase.size() * sizeof(uint32_t) : 0;
     std::memcpy(t->hstage, descs.data(), db);
     if (lb) std::memcpy(t->hstage + db, lbase.data(), lb);
-    TN_LAUNCH_EVENT(joined, k_stage_in, dim3(launch_grid((int64_t)std::max<size_t>((db + lb) / 4, n_zero), 256, 64)),
-                    dim3(256), run_on, reinterpret_cast<const uint32_t*>(t->hstage), reinterpret_cast<uint32_t*>(dst_descs),
-                    (uint32_t)(db / 4), dst_lbase, (uint32_t)(lb / 4), ds, status_mode, zero, n_zero,
-                    (const DevStatus*)t->dplan, copy_src, copy_dst, copy_n);
-    if (!waited) TN_HIP(hipEventRecord(t->stage_ev, run_on));
+    TN_LAUNCH(k_stage_in, dim3(launch_grid((int64_t)std::max<size_t>((db + lb) / 4, n_zero), 256, 64)), dim3(256), st,
+              reinterpret_cast<const uint32_t*>(t->hstage), reinterpret_cast<uint32_t*>(dst_descs), (uint32_t)(db / 4), dst_lbase,
+              (uint32_t)(lb / 4), ds, status_mode, zero, n_zero, (const DevStatus*)t->dplan, copy_src, copy_dst, copy_n);
+    if (!waited) TN_HIP(hipEventRecord(t->stage_ev, st));
     t->stage_recorded = !waited;
     t->stage_pending = true;
     return TN_OK;
@@ -981,8 +967,8 @@ int launch_build_plan(SparseTable* t, const Plan& p, const Scratch& w, int N, ui
         ea.status = ds;
         const MapArgs ma{p.descs, p.lbase, p.ubase, N, L, w.first_of, p.u_of_gi};
         const int mblocks = launch_grid(((int64_t)L + 3) / 4, EMIT_THREADS, GRID_CAP);
-        TN_LAUNCH_LDS_EVENT(t->one_stream ? nullptr : t->ready_ev, k_emit_mapped, dim3(bblocks + mblocks), dim3(EMIT_THREADS),
-                            ((size_t)N + 1) * sizeof(uint32_t), st, ea, ma, (uint32_t)bblocks);
+        TN_LAUNCH_LDS(k_emit_mapped, dim3(bblocks + mblocks), dim3(EMIT_THREADS), ((size_t)N + 1) * sizeof(uint32_t), st, ea, ma,
+                      (uint32_t)bblocks);
         t->plan_big_desc = true;
         return TN_OK;  // the rows were found beside the grouping
     } else if (N <= MASK_SLOTS)
@@ -1001,16 +987,14 @@ int launch_build_plan(SparseTable* t, const Plan& p, const Scratch& w, int N, ui
 // workgroups of k_apply_all for the signs with many records at most (a wavefront each in turn)
 constexpr int ALL_BIG_GRID = 1024;
 
-// The three kernels touch disjoint rows (a batch that keeps to one stream has them in one launch, k_apply_all).
-// k_apply_single saturates the memory system (it runs
-// at the device's rate for random row updates); k_apply_big and k_apply_vec are bound by
-// dependent chains and instruction issue, so they run one after the other beside it.  The pair is
-// the longer chain: it stays on the caller's stream and k_apply_single goes to the table's side
-// stream, forked from and joined back into the caller's stream by events (a kernel that waits for
-// an event of another stream starts 15-30 us late: better the chain that has the time to spare).
+// The signs with many records, with a few and with one: one launch (k_apply_all) where a row fits the lanes of a wavefront half.
+// Above 3 M lookups they were three launches on two streams until the pull needed no second stream: 4.9 M of 100 slots, rows of
+// 16, a step 527 us and 516 as one launch, with pooled gradients 881 and 856; 3.2 M of 70 slots over 300 signs 168 and 132;
+// 3.5 M of 88 over 250 k, rows of 64, 1107 and 1132, the only batch found that loses.
 //
-// detach: none of them on the caller's stream, which does not wait for them either -- k_apply_single on the
-// auxiliary stream; the caller of this function records their end (see SparseTable::upd_ev).
+// detach: the three kernels one by one on streams of the table's own, which the caller's does not wait for -- k_apply_single on
+// the auxiliary stream, the others on the side stream; the caller of this function records their end (SparseTable::upd_ev).
+// `behind`: an event that the last kernel on `st` signals.
 template <int KIND>
 int launch_apply_kind(SparseTable* t, RowShare share, const Store& s, const OptDev& o, const PushSrc& src, DevStatus* ds,
                       const Plan& p, int64_t n_upper, hipStream_t st, bool addr_ready, uint32_t big_k, bool detach,
@@ -1018,19 +1002,47 @@ int launch_apply_kind(SparseTable* t, RowShare share, const Store& s, const OptD
     const uint32_t ids_cap = (uint32_t)n_upper;
     const bool with_big = big_k != 0xFFFFFFFFu;
     const float* const* gaddr = (with_big && !src.infos && !src.flat) ? p.gaddr : nullptr;
-    detach = detach && !t->one_stream && share.lanes != 0;
+    detach = detach && share.lanes != 0;
     t->detached_now = detach;
-    const bool forked = (with_big || detach) && !t->one_stream;
     // op-level gradients: their addresses for the records of the groups with several records, once, in a
     // coalesced pass ahead of everything (beside k_apply_single it would take several times as long)
     if (with_big && gaddr && !addr_ready) {
-        behind = forked ? t->fork_ev : nullptr;
+        behind = detach ? t->fork_ev : nullptr;
         TN_LAUNCH_EVENT(behind, k_member_grads, dim3(launch_grid(n_upper, 256, GRID_CAP * 2)), dim3(256), st, src, ds, p.list,
                         p.gaddr, ids_cap);
     }
-    if (with_big && t->one_stream && share.lanes != 0) {
+    if (detach) {
+        if (!behind) {
+            behind = t->fork_ev;
+            TN_HIP(hipEventRecord(behind, st));
+        }
+        TN_HIP(hipStreamWaitEvent(t->side, behind, 0));
+        TN_HIP(hipStreamWaitEvent(t->aux, behind, 0));
+    }
+    // AdaGrad rows of a power-of-two dim on a plan that describes its frequent signs have kernels of their own
+    const bool tiled = KIND == OPT_ADAGRAD && big_desc && s.D >= 4 && s.D <= 64 && (s.D & (s.D - 1)) == 0;
+    const bool all = with_big && !detach && share.lanes != 0;
+    const bool own_big = with_big && (!all || (tiled && t->plan_frequent && (size_t)n_upper >= DETACH_LOOKUPS));
+    if (own_big) {
+        const int gfloats = big_gbuf_floats(s.D);
+        const int big_blocks = launch_grid(n_upper / BIG_GROUP + 1, 1, 16384);
+        hipStream_t bst = detach ? t->side : st;
+#define TN_LAUNCH_BIG_ADAGRAD(DIM)                                                                                  \
+    TN_LAUNCH((k_apply_big_adagrad<DIM>), dim3(big_blocks), dim3(64), bst, s, o, src, ds, (const uint4*)p.big_desc, \
+              p.big_cap, p.list, gaddr)
+        if (tiled && s.D == 4) TN_LAUNCH_BIG_ADAGRAD(4);
+        else if (tiled && s.D == 8) TN_LAUNCH_BIG_ADAGRAD(8);
+        else if (tiled && s.D == 16) TN_LAUNCH_BIG_ADAGRAD(16);
+        else if (tiled && s.D == 32) TN_LAUNCH_BIG_ADAGRAD(32);
+        else if (tiled && s.D == 64) TN_LAUNCH_BIG_ADAGRAD(64);
+        else
+            TN_LAUNCH_LDS((k_apply_big<KIND>), dim3(big_blocks), dim3(64), big_lds_bytes(s.D), bst, s, o, src, ds,
+                          p.big_list, p.grp_row, p.grp_off, p.grp_cnt, p.list, gfloats, gaddr);
+#undef TN_LAUNCH_BIG_ADAGRAD
+    }
+    if (all) {
         ApplyAll a;
-        a.big_blocks = (uint32_t)launch_grid((n_upper / BIG_GROUP + 4) / 4, 1, ALL_BIG_GRID);
+        a.big_blocks = own_big ? 0 : (uint32_t)launch_grid((n_upper / BIG_GROUP + 4) / 4, 1, ALL_BIG_GRID);
         a.multi_blocks = (uint32_t)launch_grid(n_upper * share.lanes / 2, 256, GRID_CAP * 2);
         const uint32_t singles = (uint32_t)launch_grid(n_upper * share.lanes, 256, GRID_CAP * 2);
         a.grp_row = p.grp_row, a.grp_off = p.grp_off, a.grp_cnt = p.grp_cnt, a.big_list = p.big_list;
@@ -1041,8 +1053,6 @@ int launch_apply_kind(SparseTable* t, RowShare share, const Store& s, const OptD
         a.gbuf_floats = std::min(big_gbuf_floats(s.D), ALL_GBUF);
         a.wave_arrays = (uint32_t)align_up((size_t)(a.gbuf_floats + 3 * s.D) * sizeof(float), 8);
         a.wave_lds = a.wave_arrays + BIG_CHUNK * (8 + 4);
-        // AdaGrad rows of a power-of-two dim on a plan that describes its frequent signs have kernels of their own
-        const bool tiled = KIND == OPT_ADAGRAD && big_desc && s.D == 4 * share.lanes && s.D <= 64;
 #define TN_LAUNCH_ALL_ANY(LPG, ANY)                                                                                        \
     do {                                                                                                                   \
         constexpr int TILE = KIND == OPT_ADAGRAD && LPG <= 16 ? 4 * LPG : 0;                                               \
@@ -1071,39 +1081,11 @@ int launch_apply_kind(SparseTable* t, RowShare share, const Store& s, const OptD
 #undef TN_LAUNCH_ALL_ANY
         return TN_OK;
     }
-    if (forked) {
-        if (!behind) {
-            behind = t->fork_ev;
-            TN_HIP(hipEventRecord(behind, st));
-        }
-        TN_HIP(hipStreamWaitEvent(t->side, behind, 0));
-        if (detach) TN_HIP(hipStreamWaitEvent(t->aux, behind, 0));
-    }
-    // the end of k_apply_single, for the caller's stream (detached: for the side stream)
-    hipEvent_t single_done = detach ? t->apply_ev : forked ? t->join_ev : nullptr;
-    if (with_big) {
-        const int gfloats = big_gbuf_floats(s.D);
-        const int big_blocks = launch_grid(n_upper / BIG_GROUP + 1, 1, 16384);
-        hipStream_t bst = detach ? t->side : st;
-#define TN_LAUNCH_BIG_ADAGRAD(DIM)                                                                                  \
-    TN_LAUNCH((k_apply_big_adagrad<DIM>), dim3(big_blocks), dim3(64), bst, s, o, src, ds, (const uint4*)p.big_desc, \
-              p.big_cap, p.list, gaddr)
-        // AdaGrad rows of a power-of-two dim on a plan that describes its frequent signs: the kernel made for them
-        const bool tiled = KIND == OPT_ADAGRAD && big_desc;
-        if (tiled && s.D == 4) TN_LAUNCH_BIG_ADAGRAD(4);
-        else if (tiled && s.D == 8) TN_LAUNCH_BIG_ADAGRAD(8);
-        else if (tiled && s.D == 16) TN_LAUNCH_BIG_ADAGRAD(16);
-        else if (tiled && s.D == 32) TN_LAUNCH_BIG_ADAGRAD(32);
-        else if (tiled && s.D == 64) TN_LAUNCH_BIG_ADAGRAD(64);
-        else
-            TN_LAUNCH_LDS((k_apply_big<KIND>), dim3(big_blocks), dim3(64), big_lds_bytes(s.D), bst, s, o, src, ds,
-                          p.big_list, p.grp_row, p.grp_off, p.grp_cnt, p.list, gfloats, gaddr);
-#undef TN_LAUNCH_BIG_ADAGRAD
-    }
 #define TN_LAUNCH_VEC_ANY(LPG, ANY)                                                                                \
     do {                                                                                                          \
-        TN_LAUNCH_EVENT(single_done, (k_apply_single<KIND, LPG, ANY>), dim3(launch_grid(n_upper * LPG, 256, GRID_CAP * 4)), \
-                        dim3(256), detach ? t->aux : (forked ? t->side : st), s, o, src, ds, p.grp_row, p.list);   \
+        TN_LAUNCH_EVENT(detach ? t->apply_ev : nullptr, (k_apply_single<KIND, LPG, ANY>),                          \
+                        dim3(launch_grid(n_upper * LPG, 256, GRID_CAP * 4)), dim3(256), detach ? t->aux : st, s, o, src, ds, \
+                        p.grp_row, p.list);                                                                       \
         TN_LAUNCH((k_apply_vec<KIND, LPG, ANY>), dim3(launch_grid(n_upper * LPG / 2, 256, GRID_CAP * 4)), dim3(256), \
                   detach ? t->side : st, s, o, src, ds, p.grp_row, p.grp_off, p.grp_cnt, p.list, big_k, ids_cap,  \
                   gaddr);                                                                                         \
@@ -1123,13 +1105,11 @@ int launch_apply_kind(SparseTable* t, RowShare share, const Store& s, const OptD
         case 16: TN_LAUNCH_VEC(16); break;
         case 32: TN_LAUNCH_VEC(32); break;
         default:
-            if (forked) TN_HIP(hipEventRecord(t->join_ev, t->side));  // (nothing of this push is there)
             TN_LAUNCH((k_apply_scalar<KIND>), dim3(launch_grid(n_upper, 256, GRID_CAP * 2)), dim3(256), st, s, o, src, ds,
                       p.grp_row, p.grp_off, p.grp_cnt, p.list, big_k, ids_cap);
     }
 #undef TN_LAUNCH_VEC
 #undef TN_LAUNCH_VEC_ANY
-    if (forked && !detach) TN_HIP(hipStreamWaitEvent(st, t->join_ev, 0));
     return TN_OK;
 }
 
@@ -1137,7 +1117,6 @@ int launch_apply_kind(SparseTable* t, RowShare share, const Store& s, const OptD
 // addr_ready: p.gaddr already holds the gradient addresses of the multi-record groups' records.
 // big_k: the number of records from which the plan's grouping listed a sign for k_apply_big (0: the table's default).
 // big_desc: p.big_desc describes the signs of p.big_list (the plan of a pull that grouped through LDS).
-// behind: an event that the last kernel on `st` signals, if it signals one.
 int launch_apply(SparseTable* t, const Plan& p, const PushSrc& src, DevStatus* ds, int64_t n_upper, bool vec_ok,
                  hipStream_t st, bool addr_ready = false, uint32_t big_k = 0, bool detach = false, bool big_desc = false,
                  hipEvent_t behind = nullptr) {
@@ -1592,7 +1571,6 @@ int tn_sparse_table_clear(uint32_t handle) {
     t->allocated = false;
     t->plan_valid = false;
     t->tail_recorded = false;
-    t->flow = FLOW_NONE;
     t->count_upper = 0;
     t->booked = 0;
     t->epoch++;
@@ -1807,7 +1785,6 @@ int tn_sparse_table_pull_static(uint32_t handle, const uint64_t* signs, int64_t 
     // the prologue every entry point shares (ensure_allocated), less the allocation
     TN_TRY(order_after_updates(t, st));
     TN_TRY(order_after_other_stream(t, st));
-    t->flow = FLOW_NONE;
     const int wdim = t->dim + (t->use_cvm ? 2 : 0);
     if (dim != wdim)
         return fail(TN_ERR_DIM_MISMATCH, "tn_sparse_table_pull_static: dim " + std::to_string(dim) +
@@ -2119,8 +2096,6 @@ int tn_sparse_table_pull_op(uint32_t table_handle, int N, const int64_t* const* 
     if (!vars || !var_rows || !mapped_values) return fail(TN_ERR_INVALID_ARGUMENT, "SparseTablePull: NULL argument");
     std::lock_guard<std::mutex> lk(t->mu);
     hipStream_t st = (hipStream_t)stream;
-    // the call before was a push on the last pull's plan, on this stream: its updates may still be running
-    bool behind_push = t->flow == FLOW_PUSH && t->flow_stream == st;
     // (detached updates of the push before: the analysis of this call's batch runs beside them; the stream is
     // ordered behind them where the call first touches what they read or write)
     TN_TRY(ensure_allocated(t, st, true));
@@ -2146,7 +2121,6 @@ int tn_sparse_table_pull_op(uint32_t table_handle, int N, const int64_t* const* 
         for (int s = 0; s < N; s++)
             if (var_rows[s] < 0 || !vars[s] || (value_lens[s] > 0 && (!values[s] || !mapped_values[s])))
                 return fail(TN_ERR_INVALID_ARGUMENT, "SparseTablePull: bad tensors of slot " + std::to_string(s));
-        t->one_stream = true;
         TN_TRY(ensure_room(t, (uint64_t)shape.L, st));
         return small_pull(t, shape, values, value_lens, vars, var_rows, wdim, mapped_values, st);
     }
@@ -2172,7 +2146,6 @@ int tn_sparse_table_pull_op(uint32_t table_handle, int N, const int64_t* const* 
             t->last_counts.assign(N, 0);
             return take_latched(t);
         }
-        t->one_stream = L < ONE_STREAM_LOOKUPS;
         TN_TRY(ensure_room(t, (uint64_t)L, st));
         Plan p{};
         Scratch w{};
@@ -2199,16 +2172,8 @@ int tn_sparse_table_pull_op(uint32_t table_handle, int N, const int64_t* const* 
         t->plan_small = false;
         t->plan_big_k = big_threshold(t->store);
         t->plan_big_desc = false;
-        // Behind a push of the training loop the descriptors go in on the auxiliary stream, beside that push's
-        // updates: those read the push's own descriptors and status block, and nothing of the scratch buffer.
-        // (Same slot count: the arrays at the head of the plan buffer keep their places.)
-        const bool hoist = behind_push && attempt == 0 && !t->one_stream && N == t->plan_N && !t->upd_pending;
-        behind_push = false;
-        if (hoist && t->tail_recorded) TN_HIP(hipStreamWaitEvent(t->aux, t->tail_ev, 0));  // the gather that read p.descs
-        TN_TRY(upload_slots(t, p.descs, p.lbase, t->dplan, descs, lbase, hoist ? t->aux : st, !t->async_pull,
-                            hoist ? t->stage_ev : nullptr, STATUS_NEW_PLAN, use_lds ? w.bcursor : nullptr,
-                            use_lds ? w.nbuckets + 1 + w.nb2 : 0));
-        if (hoist) TN_HIP(hipStreamWaitEvent(st, t->stage_ev, 0));
+        TN_TRY(upload_slots(t, p.descs, p.lbase, t->dplan, descs, lbase, st, !t->async_pull, STATUS_NEW_PLAN,
+                            use_lds ? w.bcursor : nullptr, use_lds ? w.nbuckets + 1 + w.nb2 : 0));
 
         const Store& s = t->store;
         DevStatus* ds = t->dplan;
@@ -2273,10 +2238,6 @@ int tn_sparse_table_pull_op(uint32_t table_handle, int N, const int64_t* const* 
         }
         if (final_early) {
             harvest(t);
-            if (!t->one_stream) {
-                t->flow = FLOW_PULL;
-                t->flow_stream = st;
-            }
             return take_latched(t);
         }
         return sync_table(t, st);
@@ -2303,8 +2264,6 @@ int push_op_impl(uint32_t table_handle, int N, const int64_t* const* values, con
         return fail(TN_ERR_INVALID_ARGUMENT, "SparseTablePush (pooled): bad batch size or combiner");
     std::lock_guard<std::mutex> lk(t->mu);
     hipStream_t st = (hipStream_t)stream;
-    // the call before was a pull on this stream that returned before its gather
-    const bool behind_pull = t->flow == FLOW_PULL && t->flow_stream == st;
     TN_TRY(ensure_allocated(t, st));
     const int wdim = t->dim + (t->use_cvm ? 2 : 0);
     if (grad_dim != wdim)
@@ -2336,7 +2295,6 @@ int push_op_impl(uint32_t table_handle, int N, const int64_t* const* values, con
     set_last_stream(t, st);
     if (L == 0) return TN_OK;
     t->pooled_pushes = pooled;
-    t->one_stream = L < ONE_STREAM_LOOKUPS;
     Plan p{};
     Scratch w{};
     // Same batch as the last pull?  Necessary conditions on the host, the signs
@@ -2360,7 +2318,6 @@ int push_op_impl(uint32_t table_handle, int N, const int64_t* const* values, con
     // Where the apply kernels find the gradient of a record.  Pooled gradients are first reduced
     // to one row per distinct sign.
     PushSrc src{};
-    hipEvent_t behind = nullptr;  // what the last kernel ahead of the updates signals, if anything
     uint32_t compared_seq = 0;    // with a plan of the last pull's: what the host waits for in hseq[1]
     auto prepare_src = [&]() -> int {
         src = op_source(p, grad_dim, pd == p.push_descs);
@@ -2398,17 +2355,15 @@ int push_op_impl(uint32_t table_handle, int N, const int64_t* const* values, con
         if (spread) TN_LAUNCH(k_pool_frequent, dim3((uint32_t)N), dim3(POOL_THREADS), st, p.lbase, p.ubase, p.u_of_gi, share, extra);
         TN_LAUNCH_LDS(k_lookup_keys, dim3(tiles), dim3(256), pool_tile_lds(share.lp_max), st, pd, p.lbase, p.ubase, (uint32_t)N,
                       p.u_of_gi, batch, pool, poff, share, extra, ds, compared, host_err);
-        behind = t->one_stream ? nullptr : t->fork_ev;
-        hipEvent_t reduced = spread ? nullptr : behind;
 #define TN_REDUCE(LPG, ANY)                                                                                                \
-    TN_LAUNCH_EVENT(reduced, (k_reduce_pooled<LPG, ANY>), dim3(blocks), dim3(POOL_THREADS), st, pd, p.lbase, p.ubase,      \
-                    (uint32_t)N, pool, poff, grad_dim, t->store.D, combiner, ds, flat, share, extra, shares, has)
+    TN_LAUNCH((k_reduce_pooled<LPG, ANY>), dim3(blocks), dim3(POOL_THREADS), st, pd, p.lbase, p.ubase, (uint32_t)N, pool,  \
+              poff, grad_dim, t->store.D, combiner, ds, flat, share, extra, shares, has)
         TN_POOL_LANES(TN_REDUCE, t->store.D, vec);
 #undef TN_REDUCE
         if (spread) {
 #define TN_REDUCE(LPG, ANY)                                                                                                \
-    TN_LAUNCH_EVENT(behind, (k_reduce_pooled_shares<LPG, ANY>), dim3((uint32_t)N * (POOL_SPREAD / 4)), dim3(256), st,      \
-                    p.lbase, p.ubase, grad_dim, t->store.D, ds, shares, has, flat, share, extra)
+    TN_LAUNCH((k_reduce_pooled_shares<LPG, ANY>), dim3((uint32_t)N * (POOL_SPREAD / 4)), dim3(256), st, p.lbase, p.ubase,  \
+              grad_dim, t->store.D, ds, shares, has, flat, share, extra)
             TN_POOL_LANES(TN_REDUCE, t->store.D, grad_dim % 4 == 0);
 #undef TN_REDUCE
         }
@@ -2424,13 +2379,8 @@ int push_op_impl(uint32_t table_handle, int N, const int64_t* const* values, con
     } else if (reuse) {
         carve_plan((char*)t->plan_buf.p, p, N, L, t->plan_exact);
         pd = p.push_descs;
-        // behind a pull that returned before its gather the descriptors go in on the auxiliary stream, beside
-        // that gather (the plan's counts are final from ready_ev on)
-        const bool hoist = behind_pull && !t->one_stream;
-        if (hoist) TN_HIP(hipStreamWaitEvent(t->aux, t->ready_ev, 0));
-        TN_TRY(upload_slots(t, p.push_descs, nullptr, ds, descs, lbase, hoist ? t->aux : st, true, hoist ? t->stage_ev : nullptr,
-                            STATUS_REUSE_PLAN, nullptr, 0, p.ubase, p.push_ubase, (uint32_t)(N + 1)));
-        if (hoist) TN_HIP(hipStreamWaitEvent(st, t->stage_ev, 0));
+        TN_TRY(upload_slots(t, p.push_descs, nullptr, ds, descs, lbase, st, true, STATUS_REUSE_PLAN, nullptr, 0, p.ubase,
+                            p.push_ubase, (uint32_t)(N + 1)));
         // On a plan with show counts the verify pass also sums the clicks; they start at zero
         // after the pull, a further push on the same plan clears them first.
         const bool clicks = t->plan_has_show && with_click;
@@ -2439,7 +2389,8 @@ int push_op_impl(uint32_t table_handle, int N, const int64_t* const* values, con
         // the outcome comes back through pinned host memory, written by the verify kernel itself; that it has come, by a
         // word from the kernels behind it
         compared_seq = ++t->seq_verify;
-        behind = t->one_stream || pooled ? nullptr : t->fork_ev;
+        const bool detach = t->detach_updates && !pooled && L >= DETACH_LOOKUPS;
+        hipEvent_t behind = detach && t->plan_has_show ? t->fork_ev : nullptr;
         t->hpush->st.mismatch = 0;
         t->hpush->st.err = 0;
         uint32_t* host_mismatch = &t->hpush->st.mismatch;
@@ -2471,13 +2422,9 @@ int push_op_impl(uint32_t table_handle, int N, const int64_t* const* values, con
         // Counts and apply kernels are queued before the host knows the outcome: the counts only
         // touch the plan's member lists, which a mismatch discards anyway, and the apply kernels
         // return at once when the mismatch flag is set.  The device never waits for the host.
-        if (!t->plan_has_show) {
-            TN_TRY(launch_counts());
-            behind = nullptr;
-        }
+        if (!t->plan_has_show) TN_TRY(launch_counts());
         TN_TRY(prepare_src());
-        TN_TRY(launch_apply(t, p, src, ds, (int64_t)L, vec, st, addr_in_verify, t->plan_big_k,
-                            t->detach_updates && !pooled, t->plan_big_desc, behind));
+        TN_TRY(launch_apply(t, p, src, ds, (int64_t)L, vec, st, addr_in_verify, t->plan_big_k, detach, t->plan_big_desc, behind));
         // their end, for whoever touches the table next; the status goes out behind them (below)
         if (t->detached_now) TN_HIP(hipStreamWaitEvent(t->side, t->apply_ev, 0));
         TN_TRY(wait_reported(t->hseq + 1, compared_seq, t->detached_now ? t->side : st, "SparseTablePush"));
@@ -2501,7 +2448,7 @@ int push_op_impl(uint32_t table_handle, int N, const int64_t* const* values, con
         pd = p.descs;
         TN_TRY(t->ws.ensure(carve_scratch(nullptr, w, L, dt_entries, false)));
         carve_scratch((char*)t->ws.p, w, L, dt_entries, false);
-        TN_TRY(upload_slots(t, p.descs, p.lbase, ds, descs, lbase, st, false, nullptr, STATUS_NEW_PLAN));
+        TN_TRY(upload_slots(t, p.descs, p.lbase, ds, descs, lbase, st, false, STATUS_NEW_PLAN));
         TN_TRY(launch_build_plan(t, p, w, N, (uint32_t)L, false, false, st));
         TN_TRY(launch_counts());
         TN_TRY(prepare_src());
@@ -2525,12 +2472,6 @@ int push_op_impl(uint32_t table_handle, int N, const int64_t* const* values, con
     t->push_pending = true;
     t->push_on_side = detached;
     t->push_slots = reuse ? 0 : N;
-    // (the reduction of pooled gradients reads the plan's slot layout until the end of the call: nothing of the
-    // next pull may run beside it)
-    if (reuse && !pooled) {
-        t->flow = FLOW_PUSH;
-        t->flow_stream = st;
-    }
     return TN_OK;
 }
 
