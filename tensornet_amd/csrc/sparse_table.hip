@@ -169,6 +169,7 @@ struct SparseTable {
     // and returns when it is there: tail_ev = the gather is done (what a call on another stream has to wait for).
     hipEvent_t tail_ev = nullptr;
     bool tail_recorded = false;
+    bool tail_owed = false;         // ... was on the default stream, which is there for good: recorded when another stream asks
     bool plan_clicks_dirty = false;  // a push has added clicks to the member lists of the current plan
     // Distinct records per lookup seen by the recent pulls (1 = every lookup distinct, the safe start):
     // sizes the number of second-level buckets, whose room is fixed.  A batch with more distinct
@@ -370,9 +371,23 @@ void set_last_stream(SparseTable* t, hipStream_t st) {
 // push's updates, a decay: tail_ev) is waited for on the device, and a call whose status is still pending on the host.
 int order_after_other_stream(SparseTable* t, hipStream_t st) {
     if (!other_stream(t, st)) return TN_OK;
+    if (t->tail_owed) {
+        TN_HIP(hipEventRecord(t->tail_ev, nullptr));
+        t->tail_owed = false;
+        t->tail_recorded = true;
+    }
     if (t->tail_recorded) TN_HIP(hipStreamWaitEvent(st, t->tail_ev, 0));
     if (t->push_pending || t->pull_pending) TN_HIP(hipStreamSynchronize(t->last_stream));
     return TN_OK;
+}
+
+// What the last kernel of a call signals for calls on other streams.  On the default stream nothing: that one can neither be
+// destroyed nor captured, so the event can be recorded there by the call that needs it, later than it would have been and
+// therefore behind more.  (A launch with an event takes the host 1.6 us longer, in front of the kernel.)
+hipEvent_t tail_event(SparseTable* t, hipStream_t st) {
+    t->tail_owed = st == nullptr;
+    if (st) t->tail_recorded = true;
+    return st ? t->tail_ev : nullptr;
 }
 
 // beside_updates: the caller (the pull op) orders its stream behind detached updates itself, as late as it can.
@@ -1373,9 +1388,10 @@ int small_pull(SparseTable* t, const SmallShape& b, const int64_t* const* values
     ea.big_k = t->plan_big_k = b.N <= SMALL_NO_BIG_SLOTS ? 0xFFFFFFFFu : SMALL_BIG_GROUP;
     const size_t emit_lds = small_emit_lds(b.N, b.cap, ea.table);
     const uint32_t finish = (uint32_t)b.N * chunks;
+    hipEvent_t tail = tail_event(t, st);
     if (b.N > SMALL_SPLIT_SLOTS && emit_lds <= SMALL_SHARED_LDS) {
 #define TN_LAUNCH_REST(VEC)                                                                                              \
-    TN_LAUNCH_LDS_EVENT(t->tail_ev, (k_small_pull_rest<VEC>), dim3(b.buckets() + finish), dim3(FINISH_THREADS), emit_lds, st, \
+    TN_LAUNCH_LDS_EVENT(tail, (k_small_pull_rest<VEC>), dim3(b.buckets() + finish), dim3(FINISH_THREADS), emit_lds, st, \
                         ea, chunks, per, s)
         if (width == 4) TN_LAUNCH_REST(4);
         else if (width == 2) TN_LAUNCH_REST(2);
@@ -1388,11 +1404,10 @@ int small_pull(SparseTable* t, const SmallShape& b, const int64_t* const* values
         else if (width == 2) TN_LAUNCH_FINISH(2);
         else TN_LAUNCH_FINISH(1);
 #undef TN_LAUNCH_FINISH
-        TN_LAUNCH_LDS_EVENT(t->tail_ev, (k_group_emit<true>), dim3(b.buckets()), dim3(FINISH_THREADS), emit_lds, st, ea);
+        TN_LAUNCH_LDS_EVENT(tail, (k_group_emit<true>), dim3(b.buckets()), dim3(FINISH_THREADS), emit_lds, st, ea);
     }
     TN_HIP(hipGetLastError());
     // the call returns when the first launch has reported: what follows is complete in stream order
-    t->tail_recorded = true;
     t->small_shape = b;
     t->plan_valid = true;
     t->plan_small = true;
@@ -1471,8 +1486,8 @@ int small_push(SparseTable* t, const int64_t* const* values, const float* const*
     if (pooled)
         launch_small_pool(t, vec, p, batch, dim, combiner, pool, st, &t->hpush->st.abort);
     // (tail_ev is what a call on another stream has to wait for: the updates are still running when this call returns)
-    launch_small_apply(t, row_share(t->store, (pooled || vec) && rows16), p, pool.flat, dim, st, t->hseq + 1, seq, t->tail_ev);
-    t->tail_recorded = true;
+    launch_small_apply(t, row_share(t->store, (pooled || vec) && rows16), p, pool.flat, dim, st, t->hseq + 1, seq,
+                       tail_event(t, st));
     TN_HIP(hipGetLastError());
     // the outcome of the comparison: the updates are queued behind it and do nothing on a mismatch
     TN_TRY(wait_reported(t->hseq + 1, seq, st, "SparseTablePush"));
@@ -2057,6 +2072,7 @@ int tn_sparse_table_show_decay(uint32_t handle, int delta_days, void* stream) {
               delta_days);
     TN_HIP(hipEventRecord(t->tail_ev, st));  // (still running when this call returns)
     t->tail_recorded = true;
+    t->tail_owed = false;
     TN_HIP(hipGetLastError());
     return TN_OK;
 }
@@ -2188,7 +2204,7 @@ int tn_sparse_table_pull_op(uint32_t table_handle, int N, const int64_t* const* 
         const uint32_t* rows_of_groups = (use_lds && N <= GRP_SLOTS) ? nullptr : p.grp_row;
         Publish pub{};
         if (final_early) pub = {reinterpret_cast<uint32_t*>(t->hpull), s.count, t->hseq + 0, seq};
-        hipEvent_t tail = final_early ? t->tail_ev : nullptr;
+        hipEvent_t tail = final_early ? tail_event(t, st) : nullptr;
         if (vec)
             TN_LAUNCH_EVENT(tail, (k_gather_vars<4>), dim3(1 + launch_grid((int64_t)L * (wdim / 4), 256, GRID_CAP * 4)), dim3(256),
                             st, s, ds, rows_of_groups, p.where_u, p.ubase, N, p.descs, pub);
@@ -2196,7 +2212,6 @@ int tn_sparse_table_pull_op(uint32_t table_handle, int N, const int64_t* const* 
             TN_LAUNCH_EVENT(tail, (k_gather_vars<1>), dim3(1 + launch_grid((int64_t)L * wdim, 256, GRID_CAP * 4)), dim3(256), st,
                             s, ds, rows_of_groups, p.where_u, p.ubase, N, p.descs, pub);
         TN_HIP(hipGetLastError());
-        if (tail) t->tail_recorded = true;
         if (!final_early)
             TN_LAUNCH(k_publish, dim3(1), dim3(256), st, ds, p.ubase, (uint32_t)(N + 1), reinterpret_cast<uint32_t*>(t->hpull),
                       s.count);
