@@ -208,42 +208,62 @@ static __global__ void k_report(DevStatus* status, uint64_t* host_word, uint32_t
 constexpr uint32_t KEY_ITEMS = 8;
 constexpr uint32_t KEY_WAVES = 4;
 constexpr uint32_t POOL_TILE = 64 * KEY_WAVES * KEY_ITEMS;
-constexpr uint32_t POOL_PARTS_LOG2 = 11;
-constexpr uint32_t POOL_FILL = 1600;  // (49 k lookups a slot: 32 parts 176 us, 64 parts 255; of 4 k: 4 parts 42, 8 parts 56)
+constexpr uint32_t POOL_PARTS = 2048;  // of a slot at most
+// 49 k lookups a slot: 31 parts (1600) 148 us, 28 (1800) 144, 48 (1024) 144 and the shares 12 for 9; of 4 k: 3 parts 33, 4 parts
+// (1024, 1360) 34 to 36.  (Powers of two only, three workgroups to a CU: 4 parts 44, of 211 slots one and a tenth of a round.)
+constexpr uint32_t POOL_FILL = 1600;
 constexpr uint32_t POOL_SPREAD = 64;
+// (4 M rows of 16: one at a time 167 us, two 164, four 163, eight 162)
+constexpr uint32_t POOL_ROWS_LOG2 = 2, POOL_ROWS = 1u << POOL_ROWS_LOG2;
 constexpr uint32_t POOL_EXTRA = 64;
 constexpr uint32_t POOL_SHARES = POOL_SPREAD + POOL_EXTRA;
-// Slots of 2^3 parts and more have spread signs: from 6404 lookups on.  Shorter ones of several parts have extra ones only, and
+// Slots of more than POOL_SPREAD_FROM lookups have spread signs.  Shorter ones of several parts have extra ones only, and
 // only if the pull has found a heavy sign in the batch (DevStatus::heavy), or did not look for one: it is up to three further
 // rounds there, and finding it and adding up the shares are two launches.
-constexpr uint32_t POOL_SPREAD_LOG2 = 3, POOL_SPREAD_LOG2_HEAVY = 1;
+constexpr uint32_t POOL_SPREAD_FROM = 6403;
 
 // How a slot's lookups are shared out to the backward pass's workgroups: in tiles of POOL_TILE for step 1, for step 2 in
-// 2^lp parts of POOL_FILL lookups at most on average.  The distinct indices of the slot ascend with the signs' first occurrences, so
+// as many parts as POOL_FILL lookups each on average ask for.  The distinct indices of the slot ascend with the signs' first occurrences, so
 // that the frequent signs come early.  The lookups of the first `spread` indices of a slot with many parts are dealt to these
 // run by run (64 lookups), and every part leaves a share of those signs' sums (k_reduce_pooled_shares adds them up): a sign
 // with 8 % of a slot's lookups would be three rounds of one part, and the last workgroup's.  So are those of up to POOL_EXTRA
 // further ones with half as many lookups as a part or more (k_pool_frequent).  The other indices are
-// dealt modulo 2^lp.  Tiles and parts of a call are numbered through the slots so that a slot's first is known from the
+// dealt to the parts in turn, POOL_ROWS at a time (whose rows share a line or two).  Tiles and parts of a call are numbered through the slots so that a slot's first is known from the
 // lookups before it; some numbers are nobody's.
 struct PoolShare {
-    uint32_t lp_max;  // of the longest slot
-    uint32_t spread_log2;
-    PoolShare(uint32_t max_len, bool heavy)
-        : lp_max(parts_log2(max_len)), spread_log2(heavy ? POOL_SPREAD_LOG2_HEAVY : POOL_SPREAD_LOG2) {}
-    static __host__ __device__ uint32_t parts_log2(uint32_t len) {
-        uint32_t lp = 0;
-        while (lp < POOL_PARTS_LOG2 && (len >> lp) > POOL_FILL) lp++;
-        return lp;
+    uint32_t parts_max;  // of the longest slot
+    uint32_t extra_from; // slots of more lookups may have extra spread signs
+    PoolShare(uint32_t max_len, bool heavy) : parts_max(parts(max_len)), extra_from(heavy ? POOL_FILL : POOL_SPREAD_FROM) {}
+    static __host__ __device__ uint32_t parts(uint32_t len) {
+        const uint32_t n = (len + POOL_FILL - 1) / POOL_FILL;
+        return n < 1 ? 1u : n < POOL_PARTS ? n : POOL_PARTS;
     }
-    __host__ __device__ bool spreads(uint32_t lp) const { return lp >= spread_log2; }  // has extra ones, maybe
-    static __host__ __device__ uint32_t spread(uint32_t lp) { return lp >= POOL_SPREAD_LOG2 ? POOL_SPREAD : 0u; }
+    __host__ __device__ bool spreads(uint32_t len) const { return len > extra_from; }  // has extra ones, maybe
+    static __host__ __device__ uint32_t spread(uint32_t len) { return len > POOL_SPREAD_FROM ? POOL_SPREAD : 0u; }
     static __host__ __device__ uint32_t first_tile(uint32_t slot, uint32_t lookups_before) {
         return lookups_before / POOL_TILE + slot;
     }
-    // (2^lp is one, or less than two per POOL_FILL lookups)
     static __host__ __device__ uint32_t first_part(uint32_t slot, uint32_t lookups_before) {
-        return (uint32_t)(2ull * lookups_before / POOL_FILL) + slot;
+        return lookups_before / POOL_FILL + slot;
+    }
+};
+// Turns: x = q * parts + part, without a division.
+struct PoolTurn {
+    uint32_t parts, magic;
+    __device__ __forceinline__ explicit PoolTurn(uint32_t n) : parts(n), magic(n > 1 ? 0xFFFFFFFFu / n + 1u : 0u) {}
+    __device__ __forceinline__ uint32_t turn(uint32_t x) const {
+        if (parts == 1) return x;
+        const uint32_t q = __umulhi(x, magic);  // x / parts, or one more
+        return q * parts > x ? q - 1u : q;
+    }
+    __device__ __forceinline__ uint32_t part(uint32_t x) const { return x - turn(x) * parts; }
+    // an index that is not spread: whose it is, which of its part's, and back (less the part's own first one)
+    __device__ __forceinline__ uint32_t part_of(uint32_t index) const { return part(index >> POOL_ROWS_LOG2); }
+    __device__ __forceinline__ uint32_t key_of(uint32_t index) const {
+        return (turn(index >> POOL_ROWS_LOG2) << POOL_ROWS_LOG2) | (index & (POOL_ROWS - 1u));
+    }
+    __device__ __forceinline__ uint32_t index_of(uint32_t key) const {
+        return ((key >> POOL_ROWS_LOG2) * parts << POOL_ROWS_LOG2) | (key & (POOL_ROWS - 1u));
     }
 };
 
@@ -264,8 +284,8 @@ static __global__ __launch_bounds__(POOL_THREADS) void k_pool_frequent(const uin
     __shared__ uint32_t listed[FREQUENT_LISTED], times[FREQUENT_LISTED], n_listed;
     const uint32_t sl = blockIdx.x, tid = threadIdx.x, l0 = lbase[sl], len = lbase[sl + 1] - l0, ub = ubase[sl];
     uint32_t* const out = extra + sl * (POOL_EXTRA + 1);
-    const uint32_t lp = share.parts_log2(len), spread = share.spread(lp);
-    if (!share.spreads(lp)) {
+    const uint32_t spread = share.spread(len);
+    if (!share.spreads(len)) {
         if (tid == 0) out[0] = 0;
         return;
     }
@@ -325,12 +345,12 @@ static_assert(FREQUENT_LISTED <= POOL_THREADS && FREQUENT_SAMPLES % POOL_THREADS
 // k_table_part): no atomics whose order of arrival would show.
 // An item: x the example, y bits 0-10 its lookups (POOL_COUNT_MANY: as many or more), 11 the sign's first lookup, 12-31 the
 // key: of the first `spread` distinct indices these themselves, of the extra ones spread + their place among them, of the
-// others (index - spread) / 2^lp behind those.
+// others which of their part's they are behind those.
 constexpr uint32_t POOL_COUNT_MANY = 0x7FF;
 constexpr uint32_t POOL_FIRST = 0x800;
 constexpr uint32_t POOL_KEY_SHIFT = 12;
 
-inline size_t pool_tile_lds(uint32_t lp) { return ((size_t)KEY_WAVES << lp) * sizeof(uint32_t); }
+inline size_t pool_tile_lds(uint32_t parts) { return (size_t)KEY_WAVES * parts * sizeof(uint32_t); }
 
 static __global__ __launch_bounds__(256) void k_lookup_keys(const SlotDesc* __restrict__ descs, const uint32_t* __restrict__ lbase,
                                                      const uint32_t* __restrict__ ubase, uint32_t N,
@@ -338,7 +358,7 @@ static __global__ __launch_bounds__(256) void k_lookup_keys(const SlotDesc* __re
                                                      uint2* __restrict__ pool, uint16_t* __restrict__ poff, PoolShare share,
                                                      const uint32_t* __restrict__ extra, DevStatus* status,
                                                      HostWord compared, uint32_t* host_err) {
-    extern __shared__ uint32_t cnt[];  // [2^lp][KEY_WAVES]
+    extern __shared__ uint32_t cnt[];  // [parts][KEY_WAVES]
     __shared__ uint32_t more[POOL_EXTRA];
     __shared__ uint32_t wsum[KEY_WAVES];
     __shared__ uint32_t slot;
@@ -353,9 +373,11 @@ static __global__ __launch_bounds__(256) void k_lookup_keys(const SlotDesc* __re
     __syncthreads();
     if (slot == N) return;
     const uint32_t sl = slot, l0 = lbase[sl], len = lbase[sl + 1] - l0;
-    const uint32_t t0 = (blockIdx.x - share.first_tile(sl, l0)) * POOL_TILE, lp = share.parts_log2(len);
-    const uint32_t ub = ubase[sl], parts = 1u << lp, spread = share.spread(lp);
-    const uint32_t extras = share.spreads(lp) ? extra[sl * (POOL_EXTRA + 1)] : 0u, spread_all = spread + extras;
+    const uint32_t t0 = (blockIdx.x - share.first_tile(sl, l0)) * POOL_TILE;
+    const uint32_t ub = ubase[sl], parts = share.parts(len), spread = share.spread(len);
+    const PoolTurn turn(parts);
+    const uint32_t bits = parts > 1 ? 32 - (uint32_t)__clz((int)(parts - 1)) : 0u;  // of a part's number
+    const uint32_t extras = share.spreads(len) ? extra[sl * (POOL_EXTRA + 1)] : 0u, spread_all = spread + extras;
     const Global<const int64_t> ex = example_of(descs[sl]);
     int64_t b[KEY_ITEMS], prev[KEY_ITEMS];
     uint32_t u[KEY_ITEMS];
@@ -430,9 +452,10 @@ static __global__ __launch_bounds__(256) void k_lookup_keys(const SlotDesc* __re
         count[j] = min(to_start + to_end, POOL_COUNT_MANY);
         // its place among the tile's lookups of its part: behind those of earlier runs and lanes
         const uint32_t index = u[j] & ~FIRST_BIT;
-        const uint32_t part = (index < spread_all ? i >> 6 : index - spread_all) & (parts - 1u), k = part * KEY_WAVES + wave;
+        const uint32_t part = index < spread_all ? turn.part(i >> 6) : turn.part_of(index - spread_all);
+        const uint32_t k = part * KEY_WAVES + wave;
         unsigned long long same = __ballot(active);
-        for (uint32_t q = 0; q < lp; q++) {
+        for (uint32_t q = 0; q < bits; q++) {
             const unsigned long long m = __ballot((part >> q) & 1u);
             same &= ((part >> q) & 1u) ? m : ~m;
         }
@@ -452,7 +475,7 @@ static __global__ __launch_bounds__(256) void k_lookup_keys(const SlotDesc* __re
     uint32_t sum = 0;
     for (uint32_t q = 0; q < each; q++) sum += tid * each + q < total ? cnt[tid * each + q] : 0u;
     uint32_t x = block_excl_scan_256<uint32_t>(sum, wsum, nullptr);
-    uint16_t* off = poff + (size_t)blockIdx.x * ((1u << share.lp_max) + 1);
+    uint16_t* off = poff + (size_t)blockIdx.x * (share.parts_max + 1);
     for (uint32_t q = 0; q < each; q++) {
         const uint32_t k = tid * each + q;
         if (k >= total) break;
@@ -467,8 +490,8 @@ static __global__ __launch_bounds__(256) void k_lookup_keys(const SlotDesc* __re
     for (uint32_t j = 0; j < KEY_ITEMS; j++) {
         const uint32_t i = t0 + (wave * KEY_ITEMS + j) * 64 + lane, index = u[j] & ~FIRST_BIT;
         if (i >= len) continue;
-        const uint32_t part = (index < spread_all ? i >> 6 : index - spread_all) & (parts - 1u);
-        const uint32_t key = index < spread_all ? index : spread_all + ((index - spread_all) >> lp);
+        const uint32_t part = index < spread_all ? turn.part(i >> 6) : turn.part_of(index - spread_all);
+        const uint32_t key = index < spread_all ? index : spread_all + turn.key_of(index - spread_all);
         pool[l0 + t0 + cnt[part * KEY_WAVES + wave] + at[j]] =
             make_uint2((uint32_t)b[j], count[j] | (u[j] & FIRST_BIT ? POOL_FIRST : 0u) | (key << POOL_KEY_SHIFT));
     }
@@ -498,13 +521,14 @@ __device__ __forceinline__ uint32_t lookups_of(Global<const int64_t> ex, uint32_
 // round before left; the round that meets a sign's first lookup writes its row.  The sums of the signs that are spread over
 // the parts go to the part's own rows of `shares`, `has` tells which there are.  The order of all additions is fixed.
 //
-// What bounds it is a workgroup's chain (slot, tiles, items; sort; rows; shares: 20 us, 27 with the chip full), so it wants
-// three workgroups on a CU.  4.9 M lookups in 100 slots, rows of 16: 175 us, with k_lookup_keys (46) and the shares (6) 227,
-// where a counting sort of the lookups through memory, an ordering pass and a reduction by sign took 390; 860 k in 211 slots:
-// 58 for 103.
+// What bounds it is a workgroup's chain (slot, tiles, items; sort; rows; shares), so it wants
+// as many workgroups on a CU as there is room for, four.  4.9 M lookups in 100 slots, rows of 16: 148 us, of which the list of a
+// part's items takes 39, the sort 35, the sums 50 and writing the rows 20 (each left out in turn); 860 k in 211 slots: 33.
+// (A counting sort of the lookups through memory, an ordering pass and a reduction by sign, k_lookup_keys' work included: 390
+// for 205 and 103 for 48.)
 static_assert(POOL_SPREAD == 64 && POOL_EXTRA <= POOL_SPREAD, "k_reduce_pooled_shares");
 template <int LPG, bool ANY>
-__global__ __launch_bounds__(POOL_THREADS) __attribute__((amdgpu_waves_per_eu(6, 6))) void k_reduce_pooled(const SlotDesc* __restrict__ descs,
+__global__ __launch_bounds__(POOL_THREADS) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_reduce_pooled(const SlotDesc* __restrict__ descs,
                                                                 const uint32_t* __restrict__ lbase,
                                                                 const uint32_t* __restrict__ ubase, uint32_t N,
                                                                 const uint2* __restrict__ pool,
@@ -524,16 +548,17 @@ __global__ __launch_bounds__(POOL_THREADS) __attribute__((amdgpu_waves_per_eu(6,
     __syncthreads();
     for (uint32_t s = tid; s < N; s += POOL_THREADS) {
         const uint32_t a = lbase[s], b = lbase[s + 1], q = item - share.first_part(s, a);  // (wraps before the slot)
-        if (b > a && q < (1u << share.parts_log2(b - a))) slot = s;
+        if (b > a && q < share.parts(b - a)) slot = s;
     }
     __syncthreads();
     if (slot == N) return;
     const uint32_t sl = slot, l0 = lbase[sl], len = lbase[sl + 1] - l0, ub = ubase[sl], us = ubase[sl + 1] - ub;
-    const uint32_t lp = share.parts_log2(len), part = item - share.first_part(sl, l0), tile0 = share.first_tile(sl, l0);
-    const uint32_t spread = share.spread(lp), spread_all = spread + (share.spreads(lp) ? extra[sl * (POOL_EXTRA + 1)] : 0u);
-    if (!spread_all && part >= us) return;
-    const uint32_t rest = ub + spread + part;  // the part's first row of an index that is not spread
-    const uint32_t top = us > spread ? spread_all + ((us - 1 - spread) >> lp) : us - 1, bits = top ? 32 - (uint32_t)__clz((int)top) : 0u;
+    const PoolTurn turn(share.parts(len));
+    const uint32_t part = item - share.first_part(sl, l0), tile0 = share.first_tile(sl, l0);
+    const uint32_t spread = share.spread(len), spread_all = spread + (share.spreads(len) ? extra[sl * (POOL_EXTRA + 1)] : 0u);
+    if (!spread_all && part << POOL_ROWS_LOG2 >= us) return;
+    const uint32_t rest = ub + spread + (part << POOL_ROWS_LOG2);  // the part's first row of an index that is not spread
+    const uint32_t top = us > spread ? spread_all + turn.key_of(us - 1 - spread) + POOL_ROWS : us - 1, bits = top ? 32 - (uint32_t)__clz((int)top) : 0u;
     const float* pooled = descs[sl].grads;
     const Global<const int64_t> ex = example_of(descs[sl]);
     const uint32_t mine = (len + POOL_TILE - 1) / POOL_TILE;
@@ -545,7 +570,7 @@ __global__ __launch_bounds__(POOL_THREADS) __attribute__((amdgpu_waves_per_eu(6,
             {  // (again in a further round: the sums of the one before took the list's place)
                 uint32_t c = 0, lo = 0;
                 if (g0 + tid < mine) {
-                    const uint16_t* off = poff + (size_t)(tile0 + g0 + tid) * ((1u << share.lp_max) + 1) + part;
+                    const uint16_t* off = poff + (size_t)(tile0 + g0 + tid) * (share.parts_max + 1) + part;
                     lo = off[0];
                     c = off[1] - lo;
                 }
@@ -578,7 +603,7 @@ __global__ __launch_bounds__(POOL_THREADS) __attribute__((amdgpu_waves_per_eu(6,
                         return shares + ((uint64_t)item * POOL_SHARES + key) * dim;
                     }
                     add = !first;
-                    return flat + (uint64_t)(rest + ((key - spread_all) << lp)) * dim;
+                    return flat + (uint64_t)(rest + turn.index_of(key - spread_all)) * dim;
                 });
             else
                 __syncthreads();
@@ -602,15 +627,15 @@ __global__ __launch_bounds__(256) void k_reduce_pooled_shares(const uint32_t* __
     constexpr uint32_t PER = 256 / 64;
     const uint32_t sl = blockIdx.x / (POOL_SPREAD / PER), key0 = blockIdx.x % (POOL_SPREAD / PER) * PER + threadIdx.x / 64;
     const uint32_t l0 = lbase[sl], len = lbase[sl + 1] - l0, ub = ubase[sl], us = ubase[sl + 1] - ub;
-    const uint32_t lp = share.parts_log2(len), p0 = share.first_part(sl, l0);
-    if (len == 0 || !share.spreads(lp)) return;
+    const uint32_t p0 = share.first_part(sl, l0);
+    if (len == 0 || !share.spreads(len)) return;
     const uint32_t* const more = extra + sl * (POOL_EXTRA + 1);
-    const uint32_t spread = share.spread(lp), spread_all = spread + more[0];
+    const uint32_t spread = share.spread(len), spread_all = spread + more[0];
     for (uint32_t key = key0; key < spread_all; key += POOL_SPREAD) {  // (the same for a whole wavefront)
         const uint32_t index = key < spread ? key : more[1 + key - spread];
         if (index >= us) return;
         add_shares<LPG, ANY>(
-            1u << lp, D,
+            share.parts(len), D,
             [&](uint32_t q) { return ((has[(uint64_t)(p0 + q) * (POOL_SHARES / 64) + key / 64] >> (key % 64)) & 1ull) != 0; },
             [&](uint32_t q) { return shares + ((uint64_t)(p0 + q) * POOL_SHARES + key) * dim; },
             flat + (uint64_t)(ub + index) * dim);

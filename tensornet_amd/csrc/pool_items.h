@@ -16,24 +16,26 @@ constexpr uint32_t POOL_RUN = POOL_ITEMS_MAX / POOL_WAVES;  // consecutive looku
 constexpr uint32_t POOL_WORDS = POOL_ITEMS_MAX / 64;
 constexpr uint32_t POOL_PIECE = 16;
 constexpr uint32_t POOL_PIECES = POOL_ITEMS_MAX / POOL_PIECE;
-constexpr uint32_t POOL_AHEAD = 4;  // rows of a group of lanes in flight (eight: the registers of three workgroups do not hold them)
+constexpr uint32_t POOL_AHEAD = 4;  // rows of a group of lanes in flight (eight: the registers of a workgroup of four do not hold them)
 constexpr uint32_t POOL_DIGIT = 7;  // (10, one pass for most slots, whose 8192 counters take longer: 44 -> 47 us, 175 -> 184)
+static_assert(POOL_AHEAD == 4 && POOL_PIECE % POOL_AHEAD == 0, "items are read four at a time");
 enum { POOL_SUM = 0, POOL_MEAN = 1, POOL_SQRTN = 2 };  // (the combiners of the C ABI)
 static_assert(POOL_RUN == 64 * POOL_ITEMS && 64 % POOL_PIECE == 0, "whole wavefronts, pieces inside a word");
 
-// 47 KB: three workgroups of eight wavefronts to a CU (twice the size in workgroups of sixteen: one to a CU, and 4.9 M
-// lookups took 2.5 times as long)
+// 37 KB: four workgroups of eight wavefronts to a CU (45 KB and three of them: 4.9 M lookups 161 us, so 148; twice the size in
+// workgroups of sixteen: one to a CU, 2.5 times as long).  The sort's last pass moves the items themselves, so that its orders
+// and what the pieces leave can share their room, and a piece's own sum stays in its lanes' registers.
 struct PoolLds {
-    uint32_t key[POOL_ITEMS_MAX];      // the lookup's sign
-    uint32_t example[POOL_ITEMS_MAX];  // its example
-    float scale[POOL_ITEMS_MAX];       // 1 / d(lookups of the example); negative: not its sign's first lookup
-    uint16_t ord[POOL_ITEMS_MAX];      // the lookups in the order of their signs
+    alignas(16) uint32_t key[POOL_ITEMS_MAX];      // the lookup's sign (in the end the lookups are in the order of their signs)
+    alignas(16) uint32_t example[POOL_ITEMS_MAX];  // its example
+    alignas(16) float scale[POOL_ITEMS_MAX];       // 1 / d(lookups of the example); negative: not its sign's first lookup
+    uint16_t ord[POOL_ITEMS_MAX];      // while sorting: the order after every other pass,
     union {
         struct {
-            uint16_t half[POOL_ITEMS_MAX];             // while sorting: the order after every other pass,
+            uint16_t half[POOL_ITEMS_MAX];             // ... after the others,
             uint16_t digit[POOL_WAVES << POOL_DIGIT];  // counters
         };
-        float4 part[POOL_PIECES][2][4];  // then: what a piece has of a sign that began before it / goes on behind it
+        float4 part[POOL_PIECES][4];  // then: what a piece has of a sign that began before it
         uint32_t list[2 * POOL_THREADS + 1];  // (before: k_reduce_pooled's tiles)
     };
     unsigned long long heads[POOL_WORDS];  // starts of the signs in the order
@@ -78,13 +80,9 @@ __device__ __forceinline__ void pool_items(PoolLds& lds, uint32_t n, uint32_t bi
     const uint32_t lane = tid & 63, wave = tid >> 6;
     const uint32_t passes = (bits + POOL_DIGIT - 1) / POOL_DIGIT, width = passes ? (bits + passes - 1) / passes : 0u;
     __syncthreads();
-    if (passes == 0) {
-        for (uint32_t i = tid; i < n; i += POOL_THREADS) lds.ord[i] = (uint16_t)i;
-        __syncthreads();
-    }
     for (uint32_t pass = 0; pass < passes; pass++) {
-        uint16_t* const to = (passes - 1 - pass) & 1u ? lds.half : lds.ord;
-        const uint16_t* const from = (passes - 1 - pass) & 1u ? lds.ord : lds.half;  // (the first pass takes them as they are)
+        uint16_t* const to = pass & 1u ? lds.ord : lds.half;
+        const uint16_t* const from = pass & 1u ? lds.half : lds.ord;  // (the first pass takes them as they are)
         for (uint32_t i = tid; i < POOL_WAVES << width >> 1; i += POOL_THREADS) reinterpret_cast<uint32_t*>(lds.digit)[i] = 0;
         __syncthreads();
         uint32_t item[POOL_ITEMS], dg[POOL_ITEMS], at[POOL_ITEMS];
@@ -121,17 +119,37 @@ __device__ __forceinline__ void pool_items(PoolLds& lds, uint32_t n, uint32_t bi
                 x += c;
             }
         }
-        __syncthreads();
+        if (pass + 1 < passes) {
+            __syncthreads();
 #pragma unroll
-        for (uint32_t j = 0; j < POOL_ITEMS; j++)
-            if (wave * POOL_RUN + j * 64 + lane < n) to[lds.digit[dg[j] * POOL_WAVES + wave] + at[j]] = (uint16_t)item[j];
+            for (uint32_t j = 0; j < POOL_ITEMS; j++)
+                if (wave * POOL_RUN + j * 64 + lane < n) to[lds.digit[dg[j] * POOL_WAVES + wave] + at[j]] = (uint16_t)item[j];
+        } else {  // the last one moves the items themselves
+            uint32_t key[POOL_ITEMS], example[POOL_ITEMS];
+            float scale[POOL_ITEMS];
+#pragma unroll
+            for (uint32_t j = 0; j < POOL_ITEMS; j++) {
+                key[j] = lds.key[item[j]];
+                example[j] = lds.example[item[j]];
+                scale[j] = lds.scale[item[j]];
+            }
+            __syncthreads();
+#pragma unroll
+            for (uint32_t j = 0; j < POOL_ITEMS; j++) {
+                if (wave * POOL_RUN + j * 64 + lane >= n) continue;
+                const uint32_t place = lds.digit[dg[j] * POOL_WAVES + wave] + at[j];
+                lds.key[place] = key[j];
+                lds.example[place] = example[j];
+                lds.scale[place] = scale[j];
+            }
+        }
         __syncthreads();
     }
     // starts of the signs in the order (and what lies behind it)
 #pragma unroll
     for (uint32_t j = 0; j < POOL_ITEMS; j++) {
         const uint32_t i = wave * POOL_RUN + j * 64 + lane;
-        const bool head = i >= n || i == 0 || lds.key[lds.ord[i]] != lds.key[lds.ord[i - 1]];
+        const bool head = i >= n || i == 0 || lds.key[i] != lds.key[i - 1];
         const unsigned long long m = __ballot(head);
         if (lane == 0) lds.heads[i >> 6] = m;
     }
@@ -148,25 +166,28 @@ __device__ __forceinline__ void pool_items(PoolLds& lds, uint32_t n, uint32_t bi
         }
         put_row_part<ANY>(out, sub, D - c0, v);
     };
+    // a piece per group of lanes
+    static_assert(POOL_THREADS / 4 >= POOL_PIECES, "there are as many");
+    const uint32_t q = tid / LPG, lo = q * POOL_PIECE, hi = lo + POOL_PIECE;
     for (int c0 = 0; c0 < D; c0 += 4 * LPG) {
-        for (uint32_t q = tid / LPG; q < pieces; q += POOL_THREADS / LPG) {
-            const uint32_t lo = q * POOL_PIECE, hi = lo + POOL_PIECE;
+        bool began = false, goes_on = false;  // the running sum's sign: began in the piece, goes on behind it
+        float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (q < pieces) {
             // which places start a sign, and the one behind the piece (those behind the last lookup do)
             uint32_t hb = (uint32_t)(lds.heads[lo >> 6] >> (lo & 63)) & ((1u << POOL_PIECE) - 1u);
             if (hi >= n || ((lds.heads[hi >> 6] >> (hi & 63)) & 1ull)) hb |= 1u << POOL_PIECE;
-            bool began = false, first = false;  // the running sum's sign: here, with its first lookup
-            float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+            bool first = false;  // (the running sum has its sign's first lookup)
 #pragma unroll 1
             for (uint32_t j0 = 0; j0 < POOL_PIECE && lo + j0 < n; j0 += POOL_AHEAD, hb >>= POOL_AHEAD) {
                 float4 g[POOL_AHEAD];
-                float sc[POOL_AHEAD];
-                uint32_t key[POOL_AHEAD];
+                const uint4 e4 = *reinterpret_cast<const uint4*>(lds.example + lo + j0);
+                const float4 s4 = *reinterpret_cast<const float4*>(lds.scale + lo + j0);
+                const uint32_t example[POOL_AHEAD] = {e4.x, e4.y, e4.z, e4.w};
+                const float sc[POOL_AHEAD] = {s4.x, s4.y, s4.z, s4.w};
 #pragma unroll
                 for (uint32_t w = 0; w < POOL_AHEAD; w++) {
-                    const uint32_t i = lds.ord[min(lo + j0 + w, n - 1)];
-                    sc[w] = lds.scale[i];
-                    key[w] = lds.key[i];
-                    g[w] = row_part<ANY>(pooled + (uint64_t)lds.example[i] * dim + c0, sub, D - c0);
+                    const uint32_t e = lo + j0 + w < n ? example[w] : 0u;  // (behind the last item: some row or other)
+                    g[w] = row_part<ANY>(pooled + (uint64_t)e * dim + c0, sub, D - c0);
                 }
 #pragma unroll
                 for (uint32_t w = 0; w < POOL_AHEAD; w++) {
@@ -183,26 +204,23 @@ __device__ __forceinline__ void pool_items(PoolLds& lds, uint32_t n, uint32_t bi
                     acc.w += g[w].w * scale;
                     if ((hb >> (w + 1)) & 1u) {  // the sign ends here
                         if (began)
-                            put(key[w], first, c0, acc);
+                            put(lds.key[lo + j0 + w], first, c0, acc);
                         else
-                            lds.part[q][0][sub] = acc;
+                            lds.part[q][sub] = acc;
                     }
                 }
             }
-            if (!(hb & 1u)) lds.part[q][began ? 1 : 0][sub] = acc;  // it goes on
+            goes_on = !(hb & 1u);
+            if (goes_on && !began) lds.part[q][sub] = acc;
         }
         __syncthreads();
-        for (uint32_t q = tid / LPG; q < pieces; q += POOL_THREADS / LPG) {
-            const uint32_t hi = (q + 1) * POOL_PIECE;
-            if (hi >= n || ((lds.heads[hi >> 6] >> (hi & 63)) & 1ull)) continue;  // no sign goes on behind this piece
+        if (goes_on && began) {  // with what the pieces behind have of it, in order
             const uint32_t from = bit_at_or_below(lds.heads, hi - 1);
-            if (from < q * POOL_PIECE) continue;  // it began before it
             const uint32_t end = bit_above(lds.heads, hi, POOL_WORDS, n), last = (end - 1) / POOL_PIECE;
-            float4 acc = lds.part[q][1][sub];
             for (uint32_t r = q + 1; r <= last; r += 4) {
                 float4 g[4];
 #pragma unroll
-                for (uint32_t w = 0; w < 4; w++) g[w] = lds.part[min(r + w, last)][0][sub];
+                for (uint32_t w = 0; w < 4; w++) g[w] = lds.part[min(r + w, last)][sub];
 #pragma unroll
                 for (uint32_t w = 0; w < 4; w++) {
                     if (r + w > last) break;
@@ -212,8 +230,7 @@ __device__ __forceinline__ void pool_items(PoolLds& lds, uint32_t n, uint32_t bi
                     acc.w += g[w].w;
                 }
             }
-            const uint32_t i = lds.ord[from];
-            put(lds.key[i], lds.scale[i] > 0.f, c0, acc);
+            put(lds.key[from], lds.scale[from] > 0.f, c0, acc);
         }
         __syncthreads();
     }

@@ -627,8 +627,9 @@ static_assert(SMALL_PARTS_MAX * SMALL_HEAVY_MAX <= POOL_THREADS && SMALL_HEAVY_M
 // of their sums (k_small_pool_shares adds them up).  As one workgroup's such a sign is a chain of rounds (25 us each at 16
 // elements a row): 100 slots of 8000 lookups, 80 % of them one sign, a step with rows of 16 237 us, of 64 475;
 // so 163 and 266.
+// (Four workgroups to a CU, of 64 registers: 100 slots of 6000 lookups 45 us, three 51; 26 of 1000, rows of 64, 33.4 and 33.3.)
 template <int LPG, bool ANY, bool HEAVY>
-__global__ __launch_bounds__(POOL_THREADS) __attribute__((amdgpu_waves_per_eu(6, 6))) void k_small_pool(SmallShape b, SmallPlan p, const SlotDesc* __restrict__ descs,
+__global__ __launch_bounds__(POOL_THREADS) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_small_pool(SmallShape b, SmallPlan p, const SlotDesc* __restrict__ descs,
                                                              int64_t batch, int dim, int D, int combiner,
                                                              float* __restrict__ flat, DevStatus* status, uint32_t* host_err,
                                                              uint32_t lp, float* __restrict__ shares,

@@ -2354,10 +2354,10 @@ int push_op_impl(uint32_t table_handle, int N, const int64_t* const* values, con
         float *flat, *shares;
         uint64_t* has;
         uint32_t* extra;
-        const bool spread = share.spreads(share.lp_max);
+        const bool spread = share.spreads((uint32_t)max_len);
         auto carve = [&](Carver& cv) {
             pool = cv.take<uint2>(L);
-            poff = cv.take<uint16_t>((size_t)tiles * ((1u << share.lp_max) + 1));
+            poff = cv.take<uint16_t>((size_t)tiles * (share.parts_max + 1));
             flat = cv.take<float>(L * (size_t)grad_dim);
             shares = cv.take<float>(spread ? (size_t)blocks * POOL_SHARES * grad_dim : 0);
             has = cv.take<uint64_t>(spread ? (size_t)blocks * (POOL_SHARES / 64) : 0);
@@ -2368,7 +2368,7 @@ int push_op_impl(uint32_t table_handle, int N, const int64_t* const* values, con
         Carver c2{(char*)t->pooled_ws.p};
         carve(c2);
         if (spread) TN_LAUNCH(k_pool_frequent, dim3((uint32_t)N), dim3(POOL_THREADS), st, p.lbase, p.ubase, p.u_of_gi, share, extra);
-        TN_LAUNCH_LDS(k_lookup_keys, dim3(tiles), dim3(256), pool_tile_lds(share.lp_max), st, pd, p.lbase, p.ubase, (uint32_t)N,
+        TN_LAUNCH_LDS(k_lookup_keys, dim3(tiles), dim3(256), pool_tile_lds(share.parts_max), st, pd, p.lbase, p.ubase, (uint32_t)N,
                       p.u_of_gi, batch, pool, poff, share, extra, ds, compared, host_err);
 #define TN_REDUCE(LPG, ANY)                                                                                                \
     TN_LAUNCH((k_reduce_pooled<LPG, ANY>), dim3(blocks), dim3(POOL_THREADS), st, pd, p.lbase, p.ubase, (uint32_t)N, pool,  \
