@@ -82,10 +82,13 @@ __device__ __forceinline__ uint2 ids_below(Global<const int64_t> ex, uint32_t n,
 // The variable rows of a slot are read again and again: every die of the chip takes a contiguous share of the items, so
 // that a slot's rows (1.3 MB at 20 k distinct signs of 16 elements) are in the L2 of the die that wants them.  The 4.9 M lookups
 // read 225 MB and write 105 in the 100 us, 3.3 TB/s.
+struct NoDescs {};
+__device__ __forceinline__ const SlotDesc& desc_of(const ArgDescs& a, const SlotDesc*, uint32_t sl) { return a.slot[sl]; }
+__device__ __forceinline__ const SlotDesc& desc_of(const NoDescs&, const SlotDesc* __restrict__ d, uint32_t sl) { return d[sl]; }
 constexpr uint32_t COMBINE_IDS = 2048;
 constexpr uint32_t COMBINE_AHEAD = 2;  // lookups of a thread in flight while they are checked
-template <int LPG, bool ANY>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ANY ? 6 : 7, 8))) void k_combine_fwd(const SlotDesc* __restrict__ descs, uint32_t items, uint32_t per_slot,
+template <int LPG, bool ANY, typename Descs>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ANY ? 6 : 7, 8))) void combine_fwd_kernel(Descs by_value, const SlotDesc* __restrict__ descs, uint32_t items, uint32_t per_slot,
                                                      uint32_t per, int dim, int64_t batch, int combiner, DevStatus* status) {
     extern __shared__ uint32_t range[];  // [per] first lookup of an example, [per] the lookup after its last
     __shared__ uint32_t row[COMBINE_IDS];
@@ -97,7 +100,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ANY ? 6 : 7
         const uint32_t sl = item / per_slot;
         const int64_t b0 = (int64_t)(item - sl * per_slot) * per;
         const uint32_t nb = (uint32_t)min((int64_t)per, batch - b0);
-        const SlotDesc d = descs[sl];
+        const SlotDesc d = desc_of(by_value, descs, sl);
         const Global<const int64_t> ex = example_of(d);
         const Global<const int64_t> ids = as_global(d.values);
         for (uint32_t i = threadIdx.x; i < 2 * per; i += 256) range[i] = 0;

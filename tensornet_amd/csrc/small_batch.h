@@ -106,8 +106,28 @@ inline size_t small_slots_lds(uint32_t entries, uint32_t max_len, uint32_t nbp) 
 // and then took a share of the probes repeated the slot's remap up to eight times).  What bounds it is a chain of
 // round trips -- descriptor, signs, probe, second probe -- and a CU's rate of random 64-byte reads (0.2 per ns), hence
 // many workgroups with about a hundred signs each.
-template <int THREADS>
-__device__ __forceinline__ void small_slots(const SmallShape& b, const SmallPlan& p, const SlotDesc* host_descs, uint32_t entries,
+// The descriptor of slot `sl` for the whole workgroup, into LDS, and with `keep` into the plan, for the launches after this one:
+// what is to be done before and after the workgroup clears its LDS, while a descriptor in the host's buffer is on its way.
+struct DescFetch {
+    uint32_t word = 0;
+    __device__ __forceinline__ void start(const ArgDescs&, int) {}
+    __device__ __forceinline__ void start(const HostDescs& d, int sl) {
+        if (threadIdx.x < sizeof(SlotDesc) / 4) word = reinterpret_cast<const uint32_t*>(d.slot + sl)[threadIdx.x];
+    }
+    __device__ __forceinline__ void finish(const ArgDescs& d, int sl, SlotDesc& sd, SlotDesc* keep) const {
+        if (threadIdx.x != 0) return;
+        sd = d.slot[sl];
+        if (keep) *keep = d.slot[sl];
+    }
+    __device__ __forceinline__ void finish(const HostDescs&, int, SlotDesc& sd, SlotDesc* keep) const {
+        if (threadIdx.x >= sizeof(SlotDesc) / 4) return;
+        reinterpret_cast<uint32_t*>(&sd)[threadIdx.x] = word;
+        if (keep) reinterpret_cast<uint32_t*>(keep)[threadIdx.x] = word;
+    }
+};
+
+template <int THREADS, typename Descs>
+__device__ __forceinline__ void small_slots(const SmallShape& b, const SmallPlan& p, const Descs& descs, uint32_t entries,
                                             const Store& s, const OptDev& o, uint64_t seed, DevStatus* status,
                                             uint64_t* host_words, uint32_t seq) {
     extern __shared__ unsigned long long smem64[];
@@ -125,10 +145,8 @@ __device__ __forceinline__ void small_slots(const SmallShape& b, const SmallPlan
     const int sl = blockIdx.x / b.parts;
     const uint32_t part = blockIdx.x % b.parts;
     const uint32_t tid = threadIdx.x;
-    // the slot's descriptor comes straight out of the host's staging buffer (one round trip over the bus, in flight
-    // while the tables are cleared)
-    uint32_t dword = 0;
-    if (tid < sizeof(SlotDesc) / 4) dword = reinterpret_cast<const uint32_t*>(host_descs + sl)[tid];
+    DescFetch fetch;
+    fetch.start(descs, sl);
     for (uint32_t i = tid; i <= entries; i += THREADS) {
         keys[i] = EMPTY_KEY;
         word[i] = 0xFFFF0000u;
@@ -141,10 +159,7 @@ __device__ __forceinline__ void small_slots(const SmallShape& b, const SmallPlan
         if (tid < sizeof(DevStatus) / 4) reinterpret_cast<uint32_t*>(status)[tid] = 0;
         if (tid == 0) *p.bad = 0;
     }
-    if (tid < sizeof(SlotDesc) / 4) {
-        reinterpret_cast<uint32_t*>(&sd)[tid] = dword;
-        if (part == 0) reinterpret_cast<uint32_t*>(p.descs + sl)[tid] = dword;  // for the launches after this one
-    }
+    fetch.finish(descs, sl, sd, part == 0 ? p.descs + sl : nullptr);
     __syncthreads();
     const Global<const int64_t> values = as_global(sd.values);
     const uint32_t len = sd.len, lbase = sd.lbase;
@@ -266,15 +281,18 @@ __device__ __forceinline__ void small_slots(const SmallShape& b, const SmallPlan
     }
 }
 
-static __global__ __launch_bounds__(SMALL_THREADS) void k_small_slots(SmallShape b, SmallPlan p, const SlotDesc* host_descs,
-                                                               uint32_t entries, Store s, OptDev o, uint64_t seed,
-                                                               DevStatus* status, uint64_t* host_words, uint32_t seq) {
-    small_slots<SMALL_THREADS>(b, p, host_descs, entries, s, o, seed, status, host_words, seq);
+template <typename Descs>
+__global__ __launch_bounds__(SMALL_THREADS) void small_slots_kernel(SmallShape b, SmallPlan p, Descs descs, uint32_t entries, Store s,
+                                                                    OptDev o, uint64_t seed, DevStatus* status,
+                                                                    uint64_t* host_words, uint32_t seq) {
+    small_slots<SMALL_THREADS>(b, p, descs, entries, s, o, seed, status, host_words, seq);
 }
-static __global__ __launch_bounds__(2 * SMALL_THREADS) void k_small_slots_long(SmallShape b, SmallPlan p, const SlotDesc* host_descs,
-                                                                        uint32_t entries, Store s, OptDev o, uint64_t seed,
-                                                                        DevStatus* status, uint64_t* host_words, uint32_t seq) {
-    small_slots<2 * SMALL_THREADS>(b, p, host_descs, entries, s, o, seed, status, host_words, seq);
+template <typename Descs>
+__global__ __launch_bounds__(2 * SMALL_THREADS) void small_slots_long_kernel(SmallShape b, SmallPlan p, Descs descs,
+                                                                             uint32_t entries, Store s, OptDev o, uint64_t seed,
+                                                                             DevStatus* status, uint64_t* host_words,
+                                                                             uint32_t seq) {
+    small_slots<2 * SMALL_THREADS>(b, p, descs, entries, s, o, seed, status, host_words, seq);
 }
 
 // What is left of a small pull behind its first launch: small_emit_bucket, a workgroup per bucket, and small_finish.
@@ -529,9 +547,9 @@ __global__ __launch_bounds__(FINISH_THREADS) __attribute__((amdgpu_waves_per_eu(
 // any entry).  A mismatch also goes to the host (pinned memory); that the comparison is complete, the last launch tells it.
 // The workgroups behind those, a wavefront per bucket, put the ranks of the records' first lookups into the records: the
 // updates would otherwise read them through rank_at, a round trip more (the pull works ranks and records out side by side).
-template <bool CLICKS>
-__global__ __launch_bounds__(256) void k_small_verify(SmallShape b, SmallPlan p, const SlotDesc* host_descs, uint32_t chunks,
-                                                      DevStatus* status, uint32_t* host_mismatch) {
+template <bool CLICKS, typename Descs>
+__global__ __launch_bounds__(256) void small_verify_kernel(SmallShape b, SmallPlan p, Descs descs, uint32_t chunks,
+                                                           DevStatus* status, uint32_t* host_mismatch) {
     __shared__ SlotDesc sd;
     if (blockIdx.x >= b.N * chunks) {
         const uint32_t c = (blockIdx.x - b.N * chunks) * 4 + threadIdx.x / 64;
@@ -547,7 +565,7 @@ __global__ __launch_bounds__(256) void k_small_verify(SmallShape b, SmallPlan p,
     }
     const int sl = blockIdx.x / chunks;
     const uint32_t p0 = (blockIdx.x % chunks) * SMALL_TILE;
-    // what the pull left of these positions is on its way while the descriptor comes in from the host's staging buffer
+    // what the pull left of these positions is on its way while the descriptor comes in
     const uint32_t lbase = p.descs[sl].lbase, len = p.descs[sl].len;  // (the shape is the pull's)
     constexpr int PER = SMALL_TILE / 256;
     uint64_t now[PER], then[PER];
@@ -559,11 +577,9 @@ __global__ __launch_bounds__(256) void k_small_verify(SmallShape b, SmallPlan p,
         then[j] = pos < len ? p.vals_copy[lbase + pos] : 0;
         f[j] = CLICKS && pos < len ? p.first_of[lbase + pos] : 0u;
     }
-    if (threadIdx.x < sizeof(SlotDesc) / 4) {
-        const uint32_t w = reinterpret_cast<const uint32_t*>(host_descs + sl)[threadIdx.x];
-        reinterpret_cast<uint32_t*>(&sd)[threadIdx.x] = w;
-        if (p0 == 0) reinterpret_cast<uint32_t*>(p.push_descs + sl)[threadIdx.x] = w;  // for the launches after this one
-    }
+    DescFetch fetch;
+    fetch.start(descs, sl);
+    fetch.finish(descs, sl, sd, p0 == 0 ? p.push_descs + sl : nullptr);
     bool bad = false;
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         bad = *p.bad != 0;

@@ -57,6 +57,17 @@ struct SlotDesc {
     uint32_t tcap;          // entries of the slot's dedup table (+1 special)
 };
 
+// The descriptors of a call by value, among the arguments of its first kernel, where there are few enough: a workgroup has its slot's
+// 0.44 us after it starts, where out of the host's pinned buffer it is 1.56 (HostDescs; any number of slots).  The arguments of
+// a launch have 4 KB.
+constexpr int ARG_SLOTS = 52;
+struct ArgDescs {
+    SlotDesc slot[ARG_SLOTS];
+};
+struct HostDescs {
+    const SlotDesc* slot;
+};
+
 struct DedupEntry {
     uint64_t key;
     uint32_t minpos;  // smallest in-slot position of the sign

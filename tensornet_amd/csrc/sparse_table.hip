@@ -13,6 +13,7 @@
 #include <chrono>
 #include <cstring>
 #include <thread>
+#include <type_traits>
 
 // Device memory of tn_sparse_table_pull_static, the one entry point that allocates nothing: the call's
 // status block, then the row number and the new-row list of every requested sign.  Every GPU the library
@@ -1283,8 +1284,10 @@ bool small_batch_shape(SparseTable* t, int N, const int64_t* lens, SmallShape& b
     // room for twice the records expected of a batch of distinct signs and for four signs that are in every slot
     b.cap = (uint32_t)align_up(2 * (L / b.buckets()) + 64 + 4 * (size_t)N, 64);
     if (!t->small_lds) {
-        t->small_lds = big_lds_bytes_for(reinterpret_cast<const void*>(k_small_slots), 144 * 1024);
-        t->small_lds = std::min(t->small_lds, big_lds_bytes_for(reinterpret_cast<const void*>(k_small_slots_long), 144 * 1024));
+        t->small_lds = 144 * 1024;
+        for (const void* k : {(const void*)small_slots_kernel<ArgDescs>, (const void*)small_slots_kernel<HostDescs>,
+                              (const void*)small_slots_long_kernel<ArgDescs>, (const void*)small_slots_long_kernel<HostDescs>})
+            t->small_lds = std::min(t->small_lds, big_lds_bytes_for(k, 144 * 1024));
         t->small_emit_lds = big_lds_bytes_for(reinterpret_cast<const void*>(k_group_emit<true>), 144 * 1024);
     }
     return small_slots_lds(small_entries(b.max_len, b.parts), b.max_len, b.nbp) <= t->small_lds &&
@@ -1355,8 +1358,10 @@ int small_pull(SparseTable* t, const SmallShape& b, const int64_t* const* values
     TN_TRY(t->plan_buf.ensure(bytes));
     carve_small((char*)t->plan_buf.p, p, b);
     t->plan_valid = false;
-    TN_TRY(staging_free(t));
-    SlotDesc* descs = reinterpret_cast<SlotDesc*>(t->hstage);
+    const bool by_value = b.N <= ARG_SLOTS;
+    if (!by_value) TN_TRY(staging_free(t));
+    ArgDescs args;
+    SlotDesc* descs = by_value ? args.slot : reinterpret_cast<SlotDesc*>(t->hstage);
     int width = row_width(wdim, s.wstride);
     uint32_t at = 0;
     for (int i = 0; i < b.N; i++) {
@@ -1373,12 +1378,22 @@ int small_pull(SparseTable* t, const SmallShape& b, const int64_t* const* values
     }
     const uint32_t seq = ++t->seq_pull, workgroups = (uint32_t)b.N * b.parts, entries = small_entries(b.max_len, b.parts);
     const size_t slots_lds = small_slots_lds(entries, b.max_len, b.nbp);
-    if (b.max_len <= SMALL_SLOT_SHORT)
-        TN_LAUNCH_LDS(k_small_slots, dim3(workgroups), dim3(SMALL_THREADS), slots_lds, st, b, p, (const SlotDesc*)descs, entries,
-                      s, make_optdev(t), t->seed, t->dplan, t->hwords, seq);
+    auto launch_slots = [&](const auto& by) {
+        using Descs = std::decay_t<decltype(by)>;
+        // (the names the profiler knows them by)
+        constexpr auto k_small_slots = small_slots_kernel<Descs>;
+        constexpr auto k_small_slots_long = small_slots_long_kernel<Descs>;
+        if (b.max_len <= SMALL_SLOT_SHORT)
+            TN_LAUNCH_LDS(k_small_slots, dim3(workgroups), dim3(SMALL_THREADS), slots_lds, st, b, p, by, entries, s, make_optdev(t),
+                          t->seed, t->dplan, t->hwords, seq);
+        else
+            TN_LAUNCH_LDS(k_small_slots_long, dim3(workgroups), dim3(2 * SMALL_THREADS), slots_lds, st, b, p, by, entries, s,
+                          make_optdev(t), t->seed, t->dplan, t->hwords, seq);
+    };
+    if (by_value)
+        launch_slots(args);
     else
-        TN_LAUNCH_LDS(k_small_slots_long, dim3(workgroups), dim3(2 * SMALL_THREADS), slots_lds, st, b, p, (const SlotDesc*)descs,
-                      entries, s, make_optdev(t), t->seed, t->dplan, t->hwords, seq);
+        launch_slots(HostDescs{descs});
     const uint32_t C = (uint32_t)(wdim / width), items = (size_t)b.L * C > FINISH_FULL ? FINISH_ITEMS : 1;
     const uint32_t per = items * FINISH_THREADS / C, chunks = (b.max_len + per - 1) / per;
     EmitArgs<true> ea;
@@ -1456,8 +1471,10 @@ int small_push(SparseTable* t, const int64_t* const* values, const float* const*
     carve_small((char*)t->plan_buf.p, p, b);
     SmallPool pool{};
     if (pooled) TN_TRY(small_pool_room(t, dim, pool));
-    TN_TRY(staging_free(t));
-    SlotDesc* descs = reinterpret_cast<SlotDesc*>(t->hstage);
+    const bool by_value = b.N <= ARG_SLOTS;
+    if (!by_value) TN_TRY(staging_free(t));
+    ArgDescs args;
+    SlotDesc* descs = by_value ? args.slot : reinterpret_cast<SlotDesc*>(t->hstage);
     uint32_t at = 0;
     for (int i = 0; i < b.N; i++) {
         SlotDesc d{};
@@ -1476,12 +1493,25 @@ int small_push(SparseTable* t, const int64_t* const* values, const float* const*
     const uint32_t seq = ++t->seq_verify, chunks = (b.max_len + SMALL_TILE - 1) / SMALL_TILE;
     // (the records of pooled gradients go by their first lookups, not by rank)
     const uint32_t verify_blocks = (uint32_t)b.N * chunks + (pooled ? 0u : (b.buckets() + 3) / 4);
-    if (clicks)
-        TN_LAUNCH((k_small_verify<true>), dim3(verify_blocks), dim3(256), st, b, p, (const SlotDesc*)descs, chunks,
-                  t->dplan, &t->hpush->st.mismatch);
+    auto launch_verify = [&](const auto& by) {
+        using Descs = std::decay_t<decltype(by)>;
+#define TN_VERIFY(KERNEL, CLICKS)                                                                                          \
+    do {                                                                                                                   \
+        if (g_profile_on) prof_begin(KERNEL, st);                                                                          \
+        hipLaunchKernelGGL((small_verify_kernel<CLICKS, Descs>), dim3(verify_blocks), dim3(256), 0, st, b, p, by, chunks, \
+                           t->dplan, &t->hpush->st.mismatch);                                                              \
+        if (g_profile_on) prof_end(st);                                                                                    \
+    } while (0)
+        if (clicks)
+            TN_VERIFY("k_small_verify<true>", true);
+        else
+            TN_VERIFY("k_small_verify<false>", false);
+#undef TN_VERIFY
+    };
+    if (by_value)
+        launch_verify(args);
     else
-        TN_LAUNCH((k_small_verify<false>), dim3(verify_blocks), dim3(256), st, b, p, (const SlotDesc*)descs, chunks,
-                  t->dplan, &t->hpush->st.mismatch);
+        launch_verify(HostDescs{descs});
     const bool rows16 = dim % 4 == 0 && t->store.wstride % 4 == 0;
     if (pooled)
         launch_small_pool(t, vec, p, batch, dim, combiner, pool, st, &t->hpush->st.abort);
@@ -2551,7 +2581,6 @@ int tn_sparse_table_combine_op(uint32_t table_handle, int N, const int64_t* cons
         harvest(t);
     }
     set_last_stream(t, st);
-    TN_TRY(staging_free(t));
     // A workgroup per COMBINE_EXAMPLES examples of a slot where the chip holds them all at once, else per more of them, as long
     // as their lookups' rows fit in LDS: every workgroup pays for finding its lookups.  (211 slots of 2039 examples, 256 a
     // workgroup 21 us, 128 25, 64 32; 100 slots of 16384: 1024, which do not fit 167, 512 100, 256 108, 128 127.)
@@ -2563,9 +2592,18 @@ int tn_sparse_table_combine_op(uint32_t table_handle, int N, const int64_t* cons
     const int64_t items = (int64_t)N * per_slot;
     if (items > 0x7FFFFFF0LL) return fail(TN_ERR_UNSUPPORTED, "embedding combine: too many examples");
     const int grid = launch_grid(items, 1, GRID_CAP * 4);
-    std::memcpy(t->hstage, descs.data(), (size_t)N * sizeof(SlotDesc));
-    const SlotDesc* ddescs = reinterpret_cast<const SlotDesc*>(t->hstage);
-    if (grid > COMBINE_DIRECT) {  // (few workgroups read their slot's descriptor from the host's buffer themselves: a launch less)
+    ArgDescs args;
+    const SlotDesc* ddescs = nullptr;
+    const NoDescs none;
+    const bool by_value = N <= ARG_SLOTS;
+    if (by_value) {
+        std::copy(descs.begin(), descs.end(), args.slot);
+    } else {
+        TN_TRY(staging_free(t));
+        std::memcpy(t->hstage, descs.data(), (size_t)N * sizeof(SlotDesc));
+        ddescs = reinterpret_cast<const SlotDesc*>(t->hstage);
+    }
+    if (!by_value && grid > COMBINE_DIRECT) {  // (few workgroups read their slot's descriptor from the host's buffer themselves: a launch less)
         const size_t db = (size_t)N * sizeof(SlotDesc);
         TN_TRY(t->comb_buf.ensure(align_up(db, 256)));
         TN_LAUNCH(k_stage_in, dim3(launch_grid((int64_t)db / 4, 256, 64)), dim3(256), st,
@@ -2577,9 +2615,20 @@ int tn_sparse_table_combine_op(uint32_t table_handle, int N, const int64_t* cons
     int lanes = 1;
     while (lanes < 32 && 4 * lanes < dim) lanes *= 2;
     const bool any = !vec || dim % (4 * lanes) != 0;
-#define TN_LAUNCH_COMBINE_ANY(LPG, ANY)                                                                               \
-    TN_LAUNCH_LDS((k_combine_fwd<LPG, ANY>), dim3(grid), dim3(256), (size_t)per * 8, st, ddescs, (uint32_t)items, per_slot, \
-                  per, dim, batch, combiner, t->dcomb)
+#define TN_LAUNCH_COMBINE_BY(LPG, ANY, BY)                                                                                \
+    do {                                                                                                                  \
+        if (g_profile_on) prof_begin("k_combine_fwd<" #LPG ", " #ANY ">", st);                                            \
+        hipLaunchKernelGGL((combine_fwd_kernel<LPG, ANY, std::decay_t<decltype(BY)>>), dim3(grid), dim3(256), (size_t)per * 8, \
+                           st, BY, ddescs, (uint32_t)items, per_slot, per, dim, batch, combiner, t->dcomb);                       \
+        if (g_profile_on) prof_end(st);                                                                                   \
+    } while (0)
+#define TN_LAUNCH_COMBINE_ANY(LPG, ANY)                \
+    do {                                               \
+        if (by_value)                                  \
+            TN_LAUNCH_COMBINE_BY(LPG, ANY, args);      \
+        else                                           \
+            TN_LAUNCH_COMBINE_BY(LPG, ANY, none);      \
+    } while (0)
 #define TN_LAUNCH_COMBINE(LPG)                  \
     do {                                        \
         if (any)                                \
@@ -2597,6 +2646,7 @@ int tn_sparse_table_combine_op(uint32_t table_handle, int N, const int64_t* cons
     }
 #undef TN_LAUNCH_COMBINE
 #undef TN_LAUNCH_COMBINE_ANY
+#undef TN_LAUNCH_COMBINE_BY
     const uint32_t seq = ++t->seq_comb;
     TN_LAUNCH(k_report, dim3(1), dim3(64), st, t->dcomb, t->hcomb, seq);
     TN_HIP(hipGetLastError());
