@@ -1002,8 +1002,13 @@ __device__ __forceinline__ uint32_t wave_draw(uint32_t* counter) {
 // BIG: how the signs with many records are applied -- BIG_NONE, the plan lists none; BIG_GROUPS, rows of any length
 // (apply_big_groups); else rows of as many elements (apply_big_wave).
 enum { BIG_NONE = 0, BIG_GROUPS = -1 };
+// Wavefronts a SIMD: AdaGrad rows of 64 with signs of many records fit four (128 registers, none spilled; by itself the compiler
+// takes 146): 40 slots of 8192 lookups 46.0 -> 40.0 us, 26 of 1024 14.6 -> 14.1.  Others lose by it: without such signs 12 slots of
+// 4000 19.5 -> 21.1, Adam rows of 64 (20 spilled) 50.4 -> 60.8, rows of 32, 26 of 1024, AdaGrad 9.9 -> 10.5, Adam 9.4 -> 10.7.
+constexpr int small_apply_waves(int kind, int lpg, int big) { return kind == OPT_ADAGRAD && lpg == 16 && big > 0 ? 4 : 1; }
 template <int KIND, int LPG, bool ANY, int BIG>
-__global__ __launch_bounds__(256) void k_small_apply(SmallShape b, SmallPlan p, const float* flat, Store s,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(small_apply_waves(KIND, LPG, BIG), 8))) void k_small_apply(
+                                                     SmallShape b, SmallPlan p, const float* flat, Store s,
                                                      OptDev o, const DevStatus* __restrict__ status, uint32_t* host_seq,
                                                      uint32_t seq, int dim, int gbuf_floats, uint32_t wave_lds,
                                                      uint32_t wave_arrays) {
