@@ -137,7 +137,7 @@ static_assert(LDS_TILE < (1 << 12) && MAX_SLOTS < (1 << 12), "a tile record's fi
 // It also leaves the fingerprints of the batch's signs, which a push compares its own with (k_verify_values: one
 // per 64 strided lookups of a tile of 256 x 8, which are the lookups of the wavefronts w and w + 4 here), and,
 // with exact != nullptr, a copy of the signs.
-static_assert(LDS_TILE == VERIFY_TILE && TILE_THREADS == 512, "k_tile_dedup and k_verify_values fingerprint the same runs of lookups");
+static_assert(LDS_TILE == VERIFY_TILE && TILE_THREADS == 512 && VERIFY_THREADS % 256 == 0, "k_tile_dedup and k_verify_values fingerprint the same runs of lookups");
 constexpr int TILE_LDS_SLOTS = 128;  // up to this many slots their value pointers and bucket ranges sit in LDS
 constexpr int LDS_SPAN = 4096;       // first-level buckets one tile may touch (its LDS counters)
 // dynamic LDS of k_tile_dedup: lb[N + 1], then (few slots) the slots' value pointers and bucket ranges, then a

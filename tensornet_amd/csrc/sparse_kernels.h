@@ -1401,14 +1401,16 @@ struct Fingerprint {
         }
     }
 };
-constexpr int VERIFY_ITEMS = 8;
-constexpr int VERIFY_TILE = 256 * VERIFY_ITEMS;  // lookups per tile
+constexpr int VERIFY_TILE = 2048;  // lookups per tile
+// Threads of a tile's workgroup: where the chip holds all tiles at once, twice as many with half as much each.  420 tiles 21.2 us
+// with 256 threads, 15.3 with 512; 1024 tiles 31.4 and 29.2; 2440 tiles 64.1 and 67.6.
+constexpr int VERIFY_THREADS = 256, VERIFY_THREADS_FEW = 512, VERIFY_FEW_TILES = 1024;
 constexpr int CLICK_BITS = 11;
 constexpr int CLICK_TABLE = 1 << CLICK_BITS;     // entries of the tile's click table
 constexpr int CLICK_TRIES = 16;
 
-template <bool CLICKS, bool COPY>
-__global__ __launch_bounds__(256) void k_verify_values(const SlotDesc* __restrict__ descs,
+template <bool CLICKS, bool COPY, int THREADS>
+__global__ __launch_bounds__(THREADS) void k_verify_values(const SlotDesc* __restrict__ descs,
                                                        const uint32_t* __restrict__ lbase, int N, uint32_t L,
                                                        const uint64_t* __restrict__ vals_copy, DevStatus* status,
                                                        const uint32_t* __restrict__ u_of_gi,
@@ -1418,6 +1420,9 @@ __global__ __launch_bounds__(256) void k_verify_values(const SlotDesc* __restric
     extern __shared__ uint32_t lb[];  // lb[N + 1], sized by the launch: more tiles in flight per CU than with a fixed array
     __shared__ uint32_t ckey[CLICKS ? CLICK_TABLE : 1];
     __shared__ int csum[CLICKS ? CLICK_TABLE : 1];
+    // a tile's fingerprints are four: of the lookups of wavefronts w, w + 4 .. (of its 2048 by fours of wavefronts)
+    constexpr int VERIFY_ITEMS = VERIFY_TILE / THREADS, FOURS = THREADS / 256;
+    __shared__ ulonglong2 prints[FOURS > 1 ? FOURS : 1][4];
     __shared__ uint32_t crowded;  // a label of the tile went to memory directly: its record's sum in the table is not all of it
     load_lbase(lb, lbase, N);
     bool bad = false;
@@ -1425,7 +1430,7 @@ __global__ __launch_bounds__(256) void k_verify_values(const SlotDesc* __restric
     const uint32_t ntiles = (L + VERIFY_TILE - 1) / VERIFY_TILE;
     for (uint32_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
         if (CLICKS) {
-            for (int i = threadIdx.x; i < CLICK_TABLE; i += 256) {
+            for (int i = threadIdx.x; i < CLICK_TABLE; i += THREADS) {
                 ckey[i] = 0xFFFFFFFFu;  // no distinct index: they stay below FIRST_BIT
                 csum[i] = 0;
             }
@@ -1441,7 +1446,7 @@ __global__ __launch_bounds__(256) void k_verify_values(const SlotDesc* __restric
         uint32_t u[VERIFY_ITEMS];
 #pragma unroll
         for (int j = 0; j < VERIFY_ITEMS; j++) {
-            const uint32_t gi = g0 + j * 256 + threadIdx.x;
+            const uint32_t gi = g0 + j * THREADS + threadIdx.x;
             now[j] = then[j] = 0;
             label[j] = 0;
             u[j] = 0;
@@ -1466,12 +1471,17 @@ __global__ __launch_bounds__(256) void k_verify_values(const SlotDesc* __restric
             Fingerprint print;
 #pragma unroll
             for (int j = 0; j < VERIFY_ITEMS; j++) {
-                const uint32_t gi = g0 + j * 256 + threadIdx.x;
+                const uint32_t gi = g0 + j * THREADS + threadIdx.x;
                 if (gi <= g1) print.add(gi, now[j]);
             }
             print.wave_sum();
-            const ulonglong2 left = reinterpret_cast<const ulonglong2*>(vals_copy)[tile * (256 / 64) + (threadIdx.x >> 6)];
-            bad |= print.a != left.x || print.b != left.y;
+            const uint32_t wave = threadIdx.x >> 6;
+            if (FOURS > 1) {  // (added up behind the next barrier)
+                if ((threadIdx.x & 63) == 0) prints[wave / 4][wave % 4] = make_ulonglong2(print.a, print.b);
+            } else {
+                const ulonglong2 left = reinterpret_cast<const ulonglong2*>(vals_copy)[tile * 4 + wave];
+                bad |= print.a != left.x || print.b != left.y;
+            }
         }
 #pragma unroll
         for (int j = 0; j < VERIFY_ITEMS; j++) {
@@ -1494,14 +1504,25 @@ __global__ __launch_bounds__(256) void k_verify_values(const SlotDesc* __restric
                 }
             }
         }
+        constexpr bool ADD_PRINTS = !COPY && FOURS > 1;
+        if (CLICKS || ADD_PRINTS) __syncthreads();
+        if (ADD_PRINTS && threadIdx.x < 4) {
+            const ulonglong2 left = reinterpret_cast<const ulonglong2*>(vals_copy)[tile * 4 + threadIdx.x];
+            ulonglong2 sum = make_ulonglong2(0, 0);
+#pragma unroll
+            for (int f = 0; f < FOURS; f++) {
+                const ulonglong2 v = prints[f][threadIdx.x];
+                sum = make_ulonglong2(sum.x + v.x, sum.y + v.y);
+            }
+            bad |= sum.x != left.x || sum.y != left.y;
+        }
         if (CLICKS) {
-            __syncthreads();
-            constexpr int PER = CLICK_TABLE / 256;
+            constexpr int PER = CLICK_TABLE / THREADS;
             uint32_t place[PER];
             int sum[PER];
 #pragma unroll
             for (int j = 0; j < PER; j++) {
-                const int e = j * 256 + threadIdx.x;
+                const int e = j * THREADS + threadIdx.x;
                 sum[j] = csum[e];
                 place[j] = sum[j] != 0 ? where_u[ckey[e]].x : 0u;
             }
@@ -1516,8 +1537,8 @@ __global__ __launch_bounds__(256) void k_verify_values(const SlotDesc* __restric
                 else
                     atomicAdd(&list[place[j] & WHERE_PLACE].click, sum[j]);
             }
-            __syncthreads();
         }
+        if (CLICKS || ADD_PRINTS) __syncthreads();
     }
     if (bad) {
         atomicOr(&status->mismatch, 1u);

@@ -2444,10 +2444,21 @@ int push_op_impl(uint32_t table_handle, int N, const int64_t* const* values, con
         const PushSrc vsrc = op_source(p, grad_dim, true);
         const bool addr_in_verify = !pooled && t->plan_big_k != 0xFFFFFFFFu;
         const float** vgaddr = addr_in_verify ? p.gaddr : nullptr;
-        // (a macro: the profiler names a kernel by the text of its launch)
-#define TN_VERIFY(CLICKS, COPY)                                                                                      \
-    TN_LAUNCH_LDS_EVENT(behind, (k_verify_values<CLICKS, COPY>), dim3(vblocks), dim3(256), vlds, st, pd, p.lbase, N,  \
-                        (uint32_t)L, then_vals, ds, p.u_of_gi, p.where_u, p.list, host_mismatch, vsrc, vgaddr)
+#define TN_VERIFY_BY(CLICKS, COPY, THREADS)                                                                         \
+    do {                                                                                                            \
+        if (g_profile_on) prof_begin("k_verify_values<" #CLICKS ", " #COPY ">", st);                                \
+        launch_signalling(behind, k_verify_values<CLICKS, COPY, THREADS>, dim3(vblocks), dim3(THREADS), vlds, st, pd, p.lbase, N, \
+                          (uint32_t)L, then_vals, ds, p.u_of_gi, p.where_u, p.list, host_mismatch, vsrc, vgaddr);    \
+        if (g_profile_on) prof_end(st);                                                                             \
+    } while (0)
+#define TN_VERIFY(CLICKS, COPY)                                      \
+    do {                                                             \
+        if (few)                                                     \
+            TN_VERIFY_BY(CLICKS, COPY, VERIFY_THREADS_FEW);          \
+        else                                                         \
+            TN_VERIFY_BY(CLICKS, COPY, VERIFY_THREADS);              \
+    } while (0)
+        const bool few = (L + VERIFY_TILE - 1) / VERIFY_TILE <= (size_t)VERIFY_FEW_TILES;
         const bool copy = !t->plan_prints || t->plan_exact;
         const uint64_t* then_vals = t->plan_exact ? p.vals_exact : p.vals_copy;
         if (clicks) {
@@ -2463,6 +2474,7 @@ int push_op_impl(uint32_t table_handle, int N, const int64_t* const* values, con
         } else {
             TN_VERIFY(false, false);
         }
+#undef TN_VERIFY_BY
 #undef TN_VERIFY
         // Counts and apply kernels are queued before the host knows the outcome: the counts only
         // touch the plan's member lists, which a mismatch discards anyway, and the apply kernels
