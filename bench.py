@@ -108,7 +108,7 @@ def kernel_algorithmic_bytes(name, opt, dim, shape):
         "k_gather_vars": U * (2 * row + 4),    # row read + variable row write
         # push
         # the op's signs and labels, against the pull's copy of the signs (COPY) or its fingerprints of them
-        "k_verify_values": (24 * L if name.endswith(", true>") else 16 * L + L // 32),
+        "k_verify_values": (24 * L if "".join(name.split(",")[1:2]).strip(" >") == "true" else 16 * L + L // 32),
         "k_reset_counts": 8 * U,
         "k_apply_single": apply_bytes(shape["G1"], shape["G1"]),
         "k_apply_vec": apply_bytes(shape["Rm"], shape["Gm"]),

@@ -88,7 +88,7 @@ __device__ __forceinline__ const SlotDesc& desc_of(const NoDescs&, const SlotDes
 constexpr uint32_t COMBINE_IDS = 2048;
 constexpr uint32_t COMBINE_AHEAD = 2;  // lookups of a thread in flight while they are checked
 template <int LPG, bool ANY, typename Descs>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ANY ? 6 : 7, 8))) void combine_fwd_kernel(Descs by_value, const SlotDesc* __restrict__ descs, uint32_t items, uint32_t per_slot,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ANY ? 6 : 7, 8))) void k_combine_fwd(Descs by_value, const SlotDesc* __restrict__ descs, uint32_t items, uint32_t per_slot,
                                                      uint32_t per, int dim, int64_t batch, int combiner, DevStatus* status) {
     extern __shared__ uint32_t range[];  // [per] first lookup of an example, [per] the lookup after its last
     __shared__ uint32_t row[COMBINE_IDS];

@@ -282,13 +282,13 @@ __device__ __forceinline__ void small_slots(const SmallShape& b, const SmallPlan
 }
 
 template <typename Descs>
-__global__ __launch_bounds__(SMALL_THREADS) void small_slots_kernel(SmallShape b, SmallPlan p, Descs descs, uint32_t entries, Store s,
+__global__ __launch_bounds__(SMALL_THREADS) void k_small_slots(SmallShape b, SmallPlan p, Descs descs, uint32_t entries, Store s,
                                                                     OptDev o, uint64_t seed, DevStatus* status,
                                                                     uint64_t* host_words, uint32_t seq) {
     small_slots<SMALL_THREADS>(b, p, descs, entries, s, o, seed, status, host_words, seq);
 }
 template <typename Descs>
-__global__ __launch_bounds__(2 * SMALL_THREADS) void small_slots_long_kernel(SmallShape b, SmallPlan p, Descs descs,
+__global__ __launch_bounds__(2 * SMALL_THREADS) void k_small_slots_long(SmallShape b, SmallPlan p, Descs descs,
                                                                              uint32_t entries, Store s, OptDev o, uint64_t seed,
                                                                              DevStatus* status, uint64_t* host_words,
                                                                              uint32_t seq) {
@@ -548,7 +548,7 @@ __global__ __launch_bounds__(FINISH_THREADS) __attribute__((amdgpu_waves_per_eu(
 // The workgroups behind those, a wavefront per bucket, put the ranks of the records' first lookups into the records: the
 // updates would otherwise read them through rank_at, a round trip more (the pull works ranks and records out side by side).
 template <bool CLICKS, typename Descs>
-__global__ __launch_bounds__(256) void small_verify_kernel(SmallShape b, SmallPlan p, Descs descs, uint32_t chunks,
+__global__ __launch_bounds__(256) void k_small_verify(SmallShape b, SmallPlan p, Descs descs, uint32_t chunks,
                                                            DevStatus* status, uint32_t* host_mismatch) {
     __shared__ SlotDesc sd;
     if (blockIdx.x >= b.N * chunks) {

@@ -1285,8 +1285,8 @@ bool small_batch_shape(SparseTable* t, int N, const int64_t* lens, SmallShape& b
     b.cap = (uint32_t)align_up(2 * (L / b.buckets()) + 64 + 4 * (size_t)N, 64);
     if (!t->small_lds) {
         t->small_lds = 144 * 1024;
-        for (const void* k : {(const void*)small_slots_kernel<ArgDescs>, (const void*)small_slots_kernel<HostDescs>,
-                              (const void*)small_slots_long_kernel<ArgDescs>, (const void*)small_slots_long_kernel<HostDescs>})
+        for (const void* k : {(const void*)k_small_slots<ArgDescs>, (const void*)k_small_slots<HostDescs>,
+                              (const void*)k_small_slots_long<ArgDescs>, (const void*)k_small_slots_long<HostDescs>})
             t->small_lds = std::min(t->small_lds, big_lds_bytes_for(k, 144 * 1024));
         t->small_emit_lds = big_lds_bytes_for(reinterpret_cast<const void*>(k_group_emit<true>), 144 * 1024);
     }
@@ -1381,8 +1381,8 @@ int small_pull(SparseTable* t, const SmallShape& b, const int64_t* const* values
     auto launch_slots = [&](const auto& by) {
         using Descs = std::decay_t<decltype(by)>;
         // (the names the profiler knows them by)
-        constexpr auto k_small_slots = small_slots_kernel<Descs>;
-        constexpr auto k_small_slots_long = small_slots_long_kernel<Descs>;
+        constexpr auto k_small_slots = tn::k_small_slots<Descs>;
+        constexpr auto k_small_slots_long = tn::k_small_slots_long<Descs>;
         if (b.max_len <= SMALL_SLOT_SHORT)
             TN_LAUNCH_LDS(k_small_slots, dim3(workgroups), dim3(SMALL_THREADS), slots_lds, st, b, p, by, entries, s, make_optdev(t),
                           t->seed, t->dplan, t->hwords, seq);
@@ -1498,7 +1498,7 @@ int small_push(SparseTable* t, const int64_t* const* values, const float* const*
 #define TN_VERIFY(KERNEL, CLICKS)                                                                                          \
     do {                                                                                                                   \
         if (g_profile_on) prof_begin(KERNEL, st);                                                                          \
-        hipLaunchKernelGGL((small_verify_kernel<CLICKS, Descs>), dim3(verify_blocks), dim3(256), 0, st, b, p, by, chunks, \
+        hipLaunchKernelGGL((k_small_verify<CLICKS, Descs>), dim3(verify_blocks), dim3(256), 0, st, b, p, by, chunks, \
                            t->dplan, &t->hpush->st.mismatch);                                                              \
         if (g_profile_on) prof_end(st);                                                                                    \
     } while (0)
@@ -2630,7 +2630,7 @@ int tn_sparse_table_combine_op(uint32_t table_handle, int N, const int64_t* cons
 #define TN_LAUNCH_COMBINE_BY(LPG, ANY, BY)                                                                                \
     do {                                                                                                                  \
         if (g_profile_on) prof_begin("k_combine_fwd<" #LPG ", " #ANY ">", st);                                            \
-        hipLaunchKernelGGL((combine_fwd_kernel<LPG, ANY, std::decay_t<decltype(BY)>>), dim3(grid), dim3(256), (size_t)per * 8, \
+        hipLaunchKernelGGL((k_combine_fwd<LPG, ANY, std::decay_t<decltype(BY)>>), dim3(grid), dim3(256), (size_t)per * 8, \
                            st, BY, ddescs, (uint32_t)items, per_slot, per, dim, batch, combiner, t->dcomb);                       \
         if (g_profile_on) prof_end(st);                                                                                   \
     } while (0)
