@@ -575,7 +575,7 @@ struct Carver {
 struct Plan {
     SlotDesc* descs;
     SlotDesc* push_descs;  // descriptors of the push that reuses the plan (the pull's gather may still read `descs`)
-    uint32_t* push_ubase;  // ... and its copy of ubase, which its status is published from (the next pull rewrites ubase)
+    uint32_t* push_ubase;  // ... and its copy of ubase (the next pull rewrites ubase, detached updates may still run then)
     uint32_t* lbase;
     uint32_t* ubase;
     uint64_t* vals_copy;   // signs of every lookup, concatenated; after a pull through LDS their fingerprints instead
@@ -1639,7 +1639,7 @@ int tn_sparse_table_key_count(uint32_t handle, uint64_t* count) {
     *count = 0;
     if (!t->allocated) return TN_OK;
     // Only this table's own work is waited for: the count is kept by kernels on the stream of the table's last
-    // call (a pull that publishes its status on the side stream has waited for that before it returned).
+    // call (a pull has waited for its status before it returned).
     if (t->push_pending || t->pull_pending) {
         TN_HIP(hipStreamSynchronize(t->last_stream));
         harvest(t);

@@ -198,9 +198,19 @@ def main():
             ""]
     with open(args.out, "w") as f:
         f.write("\n".join(out))
+    # kernels of the library that this workload no longer launches (other batches and options do) keep their last figures
+    kept = {}
+    if os.path.exists(args.traffic):
+        with open(args.traffic) as f:
+            old = json.load(f)
+        kept = {k: c for k, c in old.get("kept_from", {}).items() if k not in traffic}
+        for k, v in old["bytes_per_launch"].items():
+            if k not in traffic:
+                traffic[k] = v
+                kept.setdefault(k, old["commit"])
     with open(args.traffic, "w") as f:
         json.dump({"commit": commit, "fetch_factor": round(ff, 4), "write_factor": round(wf, 4),
-                   "workload": line["config"]["workload"], "bytes_per_launch": traffic}, f, indent=1, sort_keys=True)
+                   "workload": line["config"]["workload"], "bytes_per_launch": traffic, "kept_from": kept}, f, indent=1, sort_keys=True)
         f.write("\n")
     print("wrote %s and %s (%d kernels)" % (args.out, args.traffic, len(traffic)))
 
