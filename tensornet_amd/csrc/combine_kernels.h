@@ -15,6 +15,7 @@
 #ifndef TN_COMBINE_KERNELS_H_
 #define TN_COMBINE_KERNELS_H_
 
+#include "lookup_range.h"
 #include "pool_items.h"
 
 #include <algorithm>
@@ -75,7 +76,8 @@ __device__ __forceinline__ uint2 ids_below(Global<const int64_t> ex, uint32_t n,
 // The example ids are checked on the way: the workgroups' shares of a slot's lookups follow each other without a gap
 // whatever the ids are (each ends where ids_below puts the start of the next, the first starts at 0, the last ends at
 // the slot's end), so every lookup is looked at by one workgroup, which wants it to lie among its examples and not
-// before its predecessor.  The same pass checks the mapped ids and leaves them in LDS where they fit (COMBINE_IDS): read where
+// before its predecessor; what is summed lies among the lookups it looked at even where it refused some (lookup_range: a position
+// ahead of them would be an index in front of `row`).  The same pass checks the mapped ids and leaves them in LDS where they fit (COMBINE_IDS): read where
 // they are used, by every lane of a group, they were a round trip in front of every example's rows.  Rows of 16, 4.9 M lookups
 // 121 -> 100 us, 860 k 29 -> 21, 20 k (104 workgroups) 7.9 -> 7.1.
 //
@@ -144,7 +146,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ANY ? 6 : 7
         __syncthreads();
         const float* __restrict__ rows = d.grads;
         for (uint32_t e = threadIdx.x / LPG; e < nb; e += 256 / LPG) {
-            const uint32_t from = range[e], to = max(range[per + e], from);
+            const LookupRange mine = lookup_range(range[e], range[per + e], lo);
+            const uint32_t from = mine.from, to = mine.to;
             const float div = combine_divisor(to - from, combiner);
             float* o = d.var + (b0 + e) * dim;
             for (int c0 = 0; c0 < dim; c0 += 4 * LPG) {  // (rows of more than 128 elements: once more for the next ones)
