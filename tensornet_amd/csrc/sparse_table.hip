@@ -463,15 +463,15 @@ void harvest(SparseTable* t) {
         t->pull_pending = false;
         const HostStatus& h = *t->hpull;
         int N = t->pull_slots;
-        t->plan_heavy = h.st.heavy != 0;
         // the call booked room for every sign it could have inserted; keep what it did insert
         if (t->booked >= h.st.n_new) t->count_upper -= t->booked - h.st.n_new;
         t->booked = 0;
         t->last_counts.assign(N, 0);
         for (int s = 0; s < N; s++) t->last_counts[s] = (int64_t)h.ubase[s + 1] - (int64_t)h.ubase[s];
-        t->plan_counts = t->last_counts;
-        t->plan_frequent = t->pull_lookups >= OWN_BIG_LOOKUPS * h.ubase[N];
-        if (t->pull_lookups > 0) {
+        if (N > 0) {  // (a pull of the table or a load of rows has no slots: the last pull's plan stands, and so does what is known of it)
+            t->plan_heavy = h.st.heavy != 0;
+            t->plan_counts = t->last_counts;
+            t->plan_frequent = t->pull_lookups >= OWN_BIG_LOOKUPS * h.ubase[N];
             note_distinct_share(t, (double)h.ubase[N] / (double)t->pull_lookups);
             if (h.st.tile_share_q16 != 0) {  // (a pull through LDS with a slot of more than one bucket)
                 const double share = (double)h.st.tile_share_q16 / 65536.0;
