@@ -171,6 +171,7 @@ struct SparseTable {
     hipEvent_t tail_ev = nullptr;
     bool tail_recorded = false;
     bool tail_owed = false;         // ... was on the default stream, which is there for good: recorded when another stream asks
+    bool several_streams = false;   // a call has come on another stream than the one before it
     bool plan_clicks_dirty = false;  // a push has added clicks to the member lists of the current plan
     // Distinct records per lookup seen by the recent pulls (1 = every lookup distinct, the safe start):
     // sizes the number of second-level buckets, whose room is fixed.  A batch with more distinct
@@ -372,6 +373,7 @@ void set_last_stream(SparseTable* t, hipStream_t st) {
 // push's updates, a decay: tail_ev) is waited for on the device, and a call whose status is still pending on the host.
 int order_after_other_stream(SparseTable* t, hipStream_t st) {
     if (!other_stream(t, st)) return TN_OK;
+    t->several_streams = true;
     if (t->tail_owed) {
         TN_HIP(hipEventRecord(t->tail_ev, nullptr));
         t->tail_owed = false;
@@ -382,13 +384,16 @@ int order_after_other_stream(SparseTable* t, hipStream_t st) {
     return TN_OK;
 }
 
-// What the last kernel of a call signals for calls on other streams.  On the default stream nothing: that one can neither be
-// destroyed nor captured, so the event can be recorded there by the call that needs it, later than it would have been and
-// therefore behind more.  (A launch with an event takes the host 1.6 us longer, in front of the kernel.)
+// What the last kernel of a call signals for calls on other streams.  On the default stream nothing as long as the table has had no
+// calls on others: that one can neither be destroyed nor captured, so the event can be recorded there by the call that needs
+// it.  That one call waits for whatever has been queued there meanwhile; from then on every call leaves its event again, so that
+// calls on a stream of their own beside a training loop on the default one wait for the table's kernels alone.  (A launch with an
+// event takes the host 1.6 us longer, in front of the kernel.)
 hipEvent_t tail_event(SparseTable* t, hipStream_t st) {
-    t->tail_owed = st == nullptr;
-    if (st) t->tail_recorded = true;
-    return st ? t->tail_ev : nullptr;
+    t->tail_owed = st == nullptr && !t->several_streams;
+    if (t->tail_owed) return nullptr;
+    t->tail_recorded = true;
+    return t->tail_ev;
 }
 
 // beside_updates: the caller (the pull op) orders its stream behind detached updates itself, as late as it can.
@@ -1616,6 +1621,7 @@ int tn_sparse_table_clear(uint32_t handle) {
     t->allocated = false;
     t->plan_valid = false;
     t->tail_recorded = false;
+    t->tail_owed = false;
     t->count_upper = 0;
     t->booked = 0;
     t->epoch++;
