@@ -33,11 +33,6 @@ constexpr double RESERVE_LOAD = 0.5;                    // what a reservation is
 constexpr uint64_t DEFAULT_SLOTS = 8ull * 15485863ull;  // optimizer_kernel.h:43,263
 constexpr uint64_t MAX_SLOTS_PER_TABLE = 0xFFFFFFF0ull; // rows are addressed with 32 bits
 constexpr size_t DETACH_LOOKUPS = 3u << 20;  // lookups of a push from which its updates may be detached
-// A batch of as many lookups whose slots have every sign some hundred times has the signs with many records in a launch of their
-// own (k_apply_big_adagrad, which detached updates use): tests/test_gpu_big_groups.py counts on it there.  The one launch for
-// all signs would do: 3.2 M lookups of 70 slots over 300 signs, rows of 16, a step 132 us, with a launch of their own 139; 3.5 M
-// of 88 slots over 2000 signs 188 and 196, over 250 k (not such a batch) 567 and 582.
-constexpr uint64_t OWN_BIG_LOOKUPS = 256;
 constexpr uint32_t SELF_SCAN_TILES = 8192;  // tiles of the ranking pass up to which no scan kernel runs between its launches
 constexpr int GRID_CAP = 256 * 8;                       // 256 CUs x 8 workgroups of 256 threads
 constexpr int TILE_GRID = 256 * 4;                      // workgroups of k_tile_dedup: what the chip holds of it at once
@@ -147,7 +142,6 @@ struct SparseTable {
     bool plan_exact = false;   // the plan holds such a copy
     uint32_t plan_big_k = BIG_GROUP_DEFAULT;  // records from which the plan lists a sign as one for k_apply_big
     bool plan_big_desc = false;               // the plan's big_desc goes with its big_list (a pull grouped through LDS)
-    bool plan_frequent = false;               // the plan's records have OWN_BIG_LOOKUPS lookups or more on average
     hipStream_t side = nullptr;     // the signs with several records of detached updates are applied here
     hipStream_t aux = nullptr;      // k_apply_single of detached updates runs here
     hipEvent_t fork_ev = nullptr;   // detached updates may start
@@ -476,7 +470,6 @@ void harvest(SparseTable* t) {
         if (N > 0) {  // (a pull of the table or a load of rows has no slots: the last pull's plan stands, and so does what is known of it)
             t->plan_heavy = h.st.heavy != 0;
             t->plan_counts = t->last_counts;
-            t->plan_frequent = t->pull_lookups >= OWN_BIG_LOOKUPS * h.ubase[N];
             note_distinct_share(t, (double)h.ubase[N] / (double)t->pull_lookups);
             if (h.st.tile_share_q16 != 0) {  // (a pull through LDS with a slot of more than one bucket)
                 const double share = (double)h.st.tile_share_q16 / 65536.0;
@@ -1011,7 +1004,9 @@ constexpr int ALL_BIG_GRID = 1024;
 // The signs with many records, with a few and with one: one launch (k_apply_all) where a row fits the lanes of a wavefront half.
 // Above 3 M lookups they were three launches on two streams until the pull needed no second stream: 4.9 M of 100 slots, rows of
 // 16, a step 527 us and 516 as one launch, with pooled gradients 881 and 856; 3.2 M of 70 slots over 300 signs 168 and 132;
-// 3.5 M of 88 over 250 k, rows of 64, 1107 and 1132, the only batch found that loses.
+// 3.5 M of 88 over 250 k, rows of 64, 1107 and 1132, the only batch found that loses.  (With a launch of their own for the signs
+// with many records ahead of the others': 3.2 M of 70 slots over 150 signs, rows of 16 127 and 123, of 64 133 and 135; 4 M of 40
+// over 350, rows of 32, 154 and 151; 4.9 M of 100 over 50, rows of 8, 143 and 143.)
 //
 // detach: the three kernels one by one on streams of the table's own, which the caller's does not wait for -- k_apply_single on
 // the auxiliary stream, the others on the side stream; the caller of this function records their end (SparseTable::upd_ev).
@@ -1043,8 +1038,7 @@ int launch_apply_kind(SparseTable* t, RowShare share, const Store& s, const OptD
     // AdaGrad rows of a power-of-two dim on a plan that describes its frequent signs have kernels of their own
     const bool tiled = KIND == OPT_ADAGRAD && big_desc && s.D >= 4 && s.D <= 64 && (s.D & (s.D - 1)) == 0;
     const bool all = with_big && !detach && share.lanes != 0;
-    const bool own_big = with_big && (!all || (tiled && t->plan_frequent && (size_t)n_upper >= DETACH_LOOKUPS));
-    if (own_big) {
+    if (with_big && !all) {
         const int gfloats = big_gbuf_floats(s.D);
         const int big_blocks = launch_grid(n_upper / BIG_GROUP + 1, 1, 16384);
         hipStream_t bst = detach ? t->side : st;
@@ -1063,7 +1057,7 @@ int launch_apply_kind(SparseTable* t, RowShare share, const Store& s, const OptD
     }
     if (all) {
         ApplyAll a;
-        a.big_blocks = own_big ? 0 : (uint32_t)launch_grid((n_upper / BIG_GROUP + 4) / 4, 1, ALL_BIG_GRID);
+        a.big_blocks = (uint32_t)launch_grid((n_upper / BIG_GROUP + 4) / 4, 1, ALL_BIG_GRID);
         a.multi_blocks = (uint32_t)launch_grid(n_upper * share.lanes / 2, 256, GRID_CAP * 2);
         const uint32_t singles = (uint32_t)launch_grid(n_upper * share.lanes, 256, GRID_CAP * 2);
         a.grp_row = p.grp_row, a.grp_off = p.grp_off, a.grp_cnt = p.grp_cnt, a.big_list = p.big_list;

@@ -1,7 +1,7 @@
 """Signs with many records -- one in most slots of the batch -- on the large-batch path, where a wavefront
 owns each of them: AdaGrad rows of every power-of-two dim from 4 to 64 (apply_big_wave, in chunks of 8 to 64 records,
-so 70 records are several chunks, the last one partial; k_apply_all, and k_apply_big_adagrad<D> for batches of millions of
-lookups), a dim with its own general kernel (12), Adam; with the two cvm columns; all against the CPU oracle, record by record in slot
+so 70 records are several chunks, the last one partial; k_apply_all, and k_apply_big_adagrad<D> where the updates of millions
+of lookups are detached), a dim with its own general kernel (12), Adam; with the two cvm columns; all against the CPU oracle, record by record in slot
 order (core/kernels/sparse_table_ops.cc:336-367, core/ps/table/sparse_table.cc:68-83,
 core/ps/optimizer/ada_grad_kernel.cc:105-129): rows within 1e-5 relative / 1e-7 absolute, more than 99 % of them
 bit for bit."""
@@ -65,10 +65,12 @@ def test_signs_in_most_slots_on_the_large_batch_path(tn, oracle, opt, hyper, dim
 
 
 @pytest.mark.parametrize("dim", [4, 8, 16, 32, 64])
-def test_signs_in_most_slots_of_millions_of_lookups(tn, oracle, dim):
+@pytest.mark.parametrize("detached", [True, False])
+def test_signs_in_most_slots_of_millions_of_lookups(tn, oracle, dim, detached):
     """Signs with one record and with every number of records up to one in each of the 70 slots, 45 200 lookups a slot."""
     rng = np.random.default_rng(dim)
     pair = Pair(tn, oracle, "AdaGrad", dim, ADAGRAD_HP, reserve=100000, zero_init=True)
+    tn.core.set_sparse_table_detached_updates(pair.h, detached)
     pool = synth.splitmix64(np.arange(1, 2001, dtype=np.uint64)).view(np.int64)
     pair.populate(pool[:1500].view(np.uint64))
     values = []
@@ -80,5 +82,5 @@ def test_signs_in_most_slots_of_millions_of_lookups(tn, oracle, dim):
         grads = synth.make_grads(counts, pair.wf, 0.05, seed=step)
         labels = [(rng.random(len(v)) < 0.3).astype(np.int64) for v in values]
         names = kernels_of(tn, lambda: pair.push_op(values, grads, labels))
-        assert any(k.startswith("k_apply_big_adagrad") for k in names)
+        assert any(k.startswith("k_apply_big_adagrad" if detached else "k_apply_all") for k in names)
         assert pair.assert_rows_match(all_signs(values)) > 0.99
