@@ -32,7 +32,7 @@ def log(msg):
 # profiles/cfg3_adagrad_dim16_pull_push.md (counters cannot be read from inside this script).
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "cfg3_traffic.json")
 # launched by a step, a few microseconds each, no traffic worth counting
-SMALL_STEP_KERNELS = ("k_stage_in", "k_publish", "k_init_new_recs", "k_assign_init", "k_group_offsets", "k_scan_tiles")
+SMALL_STEP_KERNELS = ("k_stage_in", "k_publish", "k_assign_init", "k_group_offsets", "k_scan_tiles")
 
 
 def measured_traffic(step_kernels):
@@ -64,10 +64,9 @@ def step_algorithmic_bytes(opt, dim, L, U):
     return 32 * L + U * (8 + 8 * dim + 4 * dim + 8 + 8 * dim + state_bytes(opt, dim))
 
 
-# Launched on the table's side stream, concurrently with kernels of the caller's stream (the other
-# update kernels).
-SIDE_STREAM_KERNELS = ("k_apply_single",)
-BIG_GROUP = 16  # records from which a sign is applied by k_apply_big (sparse_table.hip)
+# Launched on the table's own streams, beside kernels of the caller's, where updates are detached.
+SIDE_STREAM_KERNELS = ("k_apply_single", "k_apply_vec", "k_apply_big")
+BIG_GROUP = 16  # records from which a sign is one with many records (sparse_table.hip)
 
 
 def kernel_algorithmic_bytes(name, opt, dim, shape):
@@ -92,7 +91,6 @@ def kernel_algorithmic_bytes(name, opt, dim, shape):
         "k_lds_flags": 4 * L,
         "k_lds_assign": 4 * U,
         "k_lds_mapped": 12 * L,                # first position in, mapped id out
-        "k_group_count": 24 * U,               # distinct records in, per-record placement out
         "k_group_emit": 52 * U + 20 * G,       # records, placement and rows in; member lists, per-record index and
                                                # row, groups out
         # global-table fallback
@@ -101,7 +99,6 @@ def kernel_algorithmic_bytes(name, opt, dim, shape):
         "k_group_insert": 16 * U,
         # table
         "k_probe": 8 * G + 4 * G,              # one stored-key compare per distinct sign, row number out
-        "k_probe_recs": 8 * U + 8 * U + 4 * U, # the record's sign in, one stored-key compare, row number out
         "k_group_probe": 24 * U + 20 * U + 4 * L,      # placement of the records, their probes, the lookups' flags
         "k_assign_init": 4 * U,
         "k_emit_mapped": 52 * U + 20 * G + 12 * L,     # member lists; mapped ids
@@ -491,7 +488,7 @@ def main():
         "kernels_frac_of_hbm_peak": {
             k: round(kernel_algorithmic_bytes(k, opt_name, dim, mean_shape) / (ms / c * 1e-3) / HBM_PEAK, 4)
             for k, (c, ms) in per_step.items() if kernel_algorithmic_bytes(k, opt_name, dim, mean_shape) > 0},
-        "side_stream_kernels": [k for k in per_step if k.startswith(SIDE_STREAM_KERNELS)],
+        "side_stream_kernels": [k for k in per_step if args.detached_updates and k.startswith(SIDE_STREAM_KERNELS)],
         "batch_shape": mean_shape,
     }
 

@@ -7,8 +7,8 @@ benchmark's roofline figures rest on:
 The runs (MI355X box, from the repository root, with TMPDIR=/tmp):
 
     rocprofv3 --kernel-trace --stats -d prof_out/prof_trace -o t -- python3 bench.py --steps 5 --warmup 2 --no-cpu --no-others --no-traffic
-    rocprofv3 --pmc FETCH_SIZE -d prof_out/prof_fetch -o f -- python3 bench.py --steps 2 --warmup 1 --no-cpu --no-others --no-traffic
-    rocprofv3 --pmc WRITE_SIZE -d prof_out/prof_write -o w -- python3 bench.py --steps 2 --warmup 1 --no-cpu --no-others --no-traffic
+    rocprofv3 --pmc FETCH_SIZE -d prof_out/prof_fetch -o f -- python3 bench.py --steps 2 --warmup 1 --no-cpu --no-others --no-traffic --detached
+    rocprofv3 --pmc WRITE_SIZE -d prof_out/prof_write -o w -- python3 bench.py --steps 2 --warmup 1 --no-cpu --no-others --no-traffic --detached
     python3 bench.py --no-traffic > prof_out/bench_full.json
     python3 -m tensornet_amd.profile_summary --trace prof_out/prof_trace --fetch prof_out/prof_fetch \\
         --write prof_out/prof_write --bench prof_out/bench_full.json --commit <commit of the profiled tree>
@@ -160,8 +160,8 @@ def main():
            "Written at commit `%s` by (MI355X box, from the repository root, with TMPDIR=/tmp):\n" % commit,
            "```\n"
            "rocprofv3 --kernel-trace --stats -d prof_out/prof_trace -o t -- python3 bench.py --steps 5 --warmup 2 --no-cpu --no-others --no-traffic\n"
-           "rocprofv3 --pmc FETCH_SIZE -d prof_out/prof_fetch -o f -- python3 bench.py --steps 2 --warmup 1 --no-cpu --no-others --no-traffic\n"
-           "rocprofv3 --pmc WRITE_SIZE -d prof_out/prof_write -o w -- python3 bench.py --steps 2 --warmup 1 --no-cpu --no-others --no-traffic\n"
+           "rocprofv3 --pmc FETCH_SIZE -d prof_out/prof_fetch -o f -- python3 bench.py --steps 2 --warmup 1 --no-cpu --no-others --no-traffic --detached\n"
+           "rocprofv3 --pmc WRITE_SIZE -d prof_out/prof_write -o w -- python3 bench.py --steps 2 --warmup 1 --no-cpu --no-others --no-traffic --detached\n"
            "python3 bench.py --no-traffic > prof_out/bench_full.json\n"
            "python3 -m tensornet_amd.profile_summary --trace prof_out/prof_trace --fetch prof_out/prof_fetch --write prof_out/prof_write "
            "--bench prof_out/bench_full.json --commit %s\n"
@@ -198,19 +198,14 @@ def main():
             ""]
     with open(args.out, "w") as f:
         f.write("\n".join(out))
-    # kernels of the library that this workload no longer launches (other batches and options do) keep their last figures
-    kept = {}
-    if os.path.exists(args.traffic):
-        with open(args.traffic) as f:
-            old = json.load(f)
-        kept = {k: c for k, c in old.get("kept_from", {}).items() if k not in traffic}
-        for k, v in old["bytes_per_launch"].items():
-            if k not in traffic:
-                traffic[k] = v
-                kept.setdefault(k, old["commit"])
+    # the kernels of the steps with detached updates, which the counter runs hold and the trace does not
+    for n in sorted(set(fetch) | set(write)):
+        both = fetch.get(n, 0.0) * ff + write.get(n, 0.0) * wf
+        if both > 0:
+            traffic.setdefault(n.split("<")[0], int(both * 1024))
     with open(args.traffic, "w") as f:
         json.dump({"commit": commit, "fetch_factor": round(ff, 4), "write_factor": round(wf, 4),
-                   "workload": line["config"]["workload"], "bytes_per_launch": traffic, "kept_from": kept}, f, indent=1, sort_keys=True)
+                   "workload": line["config"]["workload"], "bytes_per_launch": traffic}, f, indent=1, sort_keys=True)
         f.write("\n")
     print("wrote %s and %s (%d kernels)" % (args.out, args.traffic, len(traffic)))
 

@@ -2,6 +2,7 @@
 knows (by their algorithmic bytes), and bench.py must refuse a step that launches a kernel the file lacks."""
 import json
 import os
+import re
 import sys
 
 import pytest
@@ -28,12 +29,22 @@ def test_traffic_file_names_known_kernels():
         known = bench.kernel_algorithmic_bytes(k, "AdaGrad", 16, SHAPE) > 0
         assert known or k.startswith(SIDE) or k.startswith(bench.SMALL_STEP_KERNELS), "unknown kernel %s" % k
     # the kernels of the cfg3 step all have their figure
-    step = ["k_tile_dedup", "k_lds_dedup<true>", "k_lds_flags", "k_lds_assign<false>", "k_lds_mapped",
-            "k_group_count", "k_group_emit", "k_probe_recs", "k_gather_vars<4>", "k_verify_values<true, false>",
-            "k_apply_single<KIND, 4>", "k_apply_vec<KIND, 4>", "k_apply_big_adagrad<DIM>", "k_stage_in", "k_publish"]
+    step = ["k_tile_dedup", "k_lds_dedup<true>", "k_group_probe<2>", "k_assign_init", "k_emit_mapped", "k_gather_vars<4>",
+            "k_verify_values<true, false>", "k_apply_all<KIND, 4, false, TILE>", "k_stage_in"]
     per_launch, source = bench.measured_traffic(step)
     assert source["file"] == "profiles/cfg3_traffic.json" and source["profiled_at_commit"] == t["commit"]
-    assert per_launch["k_apply_single"] > bench.kernel_algorithmic_bytes("k_apply_single", "AdaGrad", 16, SHAPE) * 0.5
+    assert per_launch["k_apply_all"] > bench.kernel_algorithmic_bytes("k_apply_all", "AdaGrad", 16, SHAPE) * 0.5
+
+
+def test_the_figures_are_of_kernels_there_are():
+    """Figures come from one run of the profiler: a kernel that is no longer launched has none."""
+    csrc = os.path.join(ROOT, "tensornet_amd", "csrc")
+    text = "".join(open(os.path.join(csrc, n)).read() for n in sorted(os.listdir(csrc)))
+    with open(bench.TRAFFIC_FILE) as f:
+        t = json.load(f)
+    assert set(t) == {"commit", "fetch_factor", "write_factor", "workload", "bytes_per_launch"}
+    for k in t["bytes_per_launch"]:
+        assert re.search(r"\b%s\(" % k, text), "no kernel %s" % k
 
 
 def test_a_kernel_without_a_figure_is_refused():
