@@ -390,6 +390,17 @@ hipEvent_t tail_event(SparseTable* t, hipStream_t st) {
     return t->tail_ev;
 }
 
+// The same as an event recorded behind the last kernel.  That is a small pull's form: a program that waits for the pulled rows waits
+// longer where the kernel itself signals.  Push and pull of 1024 x 8, 4096 x 26 and 3001 x 47 x 2 lookups on a stream of the
+// caller's, us, one step after the other, and each waited for: events recorded behind both calls 42.3, 51.6, 76.4, and 44.1, 59.0,
+// 80.8; signals of both calls' last kernels 38.4, 50.0, 73.0, and 45.0, 61.8, 82.6; the push's a signal, the pull's recorded
+// 39.2, 51.0, 74.7, and 41.5, 58.0, 78.9.  (Pull and combine of 256 x 26 x 3: 40.0 and 51.5, 37.9 and 48.4, 38.5 and 50.0.)
+int record_tail(SparseTable* t, hipStream_t st) {
+    hipEvent_t tail = tail_event(t, st);
+    if (tail) TN_HIP(hipEventRecord(tail, st));
+    return TN_OK;
+}
+
 // beside_updates: the caller (the pull op) orders its stream behind detached updates itself, as late as it can.
 int ensure_allocated(SparseTable* t, hipStream_t st, bool beside_updates = false) {
     TN_TRY(ensure_side_buffers(t));
@@ -1402,11 +1413,9 @@ int small_pull(SparseTable* t, const SmallShape& b, const int64_t* const* values
     ea.big_k = t->plan_big_k = b.N <= SMALL_NO_BIG_SLOTS ? 0xFFFFFFFFu : SMALL_BIG_GROUP;
     const size_t emit_lds = small_emit_lds(b.N, b.cap, ea.table);
     const uint32_t finish = (uint32_t)b.N * chunks;
-    hipEvent_t tail = tail_event(t, st);
     if (b.N > SMALL_SPLIT_SLOTS && emit_lds <= SMALL_SHARED_LDS) {
 #define TN_LAUNCH_REST(VEC)                                                                                              \
-    TN_LAUNCH_LDS_EVENT(tail, (k_small_pull_rest<VEC>), dim3(b.buckets() + finish), dim3(FINISH_THREADS), emit_lds, st, \
-                        ea, chunks, per, s)
+    TN_LAUNCH_LDS((k_small_pull_rest<VEC>), dim3(b.buckets() + finish), dim3(FINISH_THREADS), emit_lds, st, ea, chunks, per, s)
         if (width == 4) TN_LAUNCH_REST(4);
         else if (width == 2) TN_LAUNCH_REST(2);
         else TN_LAUNCH_REST(1);
@@ -1418,8 +1427,9 @@ int small_pull(SparseTable* t, const SmallShape& b, const int64_t* const* values
         else if (width == 2) TN_LAUNCH_FINISH(2);
         else TN_LAUNCH_FINISH(1);
 #undef TN_LAUNCH_FINISH
-        TN_LAUNCH_LDS_EVENT(tail, (k_group_emit<true>), dim3(b.buckets()), dim3(FINISH_THREADS), emit_lds, st, ea);
+        TN_LAUNCH_LDS((k_group_emit<true>), dim3(b.buckets()), dim3(FINISH_THREADS), emit_lds, st, ea);
     }
+    TN_TRY(record_tail(t, st));
     TN_HIP(hipGetLastError());
     // the call returns when the first launch has reported: what follows is complete in stream order
     t->small_shape = b;
