@@ -75,7 +75,7 @@ __device__ __forceinline__ void pool_items(PoolLds& lds, uint32_t n, uint32_t bi
     static_assert(LPG <= 4, "PoolLds::part");
     uint32_t tid = threadIdx.x;
     // (addresses worked out from here on stay inside the round: held in registers across the caller's loop they cost a
-    // workgroup of the three)
+    // workgroup of the four)
     asm volatile("" : "+v"(tid));
     const uint32_t lane = tid & 63, wave = tid >> 6;
     const uint32_t passes = (bits + POOL_DIGIT - 1) / POOL_DIGIT, width = passes ? (bits + passes - 1) / passes : 0u;

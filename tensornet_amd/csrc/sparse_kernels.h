@@ -2456,10 +2456,9 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6, 8))) void
         [&] { src.no_gradient(status); });
 }
 
-// The updates of a push of up to ONE_STREAM_LOOKUPS lookups by one launch: the workgroups of the three kernels above side
-// by side, those with the longest chains first.  They touch disjoint rows and one alone leaves the chip half idle --
-// k_apply_big and k_apply_vec wait for chains, and a launch for its last workgroups --, but a batch this small does not pay
-// for a second stream (a fork and a join of 15 us).  TILE: the row length k_apply_big_adagrad is made for, 0: the signs with
+// The updates of a push whose rows fit the lanes of a wavefront half, unless they are detached, by one launch: the workgroups of
+// the three kernels above side by side, those with the longest chains first.  They touch disjoint rows and one alone leaves the
+// chip half idle: k_apply_big and k_apply_vec wait for chains, and a launch for its last workgroups.  TILE: the row length k_apply_big_adagrad is made for, 0: the signs with
 // many records the way of k_apply_big, with the staging a wavefront of a workgroup of four can have.
 // 2.1 M lookups of 64 slots, AdaGrad rows of 16: three launches 58 us (19 + 20 + 19), this one 42; 327 k of 40, rows of 64:
 // 77 -> 51, Ftrl rows of 1: 66 -> 38; 286 k of 47, rows of 8 + 2: 32 -> 18.

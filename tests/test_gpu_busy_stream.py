@@ -14,10 +14,10 @@ HP = dict(learning_rate=0.01, initial_g2sum=0.1, epsilon=1e-8)
 BUSY = 60_000_000  # cycles: well beyond what a call polls for before it looks at the stream
 
 
-@pytest.mark.parametrize("path", ["few launches", "one stream", "several streams"])
+@pytest.mark.parametrize("path", ["few launches", "small", "large"])
 def test_pull_and_push_behind_other_work(tn, oracle, path):
     rng = np.random.default_rng(3)
-    slots, lookups, vocab = (3, 1_100_000, 3000) if path == "several streams" else (12, 1500, 3000)
+    slots, lookups, vocab = (3, 1_100_000, 3000) if path == "large" else (12, 1500, 3000)
     pair = Pair(tn, oracle, "AdaGrad", 8, HP)
     tn.core.set_sparse_table_small_batch_path(pair.h, path == "few launches")
     ids = synth.splitmix64(np.arange(1, vocab + 1, dtype=np.uint64)).view(np.int64)

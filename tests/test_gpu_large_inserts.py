@@ -28,7 +28,7 @@ D = 16
 SCALE = 0.1
 HP = dict(learning_rate=0.01, initial_g2sum=0.1, initial_scale=SCALE, epsilon=1e-8)
 VOCAB = 400000
-SLOTS, PER = 64, 53500  # 3.3-3.4 M lookups: above the size from which a call uses the table's side streams
+SLOTS, PER = 64, 53500  # 3.3-3.4 M lookups: above the size from which updates are detached
 
 
 def make_batches(pool):

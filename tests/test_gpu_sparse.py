@@ -1017,7 +1017,7 @@ def test_calls_on_another_stream_wait_for_the_last_pull(tn, oracle):
     s1, s2 = torch.cuda.Stream(), torch.cuda.Stream()
     torch.cuda.synchronize()
     for step in range(3):
-        # step 0: a batch large enough for the side streams (more than 3 M lookups), step 1: a small one, step 2:
+        # step 0: a batch of more than 3 M lookups, step 1: a small one, step 2:
         # one for the path of few launches (every slot within 4096 lookups), whose pull also returns before its
         # last kernels have run
         per_slot = ((200000, 230000), (3000, 6000), (500, 3000))[step]
