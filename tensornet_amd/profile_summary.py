@@ -198,10 +198,10 @@ def main():
             ""]
     with open(args.out, "w") as f:
         f.write("\n".join(out))
-    # the kernels of the steps with detached updates, which the counter runs hold and the trace does not
+    # the library's kernels of the steps with detached updates, which the counter runs hold and the trace does not
     for n in sorted(set(fetch) | set(write)):
         both = fetch.get(n, 0.0) * ff + write.get(n, 0.0) * wf
-        if both > 0:
+        if both > 0 and n.startswith("k_"):
             traffic.setdefault(n.split("<")[0], int(both * 1024))
     with open(args.traffic, "w") as f:
         json.dump({"commit": commit, "fetch_factor": round(ff, 4), "write_factor": round(wf, 4),
