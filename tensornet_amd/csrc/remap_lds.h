@@ -1004,7 +1004,8 @@ static __global__ __launch_bounds__(REMAP_THREADS) void k_assign_init(
 // the arrays is first put together in LDS and then copied out in order; only where_u, indexed
 // by the distinct index of the record, stays a scattered store.  where_u[u] = {place in the member
 // list (with WHERE_ONE_TILE if all lookups of the record lie in one tile), table row of the record's sign
-// (rrow, from probe_bucket)}; the groups get the rows too.  A group with big_k records or more is listed in
+// (rrow, from probe_bucket)}; the groups get the rows too.  (Their signs nobody asks for again, and place and count of a group of
+// one record only k_apply_scalar: written all the same, 78 us for 4.9 M lookups of 100 slots, so 72; 2.1 M of 64 25.4 and 24.3.)  A group with big_k records or more is listed in
 // big_list and, with {row, first member, records, group}, in big_desc.
 //
 template <bool SMALL>
@@ -1021,7 +1022,7 @@ struct EmitArgs<false> {
     const uint8_t* flag8;
     const uint32_t* wordpre;
     uint32_t ids_cap, big_k;
-    uint64_t* grp_sign;
+    bool singles;  // k_apply_scalar is to read the plan: it wants place and count of the groups of one record, too
     uint32_t *grp_off, *grp_cnt, *big_list;
     uint4* big_desc;
     Member* list;
@@ -1034,18 +1035,17 @@ __device__ __forceinline__ void emit_buckets(uint32_t of, uint32_t nb2, const ui
                                              const GroupRec* __restrict__ recs, const uint2* __restrict__ aux,
                                              const uint4* __restrict__ bbase, const uint4* __restrict__ bcounts,
                                              const uint8_t* __restrict__ flag8, const uint32_t* __restrict__ wordpre,
-                                             uint32_t ids_cap, uint32_t big_k, uint64_t* __restrict__ grp_sign,
+                                             uint32_t ids_cap, uint32_t big_k, bool singles,
                                              uint32_t* __restrict__ grp_off, uint32_t* __restrict__ grp_cnt,
                                              uint32_t* __restrict__ big_list, uint4* __restrict__ big_desc,
                                              Member* __restrict__ list, uint2* __restrict__ where_u,
                                              const uint32_t* __restrict__ rrow, uint32_t* __restrict__ grp_row,
                                              DevStatus* status) {
     // [0, n1): the groups of one record (group = member); from n1 on: in s_mem the members of the other groups,
-    // last group first, in s_sign / s_row those groups themselves, whose offsets and sizes have arrays of their
+    // last group first, in s_row those groups' rows, whose offsets and sizes have arrays of their
     // own (such a group has two records at least, so there are n / 2 of them at most).  A member entry is packed
-    // into eight bytes while it waits here {u | slot << 32 | show << 40}: 35 KB per workgroup, four to a CU.
+    // into eight bytes while it waits here {u | slot << 32 | show << 40}: 23 KB per workgroup.
     __shared__ unsigned long long s_mem[GRP_CAP];
-    __shared__ unsigned long long s_sign[GRP_CAP];
     __shared__ uint32_t s_row[GRP_CAP];
     __shared__ uint32_t s_off[GRP_CAP / 2];
     __shared__ uint16_t s_cnt[GRP_CAP / 2];  // at most GRP_SLOTS records per group
@@ -1119,7 +1119,6 @@ __device__ __forceinline__ void emit_buckets(uint32_t of, uint32_t nb2, const ui
             if (k == 1) {
                 const uint32_t g = bb.x + idx;
                 s_mem[idx] = m;
-                s_sign[idx] = r.sign;
                 s_row[idx] = rows[j];
                 where_u[us[j]] = make_uint2(g | one_tile, rows[j]);
             } else {
@@ -1130,7 +1129,6 @@ __device__ __forceinline__ void emit_buckets(uint32_t of, uint32_t nb2, const ui
                 where_u[us[j]] = make_uint2((top - t) | one_tile, rows[j]);
                 if (place == 0) {
                     s_row[n1 + idx] = rows[j];  // every record of the sign was given the same row
-                    s_sign[n1 + idx] = r.sign;
                     s_off[idx] = top - (before + k - 1);
                     s_cnt[idx] = (uint16_t)k;
                     if (is_big(k, big_k)) {
@@ -1153,15 +1151,15 @@ __device__ __forceinline__ void emit_buckets(uint32_t of, uint32_t nb2, const ui
         for (uint32_t i = threadIdx.x; i < n1; i += EMIT_THREADS) {
             const uint32_t g = bb.x + i;
             list[g] = member(s_mem[i]);
-            grp_sign[g] = s_sign[i];
-            grp_off[g] = g;  // (group = member)
-            grp_cnt[g] = 1;
             grp_row[g] = s_row[i];
+            if (singles) {  // (group = member)
+                grp_off[g] = g;
+                grp_cnt[g] = 1;
+            }
         }
         for (uint32_t i = threadIdx.x; i < nr; i += EMIT_THREADS) list[top - i] = member(s_mem[n1 + i]);
         for (uint32_t i = threadIdx.x; i < nm; i += EMIT_THREADS) {
             const uint32_t g = ids_cap - 1 - (bb.y + i);
-            grp_sign[g] = s_sign[n1 + i];
             grp_off[g] = s_off[i];
             grp_cnt[g] = s_cnt[i];
             grp_row[g] = s_row[n1 + i];
@@ -1192,7 +1190,7 @@ static __global__ __launch_bounds__(EMIT_THREADS) __attribute__((amdgpu_waves_pe
     extern __shared__ uint32_t lb[];  // lb[N + 1], sized by the launch
     if (blockIdx.x < emit_blocks)
         emit_buckets(emit_blocks, a.nb2, a.cursor2, a.recs, a.aux, a.bbase, a.bcounts, a.flag8, a.wordpre, a.ids_cap, a.big_k,
-                     a.grp_sign, a.grp_off, a.grp_cnt, a.big_list, a.big_desc, a.list, a.where_u, a.rrow, a.grp_row, a.status);
+                     a.singles, a.grp_off, a.grp_cnt, a.big_list, a.big_desc, a.list, a.where_u, a.rrow, a.grp_row, a.status);
     else
         map_lookups(lb, blockIdx.x - emit_blocks, gridDim.x - emit_blocks, m.descs, m.lbase, m.ubase, m.N, m.L, m.first_of, a.flag8,
                     a.wordpre, m.u_of_gi);

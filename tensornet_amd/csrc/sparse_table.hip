@@ -980,7 +980,7 @@ int launch_build_plan(SparseTable* t, const Plan& p, const Scratch& w, int N, ui
         ea.wordpre = w.wordpre;
         ea.ids_cap = L;
         ea.big_k = big_threshold(s);
-        ea.grp_sign = p.grp_sign;
+        ea.singles = row_share(s, true).lanes == 0;
         ea.grp_off = p.grp_off;
         ea.grp_cnt = p.grp_cnt;
         ea.big_list = p.big_list;
