@@ -832,7 +832,7 @@ struct SmallGroup {
 // ONCE: the caller says that k <= AHEAD, so nothing is fetched ahead (and registers for 32 words are free).
 template <int KIND, int LPG, bool ANY, int AHEAD, bool ONCE, typename Group>
 __device__ __forceinline__ void apply_group_ahead(const Store& s, const OptDev& o, const Group& grp, uint32_t row, uint32_t k,
-                                                  int sub, int lane0, float c1, float c2) {
+                                                  int sub, float c1, float c2) {
     typedef typename Group::Entry Entry;
     const int D = s.D;
     float* wp = s.w + (uint64_t)row * s.wstride;
@@ -889,20 +889,11 @@ __device__ __forceinline__ void apply_group_ahead(const Store& s, const OptDev& 
             // with their hand-over from lane to lane, the square roots, the divisions -- is worked out for all records of
             // the window side by side; the two chains then run over the results, in record order.  The same operations
             // on the same operands as record after record.
+            float4 sq[AHEAD];
             double mq[AHEAD];
 #pragma unroll
-            for (int q = 0; q < AHEAD; q++) mq[q] = 0.0;
-            for (int l = 0; l < LPG; l++) {
-#pragma unroll
-                for (int q = 0; q < AHEAD; q++) {
-                    double cand = mq[q];  // add_g2sum: double accumulator over the float products, element order 0..D-1
-                    cand += (double)(g0[q].x * g0[q].x);
-                    cand += (double)(g0[q].y * g0[q].y);
-                    cand += (double)(g0[q].z * g0[q].z);
-                    cand += (double)(g0[q].w * g0[q].w);
-                    mq[q] = __shfl(cand, lane0 + l);
-                }
-            }
+            for (int q = 0; q < AHEAD; q++) sq[q] = squares(g0[q]);
+            square_sums<LPG>(sq, mq);
 #pragma unroll
             for (int q = 0; q < AHEAD; q++) mq[q] = mq[q] / (double)D;
             float g2[AHEAD];
@@ -1048,7 +1039,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(small_apply
     src.click_at = p.click_at;
     src.dim = dim;
     const float c1 = 1 - o.beta1, c2 = 1 - o.beta2;
-    const int wave = (int)(threadIdx.x >> 6), lane = (int)(threadIdx.x & 63), sub = lane % LPG, lane0 = lane - sub;
+    const int wave = (int)(threadIdx.x >> 6), lane = (int)(threadIdx.x & 63), sub = lane % LPG;
     auto describe = [](uint2 g) { return make_uint4(g.x, g.y & 0xFFFFu, g.y >> 16, 0u); };
     auto group = [&](uint32_t bi) { return describe(p.group[first + b.cap - 1 - bi]); };
     auto record = [&](const uint4& m, const float*& gp, int& sh, int& ck, bool there) {
@@ -1092,7 +1083,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(small_apply
             const uint2 d = g < head.y ? p.group[first + head.x + g] : make_uint2(NO_ROW, 0);
             if (d.x <= s.cap) {  // (no row number at all: never address the table with it)
                 const SmallGroup grp{src, p.member + first + (d.y & 0xFFFFu)};
-                apply_group_ahead<KIND, LPG, ANY, 4, BIG != BIG_NONE>(s, o, grp, d.x, d.y >> 16, sub, lane0, c1, c2);
+                apply_group_ahead<KIND, LPG, ANY, 4, BIG != BIG_NONE>(s, o, grp, d.x, d.y >> 16, sub, c1, c2);
             }
         } else {
             uint2 d[AT_ONCE];
@@ -1123,7 +1114,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(small_apply
 #pragma unroll
             for (uint32_t q = 0; q < AT_ONCE; q++) {
                 if (gp[q])
-                    finish_record<KIND, LPG, ANY>(s, o, d[q].x, row[q], (int)mem[q].z, ck[q], sub, lane0, c1, c2);
+                    finish_record<KIND, LPG, ANY>(s, o, d[q].x, row[q], (int)mem[q].z, ck[q], sub, c1, c2);
                 // (a record without a gradient row, too: the caller may push the batch again on this plan)
                 if (KIND == OPT_ADAGRAD && ok[q] && sub == 0) src.click_at[mem[q].x] = 0;
             }

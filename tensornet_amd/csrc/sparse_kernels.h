@@ -1570,6 +1570,50 @@ __device__ __forceinline__ void ftrl_elem(const OptDev& o, float g, float& w, fl
     }
 }
 
+// x of lane L of every group of LPG lanes, in all lanes of the group (which are active together).
+template <int LPG, int L>
+__device__ __forceinline__ int from_group_lane(int x) {
+    static_assert(L < LPG && LPG <= 32, "a lane of the group");
+    if constexpr (LPG == 1) {
+        return x;
+    } else if constexpr (LPG == 2) {
+        return __builtin_amdgcn_update_dpp(x, x, L == 0 ? 0xA0 : 0xF5, 0xF, 0xF, false);  // quad_perm:[L,L,2+L,2+L]
+    } else if constexpr (LPG == 4) {
+        return __builtin_amdgcn_update_dpp(x, x, 0x55 * L, 0xF, 0xF, false);  // quad_perm:[L,L,L,L]
+    } else if constexpr (LPG == 8) {  // row_newbcast: the first two banks of a row from its lane L, the others from lane 8 + L
+        const int lower = __builtin_amdgcn_update_dpp(x, x, 0x150 + L, 0xF, 0x3, false);
+        return __builtin_amdgcn_update_dpp(lower, x, 0x150 + 8 + L, 0xF, 0xC, false);
+    } else if constexpr (LPG == 16) {
+        return __builtin_amdgcn_update_dpp(x, x, 0x150 + L, 0xF, 0xF, false);
+    } else {
+        return __shfl(x, (int)(__lane_id() & ~31u) + L);
+    }
+}
+template <int LPG, int L>
+__device__ __forceinline__ double from_group_lane(double x) {
+    return __hiloint2double(from_group_lane<LPG, L>(__double2hiint(x)), from_group_lane<LPG, L>(__double2loint(x)));
+}
+
+// AdaGrad's add_g2sum of the N gradients whose rows LPG lanes hold, four elements each: double sums over the float products, in
+// element order 0 .. D-1.  A chain through the lanes; the N chains run side by side, and the sum goes from lane to lane
+// through registers (data-parallel primitives), a tenth of the time it takes by way of LDS (__shfl).  k_apply_all, rows of 16: 4.9 M
+// lookups of 100 slots 142 -> 137 us, 2.1 M of 64 40.8 -> 38.5; k_small_apply, rows of 64, 40 slots of 8192 50 -> 47.  (Four records
+// of rows of 64 side by side there, too: 57, the registers of their squares are spilled.)
+template <int LPG, int N, int L = 0>
+__device__ __forceinline__ void square_sums(const float4 (&sq)[N], double (&tot)[N]) {
+#pragma unroll
+    for (int q = 0; q < N; q++) {
+        double cand = L == 0 ? 0.0 : tot[q];
+        cand += (double)sq[q].x;
+        cand += (double)sq[q].y;
+        cand += (double)sq[q].z;
+        cand += (double)sq[q].w;
+        tot[q] = from_group_lane<LPG, L>(cand);
+    }
+    if constexpr (L + 1 < LPG) square_sums<LPG, N, L + 1>(sq, tot);
+}
+__device__ __forceinline__ float4 squares(float4 g) { return make_float4(g.x * g.x, g.y * g.y, g.z * g.z, g.w * g.w); }
+
 // One record applied to its sign's row by LPG lanes: gradient, row and state once.  In two halves, for callers that have
 // several records on their way at a time.
 struct RecordRow {
@@ -1595,22 +1639,15 @@ __device__ __forceinline__ RecordRow fetch_record(const Store& s, uint32_t row, 
 }
 template <int KIND, int LPG, bool ANY>
 __device__ __forceinline__ void finish_record(const Store& s, const OptDev& o, uint32_t row, RecordRow& r, int bshow, int bclick,
-                                              int sub, int lane0, float c1, float c2) {
+                                              int sub, float c1, float c2) {
     const int D = s.D;
     float* wp = s.w + (uint64_t)row * s.wstride;
     float* sp = s.st + (uint64_t)row * s.sstride;
     if (KIND == OPT_ADAGRAD) {
-        const float p0 = r.g.x * r.g.x, p1 = r.g.y * r.g.y, p2 = r.g.z * r.g.z, p3 = r.g.w * r.g.w;
-        double tot = 0.0;  // add_g2sum: double accumulator over the float products, element order 0..D-1
-        for (int l = 0; l < LPG; l++) {
-            double cand = tot;
-            cand += (double)p0;
-            cand += (double)p1;
-            cand += (double)p2;
-            cand += (double)p3;
-            tot = __shfl(cand, lane0 + l);
-        }
-        const float g2sum = (float)((double)r.a.x + tot / (double)D);
+        const float4 sq[1] = {squares(r.g)};
+        double tot[1];
+        square_sums<LPG>(sq, tot);
+        const float g2sum = (float)((double)r.a.x + tot[0] / (double)D);
         const float den = o.eps + sqrtf(g2sum);
         r.w.x -= o.lr * r.g.x / den;
         r.w.y -= o.lr * r.g.y / den;
@@ -1645,9 +1682,9 @@ __device__ __forceinline__ void finish_record(const Store& s, const OptDev& o, u
 }
 template <int KIND, int LPG, bool ANY>
 __device__ __forceinline__ void apply_one_record(const Store& s, const OptDev& o, uint32_t row, const float* gp, int bshow,
-                                                 int bclick, int sub, int lane0, float c1, float c2) {
+                                                 int bclick, int sub, float c1, float c2) {
     RecordRow r = fetch_record<KIND, ANY>(s, row, gp, sub);
-    finish_record<KIND, LPG, ANY>(s, o, row, r, bshow, bclick, sub, lane0, c1, c2);
+    finish_record<KIND, LPG, ANY>(s, o, row, r, bshow, bclick, sub, c1, c2);
 }
 
 // Most signs occur in one slot only: one record, no ordering problem, no
@@ -1660,7 +1697,6 @@ __device__ __forceinline__ void apply_singles(const Store& s, const OptDev& o, c
                                               uint32_t at, uint32_t stride) {
     const uint32_t n_single = status->n_single;
     const int sub = threadIdx.x % LPG;
-    const int lane0 = (int)__lane_id() - sub;
     const float c1 = 1 - o.beta1, c2 = 1 - o.beta2;
     for (uint32_t g = at * (256 / LPG) + threadIdx.x / LPG; g < n_single; g += stride * (256 / LPG)) {
         const uint32_t row = grp_row[g];
@@ -1671,7 +1707,7 @@ __device__ __forceinline__ void apply_singles(const Store& s, const OptDev& o, c
             if (sub == 0) src.no_gradient(status);
             continue;
         }
-        apply_one_record<KIND, LPG, ANY>(s, o, row, gp, bshow, bclick, sub, lane0, c1, c2);
+        apply_one_record<KIND, LPG, ANY>(s, o, row, gp, bshow, bclick, sub, c1, c2);
     }
 }
 
@@ -1693,7 +1729,7 @@ __global__ __launch_bounds__(256) void k_apply_single(Store s, OptDev o, PushSrc
 template <int KIND, int LPG, bool ANY>
 __device__ __forceinline__ void apply_group_vec(const Store& s, const OptDev& o, const PushSrc& src, DevStatus* status,
                                                 uint32_t row, uint32_t k, const Member* mem, const float* const* ga,
-                                                int sub, int lane0, float c1, float c2) {
+                                                int sub, float c1, float c2) {
     const int D = s.D;
     float* wp = s.w + (uint64_t)row * s.wstride;
     float* sp = s.st + (uint64_t)row * s.sstride;
@@ -1718,18 +1754,10 @@ __device__ __forceinline__ void apply_group_vec(const Store& s, const OptDev& o,
         if (KIND == OPT_ADAGRAD) {
             show += (float)bshow;
             click += (float)bclick;
-            const float p0 = gr.x * gr.x, p1 = gr.y * gr.y, p2 = gr.z * gr.z, p3 = gr.w * gr.w;
-            // add_g2sum: double accumulator over the float products, element order 0..D-1
-            double tot = 0.0;
-            for (int l = 0; l < LPG; l++) {
-                double cand = tot;
-                cand += (double)p0;
-                cand += (double)p1;
-                cand += (double)p2;
-                cand += (double)p3;
-                tot = __shfl(cand, lane0 + l);
-            }
-            g2sum = (float)((double)g2sum + tot / (double)D);
+            const float4 sq[1] = {squares(gr)};
+            double tot[1];
+            square_sums<LPG>(sq, tot);
+            g2sum = (float)((double)g2sum + tot[0] / (double)D);
             const float den = o.eps + sqrtf(g2sum);
             w.x -= o.lr * gr.x / den;
             w.y -= o.lr * gr.y / den;
@@ -1797,7 +1825,6 @@ __device__ __forceinline__ void apply_multis(const Store& s, const OptDev& o, co
                                              uint32_t at, uint32_t stride) {
     const uint32_t n_multi = status->n_multi;
     const int sub = threadIdx.x % LPG;                       // my float4 inside the row
-    const int lane0 = (int)__lane_id() - sub;                // first lane of my group in the wavefront
     const float c1 = 1 - o.beta1, c2 = 1 - o.beta2;
     for (uint32_t gi = at * (256 / LPG) + threadIdx.x / LPG; gi < n_multi; gi += stride * (256 / LPG)) {
         const uint32_t g = ids_cap - n_multi + gi;  // groups with several records sit at the top of the id space
@@ -1806,7 +1833,7 @@ __device__ __forceinline__ void apply_multis(const Store& s, const OptDev& o, co
         const uint32_t k = grp_cnt[g];
         if (is_big(k, big_k)) continue;
         apply_group_vec<KIND, LPG, ANY>(s, o, src, status, row, k, list + grp_off[g],
-                                        gaddr ? gaddr + grp_off[g] : nullptr, sub, lane0, c1, c2);
+                                        gaddr ? gaddr + grp_off[g] : nullptr, sub, c1, c2);
     }
 }
 

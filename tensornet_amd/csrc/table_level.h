@@ -243,7 +243,7 @@ __global__ __launch_bounds__(256) void k_table_apply(TableShape b, Store s, OptD
         m += total;
     }
     if (tid == 0) spre[b.tiles] = m;
-    const int sub = tid % LPG, lane0 = (int)__lane_id() - sub;
+    const int sub = tid % LPG;
     const float c1 = 1 - o.beta1, c2 = 1 - o.beta2;
     TableGroup grp;
     grp.idx = ridx;
@@ -361,14 +361,14 @@ __global__ __launch_bounds__(256) void k_table_apply(TableShape b, Store s, OptD
                 if (g < n_multi) {
                     const uint32_t e = multi[g];
                     grp.sorted = sorted + toff[e];
-                    apply_group_ahead<KIND, LPG, ANY, 4, false>(s, o, grp, trow[e], tcnt[e], sub, lane0, c1, c2);
+                    apply_group_ahead<KIND, LPG, ANY, 4, false>(s, o, grp, trow[e], tcnt[e], sub, c1, c2);
                 }
             } else {
                 const uint32_t g = (r - rounds_multi) * (64 / LPG) + lane / LPG;
                 if (g < n_single) {
                     const uint32_t i = single[g], e = ridx[i];
                     apply_one_record<KIND, LPG, ANY>(s, o, rrow[i], grads + (uint64_t)e * dim, infos[e].batch_show,
-                                                     infos[e].batch_click, sub, lane0, c1, c2);
+                                                     infos[e].batch_click, sub, c1, c2);
                 }
             }
         }
