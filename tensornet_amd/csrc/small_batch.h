@@ -36,6 +36,14 @@ constexpr int SMALL_WORKGROUPS = SMALL_SLOTS > SMALL_SEGMENTS ? SMALL_SLOTS : SM
 constexpr int SMALL_PART_LOOKUPS = 128;      // lookups of a slot per workgroup aimed at
 constexpr int SMALL_BUCKET_RECORDS = 64;     // records per bucket aimed at (if every lookup were distinct)
 constexpr int SMALL_BUCKETS_MAX = 2048;
+// Larger batches: as many buckets as the chip holds workgroups of k_small_apply at once, four on a CU, then one for so many
+// lookups.  (Two thousand of 64 lookups each are two rounds of workgroups and twice the heads, scans and slots to go through.)
+// Push and pull, sum of the kernels, us, up to 2048 buckets of 64 lookups and so: 26 slots of 4096, Adam rows of 16 43.0 and 40.2
+// (768 of them 41.7); AdaGrad rows of 16 80 of 2000 54.0 and 50.2, 40 of 4000 50.8 and 48.1, 12 of 8000 46.6 and 44.5; rows of 64 80
+// of 2000 74.5 and 71.4; 30 of 8000, Adam rows of 16 55.9 and 53.2 (one for 256 52.0); 47 of 6400, rows of 8 + 2 65.5 and 63.2 (65.8);
+// 40 of 8192, rows of 64, one for 160 183.2, 192 189.
+constexpr size_t SMALL_BUCKETS_FEW = 1024;
+constexpr size_t small_bucket_lookups(int dim) { return dim > 32 ? 160 : 192; }
 constexpr int SMALL_THREADS = 512;           // k_small_slots; twice as many for slots of more than SMALL_SLOT_SHORT lookups
 constexpr int SMALL_ITEMS = SMALL_SLOT_SHORT / SMALL_THREADS;
 constexpr int SMALL_WORDS = SMALL_SLOT_MAX / 64;  // 64-lookup words of a slot

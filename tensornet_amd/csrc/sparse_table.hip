@@ -1288,11 +1288,16 @@ bool small_batch_shape(SparseTable* t, int N, const int64_t* lens, SmallShape& b
     b.parts = (uint32_t)std::min<size_t>(SMALL_PARTS_MAX, (max_len + SMALL_PART_LOOKUPS - 1) / SMALL_PART_LOOKUPS);
     while (b.parts > 1 && (size_t)N * b.parts > (size_t)SMALL_SEGMENTS) b.parts--;
     // (every bucket's workgroup looks at all slots: fewer buckets where there are many)
-    const size_t want = std::min<size_t>({(L + SMALL_BUCKET_RECORDS - 1) / SMALL_BUCKET_RECORDS, (size_t)SMALL_BUCKETS_MAX,
+    const size_t most = std::min<size_t>({(L + SMALL_BUCKET_RECORDS - 1) / SMALL_BUCKET_RECORDS, (size_t)SMALL_BUCKETS_MAX,
                                           std::max<size_t>(64, (size_t)(1 << 18) / N)});
-    b.nbp = (uint32_t)std::max<size_t>(1, (want + b.parts - 1) / b.parts);
-    // room for twice the records expected of a batch of distinct signs and for four signs that are in every slot
-    b.cap = (uint32_t)align_up(2 * (L / b.buckets()) + 64 + 4 * (size_t)N, 64);
+    for (size_t want = std::min(most, std::max<size_t>(SMALL_BUCKETS_FEW, L / small_bucket_lookups(t->dim)));;
+         want = std::min(most, want + want / 4)) {
+        b.nbp = (uint32_t)std::max<size_t>(1, (want + b.parts - 1) / b.parts);
+        // room for twice the records expected of a batch of distinct signs and for four signs that are in every slot
+        b.cap = (uint32_t)align_up(2 * (L / b.buckets()) + 64 + 4 * (size_t)N, 64);
+        // (no fewer than let the pull's second half be one launch)
+        if (want == most || small_emit_lds(N, b.cap, small_emit_table(b.cap)) <= SMALL_SHARED_LDS) break;
+    }
     if (!t->small_lds) {
         t->small_lds = 144 * 1024;
         for (const void* k : {(const void*)k_small_slots<ArgDescs>, (const void*)k_small_slots<HostDescs>,
