@@ -49,15 +49,21 @@ void launch_table_apply(const TableApplyCall& c) {
     const bool lds_big = s.D > 64 || (s.D & (s.D - 1)) != 0;
     const size_t wave_lds = small_apply_wave_lds(s.D), lists = table_apply_lists_lds(c.b.tiles);
     const size_t lds = lists + (lds_big ? TABLE_WAVES * wave_lds : 0);
-#define TN_LAUNCH_TABLE_BIG(LPG, ANY, BIG)                                                                            \
+#define TN_LAUNCH_TABLE_BY(LPG, ANY, BIG, MOST)                                                                       \
     do {                                                                                                              \
         if (lds_big && !c.lds_told[ANY]) {                                                                            \
             c.lds_told[ANY] = true;                                                                                   \
-            (void)big_lds_bytes_for(reinterpret_cast<const void*>(k_table_apply<KIND, LPG, ANY, BIG>));               \
+            (void)big_lds_bytes_for(reinterpret_cast<const void*>(k_table_apply<KIND, LPG, ANY, BIG, MOST>));         \
         }                                                                                                             \
-        TN_LAUNCH_LDS((k_table_apply<KIND, LPG, ANY, BIG>), dim3(c.b.nb), dim3(256), lds, c.st, c.b, s, c.o, c.infos, \
-                      c.grads, c.dim, c.recs, c.boff, c.ds, c.host_err, big_gbuf_floats(s.D), (uint32_t)wave_lds,     \
-                      (uint32_t)align_up(big_lds_bytes(s.D), 8), (uint32_t)lists);                                    \
+        TN_LAUNCH_LDS((k_table_apply<KIND, LPG, ANY, BIG, MOST>), dim3(c.b.nb), dim3(256), lds, c.st, c.b, s, c.o,    \
+                      c.infos, c.grads, c.dim, c.recs, c.boff, c.ds, c.host_err, big_gbuf_floats(s.D),                \
+                      (uint32_t)wave_lds, (uint32_t)align_up(big_lds_bytes(s.D), 8), (uint32_t)lists);                \
+    } while (0)
+#define TN_LAUNCH_TABLE_BIG(LPG, ANY, BIG)                                              \
+    do {                                                                                \
+        constexpr int FEW = table_apply_most(KIND, BIG, false), MANY = table_apply_most(KIND, BIG, true); \
+        if (MANY != FEW && c.b.nb > TABLE_MANY) TN_LAUNCH_TABLE_BY(LPG, ANY, BIG, MANY);  \
+        else TN_LAUNCH_TABLE_BY(LPG, ANY, BIG, FEW);                                      \
     } while (0)
 #define TN_LAUNCH_TABLE(LPG)                                                      \
     do {                                                                          \
@@ -78,6 +84,7 @@ void launch_table_apply(const TableApplyCall& c) {
     }
 #undef TN_LAUNCH_TABLE
 #undef TN_LAUNCH_TABLE_BIG
+#undef TN_LAUNCH_TABLE_BY
 }
 template void launch_table_apply<TN_KIND>(const TableApplyCall& c);
 

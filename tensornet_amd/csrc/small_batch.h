@@ -1004,15 +1004,12 @@ enum { BIG_NONE = 0, BIG_GROUPS = -1 };
 // Wavefronts a SIMD: AdaGrad rows of 64 with signs of many records fit four (128 registers, none spilled; by itself the compiler
 // takes 146): 40 slots of 8192 lookups 46.0 -> 40.0 us, 26 of 1024 14.6 -> 14.1.  Others lose by it: without such signs 12 slots of
 // 4000 19.5 -> 21.1, Adam rows of 64 (20 spilled) 50.4 -> 60.8, rows of 32, 26 of 1024, AdaGrad 9.9 -> 10.5, Adam 9.4 -> 10.7.
-// Rounds a chunk of apply_big_wave: sixteen where their LDS (half a chunk's gradients and what a row's second moment or factors
-// take beside them) lets the chip hold the buckets' workgroups, else four.  Four workgroups to a CU instead of seven or eight,
-// us with sixteen and with four: 26 slots of 4096, Adam rows of 16 17.1 and 14.8, of 32 19.7 and 16.9; 80 of 2000 32.5 (4000
-// lookups) and 26.2, 29.9 and 25.5; 300 of 300 47.9 and 46.4, 57.8 and 58.1; Ftrl rows of 32 21.0 and 20.2, 35.4 and 33.5, 84.6 and
-// 85.1.  Others lose where signs have hundreds of records (300 slots of 300): AdaGrad rows of 16 34.1 and 40.6, of 32 44.4 and
-// 62.6, Adam rows of 8 44.2 and 45.6, of 64 73.0 and 90.3.
-constexpr int small_apply_most(int kind, int big) {
-    return (kind == OPT_ADAM && (big == 16 || big == 32)) || (kind == OPT_FTRL && big == 32) ? 4 : 16;
-}
+// Rounds a chunk of apply_big_wave: sixteen, but for Adam rows of 16 and 32, whose chunk (gradients and second moments of 64 or 32
+// records, 9 KB) would let a CU hold four workgroups, four.  us with sixteen and with four: 26 slots of 4096 lookups 15.6 and 11.9, rows
+// of 32 17.2 and 14.6; of 1200 10.0 and 8.9, 10.7 and 10.4; 80 slots of 2000 32.5 (4000 lookups) and 26.2, 29.9 and 25.5, of 400 15.8
+// and 14.5, 18.0 and 17.0; 300 of 300 47.9 and 46.4, 57.8 and 58.1.  Others lose where signs have many records: 300 slots of 300, AdaGrad
+// rows of 16 34.1 and 40.6, of 32 44.4 and 62.6, Adam rows of 8 44.2 and 45.6, of 64 73.0 and 90.3; 80 of 400, Ftrl rows of 32 24.0 and 24.7.
+constexpr int small_apply_most(int kind, int big) { return kind == OPT_ADAM && (big == 16 || big == 32) ? 4 : 16; }
 constexpr int small_apply_waves(int kind, int lpg, int big) { return kind == OPT_ADAGRAD && lpg == 16 && big > 0 ? 4 : 1; }
 template <int KIND, int LPG, bool ANY, int BIG>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(small_apply_waves(KIND, LPG, BIG), 8))) void k_small_apply(

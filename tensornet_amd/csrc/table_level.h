@@ -187,6 +187,16 @@ struct TableGroup {
     __device__ __forceinline__ void taken(uint32_t, int, int) const {}
 };
 
+// Rounds a chunk of apply_big_wave: as in small_apply_most, and four also for Adam rows of 8 and Ftrl rows of 32 where there are more
+// workgroups than the three that a CU holds of them with sixteen.  us with sixteen and with four: 300 000 records of 200 times 1500
+// signs, Adam rows of 8 98 and 83, of 16 130 and 87, of 32 141 and 94, Ftrl rows of 32 149 and 127; 128 000 of 40 times 3200 30.9 and
+// 27.1, 36.8 and 27.4, 40.4 and 30.0, 41.0 and 37.5; 64 000 23.0 and 24.5, 24.0 and 23.8, 27.0 and 25.1, 33.2 and 33.1; 5600 24.8 and
+// 25.4, 24.6 and 24.2, 26.5 and 25.6, 33.9 and 35.3.  AdaGrad rows lose: of 8 (100 000 records) 45 and 54, of 64 (300 000) 166 and 234.
+constexpr uint32_t TABLE_MANY = 768;
+constexpr int table_apply_most(int kind, int big, bool many) {
+    return many && ((kind == OPT_ADAM && big == 8) || (kind == OPT_FTRL && big == 32)) ? 4 : small_apply_most(kind, big);
+}
+
 inline size_t table_apply_lists_lds(uint32_t tiles) {
     // per tile: records before it, where they are; table: row, records, first place; per record: row, number, entry |
     // arrival, places in order of arrival and of records, signs with one record, with several
@@ -201,7 +211,7 @@ inline size_t table_apply_lists_lds(uint32_t tiles) {
 // workgroups fit on a CU (a chunk of 1536 records left room for one: 59 us for 34 at 60 000 records).  Rows of a power of two up to
 // 64 elements have the long signs taken by apply_big_wave (BIG > 0), the others by apply_big_groups (60 000 records of 40 times
 // 1500 signs, AdaGrad rows of 16: 28 us by the latter, 19.5 by the former).
-template <int KIND, int LPG, bool ANY, int BIG>
+template <int KIND, int LPG, bool ANY, int BIG, int MOST>
 __global__ __launch_bounds__(256) void k_table_apply(TableShape b, Store s, OptDev o, const tn_sign_info* __restrict__ infos,
                                                      const float* __restrict__ grads, int dim, const uint2* __restrict__ recs,
                                                      const uint16_t* __restrict__ boff, DevStatus* status, uint32_t* host_err,
@@ -312,7 +322,7 @@ __global__ __launch_bounds__(256) void k_table_apply(TableShape b, Store s, OptD
         // (10 us for 40 records) go on meanwhile.
         const int wave = (int)(tid >> 6), lane = (int)(tid & 63);
         if constexpr (BIG > 0) {
-            __shared__ BigWave<KIND, BIG> tiles[TABLE_WAVES];
+            __shared__ BigWave<KIND, BIG, MOST> tiles[TABLE_WAVES];
             auto group = [&](uint32_t bi) {
                 const uint32_t e = big[bi];
                 return make_uint4(trow[e], toff[e], tcnt[e], 0u);
