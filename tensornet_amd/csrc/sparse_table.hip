@@ -1939,7 +1939,7 @@ int tn_sparse_table_push(uint32_t handle, const tn_sign_info* infos, const float
         TN_TRY(t->ws.ensure(align_up(room.off, 256) + 256));
         Carver c{(char*)t->ws.p};
         carve(c, recs, boff);
-        const size_t part_lds = (size_t)b.nb * TABLE_WAVES * sizeof(uint32_t);
+        const size_t part_lds = ((size_t)part_word(b.nb * TABLE_WAVES) + 1) * sizeof(uint32_t);
         if (b.tile == TABLE_THREADS)
             TN_LAUNCH_LDS((k_table_part<1>), dim3(b.tiles), dim3(TABLE_THREADS), part_lds, st, b, s, infos, recs, boff, ds);
         else if (b.tile == 4 * TABLE_THREADS)

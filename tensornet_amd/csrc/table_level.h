@@ -119,11 +119,15 @@ struct TableShape {
 // A tile's records in order of their buckets, and in record order inside a bucket: the place of a record is the number
 // of records of earlier buckets, of earlier wavefronts and of earlier lanes, which ballots over the bits of the bucket
 // number tell -- no sort, no atomics whose order of arrival would show.  Records of unknown signs are dropped.
+// The counters of a bucket's wavefronts stand in LDS behind each other with a free word after every 32 (part_word): the scan gives a
+// thread consecutive ones, 32 of them where there are 2048 buckets, which would all be in one bank: k_table_part, 300 000 records
+// 33 us and 17, 500 000 35 and 20, 1.3 M 59 and 46, 60 000 (469 buckets) 8.4 and 7.5.
+__host__ __device__ constexpr uint32_t part_word(uint32_t k) { return k + (k >> 5); }
 template <int ITEMS>
 __global__ __launch_bounds__(TABLE_THREADS) void k_table_part(TableShape b, Store s, const tn_sign_info* __restrict__ infos,
                                                               uint2* __restrict__ recs, uint16_t* __restrict__ boff,
                                                               DevStatus* status) {
-    extern __shared__ uint32_t cnt[];  // [nb][TABLE_WAVES]
+    extern __shared__ uint32_t cnt[];  // [nb][TABLE_WAVES], by part_word
     __shared__ uint32_t wsum[TABLE_WAVES];
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const uint32_t first = blockIdx.x * b.tile;
@@ -140,7 +144,7 @@ __global__ __launch_bounds__(TABLE_THREADS) void k_table_part(TableShape b, Stor
         }
         bk[j] = row[j] == NO_ROW ? 0u : (uint32_t)(((uint64_t)row[j] * b.scale) >> 32);
     }
-    for (uint32_t i = tid; i < b.nb * TABLE_WAVES; i += TABLE_THREADS) cnt[i] = 0;
+    for (uint32_t i = tid; i < part_word(b.nb * TABLE_WAVES); i += TABLE_THREADS) cnt[i] = 0;
     if (unknown) atomicOr(&status->err, DEV_ERR_UNKNOWN_KEY);
     __syncthreads();
 #pragma unroll
@@ -152,7 +156,7 @@ __global__ __launch_bounds__(TABLE_THREADS) void k_table_part(TableShape b, Stor
             same &= ((bk[j] >> q) & 1u) ? m : ~m;
         }
         at[j] = 0;
-        const uint32_t k = bk[j] * TABLE_WAVES + wave;
+        const uint32_t k = part_word(bk[j] * TABLE_WAVES + wave);
         if (valid) at[j] = cnt[k] + (uint32_t)__popcll(same & ((1ull << lane) - 1ull));
         wave_sync();
         if (valid && (uint32_t)__ffsll((long long)same) - 1 == lane) cnt[k] += (uint32_t)__popcll(same);
@@ -163,7 +167,7 @@ __global__ __launch_bounds__(TABLE_THREADS) void k_table_part(TableShape b, Stor
     uint32_t sum = 0;
     for (uint32_t q = 0; q < each; q++) {
         const uint32_t k = tid * each + q;
-        sum += k < total ? cnt[k] : 0u;
+        sum += k < total ? cnt[part_word(k)] : 0u;
     }
     uint32_t all;
     uint32_t x = block_excl_scan<uint32_t, TABLE_WAVES>(sum, wsum, &all);
@@ -171,8 +175,8 @@ __global__ __launch_bounds__(TABLE_THREADS) void k_table_part(TableShape b, Stor
     for (uint32_t q = 0; q < each; q++) {
         const uint32_t k = tid * each + q;
         if (k >= total) break;
-        const uint32_t c = cnt[k];
-        cnt[k] = x;
+        const uint32_t c = cnt[part_word(k)];
+        cnt[part_word(k)] = x;
         if (k % TABLE_WAVES == 0) off[k / TABLE_WAVES] = (uint16_t)x;
         x += c;
     }
@@ -181,7 +185,7 @@ __global__ __launch_bounds__(TABLE_THREADS) void k_table_part(TableShape b, Stor
 #pragma unroll
     for (int j = 0; j < ITEMS; j++)
         if (row[j] != NO_ROW)
-            recs[first + cnt[bk[j] * TABLE_WAVES + wave] + at[j]] =
+            recs[first + cnt[part_word(bk[j] * TABLE_WAVES + wave)] + at[j]] =
                 make_uint2(row[j], first + wave * (64 * ITEMS) + j * 64 + lane);
 }
 
