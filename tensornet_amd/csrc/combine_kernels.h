@@ -9,7 +9,7 @@
 //   backward  g[u, :]   = sum over the lookups i of distinct sign u of dout[b(i), :] * (1 / d(n_b(i)))
 //
 // Both are deterministic.  The forward sums run in occurrence order.  So do the backward sums, but cut up: a workgroup's
-// lookups, in the order of their signs, every POOL_PIECE (16) places; what a sign has in several pieces is added in order,
+// lookups, in the order of their signs, every POOL_PIECE (16) places (8, 4 of a few lookups); what a sign has in several pieces is added in order,
 // what it has in several rounds of a workgroup round by round, what a frequent one has in several workgroups by halves
 // (k_reduce_pooled, on the path of few launches k_small_pool; add_shares).
 #ifndef TN_COMBINE_KERNELS_H_

@@ -12,13 +12,13 @@ constexpr int POOL_THREADS = 512;
 constexpr uint32_t POOL_ITEMS_MAX = 2048;
 constexpr uint32_t POOL_ITEMS = POOL_ITEMS_MAX / POOL_THREADS;
 constexpr uint32_t POOL_WAVES = POOL_THREADS / 64;
-constexpr uint32_t POOL_RUN = POOL_ITEMS_MAX / POOL_WAVES;  // consecutive lookups a wavefront sorts
+constexpr uint32_t POOL_RUN = POOL_ITEMS_MAX / POOL_WAVES;  // consecutive places of a wavefront, of all of them
 constexpr uint32_t POOL_WORDS = POOL_ITEMS_MAX / 64;
-constexpr uint32_t POOL_PIECE = 16;
+constexpr uint32_t POOL_PIECE = 16;  // places of a piece; a half, a quarter where there are half, a quarter as many items
 constexpr uint32_t POOL_PIECES = POOL_ITEMS_MAX / POOL_PIECE;
 constexpr uint32_t POOL_AHEAD = 4;  // rows of a group of lanes in flight (eight: the registers of a workgroup of four do not hold them)
 constexpr uint32_t POOL_DIGIT = 7;  // (10, one pass for most slots, whose 8192 counters take longer: 44 -> 47 us, 175 -> 184)
-static_assert(POOL_AHEAD == 4 && POOL_PIECE % POOL_AHEAD == 0, "items are read four at a time");
+static_assert(POOL_AHEAD == 4 && POOL_PIECE / 4 % POOL_AHEAD == 0, "items are read four at a time");
 enum { POOL_SUM = 0, POOL_MEAN = 1, POOL_SQRTN = 2 };  // (the combiners of the C ABI)
 static_assert(POOL_RUN == 64 * POOL_ITEMS && 64 % POOL_PIECE == 0, "whole wavefronts, pieces inside a word");
 
@@ -64,7 +64,7 @@ __device__ __forceinline__ float pool_scale(float count, int combiner) {
 }
 
 // lds.key, example, scale [0, n) are filled, keys of `bits` bits, n > 0.  A stable radix sort (passes of up to 7 bits,
-// a wavefront's lanes told apart by ballots); then every group of LPG lanes takes POOL_PIECE consecutive places of the order,
+// a wavefront's lanes told apart by ballots); then every group of LPG lanes takes a piece of consecutive places of the order,
 // whatever signs they hold, POOL_AHEAD rows in flight, sixteen elements of them at a time (LPG 4).  (A group per sign has one
 // row in flight where most signs have one lookup, and waits for the longest of its wavefront: twice as long.)  A sign
 // with lookups in several pieces: their shares are added in order.  row(key, first, add): where its sum goes, and whether it
@@ -78,6 +78,10 @@ __device__ __forceinline__ void pool_items(PoolLds& lds, uint32_t n, uint32_t bi
     // workgroup of the four)
     asm volatile("" : "+v"(tid));
     const uint32_t lane = tid & 63, wave = tid >> 6;
+    // Turns of 64 items that the wavefronts take, and the consecutive items of one: as few as n asks for, so that all wavefronts have
+    // their share of them.  (Always four of each: 349 lookups in one slot, k_small_pool 17.4 us, 20 slots of 500 16.1; so 11.8 and
+    // 12.0, with the shorter pieces below.  k_reduce_pooled, 4.9 M lookups in parts of 1600 on average, 151 and 139.)
+    const uint32_t turns = (n + POOL_THREADS - 1) / POOL_THREADS, run = turns * 64;
     const uint32_t passes = (bits + POOL_DIGIT - 1) / POOL_DIGIT, width = passes ? (bits + passes - 1) / passes : 0u;
     __syncthreads();
     for (uint32_t pass = 0; pass < passes; pass++) {
@@ -88,19 +92,20 @@ __device__ __forceinline__ void pool_items(PoolLds& lds, uint32_t n, uint32_t bi
         uint32_t item[POOL_ITEMS], dg[POOL_ITEMS], at[POOL_ITEMS];
 #pragma unroll
         for (uint32_t j = 0; j < POOL_ITEMS; j++) {
-            const uint32_t i = wave * POOL_RUN + j * 64 + lane;
-            item[j] = i < n ? (pass == 0 ? i : (uint32_t)from[i]) : 0u;
+            const uint32_t i = wave * run + j * 64 + lane;
+            item[j] = j < turns && i < n ? (pass == 0 ? i : (uint32_t)from[i]) : 0u;
         }
 #pragma unroll
         for (uint32_t j = 0; j < POOL_ITEMS; j++) {
-            const bool valid = wave * POOL_RUN + j * 64 + lane < n;
+            dg[j] = at[j] = 0;
+            if (j >= turns) continue;
+            const bool valid = wave * run + j * 64 + lane < n;
             dg[j] = (lds.key[item[j]] >> (pass * width)) & ((1u << width) - 1u);
             unsigned long long same = __ballot(valid);
             for (uint32_t q = 0; q < width; q++) {
                 const unsigned long long m = __ballot((dg[j] >> q) & 1u);
                 same &= ((dg[j] >> q) & 1u) ? m : ~m;
             }
-            at[j] = 0;
             const uint32_t k = dg[j] * POOL_WAVES + wave;
             if (valid) at[j] = lds.digit[k] + (uint32_t)__popcll(same & ((1ull << lane) - 1ull));  // (before this round)
             wave_sync();
@@ -123,7 +128,7 @@ __device__ __forceinline__ void pool_items(PoolLds& lds, uint32_t n, uint32_t bi
             __syncthreads();
 #pragma unroll
             for (uint32_t j = 0; j < POOL_ITEMS; j++)
-                if (wave * POOL_RUN + j * 64 + lane < n) to[lds.digit[dg[j] * POOL_WAVES + wave] + at[j]] = (uint16_t)item[j];
+                if (j < turns && wave * run + j * 64 + lane < n) to[lds.digit[dg[j] * POOL_WAVES + wave] + at[j]] = (uint16_t)item[j];
         } else {  // the last one moves the items themselves
             uint32_t key[POOL_ITEMS], example[POOL_ITEMS];
             float scale[POOL_ITEMS];
@@ -136,7 +141,7 @@ __device__ __forceinline__ void pool_items(PoolLds& lds, uint32_t n, uint32_t bi
             __syncthreads();
 #pragma unroll
             for (uint32_t j = 0; j < POOL_ITEMS; j++) {
-                if (wave * POOL_RUN + j * 64 + lane >= n) continue;
+                if (j >= turns || wave * run + j * 64 + lane >= n) continue;
                 const uint32_t place = lds.digit[dg[j] * POOL_WAVES + wave] + at[j];
                 lds.key[place] = key[j];
                 lds.example[place] = example[j];
@@ -154,7 +159,9 @@ __device__ __forceinline__ void pool_items(PoolLds& lds, uint32_t n, uint32_t bi
         if (lane == 0) lds.heads[i >> 6] = m;
     }
     __syncthreads();
-    const uint32_t pieces = (n + POOL_PIECE - 1) / POOL_PIECE;
+    // (a piece is a chain of round trips: shorter ones where the groups of lanes are enough for them)
+    const uint32_t piece = n > POOL_ITEMS_MAX / 2 ? POOL_PIECE : n > POOL_ITEMS_MAX / 4 ? POOL_PIECE / 2 : POOL_PIECE / 4;
+    const uint32_t pieces = (n + piece - 1) / piece;
     asm volatile("" : "+v"(tid));
     const int sub = tid % LPG;
     auto put = [&](uint32_t key, bool first, int c0, float4 v) {
@@ -168,17 +175,17 @@ __device__ __forceinline__ void pool_items(PoolLds& lds, uint32_t n, uint32_t bi
     };
     // a piece per group of lanes
     static_assert(POOL_THREADS / 4 >= POOL_PIECES, "there are as many");
-    const uint32_t q = tid / LPG, lo = q * POOL_PIECE, hi = lo + POOL_PIECE;
+    const uint32_t q = tid / LPG, lo = q * piece, hi = lo + piece;
     for (int c0 = 0; c0 < D; c0 += 4 * LPG) {
         bool began = false, goes_on = false;  // the running sum's sign: began in the piece, goes on behind it
         float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
         if (q < pieces) {
             // which places start a sign, and the one behind the piece (those behind the last lookup do)
-            uint32_t hb = (uint32_t)(lds.heads[lo >> 6] >> (lo & 63)) & ((1u << POOL_PIECE) - 1u);
-            if (hi >= n || ((lds.heads[hi >> 6] >> (hi & 63)) & 1ull)) hb |= 1u << POOL_PIECE;
+            uint32_t hb = (uint32_t)(lds.heads[lo >> 6] >> (lo & 63)) & ((1u << piece) - 1u);
+            if (hi >= n || ((lds.heads[hi >> 6] >> (hi & 63)) & 1ull)) hb |= 1u << piece;
             bool first = false;  // (the running sum has its sign's first lookup)
 #pragma unroll 1
-            for (uint32_t j0 = 0; j0 < POOL_PIECE && lo + j0 < n; j0 += POOL_AHEAD, hb >>= POOL_AHEAD) {
+            for (uint32_t j0 = 0; j0 < piece && lo + j0 < n; j0 += POOL_AHEAD, hb >>= POOL_AHEAD) {
                 float4 g[POOL_AHEAD];
                 const uint4 e4 = *reinterpret_cast<const uint4*>(lds.example + lo + j0);
                 const float4 s4 = *reinterpret_cast<const float4*>(lds.scale + lo + j0);
@@ -216,7 +223,7 @@ __device__ __forceinline__ void pool_items(PoolLds& lds, uint32_t n, uint32_t bi
         __syncthreads();
         if (goes_on && began) {  // with what the pieces behind have of it, in order
             const uint32_t from = bit_at_or_below(lds.heads, hi - 1);
-            const uint32_t end = bit_above(lds.heads, hi, POOL_WORDS, n), last = (end - 1) / POOL_PIECE;
+            const uint32_t end = bit_above(lds.heads, hi, POOL_WORDS, n), last = (end - 1) / piece;
             for (uint32_t r = q + 1; r <= last; r += 4) {
                 float4 g[4];
 #pragma unroll
