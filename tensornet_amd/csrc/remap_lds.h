@@ -883,8 +883,10 @@ __device__ __forceinline__ void probe_bucket(uint32_t c, uint32_t* s_count, cons
 // second-level bucket, LDS), the signs' rows (a workgroup per bucket, random reads: every other workgroup, so that a CU has some
 // of both), the first-occurrence flags (two tiles a workgroup) and what the slots' buckets were handed (a wavefront per slot).
 // Three launches on a stream take the sum of their times; three streams beside each other left most of it in the hand-overs.
-// 2.1 M lookups of 64 slots: 28 us as three launches, 21.5; 4.9 M of 100: 86 alone, about 90 with the hand-overs of three
-// streams, 68.  It wants six wavefronts a SIMD (three workgroups to a CU; two, 83 registers: 82 us).
+// An item per workgroup, however many there are: where one went on to the next, what all four passes keep for theirs stood in scalar
+// registers together, 73 of them spilled, and twice the vector registers.
+// 2.1 M lookups of 64 slots: 28 us as three launches, 20.1 (22.9 with the loop); 4.9 M of 100: 86 alone, about 90 with the hand-overs
+// of three streams, 62 (70); 860 k of 211 22.9 (25.2).  It wants six wavefronts a SIMD (three workgroups to a CU; two: 82 us).
 struct GroupProbeArgs {
     uint32_t nb2, ntiles, L;
     const uint32_t* cursor2;
@@ -908,20 +910,17 @@ __global__ __launch_bounds__(GRP_THREADS) __attribute__((amdgpu_waves_per_eu(WOR
     } lds;
     constexpr uint32_t TILES = GRP_THREADS / REMAP_THREADS, SLOTS = GRP_THREADS / 64;
     const uint32_t flags0 = 2 * a.nb2, slots0 = flags0 + (a.ntiles + TILES - 1) / TILES;
-    const uint32_t items = slots0 + ((uint32_t)a.N + SLOTS - 1) / SLOTS;
-    for (uint32_t item = blockIdx.x; item < items; item += gridDim.x) {
-        if (item < flags0) {
-            if (item & 1u)
-                group_count_bucket(item / 2, lds.group, a.cursor2, a.recs, a.big_k, a.aux, a.bcounts);
-            else
-                probe_bucket(item / 2, lds.red, a.cursor2, a.recs, a.rrow, a.newrec, a.newcnt, s, status);
-        } else if (item < slots0) {
-            flag_tiles((item - flags0) * TILES, a.ntiles, a.L, a.first_of, a.flag8, a.tilesum, lds.red);
-        } else {
-            const uint32_t sl = (item - slots0) * SLOTS + threadIdx.x / 64;
-            if (sl < (uint32_t)a.N) slot_tile_share(a.descs[sl], a.bcursor, status);
-        }
-        __syncthreads();
+    const uint32_t item = blockIdx.x;
+    if (item < flags0) {
+        if (item & 1u)
+            group_count_bucket(item / 2, lds.group, a.cursor2, a.recs, a.big_k, a.aux, a.bcounts);
+        else
+            probe_bucket(item / 2, lds.red, a.cursor2, a.recs, a.rrow, a.newrec, a.newcnt, s, status);
+    } else if (item < slots0) {
+        flag_tiles((item - flags0) * TILES, a.ntiles, a.L, a.first_of, a.flag8, a.tilesum, lds.red);
+    } else {
+        const uint32_t sl = (item - slots0) * SLOTS + threadIdx.x / 64;
+        if (sl < (uint32_t)a.N) slot_tile_share(a.descs[sl], a.bcursor, status);
     }
 }
 

@@ -923,7 +923,7 @@ int launch_build_plan(SparseTable* t, const Plan& p, const Scratch& w, int N, ui
             ga.descs = p.descs;
             ga.N = N;
             ga.bcursor = w.bcursor;
-            const int gblocks = launch_grid(2 * (int64_t)w.nb2 + (w.ntiles + 1) / 2 + (N + 7) / 8, 1, GRID_CAP * 16);
+            const uint32_t gblocks = 2 * w.nb2 + (w.ntiles + 1) / 2 + ((uint32_t)N + 7) / 8;  // (an item each)
             if (N <= GRP_NARROW)
                 TN_LAUNCH((k_group_probe<2>), dim3(gblocks), dim3(GRP_THREADS), st, ga, s, ds);
             else
