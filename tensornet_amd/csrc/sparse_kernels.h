@@ -1397,12 +1397,15 @@ constexpr int VERIFY_TILE = 2048;  // lookups per tile
 // Threads of a tile's workgroup: where the chip holds all tiles at once, twice as many with half as much each.  420 tiles 21.2 us
 // with 256 threads, 15.3 with 512; 1024 tiles 31.4 and 29.2; 2440 tiles 64.1 and 67.6.
 constexpr int VERIFY_THREADS = 256, VERIFY_THREADS_FEW = 512, VERIFY_FEW_TILES = 1024;
+// Four of the latter to a CU (64 registers, none spilled; by itself the compiler takes more): 1024 tiles 28.3 -> 24.6 us, 880 of 20 slots
+// 28.8 -> 24.0.  (Eight of the former: 2440 tiles 63.6 -> 67.1.)
+constexpr int verify_waves(int threads) { return threads == VERIFY_THREADS_FEW ? 8 : 1; }
 constexpr int CLICK_BITS = 11;
 constexpr int CLICK_TABLE = 1 << CLICK_BITS;     // entries of the tile's click table
 constexpr int CLICK_TRIES = 16;
 
 template <bool CLICKS, bool COPY, int THREADS>
-__global__ __launch_bounds__(THREADS) void k_verify_values(const SlotDesc* __restrict__ descs,
+__global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(verify_waves(THREADS), 8))) void k_verify_values(const SlotDesc* __restrict__ descs,
                                                        const uint32_t* __restrict__ lbase, int N, uint32_t L,
                                                        const uint64_t* __restrict__ vals_copy, DevStatus* status,
                                                        const uint32_t* __restrict__ u_of_gi,
