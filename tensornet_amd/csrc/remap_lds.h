@@ -910,7 +910,7 @@ __global__ __launch_bounds__(GRP_THREADS) __attribute__((amdgpu_waves_per_eu(WOR
     } lds;
     constexpr uint32_t TILES = GRP_THREADS / REMAP_THREADS, SLOTS = GRP_THREADS / 64;
     const uint32_t flags0 = 2 * a.nb2, slots0 = flags0 + (a.ntiles + TILES - 1) / TILES;
-    const uint32_t item = blockIdx.x;
+    const uint32_t item = item_of_block();
     if (item < flags0) {
         if (item & 1u)
             group_count_bucket(item / 2, lds.group, a.cursor2, a.recs, a.big_k, a.aux, a.bcounts);

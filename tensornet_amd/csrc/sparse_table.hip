@@ -923,11 +923,11 @@ int launch_build_plan(SparseTable* t, const Plan& p, const Scratch& w, int N, ui
             ga.descs = p.descs;
             ga.N = N;
             ga.bcursor = w.bcursor;
-            const uint32_t gblocks = 2 * w.nb2 + (w.ntiles + 1) / 2 + ((uint32_t)N + 7) / 8;  // (an item each)
+            const dim3 gblocks = item_grid(2 * (uint64_t)w.nb2 + (w.ntiles + 1) / 2 + ((uint32_t)N + 7) / 8);
             if (N <= GRP_NARROW)
-                TN_LAUNCH((k_group_probe<2>), dim3(gblocks), dim3(GRP_THREADS), st, ga, s, ds);
+                TN_LAUNCH((k_group_probe<2>), gblocks, dim3(GRP_THREADS), st, ga, s, ds);
             else
-                TN_LAUNCH((k_group_probe<4>), dim3(gblocks), dim3(GRP_THREADS), st, ga, s, ds);
+                TN_LAUNCH((k_group_probe<4>), gblocks, dim3(GRP_THREADS), st, ga, s, ds);
             if (!own_offsets) TN_LAUNCH(k_group_offsets, dim3(1), dim3(1024), st, w.bcounts, w.bbase, w.nb2, ds);
         } else {
             TN_LAUNCH(k_lds_flags, dim3(w.ntiles), dim3(REMAP_THREADS), st, L, w.first_of, w.flag8, w.tilesum, p.descs, N,

@@ -112,6 +112,14 @@ struct DieShare {
     }
 };
 
+// One workgroup per item, however many: rows of ITEM_ROW workgroups (a launch's threads in one direction are numbered with 32 bits),
+// at most a row more than there are items.
+constexpr uint32_t ITEM_ROW = 1u << 16;
+inline dim3 item_grid(uint64_t items) {
+    return items <= ITEM_ROW ? dim3((uint32_t)items) : dim3(ITEM_ROW, (uint32_t)((items + ITEM_ROW - 1) / ITEM_ROW));
+}
+__device__ __forceinline__ uint32_t item_of_block() { return blockIdx.y * gridDim.x + blockIdx.x; }
+
 __device__ __forceinline__ uint64_t mix64(uint64_t x) {
     x ^= x >> 33;
     x *= 0xff51afd7ed558ccdull;
