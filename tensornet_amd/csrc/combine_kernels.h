@@ -345,9 +345,10 @@ static_assert(FREQUENT_LISTED <= POOL_THREADS && FREQUENT_SAMPLES % POOL_THREADS
 // Backward, step 1.  A tile of POOL_TILE lookups of a slot leaves an item for every lookup -- example, sign, lookups of the
 // example --, the items of a part side by side in the order of their positions, and where the parts start among them.
 //
-// 20 bytes move per lookup (4.9 M: 2.1 TB/s).  A wavefront takes KEY_ITEMS runs of 64 lookups, their loads in flight together, and reads the
-// extents of its examples off a ballot of the places where the id changes; an example that goes on beyond the run is
-// followed there by the whole wavefront.  Places in a part come from ballots over the bits of the part's number (as in
+// 20 bytes move per lookup (4.9 M: 34 us, 2.9 TB/s).  A wavefront takes KEY_ITEMS runs of 64 lookups and the ids of the 64 lookups on
+// either side, their loads in flight together, and reads the extents of its examples off ballots of the places where the id changes;
+// an example that goes on beyond those is followed there by the whole wavefront.  (Every run's ends followed through memory, a
+// round trip each, sixteen one after the other: 4.9 M 48 us, 860 k of 211 slots 15.7 and now 11.9.)  Places in a part come from ballots over the bits of the part's number (as in
 // k_table_part): no atomics whose order of arrival would show.
 // An item: x the example, y bits 0-10 its lookups (POOL_COUNT_MANY: as many or more), 11 the sign's first lookup, 12-31 the
 // key: of the first `spread` distinct indices these themselves, of the extra ones spread + their place among them, of the
@@ -385,19 +386,16 @@ static __global__ __launch_bounds__(256) void k_lookup_keys(const SlotDesc* __re
     const uint32_t bits = parts > 1 ? 32 - (uint32_t)__clz((int)(parts - 1)) : 0u;  // of a part's number
     const uint32_t extras = share.spreads(len) ? extra[sl * (POOL_EXTRA + 1)] : 0u, spread_all = spread + extras;
     const Global<const int64_t> ex = example_of(descs[sl]);
-    int64_t b[KEY_ITEMS], prev[KEY_ITEMS];
+    // the wavefront's lookups, and the 64 on either side of them (places outside the slot: another lookup's, not looked at)
+    const uint32_t w0 = t0 + wave * KEY_ITEMS * 64;
+    int64_t id[KEY_ITEMS];
     uint32_t u[KEY_ITEMS];
 #pragma unroll
-    for (uint32_t j = 0; j < KEY_ITEMS; j++) {
-        const uint32_t i = t0 + (wave * KEY_ITEMS + j) * 64 + lane;
-        b[j] = prev[j] = -1;
-        u[j] = 0;
-        if (i < len) {
-            b[j] = ex[i];
-            if (i > 0) prev[j] = ex[i - 1];
-            u[j] = u_of_gi[l0 + i];
-        }
-    }
+    for (uint32_t j = 0; j < KEY_ITEMS; j++) id[j] = ex[min(w0 + j * 64 + lane, len - 1)];
+    const int64_t id_before = ex[min(w0 > lane ? w0 - 1 - lane : 0u, len - 1)];
+    const int64_t id_behind = ex[min(w0 + KEY_ITEMS * 64 + lane, len - 1)];
+#pragma unroll
+    for (uint32_t j = 0; j < KEY_ITEMS; j++) u[j] = u_of_gi[l0 + min(w0 + j * 64 + lane, len - 1)];
     for (uint32_t i = tid; i < parts * KEY_WAVES; i += 256) cnt[i] = 0;
     if (tid < extras) more[tid] = extra[sl * (POOL_EXTRA + 1) + 1 + tid];
     __syncthreads();
@@ -420,42 +418,57 @@ static __global__ __launch_bounds__(256) void k_lookup_keys(const SlotDesc* __re
 #pragma unroll
         for (uint32_t j = 0; j < KEY_ITEMS; j++) u[j] = (u[j] & FIRST_BIT) | ((int)to[j] < 0 ? ~to[j] : to[j]);
     }
-    uint32_t count[KEY_ITEMS], at[KEY_ITEMS];
+    // Example ids in 32 bits from here on: those that do not fit are refused.  Where an example starts (the first lookup of a slot
+    // does, and what lies behind the last one):
+    uint32_t b[KEY_ITEMS];
+    unsigned long long heads[KEY_ITEMS];
     bool bad = false;
+    uint32_t last = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)id_before);  // of the run before
 #pragma unroll
     for (uint32_t j = 0; j < KEY_ITEMS; j++) {
-        const uint32_t base = t0 + (wave * KEY_ITEMS + j) * 64, i = base + lane;
+        const uint32_t i = w0 + j * 64 + lane;
         const bool active = i < len;
-        bad |= active && (b[j] < 0 || b[j] >= batch || prev[j] > b[j]);
-        // where an example starts (the first lookup of a slot does: prev is -1 there; and what lies behind the last one)
-        const unsigned long long heads = __ballot(!active || b[j] != prev[j]);
-        uint32_t back = 0, ahead = 0;  // lookups of the first / last example of the run before / behind it
-        if (!(heads & 1ull)) {
-            const int64_t x = __shfl(b[j], 0);
-            for (uint32_t e = base;; e -= 64) {  // lookups [0, e) of the slot are left
-                const unsigned long long other = __ballot(lane >= e || ex[e - 1 - lane] != x);
-                if (other) {
-                    back += (uint32_t)__ffsll((long long)other) - 1;
-                    break;
-                }
-                back += 64;
-            }
+        b[j] = (uint32_t)id[j];
+        uint32_t prev = (uint32_t)__shfl_up((int)b[j], 1);
+        if (lane == 0) prev = last;
+        last = (uint32_t)__builtin_amdgcn_readlane((int)b[j], 63);
+        bad |= active && ((uint64_t)id[j] >= (uint64_t)batch || (i > 0 && prev > b[j]));
+        heads[j] = __ballot(!active || i == 0 || b[j] != prev);
+    }
+    // lookups of a run's last example behind it: as far as the next run's ids go, from the last one on through memory
+    uint32_t ahead[KEY_ITEMS];
+    ahead[KEY_ITEMS - 1] = 0;
+    if (w0 + KEY_ITEMS * 64 < len) {
+        unsigned long long other = __ballot(w0 + KEY_ITEMS * 64 + lane >= len || (uint32_t)id_behind != last);
+        for (uint32_t e = w0 + KEY_ITEMS * 64; !other; other = __ballot(e + lane >= len || (uint32_t)ex[min(e + lane, len - 1)] != last)) {
+            ahead[KEY_ITEMS - 1] += 64;
+            e += 64;
         }
-        if (base + 64 < len) {
-            const int64_t x = __shfl(b[j], 63);
-            for (uint32_t e = base + 64;; e += 64) {
-                const unsigned long long other = __ballot(e + lane >= len || ex[e + lane] != x);
-                if (other) {
-                    ahead += (uint32_t)__ffsll((long long)other) - 1;
-                    break;
-                }
-                ahead += 64;
-            }
+        ahead[KEY_ITEMS - 1] += (uint32_t)__ffsll((long long)other) - 1;
+    }
+#pragma unroll
+    for (uint32_t j = KEY_ITEMS - 1; j > 0; j--) ahead[j - 1] = heads[j] ? (uint32_t)__ffsll((long long)heads[j]) - 1 : 64 + ahead[j];
+    uint32_t back = 0;  // ... of its first example ahead of it
+    if (!(heads[0] & 1ull)) {
+        const uint32_t x = (uint32_t)__builtin_amdgcn_readfirstlane((int)b[0]);
+        unsigned long long other = __ballot(lane >= w0 || (uint32_t)id_before != x);
+        for (uint32_t e = w0; !other; other = __ballot(lane >= e || (uint32_t)ex[e > lane ? e - 1 - lane : 0u] != x)) {  // lookups [0, e) are left
+            back += 64;
+            e -= 64;
         }
-        const unsigned long long below = heads & (~0ull >> (63 - lane)), above = heads & ~(~0ull >> (63 - lane));
+        back += (uint32_t)__ffsll((long long)other) - 1;
+    }
+    uint32_t count[KEY_ITEMS], at[KEY_ITEMS];
+#pragma unroll
+    for (uint32_t j = 0; j < KEY_ITEMS; j++) {
+        const uint32_t i = w0 + j * 64 + lane;
+        const bool active = i < len;
+        const unsigned long long below = heads[j] & (~0ull >> (63 - lane)), above = heads[j] & ~(~0ull >> (63 - lane));
         const uint32_t to_start = below ? lane - (63 - (uint32_t)__clzll((long long)below)) : lane + back;
-        const uint32_t to_end = above ? (uint32_t)__ffsll((long long)above) - 1 - lane : 64 - lane + ahead;
+        const uint32_t to_end = above ? (uint32_t)__ffsll((long long)above) - 1 - lane : 64 - lane + ahead[j];
         count[j] = min(to_start + to_end, POOL_COUNT_MANY);
+        // the next run's first example, if that is not its own first
+        if (j + 1 < KEY_ITEMS && !(heads[j + 1 < KEY_ITEMS ? j + 1 : j] & 1ull)) back = heads[j] ? 1 + (uint32_t)__clzll((long long)heads[j]) : 64 + back;
         // its place among the tile's lookups of its part: behind those of earlier runs and lanes
         const uint32_t index = u[j] & ~FIRST_BIT;
         const uint32_t part = index < spread_all ? turn.part(i >> 6) : turn.part_of(index - spread_all);
@@ -494,12 +507,12 @@ static __global__ __launch_bounds__(256) void k_lookup_keys(const SlotDesc* __re
     __syncthreads();
 #pragma unroll
     for (uint32_t j = 0; j < KEY_ITEMS; j++) {
-        const uint32_t i = t0 + (wave * KEY_ITEMS + j) * 64 + lane, index = u[j] & ~FIRST_BIT;
+        const uint32_t i = w0 + j * 64 + lane, index = u[j] & ~FIRST_BIT;
         if (i >= len) continue;
         const uint32_t part = index < spread_all ? turn.part(i >> 6) : turn.part_of(index - spread_all);
         const uint32_t key = index < spread_all ? index : spread_all + turn.key_of(index - spread_all);
         pool[l0 + t0 + cnt[part * KEY_WAVES + wave] + at[j]] =
-            make_uint2((uint32_t)b[j], count[j] | (u[j] & FIRST_BIT ? POOL_FIRST : 0u) | (key << POOL_KEY_SHIFT));
+            make_uint2(b[j], count[j] | (u[j] & FIRST_BIT ? POOL_FIRST : 0u) | (key << POOL_KEY_SHIFT));
     }
 }
 
