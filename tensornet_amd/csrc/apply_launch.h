@@ -52,7 +52,7 @@ struct TableApplyCall {
     uint32_t* host_err;
     RowShare share;
     hipStream_t st;
-    bool* lds_told;  // [2]: the kernels for rows in 16-byte pieces / any have been told how much LDS they may have
+    bool* lds_told;  // [4]: the kernels (rows in 16-byte pieces / any, the variants for few / many workgroups) have been told how much LDS they may have
 };
 template <int KIND>
 void launch_table_apply(const TableApplyCall& c);

@@ -135,7 +135,7 @@ struct SparseTable {
     std::vector<int64_t> plan_counts;  // distinct signs per slot of the pull that left the plan
     SmallShape small_shape{};          // how that pull laid its batch out
     size_t small_lds = 0, small_emit_lds = 0;
-    bool table_lds[2] = {false, false};  // k_table_apply (rows in 16-byte pieces / any) has been told how much it may have
+    bool table_lds[4] = {};  // k_table_apply (rows in 16-byte pieces / any, few / many workgroups) has been told how much it may have
     bool plan_small = false;   // the plan was left by a small pull: a push may take the small path, too
     bool plan_prints = false;  // the plan holds fingerprints of the batch's signs, not a copy of them
     bool exact_verify = false; // pulls that leave fingerprints keep a copy of the signs as well, pushes compare that

@@ -204,15 +204,30 @@ struct TableGroup {
     __device__ __forceinline__ void taken(uint32_t, int, int) const {}
 };
 
-// Rounds a chunk of apply_big_wave: as in small_apply_most, and four also for Adam rows of 8 and Ftrl rows of 32 where there are more
-// workgroups than the three that a CU holds of them with sixteen.  us with sixteen and with four: 300 000 records of 200 times 1500
-// signs, Adam rows of 8 98 and 83, of 16 130 and 87, of 32 141 and 94, Ftrl rows of 32 149 and 127; 128 000 of 40 times 3200 30.9 and
-// 27.1, 36.8 and 27.4, 40.4 and 30.0, 41.0 and 37.5; 64 000 23.0 and 24.5, 24.0 and 23.8, 27.0 and 25.1, 33.2 and 33.1; 5600 24.8 and
-// 25.4, 24.6 and 24.2, 26.5 and 25.6, 33.9 and 35.3.  AdaGrad rows lose: of 8 (100 000 records) 45 and 54, of 64 (300 000) 166 and 234.
-constexpr uint32_t TABLE_MANY = 768;
+// Where there are more workgroups than the chip holds of a kernel at once, two or three on a CU, a variant of which a CU holds more.
+// Rounds a chunk of apply_big_wave: as in small_apply_most, and four also for Adam rows of 8 and 64, Ftrl rows of 8, 16 and 32, whose
+// chunk of sixteen takes 21 to 34 KB.  us with sixteen and with four: 300 000 records of 200 times 1500 signs, Adam rows of 8 98 and 83,
+// of 16 130 and 87, of 32 141 and 94, of 64 170 and 138, Ftrl rows of 8 131 and 108, of 32 149 and 127; 104 000 of 40 times 2600, Adam
+// rows of 64 46.0 and 35.5, Ftrl rows of 8 37.7 and 27.2; 128 000, Adam 30.9 and 27.1, 36.8 and 27.4, 40.4 and 30.0, 47.2 and 41.3, Ftrl
+// rows of 8 38.5 and 31.6, of 32 41.0 and 37.5.  Fewer, 64 000: Adam rows of 8 23.0 and 24.5, of 16 24.0 and 23.8, of 32 27.0 and 25.1,
+// Ftrl rows of 32 33.2 and 33.1; 5600 24.8 and 25.4, 24.6 and 24.2, 26.5 and 25.6, 33.9 and 35.3.  Ftrl rows of 64 gain 6 % at 300 000
+// and lose 5 at 104 000.  AdaGrad rows lose: of 8 (100 000 records) 45 and 54, of 64 (300 000) 166 and 234.
 constexpr int table_apply_most(int kind, int big, bool many) {
-    return many && ((kind == OPT_ADAM && big == 8) || (kind == OPT_FTRL && big == 32)) ? 4 : small_apply_most(kind, big);
+    return many && ((kind == OPT_ADAM && (big == 8 || big == 64)) || (kind == OPT_FTRL && (big == 8 || big == 16 || big == 32)))
+               ? 4 : small_apply_most(kind, big);
 }
+// Wavefronts a SIMD.  AdaGrad rows of more than 8 elements take up to 216 registers by themselves, a CU holds two workgroups; held to
+// three wavefronts (168 registers, 4 to 27 spilled), us by two and by three: 300 000 records of 200 times 1500 signs, rows of 12 144 and
+// 118, of 16 97 and 82, of 32 113 and 95, of 64 149 and 129; 1 040 000 of 26 times 40 000, of 12 169 and 136, of 16 136 and 114; but 60 000
+// (469 workgroups) 27.9 and 28.4, 19.4 and 20.3, 22.0 and 23.0, 29.3 and 30.4.  (Four, 31 to 59 spilled: 129, 99, 104 and 164 for the
+// first four.)  Ftrl rows of 8 and 16 take 139 and 142, three workgroups; with four, and chunks of four rounds: rows of 16, 104 000
+// records 38.3 and 29.9, 240 000 62.4 and 54.6, 300 000 118 and 101, 1 040 000 153 and 140; rows of 8, 240 000 57.4 and 48.7, the others
+// the same.
+constexpr int table_apply_waves(int kind, int big, int lpg, bool many) {
+    return many && kind == OPT_ADAGRAD && lpg > 2 ? 3 : many && kind == OPT_FTRL && (big == 8 || big == 16) ? 4 : 1;
+}
+// How many workgroups the chip holds of the variant for few.
+constexpr uint32_t table_apply_held(int kind) { return kind == OPT_ADAGRAD ? 512 : 768; }
 
 inline size_t table_apply_lists_lds(uint32_t tiles) {
     // per tile: records before it, where they are; table: row, records, first place; per record: row, number, entry |
@@ -228,8 +243,8 @@ inline size_t table_apply_lists_lds(uint32_t tiles) {
 // workgroups fit on a CU (a chunk of 1536 records left room for one: 59 us for 34 at 60 000 records).  Rows of a power of two up to
 // 64 elements have the long signs taken by apply_big_wave (BIG > 0), the others by apply_big_groups (60 000 records of 40 times
 // 1500 signs, AdaGrad rows of 16: 28 us by the latter, 19.5 by the former).
-template <int KIND, int LPG, bool ANY, int BIG, int MOST>
-__global__ __launch_bounds__(256) void k_table_apply(TableShape b, Store s, OptDev o, const tn_sign_info* __restrict__ infos,
+template <int KIND, int LPG, bool ANY, int BIG, int MOST, int WAVES>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES, 8))) void k_table_apply(TableShape b, Store s, OptDev o, const tn_sign_info* __restrict__ infos,
                                                      const float* __restrict__ grads, int dim, const uint2* __restrict__ recs,
                                                      const uint16_t* __restrict__ boff, DevStatus* status, uint32_t* host_err,
                                                      int gbuf_floats, uint32_t wave_lds, uint32_t wave_arrays,
