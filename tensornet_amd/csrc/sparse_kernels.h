@@ -2451,16 +2451,28 @@ struct BigSrc {
 // signs: four 26.7, eight with five 28.8
 // rows of 64, 860 k of 211 slots over 10^6 ids: two 206, four 122.5 (2), eight with six 136.5 (27), with five 91.0; over 10^8:
 // four 123.9, eight with five 110.0, with four 124.6; 600 k of 20 slots: 59.5, 63.0, 69.8
-constexpr int big_most(int D) { return D <= 8 ? 2 : D <= 32 ? 4 : 8; }
-constexpr int big_waves(int D) { return D == 64 ? 5 : 6; }
+//
+// Adam and Ftrl: four rounds, five wavefronts, for rows of 16 under Ftrl two and six.  us by apply_big_groups (TILE 0) and so; 2.05 M
+// lookups of 88 slots over 10^5 ids, Adam rows of 4 52.6 and 35.1, of 8 53.9 and 35.6, of 16 56.8 and 44.1, of 32 (1.6 M) 63.5 and 52.2, of
+// 64 (0.8 M) 59.4 and 51.3, Ftrl 61.9 and 41.9, 64.2 and 44.3, 69.6 and 52.3, 74.5 and 62.2; 840 k of 211 over 10^6, Adam 60.9 and 38.2,
+// 60.8 and 40.6, 64.4 and 45.5, 74.8 and 57.7, 104 and 95, Ftrl 86 and 46, 91 and 52, 83 and 61, 94 and 78; 600 k of 20 over 10^8, few
+// frequent signs, the same within 4 %.  (Four rounds with six wavefronts, rows of 4 and 8, 22 spilled: 42 to 44; eight rounds, rows of 32
+// and 64: 54 and 53, 57 and 87.)  Ftrl rows of 64 gain 5 % with some batches and lose as much with others: they stay as they are.
+constexpr int big_most(int kind, int D) {
+    return kind == OPT_ADAGRAD ? (D <= 8 ? 2 : D <= 32 ? 4 : 8) : kind == OPT_FTRL && D == 16 ? 2 : 4;
+}
+constexpr int big_waves(int kind, int D) {
+    return kind == OPT_ADAGRAD ? (D == 64 ? 5 : 6) : D == 0 || (kind == OPT_FTRL && D == 16) ? 6 : 5;
+}
+constexpr int big_tile(int kind, int lpg) { return lpg <= 16 && !(kind == OPT_FTRL && lpg == 16) ? 4 * lpg : 0; }
 // k_apply_big_adagrad, a kernel of its own, has room for more at six wavefronts a SIMD.  3.5 M lookups of 88 slots: rows of 4 two
 // rounds 30.6 us (2 registers spilled), four 29.6; of 8 two 33.5, four 35.7 (8), eight 31.9; of 32 four 57.5, eight 51.7; of 64
 // four 121.7 (and k_apply_single beside it 100), eight 86.3 (78).  Rows of 16: four 38.8, eight spill 5.
 constexpr int big_most_alone(int D) { return D == 4 || D == 16 ? 4 : 8; }
 
 // k_apply_big for AdaGrad rows of D elements, D a power of two from 4 to 64, on a plan whose big_desc lists {row, first member,
-// records, group} of every sign with many records (written by k_emit_mapped): one wavefront per sign, by apply_big_wave.  (Adam and
-// Ftrl the same way: 800 k lookups, Adam rows of 16, 136 us a step with and without; not worth their kernels.)
+// records, group} of every sign with many records (written by k_emit_mapped): one wavefront per sign, by apply_big_wave.  It is for
+// detached updates alone; Adam's and Ftrl's take k_apply_big there.
 template <int D>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6, 8))) void k_apply_big_adagrad(
     Store s, OptDev o, PushSrc src, DevStatus* status, const uint4* __restrict__ big_desc, uint32_t desc_cap,
@@ -2480,7 +2492,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6, 8))) void
 
 // The updates of a push whose rows fit the lanes of a wavefront half, unless they are detached, by one launch: the workgroups of
 // the three kernels above side by side, those with the longest chains first.  They touch disjoint rows and one alone leaves the
-// chip half idle: k_apply_big and k_apply_vec wait for chains, and a launch for its last workgroups.  TILE: the row length k_apply_big_adagrad is made for, 0: the signs with
+// chip half idle: k_apply_big and k_apply_vec wait for chains, and a launch for its last workgroups.  TILE: the row length apply_big_wave is made for, 0: the signs with
 // many records the way of k_apply_big, with the staging a wavefront of a workgroup of four can have.
 // 2.1 M lookups of 64 slots, AdaGrad rows of 16: three launches 58 us (19 + 20 + 19), this one 42; 327 k of 40, rows of 64:
 // 77 -> 51, Ftrl rows of 1: 66 -> 38; 286 k of 47, rows of 8 + 2: 32 -> 18.
@@ -2497,7 +2509,7 @@ struct ApplyAll {
 constexpr int ALL_GBUF = 1088;  // floats of gradient staging per wavefront at most: eight workgroups to a CU up to 64 elements
 
 template <int KIND, int LPG, bool ANY, int TILE>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(big_waves(TILE), 8))) void k_apply_all(Store s, OptDev o, PushSrc src,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(big_waves(KIND, TILE), 8))) void k_apply_all(Store s, OptDev o, PushSrc src,
                                                                                               DevStatus* status, ApplyAll a) {
     src.compared.tell();
     // a push launched on a plan that turned out not to be its batch's (the host redoes it), or whose inputs are unusable
@@ -2505,7 +2517,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(big_waves(T
     if (blockIdx.x < a.big_blocks) {
         const uint32_t wave = threadIdx.x >> 6, first = blockIdx.x * 4 + wave, stride = a.big_blocks * 4;
         if constexpr (TILE != 0) {
-            __shared__ BigWave<KIND, TILE, big_most(TILE)> lds[4];
+            __shared__ BigWave<KIND, TILE, big_most(KIND, TILE)> lds[4];
             const BigSrc from{src, a.list, a.gaddr};
             const uint4 head = a.big_desc[first < a.big_cap ? first : a.big_cap - 1];
             apply_big_wave<KIND, TILE>(

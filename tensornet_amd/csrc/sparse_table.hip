@@ -1046,8 +1046,8 @@ int launch_apply_kind(SparseTable* t, RowShare share, const Store& s, const OptD
         TN_HIP(hipStreamWaitEvent(t->side, behind, 0));
         TN_HIP(hipStreamWaitEvent(t->aux, behind, 0));
     }
-    // AdaGrad rows of a power-of-two dim on a plan that describes its frequent signs have kernels of their own
-    const bool tiled = KIND == OPT_ADAGRAD && big_desc && s.D >= 4 && s.D <= 64 && (s.D & (s.D - 1)) == 0;
+    // rows of a power-of-two dim on a plan that describes its frequent signs: apply_big_wave (by a launch of its own AdaGrad's only)
+    const bool tiled = (KIND == OPT_ADAGRAD || !detach) && big_desc && s.D >= 4 && s.D <= 64 && (s.D & (s.D - 1)) == 0;
     const bool all = with_big && !detach && share.lanes != 0;
     if (with_big && !all) {
         const int gfloats = big_gbuf_floats(s.D);
@@ -1081,9 +1081,9 @@ int launch_apply_kind(SparseTable* t, RowShare share, const Store& s, const OptD
         a.wave_lds = a.wave_arrays + BIG_CHUNK * (8 + 4);
 #define TN_LAUNCH_ALL_ANY(LPG, ANY)                                                                                        \
     do {                                                                                                                   \
-        constexpr int TILE = KIND == OPT_ADAGRAD && LPG <= 16 ? 4 * LPG : 0;                                               \
+        constexpr int TILE = big_tile(KIND, LPG);                                                                          \
         const dim3 grid(a.big_blocks + a.multi_blocks + singles);                                                         \
-        if (tiled)                                                                                                         \
+        if (tiled && TILE != 0)                                                                                             \
             TN_LAUNCH((k_apply_all<KIND, LPG, ANY, TILE>), grid, dim3(256), st, s, o, src, ds, a);                         \
         else                                                                                                               \
             TN_LAUNCH_LDS((k_apply_all<KIND, LPG, ANY, 0>), grid, dim3(256), 4 * a.wave_lds, st, s, o, src, ds, a);        \
