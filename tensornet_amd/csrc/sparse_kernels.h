@@ -2458,8 +2458,11 @@ struct BigSrc {
 // 60.8 and 40.6, 64.4 and 45.5, 74.8 and 57.7, 104 and 95, Ftrl 86 and 46, 91 and 52, 83 and 61, 94 and 78; 600 k of 20 over 10^8, few
 // frequent signs, the same within 4 %.  (Four rounds with six wavefronts, rows of 4 and 8, 22 spilled: 42 to 44; eight rounds, rows of 32
 // and 64: 54 and 53, 57 and 87.)  Ftrl rows of 64 gain 5 % with some batches and lose as much with others: they stay as they are.
+// Rows of 1 and 2, one round (64 or 32 records; two the same), by apply_big_groups and so, the same two batches (2.05 M lookups): AdaGrad
+// 46.3 and 26.6, 48.7 and 28.6; 48.3 and 26.7, 49.7 and 30.0; Adam 51.0 and 29.0, 51.6 and 32.0; 60.4 and 32.4, 61.2 and 37.9; Ftrl 57.2
+// and 33.4, 60.2 and 36.7; 74.5 and 39.1, 78.2 and 42.9.
 constexpr int big_most(int kind, int D) {
-    return kind == OPT_ADAGRAD ? (D <= 8 ? 2 : D <= 32 ? 4 : 8) : kind == OPT_FTRL && D == 16 ? 2 : 4;
+    return D <= 2 ? 1 : kind == OPT_ADAGRAD ? (D <= 8 ? 2 : D <= 32 ? 4 : 8) : kind == OPT_FTRL && D == 16 ? 2 : 4;
 }
 constexpr int big_waves(int kind, int D) {
     return kind == OPT_ADAGRAD ? (D == 64 ? 5 : 6) : D == 0 || (kind == OPT_FTRL && D == 16) ? 6 : 5;

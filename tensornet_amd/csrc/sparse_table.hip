@@ -1046,8 +1046,8 @@ int launch_apply_kind(SparseTable* t, RowShare share, const Store& s, const OptD
         TN_HIP(hipStreamWaitEvent(t->side, behind, 0));
         TN_HIP(hipStreamWaitEvent(t->aux, behind, 0));
     }
-    // rows of a power-of-two dim on a plan that describes its frequent signs: apply_big_wave (by a launch of its own AdaGrad's only)
-    const bool tiled = (KIND == OPT_ADAGRAD || !detach) && big_desc && s.D >= 4 && s.D <= 64 && (s.D & (s.D - 1)) == 0;
+    // rows of a power-of-two dim on a plan that describes its frequent signs: apply_big_wave (detached AdaGrad's from 4 on only)
+    const bool tiled = big_desc && s.D <= 64 && (s.D & (s.D - 1)) == 0 && (!detach || (KIND == OPT_ADAGRAD && s.D >= 4));
     const bool all = with_big && !detach && share.lanes != 0;
     if (with_big && !all) {
         const int gfloats = big_gbuf_floats(s.D);
@@ -1079,14 +1079,20 @@ int launch_apply_kind(SparseTable* t, RowShare share, const Store& s, const OptD
         a.gbuf_floats = std::min(big_gbuf_floats(s.D), ALL_GBUF);
         a.wave_arrays = (uint32_t)align_up((size_t)(a.gbuf_floats + 3 * s.D) * sizeof(float), 8);
         a.wave_lds = a.wave_arrays + BIG_CHUNK * (8 + 4);
-#define TN_LAUNCH_ALL_ANY(LPG, ANY)                                                                                        \
+#define TN_LAUNCH_ALL_BY(LPG, ANY, TILE)                                                                                   \
     do {                                                                                                                   \
-        constexpr int TILE = big_tile(KIND, LPG);                                                                          \
-        const dim3 grid(a.big_blocks + a.multi_blocks + singles);                                                         \
-        if (tiled && TILE != 0)                                                                                             \
+        const dim3 grid(a.big_blocks + a.multi_blocks + singles);                                                          \
+        if (tiled && TILE != 0)                                                                                            \
             TN_LAUNCH((k_apply_all<KIND, LPG, ANY, TILE>), grid, dim3(256), st, s, o, src, ds, a);                         \
         else                                                                                                               \
             TN_LAUNCH_LDS((k_apply_all<KIND, LPG, ANY, 0>), grid, dim3(256), 4 * a.wave_lds, st, s, o, src, ds, a);        \
+    } while (0)
+#define TN_LAUNCH_ALL_ANY(LPG, ANY)  /* (rows of 1 and 2 are a lane's, which they do not fill) */                       \
+    do {                                                                                                               \
+        constexpr int TILE = big_tile(KIND, LPG);                                                                      \
+        if (LPG == 1 && ANY && s.D == 1) TN_LAUNCH_ALL_BY(LPG, ANY, (LPG == 1 && ANY ? 1 : TILE));                     \
+        else if (LPG == 1 && ANY && s.D == 2) TN_LAUNCH_ALL_BY(LPG, ANY, (LPG == 1 && ANY ? 2 : TILE));                \
+        else TN_LAUNCH_ALL_BY(LPG, ANY, TILE);                                                                         \
     } while (0)
 #define TN_LAUNCH_ALL(LPG)                    \
     do {                                      \
@@ -1105,6 +1111,7 @@ int launch_apply_kind(SparseTable* t, RowShare share, const Store& s, const OptD
         }
 #undef TN_LAUNCH_ALL
 #undef TN_LAUNCH_ALL_ANY
+#undef TN_LAUNCH_ALL_BY
         return TN_OK;
     }
 #define TN_LAUNCH_VEC_ANY(LPG, ANY)                                                                                \
