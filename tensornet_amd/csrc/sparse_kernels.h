@@ -2464,8 +2464,12 @@ struct BigSrc {
 constexpr int big_most(int kind, int D) {
     return D <= 2 ? 1 : kind == OPT_ADAGRAD ? (D <= 8 ? 2 : D <= 32 ? 4 : 8) : kind == OPT_FTRL && D == 16 ? 2 : 4;
 }
-constexpr int big_waves(int kind, int D) {
-    return kind == OPT_ADAGRAD ? (D == 64 ? 5 : 6) : D == 0 || (kind == OPT_FTRL && D == 16) ? 6 : 5;
+// TILE 0 spills 14 to 21 registers with six wavefronts, 2 to 4 with five; 2.05 M lookups of 88 slots over 10^5 ids, 840 k of 211 over 10^6,
+// 600 k of 20 over 10^8, AdaGrad rows of 6 55.1, 58.0, 29.6 and 45.2, 50.6, 28.6, of 12 59.9, 66.7, 25.5 and 50.4, 57.8, 25.1; longer
+// rows, of which more wavefronts wait for memory, gain and lose (of 24 86, 88, 36.9 and 71, 76, 39.6; of 96 up to 7 % lost).
+constexpr int big_waves(int kind, int lpg, int D) {
+    if (D == 0) return lpg <= 4 ? 5 : 6;
+    return kind == OPT_ADAGRAD ? (D == 64 ? 5 : 6) : kind == OPT_FTRL && D == 16 ? 6 : 5;
 }
 constexpr int big_tile(int kind, int lpg) { return lpg <= 16 && !(kind == OPT_FTRL && lpg == 16) ? 4 * lpg : 0; }
 // k_apply_big_adagrad, a kernel of its own, has room for more at six wavefronts a SIMD.  3.5 M lookups of 88 slots: rows of 4 two
@@ -2512,7 +2516,7 @@ struct ApplyAll {
 constexpr int ALL_GBUF = 1088;  // floats of gradient staging per wavefront at most: eight workgroups to a CU up to 64 elements
 
 template <int KIND, int LPG, bool ANY, int TILE>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(big_waves(KIND, TILE), 8))) void k_apply_all(Store s, OptDev o, PushSrc src,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(big_waves(KIND, LPG, TILE), 8))) void k_apply_all(Store s, OptDev o, PushSrc src,
                                                                                               DevStatus* status, ApplyAll a) {
     src.compared.tell();
     // a push launched on a plan that turned out not to be its batch's (the host redoes it), or whose inputs are unusable
