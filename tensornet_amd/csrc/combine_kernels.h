@@ -542,7 +542,8 @@ __device__ __forceinline__ uint32_t lookups_of(Global<const int64_t> ex, uint32_
 //
 // What bounds it is a workgroup's chain (slot, tiles, items; sort; rows; shares), so it wants
 // as many workgroups on a CU as there is room for, four.  4.9 M lookups in 100 slots, rows of 16: 148 us, of which the list of a
-// part's items takes 39, the sort 35, the sums 50 and writing the rows 20 (each left out in turn); 860 k in 211 slots: 33.
+// part's items takes 39, the sort 35, the sums 50 and writing the rows 20 (each left out in turn), and 134 to 139 since the sort's turns
+// follow the items (pool_items); 860 k in 211 slots: 34.
 // (A counting sort of the lookups through memory, an ordering pass and a reduction by sign, k_lookup_keys' work included: 390
 // for 205 and 103 for 48.)
 static_assert(POOL_SPREAD == 64 && POOL_EXTRA <= POOL_SPREAD, "k_reduce_pooled_shares");
