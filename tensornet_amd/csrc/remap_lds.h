@@ -1030,7 +1030,7 @@ struct EmitArgs<false> {
     uint32_t* grp_row;
     DevStatus* status;
 };
-__device__ __forceinline__ void emit_buckets(uint32_t at, uint32_t of, uint32_t nb2, const uint32_t* __restrict__ cursor2,
+__device__ __forceinline__ void emit_buckets(uint32_t of, uint32_t nb2, const uint32_t* __restrict__ cursor2,
                                              const GroupRec* __restrict__ recs, const uint2* __restrict__ aux,
                                              const uint4* __restrict__ bbase, const uint4* __restrict__ bcounts,
                                              const uint8_t* __restrict__ flag8, const uint32_t* __restrict__ wordpre,
@@ -1049,7 +1049,7 @@ __device__ __forceinline__ void emit_buckets(uint32_t at, uint32_t of, uint32_t 
     __shared__ uint32_t s_off[GRP_CAP / 2];
     __shared__ uint16_t s_cnt[GRP_CAP / 2];  // at most GRP_SLOTS records per group
     __shared__ uint4 s_part[EMIT_THREADS / 64];
-    for (uint32_t c = at; c < nb2; c += of) {
+    for (uint32_t c = blockIdx.x; c < nb2; c += of) {
         const uint32_t n = min(cursor2[c], (uint32_t)GRP_CAP);
         const size_t first = (size_t)c * GRP_CAP;
         // the bucket's records first: their loads are in flight while the bucket's offsets are worked out
@@ -1184,22 +1184,15 @@ struct MapArgs {
     const uint32_t* first_of;
     uint32_t* u_of_gi;
 };
-// The call's status (counts, new rows, errors) is final before either: the first workgroup publishes it (a launch of its own took
-// 4.6 us), and the host prepares its next call while this kernel and the gather run.  By the gather's first workgroup it had the gather
-// alone to do that in: push and pull of 2.1 M lookups in 64 slots 174.2 us a step and so 172.3, a pooled step of 211 slots, whose
-// lists of tensors take the host longer, 294 and 287.
 static __global__ __launch_bounds__(EMIT_THREADS) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_emit_mapped(
-    EmitArgs<false> a, MapArgs m, uint32_t emit_blocks, Publish pub) {
+    EmitArgs<false> a, MapArgs m, uint32_t emit_blocks) {
     extern __shared__ uint32_t lb[];  // lb[N + 1], sized by the launch
-    if (blockIdx.x == 0)
-        publish(a.status, m.ubase, (uint32_t)(m.N + 1), pub.host_dst, pub.count, pub.host_seq, pub.seq);
-    else if (blockIdx.x <= emit_blocks)
-        emit_buckets(blockIdx.x - 1, emit_blocks, a.nb2, a.cursor2, a.recs, a.aux, a.bbase, a.bcounts, a.flag8, a.wordpre, a.ids_cap,
-                     a.big_k, a.singles, a.grp_off, a.grp_cnt, a.big_list, a.big_desc, a.list, a.where_u, a.rrow, a.grp_row,
-                     a.status);
+    if (blockIdx.x < emit_blocks)
+        emit_buckets(emit_blocks, a.nb2, a.cursor2, a.recs, a.aux, a.bbase, a.bcounts, a.flag8, a.wordpre, a.ids_cap, a.big_k,
+                     a.singles, a.grp_off, a.grp_cnt, a.big_list, a.big_desc, a.list, a.where_u, a.rrow, a.grp_row, a.status);
     else
-        map_lookups(lb, blockIdx.x - 1 - emit_blocks, gridDim.x - 1 - emit_blocks, m.descs, m.lbase, m.ubase, m.N, m.L, m.first_of,
-                    a.flag8, a.wordpre, m.u_of_gi);
+        map_lookups(lb, blockIdx.x - emit_blocks, gridDim.x - emit_blocks, m.descs, m.lbase, m.ubase, m.N, m.L, m.first_of, a.flag8,
+                    a.wordpre, m.u_of_gi);
 }
 
 }  // namespace tn

@@ -213,7 +213,7 @@ static __global__ __launch_bounds__(256) void k_publish(const DevStatus* __restr
                                                  uint32_t* __restrict__ host_dst, unsigned long long* count) {
     publish(status, ubase, n_ubase, host_dst, count, nullptr, 0);
 }
-// The same as the first workgroup of another kernel.
+// The same as the first workgroup of another kernel (host_dst == nullptr: nothing to publish).
 struct Publish {
     uint32_t* host_dst;
     unsigned long long* count;
@@ -1265,20 +1265,28 @@ static __global__ __launch_bounds__(256) void k_mask_fill(const DevStatus* statu
 // vars[slot][rank, :] = table row of the sign, for every distinct sign u of
 // every slot (PopulatePulledVariable_, sparse_table_ops.cc:244-265).
 // grp_row == nullptr: where_u[u].y is the row itself instead of the group that has it.
+// pub: a call whose status is final by now publishes it here, by a workgroup of its own, the first: the host has it while the
+// others still copy (a launch of its own took 4.6 us of a pull that keeps to one stream, and where it ran on a second one, the
+// hand-over).
 template <int VEC>
 __global__ __launch_bounds__(256) void k_gather_vars(Store s, DevStatus* status, const uint32_t* __restrict__ grp_row,
                                                      const uint2* __restrict__ where_u,
                                                      const uint32_t* __restrict__ ubase, int N,
-                                                     const SlotDesc* __restrict__ descs) {
+                                                     const SlotDesc* __restrict__ descs, Publish pub) {
     __shared__ uint32_t ub[MAX_SLOTS + 1];
+    const uint32_t first = pub.host_dst ? 1u : 0u;
+    if (blockIdx.x < first) {
+        publish(status, ubase, (uint32_t)(N + 1), pub.host_dst, pub.count, pub.host_seq, pub.seq);
+        return;
+    }
     // A remap whose LDS tables overflowed dropped records: their where_u entries were never written (the
     // host repeats the call on the other path).  The flag is final before this kernel starts.
     if (status->err & DEV_ERR_REMAP_OVERFLOW) return;
     load_lbase(ub, ubase, N);
     const int chunks = s.wdim / VEC;
     const int64_t total = (int64_t)status->n_unique * chunks;
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < total; t += stride) {
+    const int64_t stride = (int64_t)(gridDim.x - first) * blockDim.x;
+    for (int64_t t = (int64_t)(blockIdx.x - first) * blockDim.x + threadIdx.x; t < total; t += stride) {
         const int64_t u = t / chunks;
         const int c = (int)(t - u * chunks);
         const uint32_t row = grp_row ? grp_row[where_u[u].y] : where_u[u].y;
