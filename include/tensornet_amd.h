@@ -296,7 +296,8 @@ int tn_sparse_table_combine_op(uint32_t table_handle, int N, const int64_t* cons
  * core/kernels/sparse_table_ops.cc:336-352 -- is
  *   sum over the lookups of that sign of pooled_grads[s][example, :] * (1 / d(n_example))
  * computed on the device (the segmented reduction of the per-lookup gradients)
- * and applied like a push.  The sum runs in the order of the lookups; that of a
+ * and applied like a push.  Example ids are as for the forward op, and below
+ * 2^32 however large the batch.  The sum runs in the order of the lookups; that of a
  * sign with more than 32 lookups in the slot may be put together from partial
  * sums, in an order that is the same in every run.  Enqueues and returns like tn_sparse_table_push_op.
  */

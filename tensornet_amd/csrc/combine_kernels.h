@@ -418,8 +418,8 @@ static __global__ __launch_bounds__(256) void k_lookup_keys(const SlotDesc* __re
 #pragma unroll
         for (uint32_t j = 0; j < KEY_ITEMS; j++) u[j] = (u[j] & FIRST_BIT) | ((int)to[j] < 0 ? ~to[j] : to[j]);
     }
-    // Example ids in 32 bits from here on: those that do not fit are refused.  Where an example starts (the first lookup of a slot
-    // does, and what lies behind the last one):
+    // Example ids in 32 bits from here on: those that do not fit are refused (batch is 2^32 at most).  Where an example starts
+    // (the first lookup of a slot does, and what lies behind the last one):
     uint32_t b[KEY_ITEMS];
     unsigned long long heads[KEY_ITEMS];
     bool bad = false;

@@ -2331,6 +2331,8 @@ int push_op_impl(uint32_t table_handle, int N, const int64_t* const* values, con
     const bool pooled = example_ids != nullptr;
     if (pooled && (batch <= 0 || combiner < COMBINE_SUM || combiner > COMBINE_SQRTN))
         return fail(TN_ERR_INVALID_ARGUMENT, "SparseTablePush (pooled): bad batch size or combiner");
+    // an item of the reduction has 32 bits for its example: lookups of examples beyond are refused as those beyond the batch are
+    if (pooled) batch = std::min(batch, (int64_t)1 << 32);
     std::lock_guard<std::mutex> lk(t->mu);
     hipStream_t st = (hipStream_t)stream;
     TN_TRY(ensure_allocated(t, st));
