@@ -1772,6 +1772,8 @@ int tn_sparse_table_pull(uint32_t handle, const uint64_t* signs, int64_t n, int 
     const uint32_t per = n > 64 * (int64_t)TABLE_PULL_FEW ? 256 : 64;
     const uint32_t workgroups = (uint32_t)std::min<int64_t>((n + per - 1) / per, TABLE_PULL_WORDS);
     const uint32_t seq = ++t->seq_pull;
+    const auto k_table_pull =
+        table_pull_few(n, per, (uint32_t)(vec ? wdim / 4 : wdim)) ? tn::k_table_pull<1> : tn::k_table_pull<PULL_AHEAD>;
     TN_LAUNCH(k_table_pull, dim3(workgroups), dim3(256), st, s, make_optdev(t), t->seed, signs, n, per, vec ? 1 : 0, out, rows,
               t->hwords, seq);
     // The rows are written when the call returns, for readers on any stream: a launch behind the pull says that it has

@@ -20,28 +20,33 @@ namespace tn {
 constexpr uint32_t TABLE_PULL_WORDS = 1024;  // workgroups of k_table_pull at most (the host reads a word of each)
 constexpr uint32_t TABLE_PULL_FEW = 256;     // ... as many as there are CUs: with fewer a workgroup takes 64 signs instead of 256
 
-// The m rows of a workgroup's signs, row after row, in pieces, several of a thread on their way (each written before the next is read,
+// The m rows of a workgroup's signs, row after row, in pieces, AHEAD of a thread on their way (each written before the next is read,
 // as the compiler leaves it -- the output might be the table -- they are a round trip each).  k_table_pull: 60 000 signs, rows of 16
-// 9.1 us one by one and 8.4 so, of 64 14.7 and 11.4; 300 000, of 16 14.0 and 13.1, of 64 28.3 and 23.8 (four on their way 25.0).
-constexpr uint32_t PULL_AHEAD = 8;
-template <typename Piece>
+// 9.1 us one by one and 8.4 by eight, of 64 14.7 and 11.4; 300 000, of 16 14.0 and 13.1, of 64 28.3 and 23.8 (four on their way 25.0).
+// One by one where a thread has two pieces at most, which it works out eight places for otherwise, in 125 registers instead of 51: 500
+// signs, rows of 1 5.1 us by eight and 4.6 so, 5000, of 4 5.7 and 5.1, of 16 5.8 and 4.9, 20 000, of 1 6.4 and 5.6.
+constexpr uint32_t PULL_AHEAD = 8, PULL_FEW = 2;
+template <uint32_t AHEAD, typename Piece>
 __device__ __forceinline__ void table_rows_out(const Store& s, const uint32_t* row, uint32_t m, float* __restrict__ out) {
     constexpr uint32_t VEC = sizeof(Piece) / sizeof(float);
     const uint32_t C = (uint32_t)s.wdim / VEC, pieces = m * C;
-    for (uint32_t q0 = threadIdx.x; q0 < pieces; q0 += 256 * PULL_AHEAD) {
-        Piece v[PULL_AHEAD];
+    for (uint32_t q0 = threadIdx.x; q0 < pieces; q0 += 256 * AHEAD) {
+        Piece v[AHEAD];
 #pragma unroll
-        for (uint32_t k = 0; k < PULL_AHEAD; k++) {
+        for (uint32_t k = 0; k < AHEAD; k++) {
             const uint32_t q = q0 + 256 * k, i = q / C, c = q - i * C, r = q < pieces ? row[i] : NO_ROW;
             v[k] = Piece{};
             if (r != NO_ROW) v[k] = *reinterpret_cast<const Piece*>(s.w + (uint64_t)r * s.wstride + c * VEC);
         }
 #pragma unroll
-        for (uint32_t k = 0; k < PULL_AHEAD; k++) {
+        for (uint32_t k = 0; k < AHEAD; k++) {
             const uint32_t q = q0 + 256 * k;
             if (q < pieces) *reinterpret_cast<Piece*>(out + (uint64_t)q * VEC) = v[k];
         }
     }
+}
+inline bool table_pull_few(int64_t n, uint32_t per, uint32_t pieces_of_row) {
+    return (uint64_t)std::min<int64_t>(n, per) * pieces_of_row <= 256 * PULL_FEW;
 }
 
 // `per` signs at a time per workgroup (256 at most): few for a short request, which then has its probes on many CUs.  A
@@ -49,7 +54,8 @@ __device__ __forceinline__ void table_rows_out(const Store& s, const uint32_t* r
 // workgroup that holds the same sign may copy it too early, so a request that inserted anything is copied out once more
 // (k_gather_rows, from rows[]).  Every workgroup tells the host itself: rows inserted | out of slots << 31 | seq << 32.
 // Bound by the two dependent reads of a row (keys, then weights).
-static __global__ __launch_bounds__(256) void k_table_pull(Store s, OptDev o, uint64_t seed, const uint64_t* __restrict__ signs,
+template <uint32_t AHEAD>
+__global__ __launch_bounds__(256) void k_table_pull(Store s, OptDev o, uint64_t seed, const uint64_t* __restrict__ signs,
                                                     int64_t n, uint32_t per, int vec, float* __restrict__ out,
                                                     uint32_t* __restrict__ rows, uint64_t* host_words, uint32_t seq) {
     __shared__ uint32_t row[256];
@@ -82,9 +88,9 @@ static __global__ __launch_bounds__(256) void k_table_pull(Store s, OptDev o, ui
             __syncthreads();
         }
         if (vec)
-            table_rows_out<float4>(s, row, m, out + first * s.wdim);
+            table_rows_out<AHEAD, float4>(s, row, m, out + first * s.wdim);
         else
-            table_rows_out<float>(s, row, m, out + first * s.wdim);
+            table_rows_out<AHEAD, float>(s, row, m, out + first * s.wdim);
         __syncthreads();
     }
     if (tid == 0) {

@@ -1,5 +1,6 @@
 """Table-level push at the numbers of buckets around which its counters' places in LDS jump, table-level pull of rows whose pieces
-fill a workgroup's turns exactly, just not, or by one more, in pieces of four elements and of one."""
+fill a workgroup's turns exactly, just not, or by one more, in pieces of four elements and of one, on either side of the two pieces of a
+thread up to which they are copied one by one."""
 import numpy as np
 import pytest
 
@@ -26,7 +27,7 @@ def test_push_of_so_many_buckets(tn, oracle, n, opt, dim):
     pair.assert_rows_match(base)
 
 
-@pytest.mark.parametrize("dim", [3, 4, 32, 36, 64])
+@pytest.mark.parametrize("dim", [1, 2, 3, 4, 8, 12, 32, 36, 64])
 @pytest.mark.parametrize("n", [1, 63, 64, 65, 16384, 16385, 17000])
 def test_pull_of_rows(tn, oracle, dim, n):
     rng = np.random.default_rng(n + dim)
