@@ -1573,7 +1573,8 @@ __device__ __forceinline__ void ftrl_elem(const OptDev& o, float g, float& w, fl
     }
 }
 
-// x of lane L of every group of LPG lanes, in all lanes of the group (which are active together).
+// x of lane L of every group of LPG lanes, in all lanes of the group (which are active together); of 32 lanes, in the half that lane
+// L is in, where L is its last lane in both.
 template <int LPG, int L>
 __device__ __forceinline__ int from_group_lane(int x) {
     static_assert(L < LPG && LPG <= 32, "a lane of the group");
@@ -1586,8 +1587,8 @@ __device__ __forceinline__ int from_group_lane(int x) {
     } else if constexpr (LPG == 8) {  // row_newbcast: the first two banks of a row from its lane L, the others from lane 8 + L
         const int lower = __builtin_amdgcn_update_dpp(x, x, 0x150 + L, 0xF, 0x3, false);
         return __builtin_amdgcn_update_dpp(lower, x, 0x150 + 8 + L, 0xF, 0xC, false);
-    } else if constexpr (LPG == 16) {
-        return __builtin_amdgcn_update_dpp(x, x, 0x150 + L, 0xF, 0xF, false);
+    } else if constexpr (LPG == 16 || L % 16 != 15) {
+        return __builtin_amdgcn_update_dpp(x, x, 0x150 + L % 16, 0xF, 0xF, false);
     } else {
         return __shfl(x, (int)(__lane_id() & ~31u) + L);
     }
@@ -1601,7 +1602,10 @@ __device__ __forceinline__ double from_group_lane(double x) {
 // element order 0 .. D-1.  A chain through the lanes; the N chains run side by side, and the sum goes from lane to lane
 // through registers (data-parallel primitives), a tenth of the time it takes by way of LDS (__shfl).  k_apply_all, rows of 16: 4.9 M
 // lookups of 100 slots 142 -> 137 us, 2.1 M of 64 40.8 -> 38.5; k_small_apply, rows of 64, 40 slots of 8192 50 -> 47.  (Four records
-// of rows of 64 side by side there, too: 57, the registers of their squares are spilled.)
+// of rows of 64 side by side there, too: 57, the registers of their squares are spilled.)  Of 32 lanes the halves go by registers, too, and
+// only from half to half by LDS: k_table_apply, 520 000 records, rows of 66 384 us in a loop by way of LDS and 329, of 128 477 and 451;
+// push and pull of 26 slots of 4096 lookups, of 100 86 and 75, 8 of 1024 42 and 36.  (All 32 steps by LDS one behind the other: 30
+// registers more, of 128 520.)
 template <int LPG, int N, int L = 0>
 __device__ __forceinline__ void square_sums(const float4 (&sq)[N], double (&tot)[N]) {
 #pragma unroll

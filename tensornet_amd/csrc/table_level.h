@@ -226,7 +226,9 @@ constexpr int table_apply_most(int kind, int big, bool many) {
 // three wavefronts (168 registers, 4 to 27 spilled), us by two and by three: 300 000 records of 200 times 1500 signs, rows of 12 144 and
 // 118, of 16 97 and 82, of 32 113 and 95, of 64 149 and 129; 1 040 000 of 26 times 40 000, of 12 169 and 136, of 16 136 and 114; but 60 000
 // (469 workgroups) 27.9 and 28.4, 19.4 and 20.3, 22.0 and 23.0, 29.3 and 30.4.  (Four, 31 to 59 spilled: 129, 99, 104 and 164 for the
-// first four.)  Ftrl rows of 8 and 16 take 139 and 142, three workgroups; with four, and chunks of four rounds: rows of 16, 104 000
+// first four.)  Rows of more than 64, of which LDS holds two workgroups at most, are the same either way: 300 000, of 66 327 and 331, of
+// 128 521 and 517; 520 000 of 26 times 20 000 329 and 323, 451 and 438.
+// Ftrl rows of 8 and 16 take 139 and 142, three workgroups; with four, and chunks of four rounds: rows of 16, 104 000
 // records 38.3 and 29.9, 240 000 62.4 and 54.6, 300 000 118 and 101, 1 040 000 153 and 140; rows of 8, 240 000 57.4 and 48.7, the others
 // the same.
 constexpr int table_apply_waves(int kind, int big, int lpg, bool many) {
