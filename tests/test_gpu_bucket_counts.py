@@ -25,3 +25,20 @@ def test_larger_buckets(tn, oracle, slots, lookups, dim):
         names = kernels_of(tn, lambda: pair.push_op(values, grads, [(rng.random(len(v)) < 0.3).astype(np.int64) for v in values]))
         assert any(k.startswith("k_small_apply") for k in names) and "k_remap_insert" not in names  # (no bucket overflowed)
         assert pair.assert_rows_match(all_signs(values)) > 0.99
+
+
+@pytest.mark.parametrize("slots,lookups", [(20, 4700), (20, 5300), (20, 8100)])
+def test_buckets_of_distinct_signs(tn, oracle, slots, lookups):
+    """Nearly as many signs as records: the buckets' tables are as full as they get."""
+    rng = np.random.default_rng(lookups)
+    pool = synth.splitmix64(np.arange(1, slots * lookups + 1, dtype=np.uint64)).view(np.int64)
+    pair = Pair(tn, oracle, "AdaGrad", 4, dict(learning_rate=0.01, initial_g2sum=0.1, epsilon=1e-8), reserve=400000, zero_init=True)
+    pair.populate(pool.view(np.uint64))
+    for _ in range(2):
+        values = list(rng.permutation(pool).reshape(slots, lookups))
+        values[1][:50] = values[0][:50]
+        counts = check_pull(pair, values)
+        grads = synth.make_grads(counts, 4, 0.01)
+        names = kernels_of(tn, lambda: pair.push_op(values, grads, [(rng.random(len(v)) < 0.3).astype(np.int64) for v in values]))
+        assert any(k.startswith("k_small_apply") for k in names) and "k_remap_insert" not in names
+        assert pair.assert_rows_match(all_signs(values)) > 0.99
