@@ -41,7 +41,13 @@ constexpr int SMALL_BUCKETS_MAX = 2048;
 // Push and pull, sum of the kernels, us, up to 2048 buckets of 64 lookups and so: 26 slots of 4096, Adam rows of 16 43.0 and 40.2
 // (768 of them 41.7); AdaGrad rows of 16 80 of 2000 54.0 and 50.2, 40 of 4000 50.8 and 48.1, 12 of 8000 46.6 and 44.5; rows of 64 80
 // of 2000 74.5 and 71.4; 30 of 8000, Adam rows of 16 55.9 and 53.2 (one for 256 52.0); 47 of 6400, rows of 8 + 2 65.5 and 63.2 (65.8);
-// 40 of 8192, rows of 64, one for 160 183.2, 192 189.
+// 40 of 8192, rows of 64, one for 160 183.2, 192 189.  Not a few more than the chip holds: 1032 instead of 1020, 20 slots of 6500, rows
+// of 64, k_small_apply 30.2 and 28.3.
+// Rows of more than 32 elements: only as few as leave a CU as many workgroups of k_small_pull_rest, most of which copy rows then
+// (small_rest_held).  With five to a CU instead of eight: 24 slots of 8192, AdaGrad rows of 64 22.7 us and 18.3, 20 of 8192 under Adam
+// 19.8 and 17.0; shorter rows gain more by fewer buckets.
+// Batches whose signs are nearly all in most slots lose: 10 000 ids in 20 slots of 8192, Adam rows of 1 44.7 and 47.0, the signs with
+// many records having half as many wavefronts.
 constexpr size_t SMALL_BUCKETS_FEW = 1024;
 constexpr size_t small_bucket_lookups(int dim) { return dim > 32 ? 160 : 192; }
 constexpr int SMALL_THREADS = 512;           // k_small_slots; twice as many for slots of more than SMALL_SLOT_SHORT lookups
@@ -322,6 +328,12 @@ inline size_t small_emit_lds(int N, uint32_t cap, uint32_t table) {
     // per slot: records before it, where its records are, its first lookup; table: row, records / number;
     // per record: row, gi, occurrences | entry, arrival, slot, list
     return align_up((size_t)(N + 1) * 4 + (size_t)N * 8 + (size_t)table * 12 + (size_t)cap * 20, 8);
+}
+
+// Workgroups of k_small_pull_rest on a CU, of the eight that its registers let there be: all of them are given the buckets' LDS.
+inline uint32_t small_rest_held(size_t emit_lds) {
+    constexpr size_t own = (FINISH_THREADS / 64 + 1) * SMALL_WORDS * 8 + SMALL_WORDS * 4 + 64;  // (small_finish, the counters)
+    return (uint32_t)std::min<size_t>(8, 160 * 1024 / (emit_lds + own));
 }
 
 // The records of a bucket, slot after slot, grouped by row in LDS.

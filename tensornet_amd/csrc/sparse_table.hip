@@ -1297,13 +1297,19 @@ bool small_batch_shape(SparseTable* t, int N, const int64_t* lens, SmallShape& b
     // (every bucket's workgroup looks at all slots: fewer buckets where there are many)
     const size_t most = std::min<size_t>({(L + SMALL_BUCKET_RECORDS - 1) / SMALL_BUCKET_RECORDS, (size_t)SMALL_BUCKETS_MAX,
                                           std::max<size_t>(64, (size_t)(1 << 18) / N)});
+    // room for twice the records expected of a batch of distinct signs and for four signs that are in every slot
+    auto lay_out = [&](size_t want) {
+        // (as many as the chip holds, and not a few more)
+        b.nbp = (uint32_t)std::max<size_t>(1, (want + (want < SMALL_BUCKETS_FEW ? b.parts - 1 : 0)) / b.parts);
+        b.cap = (uint32_t)align_up(2 * (L / b.buckets()) + 64 + 4 * (size_t)N, 64);
+        return small_emit_lds(N, b.cap, small_emit_table(b.cap));
+    };
+    const uint32_t wide_held = t->dim > 32 ? small_rest_held(lay_out(most)) : 0;
     for (size_t want = std::min(most, std::max<size_t>(SMALL_BUCKETS_FEW, L / small_bucket_lookups(t->dim)));;
          want = std::min(most, want + want / 4)) {
-        b.nbp = (uint32_t)std::max<size_t>(1, (want + b.parts - 1) / b.parts);
-        // room for twice the records expected of a batch of distinct signs and for four signs that are in every slot
-        b.cap = (uint32_t)align_up(2 * (L / b.buckets()) + 64 + 4 * (size_t)N, 64);
-        // (no fewer than let the pull's second half be one launch)
-        if (want == most || small_emit_lds(N, b.cap, small_emit_table(b.cap)) <= SMALL_SHARED_LDS) break;
+        // no fewer than let the pull's second half be one launch, and a CU hold as many workgroups of it where rows are wide
+        const size_t lds = lay_out(want);
+        if (want == most || (lds <= SMALL_SHARED_LDS && small_rest_held(lds) >= wide_held)) break;
     }
     if (!t->small_lds) {
         t->small_lds = 144 * 1024;

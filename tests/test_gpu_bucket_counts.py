@@ -10,7 +10,9 @@ from helpers import Pair, all_signs, check_pull, kernels_of
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("slots,lookups,dim", [(16, 4096, 8), (17, 3856, 8), (24, 8192, 16), (40, 5000, 40), (100, 2000, 4), (200, 500, 8)])
+@pytest.mark.parametrize("slots,lookups,dim", [(16, 4096, 8), (17, 3856, 8), (24, 8192, 16), (40, 5000, 40), (100, 2000, 4), (200, 500, 8),
+                                               # parts of slots that do not divide the buckets; fewer of them where rows are wide
+                                               (20, 6500, 16), (20, 5494, 40), (20, 8192, 64)])
 def test_larger_buckets(tn, oracle, slots, lookups, dim):
     rng = np.random.default_rng(slots + lookups)
     pool = synth.splitmix64(np.arange(1, 60001, dtype=np.uint64)).view(np.int64)
