@@ -50,17 +50,18 @@ void launch_table_apply(const TableApplyCall& c) {
     const size_t wave_lds = small_apply_wave_lds(s.D), lists = table_apply_lists_lds(c.b.tiles);
     const size_t lds = lists + (lds_big ? TABLE_WAVES * wave_lds : 0);
     const bool many = c.b.nb > table_apply_held(KIND);
-#define TN_LAUNCH_TABLE_BY(LPG, ANY, BIG, MANY)                                                                       \
-    do {                                                                                                              \
-        constexpr int MOST = table_apply_most(KIND, BIG, MANY), WAVES = table_apply_waves(KIND, BIG, LPG, MANY);      \
-        bool& told = c.lds_told[(MANY ? 2 : 0) + ANY];                                                                \
-        if (lds_big && !told) {                                                                                       \
-            told = true;                                                                                              \
-            (void)big_lds_bytes_for(reinterpret_cast<const void*>(k_table_apply<KIND, LPG, ANY, BIG, MOST, WAVES>));  \
-        }                                                                                                             \
-        TN_LAUNCH_LDS((k_table_apply<KIND, LPG, ANY, BIG, MOST, WAVES>), dim3(c.b.nb), dim3(256), lds, c.st, c.b, s,  \
-                      c.o, c.infos, c.grads, c.dim, c.recs, c.boff, c.ds, c.host_err, big_gbuf_floats(s.D),           \
-                      (uint32_t)wave_lds, (uint32_t)align_up(big_lds_bytes(s.D), 8), (uint32_t)lists);                \
+// (MANY in the kernel's arguments: the profiler's name of the launch tells which variant it is)
+#define TN_LAUNCH_TABLE_BY(LPG, ANY, BIG, MANY)                                                                             \
+    do {                                                                                                                    \
+        bool& told = c.lds_told[(MANY ? 2 : 0) + ANY];                                                                      \
+        if (lds_big && !told) {                                                                                             \
+            told = true;                                                                                                    \
+            (void)big_lds_bytes_for(reinterpret_cast<const void*>(                                                          \
+                k_table_apply<KIND, LPG, ANY, BIG, table_apply_most(KIND, BIG, MANY), table_apply_waves(KIND, BIG, LPG, MANY)>)); \
+        }                                                                                                                   \
+        TN_LAUNCH_LDS((k_table_apply<KIND, LPG, ANY, BIG, table_apply_most(KIND, BIG, MANY), table_apply_waves(KIND, BIG, LPG, MANY)>), \
+                      dim3(c.b.nb), dim3(256), lds, c.st, c.b, s, c.o, c.infos, c.grads, c.dim, c.recs, c.boff, c.ds, c.host_err, \
+                      big_gbuf_floats(s.D), (uint32_t)wave_lds, (uint32_t)align_up(big_lds_bytes(s.D), 8), (uint32_t)lists); \
     } while (0)
 #define TN_LAUNCH_TABLE_BIG(LPG, ANY, BIG)                             \
     do {                                                               \

@@ -25,6 +25,8 @@ def test_signs_in_most_slots(tn, oracle, opt, dim, cvm):
         counts = check_pull(pair, values, loose_col=(dim + 1) if cvm else None)
         grads = synth.make_grads(counts, pair.wf, 0.05, seed=step)
         labels = [(rng.random(len(v)) < 0.3).astype(np.int64) for v in values]
-        assert any(k.startswith("k_apply_all") for k in kernels_of(tn, lambda: pair.push_op(values, grads, labels)))
+        applied = [k for k in kernels_of(tn, lambda: pair.push_op(values, grads, labels)) if k.startswith("k_apply_all<")]
+        # (", 0>": the kernel whose signs with many records go through LDS record by record, whatever the row's length)
+        assert [k.endswith(", 0>") for k in applied] == [dim == 12 or opt == "Ftrl" and dim == 64]
         # (with cvm one of the dim + 2 columns is a logarithm, which follows the libm in use)
         assert pair.assert_rows_match(all_signs(values)) > 0.99 * ((dim + 1) / (dim + 2) if cvm else 1)

@@ -6,7 +6,7 @@ import pytest
 
 from tensornet_amd import synth
 
-from helpers import Pair, dev
+from helpers import Pair, dev, kernels_of
 
 from test_gpu_table_level import HP, pushed
 
@@ -22,7 +22,11 @@ def test_push_of_so_many_buckets(tn, oracle, n, opt, dim):
     pair = Pair(tn, oracle, opt, dim, HP[opt], reserve=200000)
     base = pair.populate(synth.splitmix64(np.arange(1, 60001, dtype=np.uint64)))
     req = base[(rng.random(n) ** (2 if dim == 4 else 6) * len(base)).astype(np.int64)]
-    infos, grads = pushed(tn, oracle, pair, req, rng)
+    out = []
+    names = kernels_of(tn, lambda: out.append(pushed(tn, oracle, pair, req, rng)))
+    many = n > 128 * (512 if opt == "AdaGrad" else 768)
+    assert [k.endswith(", true)>") for k in names if k.startswith("k_table_apply<")] == [many]
+    infos, grads = out[0]
     assert pair.o.push(infos, grads) == 0
     pair.assert_rows_match(base)
 
