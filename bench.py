@@ -91,8 +91,6 @@ def kernel_algorithmic_bytes(name, opt, dim, shape):
         "k_lds_flags": 4 * L,
         "k_lds_assign": 4 * U,
         "k_lds_mapped": 12 * L,                # first position in, mapped id out
-        "k_group_emit": 52 * U + 20 * G,       # records, placement and rows in; member lists, per-record index and
-                                               # row, groups out
         # global-table fallback
         "k_remap_insert": 8 * L, "k_assign_rank": 8 * U, "k_write_mapped": 8 * L, "k_count_show": 8 * L,
         "k_mask_insert": 16 * U, "k_mask_compact": 16 * G, "k_mask_fill": 32 * U,
@@ -101,7 +99,9 @@ def kernel_algorithmic_bytes(name, opt, dim, shape):
         "k_probe": 8 * G + 4 * G,              # one stored-key compare per distinct sign, row number out
         "k_group_probe": 24 * U + 20 * U + 4 * L,      # placement of the records, their probes, the lookups' flags
         "k_assign_init": 4 * U,
-        "k_emit_mapped": 52 * U + 20 * G + 12 * L,     # member lists; mapped ids
+        # records, placement and rows in; member lists, per-record index and row, the groups' rows, place and count of those of
+        # several records (of all for k_apply_scalar) out; mapped ids
+        "k_emit_mapped": 52 * U + 4 * G + 8 * (G - shape["G1"] if dim <= 128 else G) + 12 * L,
         "k_gather_vars": U * (2 * row + 4),    # row read + variable row write
         # push
         # the op's signs and labels, against the pull's copy of the signs (COPY) or its fingerprints of them
@@ -117,6 +117,7 @@ def kernel_algorithmic_bytes(name, opt, dim, shape):
         "k_small_slots": 18 * L + 24 * U,      # signs in, their copy and first positions out; a stored-key compare, record and
         "k_small_slots_long": 18 * L + 24 * U, # row of every distinct sign
         "k_small_group_finish": 10 * L + U * (2 * row + 4),       # first position in, mapped id out; rows into the variables
+        "k_group_emit": 24 * U,                # the records in, by sign out
         "k_small_pull_rest": 10 * L + U * (2 * row + 4) + 24 * U, # the same; the records in, by sign out
         "k_small_verify": 26 * L,              # signs, their copy, labels, first positions
         "k_small_apply": apply_bytes(U, G),

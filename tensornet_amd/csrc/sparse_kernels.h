@@ -2464,21 +2464,26 @@ struct BigSrc {
 // rows of 64, 860 k of 211 slots over 10^6 ids: two 206, four 122.5 (2), eight with six 136.5 (27), with five 91.0; over 10^8:
 // four 123.9, eight with five 110.0, with four 124.6; 600 k of 20 slots: 59.5, 63.0, 69.8
 //
-// Adam and Ftrl: four rounds, five wavefronts, for rows of 16 under Ftrl two and six.  us by apply_big_groups (TILE 0) and so; 2.05 M
-// lookups of 88 slots over 10^5 ids, Adam rows of 4 52.6 and 35.1, of 8 53.9 and 35.6, of 16 56.8 and 44.1, of 32 (1.6 M) 63.5 and 52.2, of
-// 64 (0.8 M) 59.4 and 51.3, Ftrl 61.9 and 41.9, 64.2 and 44.3, 69.6 and 52.3, 74.5 and 62.2; 840 k of 211 over 10^6, Adam 60.9 and 38.2,
-// 60.8 and 40.6, 64.4 and 45.5, 74.8 and 57.7, 104 and 95, Ftrl 86 and 46, 91 and 52, 83 and 61, 94 and 78; 600 k of 20 over 10^8, few
-// frequent signs, the same within 4 %.  (Four rounds with six wavefronts, rows of 4 and 8, 22 spilled: 42 to 44; eight rounds, rows of 32
-// and 64: 54 and 53, 57 and 87.)  Ftrl rows of 64 gain 5 % with some batches and lose as much with others: they stay as they are.
-// Rows of 1 and 2, one round (64 or 32 records; two the same), by apply_big_groups and so, the same two batches (2.05 M lookups): AdaGrad
-// 46.3 and 26.6, 48.7 and 28.6; 48.3 and 26.7, 49.7 and 30.0; Adam 51.0 and 29.0, 51.6 and 32.0; 60.4 and 32.4, 61.2 and 37.9; Ftrl 57.2
-// and 33.4, 60.2 and 36.7; 74.5 and 39.1, 78.2 and 42.9.
+// Adam and Ftrl: four rounds, five wavefronts, for rows of 16 under Ftrl two and six.  us by apply_big_groups (TILE 0) and so, of three
+// batches: 2.05 M lookups of 88 slots over 10^5 ids; 840 k of 211 over 10^6; 600 k of 20 over 10^8, few frequent signs.
+//   Adam rows of 4 54.5, 56.0, 26.8 and 35.8, 36.4, 23.7; of 8 56.3, 56.8, 22.4 and 36.2, 38.0, 21.0; of 16 60.1, 59.4, 28.6 and 44.9,
+//   42.3, 27.5; of 32 73.8, 74.1, 42.7 and 61.5, 58.1, 38.7; of 64 113, 106, 77.4 and 98.4, 98.0, 73.7
+//   Ftrl rows of 4 68.2, 81.5, 30.0 and 42.6, 44.2, 27.4; of 8 70.7, 81.9, 26.0 and 44.9, 49.0, 25.3; of 16 76.6, 83.6, 29.3 and 53.6,
+//   59.5, 28.7 (by four rounds and five wavefronts 54.7, 60.1, 28.4; 2.05 M spread evenly over 10^5 ids 167 and 196); of 32 88.8, 93.2,
+//   42.5 and 77.1, 77.6, 43.2
+// (Four rounds with six wavefronts, rows of 4 and 8, 22 spilled: 42 to 44; eight rounds, rows of 32 and 64: 54 and 53, 57 and 87.)  Ftrl
+// rows of 64 gain 5 % with some batches and lose as much with others: they stay as they are.
+// Rows of 1 and 2, one round (64 or 32 records; two the same), the first two batches: AdaGrad 48.1, 46.3 and 27.4, 25.3; 50.5, 49.8 and
+// 29.2, 29.9; Adam 53.3, 56.9 and 30.5, 32.2; 53.7, 56.3 and 32.2, 35.8; Ftrl 63.7, 76.6 and 36.2, 38.8; 66.5, 77.7 and 39.6, 41.7.
 constexpr int big_most(int kind, int D) {
     return D <= 2 ? 1 : kind == OPT_ADAGRAD ? (D <= 8 ? 2 : D <= 32 ? 4 : 8) : kind == OPT_FTRL && D == 16 ? 2 : 4;
 }
-// TILE 0 spills 14 to 21 registers with six wavefronts, 2 to 4 with five; 2.05 M lookups of 88 slots over 10^5 ids, 840 k of 211 over 10^6,
-// 600 k of 20 over 10^8, AdaGrad rows of 6 55.1, 58.0, 29.6 and 45.2, 50.6, 28.6, of 12 59.9, 66.7, 25.5 and 50.4, 57.8, 25.1; longer
-// rows, of which more wavefronts wait for memory, gain and lose (of 24 86, 88, 36.9 and 71, 76, 39.6; of 96 up to 7 % lost).
+// TILE 0 spills 14 to 21 registers with six wavefronts, 2 to 4 with five; the same three batches, AdaGrad rows of 6 55.6, 55.9, 24.5 and
+// 45.5, 50.7, 22.9, of 12 61.3, 64.7, 21.3 and 51.2, 55.9, 20.1; Adam 59.8, 59.3, 27.2 and 52.6, 53.8, 25.8, 62.8, 64.8, 28.2 and 54.2,
+// 57.9, 27.9; Ftrl 73.8, 87.4, 29.3 and 65.2, 83.6, 27.3, 78.3, 87.3, 28.6 and 69.5, 79.2, 28.8.  Longer rows, of which more wavefronts
+// wait for memory, gain and lose (AdaGrad of 24 86, 88, 36.9 and 71, 76, 39.6; of 96 up to 7 % lost).  Pushes of another batch than the
+// last pull's, whose plan has no big_desc, rows of every length to 16: 0.82 to 1.01 of the time; slower where few signs are frequent,
+// 800 k of 40 slots over 10^7 ids, rows of 3 and 12, Ftrl 31.5 and 34.5, 28.6 and 29.6, Adam 30.6 and 31.0, 26.5 and 27.2.
 constexpr int big_waves(int kind, int lpg, int D) {
     if (D == 0) return lpg <= 4 ? 5 : 6;
     return kind == OPT_ADAGRAD ? (D == 64 ? 5 : 6) : kind == OPT_FTRL && D == 16 ? 6 : 5;
@@ -2491,7 +2496,7 @@ constexpr int big_most_alone(int D) { return D == 4 || D == 16 ? 4 : 8; }
 
 // k_apply_big for AdaGrad rows of D elements, D a power of two from 4 to 64, on a plan whose big_desc lists {row, first member,
 // records, group} of every sign with many records (written by k_emit_mapped): one wavefront per sign, by apply_big_wave.  It is for
-// detached updates alone; Adam's and Ftrl's take k_apply_big there.
+// detached updates alone, where Adam's and Ftrl's and AdaGrad's of other lengths take k_apply_big.
 template <int D>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6, 8))) void k_apply_big_adagrad(
     Store s, OptDev o, PushSrc src, DevStatus* status, const uint4* __restrict__ big_desc, uint32_t desc_cap,
