@@ -298,7 +298,7 @@ int tn_sparse_table_combine_op(uint32_t table_handle, int N, const int64_t* cons
  * computed on the device (the segmented reduction of the per-lookup gradients)
  * and applied like a push.  Example ids are as for the forward op, and below
  * 2^32 however large the batch.  The sum runs in the order of the lookups; that of a
- * sign with more than 32 lookups in the slot may be put together from partial
+ * sign with three lookups or more in the slot may be put together from partial
  * sums, in an order that is the same in every run.  Enqueues and returns like tn_sparse_table_push_op.
  */
 int tn_sparse_table_push_pooled_op(uint32_t table_handle, int N, const int64_t* const* values,
